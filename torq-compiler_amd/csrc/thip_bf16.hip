@@ -306,6 +306,10 @@ hipError_t launchFcBf16(const FcBf16Args &a, const LaunchCtx &ctx) {
     // a very wide N with a short K and no K split: every wave streams its own columns (THIP_NO_FC_WIDE: off)
     const bool wide = a.w_fragments >= 1 && a.ksplit == 1 && (a.K + 63) / 64 <= kFcBf16WideMaxSteps && (a.N + 31) / 32 >= 1024 &&
                       !ctx.tuning->noFcWide;
+    // more rows than the wide kernel reads its weights once or twice for, or than one block of rows: whole tiles
+    if (a.w_fragments != 2 && !(wide && a.M <= 64)) {
+        if (const int tile = fcBf16TileChoice(a, ctx)) return launchFcBf16Tile(a, tile, ctx);
+    }
     if (a.w_fragments == 2) {
         if (!a.qscale || !a.qbias || a.qblock < 32 || a.qblock % 32 != 0 || a.qcols < (a.N + 31) / 32 * 32 || a.qcols % 32 != 0) return hipErrorInvalidValue;
         if ((((uintptr_t)a.qscale) & 1) || (((uintptr_t)a.qbias) & 3)) return hipErrorInvalidValue;

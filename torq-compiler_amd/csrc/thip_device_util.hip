@@ -268,6 +268,7 @@ Tuning tuningFromEnvironment() {
     if (const char *v = getenv("THIP_DEPTHWISE_P")) t.depthwisePixels = atoi(v);
     if (const char *v = getenv("THIP_FC_WIDE_U")) t.fcWideU = atoi(v);
     if (const char *v = getenv("THIP_FC_WIDE_WAVES")) t.fcWideWaves = atoi(v);
+    t.fcTile = digit("THIP_FC_TILE", -1);
     if (const char *v = getenv("THIP_DENSE_SHORT_K")) t.denseShortK = atoi(v);
     t.noK128 = flag("THIP_NO_K128");
     t.noFcDeep = flag("THIP_NO_FC_DEEP");

@@ -37,6 +37,7 @@ struct Tuning {
     int depthwisePixels = 0;        // THIP_DEPTHWISE_P: pixels per thread of the window-row kernel
     int fcWideU = 0;                // THIP_FC_WIDE_U: k-steps per register buffer of the wide bf16 kernel
     int fcWideWaves = 0;            // THIP_FC_WIDE_WAVES=4 / 8 / 16: waves per block of the wide bf16 kernel (0: by weight format and rows)
+    int fcTile = -1;                // THIP_FC_TILE=1 .. 5: tile of the bf16 linears with many rows (0: none of them; < 0: by shape)
     int denseShortK = 384;          // THIP_DENSE_SHORT_K: padded K up to which the 128 x 128 dense tile runs two stages deep, four blocks per CU
     bool noK128 = false;            // THIP_NO_K128: no 128-byte k-tiles chosen at launch (the emitter reads the same switch for its own choice)
     bool noFcDeep = false;          // THIP_NO_FC_DEEP
@@ -196,6 +197,9 @@ inline int fcBf16PreferredSplit(int M, int N, int K) {
     return split < 2 ? 1 : (int)split;
 }
 hipError_t launchFcBf16(const FcBf16Args &a, const LaunchCtx &ctx);
+// Its tile form for many input rows: which tile these operands take (0: none), and its launch.
+int fcBf16TileChoice(const FcBf16Args &a, const LaunchCtx &ctx);
+hipError_t launchFcBf16Tile(const FcBf16Args &a, int choice, const LaunchCtx &ctx);
 // ---- decode-shaped bf16 programs: at most 32 input rows, the weights dominate the traffic ---------------------
 //
 // dec_linear: out[m][n] = bf16(clamp(sum_k x[m][k] * W[k][n] + bias[n])) with W = the expansion of block-quantized
