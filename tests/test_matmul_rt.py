@@ -1,0 +1,32 @@
+"""int8 matmuls with a run-time input2 as one launch: every tile height, ragged ends of every kind, against the oracle."""
+import numpy as np
+import pytest
+
+from helpers import assert_bit_exact, oracle_eval, run_on_gpu
+from torq_compiler_amd import workloads as w
+
+pytestmark = pytest.mark.gpu
+
+I8 = dict(out_dtype=np.int8, scale=(1 << 30) + 12345, shift=41, output_zp=3)
+
+
+@pytest.mark.parametrize("kw", [
+    dict(B=1, M=1, K=16, N=4), dict(B=3, M=5, K=7, N=3, **I8),            # fewer bytes per batch than one load
+    dict(B=2, M=3, K=130, N=2, out_dtype=np.int32), dict(B=1, M=33, K=257, N=1), dict(B=2, M=40, K=129, N=3, **I8),
+    dict(B=2, M=33, K=130, N=131, **I8), dict(B=2, M=31, K=100, N=129, bias=-77, out_dtype=np.int8, scale=3, shift=4, output_zp=-5, clamp=(-100, 90)),
+    dict(B=3, M=70, K=200, N=90, batch1=False), dict(B=3, M=70, K=200, N=90, batch2=False, out_dtype=np.int32),
+    dict(B=16, M=65, K=48, N=1030), dict(B=16, M=65, K=33, N=1030, **I8),  # 64 rows
+    dict(B=16, M=300, K=40, N=1300), dict(B=16, M=300, K=45, N=1301, out_dtype=np.int32),  # 128 rows
+], ids=lambda kw: "-".join(str(getattr(v, "__name__", v)) for v in kw.values()))
+def test_runtime_input2(device, kw, tmp_path):
+    wl = w.matmul_workload(**kw)
+    print("[gpu-case]", wl.name, flush=True)
+    want = oracle_eval(wl)[0]
+    got, _ = run_on_gpu(device, wl, via="device")
+    assert_bit_exact(got[0], want, wl.name)
+    device.set_event_log(str(tmp_path / "log.csv"))  # a log has its records launched one by one
+    try:
+        got, _ = run_on_gpu(device, wl, via="device")
+    finally:
+        device.set_event_log(None)
+    assert_bit_exact(got[0], want, wl.name + " record by record")

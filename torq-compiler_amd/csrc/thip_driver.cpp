@@ -29,6 +29,7 @@
 
 #include "thip_descriptor.h"
 #include "thip_kernels.h"
+#include "thip_plan.h"
 #include "thip_status.h"
 #include "thip_validate.h"
 
@@ -76,6 +77,7 @@ struct thip_executable_t {
     std::vector<std::string> kernelNames;  // per record: the kernel its launcher resolved at creation
     // thip_executable_enqueue_noalloc: where each record's scratch (a K-split workspace) sits in the static array,
     // and the program's total
+    std::vector<Step> steps;             // the launches of a dispatch, in order
     std::vector<uint64_t> scratchOffset;
     uint64_t scratchBytes = 0;
 };
@@ -483,8 +485,42 @@ static thip_status_t dumpOpOutput(thip_executable_t *e, uint32_t i, uint8_t *con
     return THIP_OK;
 }
 
-// Enqueues every kernel record of the program.  `bp` holds one device pointer per binding.
+// Launches one step: a record by its own launcher, a run of records by the kernel that does them as a whole.
+static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr) {
+    hipError_t err = hipSuccess;
+    switch (s.kind) {
+    case kStepMatmulRt: {
+        const DescOp &g = e->ops[s.first + s.count - 1];
+        MatmulRtArgs a;
+        memset(&a, 0, sizeof(a));
+        a.A = (const int8_t *)resolve(e, s.a, bp);
+        a.B = (const int8_t *)resolve(e, s.b, bp);
+        a.out = resolve(e, s.out, bp);
+        a.M = g.M; a.N = g.Nn; a.K = g.K; a.batches = s.batches;
+        a.a_stride = s.a_stride; a.b_stride = s.b_stride; a.out_stride = s.out_stride;
+        a.a_bytes = (int64_t)(s.a_stride ? s.batches : 1) * g.M * g.K;
+        a.b_bytes = (int64_t)(s.b_stride ? s.batches : 1) * g.K * g.Nn;
+        a.bias = s.bias; a.scale = s.scale; a.out_dtype = g.out_dtype;
+        a.rq = Requant{g.shift, g.output_zp, g.output_min, g.output_max, g.pre_shift, g.t0_clamp};
+        err = launchMatmulRt(a, ctx);
+        break;
+    }
+    default: return launchOp(e, s.first, bp, ctx, scratch);
+    }
+    if (err != hipSuccess) return fail(THIP_INTERNAL, "ops %u .. %u: launch failed: %s", s.first, s.first + s.count - 1, hipGetErrorString(err));
+    return THIP_OK;
+}
+
+// Enqueues every kernel of the program.  `bp` holds one device pointer per binding.  A log or a dump is told of every
+// record, so these launch the records one by one.
 static thip_status_t enqueueOps(thip_executable_t *e, uint8_t *const *bp) {
+    if (!e->device->eventLog && e->device->dumpBuffersDir.empty()) {
+        const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0};
+        for (const Step &s : e->steps) {
+            if (thip_status_t st = launchStep(e, s, bp, ctx)) return st;
+        }
+        return THIP_OK;
+    }
     for (uint32_t i = 0; i < e->header.op_count; i++) {
         // a kernel launch is what starting an NSS task is on the reference's hardware
         logEvent(e, e->invocation, (int32_t)i, "NSS_START", "BEGIN", e->kernelNames[i].c_str());
@@ -512,7 +548,7 @@ static void dropGraph(thip_executable_t *e) {
 // Enqueues one dispatch on device bindings, through the graph when there is one.
 static thip_status_t enqueueDevice(thip_executable_t *e, uint8_t *const *bp) {
     const uint32_t nb = e->header.binding_count;
-    const bool eligible = !e->graphsDisabled && e->header.op_count >= kGraphMinOps && !e->device->eventLog && e->device->dumpBuffersDir.empty();
+    const bool eligible = !e->graphsDisabled && e->steps.size() >= kGraphMinOps && !e->device->eventLog && e->device->dumpBuffersDir.empty();
     if (!eligible) return enqueueOps(e, bp);
     std::vector<uint8_t *> key(bp, bp + nb);
     if (e->graphExec && key == e->graphPtrs) {
@@ -782,6 +818,7 @@ thip_status_t thip_executable_create(thip_device_t *device, const void *blob, si
             e->kernelNames[i] = name[0] ? name : opKernelName(e->ops[i]);
         }
     }
+    e->steps = planSteps(DescriptorView{e->blob.data(), h, e->ops, e->bindings, e->temps, e->consts});
     *out_executable = e;
     return THIP_OK;
 }
@@ -887,10 +924,10 @@ thip_status_t thip_executable_enqueue_noalloc(thip_executable_t *e, const thip_d
     for (uint32_t i = 0; i < e->header.binding_count; i++) bp[i] = (uint8_t *)st->binding_ptrs[i];
     const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0};
     thip_status_t result = THIP_OK;
-    for (uint32_t i = 0; i < e->header.op_count && result == THIP_OK; i++) {
+    for (const Step &s : e->steps) {
         // the array keeps what the last call left there, whoever made it; nothing in a K-split workspace has to start
         // at zero (every slot that is read has been written by the same dispatch)
-        if (result == THIP_OK) result = launchOp(e, i, bp, ctx, scratch);
+        if (result == THIP_OK) result = launchStep(e, s, bp, ctx, scratch);
     }
     e->invocation++;
     return result;

@@ -127,6 +127,25 @@ inline bool igemmStreamFits(int64_t N, int64_t K, int32_t out_dtype) {
 }
 hipError_t launchIgemm(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ctx);
 
+// A batch of int8 matmuls whose second operand is produced at run time, [K][N] as it lies in memory; one (bias, scale) pair.
+struct MatmulRtArgs {
+    const int8_t *A;  // [M][K] per batch element
+    const int8_t *B;  // [K][N]
+    void *out;        // [M][N] of out_dtype
+    int32_t M, N, K, batches;
+    int64_t a_stride, b_stride, out_stride;  // elements between batch elements (0: shared)
+    int64_t a_bytes, b_bytes;                // of the whole tensors: no load goes past them
+    int32_t bias, scale, out_dtype;
+    Requant rq;
+};
+// Whether the kernel's 32-bit offsets reach every byte of the tensors (and a row or a tile past them), and each holds one
+// load of it.
+inline bool matmulRtFits(int64_t aBytes, int64_t bBytes, int64_t M, int64_t N, int64_t K) {
+    constexpr int64_t most = (1LL << 31) - 65536;
+    return aBytes >= 16 && bBytes >= 4 && aBytes + K + 256 <= most && bBytes + 17 * N + 256 <= most && M < most && N < most && K < most;
+}
+hipError_t launchMatmulRt(const MatmulRtArgs &a, const LaunchCtx &ctx);
+
 struct FcSkinnyArgs {
     const int8_t *x;      // [M][K]
     const int8_t *w;      // [N][K] (as given by the op)

@@ -1,0 +1,135 @@
+#include "thip_plan.h"
+
+#include <string.h>
+
+#include "thip_kernels.h"
+
+namespace thip {
+
+static size_t elemBytes(int32_t dtype) { return dtype == 1 ? 1 : dtype == 2 ? 2 : 4; }
+static bool sameRef(const DescRef &a, const DescRef &b) { return a.space == b.space && a.index == b.index && a.offset == b.offset; }
+static bool sameBuffer(const DescRef &a, const DescRef &b) { return a.space == b.space && a.index == b.index; }
+
+// How often the records name each intermediate.
+static std::vector<uint32_t> tempUses(const DescriptorView &v) {
+    std::vector<uint32_t> uses(v.header.temp_count, 0);
+    auto count = [&](const DescRef &r) {
+        if (r.space == kSpaceTemp) uses[r.index]++;
+    };
+    for (uint32_t i = 0; i < v.header.op_count; i++) {
+        const DescOp &op = v.ops[i];
+        for (const DescRef *r : {&op.in0, &op.in1, &op.weights, &op.bias, &op.scale, &op.table, &op.out}) count(*r);
+        if (op.kind == kKindDecLinear) {
+            DecLinearExt x;
+            memcpy(&x, v.blob + v.header.data_offset + v.consts[op.table.index].offset + op.table.offset, sizeof(x));
+            for (int m = 0; m < 3; m++) {
+                for (const DescRef *r : {&x.weights[m], &x.bias[m], &x.out[m]}) count(*r);
+            }
+            count(x.res);
+            count(x.add_out);
+        }
+    }
+    return uses;
+}
+
+// The value all `n` words of a constant have; false where they differ or are none.
+static bool uniformWords(const DescriptorView &v, const DescRef &r, int n, int32_t *out) {
+    if (r.space != kSpaceConst) return false;
+    const uint8_t *p = v.blob + v.header.data_offset + v.consts[r.index].offset + r.offset;
+    for (int i = 0; i < n; i++) {
+        int32_t w;
+        memcpy(&w, p + (size_t)i * 4, 4);
+        if (i == 0) *out = w;
+        else if (w != *out) return false;
+    }
+    return n > 0;
+}
+
+// Transposes of one matrix (or of one per batch element) into intermediates, and behind them the GEMMs that read these.
+static bool matchMatmulRt(const DescriptorView &v, const std::vector<uint32_t> &uses, uint32_t first, Step *s) {
+    uint32_t n = first;
+    while (n < v.header.op_count && v.ops[n].kind == kKindTranspose) n++;
+    const uint32_t matrices = n - first;
+    if (matrices == 0 || n == v.header.op_count) return false;
+    const DescOp &t0 = v.ops[first], &g0 = v.ops[n];
+    if (g0.kind != kKindIgemm || (g0.loader != kLoaderDense && g0.loader != kLoaderGather) || g0.in1.space != kSpaceNone) return false;
+    const int64_t M = g0.M, K = g0.K, N = g0.Nn;
+    // a 1 x 1 window over a [M][K] matrix: what torq_hl.matmul becomes under either loader
+    if (g0.H != 1 || g0.W != 1 || g0.OH != 1 || g0.OW != 1 || g0.KH != 1 || g0.KW != 1 || g0.PT != 0 || g0.PL != 0 || g0.N != M || g0.C != K) return false;
+    for (uint32_t i = 0; i < matrices; i++) {
+        const DescOp &t = v.ops[first + i];
+        if (t.gran == 2 || t.TB != 1 || t.TR != K || t.TS != N || t.TP != g0.Kp || t.out.space != kSpaceTemp || t.out.offset != 0) return false;
+        if (!sameBuffer(t.in0, t0.in0) || t.in0.offset != t0.in0.offset + (uint64_t)i * (uint64_t)(K * N)) return false;
+    }
+    uint32_t batches = 0;
+    while (n + batches < v.header.op_count) {
+        const DescOp &g = v.ops[n + batches];
+        if (g.kind != kKindIgemm || g.weights.space != kSpaceTemp) break;
+        if (!sameRef(g.weights, v.ops[first + (matrices == 1 ? 0 : batches < matrices ? batches : 0)].out)) break;
+        batches++;
+        if (matrices > 1 && batches == matrices) break;
+    }
+    if (batches == 0 || (matrices > 1 && batches != matrices)) return false;
+    const uint64_t aStep = batches > 1 ? v.ops[n + 1].in0.offset - g0.in0.offset : 0, outStep = (uint64_t)(M * N) * elemBytes(g0.out_dtype);
+    if (aStep != 0 && aStep != (uint64_t)(M * K)) return false;
+    for (uint32_t i = 0; i < batches; i++) {
+        const DescOp &g = v.ops[n + i];
+        if (!sameBuffer(g.in0, g0.in0) || g.in0.offset != g0.in0.offset + i * aStep || !sameBuffer(g.out, g0.out) || g.out.offset != g0.out.offset + i * outStep) return false;
+        // everything else of the records is the same (their constants hold the same words)
+        DescOp x = g, y = g0;
+        for (DescOp *o : {&x, &y}) {
+            for (DescRef *r : {&o->in0, &o->out, &o->weights, &o->bias, &o->scale, &o->table}) memset(r, 0, sizeof(*r));
+        }
+        int32_t bias, scale;
+        if (memcmp(&x, &y, sizeof(x)) != 0 || !uniformWords(v, g.bias, (int)N, &bias) || !uniformWords(v, g.scale, (int)N, &scale)) return false;
+        if (i == 0) {
+            s->bias = bias;
+            s->scale = scale;
+        } else if (bias != s->bias || scale != s->scale) {
+            return false;
+        }
+    }
+    for (uint32_t i = 0; i < matrices; i++) {
+        // written by its transpose, read by its GEMMs, and the operands are not what the step writes
+        const DescRef &t = v.ops[first + i].out;
+        if (uses[t.index] != 1 + (matrices == 1 ? batches : 1)) return false;
+        for (uint32_t j = 0; j < i; j++) {
+            if (v.ops[first + j].out.index == t.index) return false;
+        }
+    }
+    if (sameBuffer(g0.out, g0.in0) || sameBuffer(g0.out, t0.in0)) return false;
+    // a product this large is worth its transpose: the ring kernel behind it is faster per multiply-add (4096x2048x4096 48.9 us
+    // against 57; 2048x1024x2048 16.0 against 13.0)
+    if (M * N * K > (1LL << 34)) return false;
+    if (!matmulRtFits((aStep ? (int64_t)batches : 1) * M * K, (int64_t)matrices * K * N, M, N, K)) return false;
+    s->kind = kStepMatmulRt;
+    s->first = first;
+    s->count = matrices + batches;
+    s->a = g0.in0;
+    s->b = t0.in0;
+    s->out = g0.out;
+    s->batches = (int32_t)batches;
+    s->a_stride = (int64_t)aStep;
+    s->b_stride = matrices > 1 ? K * N : 0;
+    s->out_stride = M * N;
+    return true;
+}
+
+std::vector<Step> planSteps(const DescriptorView &v) {
+    const std::vector<uint32_t> uses = tempUses(v);
+    std::vector<Step> steps;
+    for (uint32_t i = 0; i < v.header.op_count;) {
+        Step s;
+        memset(&s, 0, sizeof(s));
+        if (!matchMatmulRt(v, uses, i, &s)) {
+            s.kind = kStepRecord;
+            s.first = i;
+            s.count = 1;
+        }
+        steps.push_back(s);
+        i += s.count;
+    }
+    return steps;
+}
+
+}  // namespace thip

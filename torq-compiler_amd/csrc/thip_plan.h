@@ -1,0 +1,31 @@
+// From the records of a descriptor to the launches of a dispatch: runs of records that one kernel does as a whole.
+// Host-only (no HIP calls).
+#pragma once
+
+#include <vector>
+
+#include "thip_validate.h"
+
+namespace thip {
+
+enum StepKind {
+    kStepRecord,    // one record, by its own launcher
+    kStepMatmulRt,  // a batch of int8 matmuls with a run-time input2: its transposes and its GEMMs (igemm_rt_i8)
+};
+
+struct Step {
+    StepKind kind;
+    uint32_t first, count;  // the records it stands for
+    // kStepMatmulRt: the matrices of batch element 0, elements from one batch element to the next (0: shared), and the one
+    // (bias, scale) pair
+    DescRef a, b, out;
+    int32_t batches;
+    int64_t a_stride, b_stride, out_stride;
+    int32_t bias, scale;
+};
+
+// The launches of a dispatch in order.  Every record belongs to exactly one step; a step that stands for several leaves
+// the intermediates between them unwritten, so it is only formed where no other record reads them.
+std::vector<Step> planSteps(const DescriptorView &view);
+
+}  // namespace thip
