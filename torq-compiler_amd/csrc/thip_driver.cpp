@@ -489,6 +489,25 @@ static thip_status_t dumpOpOutput(thip_executable_t *e, uint32_t i, uint8_t *con
 static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr) {
     hipError_t err = hipSuccess;
     switch (s.kind) {
+    case kStepExpandDw: {
+        const DescOp &x = e->ops[s.first], &d = e->ops[s.first + 1];
+        IrExpandDwArgs a;
+        memset(&a, 0, sizeof(a));
+        a.x = (const int8_t *)resolve(e, x.in0, bp);
+        a.wexp = (const int8_t *)resolve(e, x.weights, bp);
+        a.bias1 = (const int32_t *)resolve(e, x.bias, bp);
+        a.scale1 = (const int32_t *)resolve(e, x.scale, bp);
+        a.wdw = (const int32_t *)resolve(e, d.weights, bp);
+        a.bias2 = (const int32_t *)resolve(e, d.bias, bp);
+        a.scale2 = (const int32_t *)resolve(e, d.scale, bp);
+        a.out = (int8_t *)resolve(e, d.out, bp);
+        a.N = d.N; a.H = d.H; a.W = d.W; a.K = x.K; a.Kp = x.Kp; a.Np = x.Np; a.C = d.C;
+        a.OH = d.OH; a.OW = d.OW; a.S = d.SW; a.PT = d.PT; a.PL = d.PL; a.zp = d.input_zp;
+        a.rq1 = Requant{x.shift, x.output_zp, x.output_min, x.output_max, x.pre_shift, x.t0_clamp};
+        a.rq2 = Requant{d.shift, d.output_zp, d.output_min, d.output_max, d.pre_shift, d.t0_clamp};
+        err = launchIrExpandDw(a, ctx);
+        break;
+    }
     case kStepMatmulRt: {
         const DescOp &g = e->ops[s.first + s.count - 1];
         MatmulRtArgs a;

@@ -127,6 +127,22 @@ inline bool igemmStreamFits(int64_t N, int64_t K, int32_t out_dtype) {
 }
 hipError_t launchIgemm(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ctx);
 
+// A pointwise convolution (dense int8 [N H W][K] -> C channels) and the 3 x 3 depthwise convolution that alone reads its result.
+struct IrExpandDwArgs {
+    const int8_t *x;        // [N][H][W][K]
+    const int8_t *wexp;     // [Np][Kp], zero padded
+    const int32_t *bias1, *scale1;  // [Np]
+    const int32_t *wdw;     // [3][C] dwords, byte kw of a dword = tap kw
+    const int32_t *bias2, *scale2;  // [C]
+    int8_t *out;            // [N][OH][OW][C]
+    int32_t N, H, W, K, Kp, Np, C, OH, OW, S, PT, PL;
+    int32_t zp;             // of the depthwise op's input: what lies outside the image
+    Requant rq1, rq2;       // both with a 32-bit tail
+    int32_t images, stripRows, strips, segmentRows, segments, cellCols;  // the launcher sets these
+};
+bool irExpandDwFits(int K, int OW, int stride, int PT, int PL);
+hipError_t launchIrExpandDw(const IrExpandDwArgs &a, const LaunchCtx &ctx);
+
 // A batch of int8 matmuls whose second operand is produced at run time, [K][N] as it lies in memory; one (bias, scale) pair.
 struct MatmulRtArgs {
     const int8_t *A;  // [M][K] per batch element

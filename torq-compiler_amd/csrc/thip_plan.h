@@ -10,6 +10,7 @@ namespace thip {
 
 enum StepKind {
     kStepRecord,    // one record, by its own launcher
+    kStepExpandDw,  // a pointwise convolution and the depthwise one behind it (ir_expand_dw_i8)
     kStepMatmulRt,  // a batch of int8 matmuls with a run-time input2: its transposes and its GEMMs (igemm_rt_i8)
 };
 
