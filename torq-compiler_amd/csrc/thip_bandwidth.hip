@@ -644,6 +644,37 @@ hipError_t launchDepthwise(const DepthwiseArgs &a, const LaunchCtx &ctx) {
     }
 }
 
+// Rows of bytes to a pitch of whole 16-byte chunks, one chunk per thread.  The bytes behind a row are whatever followed it in the
+// input; only the chunks at the very end of the input are put together byte by byte.
+struct __attribute__((packed)) UnalignedChunk {
+    v4i v;
+};
+__global__ __launch_bounds__(256) void pad_rows_i8(const int8_t *in, int8_t *out, long long rows, int from, FastDiv chunks, long long bytes) {
+    const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (t >= rows * chunks.d) return;
+    const uint32_t row = fastDiv((uint32_t)t, chunks);
+    const long long off = (long long)row * from + ((uint32_t)t - row * chunks.d) * 16;
+    v4i v = {0, 0, 0, 0};
+    if (off + 16 <= bytes) {
+        v = ((const UnalignedChunk *)(in + off))->v;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            if (off + e < bytes) v[e >> 2] |= (int)((uint32_t)(uint8_t)in[off + e] << (8 * (e & 3)));
+        }
+    }
+    *(v4i *)(out + t * 16) = v;
+}
+
+hipError_t launchPadRows(const int8_t *in, int8_t *out, int64_t rows, int32_t from, int32_t to, const LaunchCtx &ctx) {
+    if (!in || !out || ((uintptr_t)out & 15) || rows <= 0 || from <= 0 || to < from || to % 16 != 0 || to - from >= 16) return hipErrorInvalidValue;
+    const long long threads = (long long)rows * (to / 16);
+    if (threads >= (1LL << 31)) return hipErrorInvalidValue;
+    THIP_ENQUEUE(ctx, "pad_rows_i8", pad_rows_i8, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, in, out, (long long)rows, from,
+                 makeFastDiv((uint32_t)(to / 16)), (long long)rows * from);
+    return hipGetLastError();
+}
+
 template <int VEC>
 __global__ __launch_bounds__(256) void maxpool_i8(MaxPoolArgs p, WorkSplit ws) {
     const int cg = p.C / VEC;

@@ -78,6 +78,7 @@ struct thip_executable_t {
     // thip_executable_enqueue_noalloc: where each record's scratch (a K-split workspace) sits in the static array,
     // and the program's total
     std::vector<Step> steps;             // the launches of a dispatch, in order
+    std::vector<uint8_t *> stepBuffers;  // two per step: operands of space kSpacePlan (null: none)
     std::vector<uint64_t> scratchOffset;
     uint64_t scratchBytes = 0;
 };
@@ -137,10 +138,14 @@ static uint8_t *resolve(const thip_executable_t *e, const DescRef &r, uint8_t *c
     }
 }
 
-// Launches record i, or (ctx.name set) only asks its launcher which kernel it takes for these operands.
-// `scratch` (or null): the static scratch array, which then stands in for the record's workspace intermediate.
-static thip_status_t launchOp(thip_executable_t *e, uint32_t i, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr) {
-    const DescOp &op = e->ops[i];
+// Launches `op`, which is record i or stands in for it, or (ctx.name set) only asks its launcher which kernel it takes for these
+// operands.  `scratch` (or null): the static scratch array, which then stands in for the record's workspace intermediate.
+// `step` (or null): the buffers of space kSpacePlan.
+static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr,
+                              uint8_t *const *step = nullptr) {
+    auto resolve = [step](const thip_executable_t *exe, const DescRef &r, uint8_t *const *bindings) {
+        return r.space == kSpacePlan ? step[r.index] + r.offset : ::resolve(exe, r, bindings);
+    };
     const Requant rq{op.shift, op.output_zp, op.output_min, op.output_max, op.pre_shift, op.t0_clamp};
     hipError_t err = hipSuccess;
     switch (op.kind) {
@@ -524,7 +529,13 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
         err = launchMatmulRt(a, ctx);
         break;
     }
-    default: return launchOp(e, s.first, bp, ctx, scratch);
+    case kStepPadded: {
+        uint8_t *const *buffers = &e->stepBuffers[2 * (size_t)(&s - e->steps.data())];
+        err = launchPadRows((const int8_t *)resolve(e, e->ops[s.first].in0, bp), (int8_t *)buffers[0], s.rows, s.from, s.to, ctx);
+        if (err == hipSuccess) return launchOp(e, s.first, s.op, bp, ctx, scratch, buffers);
+        break;
+    }
+    default: return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch);
     }
     if (err != hipSuccess) return fail(THIP_INTERNAL, "ops %u .. %u: launch failed: %s", s.first, s.first + s.count - 1, hipGetErrorString(err));
     return THIP_OK;
@@ -543,7 +554,7 @@ static thip_status_t enqueueOps(thip_executable_t *e, uint8_t *const *bp) {
     for (uint32_t i = 0; i < e->header.op_count; i++) {
         // a kernel launch is what starting an NSS task is on the reference's hardware
         logEvent(e, e->invocation, (int32_t)i, "NSS_START", "BEGIN", e->kernelNames[i].c_str());
-        if (thip_status_t s = launchOp(e, i, bp, LaunchCtx{e->stream, &e->tuning, nullptr, 0})) return s;
+        if (thip_status_t s = launchOp(e, i, e->ops[i], bp, LaunchCtx{e->stream, &e->tuning, nullptr, 0})) return s;
         logEvent(e, e->invocation, (int32_t)i, "NSS_START", "END", e->kernelNames[i].c_str());
         if (!e->device->dumpBuffersDir.empty()) {
             // buffer dumps: each record runs to its end and what it wrote is read back before the next one starts
@@ -756,6 +767,9 @@ void thip_executable_destroy(thip_executable_t *e) {
     for (uint8_t *p : e->staging) {
         if (p) (void)hipFree(p);
     }
+    for (uint8_t *p : e->stepBuffers) {
+        if (p) (void)hipFree(p);
+    }
     if (e->constData) (void)hipFree(e->constData);
     if (e->evStart) (void)hipEventDestroy(e->evStart);
     if (e->evStop) (void)hipEventDestroy(e->evStop);
@@ -833,11 +847,22 @@ thip_status_t thip_executable_create(thip_device_t *device, const void *blob, si
         for (auto &ptr : placeholder) ptr = (uint8_t *)(uintptr_t)0x1000000;
         for (uint32_t i = 0; i < h.op_count; i++) {
             char name[96] = "";
-            if (thip_status_t st = launchOp(e, i, placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name)})) return bail(st);
+            if (thip_status_t st = launchOp(e, i, e->ops[i], placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name)})) return bail(st);
             e->kernelNames[i] = name[0] ? name : opKernelName(e->ops[i]);
         }
     }
     e->steps = planSteps(DescriptorView{e->blob.data(), h, e->ops, e->bindings, e->temps, e->consts});
+    e->stepBuffers.assign(2 * e->steps.size(), nullptr);
+    for (size_t i = 0; i < e->steps.size(); i++) {
+        Step &step = e->steps[i];
+        if (step.kind != kStepPadded) continue;
+        uint8_t **buffers = &e->stepBuffers[2 * i];
+        err = hipMalloc((void **)&buffers[0], (size_t)step.rows * step.to);
+        if (err == hipSuccess) err = hipMalloc((void **)&buffers[1], step.constants.size());
+        if (err == hipSuccess) err = hipMemcpy(buffers[1], step.constants.data(), step.constants.size(), hipMemcpyHostToDevice);
+        if (err != hipSuccess) return bail(hipFail(err, "allocating a step's operands"));
+        std::vector<uint8_t>().swap(step.constants);
+    }
     *out_executable = e;
     return THIP_OK;
 }

@@ -143,6 +143,9 @@ struct IrExpandDwArgs {
 bool irExpandDwFits(int K, int OW, int stride, int PT, int PL);
 hipError_t launchIrExpandDw(const IrExpandDwArgs &a, const LaunchCtx &ctx);
 
+// Rows of `from` bytes copied to rows of `to` bytes, to a multiple of 16 and at least `from`; what lies between is unspecified.
+hipError_t launchPadRows(const int8_t *in, int8_t *out, int64_t rows, int32_t from, int32_t to, const LaunchCtx &ctx);
+
 // A batch of int8 matmuls whose second operand is produced at run time, [K][N] as it lies in memory; one (bias, scale) pair.
 struct MatmulRtArgs {
     const int8_t *A;  // [M][K] per batch element

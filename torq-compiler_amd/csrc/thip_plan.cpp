@@ -2,10 +2,12 @@
 
 #include <string.h>
 
+#include "../../include/thip.h"
 #include "thip_kernels.h"
 
 namespace thip {
 
+static int64_t roundUp(int64_t v, int64_t to) { return (v + to - 1) / to * to; }
 static size_t elemBytes(int32_t dtype) { return dtype == 1 ? 1 : dtype == 2 ? 2 : 4; }
 static bool sameRef(const DescRef &a, const DescRef &b) { return a.space == b.space && a.index == b.index && a.offset == b.offset; }
 static bool sameBuffer(const DescRef &a, const DescRef &b) { return a.space == b.space && a.index == b.index; }
@@ -138,13 +140,64 @@ static bool matchExpandDw(const DescriptorView &v, const std::vector<uint32_t> &
     return true;
 }
 
+// A convolution, fully_connected or matmul over a channel count that is no multiple of 16.  Its own kernel gathers the
+// operand in the pieces that divide the channels, down to single bytes (1429 rows of K = 1333: 65 us); with every row
+// padded to whole chunks the kernels of aligned operands take it (one copy of the input, 2-5 us, and 4-5 us), the packed
+// weights spread to match, with zeros against the padding.
+static bool matchPadded(const DescriptorView &v, uint32_t first, Step *s) {
+    const DescOp &g = v.ops[first];
+    if (g.kind != kKindIgemm || g.loader != kLoaderGather || g.in1.space != kSpaceNone || g.weights.space != kSpaceConst || g.C % 16 == 0) return false;
+    const bool pointwise = g.KH == 1 && g.KW == 1 && g.SH == 1 && g.SW == 1 && g.PT == 0 && g.PL == 0 && g.OH == g.H && g.OW == g.W;
+    const int64_t C = g.C, Cp = roundUp(C, 16), taps = (int64_t)g.KH * g.KW, rows = (int64_t)g.N * g.H * g.W, K = taps * Cp, N = g.Nn;
+    if (g.K != taps * C || g.Kp < g.K || g.PT < 0 || g.PL < 0 || rows * Cp >= (1LL << 31) || K >= (1LL << 31)) return false;
+    DescOp op = g;
+    op.C = (int32_t)Cp;
+    op.K = (int32_t)K;
+    op.gran = 16;
+    int64_t Kp = Cp, Np = N;
+    if (pointwise && g.M <= kFcSkinnyMaxRows) {
+        op.kind = kKindFcSkinny;
+    } else {
+        uint32_t variant;
+        op.loader = pointwise ? kLoaderDense : kLoaderWindow;
+        if (thip_gemm_tile_choice((int32_t)op.loader, g.M, N, K, Cp, g.out_dtype, 0, &variant, nullptr, 0) != THIP_OK) return false;
+        const IgemmTile &t = igemmTile(variant);
+        Kp = roundUp(K, t.bk);
+        Np = roundUp(N, t.bn);
+        op.variant = variant;
+    }
+    // the (bias, scale) arrays were padded for the record's own tile
+    for (const DescRef *r : {&g.bias, &g.scale}) {
+        if (r->space != kSpaceConst || v.consts[r->index].size - r->offset < (uint64_t)Np * 4) return false;
+    }
+    op.Kp = (int32_t)Kp;
+    op.Np = (int32_t)Np;
+    const uint64_t weightBytes = (uint64_t)roundUp(Np * Kp, 256);
+    s->constants.assign(weightBytes + 128, 0);
+    const uint8_t *w = v.blob + v.header.data_offset + v.consts[g.weights.index].offset + g.weights.offset;
+    for (int64_t n = 0; n < N; n++) {
+        for (int64_t tap = 0; tap < taps; tap++) memcpy(&s->constants[(size_t)(n * Kp + tap * Cp)], w + n * g.Kp + tap * C, (size_t)C);
+    }
+    memset(&s->constants[weightBytes], g.input_zp, 128);  // what a tap outside the image reads
+    op.in0 = DescRef{kSpacePlan, 0, 0};
+    op.weights = DescRef{kSpacePlan, 1, 0};
+    op.table = op.kind == kKindIgemm && op.loader == kLoaderWindow ? DescRef{kSpacePlan, 1, weightBytes} : DescRef{kSpaceNone, 0, 0};
+    s->kind = kStepPadded;
+    s->first = first;
+    s->count = 1;
+    s->rows = rows;
+    s->from = (int32_t)C;
+    s->to = (int32_t)Cp;
+    s->op = op;
+    return true;
+}
+
 std::vector<Step> planSteps(const DescriptorView &v) {
     const std::vector<uint32_t> uses = tempUses(v);
     std::vector<Step> steps;
     for (uint32_t i = 0; i < v.header.op_count;) {
-        Step s;
-        memset(&s, 0, sizeof(s));
-        if (!matchExpandDw(v, uses, i, &s) && !matchMatmulRt(v, uses, i, &s)) {
+        Step s{};
+        if (!matchExpandDw(v, uses, i, &s) && !matchMatmulRt(v, uses, i, &s) && !matchPadded(v, i, &s)) {
             s.kind = kStepRecord;
             s.first = i;
             s.count = 1;
