@@ -24,6 +24,10 @@ namespace thip {
 // igemmEpilogueLds<...>() bytes; myBias / myScale are the (bias, scale) of channel n0 + threadIdx.x.
 // ---------------------------------------------------------------------------
 
+struct __attribute__((packed)) UnalignedV4 {
+    v4i v;
+};
+
 template <int WTM, int NW, int BN>
 constexpr size_t igemmEpilogueLds() {
     return (size_t)NW * WTM * (32 * 4 + 16) + 2 * (size_t)BN * 4;
@@ -48,7 +52,6 @@ __device__ __forceinline__ void igemmEpilogue(v16i (&acc)[WTN / 32][WTM / 32], i
     __syncthreads();
     const long long rnd = roundTerm(p.rq.shift);
     const int hi4 = (lane >> 5) * 4;
-    const bool wide = p.out_dtype == kDtypeI8 && (p.N & 15) == 0 && (((uintptr_t)p.out) & 15) == 0;
     const WideRequant wrq = wideRequant(p.rq);
     // One 32-channel column of MFMA tiles at a time goes through the wave's own LDS slice as int32;
     // a compact loop then requantises 16 consecutive channels of one row per lane and stores them
@@ -98,13 +101,27 @@ __device__ __forceinline__ void igemmEpilogue(v16i (&acc)[WTN / 32][WTM / 32], i
                     }
                 }
                 if (m < p.M) {
-                    if (wide && nb + 15 < p.N) {
+                    // 16 results in whole vectors wherever the row has 16 more, at whatever alignment an odd N gives it (element
+                    // by element 1204 x 362 -> 2236 took 17.3 us)
+                    const size_t at = (size_t)m * p.N + nb;
+                    if (nb + 15 < p.N && p.out_dtype == kDtypeI8) {
                         v4i w;
 #pragma unroll
                         for (int c = 0; c < 4; c++) {
                             w[c] = (int)packBytes(q[4 * c], q[4 * c + 1], q[4 * c + 2], q[4 * c + 3]);
                         }
-                        *(v4i *)((int8_t *)p.out + (size_t)m * p.N + nb) = w;
+                        ((UnalignedV4 *)((int8_t *)p.out + at))->v = w;
+                    } else if (nb + 15 < p.N && p.out_dtype == kDtypeI16) {
+#pragma unroll
+                        for (int h = 0; h < 2; h++) {
+                            v4i w;
+#pragma unroll
+                            for (int c = 0; c < 4; c++) w[c] = (int)__builtin_amdgcn_perm((uint32_t)q[8 * h + 2 * c + 1], (uint32_t)q[8 * h + 2 * c], 0x05040100u);
+                            ((UnalignedV4 *)((int16_t *)p.out + at + 8 * h))->v = w;
+                        }
+                    } else if (nb + 15 < p.N) {
+#pragma unroll
+                        for (int c = 0; c < 4; c++) ((UnalignedV4 *)((int32_t *)p.out + at + 4 * c))->v = v4i{q[4 * c], q[4 * c + 1], q[4 * c + 2], q[4 * c + 3]};
                     } else {
 #pragma unroll
                         for (int e = 0; e < 16; e++) {
@@ -236,9 +253,6 @@ __device__ __forceinline__ v4i gatherChunk(const int8_t *__restrict__ A,
 }
 
 // One window row of a few-channel convolution: 16 bytes starting at pixel (iy, ix0), channel 0.
-struct __attribute__((packed)) UnalignedV4 {
-    v4i v;
-};
 __device__ __forceinline__ v4i gatherRun(const int8_t *__restrict__ A, uint32_t entry, int iy0, int ix0, size_t base,
                                          int H, int W, int C, uint32_t zpb, long long aBytes) {
     if (entry & kKEntryInvalid) return v4i{0, 0, 0, 0};
