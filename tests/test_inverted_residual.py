@@ -8,26 +8,28 @@ from torq_compiler_amd import Program, workloads as w
 pytestmark = pytest.mark.gpu
 
 
-def block(N, H, W, C, E, stride, pad=(1, 1, 1, 1), shift=None, seed=1060):
-    """widen (pointwise) -> depthwise 3x3, the wide image an intermediate; `shift`: a literal requant range for both (results
+def block(N, H, W, C, E, stride, pad=(1, 1, 1, 1), shift=None, first=None, seed=1060):
+    """widen (pointwise, or `first` = (window, stride, pad) over few channels) -> depthwise 3x3, the wide image an intermediate; `shift`: a literal requant range for both (results
     saturate, the general 32-bit tail) instead of one that spreads them."""
     rng = np.random.default_rng(seed)
     x = rng.integers(-128, 128, size=(N, H, W, C)).astype(np.int8)
     layers = []
-    for op, shape, fan, zp, zout in (("conv2d", (E, C, 1, 1), C, -3, -120), ("depthwise_conv2d", (E, 1, 3, 3), 9, -120, 7)):
+    k, cs, cpad = first or (1, 1, (0, 0, 0, 0))
+    for op, shape, fan, zp, zout in (("conv2d", (E, C, k, k), C * k * k, -3, -120), ("depthwise_conv2d", (E, 1, 3, 3), 9, -120, 7)):
         wt = rng.integers(-127, 128, size=shape).astype(np.int8)
         mult, sh = w.quantize_multiplier(60 / (np.sqrt(fan) * 5400) * rng.uniform(0.8, 1.2, E))
         if shift is not None:
             sh = np.full(E, shift, dtype=np.int8)
         sb, sf = w.derive_scale_bias(mult, sh, rng.integers(-4000, 4000, E), wt, zp)
         attrs = dict(input_zp=zp, output_zp=zout, output_min=-120 if op == "conv2d" else -128, output_max=127, shift_factor=sf)
-        attrs.update(pad=(0, 0, 0, 0), stride=(1, 1)) if op == "conv2d" else attrs.update(pad=pad, stride=(stride, stride))
+        attrs.update(pad=cpad, stride=(cs, cs)) if op == "conv2d" else attrs.update(pad=pad, stride=(stride, stride))
         layers.append(w.Layer(op, [len(layers)], attrs, wt, sb))
+    H, W = (H + cpad[2] + cpad[3] - k) // cs + 1, (W + cpad[0] + cpad[1] - k) // cs + 1
     oh, ow = (H + pad[2] + pad[3] - 3) // stride + 1, (W + pad[0] + pad[1] - 3) // stride + 1
     p = Program()
     h = p.conv2d(p.binding(0, x.shape), layers[0].weights, layers[0].scale_bias, nhwc_input=True, **layers[0].attrs)
     p.depthwise_conv2d(h, layers[1].weights, layers[1].scale_bias, nhwc_input=True, init=p.binding(1, (N, oh, ow, E)), **layers[1].attrs)
-    return w.Workload("block_%dx%dx%dx%d_e%d_s%d" % (N, H, W, C, E, stride), p, [x], [((N, oh, ow, E), np.int8)], 0, 0, dict(layers=layers, nhwc=True))
+    return w.Workload("block_%dx%dx%dx%d_k%d_e%d_s%d" % (N, H, W, C, k, E, stride), p, [x], [((N, oh, ow, E), np.int8)], 0, 0, dict(layers=layers, nhwc=True))
 
 
 @pytest.mark.parametrize("kw", [
@@ -36,6 +38,9 @@ def block(N, H, W, C, E, stride, pad=(1, 1, 1, 1), shift=None, seed=1060):
     dict(N=1, H=1, W=1, C=16, E=32, stride=1), dict(N=1, H=2, W=2, C=16, E=32, stride=2, pad=(0, 1, 0, 1)), dict(N=2, H=9, W=11, C=32, E=64, stride=1, pad=(2, 2, 2, 2)),
     dict(N=1, H=40, W=131, C=16, E=96, stride=1), dict(N=1, H=41, W=130, C=24 + 8, E=96, stride=2),   # several strips
     dict(N=130, H=5, W=9, C=48, E=272, stride=1), dict(N=131, H=9, W=5, C=48, E=272, stride=2), dict(N=200, H=7, W=7, C=32, E=192, stride=1),  # several images per workgroup
+    dict(N=2, H=31, W=30, C=3, E=32, stride=1, first=(3, 2, (0, 1, 0, 1))), dict(N=1, H=224, W=224, C=3, E=32, stride=1, first=(3, 2, (0, 1, 0, 1))),
+    dict(N=3, H=19, W=23, C=1, E=16, stride=2, first=(4, 1, (2, 1, 1, 2))), dict(N=2, H=16, W=17, C=5, E=64, stride=1, first=(3, 1, (1, 1, 1, 1))),
+    dict(N=600, H=12, W=10, C=4, E=32, stride=1, first=(2, 2, (0, 0, 0, 0))),
     dict(N=1, H=12, W=12, C=32, E=48, stride=1, shift=8), dict(N=1, H=12, W=12, C=32, E=48, stride=2, shift=32),
 ], ids=lambda kw: "x".join(str(v) for v in kw.values()))
 def test_expand_depthwise(device, kw, tmp_path):

@@ -646,9 +646,6 @@ hipError_t launchDepthwise(const DepthwiseArgs &a, const LaunchCtx &ctx) {
 
 // Rows of bytes to a pitch of whole 16-byte chunks, one chunk per thread.  The bytes behind a row are whatever followed it in the
 // input; only the chunks at the very end of the input are put together byte by byte.
-struct __attribute__((packed)) UnalignedChunk {
-    v4i v;
-};
 __global__ __launch_bounds__(256) void pad_rows_i8(const int8_t *in, int8_t *out, long long rows, int from, FastDiv chunks, long long bytes) {
     const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
     if (t >= rows * chunks.d) return;
@@ -656,7 +653,7 @@ __global__ __launch_bounds__(256) void pad_rows_i8(const int8_t *in, int8_t *out
     const long long off = (long long)row * from + ((uint32_t)t - row * chunks.d) * 16;
     v4i v = {0, 0, 0, 0};
     if (off + 16 <= bytes) {
-        v = ((const UnalignedChunk *)(in + off))->v;
+        v = ((const UnalignedV4 *)(in + off))->v;
     } else {
 #pragma unroll
         for (int e = 0; e < 16; e++) {

@@ -510,6 +510,11 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
         a.OH = d.OH; a.OW = d.OW; a.S = d.SW; a.PT = d.PT; a.PL = d.PL; a.zp = d.input_zp;
         a.rq1 = Requant{x.shift, x.output_zp, x.output_min, x.output_max, x.pre_shift, x.t0_clamp};
         a.rq2 = Requant{d.shift, d.output_zp, d.output_min, d.output_max, d.pre_shift, d.t0_clamp};
+        if (x.loader == kLoaderRuns) {
+            a.CKH = x.KH; a.CS = x.SH; a.CPT = x.PT; a.CPL = x.PL; a.IH = x.H; a.IW = x.W; a.IC = x.C;
+            a.runBytes = x.KW * x.C; a.czp = x.input_zp;
+            a.xBytes = (int64_t)x.N * x.H * x.W * x.C;
+        }
         err = launchIrExpandDw(a, ctx);
         break;
     }

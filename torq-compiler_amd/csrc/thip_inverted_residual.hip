@@ -26,6 +26,8 @@ static inline int irCellColumns(int OW, int S) { return S == 1 ? 2 * ((OW + 1) /
 // them at a time straight from memory in MFMA operand layout (K <= 192: at most six loads per lane, prefetched one tile ahead), the
 // 32 channels' weights stay in registers, and the requantised bytes go to LDS as cells [row][column][32 channels]. Cells outside the
 // image hold the depthwise op's zero point.
+// RUNS: a convolution over few channels instead (the first layer of an image network): K is one 16-byte run per window row (see
+// gatherRun), and the pixels are gathered from the image.
 // Phase 2, the depthwise convolution: a thread owns four channels of two output columns (one at stride 2) and walks down rows:
 // per input row three to four dwords from LDS, a byte transpose so that a dword holds one channel at neighbouring
 // columns, and one v_dot4_i32_i8 per window row, channel and output. No address clamping and no padding selects are left in the loop.
@@ -37,8 +39,8 @@ static inline int irCellColumns(int OW, int S) { return S == 1 ? 2 * ((OW + 1) /
 //   batch 32   112x112x16 -> 96 stride 2 30.9 / 18.5, 56x56x32 -> 144 24.2 / 15.9, 14x14x96 -> 576 10.0 / 8.0
 //   batch 1    56x56x32 -> 144 6.8 / 4.8, 14x14x96 -> 576 6.7 / 3.8, 7x7x160 -> 960 6.8 / 4.1
 // ---------------------------------------------------------------------------
-template <int KS, int S>
-__global__ __launch_bounds__(256, 4) void ir_expand_dw_i8(IrExpandDwArgs p, FastDiv divW, FastDiv divH, FastDiv divCols, FastDiv divSegments) {
+template <int KS, int S, bool RUNS>
+__global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpandDwArgs p, FastDiv divW, FastDiv divH, FastDiv divCols, FastDiv divSegments) {
     extern __shared__ __attribute__((aligned(16))) int8_t cells[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // channel chunks of a strip are neighbours on one XCD: they read the same pixels and write pieces of the same lines
@@ -80,7 +82,7 @@ __global__ __launch_bounds__(256, 4) void ir_expand_dw_i8(IrExpandDwArgs p, Fast
             }
         }
     }
-    const int8_t *x = p.x + ((size_t)n * p.H + iyLo) * p.W * p.K;
+    const int8_t *x = RUNS ? p.x : p.x + ((size_t)n * p.H + iyLo) * p.W * p.K;
     // bytes of K a lane has no chunk for meet zero weights: it re-reads its first chunk of the pixel
     int kOff[KS];
 #pragma unroll
@@ -89,9 +91,21 @@ __global__ __launch_bounds__(256, 4) void ir_expand_dw_i8(IrExpandDwArgs p, Fast
     auto loadTile = [&](int t, v4i(&a)[KS]) {
         int m = t * 32 + fr;
         m = m < pixels ? m : pixels - 1;
-        const int8_t *src = x + (uint32_t)(m * p.K);
+        if constexpr (RUNS) {
+            const int r = (int)fastDiv((uint32_t)m, divW), c = m - r * p.W;
+            const int image = p.images > 1 ? (int)fastDiv((uint32_t)r, divH) : 0;
+            const int iy = (r - image * p.H + iyLo) * p.CS - p.CPT, ix = c * p.CS - p.CPL;
+            const size_t base = (size_t)(n + image) * p.IH * p.IW * p.IC;
 #pragma unroll
-        for (int s = 0; s < KS; s++) a[s] = *(const v4i *)(src + kOff[s]);
+            for (int s = 0; s < KS; s++) {
+                const int kh = 2 * s + half;
+                a[s] = gatherRun(x, kh < p.CKH ? ((uint32_t)kh << 24) | (uint32_t)p.runBytes : kKEntryInvalid, iy, ix, base, p.IH, p.IW, p.IC, (uint32_t)(p.czp & 0xff), p.xBytes);
+            }
+        } else {
+            const int8_t *src = x + (uint32_t)(m * p.K);
+#pragma unroll
+            for (int s = 0; s < KS; s++) a[s] = *(const v4i *)(src + kOff[s]);
+        }
     };
     v4i a0[KS], a1[KS];
     loadTile(wave, a0);
@@ -233,22 +247,23 @@ static size_t irLds(int images, int stripRows, int S, int cellCols) {
 }
 constexpr size_t kIrMaxLds = 64 * 1024;
 
-bool irExpandDwFits(int K, int OW, int stride, int PT, int PL) {
+bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL) {
     // a window of three rows with at most two above the image reaches into it
-    return PT >= 0 && PT <= 2 && PL >= 0 && PL <= 2 && K > 0 && K % 16 == 0 && K <= 192 && (stride == 1 || stride == 2) && irLds(1, 1, stride, irCellColumns(OW, stride)) <= kIrMaxLds;
+    return PT >= 0 && PT <= 2 && PL >= 0 && PL <= 2 && (runRows > 0 ? runRows <= 4 : K > 0 && K % 16 == 0 && K <= 192) && (stride == 1 || stride == 2) && irLds(1, 1, stride, irCellColumns(OW, stride)) <= kIrMaxLds;
 }
 
-template <int KS, int S>
+template <int KS, int S, bool RUNS = false>
 static hipError_t launchIr(const IrExpandDwArgs &a, const LaunchCtx &ctx) {
     const long long blocks = (long long)((a.N + a.images - 1) / a.images) * a.strips * ((a.C + kIrChunk - 1) / kIrChunk);
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    THIP_ENQUEUE(ctx, kernelLabel("ir_expand_dw_i8", {KS, S}), (ir_expand_dw_i8<KS, S>), dim3((unsigned)blocks), dim3(256), irLds(a.images, a.stripRows, S, a.cellCols), a,
+    THIP_ENQUEUE(ctx, kernelLabel("ir_expand_dw_i8", {KS, S, (int)RUNS}), (ir_expand_dw_i8<KS, S, RUNS>), dim3((unsigned)blocks), dim3(256), irLds(a.images, a.stripRows, S, a.cellCols), a,
                  makeFastDiv((uint32_t)a.W), makeFastDiv((uint32_t)a.H), makeFastDiv((uint32_t)(S == 1 ? (a.OW + 1) / 2 : a.OW)), makeFastDiv((uint32_t)a.segments));
     return hipGetLastError();
 }
 
 template <int S>
 static hipError_t launchIrS(const IrExpandDwArgs &a, const LaunchCtx &ctx) {
+    if (a.CKH > 0) return a.CKH <= 2 ? launchIr<1, S, true>(a, ctx) : launchIr<2, S, true>(a, ctx);
     switch ((a.K + 31) / 32) {
     case 1: return launchIr<1, S>(a, ctx);
     case 2: return launchIr<2, S>(a, ctx);
@@ -264,9 +279,16 @@ hipError_t launchIrExpandDw(const IrExpandDwArgs &in, const LaunchCtx &ctx) {
     IrExpandDwArgs a = in;
     if (!a.x || !a.wexp || !a.bias1 || !a.scale1 || !a.wdw || !a.bias2 || !a.scale2 || !a.out) return hipErrorInvalidValue;
     if (a.N <= 0 || a.H <= 0 || a.W <= 0 || a.C <= 0 || a.C % 16 != 0 || a.OH <= 0 || a.OW <= 0) return hipErrorInvalidValue;
-    if (!irExpandDwFits(a.K, a.OW, a.S, a.PT, a.PL) || a.Kp < (a.K + 31) / 32 * 32 || a.Np < (a.C + 31) / 32 * 32) return hipErrorInvalidValue;
-    if (((uintptr_t)a.x | (uintptr_t)a.wexp | (uintptr_t)a.bias1 | (uintptr_t)a.scale1 | (uintptr_t)a.wdw | (uintptr_t)a.bias2 | (uintptr_t)a.scale2) & 15) return hipErrorInvalidValue;
-    if (((uintptr_t)a.out) & 3 || (long long)a.H * a.W * a.K >= (1LL << 31)) return hipErrorInvalidValue;
+    if (!irExpandDwFits(a.K, a.CKH, a.OW, a.S, a.PT, a.PL) || a.Kp < (a.CKH > 0 ? (a.CKH + 1) / 2 * 32 : (a.K + 31) / 32 * 32) || a.Np < (a.C + 31) / 32 * 32) return hipErrorInvalidValue;
+    if (a.CKH > 0) {
+        // the runs of every output pixel start inside the image or its padding (gatherRun checks every byte against the image)
+        if (a.IH <= 0 || a.IW <= 0 || a.IC <= 0 || a.CS <= 0 || a.CPT < 0 || a.CPL < 0 || a.runBytes <= 0 || a.runBytes > 16 || a.runBytes % a.IC != 0) return hipErrorInvalidValue;
+        if (a.xBytes != (int64_t)a.N * a.IH * a.IW * a.IC || a.xBytes < 16) return hipErrorInvalidValue;
+    } else if ((uintptr_t)a.x & 15) {
+        return hipErrorInvalidValue;
+    }
+    if (((uintptr_t)a.wexp | (uintptr_t)a.bias1 | (uintptr_t)a.scale1 | (uintptr_t)a.wdw | (uintptr_t)a.bias2 | (uintptr_t)a.scale2) & 15) return hipErrorInvalidValue;
+    if (((uintptr_t)a.out) & 3 || (a.CKH == 0 && (long long)a.H * a.W * a.K >= (1LL << 31))) return hipErrorInvalidValue;
     // every window starts inside the image or its padding and none needs a row the strip does not make
     if ((a.OH - 1) * a.S - a.PT >= a.H || (a.OW - 1) * a.S - a.PL >= a.W) return hipErrorInvalidValue;
     a.cellCols = irCellColumns(a.OW, a.S);
@@ -280,7 +302,9 @@ hipError_t launchIrExpandDw(const IrExpandDwArgs &in, const LaunchCtx &ctx) {
     int strips = 1;
     auto rowsOf = [&](int s) { return (a.OH + s - 1) / s; };
     auto lds = [&](int images, int s) { return irLds(images, rowsOf(s), a.S, a.cellCols); };
-    while (rowsOf(strips) > 1 && (lds(1, strips) > ldsAim || (perStrip * strips < wgAim && rowsOf(strips) > 4))) strips++;
+    // phase 1's rounds of a workgroup's four waves: where not even every second CU has a workgroup they are the launch's time
+    auto rounds = [&](int s) { return (((rowsOf(s) - 1) * a.S + 3) * a.W + 127) / 128; };
+    while (rowsOf(strips) > 1 && (lds(1, strips) > ldsAim || (perStrip * strips < wgAim && rowsOf(strips) > 4) || (perStrip * strips < 128 && rounds(strips) > 2))) strips++;
     a.stripRows = rowsOf(strips);
     a.strips = (a.OH + a.stripRows - 1) / a.stripRows;
     a.images = 1;

@@ -127,7 +127,7 @@ inline bool igemmStreamFits(int64_t N, int64_t K, int32_t out_dtype) {
 }
 hipError_t launchIgemm(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ctx);
 
-// A pointwise convolution (dense int8 [N H W][K] -> C channels) and the 3 x 3 depthwise convolution that alone reads its result.
+// A pointwise convolution (dense int8 [N H W][K] -> C channels), or one over few channels, and the 3 x 3 depthwise convolution that alone reads its result.
 struct IrExpandDwArgs {
     const int8_t *x;        // [N][H][W][K]
     const int8_t *wexp;     // [Np][Kp], zero padded
@@ -138,9 +138,13 @@ struct IrExpandDwArgs {
     int32_t N, H, W, K, Kp, Np, C, OH, OW, S, PT, PL;
     int32_t zp;             // of the depthwise op's input: what lies outside the image
     Requant rq1, rq2;       // both with a 32-bit tail
+    // CKH > 0: x is an image [N][IH][IW][IC] and the first op a convolution of CKH window rows of runBytes each (at most 16) with
+    // stride CS, whose H x W outputs take the pixels' place; K is unused
+    int32_t CKH, CS, CPT, CPL, IH, IW, IC, runBytes, czp;
+    int64_t xBytes;
     int32_t images, stripRows, strips, segmentRows, segments, cellCols;  // the launcher sets these
 };
-bool irExpandDwFits(int K, int OW, int stride, int PT, int PL);
+bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL);
 hipError_t launchIrExpandDw(const IrExpandDwArgs &a, const LaunchCtx &ctx);
 
 // Rows of `from` bytes copied to rows of `to` bytes, to a multiple of 16 and at least `from`; what lies between is unspecified.

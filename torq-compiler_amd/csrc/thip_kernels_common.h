@@ -349,4 +349,58 @@ __device__ __forceinline__ void streamStore(void *p, T v) {
     __builtin_nontemporal_store(v, (T *)p);
 }
 
+// A load or store of 16 bytes at any alignment (global memory takes it in one instruction).
+struct __attribute__((packed)) UnalignedV4 {
+    v4i v;
+};
+
+// One window row of a few-channel convolution: 16 bytes starting at pixel (iy, ix0), channel 0.
+__device__ __forceinline__ v4i gatherRun(const int8_t *__restrict__ A, uint32_t entry, int iy0, int ix0, size_t base,
+                                         int H, int W, int C, uint32_t zpb, long long aBytes) {
+    if (entry & kKEntryInvalid) return v4i{0, 0, 0, 0};
+    const int kh = (int)((entry >> 24) & 0x7f), len = (int)(entry & 0xffff);
+    const int iy = iy0 + kh;
+    const bool rowIn = (unsigned)iy < (unsigned)H;
+    const long long off = (long long)base + ((long long)iy * W + ix0) * C;
+    const uint32_t zp4 = zpb * 0x01010101u;
+    if (!rowIn) return v4i{(int)zp4, (int)zp4, (int)zp4, (int)zp4};  // bytes past the run meet zero weights
+    if (off >= 0 && off + 16 <= aBytes) {
+        v4i v = ((const UnalignedV4 *)(A + off))->v;
+        // bytes [lo, hi) of the run lie inside the image row; the others are padding
+        const int lo = ix0 < 0 ? (-ix0 * C < len ? -ix0 * C : len) : 0;
+        const int room = (W - ix0) * C;
+        const int hi = room < len ? (room > 0 ? room : 0) : len;
+        if (lo == 0 && hi == len) return v;
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+            const int a = lo - 4 * d, b = hi - 4 * d;
+            const uint32_t below = a <= 0 ? 0u : a >= 4 ? 0xffffffffu : (1u << (8 * a)) - 1u;
+            const uint32_t upto = b <= 0 ? 0u : b >= 4 ? 0xffffffffu : (1u << (8 * b)) - 1u;
+            const uint32_t m = upto & ~below;
+            v[d] = (int)(((uint32_t)v[d] & m) | (zp4 & ~m));
+        }
+        return v;
+    }
+    // window row touches the padding (or the last bytes of the tensor): byte by byte
+    union {
+        v4i v;
+        uint8_t b[16];
+    } u;
+    int kw = 0, ci = 0;
+#pragma unroll
+    for (int b = 0; b < 16; b++) {
+        uint8_t x = 0;
+        if (b < len) {
+            const int ix = ix0 + kw;
+            x = (rowIn && (unsigned)ix < (unsigned)W) ? (uint8_t)A[off + b] : (uint8_t)zpb;
+            if (++ci == C) {
+                ci = 0;
+                kw++;
+            }
+        }
+        u.b[b] = x;
+    }
+    return u.v;
+}
+
 }  // namespace thip

@@ -4,9 +4,6 @@
 
 namespace thip {
 
-struct __attribute__((packed)) UnalignedChunk {
-    v4i v;
-};
 struct __attribute__((packed)) UnalignedWord {
     uint32_t v;
 };
@@ -79,7 +76,7 @@ __global__ __launch_bounds__(256, 2) void igemm_rt_i8(MatmulRtArgs p) {
 #pragma unroll
         for (int i = 0; i < LA; i++) {
             const int off = aOff[i] + kt * 128;
-            ra[i] = ((const UnalignedChunk *)(p.A + (uint32_t)(off < aLast ? off : aLast)))->v;
+            ra[i] = ((const UnalignedV4 *)(p.A + (uint32_t)(off < aLast ? off : aLast)))->v;
         }
         const int k0 = kt * 128 + bc * 16;
         int off = bBase + (k0 < p.K ? k0 : p.K) * p.N;
@@ -218,7 +215,7 @@ __global__ __launch_bounds__(256, 2) void igemm_rt_i8(MatmulRtArgs p) {
                     if (n >= p.N) continue;
                     int8_t *dst = out + ((size_t)m * p.N + n) * ELEM;
                     if (n + PER <= p.N) {
-                        ((UnalignedChunk *)dst)->v = w[s];
+                        ((UnalignedV4 *)dst)->v = w[s];
                     } else {
 #pragma unroll
                         for (int e = 0; e < PER; e++) {

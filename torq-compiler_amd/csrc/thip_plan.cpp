@@ -120,18 +120,20 @@ static bool matchMatmulRt(const DescriptorView &v, const std::vector<uint32_t> &
 // Whether the requant of a record has a tail of 32-bit arithmetic (see WideRequant).
 static bool narrowRequant(const DescOp &op) { return op.shift == 32 || op.shift + op.pre_shift >= 33; }
 
-// A pointwise convolution whose only reader is the 3 x 3 depthwise convolution right behind it.
+// A pointwise convolution, or one over few channels, whose only reader is the 3 x 3 depthwise convolution right behind it.
 static bool matchExpandDw(const DescriptorView &v, const std::vector<uint32_t> &uses, uint32_t first, Step *s) {
     if (first + 1 >= v.header.op_count) return false;
     const DescOp &e = v.ops[first], &d = v.ops[first + 1];
-    if (e.kind != kKindIgemm || e.loader != kLoaderDense || e.in1.space != kSpaceNone || e.out_dtype != 1 || e.KH != 1 || e.KW != 1) return false;
+    const bool runs = e.loader == kLoaderRuns;
+    if (e.kind != kKindIgemm || (!runs && (e.loader != kLoaderDense || e.KH != 1 || e.KW != 1)) || e.in1.space != kSpaceNone || e.out_dtype != 1) return false;
+    if (runs && (e.SH != e.SW || e.OH != d.H || e.OW != d.W || e.N != d.N || (int64_t)e.N * e.H * e.W * e.C < 16)) return false;
     if (d.kind != kKindDepthwise || d.variant != kDepthwiseDot4Rows || d.KH != 3 || d.KW != 3 || d.SH != d.SW) return false;
     if (e.out.space != kSpaceTemp || !sameRef(e.out, d.in0) || uses[e.out.index] != 2) return false;
     if (d.C != e.Nn || (int64_t)d.N * d.H * d.W != e.M || !narrowRequant(e) || !narrowRequant(d)) return false;
-    if (!irExpandDwFits(e.K, d.OW, d.SW, d.PT, d.PL) || e.Kp < (e.K + 31) / 32 * 32 || e.Np < (e.Nn + 31) / 32 * 32) return false;
+    if (!irExpandDwFits(e.K, runs ? e.KH : 0, d.OW, d.SW, d.PT, d.PL) || e.Kp < (runs ? (e.KH + 1) / 2 : (e.K + 31) / 32) * 32 || e.Np < (e.Nn + 31) / 32 * 32) return false;
     if ((int64_t)d.H * d.W * e.K >= (1LL << 31) || (d.OH - 1) * d.SH - d.PT >= d.H || (d.OW - 1) * d.SW - d.PL >= d.W) return false;
     for (const DescRef *r : {&e.in0, &e.weights, &e.bias, &e.scale, &d.weights, &d.bias, &d.scale, &d.out}) {
-        if (r->offset % 16 != 0) return false;
+        if (r->offset % 16 != 0 && !(runs && r == &e.in0)) return false;
     }
     if (sameBuffer(d.out, e.in0)) return false;
     s->kind = kStepExpandDw;
