@@ -594,10 +594,12 @@ thip_status_t thip_executable_time_rotating(thip_executable_t *executable,
 
 /* Introspection used by the harness and the tests. */
 thip_status_t thip_executable_op_count(thip_executable_t *executable, uint32_t *out_count);
-/* Name of the kernel that op `index` launches, as a profiler shows it without namespace and argument list
+/* Name of the kernel that op `index` has of its own, as a profiler shows it without namespace and argument list
  * (e.g. "igemm_dense_i8<256,256,2,2,4,1,1,0>", "depthwise3x3_strip_i8<2,2,1,3,1>").  It is settled when the
  * executable is created (from the record, the alignment of its operands and the THIP_* environment switches as
- * they are then) and does not change afterwards. */
+ * they are then) and does not change afterwards.  Dispatches that keep an event log or buffer dumps launch exactly these;
+ * the others may run neighbouring ops as one launch, pad an input for an aligned kernel or take a small op by a kernel
+ * without tiles, with the same results (THIP_PLAIN_RECORDS in the environment at creation: they do not). */
 thip_status_t thip_executable_op_kernel(thip_executable_t *executable, uint32_t index,
                                         char *name, size_t capacity);
 thip_status_t thip_executable_binding_count(thip_executable_t *executable, uint32_t *out_count);

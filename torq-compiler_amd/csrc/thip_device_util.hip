@@ -271,6 +271,9 @@ Tuning tuningFromEnvironment() {
     t.fcTile = digit("THIP_FC_TILE", -1);
     if (const char *v = getenv("THIP_DENSE_SHORT_K")) t.denseShortK = atoi(v);
     t.noK128 = flag("THIP_NO_K128");
+    for (const char *name : {"THIP_IGEMM_VARIANT", "THIP_IGEMM_DENSE_VARIANT", "THIP_WINDOW_VARIANT", "THIP_NO_WINDOW_RING", "THIP_NO_DIRECT_EPILOGUE", "THIP_PLAIN_RECORDS"}) {
+        t.plainRecords = t.plainRecords || flag(name);
+    }
     t.noFcDeep = flag("THIP_NO_FC_DEEP");
     t.noFcWide = flag("THIP_NO_FC_WIDE");
     t.maxpoolGeneric = flag("THIP_MAXPOOL_GENERIC");

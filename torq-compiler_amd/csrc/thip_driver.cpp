@@ -140,9 +140,9 @@ static uint8_t *resolve(const thip_executable_t *e, const DescRef &r, uint8_t *c
 
 // Launches `op`, which is record i or stands in for it, or (ctx.name set) only asks its launcher which kernel it takes for these
 // operands.  `scratch` (or null): the static scratch array, which then stands in for the record's workspace intermediate.
-// `step` (or null): the buffers of space kSpacePlan.
+// `step` (or null): the buffers of space kSpacePlan.  `planned`: a dispatch, which may take another kernel than the record's own.
 static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr,
-                              uint8_t *const *step = nullptr) {
+                              uint8_t *const *step = nullptr, bool planned = false) {
     auto resolve = [step](const thip_executable_t *exe, const DescRef &r, uint8_t *const *bindings) {
         return r.space == kSpacePlan ? step[r.index] + r.offset : ::resolve(exe, r, bindings);
     };
@@ -181,7 +181,7 @@ static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op
             a.add_w0 = ap.w0; a.add_w1 = ap.w1; a.add_bias = ap.bias; a.add_scale = ap.scale;
             a.arq = Requant{ap.shift, ap.output_zp, ap.output_min, ap.output_max, 0, 0};
         }
-        err = launchIgemm(a, op.variant, ctx);
+        err = planned && !e->tuning.plainRecords && igemmDirectBetter(a) ? launchIgemmDirect(a, ctx) : launchIgemm(a, op.variant, ctx);
         break;
     }
     case kKindFcSkinny: {
@@ -537,10 +537,10 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
     case kStepPadded: {
         uint8_t *const *buffers = &e->stepBuffers[2 * (size_t)(&s - e->steps.data())];
         err = launchPadRows((const int8_t *)resolve(e, e->ops[s.first].in0, bp), (int8_t *)buffers[0], s.rows, s.from, s.to, ctx);
-        if (err == hipSuccess) return launchOp(e, s.first, s.op, bp, ctx, scratch, buffers);
+        if (err == hipSuccess) return launchOp(e, s.first, s.op, bp, ctx, scratch, buffers, true);
         break;
     }
-    default: return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch);
+    default: return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch, nullptr, true);
     }
     if (err != hipSuccess) return fail(THIP_INTERNAL, "ops %u .. %u: launch failed: %s", s.first, s.first + s.count - 1, hipGetErrorString(err));
     return THIP_OK;
@@ -856,7 +856,7 @@ thip_status_t thip_executable_create(thip_device_t *device, const void *blob, si
             e->kernelNames[i] = name[0] ? name : opKernelName(e->ops[i]);
         }
     }
-    e->steps = planSteps(DescriptorView{e->blob.data(), h, e->ops, e->bindings, e->temps, e->consts});
+    e->steps = planSteps(DescriptorView{e->blob.data(), h, e->ops, e->bindings, e->temps, e->consts}, e->tuning.plainRecords);
     e->stepBuffers.assign(2 * e->steps.size(), nullptr);
     for (size_t i = 0; i < e->steps.size(); i++) {
         Step &step = e->steps[i];

@@ -41,6 +41,7 @@ struct Tuning {
     int denseShortK = 384;          // THIP_DENSE_SHORT_K: padded K up to which the 128 x 128 dense tile runs two stages deep, four blocks per CU
     bool noK128 = false;            // THIP_NO_K128: no 128-byte k-tiles chosen at launch (the emitter reads the same switch for its own choice)
     bool noFcDeep = false;          // THIP_NO_FC_DEEP
+    bool plainRecords = false;      // a switch asks for a tile or a loader by name: every record runs by its own launcher
     bool noFcWide = false;          // THIP_NO_FC_WIDE
     bool addGeneric = false;        // THIP_ADD_GENERIC: the quantised add always through the 64-bit ACT stage
     bool maxpoolGeneric = false;    // THIP_MAXPOOL_GENERIC: the any-window max pool kernel also for 2 x 2 stride 2
@@ -146,6 +147,10 @@ struct IrExpandDwArgs {
 };
 bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL);
 hipError_t launchIrExpandDw(const IrExpandDwArgs &a, const LaunchCtx &ctx);
+
+// The small records of the ring kernels (dense or window loader): whether the kernel without tiles in LDS is ahead, and its launch.
+bool igemmDirectBetter(const IgemmArgs &a);
+hipError_t launchIgemmDirect(const IgemmArgs &a, const LaunchCtx &ctx);
 
 // Rows of `from` bytes copied to rows of `to` bytes, to a multiple of 16 and at least `from`; what lies between is unspecified.
 hipError_t launchPadRows(const int8_t *in, int8_t *out, int64_t rows, int32_t from, int32_t to, const LaunchCtx &ctx);

@@ -194,12 +194,12 @@ static bool matchPadded(const DescriptorView &v, uint32_t first, Step *s) {
     return true;
 }
 
-std::vector<Step> planSteps(const DescriptorView &v) {
+std::vector<Step> planSteps(const DescriptorView &v, bool plain) {
     const std::vector<uint32_t> uses = tempUses(v);
     std::vector<Step> steps;
     for (uint32_t i = 0; i < v.header.op_count;) {
         Step s{};
-        if (!matchExpandDw(v, uses, i, &s) && !matchMatmulRt(v, uses, i, &s) && !matchPadded(v, i, &s)) {
+        if (plain || (!matchExpandDw(v, uses, i, &s) && !matchMatmulRt(v, uses, i, &s) && !matchPadded(v, i, &s))) {
             s.kind = kStepRecord;
             s.first = i;
             s.count = 1;

@@ -35,6 +35,7 @@ constexpr uint32_t kSpacePlan = 16;
 
 // The launches of a dispatch in order.  Every record belongs to exactly one step; a step that stands for several leaves
 // the intermediates between them unwritten, so it is only formed where no other record reads them.
-std::vector<Step> planSteps(const DescriptorView &view);
+// `plain`: one step per record.
+std::vector<Step> planSteps(const DescriptorView &view, bool plain);
 
 }  // namespace thip
