@@ -126,7 +126,7 @@ static bool matchExpandDw(const DescriptorView &v, const std::vector<uint32_t> &
     const DescOp &e = v.ops[first], &d = v.ops[first + 1];
     const bool runs = e.loader == kLoaderRuns;
     if (e.kind != kKindIgemm || (!runs && (e.loader != kLoaderDense || e.KH != 1 || e.KW != 1)) || e.in1.space != kSpaceNone || e.out_dtype != 1) return false;
-    if (runs && (e.SH != e.SW || e.OH != d.H || e.OW != d.W || e.N != d.N || (int64_t)e.N * e.H * e.W * e.C < 16)) return false;
+    if (runs && (e.SH != e.SW || e.OH != d.H || e.OW != d.W || e.N != d.N || (int64_t)e.N * e.H * e.W * e.C < 16 || (int64_t)e.H * e.W * e.C > (1LL << 27))) return false;
     if (d.kind != kKindDepthwise || d.variant != kDepthwiseDot4Rows || d.KH != 3 || d.KW != 3 || d.SH != d.SW) return false;
     if (e.out.space != kSpaceTemp || !sameRef(e.out, d.in0) || uses[e.out.index] != 2) return false;
     if (d.C != e.Nn || (int64_t)d.N * d.H * d.W != e.M || !narrowRequant(e) || !narrowRequant(d)) return false;
