@@ -63,3 +63,16 @@ def test_expand_depthwise_ragged_channels(device):
         wl = block(**kw)
         got, _ = run_on_gpu(device, wl, via="device")
         assert_bit_exact(got[0], oracle_network(wl), wl.name)
+
+
+@pytest.mark.parametrize("kw", [
+    dict(N=1100, H=1, W=1, C=16, E=256, stride=1), dict(N=300, H=8, W=16, C=16, E=256, stride=1), dict(N=300, H=4, W=3, C=64, E=512, stride=2),
+    dict(N=300, H=4, W=3, C=80, E=512, stride=1), dict(N=2, H=5, W=64, C=32, E=64, stride=1), dict(N=1, H=3, W=128, C=16, E=32, stride=2), dict(N=1, H=6, W=129, C=16, E=32, stride=1),
+    dict(N=700, H=5, W=7, C=3, E=96, stride=1, first=(3, 1, (1, 1, 1, 1))), dict(N=1, H=300, W=3, C=2, E=16, stride=1, first=(3, 1, (1, 1, 1, 1))),
+], ids=lambda kw: "x".join(str(v) for v in kw.values()))
+def test_expand_depthwise_walk(device, kw):
+    """A tile's 128 pixels that are whole images, whole rows, a row and a bit, less than a row; images that share a workgroup."""
+    wl = block(**kw)
+    print("[gpu-case]", wl.name, flush=True)
+    got, _ = run_on_gpu(device, wl, via="device")
+    assert_bit_exact(got[0], oracle_network(wl), wl.name)

@@ -37,6 +37,9 @@ static inline int irCellColumns(int OW, int S) { return S == 1 ? 2 * ((OW + 1) /
 //   batch 256  112x112x16 -> 96 stride 2 151 / 99, 56x56x32 -> 144 80 / 69, 28x28x32 -> 192 42 / 26, 14x14x96 -> 576 34 / 25
 //   batch 32   112x112x16 -> 96 stride 2 30.9 / 18.5, 56x56x32 -> 144 24.2 / 15.9, 14x14x96 -> 576 10.0 / 8.0
 //   batch 1    56x56x32 -> 144 6.8 / 4.8, 14x14x96 -> 576 6.7 / 3.8, 7x7x160 -> 960 6.8 / 4.1
+// and since, with pixels and cells reached by a walk instead of divisions and 32-bit offsets of the results (in a trace of the network,
+// batch 256): 224x224x3 -> 112x112x32 104.9 -> 94.9, 112x112x16 -> 96 stride 2 115.1 -> 108.6, 56x56x32 -> 144 80.0 -> 77.2. The busy
+// cycles are 90 % vector instructions there; more tiles prefetched, or strips of 26, 32 or 53 KB, change nothing.
 // ---------------------------------------------------------------------------
 template <int KS, int S, bool RUNS>
 __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpandDwArgs p, FastDiv divW, FastDiv divH, FastDiv divCols, FastDiv divSegments) {
@@ -111,10 +114,6 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
         int off[KS], iy, ix;
         runOffsets(r, c, off, &iy, &ix);
         const int row = p.IW * p.IC, at = ix * p.IC;
-        bool bad = iy < 0 || iy + p.CKH > p.IH || at < 0 || at + p.runBytes > row;
-#pragma unroll
-        for (int s = 0; s < KS; s++) bad = bad || off[s] > runHi;
-        if (__ballot(bad) == 0) return;
         const uint32_t zp4 = (uint32_t)(p.czp & 0xff) * 0x01010101u;
         // bytes [lo, hi) of a run lie inside its row
         const int lo = at < 0 ? -at : 0, room = row - at;
@@ -138,23 +137,64 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
             }
         }
     };
-    auto loadTile = [&](int t, v4i(&a)[KS]) {
-        int m = t * 32 + fr;
-        m = m < pixels ? m : pixels - 1;
-        if constexpr (RUNS) {
-            int off[KS];
-            const int r = (int)fastDiv((uint32_t)m, divW);
-            runOffsets(r, m - r * p.W, off, nullptr, nullptr);
+    // A wave's next tile lies 128 pixels on.  Where its pixels are (the row and column of the cell, the cell, the first run) is
+    // advanced by a constant and put right where a row or an image ends, without the divisions and products that say it for any pixel:
+    // the launch is bound by the vector pipes (90 % of its busy cycles), and these were some 40 of a tile's 110 instructions.
+    struct Walk {
+        int column, row, at;  // at: bytes, of the cell from `cells` or of the first run from x
+    };
+    auto walkFrom = [&](int imageStep, int rowStep, int columnStep, int first) {
+        const int m = wave * 32 + fr;
+        const int r = (int)fastDiv((uint32_t)m, divW), image = p.images > 1 ? (int)fastDiv((uint32_t)r, divH) : 0;
+        Walk k;
+        k.column = m - r * p.W;
+        k.row = r - image * p.H;
+        k.at = first + image * imageStep + k.row * rowStep + k.column * columnStep;
+        return k;
+    };
+    auto walkOn = [&](Walk &k, int imageStep, int rowStep, int columnStep) {
+        k.column += p.stepColumns;
+        k.row += p.stepRows;
+        k.at += p.stepImages * imageStep + p.stepRows * rowStep + p.stepColumns * columnStep;
+        const bool wrap = k.column >= p.W;
+        k.column -= wrap ? p.W : 0;
+        k.row += wrap ? 1 : 0;
+        k.at += wrap ? rowStep - p.W * columnStep : 0;
+        if (p.images > 1) {
+            const bool next = k.row >= p.H;
+            k.row -= next ? p.H : 0;
+            k.at += next ? imageStep - p.H * rowStep : 0;
+        }
+    };
+    const int cellRowBytes = cellCols * kIrPitch, cellImageBytes = cellRows * cellRowBytes;
+    Walk cell = walkFrom(cellImageBytes, cellRowBytes, kIrPitch, (iyLo - iyFirst) * cellRowBytes + p.PL * kIrPitch + 4 * half);
+    const int runRow = RUNS ? p.CS * p.IW * p.IC : 0, runColumn = RUNS ? p.CS * p.IC : 0;
+    Walk run{};
+    int khOff[KS];
+    if constexpr (RUNS) {
+        run = walkFrom(imageBytes, runRow, runColumn, ((iyLo * p.CS - p.CPT) * p.IW - p.CPL) * p.IC);
 #pragma unroll
-            for (int s = 0; s < KS; s++) a[s] = ((const UnalignedV4 *)(x + clampRun(off[s])))->v;
+        for (int s = 0; s < KS; s++) khOff[s] = (2 * s + half < p.CKH ? 2 * s + half : 0) * p.IW * p.IC;
+    }
+    // every run that starts inside this workgroup's images can be read as 16 bytes
+    const bool roomBehind = runHi >= images * imageBytes;
+    uint32_t next = (uint32_t)((wave * 32 + fr) * p.K);
+    const uint32_t last = (uint32_t)((pixels - 1) * p.K);
+    // the wave's next tile; past the last pixel, the last one again or (RUNS) whatever lies there
+    auto loadTile = [&](v4i(&a)[KS]) {
+        if constexpr (RUNS) {
+#pragma unroll
+            for (int s = 0; s < KS; s++) a[s] = ((const UnalignedV4 *)(x + clampRun(run.at + khOff[s])))->v;
+            walkOn(run, imageBytes, runRow, runColumn);
         } else {
-            const int8_t *src = x + (uint32_t)(m * p.K);
+            const int8_t *src = x + (next < last ? next : last);
 #pragma unroll
             for (int s = 0; s < KS; s++) a[s] = *(const v4i *)(src + kOff[s]);
+            next += 128u * (uint32_t)p.K;
         }
     };
     v4i a0[KS], a1[KS];
-    loadTile(wave, a0);
+    loadTile(a0);
     {
         const int zp4 = (int)((uint32_t)(p.zp & 0xff) * 0x01010101u);
         const int words = images * cellRows * cellCols * (kIrPitch / 4);
@@ -166,18 +206,22 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
         constexpr int kMode = decltype(tag)::value;
         auto computeTile = [&](int t, v4i(&a)[KS]) {
             const int m = t * 32 + fr;
-            int r = (int)fastDiv((uint32_t)m, divW);
-            const int column = m - r * p.W, c = column + p.PL;
             if constexpr (RUNS) {
-                // rows past the last pixel were read as the last one and are stored nowhere
-                if (m < pixels) fixRuns(r, column, a);
+                const int iy = (cell.row + iyLo) * p.CS - p.CPT, at = (cell.column * p.CS - p.CPL) * p.IC;
+                const bool bad = !roomBehind || iy < 0 || iy + p.CKH > p.IH || at < 0 || at + p.runBytes > p.IW * p.IC;
+                // rows past the last pixel are stored nowhere
+                if (__ballot(bad && m < pixels) != 0 && m < pixels) {
+                    const int r = (int)fastDiv((uint32_t)m, divW);
+                    fixRuns(r, m - r * p.W, a);
+                }
             }
             v16i acc = bias;
 #pragma unroll
             for (int s = 0; s < KS; s++) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[s], a[s], acc, 0, 0, 0);
-            if (p.images > 1) r += (int)fastDiv((uint32_t)r, divH) * (cellRows - p.H);  // the cells of an image have the padding's rows too
-            if (m >= pixels || c >= cellCols) return;
-            int8_t *dst = cells + ((r + iyLo - iyFirst) * cellCols + c) * kIrPitch + 4 * half;
+            int8_t *dst = cells + cell.at;
+            const bool inside = m < pixels && cell.column + p.PL < cellCols;
+            walkOn(cell, cellImageBytes, cellRowBytes, kIrPitch);
+            if (!inside) return;
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 int32_t v[4];
@@ -187,10 +231,10 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
             }
         };
         for (int t = wave; t < tiles; t += 8) {
-            loadTile(t + 4, a1);
+            loadTile(a1);
             computeTile(t, a0);
             if (t + 4 >= tiles) break;
-            loadTile(t + 8, a0);
+            loadTile(a0);
             computeTile(t + 4, a1);
         }
     });
@@ -215,11 +259,15 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
     const WideRequant w2 = wideRequant(p.rq2);
     const int colGroups = (p.OW + P - 1) / P, items = colGroups * p.segments * images;
     const int rowBytes = cellCols * kIrPitch;
+    int8_t *out = p.out + ((size_t)n * p.OH + oy0) * p.OW * p.C;
     withNarrowRequantMode(w2, [&](auto tag) {
         constexpr int kMode = decltype(tag)::value;
         for (int item = slot; item < items; item += 32) {
-            int seg = (int)fastDiv((uint32_t)item, divCols), image = 0;
-            const int j = item - seg * colGroups;
+            int seg = 0, image = 0, j = item;
+            if (p.segments * p.images > 1) {
+                seg = (int)fastDiv((uint32_t)item, divCols);
+                j -= seg * colGroups;
+            }
             if (p.images > 1) {
                 image = (int)fastDiv((uint32_t)seg, divSegments);
                 seg -= image * p.segments;
@@ -228,7 +276,7 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
             if (oyA >= oyB) continue;
             const int ox = j * P;
             const int8_t *src = cells + ((image * cellRows + oyA * S) * cellCols + ox * S) * kIrPitch + 4 * c4;
-            int8_t *dst = p.out + (((size_t)(n + image) * p.OH + oy0 + oyA) * p.OW + ox) * p.C + ch;
+            uint32_t dst = (uint32_t)(((image * p.OH + oyA) * p.OW + ox) * p.C + ch);
             const bool second = P == 2 && ox + 1 < p.OW;
             uint32_t ring[3][4];
             auto row = [&](uint32_t(&o)[4]) {
@@ -257,9 +305,9 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
                         v[P - 1][c] = requantT0<kMode>(acc, scale2[c], 0, p.rq2, w2);
                     }
                 }
-                *(uint32_t *)dst = packBytes(v[0][0], v[0][1], v[0][2], v[0][3]);
-                if (second) *(uint32_t *)(dst + p.C) = packBytes(v[P - 1][0], v[P - 1][1], v[P - 1][2], v[P - 1][3]);
-                dst += (size_t)p.OW * p.C;
+                *(uint32_t *)(out + dst) = packBytes(v[0][0], v[0][1], v[0][2], v[0][3]);
+                if (second) *(uint32_t *)(out + (dst + (uint32_t)p.C)) = packBytes(v[P - 1][0], v[P - 1][1], v[P - 1][2], v[P - 1][3]);
+                dst += (uint32_t)(p.OW * p.C);
             };
             if (S == 1) {
                 row(ring[0]);
@@ -344,10 +392,13 @@ hipError_t launchIrExpandDw(const IrExpandDwArgs &in, const LaunchCtx &ctx) {
     // every window starts inside the image or its padding and none needs a row the strip does not make
     if ((a.OH - 1) * a.S - a.PT >= a.H || (a.OW - 1) * a.S - a.PL >= a.W) return hipErrorInvalidValue;
     a.cellCols = irCellColumns(a.OW, a.S);
+    if ((long long)a.C > kIrMaxChannels) return hipErrorInvalidValue;
     // Four workgroups per CU (160 KB of LDS, 16 waves) overlap one another's phases: strips as high as 40 KB of cells hold
     // (56x56x32 -> 144, 256 images: 79 us at 20 KB, whose strips make more rows twice, 69 at 40, 76 at 64), lower where that
     // leaves fewer than two workgroups per CU (14x14x96 -> 576, 32 images: 8.0 us with at least 512, 9.1 with 1024), and down
     // to four rows; images that leave room share a workgroup (7x7x160 -> 960, 256 images: 37.3 us one by one, 17.3 by eight).
+    // Images that share cost no rows twice, so where the registers (K <= 64) let eight workgroups run on a CU they get 20 KB each
+    // (14x14x64 -> 384, 256 images: 23.4 -> 19.5 us; with K = 96 18.6 -> 21.0 at stride 2, with 160 18.7 -> 20.0, the other way).
     constexpr size_t ldsAim = 40 * 1024;
     constexpr long long wgAim = 512;
     const long long perStrip = (long long)a.N * ((a.C + kIrChunk - 1) / kIrChunk);
@@ -361,8 +412,13 @@ hipError_t launchIrExpandDw(const IrExpandDwArgs &in, const LaunchCtx &ctx) {
     a.strips = (a.OH + a.stripRows - 1) / a.stripRows;
     a.images = 1;
     if (a.strips == 1) {
-        while (a.images < 8 && lds(a.images + 1, 1) <= ldsAim && perStrip / (a.images + 1) >= 1024) a.images++;
+        const size_t aim = a.CKH == 0 && a.K <= 64 ? ldsAim / 2 : ldsAim;
+        while (a.images < 8 && lds(a.images + 1, 1) <= aim && perStrip / (a.images + 1) >= 1024) a.images++;
     }
+    // 128 pixels on, in images, rows and columns
+    a.stepImages = a.images > 1 ? 128 / (a.H * a.W) : 0;
+    a.stepRows = (128 - a.stepImages * a.H * a.W) / a.W;
+    a.stepColumns = (128 - a.stepImages * a.H * a.W) % a.W;
     const int P = a.S == 1 ? 2 : 1, columns = (a.OW + P - 1) / P * a.images;
     a.segments = columns >= 32 ? 1 : 32 / columns;
     if (a.segments > a.stripRows) a.segments = a.stripRows;

@@ -144,7 +144,10 @@ struct IrExpandDwArgs {
     int32_t CKH, CS, CPT, CPL, IH, IW, IC, runBytes, czp;
     int64_t xBytes;
     int32_t images, stripRows, strips, segmentRows, segments, cellCols;  // the launcher sets these
+    int32_t stepImages, stepRows, stepColumns;  // and these: 128 pixels
 };
+// A strip's results are addressed with 32 bits: its cells fit LDS, so they are fewer than 2^11 pixels.
+constexpr int kIrMaxChannels = 1 << 20;
 bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL);
 hipError_t launchIrExpandDw(const IrExpandDwArgs &a, const LaunchCtx &ctx);
 

@@ -129,7 +129,7 @@ static bool matchExpandDw(const DescriptorView &v, const std::vector<uint32_t> &
     if (runs && (e.SH != e.SW || e.OH != d.H || e.OW != d.W || e.N != d.N || (int64_t)e.N * e.H * e.W * e.C < 16 || (int64_t)e.H * e.W * e.C > (1LL << 27))) return false;
     if (d.kind != kKindDepthwise || d.variant != kDepthwiseDot4Rows || d.KH != 3 || d.KW != 3 || d.SH != d.SW) return false;
     if (e.out.space != kSpaceTemp || !sameRef(e.out, d.in0) || uses[e.out.index] != 2) return false;
-    if (d.C != e.Nn || (int64_t)d.N * d.H * d.W != e.M || !narrowRequant(e) || !narrowRequant(d)) return false;
+    if (d.C != e.Nn || d.C > kIrMaxChannels || (int64_t)d.N * d.H * d.W != e.M || !narrowRequant(e) || !narrowRequant(d)) return false;
     if (!irExpandDwFits(e.K, runs ? e.KH : 0, d.OW, d.SW, d.PT, d.PL) || e.Kp < (runs ? (e.KH + 1) / 2 : (e.K + 31) / 32) * 32 || e.Np < (e.Nn + 31) / 32 * 32) return false;
     if ((int64_t)d.H * d.W * e.K >= (1LL << 31) || (d.OH - 1) * d.SH - d.PT >= d.H || (d.OW - 1) * d.SW - d.PL >= d.W) return false;
     for (const DescRef *r : {&e.in0, &e.weights, &e.bias, &e.scale, &d.weights, &d.bias, &d.scale, &d.out}) {
