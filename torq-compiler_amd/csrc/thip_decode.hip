@@ -48,7 +48,11 @@ constexpr int kDecLdsSlot = 2048 + 128;  // a k-block's weights, scales and (roo
 // global load of a wave is an LDS-DMA load issued up front and each k-block is computed as soon as it has landed.
 // Otherwise the rows come through registers, CH k-blocks at a time, double-buffered.  QB: the slots carry block biases.
 // QC: the expansion clamps.
-template <int MR, int CH, bool XLDS, bool QB, bool QC>
+// S (XLDS only): the 16-column tile is shared out over S workgroups of CW = 16 / S columns, each an MFMA's row operand made of S
+// k-blocks of its columns: operand row c holds column c % CW of k-block c / CW and input column c holds input row c % CW of k-block
+// c / CW, so of the 16 x 16 products the S blocks on the diagonal are wanted; their sum is the result.  The lanes, loads and expansions of
+// a workgroup are as full as with one k-block, of which it has S times fewer.
+template <int MR, int CH, bool XLDS, bool QB, bool QC, int S>
 __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p) {
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
     const int lane = threadIdx.x & 63;
@@ -59,8 +63,12 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
     const int row0 = (int)blockIdx.y * p.rows_per_group;
     const int M = p.M - row0 < p.rows_per_group ? p.M - row0 : p.rows_per_group;
     const uint16_t *x = p.x + (size_t)row0 * p.K;
+    static_assert(S == 1 || (XLDS && MR == 1), "");
+    constexpr int CW = 16 / S;
+    const int cj = c / CW;  // of the S k-blocks at a time, the one this lane's column (and input row) belongs to
     // the tile of this workgroup: (matrix, 16 columns of it); a pair owns the same columns of both matrices
-    int tile = (int)blockIdx.x, seg = 0;
+    int tile = (int)blockIdx.x / S, seg = 0;
+    const int col0 = ((int)blockIdx.x % S) * CW;  // its first column of the tile
     if (!p.pair) {
         if (p.nseg > 1 && tile >= p.N[0] / 16) {
             tile -= p.N[0] / 16;
@@ -73,10 +81,11 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
     }
     const int nmat = p.pair ? 2 : 1;
     const int kblocks = p.K >> 7;  // K % 128 == 0
-    const int nkb = wave < kblocks ? (kblocks - wave + NW - 1) / NW : 0;  
-    const int maxkb = (kblocks + NW - 1) / NW;
+    const int units = (kblocks + S - 1) / S;  // S k-blocks each
+    const int nkb = wave < units ? (units - wave + NW - 1) / NW : 0;
+    const int maxkb = (units + NW - 1) / NW;
     const int slotBytes = kDecSlotBytes + (QB ? 64 : 0);
-    const int xRowBytes = XLDS ? M * 256 : 0;  // a k-block of the input rows in LDS
+    const int xRowBytes = XLDS ? M * S * 256 : 0;  // a unit of the input rows in LDS
     const unsigned regionBytes = (unsigned)maxkb * (unsigned)(xRowBytes + nmat * kDecLdsSlot);
     int8_t *region = smem + (size_t)wave * regionBytes;
     int8_t *slots = region + (size_t)maxkb * xRowBytes;
@@ -92,18 +101,34 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
         // lane l brings 16 bytes of row l >> 4: a k-block of one row is 16 lanes x 16 bytes
         for (int i = 0; i < nkb; i++) {
             const int kb = wave + NW * i;
-            if (lane < 16 * M) dmaLoad16(x + (size_t)(lane >> 4) * p.K + kb * 128 + (lane & 15) * 8, regionLds + (unsigned)(i * xRowBytes));
+            if constexpr (S == 1) {
+                if (lane < 16 * M) dmaLoad16(x + (size_t)(lane >> 4) * p.K + kb * 128 + (lane & 15) * 8, regionLds + (unsigned)(i * xRowBytes));
+            } else {
+                // piece = (row, k-block of the unit); a k-block past the last one is read as the last (its weights expand to zero)
+                for (int q = 0; q < M * S; q += 4) {
+                    const int piece = q + (lane >> 4), row = piece / S, b = kb * S + piece % S;
+                    if (piece < M * S) dmaLoad16(x + (size_t)row * p.K + (b < kblocks ? b : kblocks - 1) * 128 + (lane & 15) * 8, regionLds + (unsigned)(i * xRowBytes + q * 256));
+                }
+            }
         }
     }
     // the wave's whole share of the weights, one burst: per k-block and matrix 2 KiB and the scales, straight into LDS
     for (int i = 0; i < ((p.ablate & 1) ? 0 : nkb); i++) {
         const int kb = wave + NW * i;
         for (int m = 0; m < nmat; m++) {
-            const int8_t *src = wsrc[m] + ((size_t)tile * kblocks + kb) * slotBytes;
             const unsigned dst = slotsLds + (unsigned)(i * nmat + m) * kDecLdsSlot;
-            dmaLoad16(src + (size_t)lane * 16, dst);
-            dmaLoad16(src + 1024 + (size_t)lane * 16, dst + 1024u);
-            if (lane < (QB ? 32 : 16)) dmaLoad4(src + 2048 + (size_t)lane * 4, dst + 2048u);
+            if constexpr (S == 1) {
+                const int8_t *src = wsrc[m] + ((size_t)tile * kblocks + kb) * slotBytes;
+                dmaLoad16(src + (size_t)lane * 16, dst);
+                dmaLoad16(src + 1024 + (size_t)lane * 16, dst + 1024u);
+                if (lane < (QB ? 32 : 16)) dmaLoad4(src + 2048 + (size_t)lane * 4, dst + 2048u);
+            } else {
+                const int b = kb * S + cj, column = col0 + c % CW;
+                const int8_t *src = wsrc[m] + ((size_t)tile * kblocks + (b < kblocks ? b : kblocks - 1)) * slotBytes;
+                dmaLoad16(src + (size_t)(g * 16 + column) * 16, dst);
+                dmaLoad16(src + 1024 + (size_t)(g * 16 + column) * 16, dst + 1024u);
+                if (lane < (QB ? 32 : 16)) dmaLoad4(src + 2048 + (size_t)(g * 16 + column) * 4, dst + 2048u);
+            }
         }
     }
     v4f acc[2][MR];
@@ -116,14 +141,23 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
     auto kblock = [&](int i, int m, const v4i (&xp)[4][MR]) {
         const int8_t *slot = slots + (size_t)(i * nmat + m) * kDecLdsSlot;
         const v4i p0 = *(const v4i *)(slot + lane * 16), p1 = *(const v4i *)(slot + 1024 + lane * 16);
-        const float sc = *(const float *)(slot + 2048 + c * 4);
-        const float bi = QB ? *(const float *)(slot + 2048 + 64 + c * 4) : 0.0f;
+        float sc = *(const float *)(slot + 2048 + c * 4);
+        float bi = QB ? *(const float *)(slot + 2048 + 64 + c * 4) : 0.0f;
+        bool beyond = false;
+        if constexpr (S > 1) {
+            beyond = (wave + NW * i) * S + cj >= kblocks;
+            if (beyond) sc = bi = 0.0f;
+        }
         const int dw[8] = {p0[0], p0[1], p0[2], p0[3], p1[0], p1[1], p1[2], p1[3]};
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             int o[4];
             expandQ8<QC>(dw[2 * j], sc, bi, p.qlo, p.qhi, &o[0], &o[1]);
             expandQ8<QC>(dw[2 * j + 1], sc, bi, p.qlo, p.qhi, &o[2], &o[3]);
+            if constexpr (QC && S > 1) {  // zero may lie outside the expansion's clamp
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[e] = beyond ? 0 : o[e];
+            }
             const v8bf wfrag = __builtin_bit_cast(v8bf, v4i{o[0], o[1], o[2], o[3]});
 #pragma unroll
             for (int mr = 0; mr < MR; mr++) {
@@ -132,12 +166,19 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
         }
     };
     if constexpr (XLDS) {
-        const int xrow = (c < M ? c : 0) * 256 + g * 16;  // lanes of rows the input does not have read row 0 (never stored)
+        // lanes of rows the input does not have read row 0 (never stored)
+        const int xrow = ((c % CW < M ? c % CW : 0) * S + cj) * 256 + g * 16;
         for (int i = 0; i < ((p.ablate & 2) ? 0 : nkb); i++) {
             waitVmcntDyn((p.ablate & 1) ? 0 : (nkb - 1 - i) * 3 * nmat);  // everything up to this k-block has landed
             v4i xp[4][MR];
 #pragma unroll
             for (int j = 0; j < 4; j++) xp[j][0] = *(const v4i *)(region + (size_t)i * xRowBytes + xrow + j * 64);
+            if constexpr (S > 1) {
+                if ((wave + NW * i) * S + cj >= kblocks) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) xp[j][0] = v4i{0, 0, 0, 0};
+                }
+            }
             kblock(i, 0, xp);
             if (nmat > 1) kblock(i, 1, xp);
         }
@@ -195,21 +236,22 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
     __syncthreads();
     if (wave >= MR) return;
     const int mr = wave;  // this wave finishes row group `wave`
-    if (c + 16 * mr >= M) return;
+    const bool mine = c + 16 * mr < M && 4 * g < CW;
+    if (S == 1 && !mine) return;  // S > 1: every lane's sums are wanted below
     const int row = row0 + c + 16 * mr;  // as the whole launch counts them
     const int s0 = p.pair ? 0 : seg;
     const int Nseg = s0 == 0 ? p.N[0] : s0 == 1 ? p.N[1] : p.N[2];
-    const int n = tile * 16 + 4 * g;
+    const int n = tile * 16 + col0 + 4 * g;
     // what the epilogue reads from memory, issued before the sums are collected
     v4f bias4[2];
 #pragma unroll
     for (int m = 0; m < 2; m++) {
         const int sm = p.pair ? m : seg;
         const float *bias = sm == 0 ? p.bias[0] : sm == 1 ? p.bias[1] : p.bias[2];
-        bias4[m] = m < nmat ? *(const v4f *)(bias + n) : v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        bias4[m] = m < nmat && mine ? *(const v4f *)(bias + n) : v4f{0.0f, 0.0f, 0.0f, 0.0f};
     }
     v2i rv = v2i{0, 0};
-    if (p.add_mode == 1) rv = *(const v2i *)(p.res + (size_t)row * Nseg + n);
+    if (p.add_mode == 1 && mine) rv = *(const v2i *)(p.res + (size_t)row * Nseg + n);
     uint16_t y[2][4];
 #pragma unroll
     for (int m = 0; m < 2; m++) {
@@ -219,6 +261,16 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
             const v4f t = ((const v4f *)(smem + (size_t)w * regionBytes))[(m * MR + mr) * 64 + lane];
             s += t;
         }
+        if constexpr (S > 1) {
+            // block j of the diagonal lies in the lanes 5 CW further on: input columns CW j .., weight rows CW j .. in lane groups CW / 4 j ..
+            v4f d = s;
+#pragma unroll
+            for (int j = 1; j < S; j++) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) d[e] += __shfl(s[e], lane + 5 * CW * j);
+            }
+            s = d;
+        }
         const int sm = p.pair ? m : seg;
         uint16_t *out = sm == 0 ? p.out[0] : sm == 1 ? p.out[1] : p.out[2];
 #pragma unroll
@@ -226,11 +278,11 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
             const float t0 = s[e] + bias4[m][e];
             y[m][e] = bf16Bits(t0 < p.lo ? p.lo : (t0 > p.hi ? p.hi : t0));
         }
-        if (out) {
+        if (out && mine) {
             *(v2i *)(out + (size_t)row * Nseg + n) = v2i{(int)((uint32_t)y[m][0] | ((uint32_t)y[m][1] << 16)), (int)((uint32_t)y[m][2] | ((uint32_t)y[m][3] << 16))};
         }
     }
-    if (p.add_mode == 0) return;
+    if (p.add_mode == 0 || !mine) return;
     uint16_t z[4];
     if (p.add_mode == 1) {
         const uint16_t r[4] = {(uint16_t)rv[0], (uint16_t)((uint32_t)rv[0] >> 16), (uint16_t)rv[1], (uint16_t)((uint32_t)rv[1] >> 16)};
@@ -245,15 +297,15 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
     *(v2i *)(p.add_out + (size_t)row * Nseg + n) = v2i{(int)((uint32_t)z[0] | ((uint32_t)z[1] << 16)), (int)((uint32_t)z[2] | ((uint32_t)z[3] << 16))};
 }
 
-template <int MR, int CH, bool XLDS, bool QB, bool QC>
+template <int MR, int CH, bool XLDS, bool QB, bool QC, int S = 1>
 static hipError_t launchDecLinearT(const DecLinearArgs &a, int tiles, size_t lds, const LaunchCtx &ctx) {
-    auto kernel = dec_linear<MR, CH, XLDS, QB, QC>;
+    auto kernel = dec_linear<MR, CH, XLDS, QB, QC, S>;
     static std::once_flag once;
     static hipError_t configured = hipSuccess;
     std::call_once(once, [&] { configured = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
     if (configured != hipSuccess) return configured;
     const int groups = (a.M + a.rows_per_group - 1) / a.rows_per_group;
-    THIP_ENQUEUE(ctx, kernelLabel("dec_linear", {MR, CH, (int)XLDS, (int)QB, (int)QC, a.pair ? 2 : a.nseg, a.add_mode}), kernel, dim3((unsigned)tiles, (unsigned)groups),
+    THIP_ENQUEUE(ctx, kernelLabel("dec_linear", {MR, CH, (int)XLDS, (int)QB, (int)QC, a.pair ? 2 : a.nseg, a.add_mode, S}), kernel, dim3((unsigned)tiles * S, (unsigned)groups),
                  dim3((unsigned)a.nwaves * 64), lds, a);
     return hipGetLastError();
 }
@@ -285,6 +337,16 @@ static int decLinearRowGroups(int M, int tiles, const Tuning *tuning) {
     return groups;
 }
 
+// Workgroups that share a 16-column tile, eight columns each (see dec_linear's S).  A K of more k-blocks than a workgroup has
+// waves is walked in rounds, on as many CUs as there are tiles: two workgroups per tile halve the rounds where that still is one per
+// CU (one row, 6912 -> 1152: 7.6 us with 72 workgroups of 16 waves, 6.35 with 144 of 14, 7.0 with 288, four columns each; 1152 ->
+// 1536 and 1024 -> 1152, one round either way, 4.2 and 4.6 us against 4.3 and 4.5; 1152 -> 2 x 6912, whose 432 tiles fill the chip,
+// 7.8 against 9.2).
+static int decLinearSplit(int K, int tiles, const Tuning *tuning) {
+    if (tuning && tuning->decSplit > 0) return tuning->decSplit;
+    return K / 128 > kDecMaxWaves && tiles * 2 <= 256 ? 2 : 1;
+}
+
 template <bool QB, bool QC>
 static hipError_t launchDecLinearQ(const DecLinearArgs &in, int tiles, const LaunchCtx &ctx) {
     DecLinearArgs a = in;
@@ -294,6 +356,13 @@ static hipError_t launchDecLinearQ(const DecLinearArgs &in, int tiles, const Lau
         // the input rows through LDS as well, with the most waves whose regions still fit
         for (int nw = a.nwaves; nw >= kDecWaves; nw--) {
             if (decLinearLds(a.K, nmat, a.M, nw) > kDecMaxLds) continue;
+            const int split = decLinearSplit(a.K, tiles, ctx.tuning);
+            if (split > 1) {  // less LDS than one workgroup per tile, which fits
+                const int units = (a.K / 128 + split - 1) / split, rounds = (units + kDecMaxWaves - 1) / kDecMaxWaves;
+                a.nwaves = (units + rounds - 1) / rounds;
+                const size_t lds = (size_t)a.nwaves * rounds * (size_t)(a.M * split * 256 + nmat * kDecLdsSlot);
+                return launchDecLinearT<1, 1, true, QB, QC, 2>(a, tiles, lds, ctx);
+            }
             a.nwaves = nw;
             return launchDecLinearT<1, 1, true, QB, QC>(a, tiles, decLinearLds(a.K, nmat, a.M, nw), ctx);
         }

@@ -45,6 +45,7 @@ struct Tuning {
     bool noFcWide = false;          // THIP_NO_FC_WIDE
     bool addGeneric = false;        // THIP_ADD_GENERIC: the quantised add always through the 64-bit ACT stage
     bool maxpoolGeneric = false;    // THIP_MAXPOOL_GENERIC: the any-window max pool kernel also for 2 x 2 stride 2
+    int decSplit = 0;               // THIP_DEC_SPLIT: workgroups per 16-column tile of a dec_linear launch of at most four rows: 1 or 2 (0: by its size)
     int decAblate = 0;              // THIP_DEC_ABLATE: parts of dec_linear left out, for timing experiments (wrong results)
     int decTargetGroups = 0;        // THIP_DEC_TARGET_WORKGROUPS: workgroups a dec_linear launch with few column tiles shares its rows out to (0: 256)
 };
