@@ -185,7 +185,10 @@ static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op
             a.add_w0 = ap.w0; a.add_w1 = ap.w1; a.add_bias = ap.bias; a.add_scale = ap.scale;
             a.arq = Requant{ap.shift, ap.output_zp, ap.output_min, ap.output_max, 0, 0};
         }
-        err = planned && !e->tuning.plainRecords && igemmDirectBetter(a) ? launchIgemmDirect(a, ctx) : launchIgemm(a, op.variant, ctx);
+        if (!planned || e->tuning.plainRecords) err = launchIgemm(a, op.variant, ctx);
+        else if (igemmDirectBetter(a)) err = launchIgemmDirect(a, ctx);
+        else if (convPatchBetter(a)) err = launchConvPatch(a, ctx);
+        else err = launchIgemm(a, op.variant, ctx);
         break;
     }
     case kKindFcSkinny: {

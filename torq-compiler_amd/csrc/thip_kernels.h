@@ -156,6 +156,10 @@ hipError_t launchIrExpandDw(const IrExpandDwArgs &a, const LaunchCtx &ctx);
 bool igemmDirectBetter(const IgemmArgs &a);
 hipError_t launchIgemmDirect(const IgemmArgs &a, const LaunchCtx &ctx);
 
+// The convolutions whose weights fit LDS beside a patch of the image: whether the kernel that keeps both there is ahead, and its launch.
+bool convPatchBetter(const IgemmArgs &a);
+hipError_t launchConvPatch(const IgemmArgs &a, const LaunchCtx &ctx);
+
 // Rows of `from` bytes copied to rows of `to` bytes, to a multiple of 16 and at least `from`; what lies between is unspecified.
 hipError_t launchPadRows(const int8_t *in, int8_t *out, int64_t rows, int32_t from, int32_t to, const LaunchCtx &ctx);
 
