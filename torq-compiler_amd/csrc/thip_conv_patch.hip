@@ -12,7 +12,7 @@ namespace thip {
 // Why: the ring kernel addresses the window in memory, so a 3x3 convolution brings every pixel from L2 into LDS nine times, and a tile
 // column of 128 brings and multiplies 128 channels where there are 96. Both go at what L2 delivers (11 TB/s for the chip).
 //
-// What is left is serial in a workgroup, one to a CU: weights and patch in (about 4 us of 56x56x96 -> 96), 54 MFMA steps, the epilogue.
+// What is left is serial in a workgroup, mostly one to a CU: weights and patch into LDS, the MFMA steps, the epilogue.
 //
 // Pixels and weight rows are padded in LDS to pitches of 16-byte units that are no multiple of four, so that the eight
 // lanes that a ds_read_b128 serves at a time hit all banks once.

@@ -139,7 +139,8 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
     };
     // A wave's next tile lies 128 pixels on.  Where its pixels are (the row and column of the cell, the cell, the first run) is
     // advanced by a constant and put right where a row or an image ends, without the divisions and products that say it for any pixel:
-    // the launch is bound by the vector pipes (90 % of its busy cycles), and these were some 40 of a tile's 110 instructions.
+    // the launch is bound by the vector pipes (90 % of its busy cycles). Vector instructions of 256 images, millions of waves': the first
+    // layer 47.4 -> 40.9, 112x112x16 -> 96 52.9 -> 49.5.
     struct Walk {
         int column, row, at;  // at: bytes, of the cell from `cells` or of the first run from x
     };
