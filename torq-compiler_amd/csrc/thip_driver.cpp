@@ -899,6 +899,13 @@ thip_status_t thip_executable_create(thip_device_t *device, const void *blob, si
         if (err != hipSuccess) return bail(hipFail(err, "allocating a step's operands"));
         std::vector<uint8_t>().swap(step.constants);
     }
+    {
+        // the launches' own kernels are configured now too (naming mode again; an error is the dispatch's to report)
+        uint8_t *placeholder[64];
+        for (auto &ptr : placeholder) ptr = (uint8_t *)(uintptr_t)0x1000000;
+        char name[96];
+        for (const Step &step : e->steps) (void)launchStep(e, step, placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name)});
+    }
     *out_executable = e;
     return THIP_OK;
 }
