@@ -1,0 +1,76 @@
+// The index arithmetic of ir_expand_dw_i8 on the host: every cell that a window reads is written once, by its own pixel, and nothing
+// else is written; the walk over the runs of a first layer names the runs of the same pixel.
+// Arguments: N H W K C OH OW S PT PL, and for a first layer CKH CS CPT CPL IH IW IC KW behind them.  Prints the images per workgroup.
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include <vector>
+
+#include "thip_inverted_residual.h"
+
+using namespace thip;
+
+static int fail(const char *what, int a, int b, int c) {
+    printf("%s (%d, %d, %d)\n", what, a, b, c);
+    return 1;
+}
+
+int main(int argc, char **argv) {
+    if (argc != 11 && argc != 19) return 2;
+    int v[18] = {0};
+    for (int i = 1; i < argc; i++) v[i - 1] = atoi(argv[i]);
+    IrExpandDwArgs p;
+    memset(&p, 0, sizeof(p));
+    static int8_t *const somewhere = (int8_t *)0x1000000;
+    p.x = p.wexp = p.out = somewhere;
+    p.bias1 = p.scale1 = p.wdw = p.bias2 = p.scale2 = (const int32_t *)somewhere;
+    p.N = v[0]; p.H = v[1]; p.W = v[2]; p.K = v[3]; p.C = v[4]; p.OH = v[5]; p.OW = v[6]; p.S = v[7]; p.PT = v[8]; p.PL = v[9];
+    p.Kp = (p.K + 63) / 64 * 64;
+    p.Np = (p.C + 63) / 64 * 64;
+    p.CKH = v[10]; p.CS = v[11]; p.CPT = v[12]; p.CPL = v[13]; p.IH = v[14]; p.IW = v[15]; p.IC = v[16];
+    p.runBytes = v[17] * p.IC;
+    p.xBytes = (int64_t)p.N * p.IH * p.IW * p.IC;
+    if (p.CKH) p.Kp = 64;
+    if (!planIrExpandDw(&p)) return fail("refused", 0, 0, 0);
+    const bool runs = p.CKH > 0;
+    const int rowBytes = p.cellCols * kIrPitch;
+    for (int n = 0; n < p.N; n += p.images) {
+        for (int strip = 0; strip < p.strips; strip++) {
+            const IrStrip s = irStrip(p, n, strip);
+            const int imageBytes = s.cellRows * rowBytes;
+            std::vector<int> writer((size_t)s.images * s.cellRows * p.cellCols, -1);  // the pixel that wrote a cell
+            for (int wave = 0; wave < 4; wave++) {
+                for (int fr = 0; fr < 32; fr++) {
+                    const int first = wave * 32 + fr, r = first / p.W, image = p.images > 1 ? r / p.H : 0;
+                    IrWalk cell = irWalkFrom(p, first, r, image, imageBytes, rowBytes, kIrPitch, (s.iyLo - s.iyFirst) * rowBytes + p.PL * kIrPitch);
+                    const int in = p.IH * p.IW * p.IC, inRow = p.CS * p.IW * p.IC, inColumn = p.CS * p.IC;
+                    IrWalk run = irWalkFrom(p, first, r, image, in, inRow, inColumn, ((s.iyLo * p.CS - p.CPT) * p.IW - p.CPL) * p.IC);
+                    for (int m = first; m < s.pixels; m += 128) {
+                        // pixel m of the strip's dense rows, which are consecutive in memory from row iyLo of the first image on
+                        const int row = m / p.W + s.iyLo, im = p.images > 1 ? row / p.H : 0, iy = row - im * p.H, ix = m % p.W;
+                        if (runs && run.at != im * in + ((iy * p.CS - p.CPT) * p.IW + ix * p.CS - p.CPL) * p.IC) return fail("the run of another pixel", n, strip, m);
+                        if (runs && (run.row + s.iyLo != iy || run.column != ix)) return fail("another pixel", n, strip, m);
+                        if (irHasCell(p, s, m, cell)) {
+                            if (cell.at < 0 || cell.at % kIrPitch != 0 || (size_t)(cell.at / kIrPitch) >= writer.size()) return fail("a write outside the cells", n, strip, m);
+                            if (writer[cell.at / kIrPitch] >= 0) return fail("a cell written twice", n, strip, m);
+                            writer[cell.at / kIrPitch] = (im * p.H + iy) * p.W + ix;
+                        }
+                        irWalkOn(p, cell, imageBytes, rowBytes, kIrPitch);
+                        irWalkOn(p, run, in, inRow, inColumn);
+                    }
+                }
+            }
+            for (int im = 0; im < s.images; im++) {
+                for (int y = 0; y < s.cellRows; y++) {
+                    for (int x = 0; x < p.cellCols; x++) {
+                        const int iy = s.iyFirst + y, ix = x - p.PL, inside = iy >= 0 && iy < p.H && ix >= 0 && ix < p.W;
+                        if (writer[((size_t)im * s.cellRows + y) * p.cellCols + x] != (inside ? (im * p.H + iy) * p.W + ix : -1)) return fail("a cell of another pixel, or of none", n + im, iy, ix);
+                    }
+                }
+            }
+        }
+    }
+    printf("%d\n", p.images);
+    return 0;
+}

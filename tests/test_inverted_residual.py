@@ -76,3 +76,16 @@ def test_expand_depthwise_walk(device, kw):
     print("[gpu-case]", wl.name, flush=True)
     got, _ = run_on_gpu(device, wl, via="device")
     assert_bit_exact(got[0], oracle_network(wl), wl.name)
+
+
+@pytest.mark.parametrize("kw", [
+    dict(N=300, H=8, W=8, C=16, E=256, stride=2, pad=(0, 0, 0, 0)), dict(N=256, H=14, W=14, C=96, E=576, stride=2, pad=(0, 0, 0, 0)), dict(N=300, H=7, W=7, C=16, E=256, stride=2, pad=(1, 1, 1, 0)),
+    dict(N=300, H=8, W=8, C=3, E=256, stride=2, pad=(0, 0, 0, 0), first=(3, 1, (1, 1, 1, 1))), dict(N=256, H=14, W=14, C=3, E=576, stride=2, pad=(0, 0, 0, 0), first=(3, 1, (1, 1, 1, 1))),
+    dict(N=300, H=7, W=7, C=3, E=256, stride=2, pad=(1, 1, 1, 0), first=(3, 1, (1, 1, 1, 1))),
+], ids=lambda kw: "x".join(str(v) for v in kw.values()))
+def test_rows_no_window_reaches(device, kw):
+    """Several images per workgroup whose last row lies below every window."""
+    wl = block(**kw)
+    print("[gpu-case]", wl.name, flush=True)
+    got, _ = run_on_gpu(device, wl, via="device")
+    assert_bit_exact(got[0], oracle_network(wl), wl.name)

@@ -1,0 +1,69 @@
+"""The index arithmetic of the fused widening + depthwise launch, on the host: the library's own plan and the kernel's own walk, over
+frames, strides, paddings and shared workgroups (tests/host/ir_cells.cpp says what is checked)."""
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+from torq_compiler_amd import runtime
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "torq-compiler_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    gxx = shutil.which("g++")
+    assert gxx, "g++ is needed for the host check"
+    exe = str(tmp_path_factory.mktemp("ir") / "ir_cells")
+    built = subprocess.run([gxx, "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + CSRC,
+                            os.path.join(ROOT, "tests", "host", "ir_cells.cpp"), runtime.LIB_PATH, "-Wl,-rpath," + os.path.dirname(runtime.LIB_PATH),
+                            "-Wl,--allow-shlib-undefined", "-o", exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert built.returncode == 0, built.stdout[-3000:]
+
+    def run(N, H, W, K, C, stride, pad, first=None):
+        """pad: (top, bottom, left, right); first: (window, stride, channels), unpadded, its image as large as its windows need.
+        -> images per workgroup"""
+        OH, OW = (H + pad[0] + pad[1] - 3) // stride + 1, (W + pad[2] + pad[3] - 3) // stride + 1
+        args = [N, H, W, K, C, OH, OW, stride, pad[0], pad[2]]
+        if first:
+            k, s, c = first
+            args += [k, s, 0, 0, (H - 1) * s + k, (W - 1) * s + k, c, k]
+        done = subprocess.run([exe] + [str(a) for a in args], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+        assert done.returncode == 0, (args, done.stdout)
+        return int(done.stdout)
+
+    return run
+
+
+# windows that stop short of the image's last row, in workgroups of several images
+SHORT = [((300, 8, 8, 16, 256, 2, (0, 0, 0, 0)), 2), ((256, 14, 14, 96, 576, 2, (0, 0, 0, 0)), 4), ((300, 7, 7, 16, 256, 2, (1, 0, 1, 1)), 2)]
+
+
+@pytest.mark.parametrize("runs", [False, True])
+@pytest.mark.parametrize("case,images", SHORT, ids=["8x8_s2", "14x14_s2", "7x7_s2_top"])
+def test_rows_no_window_reaches(check, case, images, runs):
+    shared = check(*case, first=(3, 1, 3) if runs else None)
+    assert shared >= images, "the case is about images that share a workgroup"
+
+
+def test_drawn_geometries(check):
+    rng = np.random.default_rng(11)
+    shared = 0
+    for _ in range(200):
+        H, W = int(rng.integers(1, 24)), int(rng.integers(1, 40))
+        pad = tuple(int(v) for v in rng.integers(0, 3, size=4))
+        stride = int(rng.integers(1, 3))
+        if H + pad[0] + pad[1] < 3 or W + pad[2] + pad[3] < 3:
+            continue
+        # what the planner asks too: no window starts behind the image
+        if (H + pad[0] + pad[1] - 3) // stride * stride - pad[0] >= H or (W + pad[2] + pad[3] - 3) // stride * stride - pad[2] >= W:
+            continue
+        K = int(rng.choice([16, 48, 64, 160]))
+        first = (int(rng.integers(1, 5)), int(rng.integers(1, 3)), int(rng.integers(1, 5))) if rng.integers(0, 3) == 0 else None
+        if first and first[0] * first[2] > 16:
+            continue
+        shared += check(int(rng.choice([1, 40, 300, 1100])), H, W, K, int(rng.choice([16, 80, 256, 576])), stride, pad, first) > 1
+    assert shared >= 20

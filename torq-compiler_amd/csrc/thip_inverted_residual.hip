@@ -1,11 +1,9 @@
 // gfx950 kernel of the front half of an inverted-residual block: the pointwise convolution that widens the channels and the
 // 3 x 3 depthwise convolution behind it as one launch, the widened image never leaving LDS.
+#include "thip_inverted_residual.h"
 #include "thip_kernels_common.h"
 
 namespace thip {
-
-constexpr int kIrChunk = 32;           // channels of a workgroup
-constexpr int kIrPitch = kIrChunk + 4;  // bytes of a cell in LDS: the padding spreads neighbouring cells over the banks
 
 // The requant tails that need 32-bit arithmetic only (withRequantMode without its 64-bit one; the planner keeps such records
 // apart).
@@ -58,12 +56,10 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
         strip = rest - n * p.strips;
     }
     n *= p.images;
-    const int images = p.N - n < p.images ? p.N - n : p.images;  // more than one only where a strip is a whole image
     const int ch0 = chunk * kIrChunk;
-    const int oy0 = strip * p.stripRows, rows = p.OH - oy0 < p.stripRows ? p.OH - oy0 : p.stripRows;
-    const int iyFirst = oy0 * S - p.PT, cellRows = (rows - 1) * S + 3, cellCols = p.cellCols;
-    const int iyLo = iyFirst < 0 ? 0 : iyFirst, iyHi = iyFirst + cellRows < p.H ? iyFirst + cellRows : p.H;
-    const int pixels = images * (iyHi - iyLo) * p.W;
+    const IrStrip part = irStrip(p, n, strip);
+    const int images = part.images, oy0 = part.oy0, rows = part.rows, iyFirst = part.iyFirst, iyLo = part.iyLo, cellRows = part.cellRows, pixels = part.pixels;
+    const int cellCols = p.cellCols;
 
     // ---- phase 1 ----
     const int fr = lane & 31, half = lane >> 5;
@@ -137,40 +133,16 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
             }
         }
     };
-    // A wave's next tile lies 128 pixels on.  Where its pixels are (the row and column of the cell, the cell, the first run) is
-    // advanced by a constant and put right where a row or an image ends, without the divisions and products that say it for any pixel:
-    // the launch is bound by the vector pipes (90 % of its busy cycles). Vector instructions of 256 images, millions of waves': the first
-    // layer 47.4 -> 40.9, 112x112x16 -> 96 52.9 -> 49.5.
-    struct Walk {
-        int column, row, at;  // at: bytes, of the cell from `cells` or of the first run from x
-    };
+    // the wave's first pixel, and its tiles' pixels behind it
     auto walkFrom = [&](int imageStep, int rowStep, int columnStep, int first) {
         const int m = wave * 32 + fr;
         const int r = (int)fastDiv((uint32_t)m, divW), image = p.images > 1 ? (int)fastDiv((uint32_t)r, divH) : 0;
-        Walk k;
-        k.column = m - r * p.W;
-        k.row = r - image * p.H;
-        k.at = first + image * imageStep + k.row * rowStep + k.column * columnStep;
-        return k;
-    };
-    auto walkOn = [&](Walk &k, int imageStep, int rowStep, int columnStep) {
-        k.column += p.stepColumns;
-        k.row += p.stepRows;
-        k.at += p.stepImages * imageStep + p.stepRows * rowStep + p.stepColumns * columnStep;
-        const bool wrap = k.column >= p.W;
-        k.column -= wrap ? p.W : 0;
-        k.row += wrap ? 1 : 0;
-        k.at += wrap ? rowStep - p.W * columnStep : 0;
-        if (p.images > 1) {
-            const bool next = k.row >= p.H;
-            k.row -= next ? p.H : 0;
-            k.at += next ? imageStep - p.H * rowStep : 0;
-        }
+        return irWalkFrom(p, m, r, image, imageStep, rowStep, columnStep, first);
     };
     const int cellRowBytes = cellCols * kIrPitch, cellImageBytes = cellRows * cellRowBytes;
-    Walk cell = walkFrom(cellImageBytes, cellRowBytes, kIrPitch, (iyLo - iyFirst) * cellRowBytes + p.PL * kIrPitch + 4 * half);
+    IrWalk cell = walkFrom(cellImageBytes, cellRowBytes, kIrPitch, (iyLo - iyFirst) * cellRowBytes + p.PL * kIrPitch + 4 * half);
     const int runRow = RUNS ? p.CS * p.IW * p.IC : 0, runColumn = RUNS ? p.CS * p.IC : 0;
-    Walk run{};
+    IrWalk run{};
     int khOff[KS];
     if constexpr (RUNS) {
         run = walkFrom(imageBytes, runRow, runColumn, ((iyLo * p.CS - p.CPT) * p.IW - p.CPL) * p.IC);
@@ -186,7 +158,7 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
         if constexpr (RUNS) {
 #pragma unroll
             for (int s = 0; s < KS; s++) a[s] = ((const UnalignedV4 *)(x + clampRun(run.at + khOff[s])))->v;
-            walkOn(run, imageBytes, runRow, runColumn);
+            irWalkOn(p, run, imageBytes, runRow, runColumn);
         } else {
             const int8_t *src = x + (next < last ? next : last);
 #pragma unroll
@@ -220,8 +192,8 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
 #pragma unroll
             for (int s = 0; s < KS; s++) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[s], a[s], acc, 0, 0, 0);
             int8_t *dst = cells + cell.at;
-            const bool inside = m < pixels && cell.column + p.PL < cellCols;
-            walkOn(cell, cellImageBytes, cellRowBytes, kIrPitch);
+            const bool inside = irHasCell(p, part, m, cell);
+            irWalkOn(p, cell, cellImageBytes, cellRowBytes, kIrPitch);
             if (!inside) return;
 #pragma unroll
             for (int q = 0; q < 4; q++) {
@@ -341,21 +313,19 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
     });
 }
 
-static size_t irLds(int images, int stripRows, int S, int cellCols) {
-    return (((size_t)images * ((stripRows - 1) * S + 3) * cellCols * kIrPitch) + 15) / 16 * 16;
-}
+static size_t irLds(int images, int cellRows, int cellCols) { return ((size_t)images * cellRows * cellCols * kIrPitch + 15) / 16 * 16; }
 constexpr size_t kIrMaxLds = 64 * 1024;
 
 bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL) {
     // a window of three rows with at most two above the image reaches into it
-    return PT >= 0 && PT <= 2 && PL >= 0 && PL <= 2 && (runRows > 0 ? runRows <= 4 : K > 0 && K % 16 == 0 && K <= 192) && (stride == 1 || stride == 2) && irLds(1, 1, stride, irCellColumns(OW, stride)) <= kIrMaxLds;
+    return PT >= 0 && PT <= 2 && PL >= 0 && PL <= 2 && (runRows > 0 ? runRows <= 4 : K > 0 && K % 16 == 0 && K <= 192) && (stride == 1 || stride == 2) && irLds(1, 3, irCellColumns(OW, stride)) <= kIrMaxLds;
 }
 
 template <int KS, int S, bool RUNS = false>
 static hipError_t launchIr(const IrExpandDwArgs &a, const LaunchCtx &ctx) {
     const long long blocks = (long long)((a.N + a.images - 1) / a.images) * a.strips * ((a.C + kIrChunk - 1) / kIrChunk);
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    THIP_ENQUEUE(ctx, kernelLabel("ir_expand_dw_i8", {KS, S, (int)RUNS}), (ir_expand_dw_i8<KS, S, RUNS>), dim3((unsigned)blocks), dim3(256), irLds(a.images, a.stripRows, S, a.cellCols), a,
+    THIP_ENQUEUE(ctx, kernelLabel("ir_expand_dw_i8", {KS, S, (int)RUNS}), (ir_expand_dw_i8<KS, S, RUNS>), dim3((unsigned)blocks), dim3(256), irLds(a.images, irCellRows(a, a.images, a.stripRows), a.cellCols), a,
                  makeFastDiv((uint32_t)a.W), makeFastDiv((uint32_t)a.H), makeFastDiv((uint32_t)(S == 1 ? (a.OW + 1) / 2 : a.OW)), makeFastDiv((uint32_t)a.segments));
     return hipGetLastError();
 }
@@ -374,26 +344,26 @@ static hipError_t launchIrS(const IrExpandDwArgs &a, const LaunchCtx &ctx) {
     }
 }
 
-hipError_t launchIrExpandDw(const IrExpandDwArgs &in, const LaunchCtx &ctx) {
-    IrExpandDwArgs a = in;
-    if (!a.x || !a.wexp || !a.bias1 || !a.scale1 || !a.wdw || !a.bias2 || !a.scale2 || !a.out) return hipErrorInvalidValue;
-    if (a.N <= 0 || a.H <= 0 || a.W <= 0 || a.C <= 0 || a.C % 16 != 0 || a.OH <= 0 || a.OW <= 0) return hipErrorInvalidValue;
-    if (!irExpandDwFits(a.K, a.CKH, a.OW, a.S, a.PT, a.PL) || a.Kp < (a.CKH > 0 ? (a.CKH + 1) / 2 * 32 : (a.K + 31) / 32 * 32) || a.Np < (a.C + 31) / 32 * 32) return hipErrorInvalidValue;
+bool planIrExpandDw(IrExpandDwArgs *args) {
+    IrExpandDwArgs &a = *args;
+    if (!a.x || !a.wexp || !a.bias1 || !a.scale1 || !a.wdw || !a.bias2 || !a.scale2 || !a.out) return false;
+    if (a.N <= 0 || a.H <= 0 || a.W <= 0 || a.C <= 0 || a.C % 16 != 0 || a.OH <= 0 || a.OW <= 0) return false;
+    if (!irExpandDwFits(a.K, a.CKH, a.OW, a.S, a.PT, a.PL) || a.Kp < (a.CKH > 0 ? (a.CKH + 1) / 2 * 32 : (a.K + 31) / 32 * 32) || a.Np < (a.C + 31) / 32 * 32) return false;
     if (a.CKH > 0) {
         // the runs of every output pixel start inside the image or its padding (the kernel checks every byte against the image)
-        if (a.IH <= 0 || a.IW <= 0 || a.IC <= 0 || a.CS <= 0 || a.CPT < 0 || a.CPL < 0 || a.runBytes <= 0 || a.runBytes > 16 || a.runBytes % a.IC != 0) return hipErrorInvalidValue;
-        if (a.xBytes != (int64_t)a.N * a.IH * a.IW * a.IC || a.xBytes < 16) return hipErrorInvalidValue;
+        if (a.IH <= 0 || a.IW <= 0 || a.IC <= 0 || a.CS <= 0 || a.CPT < 0 || a.CPL < 0 || a.runBytes <= 0 || a.runBytes > 16 || a.runBytes % a.IC != 0) return false;
+        if (a.xBytes != (int64_t)a.N * a.IH * a.IW * a.IC || a.xBytes < 16) return false;
         // a workgroup's eight images and the padding around them, in 31 bits
-        if ((long long)a.IH * a.IW * a.IC > (1LL << 27)) return hipErrorInvalidValue;
+        if ((long long)a.IH * a.IW * a.IC > (1LL << 27)) return false;
     } else if ((uintptr_t)a.x & 15) {
-        return hipErrorInvalidValue;
+        return false;
     }
-    if (((uintptr_t)a.wexp | (uintptr_t)a.bias1 | (uintptr_t)a.scale1 | (uintptr_t)a.wdw | (uintptr_t)a.bias2 | (uintptr_t)a.scale2) & 15) return hipErrorInvalidValue;
-    if (((uintptr_t)a.out) & 3 || (a.CKH == 0 && (long long)a.H * a.W * a.K >= (1LL << 31))) return hipErrorInvalidValue;
+    if (((uintptr_t)a.wexp | (uintptr_t)a.bias1 | (uintptr_t)a.scale1 | (uintptr_t)a.wdw | (uintptr_t)a.bias2 | (uintptr_t)a.scale2) & 15) return false;
+    if (((uintptr_t)a.out) & 3 || (a.CKH == 0 && (long long)a.H * a.W * a.K >= (1LL << 31))) return false;
     // every window starts inside the image or its padding and none needs a row the strip does not make
-    if ((a.OH - 1) * a.S - a.PT >= a.H || (a.OW - 1) * a.S - a.PL >= a.W) return hipErrorInvalidValue;
+    if ((a.OH - 1) * a.S - a.PT >= a.H || (a.OW - 1) * a.S - a.PL >= a.W) return false;
     a.cellCols = irCellColumns(a.OW, a.S);
-    if ((long long)a.C > kIrMaxChannels) return hipErrorInvalidValue;
+    if ((long long)a.C > kIrMaxChannels) return false;
     // Four workgroups per CU (160 KB of LDS, 16 waves) overlap one another's phases: strips as high as 40 KB of cells hold
     // (56x56x32 -> 144, 256 images: 79 us at 20 KB, whose strips make more rows twice, 69 at 40, 76 at 64), lower where that
     // leaves fewer than two workgroups per CU (14x14x96 -> 576, 32 images: 8.0 us with at least 512, 9.1 with 1024), and down
@@ -405,7 +375,7 @@ hipError_t launchIrExpandDw(const IrExpandDwArgs &in, const LaunchCtx &ctx) {
     const long long perStrip = (long long)a.N * ((a.C + kIrChunk - 1) / kIrChunk);
     int strips = 1;
     auto rowsOf = [&](int s) { return (a.OH + s - 1) / s; };
-    auto lds = [&](int images, int s) { return irLds(images, rowsOf(s), a.S, a.cellCols); };
+    auto lds = [&](int images, int s) { return irLds(images, irCellRows(a, images, rowsOf(s)), a.cellCols); };
     // phase 1's rounds of a workgroup's four waves: where not even every second CU has a workgroup they are the launch's time
     auto rounds = [&](int s) { return (((rowsOf(s) - 1) * a.S + 3) * a.W + 127) / 128; };
     while (rowsOf(strips) > 1 && (lds(1, strips) > ldsAim || (perStrip * strips < wgAim && rowsOf(strips) > 4) || (perStrip * strips < 128 && rounds(strips) > 2))) strips++;
@@ -425,6 +395,12 @@ hipError_t launchIrExpandDw(const IrExpandDwArgs &in, const LaunchCtx &ctx) {
     if (a.segments > a.stripRows) a.segments = a.stripRows;
     a.segmentRows = (a.stripRows + a.segments - 1) / a.segments;
     a.segments = (a.stripRows + a.segmentRows - 1) / a.segmentRows;
+    return true;
+}
+
+hipError_t launchIrExpandDw(const IrExpandDwArgs &in, const LaunchCtx &ctx) {
+    IrExpandDwArgs a = in;
+    if (!planIrExpandDw(&a)) return hipErrorInvalidValue;
     return a.S == 1 ? launchIrS<1>(a, ctx) : launchIrS<2>(a, ctx);
 }
 

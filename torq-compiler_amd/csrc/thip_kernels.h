@@ -144,12 +144,14 @@ struct IrExpandDwArgs {
     // stride CS, whose H x W outputs take the pixels' place; K is unused
     int32_t CKH, CS, CPT, CPL, IH, IW, IC, runBytes, czp;
     int64_t xBytes;
-    int32_t images, stripRows, strips, segmentRows, segments, cellCols;  // the launcher sets these
+    int32_t images, stripRows, strips, segmentRows, segments, cellCols;  // planIrExpandDw sets these
     int32_t stepImages, stepRows, stepColumns;  // and these: 128 pixels
 };
 // A strip's results are addressed with 32 bits: its cells fit LDS, so they are fewer than 2^11 pixels.
 constexpr int kIrMaxChannels = 1 << 20;
 bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL);
+// Checks the arguments and sets what is the launch's own to choose; false where the kernel does not take them.
+bool planIrExpandDw(IrExpandDwArgs *a);
 hipError_t launchIrExpandDw(const IrExpandDwArgs &a, const LaunchCtx &ctx);
 
 // The small records of the ring kernels (dense or window loader): whether the kernel without tiles in LDS is ahead, and its launch.
