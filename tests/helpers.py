@@ -33,3 +33,20 @@ def families(kernels):
     return [k.split("<")[0] for k in kernels]
 
 
+def host_check(name, directory):
+    """Builds tests/host/<name>.cpp against the package's library with the host compiler; returns the program's path."""
+    import os
+    import shutil
+    import subprocess
+
+    from torq_compiler_amd import runtime
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    gxx = shutil.which("g++")
+    assert gxx, "g++ is needed for the host check"
+    exe = os.path.join(str(directory), name)
+    built = subprocess.run([gxx, "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + os.path.join(root, "torq-compiler_amd", "csrc"),
+                            os.path.join(root, "tests", "host", name + ".cpp"), runtime.LIB_PATH, "-Wl,-rpath," + os.path.dirname(runtime.LIB_PATH),
+                            "-Wl,--allow-shlib-undefined", "-o", exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert built.returncode == 0, built.stdout[-3000:]
+    return exe

@@ -1,0 +1,28 @@
+// The launches that the library plans for a serialised program (the file in argv[1]), one a line: what it is, its records, and the
+// kernel of a GEMM-shaped record.
+#include <stdio.h>
+
+#include <vector>
+
+#include "thip_plan.h"
+
+using namespace thip;
+
+int main(int argc, char **argv) {
+    if (argc != 2) return 2;
+    std::vector<uint8_t> blob;
+    FILE *f = fopen(argv[1], "rb");
+    if (!f) return 2;
+    fseek(f, 0, SEEK_END);
+    blob.resize((size_t)ftell(f));
+    rewind(f);
+    const size_t n = fread(blob.data(), 1, blob.size(), f);
+    fclose(f);
+    DescHeader h;
+    if (n != blob.size() || validateWhole(blob.data(), blob.size(), &h) != THIP_OK) return 3;
+    const DescriptorView v{blob.data(), h, (const DescOp *)(blob.data() + h.ops_offset), (const DescBinding *)(blob.data() + h.bindings_offset),
+                           (const DescTemp *)(blob.data() + h.temps_offset), (const DescConst *)(blob.data() + h.consts_offset)};
+    const char *kinds[] = {"record", "ir_expand_dw_i8", "padded", "igemm_rt_i8"}, *routes[] = {"", " igemm_direct_i8", " conv_patch_i8"};
+    for (const Step &s : planSteps(v, false)) printf("%s %u %u%s\n", kinds[s.kind], s.first, s.count, routes[s.route]);
+    return 0;
+}

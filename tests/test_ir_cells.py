@@ -1,27 +1,16 @@
 """The index arithmetic of the fused widening + depthwise launch, on the host: the library's own plan and the kernel's own walk, over
 frames, strides, paddings and shared workgroups (tests/host/ir_cells.cpp says what is checked)."""
-import os
-import shutil
 import subprocess
 
 import numpy as np
 import pytest
 
-from torq_compiler_amd import runtime
-
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-CSRC = os.path.join(ROOT, "torq-compiler_amd", "csrc")
+from helpers import host_check
 
 
 @pytest.fixture(scope="module")
 def check(tmp_path_factory):
-    gxx = shutil.which("g++")
-    assert gxx, "g++ is needed for the host check"
-    exe = str(tmp_path_factory.mktemp("ir") / "ir_cells")
-    built = subprocess.run([gxx, "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + CSRC,
-                            os.path.join(ROOT, "tests", "host", "ir_cells.cpp"), runtime.LIB_PATH, "-Wl,-rpath," + os.path.dirname(runtime.LIB_PATH),
-                            "-Wl,--allow-shlib-undefined", "-o", exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    assert built.returncode == 0, built.stdout[-3000:]
+    exe = host_check("ir_cells", tmp_path_factory.mktemp("ir"))
 
     def run(N, H, W, K, C, stride, pad, first=None):
         """pad: (top, bottom, left, right); first: (window, stride, channels), unpadded, its image as large as its windows need.

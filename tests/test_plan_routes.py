@@ -1,0 +1,91 @@
+"""Which kernel a dispatch takes for a GEMM-shaped op follows the alignment of its result too: results at every offset that the op's
+own kernel stores at, planned on the host and run on the GPU against the oracle."""
+import subprocess
+
+import numpy as np
+import pytest
+
+import desc_interp
+from helpers import assert_bit_exact, host_check, oracle_eval, run_on_gpu
+from torq_compiler_amd import workloads as w
+
+
+class Moved:
+    """A serialised single-op program whose result lies `offset` bytes into its binding, 64 bytes of room behind it."""
+
+    def __init__(self, wl, offset):
+        blob = bytearray(wl.program.serialize())
+        d = desc_interp.Descriptor(bytes(blob))
+        assert len(d.ops) == 1 and int(d.ops[0]["out"]["index"]) == 1
+        ops = np.frombuffer(blob, dtype=desc_interp.OP, count=1, offset=int(d.header["ops_offset"]))
+        bindings = np.frombuffer(blob, dtype=desc_interp.BINDING, count=2, offset=int(d.header["bindings_offset"]))
+        ops["out"]["offset"] = offset
+        bindings["size"][1] += offset + 64
+        self.blob = bytes(blob)
+
+    def serialize(self):
+        return self.blob
+
+
+def at_offset(wl, offset):
+    return w.Workload(wl.name, Moved(wl, offset), wl.inputs, [((int(np.prod(wl.outputs[0][0])) + offset + 64,), np.int8)], wl.ops, wl.bytes, wl.attrs)
+
+
+def batched():
+    """The second batch element's result lies at byte 2706."""
+    return w.matmul_workload(2, 33, 64, 41, constant_rhs=True)
+
+
+SMALL_LINEAR = lambda: w.fully_connected_workload(40, 64, 48, realistic=True)  # noqa: E731
+SMALL_CONV = lambda: w.conv2d_workload(N=1, H=12, W=12, C=64, O=32, realistic=True)  # noqa: E731
+PATCH_CONV = lambda: w.conv2d_workload(N=16, H=56, W=56, C=96, O=96, realistic=True)  # noqa: E731
+PADDED = lambda: w.fully_connected_workload(100000, 24, 128, realistic=True)  # noqa: E731
+DIRECT, PATCH, OWN = "record 0 1 igemm_direct_i8", "record 0 1 conv_patch_i8", "record 0 1"
+CASES = [
+    (SMALL_LINEAR, 4, DIRECT), (SMALL_LINEAR, 1, OWN), (SMALL_LINEAR, 2, OWN), (SMALL_LINEAR, 7, OWN), (SMALL_CONV, 8, DIRECT), (SMALL_CONV, 2, OWN),
+    (PATCH_CONV, 32, PATCH), (PATCH_CONV, 8, OWN), (PATCH_CONV, 1, OWN), (PADDED, 16, "padded 0 1"), (PADDED, 8, OWN),
+]
+IDS = ["%s-%d" % (n, c[1]) for n, c in zip(["linear"] * 4 + ["conv"] * 2 + ["patch"] * 3 + ["padded"] * 2, CASES)]
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    where = tmp_path_factory.mktemp("plan")
+    exe = host_check("plan", where)
+
+    def steps(wl):
+        path = where / "blob"
+        path.write_bytes(bytes(wl.program.serialize()))
+        done = subprocess.run([exe, str(path)], stdout=subprocess.PIPE, text=True, timeout=120)
+        assert done.returncode == 0
+        return done.stdout.splitlines()
+
+    return steps
+
+
+@pytest.mark.parametrize("make,offset,want", CASES, ids=IDS)
+def test_route_by_offset(plan, make, offset, want):
+    assert plan(at_offset(make(), offset)) == [want]
+
+
+def test_route_of_a_batch(plan):
+    assert plan(batched()) == ["record 0 1 igemm_direct_i8", "record 1 1"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("make,offset", [c[:2] for c in CASES], ids=IDS)
+def test_gpu_result_at_offset(device, make, offset):
+    wl = at_offset(make(), offset)
+    print("[gpu-case]", wl.name, offset, flush=True)
+    got, _ = run_on_gpu(device, wl, via="device")
+    want = oracle_eval(make())[0].reshape(-1)
+    assert_bit_exact(got[0][offset:offset + want.size], want, wl.name)
+    assert np.all(got[0][:offset] == 0x55) and np.all(got[0][offset + want.size:] == 0x55), "bytes around the result"
+
+
+@pytest.mark.gpu
+def test_gpu_batch(device):
+    wl = batched()
+    print("[gpu-case]", wl.name, flush=True)
+    got, _ = run_on_gpu(device, wl, via="device")
+    assert_bit_exact(got[0], oracle_eval(wl)[0], wl.name)

@@ -175,8 +175,10 @@ constexpr size_t kPatchMaxLds = 160 * 1024;
 // The pitch of rows of `bytes` (whole 16-byte units) in LDS.
 static int paddedPitch(int bytes) { return bytes / 16 % 4 == 0 ? bytes + 16 : bytes; }
 
-// Fills the plan; false where the kernel does not take the record.
+// Fills the plan; false where the kernel does not take the operands (whole 16-byte pieces of image, weights and results; the ring
+// kernel stores at any alignment).
 static bool planConvPatch(const IgemmArgs &a, ConvPatchPlan *q) {
+    if (!a.A || !a.Bp || !a.bias || !a.scale || !a.out || (((uintptr_t)a.A | (uintptr_t)a.Bp | (uintptr_t)a.out) & 15)) return false;
     if (a.loader != kLoaderWindow || a.out_dtype != kDtypeI8 || a.skip || a.M <= 0 || a.N <= 0 || a.N % 16 != 0 || a.N > 96 || a.C < 16 || a.C % 16 != 0) return false;
     if (a.KH <= 0 || a.KW <= 0 || a.KH > 16 || a.KW > 16 || a.H <= 0 || a.W <= 0 || a.OH <= 0 || a.OW <= 0 || a.SH != 1 || a.SW != 1 || a.PT < 0 || a.PL < 0) return false;
     const long long frame = (long long)a.OH * a.OW, taps = (long long)a.KH * a.KW * a.C;
@@ -234,7 +236,7 @@ static hipError_t launchPatch(const IgemmArgs &a, const ConvPatchPlan &q, const 
 
 hipError_t launchConvPatch(const IgemmArgs &a, const LaunchCtx &ctx) {
     ConvPatchPlan q;
-    if (!a.A || !a.Bp || !a.bias || !a.scale || !a.out || (((uintptr_t)a.A | (uintptr_t)a.Bp | (uintptr_t)a.out) & 15) || !planConvPatch(a, &q)) return hipErrorInvalidValue;
+    if (!planConvPatch(a, &q)) return hipErrorInvalidValue;
     switch ((a.N + 31) / 32) {
     case 1: return launchPatch<1>(a, q, ctx);
     case 2: return launchPatch<2>(a, q, ctx);

@@ -132,6 +132,8 @@ static void logEvent(const thip_executable_t *e, uint64_t invocation, int32_t ac
     fprintf(d->eventLog, "%s,%llu,%d,%lld,%s_%s,%s\n", e->header.name, (unsigned long long)invocation, action, (long long)us, event, phase, kernel);
 }
 
+static DescriptorView viewOf(const thip_executable_t *e) { return DescriptorView{e->blob.data(), e->header, e->ops, e->bindings, e->temps, e->consts}; }
+
 // Resolves an operand reference against the buffers of this dispatch.
 static uint8_t *resolve(const thip_executable_t *e, const DescRef &r, uint8_t *const *bindingPtrs) {
     switch (r.space) {
@@ -144,9 +146,9 @@ static uint8_t *resolve(const thip_executable_t *e, const DescRef &r, uint8_t *c
 
 // Launches `op`, which is record i or stands in for it, or (ctx.name set) only asks its launcher which kernel it takes for these
 // operands.  `scratch` (or null): the static scratch array, which then stands in for the record's workspace intermediate.
-// `step` (or null): the buffers of space kSpacePlan.  `planned`: a dispatch, which may take another kernel than the record's own.
+// `step` (or null): the buffers of space kSpacePlan.  `route`: the kernel of a GEMM-shaped record.
 static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr,
-                              uint8_t *const *step = nullptr, bool planned = false) {
+                              uint8_t *const *step = nullptr, IgemmRoute route = kIgemmOwnTile) {
     auto resolve = [step](const thip_executable_t *exe, const DescRef &r, uint8_t *const *bindings) {
         return r.space == kSpacePlan ? step[r.index] + r.offset : ::resolve(exe, r, bindings);
     };
@@ -159,35 +161,9 @@ static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op
         break;
     }
     case kKindIgemm: {
-        IgemmArgs a;
-        memset(&a, 0, sizeof(a));
-        a.A = (const int8_t *)resolve(e, op.in0, bp);
-        a.Bp = (const int8_t *)resolve(e, op.weights, bp);
-        a.bias = (const int32_t *)resolve(e, op.bias, bp);
-        a.scale = (const int32_t *)resolve(e, op.scale, bp);
-        a.ktab = (const uint32_t *)resolve(e, op.table, bp);
-        a.out = resolve(e, op.out, bp);
-        a.M = op.M; a.N = op.Nn; a.K = op.K; a.Kp = op.Kp; a.Np = op.Np;
-        a.H = op.H; a.W = op.W; a.C = op.C; a.OH = op.OH; a.OW = op.OW;
-        a.SH = op.SH; a.SW = op.SW; a.PT = op.PT; a.PL = op.PL;
-        a.KH = op.KH; a.KW = op.KW;
-        a.input_zp = op.input_zp;
-        a.out_dtype = op.out_dtype;
-        a.a_bytes = (int64_t)op.N * op.H * op.W * op.C;
-        a.loader = op.loader;
-        a.gran = op.gran;
-        a.rq = rq;
-        if (op.in1.space != kSpaceNone) {
-            ResidualAddParams ap;
-            memcpy(&ap, e->blob.data() + e->header.data_offset + e->consts[op.table.index].offset + op.table.offset, sizeof(ap));
-            a.skip = (const int8_t *)resolve(e, op.in1, bp);
-            a.add_skip_first = ap.other_first;
-            a.add_w0 = ap.w0; a.add_w1 = ap.w1; a.add_bias = ap.bias; a.add_scale = ap.scale;
-            a.arq = Requant{ap.shift, ap.output_zp, ap.output_min, ap.output_max, 0, 0};
-        }
-        if (!planned || e->tuning.plainRecords) err = launchIgemm(a, op.variant, ctx);
-        else if (igemmDirectBetter(a)) err = launchIgemmDirect(a, ctx);
-        else if (convPatchBetter(a)) err = launchConvPatch(a, ctx);
+        const IgemmArgs a = igemmArgs(viewOf(e), op, [&](const DescRef &r) { return resolve(e, r, bp); });
+        if (route == kIgemmDirect) err = launchIgemmDirect(a, ctx);
+        else if (route == kIgemmPatch) err = launchConvPatch(a, ctx);
         else err = launchIgemm(a, op.variant, ctx);
         break;
     }
@@ -544,10 +520,10 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
     case kStepPadded: {
         uint8_t *const *buffers = &e->stepBuffers[2 * (size_t)(&s - e->steps.data())];
         err = launchPadRows((const int8_t *)resolve(e, e->ops[s.first].in0, bp), (int8_t *)buffers[0], s.rows, s.from, s.to, ctx);
-        if (err == hipSuccess) return launchOp(e, s.first, s.op, bp, ctx, scratch, buffers, true);
+        if (err == hipSuccess) return launchOp(e, s.first, s.op, bp, ctx, scratch, buffers, s.route);
         break;
     }
-    default: return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch, nullptr, true);
+    default: return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch, nullptr, s.route);
     }
     if (err != hipSuccess) return fail(THIP_INTERNAL, "ops %u .. %u: launch failed: %s", s.first, s.first + s.count - 1, hipGetErrorString(err));
     return THIP_OK;
@@ -814,6 +790,35 @@ void thip_executable_destroy(thip_executable_t *e) {
     delete e;
 }
 
+// Adds a launch to the executable's, with the buffers of its own that it needs.  It is asked for its kernels now, as the records were; one
+// that its launchers do not take is left out again (*taken), for its records to run one by one.
+static thip_status_t addStep(thip_executable_t *e, Step &&planned, bool *taken) {
+    e->steps.push_back(std::move(planned));
+    e->stepBuffers.insert(e->stepBuffers.end(), 2, nullptr);
+    Step &step = e->steps.back();
+    if (step.kind == kStepPadded) {
+        uint8_t **buffers = &e->stepBuffers[e->stepBuffers.size() - 2];
+        hipError_t err = hipMalloc((void **)&buffers[0], (size_t)step.rows * step.to);
+        if (err == hipSuccess) err = hipMalloc((void **)&buffers[1], step.constants.size());
+        if (err == hipSuccess) err = hipMemcpy(buffers[1], step.constants.data(), step.constants.size(), hipMemcpyHostToDevice);
+        if (err != hipSuccess) return hipFail(err, "allocating a step's operands");
+        std::vector<uint8_t>().swap(step.constants);
+    }
+    uint8_t *placeholder[64];
+    for (auto &ptr : placeholder) ptr = (uint8_t *)(uintptr_t)0x1000000;
+    char name[96];
+    *taken = launchStep(e, step, placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name)}) == THIP_OK;
+    if (!*taken) {
+        (void)hipGetLastError();
+        for (int k = 0; k < 2; k++) {
+            if (uint8_t *p = e->stepBuffers.back()) (void)hipFree(p);
+            e->stepBuffers.pop_back();
+        }
+        e->steps.pop_back();
+    }
+    return THIP_OK;
+}
+
 thip_status_t thip_executable_create(thip_device_t *device, const void *blob, size_t size, const uint32_t *constants,
                                      size_t constant_count, thip_executable_t **out_executable) {
     if (!out_executable) return fail(THIP_INVALID_ARGUMENT, "null result pointer");
@@ -834,7 +839,7 @@ thip_status_t thip_executable_create(thip_device_t *device, const void *blob, si
     e->consts = (const DescConst *)(e->blob.data() + h.consts_offset);
     thip_status_t s = THIP_OK;
     {
-        const DescriptorView view{e->blob.data(), h, e->ops, e->bindings, e->temps, e->consts};
+        const DescriptorView view = viewOf(e);
         for (uint32_t i = 0; i < h.op_count && s == THIP_OK; i++) s = checkOpFootprint(&view, i);
     }
     auto bail = [&](thip_status_t code) {
@@ -887,24 +892,19 @@ thip_status_t thip_executable_create(thip_device_t *device, const void *blob, si
             e->kernelNames[i] = name[0] ? name : opKernelName(e->ops[i]);
         }
     }
-    e->steps = planSteps(DescriptorView{e->blob.data(), h, e->ops, e->bindings, e->temps, e->consts}, e->tuning.plainRecords);
-    e->stepBuffers.assign(2 * e->steps.size(), nullptr);
-    for (size_t i = 0; i < e->steps.size(); i++) {
-        Step &step = e->steps[i];
-        if (step.kind != kStepPadded) continue;
-        uint8_t **buffers = &e->stepBuffers[2 * i];
-        err = hipMalloc((void **)&buffers[0], (size_t)step.rows * step.to);
-        if (err == hipSuccess) err = hipMalloc((void **)&buffers[1], step.constants.size());
-        if (err == hipSuccess) err = hipMemcpy(buffers[1], step.constants.data(), step.constants.size(), hipMemcpyHostToDevice);
-        if (err != hipSuccess) return bail(hipFail(err, "allocating a step's operands"));
-        std::vector<uint8_t>().swap(step.constants);
-    }
-    {
-        // the launches' own kernels are configured now too (naming mode again; an error is the dispatch's to report)
-        uint8_t *placeholder[64];
-        for (auto &ptr : placeholder) ptr = (uint8_t *)(uintptr_t)0x1000000;
-        char name[96];
-        for (const Step &step : e->steps) (void)launchStep(e, step, placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name)});
+    for (Step &step : planSteps(viewOf(e), e->tuning.plainRecords)) {
+        const uint32_t first = step.first, count = step.count;
+        bool taken = false;
+        if (thip_status_t st = addStep(e, std::move(step), &taken)) return bail(st);
+        for (uint32_t i = first; !taken && i < first + count; i++) {
+            Step record{};
+            record.kind = kStepRecord;
+            record.first = i;
+            record.count = 1;
+            bool ran = false;
+            if (thip_status_t st = addStep(e, std::move(record), &ran)) return bail(st);
+            if (!ran) return bail(fail(THIP_INTERNAL, "op %u (%s): no kernel takes it", i, e->kernelNames[i].c_str()));
+        }
     }
     *out_executable = e;
     return THIP_OK;

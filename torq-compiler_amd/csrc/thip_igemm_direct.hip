@@ -118,6 +118,21 @@ __global__ __launch_bounds__(NW * 64) void igemm_direct_i8(IgemmArgs p, FastDiv 
 
 static long long directTiles(const IgemmArgs &a) { return (long long)((a.M + 31) / 32) * ((a.N + 31) / 32); }
 
+// What the kernel assumes of its operands, their addresses' alignment included (the ring kernel stores at any).
+static bool directTakes(const IgemmArgs &a) {
+    const bool window = a.loader == kLoaderWindow;
+    if (!a.A || !a.Bp || !a.bias || !a.scale || !a.out || a.M <= 0 || a.N <= 0 || a.K <= 0 || (!window && a.loader != kLoaderDense)) return false;
+    if (a.K % 16 != 0 || a.Kp < (a.K + 31) / 32 * 32 || a.Np < (a.N + 31) / 32 * 32 || a.Kp % 16 != 0) return false;
+    if (((uintptr_t)a.A | (uintptr_t)a.Bp | (uintptr_t)a.bias | (uintptr_t)a.scale) & 15) return false;
+    if (a.out_dtype < kDtypeI8 || a.out_dtype > kDtypeI32 || ((uintptr_t)a.out & 3) || (a.skip && (((uintptr_t)a.skip & 3) || a.N % 4 != 0 || a.out_dtype != kDtypeI8))) return false;
+    if (window) {
+        if (a.C < 16 || a.C % 16 != 0 || a.KH <= 0 || a.KW <= 0 || a.H <= 0 || a.W <= 0 || a.OH <= 0 || a.OW <= 0 || a.SH <= 0 || a.SW <= 0 || a.PT < 0 || a.PL < 0) return false;
+        if (a.M % (a.OH * a.OW) != 0 || (long long)a.K != (long long)a.KH * a.KW * a.C) return false;
+        if (a.a_bytes != (long long)(a.M / (a.OH * a.OW)) * a.H * a.W * a.C || a.a_bytes >= (1LL << 32)) return false;
+    }
+    return true;
+}
+
 // Against the ring kernel's own tile, us (tiles; ring / direct):
 //   dense   49 x 960 -> 160 (10) 4.2 / 3.4, 1429 x 1344 -> 48 (90) 5.0 / 4.1, 400 x 512 -> 512 (208) 3.7 / 3.6, 450 x 80 -> 752 (360)
 //           2.9 / 3.2, 28 x 5536 -> 144 (5) 12.4 / 8.6, 40 x 8192 -> 2048 (128) 17.6 / 18.1
@@ -125,7 +140,7 @@ static long long directTiles(const IgemmArgs &a) { return (long long)((a.M + 31)
 //           batch 3 (473) 8.3 / 6.0, 5x5 32x32x32 -> 64, batch 15 (960) 6.8 / 6.1, 14x14x512 -> 512, batch 8 (784) 18.0 / 33.4
 // so: up to a workgroup per CU, or, where the ring has to address a window, up to the 50 MB that its tiles' operands may be together.
 bool igemmDirectBetter(const IgemmArgs &a) {
-    if (a.loader != kLoaderDense && a.loader != kLoaderWindow) return false;
+    if (!directTakes(a)) return false;
     const long long tiles = directTiles(a), bytes = tiles * 64 * a.K;
     return a.loader == kLoaderWindow ? tiles <= 1024 && bytes <= 50000000 : tiles <= 256 && bytes <= 25000000;
 }
@@ -141,15 +156,7 @@ static hipError_t launchDirect(const IgemmArgs &a, const LaunchCtx &ctx) {
 
 hipError_t launchIgemmDirect(const IgemmArgs &a, const LaunchCtx &ctx) {
     const bool window = a.loader == kLoaderWindow;
-    if (!a.A || !a.Bp || !a.bias || !a.scale || !a.out || a.M <= 0 || a.N <= 0 || a.K <= 0 || (!window && a.loader != kLoaderDense)) return hipErrorInvalidValue;
-    if (a.K % 16 != 0 || a.Kp < (a.K + 31) / 32 * 32 || a.Np < (a.N + 31) / 32 * 32 || a.Kp % 16 != 0) return hipErrorInvalidValue;
-    if (((uintptr_t)a.A | (uintptr_t)a.Bp | (uintptr_t)a.bias | (uintptr_t)a.scale) & 15) return hipErrorInvalidValue;
-    if (a.out_dtype < kDtypeI8 || a.out_dtype > kDtypeI32 || ((uintptr_t)a.out & 3) || (a.skip && (((uintptr_t)a.skip & 3) || a.N % 4 != 0 || a.out_dtype != kDtypeI8))) return hipErrorInvalidValue;
-    if (window) {
-        if (a.C < 16 || a.C % 16 != 0 || a.KH <= 0 || a.KW <= 0 || a.H <= 0 || a.W <= 0 || a.OH <= 0 || a.OW <= 0 || a.SH <= 0 || a.SW <= 0 || a.PT < 0 || a.PL < 0) return hipErrorInvalidValue;
-        if (a.M % (a.OH * a.OW) != 0 || (long long)a.K != (long long)a.KH * a.KW * a.C) return hipErrorInvalidValue;
-        if (a.a_bytes != (long long)(a.M / (a.OH * a.OW)) * a.H * a.W * a.C || a.a_bytes >= (1LL << 32)) return hipErrorInvalidValue;
-    }
+    if (!directTakes(a)) return hipErrorInvalidValue;
     // eight waves while that leaves a CU two workgroups (3x3 56x56x64 -> 64: 3.4 us against 3.8 with four), four beyond (142x142x144
     // -> 8, batch 3: 6.0 against 6.8)
     const bool few = directTiles(a) <= 400;

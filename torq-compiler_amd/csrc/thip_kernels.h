@@ -154,11 +154,13 @@ bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL);
 bool planIrExpandDw(IrExpandDwArgs *a);
 hipError_t launchIrExpandDw(const IrExpandDwArgs &a, const LaunchCtx &ctx);
 
-// The small records of the ring kernels (dense or window loader): whether the kernel without tiles in LDS is ahead, and its launch.
+// The small records of the ring kernels (dense or window loader): whether the kernel without tiles in LDS takes these operands and is
+// ahead, and its launch.
 bool igemmDirectBetter(const IgemmArgs &a);
 hipError_t launchIgemmDirect(const IgemmArgs &a, const LaunchCtx &ctx);
 
-// The convolutions whose weights fit LDS beside a patch of the image: whether the kernel that keeps both there is ahead, and its launch.
+// The convolutions whose weights fit LDS beside a patch of the image: whether the kernel that keeps both there takes these operands and
+// is ahead, and its launch.
 bool convPatchBetter(const IgemmArgs &a);
 hipError_t launchConvPatch(const IgemmArgs &a, const LaunchCtx &ctx);
 

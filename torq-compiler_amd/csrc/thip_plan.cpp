@@ -163,6 +163,7 @@ static bool matchPadded(const DescriptorView &v, uint32_t first, Step *s) {
         uint32_t variant;
         op.loader = pointwise ? kLoaderDense : kLoaderWindow;
         if (thip_gemm_tile_choice((int32_t)op.loader, g.M, N, K, Cp, g.out_dtype, 0, &variant, nullptr, 0) != THIP_OK) return false;
+        if (variant == kIgemmStream && g.out.offset % 16 != 0) return false;  // it stores whole 16-byte pieces; the record's kernel any
         const IgemmTile &t = igemmTile(variant);
         Kp = roundUp(K, t.bk);
         Np = roundUp(N, t.bn);
@@ -194,6 +195,15 @@ static bool matchPadded(const DescriptorView &v, uint32_t first, Step *s) {
     return true;
 }
 
+// The kernel that is ahead for a GEMM-shaped record.
+static IgemmRoute igemmRoute(const DescriptorView &v, const DescOp &op) {
+    // addresses that are aligned as a dispatch's are
+    const IgemmArgs a = igemmArgs(v, op, [&](const DescRef &r) {
+        return r.space == kSpaceNone ? nullptr : (uint8_t *)(uintptr_t)(0x1000000 + (r.space == kSpaceConst ? v.consts[r.index].offset : 0) + r.offset);
+    });
+    return igemmDirectBetter(a) ? kIgemmDirect : convPatchBetter(a) ? kIgemmPatch : kIgemmOwnTile;
+}
+
 std::vector<Step> planSteps(const DescriptorView &v, bool plain) {
     const std::vector<uint32_t> uses = tempUses(v);
     std::vector<Step> steps;
@@ -204,6 +214,8 @@ std::vector<Step> planSteps(const DescriptorView &v, bool plain) {
             s.first = i;
             s.count = 1;
         }
+        const DescOp *op = s.kind == kStepRecord ? &v.ops[i] : s.kind == kStepPadded ? &s.op : nullptr;
+        s.route = !plain && op && op->kind == kKindIgemm ? igemmRoute(v, *op) : kIgemmOwnTile;
         steps.push_back(s);
         i += s.count;
     }

@@ -2,8 +2,11 @@
 // Host-only (no HIP calls).
 #pragma once
 
+#include <string.h>
+
 #include <vector>
 
+#include "thip_kernels.h"
 #include "thip_validate.h"
 
 namespace thip {
@@ -15,9 +18,17 @@ enum StepKind {
     kStepMatmulRt,  // a batch of int8 matmuls with a run-time input2: its transposes and its GEMMs (igemm_rt_i8)
 };
 
+// The kernel that a GEMM-shaped record of a dispatch runs by.
+enum IgemmRoute {
+    kIgemmOwnTile,  // the record's
+    kIgemmDirect,   // igemm_direct_i8
+    kIgemmPatch,    // conv_patch_i8
+};
+
 struct Step {
     StepKind kind;
     uint32_t first, count;  // the records it stands for
+    IgemmRoute route;       // of the record, or of `op` (kStepPadded)
     // kStepMatmulRt: the matrices of batch element 0, elements from one batch element to the next (0: shared), and the one
     // (bias, scale) pair
     DescRef a, b, out;
@@ -33,9 +44,42 @@ struct Step {
 };
 constexpr uint32_t kSpacePlan = 16;
 
+// The arguments of a GEMM-shaped record, its operands where `at` (const DescRef & -> uint8_t *) says.
+template <typename At>
+IgemmArgs igemmArgs(const DescriptorView &v, const DescOp &op, At &&at) {
+    IgemmArgs a;
+    memset(&a, 0, sizeof(a));
+    a.A = (const int8_t *)at(op.in0);
+    a.Bp = (const int8_t *)at(op.weights);
+    a.bias = (const int32_t *)at(op.bias);
+    a.scale = (const int32_t *)at(op.scale);
+    a.ktab = (const uint32_t *)at(op.table);
+    a.out = at(op.out);
+    a.M = op.M; a.N = op.Nn; a.K = op.K; a.Kp = op.Kp; a.Np = op.Np;
+    a.H = op.H; a.W = op.W; a.C = op.C; a.OH = op.OH; a.OW = op.OW;
+    a.SH = op.SH; a.SW = op.SW; a.PT = op.PT; a.PL = op.PL;
+    a.KH = op.KH; a.KW = op.KW;
+    a.input_zp = op.input_zp;
+    a.out_dtype = op.out_dtype;
+    a.a_bytes = (int64_t)op.N * op.H * op.W * op.C;
+    a.loader = op.loader;
+    a.gran = op.gran;
+    a.rq = Requant{op.shift, op.output_zp, op.output_min, op.output_max, op.pre_shift, op.t0_clamp};
+    if (op.in1.space != kSpaceNone) {
+        ResidualAddParams ap;
+        memcpy(&ap, v.blob + v.header.data_offset + v.consts[op.table.index].offset + op.table.offset, sizeof(ap));
+        a.skip = (const int8_t *)at(op.in1);
+        a.add_skip_first = ap.other_first;
+        a.add_w0 = ap.w0; a.add_w1 = ap.w1; a.add_bias = ap.bias; a.add_scale = ap.scale;
+        a.arq = Requant{ap.shift, ap.output_zp, ap.output_min, ap.output_max, 0, 0};
+    }
+    return a;
+}
+
 // The launches of a dispatch in order.  Every record belongs to exactly one step; a step that stands for several leaves
 // the intermediates between them unwritten, so it is only formed where no other record reads them.
-// `plain`: one step per record.
+// `plain`: one step per record, by the record's own kernel.  Routes are settled here, on all that their launchers ask: a dispatch's
+// buffers start at 16-byte boundaries, so the offsets say how its operands are aligned.
 std::vector<Step> planSteps(const DescriptorView &view, bool plain);
 
 }  // namespace thip
