@@ -602,6 +602,11 @@ thip_status_t thip_executable_op_count(thip_executable_t *executable, uint32_t *
  * without tiles, with the same results (THIP_PLAIN_RECORDS in the environment at creation: they do not). */
 thip_status_t thip_executable_op_kernel(thip_executable_t *executable, uint32_t index,
                                         char *name, size_t capacity);
+/* What those other dispatches launch, in order, as settled at creation: how many kernels, and the name of kernel `index`.  (The
+ * small kernel that adds the partial sums of a linear whose K is split stands with the linear.) */
+thip_status_t thip_executable_launch_count(thip_executable_t *executable, uint32_t *out_count);
+thip_status_t thip_executable_launch_kernel(thip_executable_t *executable, uint32_t index,
+                                            char *name, size_t capacity);
 thip_status_t thip_executable_binding_count(thip_executable_t *executable, uint32_t *out_count);
 thip_status_t thip_executable_binding_size(thip_executable_t *executable, uint32_t binding,
                                            size_t *out_size);
@@ -621,7 +626,8 @@ thip_status_t thip_gemm_tile_choice(int32_t addressing, int64_t M, int64_t N, in
  * dispatch_name, invocation_id, action_id, timestamp_us, event -- event an EventType name plus _BEGIN / _END:
  * DISPATCH, DISPATCH_SYNC_BINDINGS_IN / _OUT, DISPATCH_EXECUTE_ACTIONS, NSS_START per kernel launch (action_id = the
  * op's index), NSS_WAIT -- and a sixth column, kernel, naming the kernel of a launch row.  An empty path closes the
- * log.  While a log is open dispatches are not replayed as graphs. */
+ * log.  While a log is open dispatches launch every op by its own kernel (thip_executable_op_kernel) and are not replayed as
+ * graphs: its times are of these launches, not of the fused ones that a dispatch without a log makes. */
 thip_status_t thip_device_set_event_log(thip_device_t *device, const char *csv_path);
 
 #ifdef __cplusplus

@@ -1,16 +1,20 @@
 """Shared helpers of the test-suite: run a workload through the C-ABI, evaluate it with the oracle."""
 import numpy as np
+import pytest
 
 from oracle.programs import (BF16_TALLY, assert_bf16_close, assert_bit_exact, bf16_ordered,  # noqa: F401  (re-exported)
                              eval_network as oracle_network, eval_workload as oracle_eval)
 
 
-def run_on_gpu(device, wl, via="host"):
-    """Serialises the workload's program, loads it and runs one dispatch; returns the outputs."""
+def run_on_gpu(device, wl, via="host", launched=None):
+    """Serialises the workload's program, loads it and runs one dispatch; returns the outputs and the kernels that its ops have of their
+    own.  `launched` (a list): receives the kernels that the dispatch launches."""
     import torq_compiler_amd as thip
 
     blob = wl.program.serialize()
     exe = thip.Executable(device, blob)
+    if launched is not None:
+        launched += exe.launch_kernels()
     outs = [np.full(shape, 0x55, dtype=dt) for shape, dt in wl.outputs]
     try:
         if via == "host":
@@ -26,6 +30,17 @@ def run_on_gpu(device, wl, via="host"):
         return outs, exe.op_kernels()
     finally:
         exe.close()
+
+
+def check_own_kernels(device, wl, want, via="host"):
+    """Where a dispatch takes other kernels than its ops' own, a run of the ops by these, against `want` (the outputs)."""
+    with pytest.MonkeyPatch.context() as m:
+        launched = []
+        m.setenv("THIP_PLAIN_RECORDS", "1")
+        got, kernels = run_on_gpu(device, wl, via=via, launched=launched)
+        assert launched == kernels, (launched, kernels)
+        for g, e in zip(got, want):
+            assert_bit_exact(g, e, wl.name + " by the ops' own kernels")
 
 
 def families(kernels):

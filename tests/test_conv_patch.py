@@ -2,7 +2,7 @@
 requant tail; against the oracle and against the record's own kernel."""
 import pytest
 
-from helpers import assert_bit_exact, oracle_eval, run_on_gpu
+from helpers import assert_bit_exact, check_own_kernels, families, oracle_eval, run_on_gpu
 from torq_compiler_amd import workloads as w
 
 pytestmark = pytest.mark.gpu
@@ -15,12 +15,12 @@ pytestmark = pytest.mark.gpu
     dict(N=6, H=100, W=100, C=80, O=48, pad=(0, 0, 0, 0), input_zp=-90, output_min=-128), dict(N=40, H=34, W=40, C=16, O=16, KH=5, KW=5, pad=(4, 4, 4, 4)),
     dict(N=20, H=51, W=50, C=24, O=48, realistic=True),  # channels padded to 32 on the way
 ], ids=lambda kw: "x".join(str(v) for v in kw.values()))
-def test_conv_patch(device, kw, monkeypatch):
+def test_conv_patch(device, kw):
     wl = w.conv2d_workload(**kw)
     print("[gpu-case]", wl.name, flush=True)
     want = oracle_eval(wl)[0]
-    got, _ = run_on_gpu(device, wl, via="device")
+    launched = []
+    got, _ = run_on_gpu(device, wl, via="device", launched=launched)
+    assert "conv_patch_i8" in families(launched), launched
     assert_bit_exact(got[0], want, wl.name)
-    monkeypatch.setenv("THIP_PLAIN_RECORDS", "1")
-    got, _ = run_on_gpu(device, wl, via="device")
-    assert_bit_exact(got[0], want, wl.name + " by the record's own kernel")
+    check_own_kernels(device, wl, [want], "device")

@@ -8,7 +8,7 @@ import sys
 import numpy as np
 import pytest
 
-from helpers import assert_bit_exact, families, oracle_eval, oracle_network, run_on_gpu
+from helpers import assert_bit_exact, check_own_kernels, families, oracle_eval, oracle_network, run_on_gpu
 from test_emitter import CONV, MATMUL, WINDOW_RING, WINDOW_RING_FEW_CHANNELS, _chain_program, _padded_chain, matmul_id
 from torq_compiler_amd import Executable, ThipError, runtime, workloads as w
 
@@ -22,9 +22,12 @@ def announce(*what):
 
 def check(device, wl, via="host", kernel=None):
     announce(wl.name, "via", via)
-    got, kernels = run_on_gpu(device, wl, via=via)
+    launched = []
+    got, kernels = run_on_gpu(device, wl, via=via, launched=launched)
     want = oracle_eval(wl)
     assert_bit_exact(got[0], want[0], wl.name)
+    if launched != kernels:
+        check_own_kernels(device, wl, want, via)
     if kernel is not None:
         # `kernel` names what rocprof would show for the op: a whole instantiation ("name<args>") must match exactly,
         # a bare name must be the name in front of the template arguments

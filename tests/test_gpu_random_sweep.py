@@ -10,7 +10,7 @@ test asserts only that some kernel of the op's family ran, and the result.
 import numpy as np
 import pytest
 
-from helpers import assert_bit_exact, families, oracle_eval, oracle_network, run_on_gpu
+from helpers import assert_bit_exact, check_own_kernels, families, oracle_eval, oracle_network, run_on_gpu
 from torq_compiler_amd import workloads as w
 
 CHANNELS = [1, 3, 4, 8, 15, 16, 17, 24, 32, 33, 48, 64, 96, 144]
@@ -146,10 +146,13 @@ SWEEP = ([("conv2d", _conv, s, {"igemm_i8", "igemm_dense_i8", "igemm_stream_i8",
 def test_random_geometry(device, op, make, seed, allowed):
     wl = make(seed)
     print("[gpu-case]", op, seed, wl.name, flush=True)
-    got, kernels = run_on_gpu(device, wl, via="host" if seed % 2 else "device")
+    via, launched = "host" if seed % 2 else "device", []
+    got, kernels = run_on_gpu(device, wl, via=via, launched=launched)
     want = oracle_eval(wl)
     for g, e in zip(got, want):
         assert_bit_exact(g, e, "%s seed %d (%s)" % (op, seed, wl.name))
+    if launched != kernels:  # `allowed` names the ops' own kernels
+        check_own_kernels(device, wl, want, via)
     main = [k for k in families(kernels) if k != "transpose_i8"]
     assert main and set(main) <= allowed, (kernels, allowed)
 
@@ -169,8 +172,10 @@ def test_random_network(device, kw):
     wl = w.mobilenet_v2_workload(classes=37, **kw)
     print("[gpu-case]", wl.name, kw, flush=True)
     got, kernels = run_on_gpu(device, wl, via="device")
-    assert_bit_exact(got[0], oracle_network(wl), wl.name)
+    want = oracle_network(wl)
+    assert_bit_exact(got[0], want, wl.name)
     assert len(kernels) >= 50
+    check_own_kernels(device, wl, [want], "device")
 
 
 def test_networks_through_the_descriptor_interpreter():

@@ -3,7 +3,7 @@ the oracle, and against the records' own kernels."""
 import numpy as np
 import pytest
 
-from helpers import assert_bit_exact, oracle_eval, run_on_gpu
+from helpers import assert_bit_exact, check_own_kernels, families, oracle_eval, run_on_gpu
 from torq_compiler_amd import workloads as w
 
 pytestmark = pytest.mark.gpu
@@ -22,12 +22,12 @@ CASES = [
 
 
 @pytest.mark.parametrize("make", CASES, ids=range(len(CASES)))
-def test_direct(device, make, monkeypatch):
+def test_direct(device, make):
     wl = make()
     print("[gpu-case]", wl.name, flush=True)
     want = oracle_eval(wl)[0]
-    got, _ = run_on_gpu(device, wl, via="device")
+    launched = []
+    got, _ = run_on_gpu(device, wl, via="device", launched=launched)
+    assert "igemm_direct_i8" in families(launched), launched
     assert_bit_exact(got[0], want, wl.name)
-    monkeypatch.setenv("THIP_PLAIN_RECORDS", "1")
-    got, _ = run_on_gpu(device, wl, via="device")
-    assert_bit_exact(got[0], want, wl.name + " by the record's own kernel")
+    check_own_kernels(device, wl, [want], "device")

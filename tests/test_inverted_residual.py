@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from helpers import assert_bit_exact, oracle_network, run_on_gpu
+from helpers import assert_bit_exact, families, oracle_network, run_on_gpu
 from torq_compiler_amd import Program, workloads as w
 
 pytestmark = pytest.mark.gpu
@@ -32,6 +32,13 @@ def block(N, H, W, C, E, stride, pad=(1, 1, 1, 1), shift=None, first=None, seed=
     return w.Workload("block_%dx%dx%dx%d_k%d_e%d_s%d" % (N, H, W, C, k, E, stride), p, [x], [((N, oh, ow, E), np.int8)], 0, 0, dict(layers=layers, nhwc=True))
 
 
+def fused(device, wl):
+    launched = []
+    got, _ = run_on_gpu(device, wl, via="device", launched=launched)
+    assert families(launched) == ["ir_expand_dw_i8"], launched
+    return got
+
+
 @pytest.mark.parametrize("kw", [
     dict(N=1, H=14, W=14, C=64, E=384, stride=1), dict(N=2, H=13, W=15, C=16, E=48, stride=1), dict(N=1, H=9, W=7, C=48, E=80, stride=2),
     dict(N=3, H=20, W=21, C=32, E=144, stride=2, pad=(0, 1, 0, 1)), dict(N=2, H=7, W=7, C=160, E=960, stride=1), dict(N=1, H=3, W=3, C=192, E=16, stride=1, pad=(0, 0, 0, 0)),
@@ -47,7 +54,7 @@ def test_expand_depthwise(device, kw, tmp_path):
     wl = block(**kw)
     print("[gpu-case]", wl.name, flush=True)
     want = oracle_network(wl)
-    got, _ = run_on_gpu(device, wl, via="device")
+    got = fused(device, wl)
     assert_bit_exact(got[0], want, wl.name)
     device.set_event_log(str(tmp_path / "log.csv"))  # a log has its records launched one by one
     try:
@@ -61,7 +68,9 @@ def test_expand_depthwise_ragged_channels(device):
     """A widened image that something else reads too, and one the depthwise kernel has its own layout for, stay two launches."""
     for kw in (dict(N=1, H=8, W=8, C=16, E=24, stride=1), dict(N=1, H=8, W=8, C=208, E=32, stride=1), dict(N=1, H=8, W=8, C=16, E=32, stride=1, shift=0)):
         wl = block(**kw)
-        got, _ = run_on_gpu(device, wl, via="device")
+        launched = []
+        got, _ = run_on_gpu(device, wl, via="device", launched=launched)
+        assert "ir_expand_dw_i8" not in families(launched), launched
         assert_bit_exact(got[0], oracle_network(wl), wl.name)
 
 
@@ -74,8 +83,7 @@ def test_expand_depthwise_walk(device, kw):
     """A tile's 128 pixels that are whole images, whole rows, a row and a bit, less than a row; images that share a workgroup."""
     wl = block(**kw)
     print("[gpu-case]", wl.name, flush=True)
-    got, _ = run_on_gpu(device, wl, via="device")
-    assert_bit_exact(got[0], oracle_network(wl), wl.name)
+    assert_bit_exact(fused(device, wl)[0], oracle_network(wl), wl.name)
 
 
 @pytest.mark.parametrize("kw", [
@@ -87,5 +95,4 @@ def test_rows_no_window_reaches(device, kw):
     """Several images per workgroup whose last row lies below every window."""
     wl = block(**kw)
     print("[gpu-case]", wl.name, flush=True)
-    got, _ = run_on_gpu(device, wl, via="device")
-    assert_bit_exact(got[0], oracle_network(wl), wl.name)
+    assert_bit_exact(fused(device, wl)[0], oracle_network(wl), wl.name)

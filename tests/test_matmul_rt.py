@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from helpers import assert_bit_exact, oracle_eval, run_on_gpu
+from helpers import assert_bit_exact, families, oracle_eval, run_on_gpu
 from torq_compiler_amd import workloads as w
 
 pytestmark = pytest.mark.gpu
@@ -22,7 +22,9 @@ def test_runtime_input2(device, kw, tmp_path):
     wl = w.matmul_workload(**kw)
     print("[gpu-case]", wl.name, flush=True)
     want = oracle_eval(wl)[0]
-    got, _ = run_on_gpu(device, wl, via="device")
+    launched = []
+    got, _ = run_on_gpu(device, wl, via="device", launched=launched)
+    assert families(launched) == ["igemm_rt_i8"], launched
     assert_bit_exact(got[0], want, wl.name)
     device.set_event_log(str(tmp_path / "log.csv"))  # a log has its records launched one by one
     try:

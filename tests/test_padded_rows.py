@@ -24,7 +24,9 @@ def test_padded(device, make, tmp_path):
     print("[gpu-case]", wl.name, flush=True)
     want = oracle_eval(wl)[0]
     for via in ("device", "host"):
-        got, _ = run_on_gpu(device, wl, via=via)
+        launched = []
+        got, _ = run_on_gpu(device, wl, via=via, launched=launched)
+        assert "pad_rows_i8" in launched, launched
         assert_bit_exact(got[0], want, wl.name)
     device.set_event_log(str(tmp_path / "log.csv"))  # a log has its records launched one by one
     try:

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import desc_interp
-from helpers import assert_bit_exact, host_check, oracle_eval, run_on_gpu
+from helpers import assert_bit_exact, families, host_check, oracle_eval, run_on_gpu
 from torq_compiler_amd import workloads as w
 
 
@@ -73,11 +73,13 @@ def test_route_of_a_batch(plan):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("make,offset", [c[:2] for c in CASES], ids=IDS)
-def test_gpu_result_at_offset(device, make, offset):
+@pytest.mark.parametrize("make,offset,route", CASES, ids=IDS)
+def test_gpu_result_at_offset(device, make, offset, route):
     wl = at_offset(make(), offset)
     print("[gpu-case]", wl.name, offset, flush=True)
-    got, _ = run_on_gpu(device, wl, via="device")
+    launched = []
+    got, kernels = run_on_gpu(device, wl, via="device", launched=launched)
+    assert {DIRECT: "igemm_direct_i8", PATCH: "conv_patch_i8", OWN: families(kernels)[0]}.get(route, "pad_rows_i8") == families(launched)[0], launched
     want = oracle_eval(make())[0].reshape(-1)
     assert_bit_exact(got[0][offset:offset + want.size], want, wl.name)
     assert np.all(got[0][:offset] == 0x55) and np.all(got[0][offset + want.size:] == 0x55), "bytes around the result"

@@ -143,6 +143,7 @@ def _time_us(device, blob, wl, busy_ms=0.0):
     lens = [a.nbytes for a in wl.inputs] + [o.nbytes for o in outs]
     try:
         kernel = exe.op_kernels()[-1]
+        assert exe.launch_kernels() == exe.op_kernels()
         exe.time_device(ptrs, lens, 30)  # caches in the state every later pass finds them in
         # a card that has idled (while the host built the workload) takes some 100 ms of work to reach the clocks it sustains
         t0 = time.perf_counter()
@@ -168,6 +169,7 @@ def test_chosen_tile_is_within_a_tenth_of_the_best(device, row, monkeypatch):
     a few microseconds differ by on this card."""
     name, addressing, M, N, K, C, _, tile = row
     wl = _workload(row)
+    monkeypatch.setenv("THIP_PLAIN_RECORDS", "1")  # the tiles themselves: small ops have a kernel without them
     switch = "THIP_IGEMM_DENSE_VARIANT" if addressing == DENSE else "THIP_WINDOW_VARIANT"
     monkeypatch.delenv(switch, raising=False)
     chosen_blob = wl.program.serialize()

@@ -82,6 +82,7 @@ struct thip_executable_t {
     // thip_executable_enqueue_noalloc: where each record's scratch (a K-split workspace) sits in the static array,
     // and the program's total
     std::vector<Step> steps;             // the launches of a dispatch, in order
+    std::vector<std::string> launchNames;  // their kernels
     std::vector<uint8_t *> stepBuffers;  // two per step: operands of space kSpacePlan (null: none)
     std::vector<uint64_t> scratchOffset;
     uint64_t scratchBytes = 0;
@@ -806,9 +807,12 @@ static thip_status_t addStep(thip_executable_t *e, Step &&planned, bool *taken) 
     }
     uint8_t *placeholder[64];
     for (auto &ptr : placeholder) ptr = (uint8_t *)(uintptr_t)0x1000000;
-    char name[96];
+    char name[96] = "";
     *taken = launchStep(e, step, placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name)}) == THIP_OK;
-    if (!*taken) {
+    if (*taken) {
+        if (step.kind == kStepPadded) e->launchNames.push_back("pad_rows_i8");
+        e->launchNames.push_back(name[0] ? name : opKernelName(e->ops[step.first]));
+    } else {
         (void)hipGetLastError();
         for (int k = 0; k < 2; k++) {
             if (uint8_t *p = e->stepBuffers.back()) (void)hipFree(p);
@@ -1093,6 +1097,19 @@ thip_status_t thip_executable_op_kernel(thip_executable_t *e, uint32_t index, ch
     if (!e || !name || capacity == 0) return fail(THIP_INVALID_ARGUMENT, "null argument");
     if (index >= e->header.op_count) return fail(THIP_OUT_OF_RANGE, "op %u of %u", index, e->header.op_count);
     snprintf(name, capacity, "%s", e->kernelNames[index].c_str());
+    return THIP_OK;
+}
+
+thip_status_t thip_executable_launch_count(thip_executable_t *e, uint32_t *out_count) {
+    if (!e || !out_count) return fail(THIP_INVALID_ARGUMENT, "null argument");
+    *out_count = (uint32_t)e->launchNames.size();
+    return THIP_OK;
+}
+
+thip_status_t thip_executable_launch_kernel(thip_executable_t *e, uint32_t index, char *name, size_t capacity) {
+    if (!e || !name || capacity == 0) return fail(THIP_INVALID_ARGUMENT, "null argument");
+    if (index >= e->launchNames.size()) return fail(THIP_OUT_OF_RANGE, "launch %u of %zu", index, e->launchNames.size());
+    snprintf(name, capacity, "%s", e->launchNames[index].c_str());
     return THIP_OK;
 }
 

@@ -48,7 +48,8 @@ EXPORTED_SYMBOLS = [
     "thip_device_set_event_log", "thip_device_set_dump_dirs", "thip_device_mfma_rate", "thip_device_stream_floor", "thip_device_stream_floor_tuned", "thip_infer_format", "thip_descriptor_validate", "thip_descriptor_info", "thip_descriptor_binding", "thip_descriptor_segment",
     "thip_executable_create", "thip_executable_destroy", "thip_executable_run",
     "thip_executable_enqueue", "thip_executable_enqueue_noalloc", "thip_executable_wait", "thip_executable_set_wait_timeout", "thip_executable_time", "thip_executable_time_rotating",
-    "thip_executable_op_count", "thip_executable_op_kernel", "thip_executable_binding_count",
+    "thip_executable_op_count", "thip_executable_op_kernel",
+    "thip_executable_launch_count", "thip_executable_launch_kernel", "thip_executable_binding_count",
     "thip_executable_binding_size",
 ]
 
@@ -303,6 +304,8 @@ def lib():
     L.thip_executable_time_rotating.argtypes = [vp, P(DispatchState), u32, i32, P(ctypes.c_float)]
     L.thip_executable_op_count.argtypes = [vp, P(u32)]
     L.thip_executable_op_kernel.argtypes = [vp, u32, ctypes.c_char_p, sz]
+    L.thip_executable_launch_count.argtypes = [vp, P(u32)]
+    L.thip_executable_launch_kernel.argtypes = [vp, u32, ctypes.c_char_p, sz]
     L.thip_executable_binding_count.argtypes = [vp, P(u32)]
     L.thip_executable_binding_size.argtypes = [vp, u32, P(sz)]
     _lib = L
@@ -444,15 +447,23 @@ class Executable:
             ccount = self._constants.size
         check(lib().thip_executable_create(device.handle, blob, len(blob), cptr, ccount, ctypes.byref(self._h)))
 
-    def op_kernels(self):
+    def _kernel_names(self, count, name):
         n = ctypes.c_uint32()
-        check(lib().thip_executable_op_count(self._h, ctypes.byref(n)))
+        check(count(self._h, ctypes.byref(n)))
         names = []
         for i in range(n.value):
             buf = ctypes.create_string_buffer(64)
-            check(lib().thip_executable_op_kernel(self._h, i, buf, 64))
+            check(name(self._h, i, buf, 64))
             names.append(buf.value.decode())
         return names
+
+    def op_kernels(self):
+        """The kernel that each op has of its own (thip_executable_op_kernel)."""
+        return self._kernel_names(lib().thip_executable_op_count, lib().thip_executable_op_kernel)
+
+    def launch_kernels(self):
+        """The kernels that a dispatch launches, in order (thip_executable_launch_kernel)."""
+        return self._kernel_names(lib().thip_executable_launch_count, lib().thip_executable_launch_kernel)
 
     def binding_sizes(self):
         n = ctypes.c_uint32()
