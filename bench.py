@@ -124,7 +124,7 @@ def decoder_row(pkg, dev, batch, pre_ms, check):
     o.precondition(pre_ms)
     o.run(5)
     ms = min(o.run(20) for _ in range(3))
-    names = o.exe.op_kernels()
+    names = o.exe.launch_kernels()
     row = {"ms": round(ms, 4), "steps_per_s": round(1e3 / ms, 1), "tokens_per_s": round(batch * 1e3 / ms, 1), "kernels": len(names),
            "scope": "linears + attention matmuls + residual adds + vocabulary projection only", "weight_bytes": o.wl.attrs["weight_bytes"],
            "GB/s": round(o.wl.attrs["weight_bytes"] / (ms * 1e-3) / 1e9, 1), "frac": round(o.wl.attrs["weight_bytes"] / (ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 5),
@@ -214,12 +214,21 @@ MEASURED_TRAFFIC = {
 }
 
 
-def traffic_still_valid(name):
-    """Whether the kernel sources behind workload `name` are the ones its MEASURED_TRAFFIC entry was read on."""
-    family = "thip_igemm.hip" if name.startswith(("fc_", "conv")) else "thip_bandwidth.hip"
+# Where the kernels of these workloads live.
+KERNEL_SOURCES = {"igemm_direct_i8": "thip_igemm_direct.hip", "conv_patch_i8": "thip_conv_patch.hip", "igemm": "thip_igemm.hip", "fc_skinny": "thip_igemm.hip"}
+
+
+def main_kernel(exe):
+    """The kernel of a one-op program: what its dispatch launches behind copies of its operands."""
+    return [k for k in exe.launch_kernels() if not k.startswith(("transpose", "pad_rows"))][0]
+
+
+def traffic_still_valid(kernel):
+    """Whether the kernel's sources are the ones that the MEASURED_TRAFFIC entries were read on."""
+    family = next((source for name, source in KERNEL_SOURCES.items() if kernel.startswith(name)), "thip_bandwidth.hip")
     for source in ("thip_kernels_common.h", family):
         with open(os.path.join(ROOT, "torq-compiler_amd", "csrc", source), "rb") as f:
-            if hashlib.sha256(f.read()).hexdigest() != TRAFFIC_SOURCES_SHA256[source]:
+            if hashlib.sha256(f.read()).hexdigest() != TRAFFIC_SOURCES_SHA256.get(source):
                 return False
     return True
 
@@ -234,8 +243,8 @@ STREAM_SHAPES = {
 }
 
 
-def roofline(wl, bound, ms, name=None):
-    traffic = MEASURED_TRAFFIC.get(name) if name in MEASURED_TRAFFIC and traffic_still_valid(name) else None
+def roofline(wl, bound, ms, name, kernel):
+    traffic = MEASURED_TRAFFIC.get(name) if name in MEASURED_TRAFFIC and traffic_still_valid(kernel) else None
     traffic = None if traffic is None else int(round(traffic))
     if bound == "mfma":
         achieved = wl.ops / (ms * 1e-3) / 1e12
@@ -409,7 +418,7 @@ def mfma_calibration(pkg, dev, wl, args):
         o = Loaded(pkg, dev, pkg.workloads.fully_connected_workload(M, K, N, zeros=zeros))
         o.run(args.warmup)
         ms = leg(label, lambda: o.run(args.steps))
-        out[label] = {"us": round(ms * 1e3, 2), "TOP/s": round(o.wl.ops / (ms * 1e-3) / 1e12, 1), "kernel": o.exe.op_kernels()[0]}
+        out[label] = {"us": round(ms * 1e3, 2), "TOP/s": round(o.wl.ops / (ms * 1e-3) / 1e12, 1), "kernel": main_kernel(o.exe)}
         o.close()
     out["gemm_over_mfma_only_random"] = round(out["gemm_random_data"]["TOP/s"] / out["mfma_only_random_operands"], 3)
     if args.library_gemm:
@@ -499,7 +508,8 @@ def main():
     make, bound = table[args.workload]
     wl = make()
     loaded = Loaded(pkg, dev, wl)
-    kernels = loaded.exe.op_kernels()
+    kernels = loaded.exe.launch_kernels()
+    kernel = main_kernel(loaded.exe)
     pre_ms = max(0.0, args.precondition_ms)
     loaded.precondition(pre_ms)
     if args.warmup > 0:
@@ -546,8 +556,7 @@ def main():
             o.precondition(pre_ms)
             o.run(5)
             warm = min(o.run(50) for _ in range(3))  # best of three: 50 dispatches of a 3 us kernel are over before a hiccup of the host's is
-            names = o.exe.op_kernels()
-            row = {"kernel": names[-1 if "transpose" in names[0] else 0], "bound": bnd}
+            row = {"kernel": main_kernel(o.exe), "bound": bnd}
             if bnd == "hbm":
                 # what the roofline fraction is quoted on: operands cold in every dispatch; the repeated dispatch of one
                 # buffer set (served by the last-level cache where it fits) is reported next to it
@@ -563,7 +572,7 @@ def main():
             else:
                 ms = warm
                 row["us"] = round(ms * 1e3, 2)
-            r = roofline(o.wl, bnd, ms, name)
+            r = roofline(o.wl, bnd, ms, name, row["kernel"])
             row.update({"GOP/s": round(o.wl.ops / (ms * 1e-3) / 1e9, 1), "GB/s": round(o.wl.bytes / (ms * 1e-3) / 1e9, 1), "frac": r["frac"]})
             if r["traffic"] is not None:
                 row["traffic"] = r["traffic"]  # HBM bytes per launch from the rocprofv3 counters (MEASURED_TRAFFIC)
@@ -587,7 +596,7 @@ def main():
                 check = pkg.workloads.mobilenet_v2_workload(batch=min(batch, 4))  # same seed: same weights, first images
                 same = bool(np.array_equal(o.output()[:min(batch, 4)], oracle_network(check)))
             mbv2["batch_%d" % batch] = {"ms": round(ms, 4), "images_per_s": round(batch / (ms * 1e-3), 1),
-                                       "GOP/s": round(o.wl.ops / (ms * 1e-3) / 1e9, 1), "kernels": len(o.exe.op_kernels()),
+                                       "GOP/s": round(o.wl.ops / (ms * 1e-3) / 1e9, 1), "kernels": len(o.exe.launch_kernels()),
                                        "parity_checked": same}
             ok = ok and same if same is not None else ok
             o.close()
@@ -615,7 +624,7 @@ def main():
         "config": {"workload": args.workload, "kernels": kernels, "parity_checked": ok,
                    "algorithmic_ops": wl.ops, "algorithmic_bytes": wl.bytes, "buffer_sets": main_sets,
                    "clock_preconditioning_ms": pre_ms},
-        "roofline": dict(roofline(wl, bound, ev_ms, args.workload), kernel=kernels[0], kernel_ms=round(ev_ms, 5)),
+        "roofline": dict(roofline(wl, bound, ev_ms, args.workload, kernel), kernel=kernel, kernel_ms=round(ev_ms, 5)),
     }
     if not args.no_cpu and args.workload.startswith("fc_"):
         result["cpu_baseline"] = cpu_baseline(wl)
