@@ -34,3 +34,18 @@ def test_padded(device, make, tmp_path):
     finally:
         device.set_event_log(None)
     assert_bit_exact(got[0], want, wl.name + " record by record")
+
+
+@pytest.mark.parametrize("make", [lambda: w.fully_connected_workload(300, 333, 520, realistic=True), lambda: w.conv2d_workload(N=1, H=17, W=13, C=53, O=148, realistic=True)], ids=["linear", "conv"])
+def test_without_memory_for_the_padded_operands(device, make, monkeypatch):
+    """The rows padded to whole chunks and the weights spread to match want memory that the op's own kernel does not: where there is too
+    little the op runs by that."""
+    wl = make()
+    print("[gpu-case]", wl.name, flush=True)
+    want = oracle_eval(wl)[0]
+    for room, padded in ((0, False), (16 * 1024, False), (64 << 20, True)):
+        monkeypatch.setenv("THIP_STEP_BYTES", str(room))
+        launched = []
+        got, kernels = run_on_gpu(device, wl, via="device", launched=launched)
+        assert ("pad_rows_i8" in launched) == padded and (padded or launched == kernels), launched
+        assert_bit_exact(got[0], want, "%s, %d bytes" % (wl.name, room))

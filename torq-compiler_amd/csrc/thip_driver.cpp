@@ -791,36 +791,39 @@ void thip_executable_destroy(thip_executable_t *e) {
     delete e;
 }
 
-// Adds a launch to the executable's, with the buffers of its own that it needs.  It is asked for its kernels now, as the records were; one
-// that its launchers do not take is left out again (*taken), for its records to run one by one.
-static thip_status_t addStep(thip_executable_t *e, Step &&planned, bool *taken) {
+// Adds a launch to the executable's, with the buffers of its own that it needs.  It is asked for its kernels now, as the records were.  False:
+// its launchers do not take it, or there is no memory for its buffers; its records, which need none, then run one by one.
+static bool addStep(thip_executable_t *e, Step &&planned) {
     e->steps.push_back(std::move(planned));
     e->stepBuffers.insert(e->stepBuffers.end(), 2, nullptr);
     Step &step = e->steps.back();
+    hipError_t err = hipSuccess;
     if (step.kind == kStepPadded) {
         uint8_t **buffers = &e->stepBuffers[e->stepBuffers.size() - 2];
-        hipError_t err = hipMalloc((void **)&buffers[0], (size_t)step.rows * step.to);
+        const size_t rows = (size_t)step.rows * step.to, bytes = rows + step.constants.size();
+        if (e->tuning.stepBytes >= 0 && (long long)bytes > e->tuning.stepBytes) err = hipErrorOutOfMemory;
+        if (err == hipSuccess) err = hipMalloc((void **)&buffers[0], rows);
         if (err == hipSuccess) err = hipMalloc((void **)&buffers[1], step.constants.size());
         if (err == hipSuccess) err = hipMemcpy(buffers[1], step.constants.data(), step.constants.size(), hipMemcpyHostToDevice);
-        if (err != hipSuccess) return hipFail(err, "allocating a step's operands");
         std::vector<uint8_t>().swap(step.constants);
     }
-    uint8_t *placeholder[64];
-    for (auto &ptr : placeholder) ptr = (uint8_t *)(uintptr_t)0x1000000;
-    char name[96] = "";
-    *taken = launchStep(e, step, placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name)}) == THIP_OK;
-    if (*taken) {
-        if (step.kind == kStepPadded) e->launchNames.push_back("pad_rows_i8");
-        e->launchNames.push_back(name[0] ? name : opKernelName(e->ops[step.first]));
-    } else {
-        (void)hipGetLastError();
-        for (int k = 0; k < 2; k++) {
-            if (uint8_t *p = e->stepBuffers.back()) (void)hipFree(p);
-            e->stepBuffers.pop_back();
+    if (err == hipSuccess) {
+        uint8_t *placeholder[64];
+        for (auto &ptr : placeholder) ptr = (uint8_t *)(uintptr_t)0x1000000;
+        char name[96] = "";
+        if (launchStep(e, step, placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name)}) == THIP_OK) {
+            if (step.kind == kStepPadded) e->launchNames.push_back("pad_rows_i8");
+            e->launchNames.push_back(name[0] ? name : opKernelName(e->ops[step.first]));
+            return true;
         }
-        e->steps.pop_back();
     }
-    return THIP_OK;
+    (void)hipGetLastError();
+    for (int k = 0; k < 2; k++) {
+        if (uint8_t *p = e->stepBuffers.back()) (void)hipFree(p);
+        e->stepBuffers.pop_back();
+    }
+    e->steps.pop_back();
+    return false;
 }
 
 thip_status_t thip_executable_create(thip_device_t *device, const void *blob, size_t size, const uint32_t *constants,
@@ -896,18 +899,21 @@ thip_status_t thip_executable_create(thip_device_t *device, const void *blob, si
             e->kernelNames[i] = name[0] ? name : opKernelName(e->ops[i]);
         }
     }
-    for (Step &step : planSteps(viewOf(e), e->tuning.plainRecords)) {
+    std::vector<Step> planned;
+    try {
+        planned = planSteps(viewOf(e), e->tuning.plainRecords);
+    } catch (const std::bad_alloc &) {  // no room on the host to lay a launch's operands out
+        planned = planSteps(viewOf(e), true);
+    }
+    for (Step &step : planned) {
         const uint32_t first = step.first, count = step.count;
-        bool taken = false;
-        if (thip_status_t st = addStep(e, std::move(step), &taken)) return bail(st);
-        for (uint32_t i = first; !taken && i < first + count; i++) {
+        if (addStep(e, std::move(step))) continue;
+        for (uint32_t i = first; i < first + count; i++) {
             Step record{};
             record.kind = kStepRecord;
             record.first = i;
             record.count = 1;
-            bool ran = false;
-            if (thip_status_t st = addStep(e, std::move(record), &ran)) return bail(st);
-            if (!ran) return bail(fail(THIP_INTERNAL, "op %u (%s): no kernel takes it", i, e->kernelNames[i].c_str()));
+            if (!addStep(e, std::move(record))) return bail(fail(THIP_INTERNAL, "op %u (%s): no kernel takes it", i, e->kernelNames[i].c_str()));
         }
     }
     *out_executable = e;

@@ -216,8 +216,8 @@ std::vector<Step> planSteps(const DescriptorView &v, bool plain) {
         }
         const DescOp *op = s.kind == kStepRecord ? &v.ops[i] : s.kind == kStepPadded ? &s.op : nullptr;
         s.route = !plain && op && op->kind == kKindIgemm ? igemmRoute(v, *op) : kIgemmOwnTile;
-        steps.push_back(s);
         i += s.count;
+        steps.push_back(std::move(s));
     }
     return steps;
 }
