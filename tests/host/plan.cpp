@@ -23,6 +23,6 @@ int main(int argc, char **argv) {
     const DescriptorView v{blob.data(), h, (const DescOp *)(blob.data() + h.ops_offset), (const DescBinding *)(blob.data() + h.bindings_offset),
                            (const DescTemp *)(blob.data() + h.temps_offset), (const DescConst *)(blob.data() + h.consts_offset)};
     const char *kinds[] = {"record", "ir_expand_dw_i8", "padded", "igemm_rt_i8"}, *routes[] = {"", " igemm_direct_i8", " conv_patch_i8"};
-    for (const Step &s : planSteps(v, false)) printf("%s %u %u%s\n", kinds[s.kind], s.first, s.count, routes[s.route]);
+    for (const Step &s : planSteps(v, tuningFromEnvironment())) printf("%s %u %u%s\n", kinds[s.kind], s.first, s.count, routes[s.route]);
     return 0;
 }

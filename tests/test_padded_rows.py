@@ -19,7 +19,8 @@ pytestmark = pytest.mark.gpu
     lambda: w.conv2d_workload(N=2, H=12, W=12, C=40, O=24, KH=1, KW=1, stride=(2, 2), pad=(0, 0, 0, 0), realistic=True),
     lambda: w.conv2d_workload(N=1, H=20, W=20, C=200, O=300, KH=5, KW=5, pad=(2, 2, 2, 2)),
 ], ids=range(14))
-def test_padded(device, make, tmp_path):
+def test_padded(device, make, tmp_path, monkeypatch):
+    monkeypatch.setenv("THIP_PAD_ROWS", "1")
     wl = make()
     print("[gpu-case]", wl.name, flush=True)
     want = oracle_eval(wl)[0]
@@ -43,6 +44,7 @@ def test_without_memory_for_the_padded_operands(device, make, monkeypatch):
     wl = make()
     print("[gpu-case]", wl.name, flush=True)
     want = oracle_eval(wl)[0]
+    monkeypatch.setenv("THIP_PAD_ROWS", "1")
     for room, padded in ((0, False), (16 * 1024, False), (64 << 20, True)):
         monkeypatch.setenv("THIP_STEP_BYTES", str(room))
         launched = []

@@ -39,7 +39,7 @@ def batched():
 SMALL_LINEAR = lambda: w.fully_connected_workload(40, 64, 48, realistic=True)  # noqa: E731
 SMALL_CONV = lambda: w.conv2d_workload(N=1, H=12, W=12, C=64, O=32, realistic=True)  # noqa: E731
 PATCH_CONV = lambda: w.conv2d_workload(N=16, H=56, W=56, C=96, O=96, realistic=True)  # noqa: E731
-PADDED = lambda: w.fully_connected_workload(100000, 24, 128, realistic=True)  # noqa: E731
+PADDED = lambda: w.fully_connected_workload(100000, 25, 128, realistic=True)  # noqa: E731
 DIRECT, PATCH, OWN = "record 0 1 igemm_direct_i8", "record 0 1 conv_patch_i8", "record 0 1"
 CASES = [
     (SMALL_LINEAR, 4, DIRECT), (SMALL_LINEAR, 1, OWN), (SMALL_LINEAR, 2, OWN), (SMALL_LINEAR, 7, OWN), (SMALL_CONV, 8, DIRECT), (SMALL_CONV, 2, OWN),
@@ -70,6 +70,19 @@ def test_route_by_offset(plan, make, offset, want):
 
 def test_route_of_a_batch(plan):
     assert plan(batched()) == ["record 0 1 igemm_direct_i8", "record 1 1"]
+
+
+RAGGED = [
+    (lambda: w.fully_connected_workload(1500, 1333, 48), True), (lambda: w.fully_connected_workload(60, 776, 256), True), (lambda: w.fully_connected_workload(200000, 17, 16), True),
+    (lambda: w.conv2d_workload(N=1, H=7, W=7, C=33, O=64), True), (lambda: w.conv2d_workload(N=16, H=56, W=56, C=13, O=24, KH=5, KW=5, pad=(2, 2, 2, 2)), True),
+    (lambda: w.fully_connected_workload(60, 24, 64), False), (lambda: w.fully_connected_workload(30000, 72, 40), False), (lambda: w.conv2d_workload(N=1, H=112, W=112, C=8, O=32), False),
+    (lambda: w.conv2d_workload(N=32, H=112, W=112, C=40, O=32, stride=(2, 2)), False), (lambda: w.conv2d_workload(N=4, H=56, W=56, C=264, O=96, KH=1, KW=1, stride=(2, 2), pad=(0, 0, 0, 0)), False),
+]
+
+
+@pytest.mark.parametrize("make,padded", RAGGED, ids=[c[0]().name for c in RAGGED])
+def test_ragged_channels_are_padded_where_that_is_measured_ahead(plan, make, padded):
+    assert [s.split()[0] for s in plan(make())] == ["padded" if padded else "record"]
 
 
 @pytest.mark.gpu

@@ -274,6 +274,7 @@ Tuning tuningFromEnvironment() {
     for (const char *name : {"THIP_IGEMM_VARIANT", "THIP_IGEMM_DENSE_VARIANT", "THIP_WINDOW_VARIANT", "THIP_NO_WINDOW_RING", "THIP_NO_DIRECT_EPILOGUE", "THIP_PLAIN_RECORDS"}) {
         t.plainRecords = t.plainRecords || flag(name);
     }
+    t.padRows = digit("THIP_PAD_ROWS", -1);
     if (const char *v = getenv("THIP_STEP_BYTES")) t.stepBytes = atoll(v);
     t.noFcDeep = flag("THIP_NO_FC_DEEP");
     t.noFcWide = flag("THIP_NO_FC_WIDE");

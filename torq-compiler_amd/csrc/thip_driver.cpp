@@ -901,9 +901,11 @@ thip_status_t thip_executable_create(thip_device_t *device, const void *blob, si
     }
     std::vector<Step> planned;
     try {
-        planned = planSteps(viewOf(e), e->tuning.plainRecords);
+        planned = planSteps(viewOf(e), e->tuning);
     } catch (const std::bad_alloc &) {  // no room on the host to lay a launch's operands out
-        planned = planSteps(viewOf(e), true);
+        Tuning plain = e->tuning;
+        plain.plainRecords = true;
+        planned = planSteps(viewOf(e), plain);
     }
     for (Step &step : planned) {
         const uint32_t first = step.first, count = step.count;

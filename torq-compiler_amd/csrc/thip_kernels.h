@@ -42,6 +42,7 @@ struct Tuning {
     bool noK128 = false;            // THIP_NO_K128: no 128-byte k-tiles chosen at launch (the emitter reads the same switch for its own choice)
     bool noFcDeep = false;          // THIP_NO_FC_DEEP
     bool plainRecords = false;      // a switch asks for a tile or a loader by name: every record runs by its own launcher
+    int padRows = -1;               // THIP_PAD_ROWS=0 / 1: rows of ragged channels padded for the kernels of aligned operands never / wherever these take them (-1: by cost)
     long long stepBytes = -1;       // THIP_STEP_BYTES: device memory that a launch may take for operands of its own (negative: what there is); records run where it is short
     bool noFcWide = false;          // THIP_NO_FC_WIDE
     bool addGeneric = false;        // THIP_ADD_GENERIC: the quantised add always through the 64-bit ACT stage

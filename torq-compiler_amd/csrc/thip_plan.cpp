@@ -142,16 +142,35 @@ static bool matchExpandDw(const DescriptorView &v, const std::vector<uint32_t> &
     return true;
 }
 
+// Whether the copy of the rows and a kernel of aligned operands behind it are ahead of a record's own gather kernel, by the time that
+// either takes (us; storing the results costs both the same).  A k-tile of 64 costs the gather 0.55, 0.85, 1.5 or 2.5 in pieces of 8, 4, 2 or
+// 1 bytes and the aligned kernels 0.09, both more where the tiles outnumber the CUs; the copy is a launch (2.3) and its bytes at
+// 4.2 TB/s.  Fitted to 429 linears and convolutions of 3 .. 8004 channels and 4 .. 204 800 rows; the choice costs 1.5 % of the better
+// one's time over them, always padding 9 %.  Padded / own:
+//   taken   1500x1333 -> 48 7.8 / 65.4, 4096x500 -> 1024 9.3 / 16.6, 60x776 -> 256 6.0 / 10.2, 200000x17 -> 16 8.7 / 20.4,
+//           3x3 7x7x33 -> 64 5.5 / 15.4, 28x28x100 -> 64 6.3 / 15.6, 56x56x13 -> 24 by 5x5, batch 16 11.5 / 27.5
+//   left    60x24 -> 64 5.4 / 3.2, 30000x72 -> 40 9.7 / 5.3, 100000x776 -> 64 44.0 / 39.0, 3x3 112x112x8 -> 32 6.3 / 4.3,
+//           stride 2 112x112x40 -> 32, batch 32 22.3 / 15.6, 1x1 stride 2 56x56x264 -> 96, batch 4 7.3 / 5.9
+//   wrong   30000x130 -> 40 11.2 / 9.5 (taken), 100000x500 -> 64 29.7 / 37.9, pointwise 56x56x24 -> 96, batch 32 9.6 / 14.4 (left)
+static bool paddingPays(const DescOp &g, int64_t rows, int64_t Cp, int64_t K) {
+    auto tilesOf = [](int64_t n) { return (double)((n + 63) / 64); };
+    const double tiles = tilesOf(g.M) * tilesOf(g.Nn), beyond = tiles > 256 ? tiles - 256 : 0;
+    const double step = g.gran >= 8 ? 0.55 : g.gran >= 4 ? 0.85 : g.gran >= 2 ? 1.5 : 2.5;
+    const double own = 2.8 + step * tilesOf(g.K) * (1 + beyond / 600);
+    const double padded = 5.1 + 0.24e-6 * (double)rows * (double)(g.C + Cp) + 0.09 * tilesOf(K) * (1 + beyond / 170);
+    return padded + 0.8 < own;
+}
+
 // A convolution, fully_connected or matmul over a channel count that is no multiple of 16.  Its own kernel gathers the
-// operand in the pieces that divide the channels, down to single bytes (1429 rows of K = 1333: 65 us); with every row
-// padded to whole chunks the kernels of aligned operands take it (one copy of the input, 2-5 us, and 4-5 us), the packed
-// weights spread to match, with zeros against the padding.
-static bool matchPadded(const DescriptorView &v, uint32_t first, Step *s) {
+// operand in the pieces that divide the channels, down to single bytes; with every row padded to whole chunks the kernels of
+// aligned operands take it, the packed weights spread to match, with zeros against the padding.
+static bool matchPadded(const DescriptorView &v, const Tuning &tuning, uint32_t first, Step *s) {
     const DescOp &g = v.ops[first];
     if (g.kind != kKindIgemm || g.loader != kLoaderGather || g.in1.space != kSpaceNone || g.weights.space != kSpaceConst || g.C % 16 == 0) return false;
     const bool pointwise = g.KH == 1 && g.KW == 1 && g.SH == 1 && g.SW == 1 && g.PT == 0 && g.PL == 0 && g.OH == g.H && g.OW == g.W;
     const int64_t C = g.C, Cp = roundUp(C, 16), taps = (int64_t)g.KH * g.KW, rows = (int64_t)g.N * g.H * g.W, K = taps * Cp, N = g.Nn;
     if (g.K != taps * C || g.Kp < g.K || g.PT < 0 || g.PL < 0 || rows * Cp >= (1LL << 31) || K >= (1LL << 31)) return false;
+    if (tuning.padRows >= 0 ? tuning.padRows == 0 : !paddingPays(g, rows, Cp, K)) return false;
     DescOp op = g;
     op.C = (int32_t)Cp;
     op.K = (int32_t)K;
@@ -204,12 +223,13 @@ static IgemmRoute igemmRoute(const DescriptorView &v, const DescOp &op) {
     return igemmDirectBetter(a) ? kIgemmDirect : convPatchBetter(a) ? kIgemmPatch : kIgemmOwnTile;
 }
 
-std::vector<Step> planSteps(const DescriptorView &v, bool plain) {
+std::vector<Step> planSteps(const DescriptorView &v, const Tuning &tuning) {
+    const bool plain = tuning.plainRecords;
     const std::vector<uint32_t> uses = tempUses(v);
     std::vector<Step> steps;
     for (uint32_t i = 0; i < v.header.op_count;) {
         Step s{};
-        if (plain || (!matchExpandDw(v, uses, i, &s) && !matchMatmulRt(v, uses, i, &s) && !matchPadded(v, i, &s))) {
+        if (plain || (!matchExpandDw(v, uses, i, &s) && !matchMatmulRt(v, uses, i, &s) && !matchPadded(v, tuning, i, &s))) {
             s.kind = kStepRecord;
             s.first = i;
             s.count = 1;

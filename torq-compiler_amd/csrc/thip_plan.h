@@ -78,8 +78,8 @@ IgemmArgs igemmArgs(const DescriptorView &v, const DescOp &op, At &&at) {
 
 // The launches of a dispatch in order.  Every record belongs to exactly one step; a step that stands for several leaves
 // the intermediates between them unwritten, so it is only formed where no other record reads them.
-// `plain`: one step per record, by the record's own kernel.  Routes are settled here, on all that their launchers ask: a dispatch's
+// tuning.plainRecords: one step per record, by the record's own kernel.  Routes are settled here, on all that their launchers ask: a dispatch's
 // buffers start at 16-byte boundaries, so the offsets say how its operands are aligned.
-std::vector<Step> planSteps(const DescriptorView &view, bool plain);
+std::vector<Step> planSteps(const DescriptorView &view, const Tuning &tuning);
 
 }  // namespace thip
