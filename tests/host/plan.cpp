@@ -1,5 +1,5 @@
 // The launches that the library plans for a serialised program (the file in argv[1]), one a line: what it is, its records, and the
-// kernel of a GEMM-shaped record.
+// kernel of a GEMM-shaped record; then whether dispatches on buffers that come back are replayed as a graph.
 #include <stdio.h>
 
 #include <vector>
@@ -22,7 +22,9 @@ int main(int argc, char **argv) {
     if (n != blob.size() || validateWhole(blob.data(), blob.size(), &h) != THIP_OK) return 3;
     const DescriptorView v{blob.data(), h, (const DescOp *)(blob.data() + h.ops_offset), (const DescBinding *)(blob.data() + h.bindings_offset),
                            (const DescTemp *)(blob.data() + h.temps_offset), (const DescConst *)(blob.data() + h.consts_offset)};
+    const std::vector<Step> steps = planSteps(v, tuningFromEnvironment());
     const char *kinds[] = {"record", "ir_expand_dw_i8", "padded", "igemm_rt_i8"}, *routes[] = {"", " igemm_direct_i8", " conv_patch_i8"};
-    for (const Step &s : planSteps(v, tuningFromEnvironment())) printf("%s %u %u%s\n", kinds[s.kind], s.first, s.count, routes[s.route]);
+    for (const Step &s : steps) printf("%s %u %u%s\n", kinds[s.kind], s.first, s.count, routes[s.route]);
+    puts(replayPays(steps.size(), h.total_size - h.data_offset) ? "replayed" : "one by one");
     return 0;
 }

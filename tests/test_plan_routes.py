@@ -7,7 +7,7 @@ import pytest
 
 import desc_interp
 from helpers import assert_bit_exact, families, host_check, oracle_eval, run_on_gpu
-from torq_compiler_amd import workloads as w
+from torq_compiler_amd import Program, workloads as w
 
 
 class Moved:
@@ -58,7 +58,9 @@ def plan(tmp_path_factory):
         path.write_bytes(bytes(wl.program.serialize()))
         done = subprocess.run([exe, str(path)], stdout=subprocess.PIPE, text=True, timeout=120)
         assert done.returncode == 0
-        return done.stdout.splitlines()
+        lines = done.stdout.splitlines()
+        steps.replayed = lines.pop() == "replayed"
+        return lines
 
     return steps
 
@@ -70,6 +72,25 @@ def test_route_by_offset(plan, make, offset, want):
 
 def test_route_of_a_batch(plan):
     assert plan(batched()) == ["record 0 1 igemm_direct_i8", "record 1 1"]
+
+
+def chain(blocks, channels):
+    """3x3 convolutions one behind the other: 9 * channels^2 bytes of weights each."""
+    p = Program()
+    rng = np.random.default_rng(5)
+    wt = rng.integers(-127, 128, size=(channels, channels, 3, 3)).astype(np.int8)
+    mult, shift = w.quantize_multiplier(np.full(channels, 60 / (np.sqrt(channels * 9) * 5400)))
+    sb, sf = w.derive_scale_bias(mult, shift, np.zeros(channels, dtype=np.int64), wt, 0)
+    h = p.binding(0, (1, 14, 14, channels))
+    for i in range(blocks):
+        init = dict(init=p.binding(1, (1, 14, 14, channels))) if i == blocks - 1 else {}
+        h = p.conv2d(h, wt, sb, nhwc_input=True, input_zp=0, output_zp=0, output_min=-128, output_max=127, shift_factor=sf, pad=(1, 1, 1, 1), stride=(1, 1), **init)
+    return w.Workload("chain", p, [], [], 0, 0, {})
+
+
+@pytest.mark.parametrize("blocks,channels,replayed", [(3, 256, False), (6, 256, False), (40, 256, False), (41, 256, True), (54, 256, True), (4, 64, True), (3, 64, False)])
+def test_long_programs_and_short_ones_of_little_weight_are_replayed(plan, blocks, channels, replayed):
+    assert len(plan(chain(blocks, channels))) == blocks and plan.replayed == replayed
 
 
 RAGGED = [

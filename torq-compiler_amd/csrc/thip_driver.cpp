@@ -554,13 +554,6 @@ static thip_status_t enqueueOps(thip_executable_t *e, uint8_t *const *bp) {
     return THIP_OK;
 }
 
-constexpr uint32_t kGraphMinOps = 4;
-// A replay starts some 3 us later than a launch behind another, and saves the host 3 us per launch.  Launches that stream weights take
-// the device longer than that, so the host stays ahead and a short program of them is faster launch by launch: a decoder's step of 7
-// launches 33.7 us against 36.3 replayed, of 13 launches 65.6 against 69.0.  Beyond kGraphLongOps launches the 3 us are below one
-// per cent and the host's time decides; an image network's 37 launches (95 KB of constants each) take 141 us replayed, 151 one by one.
-constexpr uint32_t kGraphLongOps = 64;
-constexpr uint64_t kGraphStreamedBytes = 256 * 1024;
 // Sets of binding pointers with a graph of their own.  A caller that prepares its next inputs while a dispatch runs rotates over
 // two or three; with one graph only, every dispatch of such a caller was launched kernel by kernel (MobileNetV2, one image, three
 // sets: 151 us, the host's launches; 142 replayed).
@@ -579,8 +572,7 @@ static void dropReplay(thip_executable_t::Replay *r) {
 // Enqueues one dispatch on device bindings, through the set's graph when there is one.
 static thip_status_t enqueueDevice(thip_executable_t *e, uint8_t *const *bp) {
     const uint32_t nb = e->header.binding_count;
-    const bool streams = e->steps.size() < kGraphLongOps && e->header.total_size - e->header.data_offset >= e->steps.size() * kGraphStreamedBytes;
-    const bool eligible = !e->graphsDisabled && e->steps.size() >= kGraphMinOps && !streams && !e->device->eventLog && e->device->dumpBuffersDir.empty();
+    const bool eligible = !e->graphsDisabled && replayPays(e->steps.size(), e->header.total_size - e->header.data_offset) && !e->device->eventLog && e->device->dumpBuffersDir.empty();
     if (!eligible) return enqueueOps(e, bp);
     thip_executable_t::Replay *r = nullptr, *oldest = nullptr;
     for (auto &x : e->replays) {

@@ -223,6 +223,17 @@ static IgemmRoute igemmRoute(const DescriptorView &v, const DescOp &op) {
     return igemmDirectBetter(a) ? kIgemmDirect : convPatchBetter(a) ? kIgemmPatch : kIgemmOwnTile;
 }
 
+// A replay starts about 5 us later than a launch behind another, and costs the host 12 - 20 us in place of 3 per launch.  Launches that
+// stream weights take the device longer than that, so the host stays ahead and the program is faster launch by launch, by the same 5 us
+// whatever its length: decoder steps of 7, 13, 25 and 37 launches 25.6 / 30.8, 48.1 / 53.7, 91.6 / 97.6 and 135.4 / 141.1 us (one by
+// one / replayed; 2.4 MB of weights each), chains of 6, 18 and 30 convolutions 30.4 / 33.9, 92.4 / 97.2 and 154.2 / 158.9 (370 KB).
+// At 48 convolutions that is 1.5 % (246.6 / 250.5) for 123 us of the host's time in place of 17: beyond 40 launches the replay is taken
+// again.  An image network's 37 launches (95 KB each) take 141 us replayed, 151 one by one.
+bool replayPays(size_t launches, uint64_t constantBytes) {
+    const bool streams = constantBytes >= launches * 256 * 1024;
+    return launches >= 4 && !(streams && launches <= 40);
+}
+
 std::vector<Step> planSteps(const DescriptorView &v, const Tuning &tuning) {
     const bool plain = tuning.plainRecords;
     const std::vector<uint32_t> uses = tempUses(v);

@@ -82,4 +82,7 @@ IgemmArgs igemmArgs(const DescriptorView &v, const DescOp &op, At &&at) {
 // buffers start at 16-byte boundaries, so the offsets say how its operands are aligned.
 std::vector<Step> planSteps(const DescriptorView &view, const Tuning &tuning);
 
+// Whether a dispatch of so many launches is worth a graph; `constantBytes`: what all of them read of weights.
+bool replayPays(size_t launches, uint64_t constantBytes);
+
 }  // namespace thip
