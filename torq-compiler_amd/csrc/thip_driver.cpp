@@ -75,6 +75,13 @@ struct thip_executable_t {
         uint64_t lastUse = 0;            // the invocation
     };
     std::vector<Replay> replays;
+    // Graphs that made room for others, until the event behind their last replay says that they are done.
+    struct Retired {
+        hipGraph_t graph;
+        hipGraphExec_t exec;
+        hipEvent_t done;
+    };
+    std::vector<Retired> retired;
     bool graphsDisabled = false;
     uint64_t invocation = 0;             // dispatches so far (the event log's invocation_id)
     Tuning tuning;                       // the environment's switches as they were when the executable was created
@@ -569,6 +576,40 @@ static void dropReplay(thip_executable_t::Replay *r) {
     r->graph = nullptr;
 }
 
+// Frees the graphs put aside whose last replay is done; `all`: the caller knows that the stream is idle.
+static void freeRetired(thip_executable_t *e, bool all) {
+    size_t kept = 0;
+    for (auto &r : e->retired) {
+        if (!all && hipEventQuery(r.done) != hipSuccess) {
+            (void)hipGetLastError();  // not-ready is no error
+            e->retired[kept++] = r;
+            continue;
+        }
+        (void)hipGraphExecDestroy(r.exec);
+        (void)hipGraphDestroy(r.graph);
+        (void)hipEventDestroy(r.done);
+    }
+    e->retired.resize(kept);
+}
+
+// Makes an unused set's entry free for another, without waiting: replays of its graph may still be on the stream, so the graph is put
+// aside behind an event.  False where as many graphs as are kept lie there already.
+static bool retireReplay(thip_executable_t *e, thip_executable_t::Replay *r) {
+    if (!r->exec) return true;  // dispatched once, eagerly
+    freeRetired(e, false);
+    if (e->retired.size() >= kGraphsKept) return false;
+    hipEvent_t done = nullptr;
+    if (hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess || hipEventRecord(done, e->stream) != hipSuccess) {
+        (void)hipGetLastError();
+        if (done) (void)hipEventDestroy(done);
+        return false;
+    }
+    e->retired.push_back({r->graph, r->exec, done});
+    r->graph = nullptr;
+    r->exec = nullptr;
+    return true;
+}
+
 // Enqueues one dispatch on device bindings, through the set's graph when there is one.
 static thip_status_t enqueueDevice(thip_executable_t *e, uint8_t *const *bp) {
     const uint32_t nb = e->header.binding_count;
@@ -586,10 +627,7 @@ static thip_status_t enqueueDevice(thip_executable_t *e, uint8_t *const *bp) {
         if (e->replays.size() < kGraphsKept) {
             e->replays.emplace_back();
             r = &e->replays.back();
-        } else if (e->invocation - oldest->lastUse > kReplayMaxAge) {
-            // its last replay lies behind this many later dispatches, but nothing says that they are done
-            THIP_HIP(hipStreamSynchronize(e->stream), "hipStreamSynchronize");
-            dropReplay(oldest);
+        } else if (e->invocation - oldest->lastUse > kReplayMaxAge && retireReplay(e, oldest)) {
             r = oldest;
         }
         if (r) {
@@ -766,6 +804,7 @@ void thip_executable_destroy(thip_executable_t *e) {
     }
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     for (auto &r : e->replays) dropReplay(&r);
+    freeRetired(e, true);
     for (uint8_t *p : e->tempPtrs) {
         if (p) (void)hipFree(p);
     }
