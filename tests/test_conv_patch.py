@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
     dict(N=6, H=100, W=100, C=80, O=48, pad=(0, 0, 0, 0), input_zp=-90, output_min=-128), dict(N=40, H=34, W=40, C=16, O=16, KH=5, KW=5, pad=(4, 4, 4, 4)),
     dict(N=20, H=51, W=50, C=24, O=48, realistic=True),  # channels padded to 32 on the way
 ], ids=lambda kw: "x".join(str(v) for v in kw.values()))
-def test_conv_patch(device, kw):
+def test_conv_patch(device, kw, monkeypatch):
+    monkeypatch.setenv("THIP_PAD_ROWS", "1")
     wl = w.conv2d_workload(**kw)
     print("[gpu-case]", wl.name, flush=True)
     want = oracle_eval(wl)[0]
