@@ -5,7 +5,7 @@
 namespace thip {
 
 // ---------------------------------------------------------------------------
-// conv_patch_i8: a workgroup of eight waves keeps all weights of the convolution in LDS and walks over strips of output rows of an
+// conv_patch_i8 (stride 1): a workgroup of eight waves keeps all weights of the convolution in LDS and walks over strips of output rows of an
 // image: the strip's input pixels, padding in place, go to LDS; a wave then takes 64 output pixels by all NB * 32 channels at a time,
 // both MFMA operands read from LDS, a tap being an offset from the pixel's place in the patch.
 //
@@ -68,7 +68,7 @@ __global__ __launch_bounds__(512) void conv_patch_i8(IgemmArgs p, ConvPatchPlan 
         const int image = strip / q.stripsPerImage, oy0 = (strip - image * q.stripsPerImage) * q.rows;
         const int rows = p.OH - oy0 < q.rows ? p.OH - oy0 : q.rows;
         const int8_t *x = p.A + (size_t)image * p.H * p.W * p.C;
-        const int chunks = ((rows - 1) * p.SH + p.KH) * q.cols * pixelChunks;
+        const int chunks = (rows - 1 + p.KH) * q.cols * pixelChunks;
         __syncthreads();  // the strip before has been read
         for (int i0 = tid; i0 < chunks; i0 += 512 * 8) {
             v4i v[8];
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(512) void conv_patch_i8(IgemmArgs p, ConvPatchPlan 
                 const int i = i0 + 512 * u < chunks ? i0 + 512 * u : chunks - 1;
                 const int pixel = (int)fastDiv((uint32_t)i, divPixel), c = i - pixel * pixelChunks;
                 const int row = (int)fastDiv((uint32_t)pixel, divCols);
-                const int iy = oy0 * p.SH - p.PT + row, ix = pixel - row * q.cols - p.PL;
+                const int iy = oy0 - p.PT + row, ix = pixel - row * q.cols - p.PL;
                 inside[u] = (unsigned)iy < (unsigned)p.H && (unsigned)ix < (unsigned)p.W;
                 at[u] = pixel * q.pixelPitch + c * 16;
                 v[u] = *(const v4i *)(x + (inside[u] ? (uint32_t)((iy * p.W + ix) * p.C + c * 16) : 0u));
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(512) void conv_patch_i8(IgemmArgs p, ConvPatchPlan 
                 int m = t * 64 + 32 * i + fr;
                 m = m < pixels ? m : pixels - 1;
                 const int oy = (int)fastDiv((uint32_t)m, divOW), ox = m - oy * p.OW;
-                base[i] = patch + (oy * p.SH * q.cols + ox * p.SW) * q.pixelPitch;
+                base[i] = patch + (oy * q.cols + ox) * q.pixelPitch;
             }
             const int8_t *wbase = weights + fr * q.weightPitch + 16 * half;
             v16i acc[2][NB];
@@ -190,11 +190,11 @@ static bool planConvPatch(const IgemmArgs &a, ConvPatchPlan *q) {
     q->steps = K64 / 32;
     q->weightPitch = paddedPitch(K64);
     q->pixelPitch = paddedPitch(a.C);
-    const long long cols = (long long)(a.OW - 1) * a.SW + a.KW, fixed = (long long)nb * 32 * (q->weightPitch + 8) + K64 / 16 * 4;
+    const long long cols = (long long)a.OW - 1 + a.KW, fixed = (long long)nb * 32 * (q->weightPitch + 8) + K64 / 16 * 4;
     const long long rowBytes = cols * q->pixelPitch, room = (long long)kPatchMaxLds - fixed;
     if (cols > 65536 || rowBytes * a.KH > room) return false;
     q->cols = (int)cols;
-    long long most = (room / rowBytes - a.KH) / a.SH + 1;
+    long long most = room / rowBytes - a.KH + 1;
     if (most > a.OH) most = a.OH;
     // a strip per CU where the images give as many
     long long strips = (a.OH + most - 1) / most;
@@ -205,7 +205,7 @@ static bool planConvPatch(const IgemmArgs &a, ConvPatchPlan *q) {
     const long long all = images * q->stripsPerImage;
     if (all > 0x3fffffff) return false;
     q->strips = (int)all;
-    q->patchBytes = (int)(((long long)(q->rows - 1) * a.SH + a.KH) * rowBytes);
+    q->patchBytes = (int)((q->rows - 1 + a.KH) * rowBytes);
     q->lds = (size_t)(fixed + q->patchBytes);
     return true;
 }
