@@ -36,8 +36,8 @@ __device__ __forceinline__ uint32_t packBf16(float lo, float hi) {
 // KG groups of waves share a workgroup's outputs and take every KG-th k-tile each, with a ring of their own; their sums
 // meet in LDS (few tiles under a long K: more loads in flight per CU).
 //
-// Bound by what L2 delivers to a CU (64 KiB per k-tile of a 256 x 256 tile in 1.1 us, 0.86 us of MFMA work), with the launch,
-// the ring fill and 28 MB of output at the end next to it: 2048 x 1152 -> 6912 takes 34.4 us (950 TFLOP/s).  Eight waves
+// Bound by the ring's data path (64 KiB per k-tile of a 256 x 256 tile in 1.1 us, 58 KB/us per CU where LDS-DMA loads alone, of lines in
+// the XCD's L2, reach 138; 0.86 us of MFMA work), with the launch, the ring fill and 28 MB of output at the end next to it: 2048 x 1152 -> 6912 takes 34.4 us (950 TFLOP/s).  Eight waves
 // on the 256 x 256 tile rather than four: 35.7 -> 34.4 us, and the epilogue of a short K 13.0 -> 9.1.
 // ---------------------------------------------------------------------------
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, int KG, bool FRAG>
@@ -339,10 +339,9 @@ static hipError_t launchTileChoice(const FcBf16Args &a, int choice, const Launch
 }
 
 // Which tile, or 0 for the streaming kernel: the smallest estimate, in us, of a fixed part (launch, ring fill, epilogue)
-// plus rounds of 256 workgroups times k-tiles times what a CU takes per k-tile.  A CU is fed 60 to 80 KB/us whatever it
-// does with the bytes, so that a k-tile costs by its (BM + BN) * 128 bytes.  Fitted to 80 shapes (33 .. 4096 rows, K 72 ..
-// 6912, 128 .. 8192 columns), all of which take a tile within a fifth of their best; some of them, us on the streaming
-// kernel / 64 / 64 two groups / 128 / 128 deep / 256:
+// plus rounds of 256 workgroups times k-tiles times what a CU takes per k-tile: 0.2, 0.47 and 1.2 us for 16, 32 and 64 KB.
+// Fitted to 80 shapes (33 .. 4096 rows, K 72 .. 6912, 128 .. 8192 columns), all of which take a tile within a fifth of their best; some
+// of them, us on the streaming kernel / 64 / 64 two groups / 128 / 128 deep / 256:
 //   2048 x 1152 -> 6912  154.8 /  53 /  54 / 39.9 / 49.1 / 34.4      1024 x 1152 -> 6912  80.8 / 28.9 / 30 / 21.4 / 24.3 / 28.6
 //    512 x 6912 -> 1152   58.7 / 25.3 / 21.9 / 62.8 / 44.6 / 123      128 x 4096 -> 128    7.2 / 16.0 / 13.1 / 27.0 / 27.5 / 72
 //     64 x 256 -> 640      6.0 /  3.7 /  3.9 /  5.5 /  5.5 / 9       4096 x 256 -> 256     9.6 /  4.0 /  4.2 / 5.6 / 5.9 / 11.3

@@ -10,7 +10,8 @@ namespace thip {
 // both MFMA operands read from LDS, a tap being an offset from the pixel's place in the patch.
 //
 // Why: the ring kernel addresses the window in memory, so a 3x3 convolution brings every pixel from L2 into LDS nine times, and a tile
-// column of 128 brings and multiplies 128 channels where there are 96. Both go at what L2 delivers (11 TB/s for the chip).
+// column of 128 brings and multiplies 128 channels where there are 96 (56x56x96 -> 96, 32 images: 130 MB through LDS, 19.0 us; here 34
+// MB and 15.3).
 //
 // What is left is serial in a workgroup, mostly one to a CU: weights and patch into LDS, the MFMA steps, the epilogue.
 //
