@@ -48,8 +48,9 @@ def families(kernels):
     return [k.split("<")[0] for k in kernels]
 
 
-def host_check(name, directory):
-    """Builds tests/host/<name>.cpp against the package's library with the host compiler; returns the program's path."""
+def host_check(name, directory, sanitize=()):
+    """Builds tests/host/<name>.cpp against the package's library with the host compiler, with the library's `sanitize` sources (none of
+    them calls HIP) under the sanitizers; returns the program's path."""
     import os
     import shutil
     import subprocess
@@ -60,8 +61,10 @@ def host_check(name, directory):
     gxx = shutil.which("g++")
     assert gxx, "g++ is needed for the host check"
     exe = os.path.join(str(directory), name)
-    built = subprocess.run([gxx, "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + os.path.join(root, "torq-compiler_amd", "csrc"),
-                            os.path.join(root, "tests", "host", name + ".cpp"), runtime.LIB_PATH, "-Wl,-rpath," + os.path.dirname(runtime.LIB_PATH),
+    csrc = os.path.join(root, "torq-compiler_amd", "csrc")
+    flags = ["-g", "-fsanitize=address,undefined", "-static-libasan", "-fno-sanitize-recover=undefined"] if sanitize else []
+    built = subprocess.run([gxx, "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + csrc] + flags +
+                           [os.path.join(root, "tests", "host", name + ".cpp")] + [os.path.join(csrc, s) for s in sanitize] + [runtime.LIB_PATH, "-Wl,-rpath," + os.path.dirname(runtime.LIB_PATH),
                             "-Wl,--allow-shlib-undefined", "-o", exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     assert built.returncode == 0, built.stdout[-3000:]
     return exe

@@ -1,5 +1,6 @@
 """Which kernel a dispatch takes for a GEMM-shaped op follows the alignment of its result too: results at every offset that the op's
 own kernel stores at, planned on the host and run on the GPU against the oracle."""
+import os
 import subprocess
 
 import numpy as np
@@ -72,6 +73,23 @@ def test_route_by_offset(plan, make, offset, want):
 
 def test_route_of_a_batch(plan):
     assert plan(batched()) == ["record 0 1 igemm_direct_i8", "record 1 1"]
+
+
+def test_mutated_descriptors_are_planned(tmp_path):
+    """What the validation lets through is planned without a report of the sanitizers, every record in one launch."""
+    from test_inverted_residual import block
+    exe = host_check("plan_fuzz", tmp_path, sanitize=["thip_plan.cpp", "thip_validate.cpp", "thip_status.cpp"])
+    programs = [w.conv2d_workload(N=1, H=9, W=9, C=3, O=8, realistic=True), w.conv2d_workload(N=1, H=8, W=8, C=24, O=16, realistic=True), w.conv2d_workload(N=1, H=8, W=8, C=32, O=16, realistic=True),
+                w.fully_connected_workload(40, 72, 20, realistic=True), w.matmul_workload(2, 9, 61, 37), batched(), w.mobilenet_v2_workload(batch=1, resolution=32, classes=10, width=0.25),
+                w.grouped_linear_workload(mode="residual", K=256, N=256), w.pointwise_add_workload(N=1, H=7, W=7, C=96, O=32), block(N=2, H=8, W=8, C=16, E=32, stride=2),
+                block(N=2, H=8, W=8, C=3, E=32, stride=1, first=(3, 1, (1, 1, 1, 1)))]
+    files = []
+    for i, wl in enumerate(programs):
+        files.append(tmp_path / ("blob%d" % i))
+        files[-1].write_bytes(bytes(wl.program.serialize()))
+    env = dict(os.environ, ASAN_OPTIONS="verify_asan_link_order=0:detect_leaks=0", UBSAN_OPTIONS="print_stacktrace=1")
+    run = subprocess.run([exe, "600"] + [str(f) for f in files], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=env, timeout=300)
+    assert run.returncode == 0 and run.stdout.startswith("planned "), run.stdout[-3000:]
 
 
 def chain(blocks, channels):

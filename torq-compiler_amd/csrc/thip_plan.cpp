@@ -118,7 +118,7 @@ static bool matchMatmulRt(const DescriptorView &v, const std::vector<uint32_t> &
 }
 
 // Whether the requant of a record has a tail of 32-bit arithmetic (see WideRequant).
-static bool narrowRequant(const DescOp &op) { return op.shift == 32 || op.shift + op.pre_shift >= 33; }
+static bool narrowRequant(const DescOp &op) { return op.shift == 32 || (int64_t)op.shift + op.pre_shift >= 33; }
 
 // A pointwise convolution, or one over few channels, whose only reader is the 3 x 3 depthwise convolution right behind it.
 static bool matchExpandDw(const DescriptorView &v, const std::vector<uint32_t> &uses, uint32_t first, Step *s) {
