@@ -72,7 +72,7 @@ def test_a_new_set_does_not_wait_for_the_old_ones(device):
             longest = max(dispatch(k, times) for k, times in sets)
             exe.wait()
             total = time.perf_counter() - t0
-            assert longest < 0.25 * total, "%s: one call of %.1f ms, %.1f ms in all" % (what, longest * 1e3, total * 1e3)
+            assert longest < 0.4 * total, "%s: one call of %.1f ms, %.1f ms in all" % (what, longest * 1e3, total * 1e3)
     finally:
         exe.close()
         device.free(pin)
