@@ -1,0 +1,167 @@
+"""A decoder's step as one launch (dec_chain): which programs take it, each op against the oracle on the inputs the GPU gave it at the sizes where
+the kernel can go wrong, a launch whose workgroups give up waiting, executables in turn, and buffers that share memory."""
+import subprocess
+
+import numpy as np
+import pytest
+
+import torq_compiler_amd as thip
+from helpers import host_check
+from oracle import programs as prog
+from torq_compiler_amd import workloads as w
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    exe = host_check("plan", tmp_path_factory.mktemp("plan"))
+
+    def run(blob, env=None):
+        path = tmp_path_factory.mktemp("blob") / "p.thip"
+        path.write_bytes(blob)
+        return subprocess.run([exe, str(path)], check=True, stdout=subprocess.PIPE, text=True, env=env).stdout.splitlines()
+
+    return run
+
+
+STEP = dict(layers=2, hidden=256, heads=2, head_dim=64, ffn=512, vocab=512, cache_len=64)
+
+
+@pytest.mark.parametrize("case,chained", [
+    (dict(), True), (dict(batch=4), True), (dict(expose=True), True), (dict(batch=5), False),
+    # the input rows of one phase cost more than the launches saved (chainPays)
+    (dict(batch=4, hidden=384, heads=8, head_dim=256, ffn=6272), False), (dict(heads=8, head_dim=256, cache_len=4096), False),
+], ids=str)
+def test_planned_where_it_pays(plan, case, chained):
+    blob = w.decoder_step_workload(**dict(dict(batch=1), **dict(STEP, **case))).program.serialize()
+    lines = plan(blob)
+    assert (lines[0] == "dec_chain 0 13") == chained, lines
+    assert all(l.startswith("record ") for l in plan(blob, env={"THIP_DEC_CHAIN": "0"})[:-1])
+
+
+def test_weights_written_by_the_program_are_not_fetched_ahead(plan):
+    """A matmul whose second operand an earlier one made ends the chain in front of it."""
+    p = thip.Program()
+    zero, none = np.zeros(1, np.float32), dict(output_zp=0, output_min=w.NO_CLAMP[0], output_max=w.NO_CLAMP[1], shift=0)
+    x = p.binding(0, (1, 4, 64), np.uint16)
+    caches = p.binding(1, (4, 64, 64), np.uint16)
+    y = x
+    for i in range(4):
+        y = p.matmul(y, p.transpose(p.view(caches, (1, 64, 64), i * 4096), (0, 2, 1)), zero, **none)
+    made = p.matmul(y, p.transpose(p.view(caches, (1, 64, 64), 0), (0, 2, 1)), zero, **none)  # [1, 4, 64]
+    p.matmul(y, p.transpose(made, (0, 2, 1)), zero, init=p.binding(2, (1, 4, 4), np.uint16), **none)
+    lines = plan(p.serialize(), env={"THIP_DEC_CHAIN": "1"})
+    assert lines[:2] == ["dec_chain 0 5", "record 5 1"], lines
+
+
+# ---- GPU ----------------------------------------------------------------------------------------------------------
+
+SHAPES = [
+    dict(batch=1, layers=2, vocab=4096),                                                          # the benchmark's widths
+    dict(batch=2, layers=1, vocab=4096), dict(batch=3, layers=1, vocab=4096), dict(batch=4, layers=2, vocab=4096),
+    # eleven k-blocks in two halves per tile, the last half empty; columns of a matmul that fill no tile, K that fills no unit
+    dict(batch=1, layers=2, hidden=256, heads=2, head_dim=64, ffn=1408, vocab=48, cache_len=24),
+    dict(batch=3, layers=2, hidden=128, heads=2, head_dim=64, ffn=1408, vocab=16, cache_len=8),
+    dict(batch=2, layers=1, hidden=256, heads=16, head_dim=64, ffn=256, vocab=64, cache_len=200),   # sixteen rows of a matmul
+    dict(batch=4, layers=1, hidden=256, heads=1, head_dim=128, ffn=8192, vocab=16384, cache_len=136),  # several passes and blocks a phase
+    dict(batch=1, layers=1, hidden=1280, heads=8, head_dim=128, ffn=1536, vocab=1024, cache_len=2056),
+]
+
+
+def _id(c):
+    return "-".join("%s%s" % (k, v) for k, v in c.items())
+
+
+def _load(device, wl):
+    exe = thip.Executable(device, wl.program.serialize())
+    assert exe.launch_kernels()[0] == "dec_chain", exe.launch_kernels()
+    return exe
+
+
+def _buffers(device, wl):
+    arrays = list(wl.inputs) + [np.full(s, 0x55, dtype=d) for s, d in wl.outputs]
+    return [device.upload(a) for a in arrays], [a.nbytes for a in arrays]
+
+
+def _outputs(device, wl, ptrs):
+    return [device.download(ptrs[len(wl.inputs) + i], s, d) for i, (s, d) in enumerate(wl.outputs)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wait", [None, "0"], ids=["together", "given_up"])
+@pytest.mark.parametrize("case", SHAPES, ids=_id)
+def test_gpu_every_op(device, monkeypatch, case, wait):
+    """wait 0: every workgroup gives up at its first wait, and the last one makes everything by itself."""
+    monkeypatch.setenv("THIP_DEC_CHAIN", "1")
+    if wait is not None:
+        monkeypatch.setenv("THIP_DEC_CHAIN_WAIT", wait)
+    wl = w.decoder_step_workload(expose=True, **case)
+    print("[gpu-case]", wl.name, _id(case), wait, flush=True)
+    exe = _load(device, wl)
+    ptrs, lens = _buffers(device, wl)
+    try:
+        first = None
+        for _ in range(3):
+            exe.run_device(ptrs, lens)
+            outs = _outputs(device, wl, ptrs)
+            if first is None:
+                prog.check_decoder_step(wl, outs, prog.assert_bf16_close, prog.assert_bit_exact)
+                first = outs
+            assert all(np.array_equal(a, b) for a, b in zip(outs, first))
+    finally:
+        exe.close()
+        for q in ptrs:
+            device.free(q)
+
+
+@pytest.mark.gpu
+def test_gpu_new_inputs_and_executables_in_turn(device, monkeypatch):
+    """Two executables, two sets of buffers each, enqueued one behind the other without a wait: every dispatch leaves what one alone leaves."""
+    monkeypatch.setenv("THIP_DEC_CHAIN", "1")
+    wls = [w.decoder_step_workload(batch=1, seed=s, **STEP) for s in (3, 4)] + [w.decoder_step_workload(batch=2, seed=s, **STEP) for s in (5, 6)]
+    print("[gpu-case]", [x.name for x in wls], flush=True)
+    exes = [_load(device, wls[0]), _load(device, wls[2])]
+    sets = [_buffers(device, x) for x in wls]
+    try:
+        def alone(k):
+            exes[k // 2].run_device(*sets[k])
+            return _outputs(device, wls[k], sets[k][0])
+
+        want = [alone(k) for k in range(4)]
+        for _ in range(10):
+            for k in (0, 2, 1, 3, 0, 1, 2, 3):
+                exes[k // 2].enqueue_device(*sets[k])
+            for e in exes:
+                e.wait()
+            for k in range(4):
+                assert all(np.array_equal(a, b) for a, b in zip(_outputs(device, wls[k], sets[k][0]), want[k])), k
+    finally:
+        for e in exes:
+            e.close()
+        for ptrs, _ in sets:
+            for q in ptrs:
+                device.free(q)
+
+
+@pytest.mark.gpu
+def test_gpu_results_written_into_the_caches(device, monkeypatch):
+    """A caller that has the new keys appended to its cache in place: the scores read them, as when every op is a launch of its own."""
+    wl = w.decoder_step_workload(batch=1, **STEP)
+    print("[gpu-case]", wl.name, "in place", flush=True)
+    results = []
+    for chain in ("1", "0"):
+        monkeypatch.setenv("THIP_DEC_CHAIN", chain)
+        exe = thip.Executable(device, wl.program.serialize())
+        assert (exe.launch_kernels()[0] == "dec_chain") == (chain == "1")
+        ptrs, lens = _buffers(device, wl)
+        try:
+            at = ptrs[1] + wl.inputs[1].nbytes // 2  # layer 1's cache; its scores come after every new key
+            exe.run_device(ptrs[:4] + [at] + ptrs[5:], lens)
+            keys = device.download(ptrs[1], wl.inputs[1].shape, np.uint16)
+            outs = _outputs(device, wl, ptrs)
+            results.append([outs[0], outs[2], keys])
+        finally:
+            exe.close()
+            for q in ptrs:
+                device.free(q)
+    assert all(np.array_equal(a, b) for a, b in zip(*results))
+    assert not np.array_equal(results[0][2], wl.inputs[1])

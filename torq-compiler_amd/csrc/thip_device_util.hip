@@ -280,6 +280,8 @@ Tuning tuningFromEnvironment() {
     t.noFcWide = flag("THIP_NO_FC_WIDE");
     t.maxpoolGeneric = flag("THIP_MAXPOOL_GENERIC");
     t.addGeneric = flag("THIP_ADD_GENERIC");
+    t.decChain = digit("THIP_DEC_CHAIN", -1);
+    if (const char *v = getenv("THIP_DEC_CHAIN_WAIT")) t.decChainWait = atoll(v) > 0 ? atoll(v) : 0;
     if (const char *v = getenv("THIP_DEC_SPLIT")) t.decSplit = atoi(v) >= 2 ? 2 : atoi(v) == 1 ? 1 : 0;
     if (const char *v = getenv("THIP_DEC_ABLATE")) t.decAblate = atoi(v);
     if (const char *v = getenv("THIP_DEC_TARGET_WORKGROUPS")) t.decTargetGroups = atoi(v);

@@ -42,6 +42,7 @@ struct thip_device_t {
     std::mutex logMutex;
     FILE *eventLog = nullptr;
     std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
+    int computeUnits = 0;
     uint8_t *staticScratch = nullptr;    // this GPU's copy of the library's scratch array (kStaticScratchBytes)
     // dump directories (empty: off): bindings of every blocking dispatch / every buffer a kernel record wrote
     std::string dumpIoDir, dumpBuffersDir;
@@ -90,10 +91,23 @@ struct thip_executable_t {
     // and the program's total
     std::vector<Step> steps;             // the launches of a dispatch, in order
     std::vector<std::string> launchNames;  // their kernels
-    std::vector<uint8_t *> stepBuffers;  // two per step: operands of space kSpacePlan (null: none)
+    std::vector<uint8_t *> stepBuffers;  // two per step: operands of space kSpacePlan; or the table and the counters of a chain (null: none)
+    bool chained = false;                // a step's workgroups wait for one another (kStepDecChain)
     std::vector<uint64_t> scratchOffset;
     uint64_t scratchBytes = 0;
 };
+
+// The workgroups of a launch that wait for one another need a CU each at the same time.  Two such launches at once could each hold
+// CUs that the other waits for, so the executables of a device take turns: a dispatch on another stream than the last one's starts behind it.
+struct ChainTurn {
+    std::mutex mutex;
+    hipStream_t last = nullptr;
+    hipEvent_t event = nullptr;
+};
+static ChainTurn &chainTurn(int ordinal) {
+    static ChainTurn turns[64];
+    return turns[ordinal & 63];
+}
 
 static thip_status_t hipFail(hipError_t e, const char *what) {
     const thip_status_t code = e == hipErrorOutOfMemory ? THIP_RESOURCE_EXHAUSTED : THIP_INTERNAL;
@@ -481,6 +495,17 @@ static thip_status_t dumpOpOutput(thip_executable_t *e, uint32_t i, uint8_t *con
     return THIP_OK;
 }
 
+// Whether a binding that the program writes shares bytes with another one.  A chain fetches its inputs ahead, so it does not take these.
+static bool chainAliased(const thip_executable_t *e, uint8_t *const *bp) {
+    for (uint32_t i = 0; i < e->header.binding_count; i++) {
+        if (!(e->bindings[i].flags & kBindingWritten)) continue;
+        for (uint32_t j = 0; j < e->header.binding_count; j++) {
+            if (j != i && e->bindings[j].flags != 0 && bp[i] < bp[j] + e->bindings[j].size && bp[j] < bp[i] + e->bindings[i].size) return true;
+        }
+    }
+    return false;
+}
+
 // Launches one step: a record by its own launcher, a run of records by the kernel that does them as a whole.
 static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr) {
     hipError_t err = hipSuccess;
@@ -529,6 +554,26 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
         uint8_t *const *buffers = &e->stepBuffers[2 * (size_t)(&s - e->steps.data())];
         err = launchPadRows((const int8_t *)resolve(e, e->ops[s.first].in0, bp), (int8_t *)buffers[0], s.rows, s.from, s.to, ctx);
         if (err == hipSuccess) return launchOp(e, s.first, s.op, bp, ctx, scratch, buffers, s.route);
+        break;
+    }
+    case kStepDecChain: {
+        if (!ctx.name && chainAliased(e, bp)) {
+            for (uint32_t i = s.first; i < s.first + s.count; i++) {
+                if (thip_status_t st = launchOp(e, i, e->ops[i], bp, ctx, scratch)) return st;
+            }
+            return THIP_OK;
+        }
+        uint8_t *const *buffers = &e->stepBuffers[2 * (size_t)(&s - e->steps.data())];
+        DecChainArgs a;
+        memset(&a, 0, sizeof(a));
+        a.phases = (const ChainPhase *)buffers[0];
+        a.sync = (uint32_t *)buffers[1];
+        a.count = (int32_t)s.count;
+        a.xRoom = s.xRoom;
+        a.redRoom = s.redRoom;
+        a.waitTicks = (uint64_t)e->tuning.decChainWait;
+        for (uint32_t i = 0; i < e->header.binding_count && i < 64; i++) a.bindings[i] = bp[i];
+        err = launchDecChain(a, e->device->computeUnits, ctx);
         break;
     }
     default: return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch, nullptr, s.route);
@@ -610,8 +655,24 @@ static bool retireReplay(thip_executable_t *e, thip_executable_t::Replay *r) {
     return true;
 }
 
+// Makes a dispatch of an executable with a chain wait for the last one of another.  `turn`: held until the dispatch is enqueued.
+static thip_status_t takeChainTurn(thip_executable_t *e, std::unique_lock<std::mutex> *turn) {
+    if (!e->chained) return THIP_OK;
+    ChainTurn &t = chainTurn(e->device->ordinal);
+    *turn = std::unique_lock<std::mutex>(t.mutex);
+    if (t.last && t.last != e->stream) {
+        if (!t.event) THIP_HIP(hipEventCreateWithFlags(&t.event, hipEventDisableTiming), "hipEventCreate");
+        THIP_HIP(hipEventRecord(t.event, t.last), "hipEventRecord");
+        THIP_HIP(hipStreamWaitEvent(e->stream, t.event, 0), "hipStreamWaitEvent");
+    }
+    t.last = e->stream;
+    return THIP_OK;
+}
+
 // Enqueues one dispatch on device bindings, through the set's graph when there is one.
 static thip_status_t enqueueDevice(thip_executable_t *e, uint8_t *const *bp) {
+    std::unique_lock<std::mutex> turn;
+    if (thip_status_t s = takeChainTurn(e, &turn)) return s;
     const uint32_t nb = e->header.binding_count;
     const bool eligible = !e->graphsDisabled && replayPays(e->steps.size(), e->header.total_size - e->header.data_offset) && !e->device->eventLog && e->device->dumpBuffersDir.empty();
     if (!eligible) return enqueueOps(e, bp);
@@ -679,6 +740,7 @@ thip_status_t thip_device_create(int32_t ordinal, thip_device_t **out_device) {
     if (!d) return fail(THIP_RESOURCE_EXHAUSTED, "out of memory");
     d->ordinal = ordinal;
     d->arch = arch;
+    d->computeUnits = prop.multiProcessorCount;
     {
         // the address of this device's copy of the scratch array (the device is current)
         void *ptr = nullptr;
@@ -803,6 +865,11 @@ void thip_executable_destroy(thip_executable_t *e) {
         }
     }
     if (e->stream) (void)hipStreamSynchronize(e->stream);
+    if (e->chained) {
+        ChainTurn &t = chainTurn(e->device->ordinal);
+        std::lock_guard<std::mutex> turn(t.mutex);
+        if (t.last == e->stream) t.last = nullptr;
+    }
     for (auto &r : e->replays) dropReplay(&r);
     freeRetired(e, true);
     for (uint8_t *p : e->tempPtrs) {
@@ -837,6 +904,22 @@ static bool addStep(thip_executable_t *e, Step &&planned) {
         if (err == hipSuccess) err = hipMalloc((void **)&buffers[1], step.constants.size());
         if (err == hipSuccess) err = hipMemcpy(buffers[1], step.constants.data(), step.constants.size(), hipMemcpyHostToDevice);
         std::vector<uint8_t>().swap(step.constants);
+    }
+    if (step.kind == kStepDecChain) {
+        uint8_t **buffers = &e->stepBuffers[e->stepBuffers.size() - 2];
+        // operands that are no bindings lie where they will stay
+        auto at = [e](const DescRef &r) { return r.space == kSpaceBinding ? ((ChainRef)(r.index + 1) << 56) | r.offset : (ChainRef)(uintptr_t)resolve(e, r, nullptr); };
+        const Chain chain = layoutChain(viewOf(e), step.first, step.count, e->device->computeUnits, at);
+        if (chain.phases.size() != step.count) err = hipErrorInvalidValue;
+        step.xRoom = chain.xRoom;
+        step.redRoom = chain.redRoom;
+        const size_t tableBytes = chain.phases.size() * sizeof(ChainPhase), syncBytes = 4 * (kChainSyncHead + chain.exchangeWords);
+        if (e->tuning.stepBytes >= 0 && (long long)(tableBytes + syncBytes) > e->tuning.stepBytes) err = hipErrorOutOfMemory;
+        if (err == hipSuccess) err = hipMalloc((void **)&buffers[0], tableBytes);
+        if (err == hipSuccess) err = hipMalloc((void **)&buffers[1], syncBytes);
+        if (err == hipSuccess) err = hipMemcpy(buffers[0], chain.phases.data(), tableBytes, hipMemcpyHostToDevice);
+        if (err == hipSuccess) err = hipMemset(buffers[1], 0, syncBytes);
+        if (err == hipSuccess) e->chained = true;
     }
     if (err == hipSuccess) {
         uint8_t *placeholder[64];
@@ -988,7 +1071,12 @@ static thip_status_t runLocked(thip_executable_t *e, const thip_dispatch_state_t
         if (e->bindings[i].flags != 0 && !(st->binding_flags && (st->binding_flags[i] & THIP_BINDING_DEVICE))) allDevice = false;
     }
     logEvent(e, e->invocation, 0, "DISPATCH_EXECUTE_ACTIONS", "BEGIN", "");
-    if (thip_status_t s = allDevice ? enqueueDevice(e, bp) : enqueueOps(e, bp)) {
+    auto enqueueStaged = [&] {
+        std::unique_lock<std::mutex> turn;
+        const thip_status_t s = takeChainTurn(e, &turn);
+        return s != THIP_OK ? s : enqueueOps(e, bp);
+    };
+    if (thip_status_t s = allDevice ? enqueueDevice(e, bp) : enqueueStaged()) {
         // what was enqueued before the failure still runs: wait for it (bounded; the launch error is what is reported)
         std::string message = thip_status_message();
         if (!e->abandoned) (void)waitBounded(e, "waiting after a failed launch");
@@ -1053,7 +1141,8 @@ thip_status_t thip_executable_enqueue_noalloc(thip_executable_t *e, const thip_d
     uint8_t *bp[64] = {nullptr};
     for (uint32_t i = 0; i < e->header.binding_count; i++) bp[i] = (uint8_t *)st->binding_ptrs[i];
     const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0};
-    thip_status_t result = THIP_OK;
+    std::unique_lock<std::mutex> turn;
+    thip_status_t result = takeChainTurn(e, &turn);
     for (const Step &s : e->steps) {
         // the array keeps what the last call left there, whoever made it; nothing in a K-split workspace has to start
         // at zero (every slot that is read has been written by the same dispatch)

@@ -8,6 +8,24 @@
 
 namespace thip {
 
+// Division by a divisor that is known at the launch.  A 64-bit division by a run-time divisor costs a couple of hundred
+// instructions, more than the whole body of a pooling thread, so the launchers precompute multipliers: for n < 2^31 and a
+// divisor d with s = ceil(log2 d), n / d == umulhi(n, ceil(2^(31+s) / d)) >> (s - 1) (the multiplier fits 32 bits because
+// d > 2^(s-1)).
+struct FastDiv {
+    uint32_t mul;    // 0: the divisor is 1
+    uint32_t shift;  // s - 1
+    uint32_t d;
+};
+__host__ __device__ static inline FastDiv makeFastDiv(uint32_t d) {
+    FastDiv f{0, 0, d};
+    if (d <= 1) return f;
+    uint32_t s = 0;
+    while ((1ull << s) < d) s++;
+    f.mul = (uint32_t)((((unsigned long long)1 << (31 + s)) + d - 1) / d);
+    f.shift = s - 1;
+    return f;
+}
 // Output requantisation shared by every kernel: the ACT rescale-clamp of the
 // reference (compiler/torq/Utils/Kernel.h:610-624).
 struct Requant {
@@ -47,6 +65,8 @@ struct Tuning {
     bool noFcWide = false;          // THIP_NO_FC_WIDE
     bool addGeneric = false;        // THIP_ADD_GENERIC: the quantised add always through the 64-bit ACT stage
     bool maxpoolGeneric = false;    // THIP_MAXPOOL_GENERIC: the any-window max pool kernel also for 2 x 2 stride 2
+    int decChain = -1;              // THIP_DEC_CHAIN=0 / 1: the records of a decoder's step as one launch never / wherever it takes them (-1: by cost)
+    long long decChainWait = 20000000;  // THIP_DEC_CHAIN_WAIT: ticks of 10 ns that a workgroup of dec_chain waits for the others (0: gives up at once)
     int decSplit = 0;               // THIP_DEC_SPLIT: workgroups per 16-column tile of a dec_linear launch of at most four rows: 1 or 2 (0: by its size)
     int decAblate = 0;              // THIP_DEC_ABLATE: parts of dec_linear left out, for timing experiments (wrong results)
     int decTargetGroups = 0;        // THIP_DEC_TARGET_WORKGROUPS: workgroups a dec_linear launch with few column tiles shares its rows out to (0: 256)
@@ -330,6 +350,10 @@ struct DecMatmulArgs {
     float bias, lo, hi;
 };
 hipError_t launchDecMatmul(const DecMatmulArgs &a, const LaunchCtx &ctx);
+
+// A run of such records as one launch of `workgroups` workgroups (thip_dec_chain.h).
+struct DecChainArgs;
+hipError_t launchDecChain(const DecChainArgs &a, int workgroups, const LaunchCtx &ctx);
 
 // Sustained v_mfma_i32_32x32x32_i8 rate (TOP/s, 1 multiply-add = 2 ops) of `blocks` workgroups of four waves that
 // do nothing else, on constant or on random operand bytes.  Allocates and frees its own few KiB.

@@ -204,26 +204,9 @@ __device__ __forceinline__ void storeElem(void *out, size_t idx, int32_t v, int 
 __device__ __forceinline__ void blockBarrier() { asm volatile("s_barrier" : : : "memory"); }
 
 // ---------------------------------------------------------------------------
-// Linear work index -> (channel group, x, y, image).  A 64-bit division by a run-time divisor costs a
-// couple of hundred instructions, more than the whole body of a pooling thread, so the launchers
-// precompute multipliers: for n < 2^31 and a divisor d with s = ceil(log2 d),
-// n / d == umulhi(n, ceil(2^(31+s) / d)) >> (s - 1) (the multiplier fits 32 bits because
-// d > 2^(s-1)).  Work counts of 2^31 and more take the plain 64-bit path.
+// Linear work index -> (channel group, x, y, image): the launchers precompute the divisions (FastDiv).  Work counts
+// of 2^31 and more take the plain 64-bit path.
 // ---------------------------------------------------------------------------
-struct FastDiv {
-    uint32_t mul;    // 0: the divisor is 1
-    uint32_t shift;  // s - 1
-    uint32_t d;
-};
-__host__ __device__ static inline FastDiv makeFastDiv(uint32_t d) {
-    FastDiv f{0, 0, d};
-    if (d <= 1) return f;
-    uint32_t s = 0;
-    while ((1ull << s) < d) s++;
-    f.mul = (uint32_t)((((unsigned long long)1 << (31 + s)) + d - 1) / d);
-    f.shift = s - 1;
-    return f;
-}
 struct WorkSplit {
     FastDiv cg, xs, ys;  // channel groups, x positions, y positions per image
     int wide;            // the work count does not fit 31 bits

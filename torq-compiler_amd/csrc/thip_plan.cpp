@@ -1,6 +1,9 @@
 #include "thip_plan.h"
 
+#include <math.h>
 #include <string.h>
+
+#include <algorithm>
 
 #include "../../include/thip.h"
 #include "thip_kernels.h"
@@ -12,13 +15,13 @@ static size_t elemBytes(int32_t dtype) { return dtype == 1 ? 1 : dtype == 2 ? 2 
 static bool sameRef(const DescRef &a, const DescRef &b) { return a.space == b.space && a.index == b.index && a.offset == b.offset; }
 static bool sameBuffer(const DescRef &a, const DescRef &b) { return a.space == b.space && a.index == b.index; }
 
-// How often the records name each intermediate.
-static std::vector<uint32_t> tempUses(const DescriptorView &v) {
+// How often `n` records from `first` on name each intermediate.
+static std::vector<uint32_t> tempUses(const DescriptorView &v, uint32_t first, uint32_t n) {
     std::vector<uint32_t> uses(v.header.temp_count, 0);
     auto count = [&](const DescRef &r) {
         if (r.space == kSpaceTemp) uses[r.index]++;
     };
-    for (uint32_t i = 0; i < v.header.op_count; i++) {
+    for (uint32_t i = first; i < first + n; i++) {
         const DescOp &op = v.ops[i];
         for (const DescRef *r : {&op.in0, &op.in1, &op.weights, &op.bias, &op.scale, &op.table, &op.out}) count(*r);
         if (op.kind == kKindDecLinear) {
@@ -214,6 +217,202 @@ static bool matchPadded(const DescriptorView &v, const Tuning &tuning, uint32_t 
     return true;
 }
 
+// A grouped linear or small matmul as a phase of dec_chain, but for what the exchange carries; false: not one of its.
+static bool chainPhase(const DescriptorView &v, const DescOp &op, int workgroups, const std::function<ChainRef(const DescRef &)> &at, ChainPhase *out) {
+    ChainPhase t;
+    memset(&t, 0, sizeof(t));
+    auto asFloat = [](int32_t bits) {
+        float f;
+        memcpy(&f, &bits, 4);
+        return f;
+    };
+    t.xTag = t.resTag = t.outTag[0] = t.outTag[1] = t.outTag[2] = t.addTag = -1;
+    t.lo = asFloat(op.output_min);
+    t.hi = asFloat(op.output_max);
+    t.M = op.M;
+    t.K = op.K;
+    t.split = t.nmat = t.nseg = 1;
+    if (op.kind == kKindDecLinear) {
+        DecLinearExt x;
+        memcpy(&x, v.blob + v.header.data_offset + v.consts[op.table.index].offset + op.table.offset, sizeof(x));
+        if (op.M > kChainMaxRows || (long long)op.M * op.K > (1 << 20)) return false;
+        if (asFloat(op.bias0) != -INFINITY || asFloat(op.scale0) != INFINITY) return false;  // a clamped expansion
+        const bool pair = (op.w1 & kDecPair) != 0;
+        long long tiles = 0;
+        for (int m = 0; m < op.w0; m++) {
+            if (x.weights[m].space != kSpaceConst || x.bias[m].space != kSpaceConst) return false;
+            t.w[m] = at(x.weights[m]);
+            t.bias[m] = at(x.bias[m]);
+            t.out[m] = x.out[m].space == kSpaceNone ? 0 : at(x.out[m]);
+            t.N[m] = x.N[m];
+            if (m == 0 || !pair) tiles += x.N[m] / 16;
+        }
+        if (tiles > (1 << 20)) return false;
+        t.x = at(op.in0);
+        t.nseg = op.w0;
+        t.nmat = pair ? 2 : 1;
+        t.slotBytes = decSlotBytes(x.has_qbias != 0);
+        // two jobs share a tile where K has more units than a workgroup has waves and the chip has workgroups to spare
+        t.split = op.K / 128 > kChainWaves && tiles * 2 <= workgroups ? 2 : 1;
+        t.units = (op.K / 128 + t.split - 1) / t.split;
+        t.perPass = kChainResults / t.nmat;
+        t.jobs = (int32_t)tiles * t.split;
+        t.addMode = (op.w1 & kDecAddResidual) ? (op.w1 & kDecResFirst ? 3 : 1) : (op.w1 & kDecAddPair) ? 2 : 0;
+        if (t.addMode) {
+            if (t.addMode != 2) t.res = at(x.res);
+            t.addOut = at(x.add_out);
+            t.aw0 = asFloat((int32_t)((uint32_t)x.aw0 << 16));
+            t.aw1 = asFloat((int32_t)((uint32_t)x.aw1 << 16));
+            t.abias = asFloat(x.abias);
+            t.alo = asFloat(x.alo);
+            t.ahi = asFloat(x.ahi);
+        }
+    } else if (op.kind == kKindDecMatmul) {
+        const long long tiles = ((long long)op.Nn + 15) / 16, rows = (long long)op.M * op.K;
+        if (op.M > kChainMaxHeads || tiles * op.TB > (1 << 20) || rows > (1 << 20) || (long long)(op.w1 ? 1 : op.TB) * op.Nn * op.K >= (1 << 30)) return false;
+        t.x = at(op.in0);
+        t.w[0] = at(op.weights);
+        t.out[0] = at(op.out);
+        t.N[0] = op.Nn;
+        t.tiles = (int32_t)tiles;
+        t.jobs = (int32_t)tiles * op.TB;
+        t.units = (op.K + 63) / 64;
+        // the rows of every job of a pass are in LDS at once
+        t.perPass = (int32_t)std::max<long long>(1, std::min<long long>(kChainResults, 32 * 1024 / (rows * 2)));
+        t.aStride = op.w0 ? 0 : op.M * op.K;
+        t.wStride = op.w1 ? 0 : op.Nn * op.K;
+        t.outStride = op.M * op.Nn;
+        t.wBytes = (uint32_t)((uint64_t)(op.w1 ? 1 : op.TB) * op.Nn * op.K * 2);
+        t.bias0 = asFloat(op.bias0);
+        const FastDiv d = makeFastDiv((uint32_t)t.tiles);
+        t.tilesMul = d.mul;
+        t.tilesShift = d.shift;
+    } else {
+        return false;
+    }
+    const FastDiv units = makeFastDiv((uint32_t)t.units), items = makeFastDiv((uint32_t)(t.M * 16 / t.split));
+    t.unitsMul = units.mul;
+    t.unitsShift = units.shift;
+    t.itemsMul = items.mul;
+    t.itemsShift = items.shift;
+    *out = t;
+    return true;
+}
+
+// What a phase reads that the chain makes is read from the exchange, so it has to be one result of a phase before it, or a part of one.  Weights and
+// caches are fetched ahead: none of them is written in the chain.  Everything else that is read is there when the launch starts, and written by no phase.
+Chain layoutChain(const DescriptorView &v, uint32_t first, uint32_t most, int workgroups, const std::function<ChainRef(const DescRef &)> &at) {
+    struct Range {
+        DescRef ref;
+        uint64_t bytes;
+        int32_t *tag;    // of a result: where the exchange has it
+        ChainRef *plain;
+    };
+    Chain chain;
+    std::vector<Range> reads, writes;
+    auto meet = [](const Range &a, const Range &b) { return sameBuffer(a.ref, b.ref) && a.ref.offset < b.ref.offset + b.bytes && b.ref.offset < a.ref.offset + a.bytes; };
+    auto anyMeets = [&](const std::vector<Range> &list, const Range &r) {
+        for (const Range &x : list) {
+            if (meet(x, r)) return true;
+        }
+        return false;
+    };
+    chain.phases.reserve(kChainMaxPhases);  // tags point into it
+    most = std::min(most, std::min<uint32_t>(kChainMaxPhases, v.header.op_count - first));
+    for (uint32_t n = 0; n < most; n++) {
+        const DescOp &op = v.ops[first + n];
+        ChainPhase t;
+        if (!chainPhase(v, op, workgroups, at, &t)) break;
+        chain.phases.push_back(t);
+        ChainPhase &p = chain.phases.back();
+        std::vector<Range> in, ahead, out;
+        if (p.slotBytes == 0) {
+            in.push_back({op.in0, (uint64_t)(op.w0 ? 1 : op.TB) * op.M * op.K * 2, &p.xTag, nullptr});
+            ahead.push_back({op.weights, (uint64_t)(op.w1 ? 1 : op.TB) * op.Nn * op.K * 2, nullptr, nullptr});
+            out.push_back({op.out, (uint64_t)op.TB * op.M * op.Nn * 2, &p.outTag[0], &p.out[0]});
+        } else {
+            DecLinearExt x;
+            memcpy(&x, v.blob + v.header.data_offset + v.consts[op.table.index].offset + op.table.offset, sizeof(x));
+            in.push_back({op.in0, (uint64_t)op.M * op.K * 2, &p.xTag, nullptr});
+            if (p.addMode & 1) in.push_back({x.res, (uint64_t)op.M * x.N[0] * 2, &p.resTag, nullptr});
+            if (p.addMode) out.push_back({x.add_out, (uint64_t)op.M * x.N[0] * 2, &p.addTag, &p.addOut});
+            for (int m = 0; m < op.w0; m++) {
+                if (x.out[m].space != kSpaceNone) out.push_back({x.out[m], (uint64_t)op.M * x.N[m] * 2, &p.outTag[m], &p.out[m]});
+            }
+        }
+        bool fits = true;
+        std::vector<int32_t *> exchanged;  // results that this phase is the first to read
+        for (const Range &r : ahead) fits = fits && !anyMeets(writes, r);
+        for (const Range &r : out) fits = fits && !anyMeets(writes, r) && !anyMeets(reads, r) && !anyMeets(in, r) && !anyMeets(ahead, r);
+        uint64_t words = chain.exchangeWords;
+        for (const Range &r : in) {
+            if (!fits || !anyMeets(writes, r)) continue;
+            const Range *source = nullptr;
+            for (const Range &x : writes) {
+                if (sameBuffer(x.ref, r.ref) && x.ref.offset <= r.ref.offset && r.ref.offset + r.bytes <= x.ref.offset + x.bytes) source = &x;
+            }
+            // 16-byte loads
+            if (!source || (r.ref.offset - source->ref.offset) % 8 != 0 || words + source->bytes / 2 + 32 > (1u << 30)) {
+                fits = false;
+                break;
+            }
+            if (*source->tag < 0) {
+                *source->tag = (int32_t)words;
+                exchanged.push_back(source->tag);
+                words = (uint64_t)roundUp((int64_t)(words + source->bytes / 2), 32);
+            }
+            *r.tag = *source->tag + (int32_t)((r.ref.offset - source->ref.offset) / 2);
+        }
+        const int32_t x = std::max(chain.xRoom, (p.slotBytes == 0 ? p.perPass : 1) * p.M * p.K * 2), red = std::max(chain.redRoom, kChainResults * kChainWaves * p.M * 64);
+        if (!fits || (int64_t)(n + 1) * (int64_t)sizeof(ChainPhase) + x + red > kChainLds) {
+            for (int32_t *tag : exchanged) *tag = -1;
+            chain.phases.pop_back();
+            break;
+        }
+        p.start = n == 0 ? 0 : (chain.phases[n - 1].start + chain.phases[n - 1].jobs) % workgroups;
+        chain.exchangeWords = words;
+        chain.xRoom = x;
+        chain.redRoom = red;
+        reads.insert(reads.end(), in.begin(), in.end());
+        reads.insert(reads.end(), ahead.begin(), ahead.end());
+        writes.insert(writes.end(), out.begin(), out.end());
+    }
+    // an intermediate that only the chain reads is nowhere but in the exchange
+    const uint32_t count = (uint32_t)chain.phases.size();
+    const std::vector<uint32_t> all = tempUses(v, 0, v.header.op_count), here = tempUses(v, first, count);
+    for (const Range &r : writes) {
+        if (r.ref.space == kSpaceTemp && *r.tag >= 0 && all[r.ref.index] == here[r.ref.index]) *r.plain = 0;
+    }
+    return chain;
+}
+
+// Whether a chain is ahead of its records' own launches.  It saves 1.5 us a phase: what a launch costs beyond handing its results to the next
+// one, and the weights that are fetched meanwhile.  It costs 5 us once, and 0.25 us for every 1000 elements that a workgroup brings as input rows: it
+// reads them as dwords past its L2, where a launch reads 16-bit elements through it.  Fitted to 60 decoder steps of one to four rows, 1 to 6 layers,
+// hidden 256 .. 2048, one by one / as a chain, us:
+//   taken   26 layers, 1152, 6912, one row 843 / 616, 4 layers of it 117 / 88 (two rows 117 / 99), 4 x 1664, 640, one row 104 / 65,
+//           5 x 256, 8064, three rows 136 / 109, 1 x 1152, 6912 34.0 / 30.5
+//   left    6 x 384, 6272, four rows 169 / 180, 4 x 2048, 8192, 8 heads of 256 on 2048 positions, one row 182 / 185
+static bool chainPays(const Chain &chain, int workgroups) {
+    double gain = -6;  // 1 us more than measured: boxes differ
+    for (const ChainPhase &t : chain.phases) {
+        const int jobs = (t.jobs + workgroups - 1) / workgroups;
+        gain += 1.54 - 0.253e-3 * (double)t.M * t.K * (t.slotBytes == 0 ? std::min(jobs, (int)t.perPass) : 1);
+    }
+    return gain > 0;
+}
+
+static bool matchDecChain(const DescriptorView &v, const Tuning &tuning, uint32_t first, Step *s) {
+    if (tuning.decChain == 0 || v.header.binding_count > 64) return false;
+    if (v.ops[first].kind != kKindDecLinear && v.ops[first].kind != kKindDecMatmul) return false;
+    const Chain chain = layoutChain(v, first, v.header.op_count, kChainWorkgroups, [](const DescRef &) { return (ChainRef)1; });
+    if (chain.phases.size() < (size_t)kChainMinPhases || (tuning.decChain < 0 && !chainPays(chain, kChainWorkgroups))) return false;
+    s->kind = kStepDecChain;
+    s->first = first;
+    s->count = (uint32_t)chain.phases.size();
+    return true;
+}
+
 // The kernel that is ahead for a GEMM-shaped record.
 static IgemmRoute igemmRoute(const DescriptorView &v, const DescOp &op) {
     // addresses that are aligned as a dispatch's are
@@ -236,11 +435,11 @@ bool replayPays(size_t launches, uint64_t constantBytes) {
 
 std::vector<Step> planSteps(const DescriptorView &v, const Tuning &tuning) {
     const bool plain = tuning.plainRecords;
-    const std::vector<uint32_t> uses = tempUses(v);
+    const std::vector<uint32_t> uses = tempUses(v, 0, v.header.op_count);
     std::vector<Step> steps;
     for (uint32_t i = 0; i < v.header.op_count;) {
         Step s{};
-        if (plain || (!matchExpandDw(v, uses, i, &s) && !matchMatmulRt(v, uses, i, &s) && !matchPadded(v, tuning, i, &s))) {
+        if (plain || (!matchDecChain(v, tuning, i, &s) && !matchExpandDw(v, uses, i, &s) && !matchMatmulRt(v, uses, i, &s) && !matchPadded(v, tuning, i, &s))) {
             s.kind = kStepRecord;
             s.first = i;
             s.count = 1;

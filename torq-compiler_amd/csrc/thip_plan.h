@@ -4,8 +4,10 @@
 
 #include <string.h>
 
+#include <functional>
 #include <vector>
 
+#include "thip_dec_chain.h"
 #include "thip_kernels.h"
 #include "thip_validate.h"
 
@@ -16,6 +18,7 @@ enum StepKind {
     kStepExpandDw,  // a pointwise convolution and the depthwise one behind it (ir_expand_dw_i8)
     kStepPadded,    // a GEMM-shaped record whose channels fill no 16-byte chunks: its input padded, then a dense kernel
     kStepMatmulRt,  // a batch of int8 matmuls with a run-time input2: its transposes and its GEMMs (igemm_rt_i8)
+    kStepDecChain,  // grouped linears and small matmuls of a decoder's step, each behind the one before it (dec_chain)
 };
 
 // The kernel that a GEMM-shaped record of a dispatch runs by.
@@ -41,6 +44,8 @@ struct Step {
     int32_t from, to;
     DescOp op;
     std::vector<uint8_t> constants;
+    // kStepDecChain: bytes of LDS for input rows and for partial sums; set when its table is laid out
+    int32_t xRoom, redRoom;
 };
 constexpr uint32_t kSpacePlan = 16;
 
@@ -75,6 +80,14 @@ IgemmArgs igemmArgs(const DescriptorView &v, const DescOp &op, At &&at) {
     }
     return a;
 }
+
+// The records from `first` on that one launch of dec_chain takes, at most `most`, its operands where `at` says.
+struct Chain {
+    std::vector<ChainPhase> phases;
+    uint64_t exchangeWords = 0;
+    int32_t xRoom = 0, redRoom = 0;  // LDS of a workgroup for input rows and for partial sums
+};
+Chain layoutChain(const DescriptorView &v, uint32_t first, uint32_t most, int workgroups, const std::function<ChainRef(const DescRef &)> &at);
 
 // The launches of a dispatch in order.  Every record belongs to exactly one step; a step that stands for several leaves
 // the intermediates between them unwritten, so it is only formed where no other record reads them.
