@@ -186,7 +186,7 @@ static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op
         const IgemmArgs a = igemmArgs(viewOf(e), op, [&](const DescRef &r) { return resolve(e, r, bp); });
         if (route == kIgemmDirect) err = launchIgemmDirect(a, ctx);
         else if (route == kIgemmPatch) err = launchConvPatch(a, ctx);
-        else err = launchIgemm(a, op.variant, ctx);
+        else err = launchIgemm(a, op.variant, ctx, route == kIgemmWide);
         break;
     }
     case kKindFcSkinny: {

@@ -580,11 +580,10 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BLOCKS_PER_CU) void igemm_de
     // barrier, and while phase 1 runs it refills the stage it just finished with tile
     // kt+STAGES and reads phase 0 of tile kt+1.  LDS latency and the DMA issue thus hide
     // under MFMAs; sched_barrier pins the interleaving the source spells out.
-    auto issueTile = [&](int kt, int part, int parts, auto wholeTag) {
-        // issues this wave's DMA loads number [part * LPT / parts, (part + 1) * LPT / parts) of tile kt;
+    auto issueTile = [&](int kt, unsigned stage, int part, int parts, auto wholeTag) {
+        // issues this wave's DMA loads number [part * LPT / parts, (part + 1) * LPT / parts) of tile kt into the ring at `stage`;
         // `whole` promises that the tile lies entirely below K
         constexpr bool kWhole = decltype(wholeTag)::value;
-        const unsigned stage = ldsBase + (unsigned)(kt % STAGES) * STAGE;
         const int8_t *aBase = aTile + kt * BK;
         const int8_t *bBase = bTile + kt * BK;
         // beyond K the weights are zero, so any valid bytes will do: such lanes read chunk 0 of the
@@ -637,7 +636,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BLOCKS_PER_CU) void igemm_de
 
 #pragma unroll
     for (int t = 0; t < STAGES; t++) {
-        if (t < KT) issueTile(t, 0, 1, std::false_type{});
+        if (t < KT) issueTile(t, ldsBase + (unsigned)t * STAGE, 0, 1, std::false_type{});
     }
     // tile 0 landed?  (tiles 1 .. STAGES-1 may stay in flight)
     if (KT >= STAGES) {
@@ -650,12 +649,15 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BLOCKS_PER_CU) void igemm_de
 #pragma unroll
     for (int x = 0; x < NF; x++) readFrag(smem, 0, x, af0, bf0);
 
+    int at = 0;  // tile kt's place in the ring
     // One k-tile.  `steady` (a compile-time flag) is the branch-free body used while the tile it
     // refills the ring with exists and lies wholly below K; the rest go through the general body.
     auto step = [&](int kt, auto steady) {
         constexpr bool kSteady = decltype(steady)::value;
-        const int8_t *st = smem + (kt % STAGES) * STAGE;
-        const int8_t *stNext = smem + ((kt + 1) % STAGES) * STAGE;
+        const int8_t *st = smem + at;
+        const int refilled = at;  // tile kt + STAGES takes the place of tile kt
+        at = at + STAGE == STAGES * STAGE ? 0 : at + STAGE;
+        const int8_t *stNext = smem + at;
         // every phase but the last: MFMAs on the current fragments; the reads of the next phase's go out behind the
         // first weight row (so that the wait in front of that row only covers reads issued a phase ago) and
         // complete under the remaining rows
@@ -706,7 +708,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BLOCKS_PER_CU) void igemm_de
         // the refill of the freed stage spread between the rows
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-            if (refill) issueTile(kt + STAGES, j, TN, steady);
+            if (refill) issueTile(kt + STAGES, ldsBase + (unsigned)refilled, j, TN, steady);
 #pragma unroll
             for (int i = 0; i < TM; i++) acc[j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf1[j], af1[i], acc[j][i], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
@@ -1247,7 +1249,44 @@ static hipError_t launchIgemmDense(const IgemmArgs &a, const LaunchCtx &ctx) {
     return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 0, false, CONV, BK>(a, ctx);
 }
 
-hipError_t launchIgemm(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ctx) {
+// Whether a tile's problem is ahead in k-tiles of 128 bytes: whole cache lines per tile row, half the barriers per byte, and fewer
+// stages for the same bytes in flight.  us, in 64-byte k-tiles / in these:
+//   64 x 64, three stages, three workgroups per CU   512x1536x2048 6.3 / 5.9, 512x4096x2048 11.9 / 10.9, 128x8192x2048 18.4 / 16.3, 640x4096x2048
+//     17.3 / 13.8; 3x3 28x28x256 -> 256, batch 4 11.1 / 9.2, 14x14x512 -> 512, batch 8 18.1 / 14.4; at K = 1280 5.75 / 5.69, at 768 4.5 / 4.6
+//   64 x 128, three stages   512x1024x4096 6.1 / 6.0, 512x2048x4096 9.6 / 8.6, 600x2048x4096 14.1 / 12.0, 1200x1024x2048 8.2 / 7.8
+//   128 x 128   one tile per CU, three stages 1024x1024x4096 8.8 / 8.4, 1024x2048x4096 13.8 / 12.8, 1024x8192x4096 42.4 / 40.1; more tiles, two stages,
+//     two workgroups per CU 3000x1024x2048 12.6 / 11.0, 2000x2048x3072 20.5 / 18.0, 1400x3072x4096 29.2 / 23.7
+//   128 x 64, three stages   300x4096x4096 14.4 / 14.2, 768x4096x2048 15.2 / 14.9, but 300x2048x4096 8.4 / 8.8
+// (Four to six stages are 0 - 5 % behind three: the loads are bound by what they carry, not by their latency.)
+bool igemmWideBetter(const IgemmArgs &a, uint32_t variant) {
+    if ((a.loader != kLoaderDense && a.loader != kLoaderWindow) || a.skip != nullptr || a.Kp % 128 != 0) return false;
+    switch (variant) {
+    case kIgemmDense64x64: return a.Kp >= 1152;
+    case kIgemmDense64x128: return a.Kp >= 1024 && a.loader == kLoaderDense;
+    case kIgemmDense128x128: return a.Kp >= 1024;
+    case kIgemmDense128x64: return a.Kp >= 4096 && a.loader == kLoaderDense;
+    default: return false;
+    }
+}
+template <bool CONV>
+static hipError_t launchIgemmWide(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ctx) {
+    auto tiles = [&](int bm, int bn) { return (long long)((a.M + bm - 1) / bm) * (a.Np / bn); };
+    switch (variant) {
+    case kIgemmDense64x64: return launchIgemmDense<64, 64, 2, 2, 3, 3, CONV, 128>(a, ctx);
+    case kIgemmDense128x128: return tiles(128, 128) <= 256 ? launchIgemmDense<128, 128, 2, 2, 3, 1, CONV, 128>(a, ctx) : launchIgemmDense<128, 128, 2, 2, 2, 2, CONV, 128>(a, ctx);
+    case kIgemmDense64x128:
+        // (one workgroup per CU has all registers: 512 x 4096 x 4096 13.7 us against 14.4)
+        if constexpr (!CONV) return tiles(64, 128) <= 256 ? launchIgemmDense<64, 128, 2, 2, 3, 1, false, 128>(a, ctx) : launchIgemmDense<64, 128, 2, 2, 3, 2, false, 128>(a, ctx);
+        return hipErrorInvalidValue;
+    case kIgemmDense128x64:
+        if constexpr (!CONV) return launchIgemmDense<128, 64, 2, 2, 3, 2, false, 128>(a, ctx);
+        return hipErrorInvalidValue;
+    default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t launchIgemm(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ctx, bool wide) {
+    wide = wide && igemmWideBetter(a, variant) && !ctx.tuning->noK128;
     if (variant >= kIgemmVariantCount) return hipErrorInvalidValue;
     const IgemmTile &t = igemmTile(variant);
     // What the kernel assumes: padded sizes are whole tiles, the real sizes fit
@@ -1274,6 +1313,7 @@ hipError_t launchIgemm(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ct
         if (a.M % (a.OH * a.OW) != 0 || (long long)a.K != (long long)a.KH * a.KW * a.C || a.Kp != (a.K + t.bk - 1) / t.bk * t.bk) return hipErrorInvalidValue;
         if (a.a_bytes != (long long)(a.M / (a.OH * a.OW)) * a.H * a.W * a.C || a.a_bytes >= (1LL << 32)) return hipErrorInvalidValue;
         if (((uintptr_t)a.A & 15) != 0 || a.skip != nullptr) return hipErrorInvalidValue;
+        if (wide) return launchIgemmWide<true>(a, variant, ctx);
         switch (variant) {
         case kIgemmDense256x256: return launchIgemmDense<256, 256, 2, 2, 4, 1, true>(a, ctx);
         case kIgemmDense128x256:
@@ -1300,6 +1340,7 @@ hipError_t launchIgemm(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ct
     if (((uintptr_t)a.Bp & 15) != 0) return hipErrorInvalidValue;
     if (a.out_dtype < kDtypeI8 || a.out_dtype > kDtypeI32) return hipErrorInvalidValue;
     if (a.skip != nullptr && variant != kIgemmStream && variant != kIgemmDense64x64) return hipErrorInvalidValue;  // the kernels that can add a residual
+    if (wide) return launchIgemmWide<false>(a, variant, ctx);
     switch (variant) {
     case kIgemm128x128x64: return launchIgemmLoader<128, 128, 64>(a, ctx);
     case kIgemm256x256x64: return launchIgemmLoader<256, 256, 64>(a, ctx);

@@ -149,7 +149,9 @@ inline bool igemmStreamFits(int64_t N, int64_t K, int32_t out_dtype) {
     const int64_t chunk = igemmStreamChunk((int)Np), chunks = (Np + chunk - 1) / chunk;
     return chunk * Kp + 8 * chunk + Kp / 4 <= 64 * 1024 && (chunks - 1) * K <= N;
 }
-hipError_t launchIgemm(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ctx);
+// wide: in k-tiles of 128 bytes where these are ahead (igemmWideBetter; host-only).
+hipError_t launchIgemm(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ctx, bool wide = false);
+bool igemmWideBetter(const IgemmArgs &a, uint32_t variant);
 
 // A pointwise convolution (dense int8 [N H W][K] -> C channels), or one over few channels, and the 3 x 3 depthwise convolution that alone reads its result.
 struct IrExpandDwArgs {

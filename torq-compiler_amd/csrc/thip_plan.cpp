@@ -414,12 +414,12 @@ static bool matchDecChain(const DescriptorView &v, const Tuning &tuning, uint32_
 }
 
 // The kernel that is ahead for a GEMM-shaped record.
-static IgemmRoute igemmRoute(const DescriptorView &v, const DescOp &op) {
+static IgemmRoute igemmRoute(const DescriptorView &v, const Tuning &tuning, const DescOp &op) {
     // addresses that are aligned as a dispatch's are
     const IgemmArgs a = igemmArgs(v, op, [&](const DescRef &r) {
         return r.space == kSpaceNone ? nullptr : (uint8_t *)(uintptr_t)(0x1000000 + (r.space == kSpaceConst ? v.consts[r.index].offset : 0) + r.offset);
     });
-    return igemmDirectBetter(a) ? kIgemmDirect : convPatchBetter(a) ? kIgemmPatch : kIgemmOwnTile;
+    return igemmDirectBetter(a) ? kIgemmDirect : convPatchBetter(a) ? kIgemmPatch : !tuning.noK128 && igemmWideBetter(a, op.variant) ? kIgemmWide : kIgemmOwnTile;
 }
 
 // A replay starts about 5 us later than a launch behind another, and costs the host 12 - 20 us in place of 3 per launch.  Launches that
@@ -445,7 +445,7 @@ std::vector<Step> planSteps(const DescriptorView &v, const Tuning &tuning) {
             s.count = 1;
         }
         const DescOp *op = s.kind == kStepRecord ? &v.ops[i] : s.kind == kStepPadded ? &s.op : nullptr;
-        s.route = !plain && op && op->kind == kKindIgemm ? igemmRoute(v, *op) : kIgemmOwnTile;
+        s.route = !plain && op && op->kind == kKindIgemm ? igemmRoute(v, tuning, *op) : kIgemmOwnTile;
         i += s.count;
         steps.push_back(std::move(s));
     }

@@ -26,6 +26,7 @@ enum IgemmRoute {
     kIgemmOwnTile,  // the record's
     kIgemmDirect,   // igemm_direct_i8
     kIgemmPatch,    // conv_patch_i8
+    kIgemmWide,     // the record's tile in k-tiles of 128 bytes
 };
 
 struct Step {
