@@ -24,7 +24,11 @@ int main(int argc, char **argv) {
                            (const DescTemp *)(blob.data() + h.temps_offset), (const DescConst *)(blob.data() + h.consts_offset)};
     const std::vector<Step> steps = planSteps(v, tuningFromEnvironment());
     const char *kinds[] = {"record", "ir_expand_dw_i8", "padded", "igemm_rt_i8", "dec_chain"}, *routes[] = {"", " igemm_direct_i8", " conv_patch_i8", " igemm_dense_k128_i8"};
-    for (const Step &s : steps) printf("%s %u %u%s\n", kinds[s.kind], s.first, s.count, routes[s.route]);
+    for (const Step &s : steps) {
+        printf("%s %u %u%s", kinds[s.kind], s.first, s.count, routes[s.route]);
+        if (s.blocked) printf(" blocked %d", s.blocked);
+        puts("");
+    }
     puts(replayPays(steps.size(), h.total_size - h.data_offset) ? "replayed" : "one by one");
     return 0;
 }

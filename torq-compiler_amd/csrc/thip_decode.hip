@@ -42,11 +42,16 @@ __device__ __forceinline__ void waitVmcntDyn(int n) {
 #undef THIP_VMCNT_CASE
 }
 
+// Where element (row, n) of a result of `rows` rows and N columns lies, in elements.
+__device__ __forceinline__ size_t decResultAt(bool blocked, int rows, int row, int n, int N) {
+    return blocked ? (size_t)(n >> 5) * (size_t)(rows * 32) + (size_t)(row * 32 + (n & 31)) : (size_t)row * N + n;
+}
+
 constexpr int kDecLdsSlot = 2048 + 128;  // a k-block's weights, scales and (room for) biases in LDS
 
 // MR: groups of 16 input rows (1 or 2).  XLDS: the input rows come through LDS as well (at most four rows): then every
 // global load of a wave is an LDS-DMA load issued up front and each k-block is computed as soon as it has landed.
-// Otherwise the rows come through registers, CH k-blocks at a time, double-buffered.  QB: the slots carry block biases.
+// Otherwise the rows come through registers, CH k-blocks at a time, two such chunks in flight.  QB: the slots carry block biases.
 // QC: the expansion clamps.
 // S (XLDS only): the 16-column tile is shared out over S workgroups of CW = 16 / S columns, each an MFMA's row operand made of S
 // k-blocks of its columns: operand row c holds column c % CW of k-block c / CW and input column c holds input row c % CW of k-block
@@ -186,6 +191,14 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
         struct XBuf {
             v4i x[CH][4][MR];
         };
+        // A load brings 64 bytes of each of 16 rows: half a line each where rows lie one behind the other, and a wave's second half only hits
+        // while the first is in its CU's 32 KB cache, among the loads of 15 other waves.  Block by block it is 1 KB of whole lines.
+        const bool xBlocked = (p.blocked & kDecBlockedX) != 0;
+        const uint32_t xRow = xBlocked ? 32u : (uint32_t)p.K, xStep = xBlocked ? 32u * (uint32_t)p.M : 32u;
+        const int8_t *xFirst = (const int8_t *)(p.x + (size_t)((uint32_t)row0 * xRow));
+        uint32_t xLane[MR];  // bytes; the rest of an address is the same for the wave
+#pragma unroll
+        for (int mr = 0; mr < MR; mr++) xLane[mr] = ((uint32_t)(c + 16 * mr) * xRow + 8u * (uint32_t)g) * 2u;
         // Loads only; a k-block the wave does not have and a row beyond M read nothing and feed zeros.
         auto loadChunk = [&](int ch, XBuf &b) {
 #pragma unroll
@@ -193,11 +206,10 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
                 const int i = ch * CH + u;
                 const int kb = wave + NW * i;
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
+                for (int mr = 0; mr < MR; mr++) {
 #pragma unroll
-                    for (int mr = 0; mr < MR; mr++) {
-                        const int row = c + 16 * mr;
-                        b.x[u][j][mr] = (i < nkb && row < M) ? *(const v4i *)(x + (size_t)row * p.K + kb * 128 + 32 * j + 8 * g) : v4i{0, 0, 0, 0};
+                    for (int j = 0; j < 4; j++) {
+                        b.x[u][j][mr] = (i < nkb && c + 16 * mr < M) ? *(const v4i *)(xFirst + (size_t)(2u * (uint32_t)(4 * kb + j) * xStep) + xLane[mr]) : v4i{0, 0, 0, 0};
                     }
                 }
             }
@@ -214,13 +226,14 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
         const int nchunks = (nkb + CH - 1) / CH;
         XBuf b0, b1;
         loadChunk(0, b0);
-        waitVmcnt<0>();  // the DMA burst (and the first chunk's rows) has landed; the compiler counts only its own loads
+        if (nchunks > 1) loadChunk(1, b1);
+        waitVmcnt<0>();  // the DMA burst (and the rows of two chunks) has landed; the compiler counts only its own loads
         for (int ch = 0; ch < nchunks; ch += 2) {
-            if (ch + 1 < nchunks) loadChunk(ch + 1, b1);
             computeChunk(ch, b0);
+            if (ch + 2 < nchunks) loadChunk(ch + 2, b0);
             if (ch + 1 < nchunks) {
-                if (ch + 2 < nchunks) loadChunk(ch + 2, b0);
                 computeChunk(ch + 1, b1);
+                if (ch + 3 < nchunks) loadChunk(ch + 3, b1);
             }
         }
     }
@@ -251,7 +264,7 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
         bias4[m] = m < nmat && mine ? *(const v4f *)(bias + n) : v4f{0.0f, 0.0f, 0.0f, 0.0f};
     }
     v2i rv = v2i{0, 0};
-    if (p.add_mode == 1 && mine) rv = *(const v2i *)(p.res + (size_t)row * Nseg + n);
+    if (p.add_mode == 1 && mine) rv = *(const v2i *)(p.res + decResultAt(p.blocked & kDecBlockedRes, p.M, row, n, Nseg));
     uint16_t y[2][4];
 #pragma unroll
     for (int m = 0; m < 2; m++) {
@@ -279,7 +292,7 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
             y[m][e] = bf16Bits(t0 < p.lo ? p.lo : (t0 > p.hi ? p.hi : t0));
         }
         if (out && mine) {
-            *(v2i *)(out + (size_t)row * Nseg + n) = v2i{(int)((uint32_t)y[m][0] | ((uint32_t)y[m][1] << 16)), (int)((uint32_t)y[m][2] | ((uint32_t)y[m][3] << 16))};
+            *(v2i *)(out + decResultAt(p.blocked & (kDecBlockedOut << sm), p.M, row, n, Nseg)) = v2i{(int)((uint32_t)y[m][0] | ((uint32_t)y[m][1] << 16)), (int)((uint32_t)y[m][2] | ((uint32_t)y[m][3] << 16))};
         }
     }
     if (p.add_mode == 0 || !mine) return;
@@ -294,7 +307,7 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
 #pragma unroll
         for (int e = 0; e < 4; e++) z[e] = addBf16One(y[0][e], y[1][e], p.aw0, p.aw1, p.abias, p.alo, p.ahi);
     }
-    *(v2i *)(p.add_out + (size_t)row * Nseg + n) = v2i{(int)((uint32_t)z[0] | ((uint32_t)z[1] << 16)), (int)((uint32_t)z[2] | ((uint32_t)z[3] << 16))};
+    *(v2i *)(p.add_out + decResultAt(p.blocked & kDecBlockedAdd, p.M, row, n, Nseg)) = v2i{(int)((uint32_t)z[0] | ((uint32_t)z[1] << 16)), (int)((uint32_t)z[2] | ((uint32_t)z[3] << 16))};
 }
 
 template <int MR, int CH, bool XLDS, bool QB, bool QC, int S = 1>
@@ -323,7 +336,6 @@ int decLinearWaves(int K) {
     return kblocks < kDecWaves ? kDecWaves : (kblocks > kDecMaxWaves ? kDecMaxWaves : kblocks);
 }
 constexpr size_t kDecMaxLds = 152 * 1024;
-constexpr int kDecLdsRows = 4;  // up to this many input rows may come through LDS
 
 // Workgroups per column tile.  A workgroup streams its rows of the input next to its 16 columns of the weights: with few
 // column tiles and many rows (32 rows of K = 6912 are 442 KB per workgroup against 110 KB of weights, on 72 of 256 CUs)
@@ -383,12 +395,14 @@ hipError_t launchDecLinear(const DecLinearArgs &in, const LaunchCtx &ctx) {
     if (!a.x || a.M <= 0 || a.M > kDecMaxRows || a.K <= 0 || a.K % 128 != 0 || a.qblock <= 0 || a.qblock % 128 != 0 || a.K % a.qblock != 0) return hipErrorInvalidValue;
     if (a.nseg < 1 || a.nseg > kDecMaxSegments || (a.pair && a.nseg != 2) || (((uintptr_t)a.x) & 15)) return hipErrorInvalidValue;
     if (a.add_mode < 0 || a.add_mode > 2 || (a.add_mode == 1 && (a.nseg != 1 || !a.res)) || (a.add_mode == 2 && !a.pair) || (a.pair && a.add_mode != 2)) return hipErrorInvalidValue;
+    if (a.blocked && a.M <= kDecLdsRows) return hipErrorInvalidValue;
     if (a.add_mode != 0 && (!a.add_out || (((uintptr_t)a.add_out) & 7) || (a.res && (((uintptr_t)a.res) & 7)))) return hipErrorInvalidValue;
     long long tiles = 0;
     for (int s = 0; s < a.nseg; s++) {
         if (!a.w[s] || !a.bias[s] || a.N[s] <= 0 || a.N[s] % 16 != 0) return hipErrorInvalidValue;
         if ((((uintptr_t)a.w[s]) & 15) || (((uintptr_t)a.bias[s]) & 15) || (((uintptr_t)a.out[s]) & 7)) return hipErrorInvalidValue;
         if (!a.out[s] && a.add_mode == 0) return hipErrorInvalidValue;  // a result nobody receives
+        if (a.N[s] % 32 != 0 && (a.blocked & (kDecBlockedRes | kDecBlockedAdd | kDecBlockedOut << s))) return hipErrorInvalidValue;
         tiles += a.N[s] / 16;
     }
     if (a.pair) {
@@ -454,6 +468,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void dec_matmul(DecMatmulArgs p) {
     for (int wv = 0; wv < kDecWaves; wv++) s += red[wv][mr][lane];
     const int n = n0 + 4 * g;
     uint16_t *out = p.out + (size_t)b * p.out_stride + (size_t)row * p.N;
+    if (p.blocked) out = p.out + decResultAt(true, p.B, b, row * p.N + n, 0) - n;  // its four columns lie in one block
     uint16_t y[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
@@ -474,6 +489,7 @@ hipError_t launchDecMatmul(const DecMatmulArgs &a, const LaunchCtx &ctx) {
     if (!a.a || !a.w || !a.out || a.B <= 0 || a.B > 65535 || a.M <= 0 || a.M > kDecMaxRows || a.K <= 0 || a.K % 8 != 0 || a.N <= 0) return hipErrorInvalidValue;
     if (a.a_stride < 0 || a.w_stride < 0 || a.out_stride < 0 || a.a_stride % 8 != 0 || a.w_stride % 8 != 0) return hipErrorInvalidValue;
     if (((((uintptr_t)a.a) | ((uintptr_t)a.w)) & 15) || (((uintptr_t)a.out) & (a.N % 4 == 0 ? 7 : 1)) || (a.N % 4 == 0 && a.out_stride % 4 != 0)) return hipErrorInvalidValue;
+    if (a.blocked && (a.blocked != kDecBlockedOut || a.N % 4 != 0 || a.out_stride != (int64_t)a.M * a.N || a.out_stride % 32 != 0 || a.B * a.out_stride >= (1LL << 31))) return hipErrorInvalidValue;
     const long long tiles = ((long long)a.N + 15) / 16;
     if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 grid((unsigned)tiles, (unsigned)a.B);

@@ -179,8 +179,9 @@ static uint8_t *resolve(const thip_executable_t *e, const DescRef &r, uint8_t *c
 // Launches `op`, which is record i or stands in for it, or (ctx.name set) only asks its launcher which kernel it takes for these
 // operands.  `scratch` (or null): the static scratch array, which then stands in for the record's workspace intermediate.
 // `step` (or null): the buffers of space kSpacePlan.  `route`: the kernel of a GEMM-shaped record.
+// `blocked`: DecBlocked, the intermediates of a decoder's record that lie in blocks of columns.
 static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr,
-                              uint8_t *const *step = nullptr, IgemmRoute route = kIgemmOwnTile) {
+                              uint8_t *const *step = nullptr, IgemmRoute route = kIgemmOwnTile, int32_t blocked = 0) {
     auto resolve = [step](const thip_executable_t *exe, const DescRef &r, uint8_t *const *bindings) {
         return r.space == kSpacePlan ? step[r.index] + r.offset : ::resolve(exe, r, bindings);
     };
@@ -338,12 +339,13 @@ static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op
             memcpy(&a.alo, &x.alo, 4);
             memcpy(&a.ahi, &x.ahi, 4);
         }
+        a.blocked = blocked;
         err = launchDecLinear(a, ctx);
         break;
     }
     case kKindDecMatmul: {
         DecMatmulArgs a{(const uint16_t *)resolve(e, op.in0, bp), (const uint16_t *)resolve(e, op.weights, bp), (uint16_t *)resolve(e, op.out, bp),
-                        op.TB, op.M, op.K, op.Nn, op.w0 ? 0 : (int64_t)op.M * op.K, op.w1 ? 0 : (int64_t)op.Nn * op.K, (int64_t)op.M * op.Nn, 0.0f, 0.0f, 0.0f};
+                        op.TB, op.M, op.K, op.Nn, op.w0 ? 0 : (int64_t)op.M * op.K, op.w1 ? 0 : (int64_t)op.Nn * op.K, (int64_t)op.M * op.Nn, 0.0f, 0.0f, 0.0f, blocked};
         memcpy(&a.bias, &op.bias0, 4);
         memcpy(&a.lo, &op.output_min, 4);
         memcpy(&a.hi, &op.output_max, 4);
@@ -593,7 +595,7 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
         err = launchDecChain(a, e->device->computeUnits, ctx);
         break;
     }
-    default: return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch, nullptr, s.route);
+    default: return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch, nullptr, s.route, s.blocked);
     }
     if (err != hipSuccess) return fail(THIP_INTERNAL, "ops %u .. %u: launch failed: %s", s.first, s.first + s.count - 1, hipGetErrorString(err));
     return THIP_OK;

@@ -324,7 +324,11 @@ struct DecLinearArgs {
     int32_t nwaves;  // waves per workgroup; the launcher sets it (decLinearWaves)
     int32_t rows_per_group;  // input rows of a workgroup; the launcher sets it (grid.y workgroups share a column tile)
     int32_t ablate;  // timing experiments only (THIP_DEC_ABLATE; results are wrong): 1 no weight loads, 2 no arithmetic
+    int32_t blocked; // DecBlocked: of these operands a block of 32 columns is one [M][32] matrix, the next block behind it
 };
+// Which operands of a dec_linear (of a dec_matmul: the result, kDecBlockedOut, as a matrix of B rows) lie block by block.
+enum DecBlocked : int32_t { kDecBlockedX = 1, kDecBlockedRes = 2, kDecBlockedAdd = 4, kDecBlockedOut = 8 };  // kDecBlockedOut << m: out[m]
+constexpr int kDecLdsRows = 4;  // up to this many input rows may come through LDS; they lie row by row
 inline int decSlotBytes(bool hasBias) { return kDecSlotBytes + (hasBias ? 64 : 0); }
 // Byte offset of int8 weight (n, k) in the dec16 order, for K padded to `kblocks` blocks of 128.
 inline size_t decWeightOffset(int n, int k, int kblocks, bool hasBias) {
@@ -350,6 +354,7 @@ struct DecMatmulArgs {
     int32_t B, M, K, N;
     int64_t a_stride, w_stride, out_stride;
     float bias, lo, hi;
+    int32_t blocked;  // kDecBlockedOut or 0
 };
 hipError_t launchDecMatmul(const DecMatmulArgs &a, const LaunchCtx &ctx);
 

@@ -45,6 +45,8 @@ struct Step {
     int32_t from, to;
     DescOp op;
     std::vector<uint8_t> constants;
+    // kStepRecord, grouped linears and small matmuls: DecBlocked, the intermediates that lie in blocks of columns
+    int32_t blocked;
     // kStepDecChain: bytes of LDS for input rows and for partial sums; set when its table is laid out
     int32_t xRoom, redRoom;
 };
