@@ -21,6 +21,12 @@ CASES = [
     (lambda: FC(1025, 1024, 1040, realistic=True), 5, True), (lambda: FC(4099, 1136, 1160, realistic=True), 5, True), (lambda: FC(4099, 1024, 1168), 5, True),
     # 128 x 64
     (lambda: FC(1025, 4096, 1032, realistic=True), 12, True), (lambda: FC(1153, 4208, 976), 12, True), (lambda: FC(1153, 2048, 1032), 12, False),
+    # half of the last k-tile beyond the weights' rows, each tile
+    *[(lambda K=K: FC(1030, K, 976, realistic=True), 7, True) for K in (2576, 2592, 2608, 2624)], (lambda: FC(1030, 2496, 976), 7, False),
+    (lambda: FC(1090, 2096, 1032, realistic=True), 13, True), (lambda: FC(3137, 2112, 1000), 13, True), (lambda: FC(1090, 1984, 1032), 13, False),
+    (lambda: FC(1025, 2112, 1040, realistic=True), 5, True), (lambda: FC(4099, 2224, 1160), 5, True), (lambda: FC(1025, 1984, 1040), 5, False), (lambda: FC(1025, 4160, 1032), 12, True),
+    (lambda: CONV(N=8, H=14, W=14, C=304, O=304, realistic=True), None, True), (lambda: CONV(N=10, H=30, W=29, C=48, O=200, KH=5, KW=6, pad=(2, 3, 2, 2)), 7, True),
+    (lambda: CONV(N=9, H=30, W=31, C=112, O=264, KH=5, KW=4, pad=(1, 2, 2, 2), realistic=True), 5, True), (lambda: CONV(N=10, H=30, W=29, C=144, O=200, KH=3, KW=3), 7, True),
     # windows: fewer channels than a k-tile (several wraps of the channel), taps outside the image, strides, K that ends inside a k-tile
     (lambda: CONV(N=8, H=14, W=14, C=256, O=256, realistic=True), None, True), (lambda: CONV(N=9, H=30, W=29, C=128, O=200, realistic=True), 7, True),
     (lambda: CONV(N=10, H=61, W=60, C=48, O=336, KH=6, KW=7, pad=(2, 3, 3, 2), stride=(2, 2), realistic=True), 7, True),

@@ -447,7 +447,9 @@ __global__ __launch_bounds__(256) void igemm_i8(IgemmArgs p) {
 // DMA stream of a 4096^3 problem takes 44 us in half lines and 30 us in whole ones).  One DMA instruction then covers
 // 8 rows, slot p of row r holds chunk p ^ ((r >> 1) & 7) (row pitch 128 bytes = 32 banks: the 16 rows of a ds_read_b128
 // phase again fall into 16 distinct bank groups), and a k-tile is four MFMA phases.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, int DIRECT, bool ADD = false, bool CONV = false, int BK = 64>
+// HALF: half of the last k-tile lies beyond the weights' rows and is read from kNoWeights (in the one kernel it costs a K of whole k-tiles 2 %).
+__device__ __constant__ static const v4i kNoWeights = {0, 0, 0, 0};
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, int DIRECT, bool ADD = false, bool CONV = false, int BK = 64, bool HALF = false>
 __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BLOCKS_PER_CU) void igemm_dense_i8(IgemmArgs p) {
     static_assert(BK == 64 || BK == 128, "k-tile of 64 or 128 bytes");
     constexpr int CH = BK / 16;    // 16-byte chunks per tile row
@@ -572,7 +574,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BLOCKS_PER_CU) void igemm_de
         myScale = p.scale[n0 + tid];
     }
 
-    const int KT = p.Kp / BK;
+    const int KT = HALF ? (p.Kp + BK - 1) / BK : p.Kp / BK;
 
     // Software pipeline.  The ring holds tiles kt+1 .. kt+STAGES while tile kt is computed.
     // Each k-tile is NP MFMA phases (k slices of 32; described here for two).  While phase 0 runs, the fragments
@@ -602,7 +604,12 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BLOCKS_PER_CU) void igemm_de
                     dmaLoad16(aBase, aOff[x] - back, stage + (unsigned)(wave + NW * x) * 1024u);
                 }
             } else {
-                dmaLoad16(bBase, bOff[x - LA], stage + A_STAGE + (unsigned)((wave + NW * (x - LA)) % BWL) * 1024u);
+                const unsigned dst = stage + A_STAGE + (unsigned)((wave + NW * (x - LA)) % BWL) * 1024u;
+                if constexpr (HALF && !kWhole) {
+                    dmaLoad16(kt * BK + lchunk * 16 >= p.Kp ? (const void *)&kNoWeights : (const void *)(bBase + bOff[x - LA]), dst);
+                } else {
+                    dmaLoad16(bBase, bOff[x - LA], dst);
+                }
             }
         }
         if constexpr (CONV) {
@@ -1207,14 +1214,14 @@ static hipError_t launchIgemmLoader(const IgemmArgs &a, const LaunchCtx &ctx) {
     }
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, int DIRECT, bool ADD = false, bool CONV = false, int BK = 64>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, int DIRECT, bool ADD = false, bool CONV = false, int BK = 64, bool HALF = false>
 static hipError_t launchIgemmDenseE(const IgemmArgs &a, const LaunchCtx &ctx) {
     // the stage ring, reused by the epilogue as staging slices (one per wave) plus bias/scale
     constexpr size_t ring = (size_t)STAGES * (BM + BN) * BK;
     constexpr size_t epilogue = (size_t)(BM / WAVES_M) * (WAVES_M * WAVES_N) * (32 * 4 + 16) + 2 * BN * 4;
     constexpr size_t smem = ring > epilogue ? ring : epilogue;
     static_assert(smem * BLOCKS_PER_CU <= 160 * 1024, "LDS of one CU");
-    auto kernel = igemm_dense_i8<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, DIRECT, ADD, CONV, BK>;
+    auto kernel = igemm_dense_i8<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, DIRECT, ADD, CONV, BK, HALF>;
     static std::once_flag once;
     static hipError_t configured = hipSuccess;
     std::call_once(once, [&] { configured = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem); });
@@ -1225,7 +1232,7 @@ static hipError_t launchIgemmDenseE(const IgemmArgs &a, const LaunchCtx &ctx) {
     return hipGetLastError();
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, bool CONV = false, int BK = 64>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, bool CONV = false, int BK = 64, bool HALF = false>
 static hipError_t launchIgemmDense(const IgemmArgs &a, const LaunchCtx &ctx) {
     // the in-register epilogue takes the 32-bit requant tails: the plain one (what wideRequant() calls plain), or the
     // general one (any shift of 32 and up, or a smaller one that the record's pre_shift lifts to 33; on the small tiles
@@ -1244,9 +1251,9 @@ static hipError_t launchIgemmDense(const IgemmArgs &a, const LaunchCtx &ctx) {
             return hipErrorInvalidValue;
         }
     }
-    if (direct) return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 1, false, CONV, BK>(a, ctx);
-    if (inRegisters && wide) return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 2, false, CONV, BK>(a, ctx);
-    return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 0, false, CONV, BK>(a, ctx);
+    if (direct) return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 1, false, CONV, BK, HALF>(a, ctx);
+    if (inRegisters && wide) return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 2, false, CONV, BK, HALF>(a, ctx);
+    return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 0, false, CONV, BK, HALF>(a, ctx);
 }
 
 // Whether a tile's problem is ahead in k-tiles of 128 bytes: whole cache lines per tile row, half the barriers per byte, and fewer
@@ -1257,29 +1264,35 @@ static hipError_t launchIgemmDense(const IgemmArgs &a, const LaunchCtx &ctx) {
 //   128 x 128   one tile per CU, three stages 1024x1024x4096 8.8 / 8.4, 1024x2048x4096 13.8 / 12.8, 1024x8192x4096 42.4 / 40.1; more tiles, two stages,
 //     two workgroups per CU 3000x1024x2048 12.6 / 11.0, 2000x2048x3072 20.5 / 18.0, 1400x3072x4096 29.2 / 23.7
 //   128 x 64, three stages   300x4096x4096 14.4 / 14.2, 768x4096x2048 15.2 / 14.9, but 300x2048x4096 8.4 / 8.8
+// With half of the last k-tile beyond the weights' rows (Kp % 128 == 64) the lines lie later:
+//   64 x 64      700x2112x640 6.8 / 6.9, 512x3136x2048 9.1 / 9.0, 700x5696x640 13.7 / 12.8; windows 3x3 28x28x144 -> 256, batch 4 7.8 / 7.3, 14x14x304 -> 304, batch 8 12.1 / 10.4
+//   64 x 128     600x1472x4096 10.4 / 11.1, 600x2112x4096 15.2 / 14.4, 600x5696x4096 36.8 / 32.1
+//   128 x 128    3000x1472x1024 9.1 / 10.0, 3000x2112x1024 13.8 / 12.7, 1400x2112x3072 20.0 / 17.3, 1400x5696x3072 48.3 / 38.6
+//   128 x 64     300x3136x4096 11.2 / 11.1, 300x5696x4096 20.2 / 19.5
 // (Four to six stages are 0 - 5 % behind three: the loads are bound by what they carry, not by their latency.)
 bool igemmWideBetter(const IgemmArgs &a, uint32_t variant) {
-    if ((a.loader != kLoaderDense && a.loader != kLoaderWindow) || a.skip != nullptr || a.Kp % 128 != 0) return false;
+    if ((a.loader != kLoaderDense && a.loader != kLoaderWindow) || a.skip != nullptr) return false;
+    const bool half = a.Kp % 128 != 0, window = a.loader == kLoaderWindow;
     switch (variant) {
-    case kIgemmDense64x64: return a.Kp >= 1152;
-    case kIgemmDense64x128: return a.Kp >= 1024 && a.loader == kLoaderDense;
-    case kIgemmDense128x128: return a.Kp >= 1024;
-    case kIgemmDense128x64: return a.Kp >= 4096 && a.loader == kLoaderDense;
+    case kIgemmDense64x64: return a.Kp >= (!half ? 1152 : window ? 1344 : 2560);
+    case kIgemmDense64x128: return a.Kp >= (half ? 2048 : 1024) && !window;
+    case kIgemmDense128x128: return a.Kp >= (half ? 2048 : 1024);
+    case kIgemmDense128x64: return a.Kp >= 4096 && !window;
     default: return false;
     }
 }
-template <bool CONV>
+template <bool CONV, bool HALF>
 static hipError_t launchIgemmWide(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ctx) {
     auto tiles = [&](int bm, int bn) { return (long long)((a.M + bm - 1) / bm) * (a.Np / bn); };
     switch (variant) {
-    case kIgemmDense64x64: return launchIgemmDense<64, 64, 2, 2, 3, 3, CONV, 128>(a, ctx);
-    case kIgemmDense128x128: return tiles(128, 128) <= 256 ? launchIgemmDense<128, 128, 2, 2, 3, 1, CONV, 128>(a, ctx) : launchIgemmDense<128, 128, 2, 2, 2, 2, CONV, 128>(a, ctx);
+    case kIgemmDense64x64: return launchIgemmDense<64, 64, 2, 2, 3, 3, CONV, 128, HALF>(a, ctx);
+    case kIgemmDense128x128: return tiles(128, 128) <= 256 ? launchIgemmDense<128, 128, 2, 2, 3, 1, CONV, 128, HALF>(a, ctx) : launchIgemmDense<128, 128, 2, 2, 2, 2, CONV, 128, HALF>(a, ctx);
     case kIgemmDense64x128:
         // (one workgroup per CU has all registers: 512 x 4096 x 4096 13.7 us against 14.4)
-        if constexpr (!CONV) return tiles(64, 128) <= 256 ? launchIgemmDense<64, 128, 2, 2, 3, 1, false, 128>(a, ctx) : launchIgemmDense<64, 128, 2, 2, 3, 2, false, 128>(a, ctx);
+        if constexpr (!CONV) return tiles(64, 128) <= 256 ? launchIgemmDense<64, 128, 2, 2, 3, 1, false, 128, HALF>(a, ctx) : launchIgemmDense<64, 128, 2, 2, 3, 2, false, 128, HALF>(a, ctx);
         return hipErrorInvalidValue;
     case kIgemmDense128x64:
-        if constexpr (!CONV) return launchIgemmDense<128, 64, 2, 2, 3, 2, false, 128>(a, ctx);
+        if constexpr (!CONV) return launchIgemmDense<128, 64, 2, 2, 3, 2, false, 128, HALF>(a, ctx);
         return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
     }
@@ -1313,7 +1326,7 @@ hipError_t launchIgemm(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ct
         if (a.M % (a.OH * a.OW) != 0 || (long long)a.K != (long long)a.KH * a.KW * a.C || a.Kp != (a.K + t.bk - 1) / t.bk * t.bk) return hipErrorInvalidValue;
         if (a.a_bytes != (long long)(a.M / (a.OH * a.OW)) * a.H * a.W * a.C || a.a_bytes >= (1LL << 32)) return hipErrorInvalidValue;
         if (((uintptr_t)a.A & 15) != 0 || a.skip != nullptr) return hipErrorInvalidValue;
-        if (wide) return launchIgemmWide<true>(a, variant, ctx);
+        if (wide) return a.Kp % 128 ? launchIgemmWide<true, true>(a, variant, ctx) : launchIgemmWide<true, false>(a, variant, ctx);
         switch (variant) {
         case kIgemmDense256x256: return launchIgemmDense<256, 256, 2, 2, 4, 1, true>(a, ctx);
         case kIgemmDense128x256:
@@ -1340,7 +1353,7 @@ hipError_t launchIgemm(const IgemmArgs &a, uint32_t variant, const LaunchCtx &ct
     if (((uintptr_t)a.Bp & 15) != 0) return hipErrorInvalidValue;
     if (a.out_dtype < kDtypeI8 || a.out_dtype > kDtypeI32) return hipErrorInvalidValue;
     if (a.skip != nullptr && variant != kIgemmStream && variant != kIgemmDense64x64) return hipErrorInvalidValue;  // the kernels that can add a residual
-    if (wide) return launchIgemmWide<false>(a, variant, ctx);
+    if (wide) return a.Kp % 128 ? launchIgemmWide<false, true>(a, variant, ctx) : launchIgemmWide<false, false>(a, variant, ctx);
     switch (variant) {
     case kIgemm128x128x64: return launchIgemmLoader<128, 128, 64>(a, ctx);
     case kIgemm256x256x64: return launchIgemmLoader<256, 256, 64>(a, ctx);
