@@ -1,5 +1,5 @@
 """A decoder's step as one launch (dec_chain): which programs take it, each op against the oracle on the inputs the GPU gave it at the sizes where
-the kernel can go wrong, a launch whose workgroups give up waiting, executables in turn, and buffers that share memory."""
+the kernel can go wrong, what it may load, a launch whose workgroups give up waiting, executables in turn, and buffers that share memory."""
 import subprocess
 
 import numpy as np
@@ -21,6 +21,27 @@ def plan(tmp_path_factory):
         return subprocess.run([exe, str(path)], check=True, stdout=subprocess.PIPE, text=True, env=env).stdout.splitlines()
 
     return run
+
+
+def linears(rows, widths, zero_points=False, seed=1060):
+    """Linears on block-quantized weights one behind the other, widths[0] -> widths[1] -> ..., every result an output binding and nothing
+    behind the last one: its weights and biases are the last constants of the program."""
+    rng = np.random.default_rng(seed)
+    p = thip.Program()
+    x_in = w.to_bf16(rng.standard_normal((rows, widths[0])))
+    x, ops, names, outputs = p.binding(0, x_in.shape, np.uint16), [], ["x_in"], []
+    for i, (K, N) in enumerate(zip(widths, widths[1:])):
+        wq, scale, qbias = w._block_quantized(rng, K, N, 128, 1.0)
+        if zero_points:
+            qbias = (-rng.integers(-8, 9, size=qbias.shape)).astype(np.float32) * w.from_bf16_np(scale)
+        w16 = p.expand_weights(wq, scale, qbias, block_size=128, output_min=w.NO_CLAMP[0], output_max=w.NO_CLAMP[1])
+        x = p.matmul(x, w16, np.zeros(1, np.float32), init=p.binding(i + 1, (rows, N), np.uint16), output_zp=0, output_min=w.NO_CLAMP[0],
+                     output_max=w.NO_CLAMP[1], shift=0)
+        ops.append(w.DecoderOp("linear", "y%d" % i, [names[-1]], (rows, N), weights=wq, scale=scale, qbias=qbias, block=128))
+        names.append("y%d" % i)
+        outputs.append(((rows, N), np.uint16))
+    return w.Workload("linears_%dx%s%s" % (rows, "-".join(map(str, widths)), "_zp" if zero_points else ""), p, [x_in], outputs, 0, 0,
+                      dict(ops=ops, names=names[1:]))
 
 
 STEP = dict(layers=2, hidden=256, heads=2, head_dim=64, ffn=512, vocab=512, cache_len=64)
@@ -51,6 +72,36 @@ def test_weights_written_by_the_program_are_not_fetched_ahead(plan):
     p.matmul(y, p.transpose(made, (0, 2, 1)), zero, init=p.binding(2, (1, 4, 4), np.uint16), **none)
     lines = plan(p.serialize(), env={"THIP_DEC_CHAIN": "1"})
     assert lines[:2] == ["dec_chain 0 5", "record 5 1"], lines
+
+
+@pytest.fixture(scope="module")
+def loads(tmp_path_factory):
+    exe = host_check("chain_loads", tmp_path_factory.mktemp("loads"))
+
+    def run(blob):
+        """-> phases, linear ones, matmuls, linear ones with two jobs to a tile, and of these with an odd number of k-blocks"""
+        path = tmp_path_factory.mktemp("blob") / "p.thip"
+        path.write_bytes(blob)
+        done = subprocess.run([exe, str(path)], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120, env={"THIP_DEC_CHAIN": "1"})
+        assert done.returncode == 0, done.stdout
+        return [int(v) for v in done.stdout.split()]
+
+    return run
+
+
+# k-blocks: 11 and 13 in two halves to a tile, one half of the last unit not there; 12 and 10; 9 and 2, a job to a tile
+@pytest.mark.parametrize("zero_points", [False, True])
+@pytest.mark.parametrize("widths,shared,odd", [((256, 1408, 256, 1408, 256), 2, 2), ((1664, 1536, 1280, 48), 3, 1), ((1152, 256, 4096, 128), 1, 0),
+                                               ((1408, 2048, 2176, 1408, 16), 3, 3)], ids=str)
+def test_weights_loaded_of_linears(loads, widths, shared, odd, zero_points):
+    assert loads(linears(2, widths, zero_points).program.serialize()) == [len(widths) - 1, len(widths) - 1, 0, shared, odd]
+
+
+@pytest.mark.parametrize("case", [dict(), dict(cache_len=24, head_dim=72, heads=16), dict(cache_len=8, head_dim=8, heads=16), dict(hidden=1408, ffn=1664, vocab=2064, cache_len=1032, batch=3),
+                                  dict(heads=16, head_dim=200, hidden=128, cache_len=40, batch=4)], ids=str)
+def test_weights_loaded_of_steps(loads, case):
+    phases, linear, matmul, shared, odd = loads(w.decoder_step_workload(**dict(dict(batch=1), **dict(STEP, **case))).program.serialize())
+    assert phases >= 2 and linear + matmul == phases, (phases, linear, matmul)
 
 
 # ---- GPU ----------------------------------------------------------------------------------------------------------
@@ -107,6 +158,29 @@ def test_gpu_every_op(device, monkeypatch, case, wait):
                 prog.check_decoder_step(wl, outs, prog.assert_bf16_close, prog.assert_bit_exact)
                 first = outs
             assert all(np.array_equal(a, b) for a, b in zip(outs, first))
+    finally:
+        exe.close()
+        for q in ptrs:
+            device.free(q)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wait", [None, "0"], ids=["together", "given_up"])
+@pytest.mark.parametrize("zero_points", [False, True])
+@pytest.mark.parametrize("widths", [(256,) + (1408, 256) * 4, (1664, 1664, 48)], ids=str)
+def test_gpu_nothing_behind_the_last_weights(device, monkeypatch, widths, zero_points, wait):
+    """The last unit of the last matrix has a half that is not there, and nothing lies behind it."""
+    monkeypatch.setenv("THIP_DEC_CHAIN", "1")
+    if wait is not None:
+        monkeypatch.setenv("THIP_DEC_CHAIN_WAIT", wait)
+    wl = linears(1, widths, zero_points)
+    print("[gpu-case]", wl.name, wait, flush=True)
+    exe = _load(device, wl)
+    ptrs, lens = _buffers(device, wl)
+    try:
+        for _ in range(3):
+            exe.run_device(ptrs, lens)
+            prog.check_grouped_linear(wl, _outputs(device, wl, ptrs), prog.assert_bf16_close, prog.assert_bit_exact)
     finally:
         exe.close()
         for q in ptrs:

@@ -1,8 +1,8 @@
 // A run of decode-shaped records (grouped linears and batched small matmuls, each reading what one before it wrote) as one launch:
-// the table that the kernel walks, shared by the planner (host only) and the kernel.
+// the table that the kernel walks and the index arithmetic of its weights, shared by the planner (host only) and the kernel.
 #pragma once
 
-#include <stdint.h>
+#include "thip_kernels.h"
 
 namespace thip {
 
@@ -55,5 +55,59 @@ struct DecChainArgs {
     uint8_t *bindings[64];
 };
 constexpr uint64_t kChainSyncHead = 96;  // words in front of the exchange
+
+// Index arithmetic of the weights, shared by the kernel and a check on the host.
+
+// A job of a linear makes the same tile of a pair's matrices, or a tile of one of up to three.
+struct ChainTile {
+    int seg, tile;
+};
+__host__ __device__ inline ChainTile chainTile(int tile, int nmat, int nseg, int tiles0, int tiles1) {
+    if (nmat > 1 || nseg < 2 || tile < tiles0) return ChainTile{0, tile};
+    if (nseg < 3 || tile < tiles0 + tiles1) return ChainTile{1, tile - tiles0};
+    return ChainTile{2, tile - tiles0 - tiles1};
+}
+
+// The units of a result, one behind the other: where the first one starts in the operand, how many bytes may be read from there on (a load
+// of what lies beyond returns zero and touches no memory), and a unit's bytes; then, from the start of a unit, its scales, from its
+// weights the second half of them, and from a scale its bias.
+struct ChainUnits {
+    uint64_t first;
+    uint32_t bytes, unitBytes, scales, half, bias;
+};
+// A linear's end with their tile: where two jobs share one of an odd number of k-blocks, the second half of the last unit is not there, and
+// behind it lies another tile, or what follows the matrix, which may be nothing.
+// odd: of a shared tile's two jobs the one with columns 8 .. 15.
+__host__ __device__ inline ChainUnits chainLinearUnits(int K, int slotBytes, int split, int tile, int odd) {
+    ChainUnits u;
+    u.first = (uint64_t)((uint32_t)tile * (uint32_t)(K >> 7)) * (uint32_t)slotBytes + (uint32_t)(odd * 128);
+    u.bytes = (uint32_t)(K >> 7) * (uint32_t)slotBytes - (uint32_t)(odd * 128);
+    u.unitBytes = (uint32_t)(split * slotBytes);
+    u.scales = 2048u - (uint32_t)(odd * 96);
+    u.half = 1024;
+    u.bias = slotBytes > kDecSlotBytes ? 64 : 0;
+    return u;
+}
+// A matmul's end with the operand.  wBytes: of it; wStride: elements from one batch element to the next.
+__host__ __device__ inline ChainUnits chainMatmulUnits(int K, uint32_t wBytes, int wStride, int batch, int tile) {
+    ChainUnits u;
+    const uint32_t at = ((uint32_t)batch * (uint32_t)wStride + (uint32_t)(tile * 16 * K)) * 2u;
+    u.first = at;
+    u.bytes = wBytes - at;
+    u.unitBytes = 128;
+    u.scales = 0;
+    u.half = 64;
+    u.bias = 0;
+    return u;
+}
+// Where lane (c = lane & 15, g = lane >> 4) finds its weights and its scale in a unit (a lane of a matmul has none).
+struct ChainLane {
+    uint32_t weights, scales;
+};
+__host__ __device__ inline ChainLane chainLinearLane(int c, int g, int slotBytes, int split) {
+    const int column = split == 1 ? c : c & 7, second = split == 1 ? 0 : c >> 3;
+    return ChainLane{(uint32_t)(second * slotBytes + (g * 16 + column) * 16), (uint32_t)(second * slotBytes + column * 4)};
+}
+__host__ __device__ inline ChainLane chainMatmulLane(int c, int g, int K) { return ChainLane{(uint32_t)((c * K + 8 * g) * 2), 0}; }
 
 }  // namespace thip

@@ -133,52 +133,41 @@ struct ChainSlot {
     v4i p0, p1;
     float sc, bi;
 };
-// Where the weights of a pass lie.  Lane r: the first unit of result r, its bytes up to the end of a matmul's operand (what lies beyond reads as
-// zero), and the distance of its scales; then what all units have in common.
+// Where the weights of a pass lie (see ChainUnits).  Lane r: the first unit of result r, the bytes that may be read from there on, and its
+// scales; then what all units have in common.
 struct ChainWeights {
     uint32_t lo, hi, bytes, scales;
-    uint32_t lane0, lane1;           // of a lane, into a unit: weights, scales
-    uint32_t unitBytes, half, bias;  // uniform: of a unit; to the second half of its weights; from a scale to its bias
+    ChainLane lane;
+    uint32_t unitBytes, half, bias;  // uniform
 };
 __device__ __forceinline__ ChainWeights chainWeights(const DecChainArgs &p, const ChainGroup &q, const ChainWalk &w) {
-    ChainWeights t;
     const int c = q.lane & 15, g = q.lane >> 4, K = PHASE_INT(w.entry, K), slotBytes = PHASE_INT(w.entry, slotBytes);
     const int result = q.lane < w.results ? q.lane : 0, job = chainJob(q, w, result >> (w.nmat - 1));
+    ChainWeights t;
+    ChainUnits u;
+    uint64_t base;
     if (slotBytes == 0) {  // a matmul
-        const int b = chainBatch(w, job), tile = job - b * PHASE_INT(w.entry, tiles);
-        const uint64_t base = (uint64_t)(uintptr_t)chainAddress(p, PHASE_REF(w.entry, w, 0));
-        const uint32_t at = ((uint32_t)b * (uint32_t)PHASE_INT(w.entry, wStride) + (uint32_t)(tile * 16 * K)) * 2u;
-        t.lo = (uint32_t)(base + at);
-        t.hi = (uint32_t)((base + at) >> 32);
-        t.bytes = (uint32_t)PHASE_INT(w.entry, wBytes) - at;
-        t.scales = 0;
-        t.lane0 = (uint32_t)((c * K + 8 * g) * 2);
-        t.lane1 = 0;
-        t.unitBytes = 128;
-        t.half = 64;
-        t.bias = 0;
+        const int b = chainBatch(w, job);
+        base = (uint64_t)(uintptr_t)chainAddress(p, PHASE_REF(w.entry, w, 0));
+        u = chainMatmulUnits(K, (uint32_t)PHASE_INT(w.entry, wBytes), PHASE_INT(w.entry, wStride), b, job - b * PHASE_INT(w.entry, tiles));
+        t.lane = chainMatmulLane(c, g, K);
     } else {
-        const int split = PHASE_INT(w.entry, split), nseg = PHASE_INT(w.entry, nseg);
-        const int tiles0 = PHASE_INT(w.entry, N[0]) >> 4, tiles1 = PHASE_INT(w.entry, N[1]) >> 4;
-        int tile = split == 1 ? job : job >> 1, seg = result & (w.nmat - 1);
-        if (w.nmat == 1 && nseg > 1) {
-            seg = tile < tiles0 ? 0 : nseg < 3 || tile < tiles0 + tiles1 ? 1 : 2;
-            tile -= seg == 0 ? 0 : seg == 1 ? tiles0 : tiles0 + tiles1;
-        }
-        const int odd = split == 1 ? 0 : job & 1;  // of a tile's two jobs the one with columns 8 .. 15
-        const v2i first = *(const v2i *)(q.table + w.phase * 64 + (int)(offsetof(ChainPhase, w) / 4) + 2 * seg);  // a constant: an address
-        const uint64_t base = ((uint64_t)(uint32_t)first[0] | (uint64_t)(uint32_t)first[1] << 32) + (uint64_t)((uint32_t)tile * (uint32_t)(K >> 7)) * (uint32_t)slotBytes + (uint32_t)(odd * 128);
-        t.lo = (uint32_t)base;
-        t.hi = (uint32_t)(base >> 32);
-        t.bytes = 0x7fffffffu;
-        t.scales = 2048u - (uint32_t)(odd * 96);
-        const int column = split == 1 ? c : c & 7, second = split == 1 ? 0 : c >> 3;
-        t.lane0 = (uint32_t)(second * slotBytes + (g * 16 + column) * 16);
-        t.lane1 = (uint32_t)(second * slotBytes + column * 4);
-        t.unitBytes = (uint32_t)(split * slotBytes);
-        t.half = 1024;
-        t.bias = slotBytes > kDecSlotBytes ? 64 : 0;
+        const int split = PHASE_INT(w.entry, split);
+        const ChainTile tile = chainTile(split == 1 ? job : job >> 1, w.nmat, PHASE_INT(w.entry, nseg), PHASE_INT(w.entry, N[0]) >> 4, PHASE_INT(w.entry, N[1]) >> 4);
+        const int matrix = w.nmat > 1 ? result & 1 : tile.seg;
+        const v2i first = *(const v2i *)(q.table + w.phase * 64 + (int)(offsetof(ChainPhase, w) / 4) + 2 * matrix);  // a constant: an address
+        base = (uint64_t)(uint32_t)first[0] | (uint64_t)(uint32_t)first[1] << 32;
+        u = chainLinearUnits(K, slotBytes, split, tile.tile, split == 1 ? 0 : job & 1);
+        t.lane = chainLinearLane(c, g, slotBytes, split);
     }
+    base += u.first;
+    t.lo = (uint32_t)base;
+    t.hi = (uint32_t)(base >> 32);
+    t.bytes = u.bytes;
+    t.scales = u.scales;
+    t.unitBytes = u.unitBytes;
+    t.half = u.half;
+    t.bias = u.bias;
     return t;
 }
 // Unit `u` of `w`'s pass into a slot.  All of a slot is loaded or nothing: behind a branch around a single register of it the compiler
@@ -191,10 +180,10 @@ __device__ __forceinline__ void chainLoad(const ChainWalk &w, const ChainWeights
     const uint32_t bytes = (uint32_t)__builtin_amdgcn_readlane((int)t.bytes, result);
     const int scales = __builtin_amdgcn_readlane((int)t.scales, result);
     const auto all = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, bytes - at, 0x00027000);  // a unit's first row exists
-    s.p0 = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(all, (int)t.lane0, 0, 0));
-    s.p1 = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(all, (int)t.lane0, __builtin_amdgcn_readfirstlane((int)t.half), 0));
-    s.sc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(all, (int)t.lane1, scales, 0));
-    s.bi = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(all, (int)t.lane1, scales + __builtin_amdgcn_readfirstlane((int)t.bias), 0));
+    s.p0 = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(all, (int)t.lane.weights, 0, 0));
+    s.p1 = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(all, (int)t.lane.weights, __builtin_amdgcn_readfirstlane((int)t.half), 0));
+    s.sc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(all, (int)t.lane.scales, scales, 0));
+    s.bi = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(all, (int)t.lane.scales, scales + __builtin_amdgcn_readfirstlane((int)t.bias), 0));
 }
 
 // This wave's share of a result, to LDS.
@@ -437,14 +426,11 @@ __device__ __forceinline__ ChainItem chainItem(const DecChainArgs &p, const Chai
         it.where = (uint32_t)b * (uint32_t)PHASE_INT(w.entry, outStride) + (uint32_t)(m * N + n);
         it.bias[0] = PHASE_FLOAT(w.entry, bias0);
     } else {
-        int tile = o.split == 1 ? job : job >> 1;
-        if (w.nmat == 1 && o.nseg > 1) {
-            const int N1 = PHASE_INT(w.entry, N[1]), N2 = PHASE_INT(w.entry, N[2]), tiles0 = N >> 4, tiles1 = N1 >> 4;
-            seg = tile < tiles0 ? 0 : o.nseg < 3 || tile < tiles0 + tiles1 ? 1 : 2;
-            tile -= seg == 0 ? 0 : seg == 1 ? tiles0 : tiles0 + tiles1;
-            N = seg == 0 ? N : seg == 1 ? N1 : N2;
-        }
-        const int n = tile * 16 + (o.split == 1 ? 0 : (job & 1) * 8) + column;
+        const int N1 = PHASE_INT(w.entry, N[1]), N2 = PHASE_INT(w.entry, N[2]);
+        const ChainTile t = chainTile(o.split == 1 ? job : job >> 1, w.nmat, o.nseg, N >> 4, N1 >> 4);
+        seg = t.seg;
+        N = seg == 0 ? N : seg == 1 ? N1 : N2;
+        const int n = t.tile * 16 + (o.split == 1 ? 0 : (job & 1) * 8) + column;
         it.where = (uint32_t)(m * N + n);
         // constants: addresses
         const ChainRef b0 = PHASE_REF(w.entry, bias, 0), b1 = PHASE_REF(w.entry, bias, 1), b2 = PHASE_REF(w.entry, bias, 2);
