@@ -53,7 +53,6 @@ int main(int argc, char **argv) {
             (t.slotBytes ? linear : matmul)++;
             shared += t.split > 1;
             odd += t.split > 1 && blocks % 2 != 0;
-            if (!t.slotBytes) continue;
             for (job = 0; job < t.jobs; job++) {
                 for (int mat = 0; mat < t.nmat; mat++) {
                     ChainUnits u;
@@ -85,7 +84,7 @@ int main(int argc, char **argv) {
                                 const uint64_t slot = (uint64_t)(tile.tile * blocks + block) * t.slotBytes;
                                 if (where + l.weights != slot + (uint64_t)(g * 16 + column) * 16) return fail("other weights", unit, lane, 0);
                                 if (where + l.scales + u.scales != slot + 2048 + column * 4) return fail("another scale", unit, lane, 0);
-                                if (load(operand, where, bytes, l.weights, 0, 4, needed, unit, lane) || load(operand, where, bytes, l.weights, u.half, 4, needed, unit, lane) ||
+                                if (load(operand, where, bytes, l.weights, 0, 4, needed, unit, lane) || load(operand, where, bytes, l.weights + u.half, 0, 4, needed, unit, lane) ||
                                     load(operand, where, bytes, l.scales, u.scales, 1, needed, unit, lane) || load(operand, where, bytes, l.scales, u.scales + u.bias, 1, needed, unit, lane)) return 1;
                             } else {
                                 const ChainLane l = chainMatmulLane(c, g, t.K);

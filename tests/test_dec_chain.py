@@ -104,6 +104,18 @@ def test_weights_loaded_of_steps(loads, case):
     assert phases >= 2 and linear + matmul == phases, (phases, linear, matmul)
 
 
+@pytest.mark.parametrize("N", [1, 3, 17, 33])
+@pytest.mark.parametrize("K", [8, 24, 40, 72, 104])
+def test_weights_loaded_of_matmuls(loads, N, K):
+    """Few columns and few of K: the last row of the operand ends inside the first half of a unit."""
+    p = thip.Program()
+    zero, none = np.zeros(1, np.float32), dict(output_zp=0, output_min=w.NO_CLAMP[0], output_max=w.NO_CLAMP[1], shift=0)
+    for i in range(2):
+        rhs = p.transpose(p.binding(3 * i + 1, (2, N, K), np.uint16), (0, 2, 1))
+        p.matmul(p.binding(3 * i, (2, 4, K), np.uint16), rhs, zero, init=p.binding(3 * i + 2, (2, 4, N), np.uint16), **none)
+    assert loads(p.serialize()) == [2, 0, 2, 0, 0]
+
+
 # ---- GPU ----------------------------------------------------------------------------------------------------------
 
 SHAPES = [

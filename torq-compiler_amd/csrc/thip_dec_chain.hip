@@ -179,9 +179,11 @@ __device__ __forceinline__ void chainLoad(const ChainWalk &w, const ChainWeights
     const uint64_t base = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)t.lo, result) | (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)t.hi, result) << 32) + at;
     const uint32_t bytes = (uint32_t)__builtin_amdgcn_readlane((int)t.bytes, result);
     const int scales = __builtin_amdgcn_readlane((int)t.scales, result);
-    const auto all = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, bytes - at, 0x00027000);  // a unit's first row exists
+    // A unit's first row exists.  The second half of a matmul's unit may not: it is told apart by the lane's own offset, which is always held against
+    // `bytes`.  The uniform offset of the scales need not be (a scale that is not there lies behind weights that are not).
+    const auto all = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, bytes - at, 0x00027000);
     s.p0 = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(all, (int)t.lane.weights, 0, 0));
-    s.p1 = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(all, (int)t.lane.weights, __builtin_amdgcn_readfirstlane((int)t.half), 0));
+    s.p1 = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(all, (int)t.lane.weights + __builtin_amdgcn_readfirstlane((int)t.half), 0, 0));
     s.sc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(all, (int)t.lane.scales, scales, 0));
     s.bi = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(all, (int)t.lane.scales, scales + __builtin_amdgcn_readfirstlane((int)t.bias), 0));
 }
