@@ -1,0 +1,77 @@
+// The turns of executables that have a dec_chain launch, on a HIP of this file's own: which dispatches wait for which, and what is asked of
+// the runtime when.
+#include <stdio.h>
+
+#include <map>
+#include <set>
+#include <vector>
+
+#include "thip_chain_turn.h"
+
+using namespace thip;
+
+// A stream is busy while it is in `busy`.  An event remembers the stream that it was recorded on last.
+static std::set<hipStream_t> busy;
+static std::map<hipEvent_t, hipStream_t> recorded;
+static std::vector<std::pair<hipStream_t, hipStream_t>> waits;  // who waits, for whose work
+static int created, failures;
+
+extern "C" hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+    *e = (hipEvent_t)(intptr_t)++created;
+    return hipSuccess;
+}
+extern "C" hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+    recorded[e] = s;
+    return e ? hipSuccess : hipErrorInvalidHandle;
+}
+extern "C" hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+    waits.push_back({s, recorded[e]});
+    return hipSuccess;
+}
+extern "C" hipError_t hipStreamQuery(hipStream_t s) { return busy.count(s) ? hipErrorNotReady : hipSuccess; }
+extern "C" hipError_t hipGetLastError() { return hipSuccess; }
+
+#define CHECK(what) do { if (!(what)) failures++, printf("line %d: %s\n", __LINE__, #what); } while (0)
+
+static hipStream_t streamOf(int n) { return (hipStream_t)(intptr_t)(100 * n); }
+
+// One dispatch.
+static void dispatch(ChainTurns *turns, ChainMember *m) {
+    waits.clear();
+    ChainTurns::Turn turn;
+    CHECK(turn.take(turns, m) == hipSuccess);
+    busy.insert(m->stream);
+}
+
+static void inTurn() {
+    ChainTurns turns;
+    ChainMember a, b;
+    a.stream = streamOf(1);
+    b.stream = streamOf(2);
+    const int before = created;
+    CHECK(turns.join(&a) == hipSuccess && turns.join(&b) == hipSuccess);
+    // a dispatch makes nothing (thip_executable_enqueue_noalloc)
+    const int made = created;
+    CHECK(made > before);
+    dispatch(&turns, &a);
+    CHECK(waits.empty());
+    dispatch(&turns, &a);
+    CHECK(waits.empty());
+    dispatch(&turns, &b);
+    CHECK(waits.size() == 1 && waits[0] == std::make_pair(b.stream, a.stream));
+    dispatch(&turns, &a);
+    CHECK(waits.size() == 1 && waits[0] == std::make_pair(a.stream, b.stream));
+    CHECK(created == made);
+    busy.clear();
+    turns.leave(&a);
+    dispatch(&turns, &b);
+    CHECK(waits.empty());
+    busy.clear();
+    turns.leave(&b);
+}
+
+int main() {
+    inTurn();
+    if (failures == 0) puts("in order");
+    return failures != 0;
+}

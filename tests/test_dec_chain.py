@@ -116,6 +116,12 @@ def test_weights_loaded_of_matmuls(loads, N, K):
     assert loads(p.serialize()) == [2, 0, 2, 0, 0]
 
 
+def test_turns(tmp_path):
+    exe = host_check("chain_turn", tmp_path, sanitize=["thip_chain_turn.cpp"])
+    done = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert done.returncode == 0 and done.stdout == "in order\n", done.stdout[-3000:]
+
+
 # ---- GPU ----------------------------------------------------------------------------------------------------------
 
 SHAPES = [

@@ -14,7 +14,7 @@ LIB = os.path.join(HERE, "libthip.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
 SOURCES = ["thip_igemm.hip", "thip_bandwidth.hip", "thip_bf16.hip", "thip_bf16_tile.hip", "thip_decode.hip", "thip_dec_chain.hip", "thip_igemm_direct.hip", "thip_conv_patch.hip", "thip_matmul_rt.hip", "thip_inverted_residual.hip", "thip_device_util.hip", "thip_driver.cpp", "thip_emitter.cpp",
-           "thip_validate.cpp", "thip_plan.cpp", "thip_status.cpp", "thip_host_copy.cpp"]
+           "thip_validate.cpp", "thip_plan.cpp", "thip_status.cpp", "thip_host_copy.cpp", "thip_chain_turn.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
@@ -26,7 +26,7 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
           "-Xclang", "-target-feature", "-Xclang", "-dot6-insts"]
 
 
-HEADERS = ["thip_kernels.h", "thip_kernels_common.h", "thip_descriptor.h", "thip_status.h", "thip_validate.h", "thip_plan.h", "thip_inverted_residual.h", "thip_dec_chain.h", "thip_host_copy.h"]
+HEADERS = ["thip_kernels.h", "thip_kernels_common.h", "thip_descriptor.h", "thip_status.h", "thip_validate.h", "thip_plan.h", "thip_inverted_residual.h", "thip_dec_chain.h", "thip_host_copy.h", "thip_chain_turn.h"]
 
 
 def _up_to_date(src, obj):

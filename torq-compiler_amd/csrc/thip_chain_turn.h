@@ -1,0 +1,41 @@
+// Launches of dec_chain on a device, of all the executables that have one.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <mutex>
+
+namespace thip {
+
+// An executable's part.
+struct ChainMember {
+    hipStream_t stream = nullptr;
+};
+
+// The workgroups of a launch wait for one another and need a CU each at the same time.  Two such launches at once could each hold
+// CUs that the other waits for, so the executables of a device take turns: a dispatch on another stream than the last one's starts behind it.
+class ChainTurns {
+public:
+    static ChainTurns &of(int ordinal);  // one per device and process
+
+    // When an executable is made (its device is current): what turns need is there from then on.
+    hipError_t join(ChainMember *m);
+    // Its stream is idle.
+    void leave(ChainMember *m);
+
+    // Of one dispatch, from before its launches until they are enqueued.
+    class Turn {
+    public:
+        hipError_t take(ChainTurns *turns, ChainMember *m);
+
+    private:
+        std::unique_lock<std::mutex> lock;
+    };
+
+private:
+    std::mutex mutex;
+    ChainMember *last = nullptr;  // whose launch was the last one
+    hipEvent_t event = nullptr;   // behind it, recorded when another one's follows
+};
+
+}  // namespace thip

@@ -28,6 +28,7 @@
 #include <thread>
 #include <vector>
 
+#include "thip_chain_turn.h"
 #include "thip_descriptor.h"
 #include "thip_host_copy.h"
 #include "thip_kernels.h"
@@ -103,21 +104,10 @@ struct thip_executable_t {
     std::vector<std::string> launchNames;  // their kernels
     std::vector<uint8_t *> stepBuffers;  // two per step: operands of space kSpacePlan; or the table and the counters of a chain (null: none)
     bool chained = false;                // a step's workgroups wait for one another (kStepDecChain)
+    ChainMember chain;                   // then: among the device's executables that have such a step
     std::vector<uint64_t> scratchOffset;
     uint64_t scratchBytes = 0;
 };
-
-// The workgroups of a launch that wait for one another need a CU each at the same time.  Two such launches at once could each hold
-// CUs that the other waits for, so the executables of a device take turns: a dispatch on another stream than the last one's starts behind it.
-struct ChainTurn {
-    std::mutex mutex;
-    hipStream_t last = nullptr;
-    hipEvent_t event = nullptr;
-};
-static ChainTurn &chainTurn(int ordinal) {
-    static ChainTurn turns[64];
-    return turns[ordinal & 63];
-}
 
 static thip_status_t hipFail(hipError_t e, const char *what) {
     const thip_status_t code = e == hipErrorOutOfMemory ? THIP_RESOURCE_EXHAUSTED : THIP_INTERNAL;
@@ -674,24 +664,16 @@ static bool retireReplay(thip_executable_t *e, thip_executable_t::Replay *r) {
     return true;
 }
 
-// Makes a dispatch of an executable with a chain wait for the last one of another.  `turn`: held until the dispatch is enqueued.
-static thip_status_t takeChainTurn(thip_executable_t *e, std::unique_lock<std::mutex> *turn) {
-    if (!e->chained) return THIP_OK;
-    ChainTurn &t = chainTurn(e->device->ordinal);
-    *turn = std::unique_lock<std::mutex>(t.mutex);
-    if (t.last && t.last != e->stream) {
-        if (!t.event) THIP_HIP(hipEventCreateWithFlags(&t.event, hipEventDisableTiming), "hipEventCreate");
-        THIP_HIP(hipEventRecord(t.event, t.last), "hipEventRecord");
-        THIP_HIP(hipStreamWaitEvent(e->stream, t.event, 0), "hipStreamWaitEvent");
-    }
-    t.last = e->stream;
+// Takes the turn of a dispatch, if its launches are such that executables take turns.
+static thip_status_t takeTurn(thip_executable_t *e, ChainTurns::Turn *turn) {
+    if (e->chained) THIP_HIP(turn->take(&ChainTurns::of(e->device->ordinal), &e->chain), "waiting for another executable's launch");
     return THIP_OK;
 }
 
 // Enqueues one dispatch on device bindings, through the set's graph when there is one.
 static thip_status_t enqueueDevice(thip_executable_t *e, uint8_t *const *bp) {
-    std::unique_lock<std::mutex> turn;
-    if (thip_status_t s = takeChainTurn(e, &turn)) return s;
+    ChainTurns::Turn turn;
+    if (thip_status_t s = takeTurn(e, &turn)) return s;
     const uint32_t nb = e->header.binding_count;
     const bool eligible = !e->graphsDisabled && replayPays(e->steps.size(), e->header.total_size - e->header.data_offset) && !e->device->eventLog && e->device->dumpBuffersDir.empty();
     if (!eligible) return enqueueOps(e, bp);
@@ -894,11 +876,7 @@ void thip_executable_destroy(thip_executable_t *e) {
         }
     }
     if (e->stream) (void)hipStreamSynchronize(e->stream);
-    if (e->chained) {
-        ChainTurn &t = chainTurn(e->device->ordinal);
-        std::lock_guard<std::mutex> turn(t.mutex);
-        if (t.last == e->stream) t.last = nullptr;
-    }
+    if (e->chained) ChainTurns::of(e->device->ordinal).leave(&e->chain);
     for (auto &r : e->replays) dropReplay(&r);
     freeRetired(e, true);
     for (uint8_t *p : e->tempPtrs) {
@@ -949,7 +927,11 @@ static bool addStep(thip_executable_t *e, Step &&planned) {
         if (err == hipSuccess) err = hipMalloc((void **)&buffers[1], syncBytes);
         if (err == hipSuccess) err = hipMemcpy(buffers[0], chain.phases.data(), tableBytes, hipMemcpyHostToDevice);
         if (err == hipSuccess) err = hipMemset(buffers[1], 0, syncBytes);
-        if (err == hipSuccess) e->chained = true;
+        if (err == hipSuccess && !e->chained) {
+            e->chain.stream = e->stream;
+            err = ChainTurns::of(e->device->ordinal).join(&e->chain);
+            e->chained = err == hipSuccess;
+        }
     }
     if (err == hipSuccess) {
         uint8_t *placeholder[64];
@@ -1192,8 +1174,8 @@ static thip_status_t runLocked(thip_executable_t *e, const thip_dispatch_state_t
     }
     logEvent(e, e->invocation, 0, "DISPATCH_EXECUTE_ACTIONS", "BEGIN", "");
     auto enqueueStaged = [&] {
-        std::unique_lock<std::mutex> turn;
-        const thip_status_t s = takeChainTurn(e, &turn);
+        ChainTurns::Turn turn;
+        const thip_status_t s = takeTurn(e, &turn);
         return s != THIP_OK ? s : enqueueOps(e, bp);
     };
     if (thip_status_t s = allDevice ? enqueueDevice(e, bp) : enqueueStaged()) {
@@ -1271,8 +1253,8 @@ thip_status_t thip_executable_enqueue_noalloc(thip_executable_t *e, const thip_d
     uint8_t *bp[64] = {nullptr};
     for (uint32_t i = 0; i < e->header.binding_count; i++) bp[i] = (uint8_t *)st->binding_ptrs[i];
     const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0};
-    std::unique_lock<std::mutex> turn;
-    thip_status_t result = takeChainTurn(e, &turn);
+    ChainTurns::Turn turn;
+    thip_status_t result = takeTurn(e, &turn);
     for (const Step &s : e->steps) {
         // the array keeps what the last call left there, whoever made it; nothing in a K-split workspace has to start
         // at zero (every slot that is read has been written by the same dispatch)
