@@ -35,12 +35,14 @@ extern "C" hipError_t hipGetLastError() { return hipSuccess; }
 
 static hipStream_t streamOf(int n) { return (hipStream_t)(intptr_t)(100 * n); }
 
-// One dispatch.
-static void dispatch(ChainTurns *turns, ChainMember *m) {
+// One dispatch; whether it is one launch.
+static bool dispatch(ChainTurns *turns, ChainMember *m) {
     waits.clear();
     ChainTurns::Turn turn;
-    CHECK(turn.take(turns, m) == hipSuccess);
+    bool chained = false;
+    CHECK(turn.take(turns, m, &chained) == hipSuccess);
     busy.insert(m->stream);
+    return chained;
 }
 
 static void inTurn() {
@@ -53,25 +55,47 @@ static void inTurn() {
     // a dispatch makes nothing (thip_executable_enqueue_noalloc)
     const int made = created;
     CHECK(made > before);
-    dispatch(&turns, &a);
+    CHECK(dispatch(&turns, &a));
     CHECK(waits.empty());
-    dispatch(&turns, &a);
+    CHECK(dispatch(&turns, &a));
     CHECK(waits.empty());
-    dispatch(&turns, &b);
+    CHECK(dispatch(&turns, &b));
     CHECK(waits.size() == 1 && waits[0] == std::make_pair(b.stream, a.stream));
-    dispatch(&turns, &a);
+    CHECK(dispatch(&turns, &a));
     CHECK(waits.size() == 1 && waits[0] == std::make_pair(a.stream, b.stream));
     CHECK(created == made);
     busy.clear();
     turns.leave(&a);
-    dispatch(&turns, &b);
+    CHECK(dispatch(&turns, &b));
     CHECK(waits.empty());
     busy.clear();
     turns.leave(&b);
 }
 
+// Nobody is put behind work that does not end: neither an abandoned executable's nor what waits for that.
+static void abandoned() {
+    ChainTurns turns;
+    ChainMember a, b, c;
+    a.stream = streamOf(1);
+    b.stream = streamOf(2);
+    c.stream = streamOf(3);
+    for (ChainMember *m : {&a, &b, &c}) CHECK(turns.join(m) == hipSuccess);
+    CHECK(dispatch(&turns, &a));
+    CHECK(dispatch(&turns, &b));
+    a.abandoned = true;
+    CHECK(!dispatch(&turns, &c) && waits.empty());
+    CHECK(!dispatch(&turns, &b) && waits.empty());
+    busy.clear();  // its work has ended after all
+    CHECK(dispatch(&turns, &c));
+    CHECK(dispatch(&turns, &b));
+    CHECK(waits.size() == 1 && waits[0] == std::make_pair(b.stream, c.stream));
+    busy.clear();
+    for (ChainMember *m : {&a, &b, &c}) turns.leave(m);
+}
+
 int main() {
     inTurn();
+    abandoned();
     if (failures == 0) puts("in order");
     return failures != 0;
 }

@@ -235,6 +235,33 @@ def test_gpu_new_inputs_and_executables_in_turn(device, monkeypatch):
 
 
 @pytest.mark.gpu
+def test_gpu_an_abandoned_executable_holds_nobody_up(device, monkeypatch):
+    """One executable's wait times out with some 200 ms of its launches on the way; another one's dispatch is done long before these."""
+    monkeypatch.setenv("THIP_DEC_CHAIN", "1")
+    wls = [w.decoder_step_workload(batch=1, expose=True, seed=s, **STEP) for s in (7, 8)]
+    print("[gpu-case]", wls[0].name, "abandoned", flush=True)
+    exes = [_load(device, x) for x in wls]
+    sets = [_buffers(device, x) for x in wls]
+    try:
+        for _ in range(5000):
+            exes[0].enqueue_device(*sets[0])
+        exes[0].set_wait_timeout(1)
+        exes[1].set_wait_timeout(50)
+        with pytest.raises(thip.ThipError) as err:
+            exes[0].wait()
+        assert err.value.code == thip.runtime.INTERNAL
+        exes[1].run_device(*sets[1])
+        prog.check_decoder_step(wls[1], _outputs(device, wls[1], sets[1][0]), prog.assert_bf16_close, prog.assert_bit_exact)
+    finally:
+        device.synchronize()
+        for e in exes:
+            e.close()
+        for ptrs, _ in sets:
+            for q in ptrs:
+                device.free(q)
+
+
+@pytest.mark.gpu
 def test_gpu_results_written_into_the_caches(device, monkeypatch):
     """A caller that has the new keys appended to its cache in place: the scores read them, as when every op is a launch of its own."""
     wl = w.decoder_step_workload(batch=1, **STEP)

@@ -397,6 +397,7 @@ static thip_status_t waitBounded(thip_executable_t *e, hipEvent_t event, const c
         const auto now = std::chrono::steady_clock::now();
         if (now >= deadline) {
             e->abandoned = true;
+            e->chain.abandoned = true;
             return fail(THIP_INTERNAL, "%s: the GPU did not finish within %lld ms; the executable is abandoned", what, (long long)e->waitTimeoutMs);
         }
         // poll hard at first (dispatches are microseconds to a few milliseconds long, and a sleep of any length costs
@@ -515,8 +516,8 @@ static bool chainAliased(const thip_executable_t *e, uint8_t *const *bp) {
     return false;
 }
 
-// Launches one step: a record by its own launcher, a run of records by the kernel that does them as a whole.
-static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr) {
+// Launches one step: a record by its own launcher, a run of records by the kernel that does them as a whole.  `apart`: a chain record by record.
+static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr, bool apart = false) {
     hipError_t err = hipSuccess;
     switch (s.kind) {
     case kStepExpandDw: {
@@ -566,7 +567,7 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
         break;
     }
     case kStepDecChain: {
-        if (!ctx.name && chainAliased(e, bp)) {
+        if (!ctx.name && (apart || chainAliased(e, bp))) {
             for (uint32_t i = s.first; i < s.first + s.count; i++) {
                 if (thip_status_t st = launchOp(e, i, e->ops[i], bp, ctx, scratch)) return st;
             }
@@ -593,11 +594,11 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
 
 // Enqueues every kernel of the program.  `bp` holds one device pointer per binding.  A log or a dump is told of every
 // record, so these launch the records one by one.
-static thip_status_t enqueueOps(thip_executable_t *e, uint8_t *const *bp) {
+static thip_status_t enqueueOps(thip_executable_t *e, uint8_t *const *bp, bool apart = false) {
     if (!e->device->eventLog && e->device->dumpBuffersDir.empty()) {
         const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0};
         for (const Step &s : e->steps) {
-            if (thip_status_t st = launchStep(e, s, bp, ctx)) return st;
+            if (thip_status_t st = launchStep(e, s, bp, ctx, nullptr, apart)) return st;
         }
         return THIP_OK;
     }
@@ -664,16 +665,20 @@ static bool retireReplay(thip_executable_t *e, thip_executable_t::Replay *r) {
     return true;
 }
 
-// Takes the turn of a dispatch, if its launches are such that executables take turns.
-static thip_status_t takeTurn(thip_executable_t *e, ChainTurns::Turn *turn) {
-    if (e->chained) THIP_HIP(turn->take(&ChainTurns::of(e->device->ordinal), &e->chain), "waiting for another executable's launch");
+// Takes the turn of a dispatch, if its launches are such that executables take turns.  *apart: it runs record by record what otherwise is one launch.
+static thip_status_t takeTurn(thip_executable_t *e, ChainTurns::Turn *turn, bool *apart) {
+    bool chained = true;
+    if (e->chained) THIP_HIP(turn->take(&ChainTurns::of(e->device->ordinal), &e->chain, &chained), "waiting for another executable's launch");
+    *apart = !chained;
     return THIP_OK;
 }
 
 // Enqueues one dispatch on device bindings, through the set's graph when there is one.
 static thip_status_t enqueueDevice(thip_executable_t *e, uint8_t *const *bp) {
     ChainTurns::Turn turn;
-    if (thip_status_t s = takeTurn(e, &turn)) return s;
+    bool apart;
+    if (thip_status_t s = takeTurn(e, &turn, &apart)) return s;
+    if (apart) return enqueueOps(e, bp, true);
     const uint32_t nb = e->header.binding_count;
     const bool eligible = !e->graphsDisabled && replayPays(e->steps.size(), e->header.total_size - e->header.data_offset) && !e->device->eventLog && e->device->dumpBuffersDir.empty();
     if (!eligible) return enqueueOps(e, bp);
@@ -1175,8 +1180,9 @@ static thip_status_t runLocked(thip_executable_t *e, const thip_dispatch_state_t
     logEvent(e, e->invocation, 0, "DISPATCH_EXECUTE_ACTIONS", "BEGIN", "");
     auto enqueueStaged = [&] {
         ChainTurns::Turn turn;
-        const thip_status_t s = takeTurn(e, &turn);
-        return s != THIP_OK ? s : enqueueOps(e, bp);
+        bool apart;
+        const thip_status_t s = takeTurn(e, &turn, &apart);
+        return s != THIP_OK ? s : enqueueOps(e, bp, apart);
     };
     if (thip_status_t s = allDevice ? enqueueDevice(e, bp) : enqueueStaged()) {
         // what was enqueued before the failure still runs: wait for it (bounded; the launch error is what is reported)
@@ -1254,11 +1260,12 @@ thip_status_t thip_executable_enqueue_noalloc(thip_executable_t *e, const thip_d
     for (uint32_t i = 0; i < e->header.binding_count; i++) bp[i] = (uint8_t *)st->binding_ptrs[i];
     const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0};
     ChainTurns::Turn turn;
-    thip_status_t result = takeTurn(e, &turn);
+    bool apart;
+    thip_status_t result = takeTurn(e, &turn, &apart);
     for (const Step &s : e->steps) {
         // the array keeps what the last call left there, whoever made it; nothing in a K-split workspace has to start
         // at zero (every slot that is read has been written by the same dispatch)
-        if (result == THIP_OK) result = launchStep(e, s, bp, ctx, scratch);
+        if (result == THIP_OK) result = launchStep(e, s, bp, ctx, scratch, apart);
     }
     e->invocation++;
     return result;
