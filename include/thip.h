@@ -603,7 +603,9 @@ thip_status_t thip_executable_op_count(thip_executable_t *executable, uint32_t *
 thip_status_t thip_executable_op_kernel(thip_executable_t *executable, uint32_t index,
                                         char *name, size_t capacity);
 /* What those other dispatches launch, in order, as settled at creation: how many kernels, and the name of kernel `index`.  (The
- * small kernel that adds the partial sums of a linear whose K is split stands with the linear.) */
+ * small kernel that adds the partial sums of a linear whose K is split stands with the linear.  "dec_chain", whose workgroups need every CU at
+ * once, is launched while no other executable that has it is at work on the device; its ops' own kernels otherwise, whose fp32 sums are in
+ * another order.  THIP_DEC_CHAIN=1 in the environment at creation: always, one executable's behind the other's; 0: never.) */
 thip_status_t thip_executable_launch_count(thip_executable_t *executable, uint32_t *out_count);
 thip_status_t thip_executable_launch_kernel(thip_executable_t *executable, uint32_t index,
                                             char *name, size_t capacity);

@@ -1,6 +1,7 @@
 """A decoder's step as one launch (dec_chain): which programs take it, each op against the oracle on the inputs the GPU gave it at the sizes where
 the kernel can go wrong, what it may load, a launch whose workgroups give up waiting, executables in turn, and buffers that share memory."""
 import subprocess
+import threading
 
 import numpy as np
 import pytest
@@ -229,6 +230,58 @@ def test_gpu_new_inputs_and_executables_in_turn(device, monkeypatch):
     finally:
         for e in exes:
             e.close()
+        for ptrs, _ in sets:
+            for q in ptrs:
+                device.free(q)
+
+
+@pytest.mark.gpu
+def test_gpu_threads(device, monkeypatch):
+    """A thread for each of two decoders, as it comes: one launch or beside the other, every op is right, and each way leaves one result."""
+    wls = [w.decoder_step_workload(batch=b, expose=True, seed=9 + b, **STEP) for b in (1, 2)]
+    print("[gpu-case]", [x.name for x in wls], "threads", flush=True)
+    ways = []
+    for chain in ("0", "1", None):
+        if chain is None:
+            monkeypatch.delenv("THIP_DEC_CHAIN")
+        else:
+            monkeypatch.setenv("THIP_DEC_CHAIN", chain)
+        ways.append([thip.Executable(device, x.program.serialize()) for x in wls])
+    exes = ways[2]
+    assert all(e.launch_kernels()[0] == "dec_chain" for e in exes)
+    sets = [_buffers(device, x) for x in wls]
+    results, failed = [[], []], []
+
+    def dispatches(i):
+        try:
+            for k in range(60):
+                for _ in range(k % 3 + 1):
+                    exes[i].enqueue_device(*sets[i])
+                exes[i].wait()
+                results[i].append(_outputs(device, wls[i], sets[i][0]))
+        except Exception as e:  # reported by the test's own thread
+            failed.append(e)
+
+    try:
+        threads = [threading.Thread(target=dispatches, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(timeout=100)
+        assert not failed and not any(t.is_alive() for t in threads), failed
+        for i, wl in enumerate(wls):
+            known = []
+            for pair in ways[:2]:
+                pair[i].run_device(*sets[i])
+                known.append(_outputs(device, wl, sets[i][0]))
+                prog.check_decoder_step(wl, known[-1], prog.assert_bf16_close, prog.assert_bit_exact)
+            assert len(results[i]) == 60
+            for got in results[i]:
+                assert any(all(np.array_equal(a, b) for a, b in zip(got, want)) for want in known)
+    finally:
+        for pair in ways:
+            for e in pair:
+                e.close()
         for ptrs, _ in sets:
             for q in ptrs:
                 device.free(q)

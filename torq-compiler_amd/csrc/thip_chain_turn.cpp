@@ -29,19 +29,26 @@ void ChainTurns::leave(ChainMember *m) {
     members.erase(std::remove(members.begin(), members.end(), m), members.end());
 }
 
-static bool idle(const ChainMember *m) {
-    if (hipStreamQuery(m->stream) == hipSuccess) return true;
-    (void)hipGetLastError();  // not-ready is no error
-    return false;
-}
-
-hipError_t ChainTurns::Turn::take(ChainTurns *turns, ChainMember *m, bool *chained) {
+hipError_t ChainTurns::Turn::take(ChainTurns *turns, ChainMember *m, bool wanted, bool *chained) {
     *chained = false;
     lock = std::unique_lock<std::mutex>(turns->mutex);
-    for (const ChainMember *x : turns->members) {
-        if (x != m && x->abandoned && !idle(x)) return hipSuccess;
+    member = m;
+    m->enqueuing = m->busy = true;
+    bool apart = !wanted;
+    for (ChainMember *x : turns->members) {
+        if (apart || x == m || !x->busy || (m->always && !x->abandoned)) continue;
+        if (!x->enqueuing && hipStreamQuery(x->stream) == hipSuccess) {
+            x->busy = false;
+        } else {
+            (void)hipGetLastError();  // not-ready is no error
+            apart = true;
+        }
     }
-    if (turns->last && turns->last != m) {
+    if (apart) {  // others may enqueue at the same time
+        lock.unlock();
+        return hipSuccess;
+    }
+    if (m->always && turns->last && turns->last != m) {  // otherwise nobody else is at work
         hipError_t err = hipEventRecord(turns->event, turns->last->stream);
         if (err == hipSuccess) err = hipStreamWaitEvent(m->stream, turns->event, 0);
         if (err != hipSuccess) return err;
@@ -49,6 +56,12 @@ hipError_t ChainTurns::Turn::take(ChainTurns *turns, ChainMember *m, bool *chain
     turns->last = m;
     *chained = true;
     return hipSuccess;
+}
+
+ChainTurns::Turn::~Turn() {
+    if (!member) return;
+    if (!lock.owns_lock()) lock.lock();
+    member->enqueuing = false;
 }
 
 }  // namespace thip

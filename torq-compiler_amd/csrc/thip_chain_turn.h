@@ -12,12 +12,29 @@ namespace thip {
 // An executable's part.
 struct ChainMember {
     hipStream_t stream = nullptr;
+    bool always = false;                 // as one launch also beside others (THIP_DEC_CHAIN=1)
     std::atomic<bool> abandoned{false};  // a wait for its work timed out
+
+private:
+    friend class ChainTurns;
+    bool enqueuing = false;              // a dispatch is
+    bool busy = false;                   // there was one since the stream was last seen idle
 };
 
+// A decoder's step is one launch (dec_chain) while no other executable that has such launches is at work on the device, and otherwise runs record by
+// record.  One launch holds every CU for the whole step; as launches of their own the records of several decoders fill each other's gaps.
+// us a step, dispatches of one row from a thread for each decoder, one launch in turn / record by record, one decoder, two, three and four:
+//   26 layers, 1152, 6912, vocabulary 262144   620 / 865   623 / 516   625 / 393   625 / 506
+//   4 layers of it, vocabulary 4096             99 / 128   101 / 71    108 / 56    109 / 47
+//   4 layers, 512, 2048                         79 / 113    81 / 60     82 / 42     82 / 33
+// (and by this rule 622, 513, 395 and 505; 98, 72, 58 and 48; 78, 61, 44 and 36).  Where one thread enqueues for all of them its launches bound the
+// records: 610 / 861  622 / 527  622 / 408  621 / 525;  89 / 119  99 / 88  105 / 85  105 / 83;  69 / 106  79 / 85  78 / 82  78 / 81.
+// The two ways differ in the order of fp32 sums.  Who wants the same bits in company as alone asks for one of them when the executable is made
+// (THIP_DEC_CHAIN=0 or 1).
+//
 // The workgroups of a launch wait for one another and need a CU each at the same time.  Two such launches at once could each hold
-// CUs that the other waits for, so the executables of a device take turns: a dispatch on another stream than the last one's starts behind it.
-// Behind an abandoned executable's unfinished work (or what waits for that) nobody is put: dispatches then run record by record, which waits for nothing.
+// CUs that the other waits for, so where they are asked for beside others they take turns: a dispatch starts behind the last launch.
+// Behind an abandoned executable's unfinished work (or what waits for that) nobody is put: record by record a dispatch waits for nothing.
 class ChainTurns {
 public:
     static ChainTurns &of(int ordinal);  // one per device and process
@@ -30,10 +47,12 @@ public:
     // Of one dispatch, from before its launches until they are enqueued.
     class Turn {
     public:
-        // *chained: as one launch; otherwise record by record.
-        hipError_t take(ChainTurns *turns, ChainMember *m, bool *chained);
+        ~Turn();
+        // *chained: as one launch, if `wanted`; no other executable's turn is taken until this one ends.  Otherwise record by record.
+        hipError_t take(ChainTurns *turns, ChainMember *m, bool wanted, bool *chained);
 
     private:
+        ChainMember *member = nullptr;
         std::unique_lock<std::mutex> lock;
     };
 

@@ -592,10 +592,12 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
     return THIP_OK;
 }
 
-// Enqueues every kernel of the program.  `bp` holds one device pointer per binding.  A log or a dump is told of every
-// record, so these launch the records one by one.
+// A log or a dump is told of every record.
+static bool tellsRecords(const thip_executable_t *e) { return e->device->eventLog || !e->device->dumpBuffersDir.empty(); }
+
+// Enqueues every kernel of the program.  `bp` holds one device pointer per binding.
 static thip_status_t enqueueOps(thip_executable_t *e, uint8_t *const *bp, bool apart = false) {
-    if (!e->device->eventLog && e->device->dumpBuffersDir.empty()) {
+    if (!tellsRecords(e)) {
         const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0};
         for (const Step &s : e->steps) {
             if (thip_status_t st = launchStep(e, s, bp, ctx, nullptr, apart)) return st;
@@ -665,10 +667,11 @@ static bool retireReplay(thip_executable_t *e, thip_executable_t::Replay *r) {
     return true;
 }
 
-// Takes the turn of a dispatch, if its launches are such that executables take turns.  *apart: it runs record by record what otherwise is one launch.
-static thip_status_t takeTurn(thip_executable_t *e, ChainTurns::Turn *turn, bool *apart) {
+// Takes the turn of a dispatch, if its launches are such that executables take turns.  *apart: it runs record by record what otherwise is one launch;
+// `logged`: where a log or a dump is told of the records, in any case.
+static thip_status_t takeTurn(thip_executable_t *e, ChainTurns::Turn *turn, bool logged, bool *apart) {
     bool chained = true;
-    if (e->chained) THIP_HIP(turn->take(&ChainTurns::of(e->device->ordinal), &e->chain, &chained), "waiting for another executable's launch");
+    if (e->chained) THIP_HIP(turn->take(&ChainTurns::of(e->device->ordinal), &e->chain, !(logged && tellsRecords(e)), &chained), "waiting for another executable's launch");
     *apart = !chained;
     return THIP_OK;
 }
@@ -677,10 +680,10 @@ static thip_status_t takeTurn(thip_executable_t *e, ChainTurns::Turn *turn, bool
 static thip_status_t enqueueDevice(thip_executable_t *e, uint8_t *const *bp) {
     ChainTurns::Turn turn;
     bool apart;
-    if (thip_status_t s = takeTurn(e, &turn, &apart)) return s;
+    if (thip_status_t s = takeTurn(e, &turn, true, &apart)) return s;
     if (apart) return enqueueOps(e, bp, true);
     const uint32_t nb = e->header.binding_count;
-    const bool eligible = !e->graphsDisabled && replayPays(e->steps.size(), e->header.total_size - e->header.data_offset) && !e->device->eventLog && e->device->dumpBuffersDir.empty();
+    const bool eligible = !e->graphsDisabled && replayPays(e->steps.size(), e->header.total_size - e->header.data_offset) && !tellsRecords(e);
     if (!eligible) return enqueueOps(e, bp);
     thip_executable_t::Replay *r = nullptr, *oldest = nullptr;
     for (auto &x : e->replays) {
@@ -934,6 +937,7 @@ static bool addStep(thip_executable_t *e, Step &&planned) {
         if (err == hipSuccess) err = hipMemset(buffers[1], 0, syncBytes);
         if (err == hipSuccess && !e->chained) {
             e->chain.stream = e->stream;
+            e->chain.always = e->tuning.decChain == 1;
             err = ChainTurns::of(e->device->ordinal).join(&e->chain);
             e->chained = err == hipSuccess;
         }
@@ -1181,7 +1185,7 @@ static thip_status_t runLocked(thip_executable_t *e, const thip_dispatch_state_t
     auto enqueueStaged = [&] {
         ChainTurns::Turn turn;
         bool apart;
-        const thip_status_t s = takeTurn(e, &turn, &apart);
+        const thip_status_t s = takeTurn(e, &turn, true, &apart);
         return s != THIP_OK ? s : enqueueOps(e, bp, apart);
     };
     if (thip_status_t s = allDevice ? enqueueDevice(e, bp) : enqueueStaged()) {
@@ -1261,7 +1265,7 @@ thip_status_t thip_executable_enqueue_noalloc(thip_executable_t *e, const thip_d
     const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0};
     ChainTurns::Turn turn;
     bool apart;
-    thip_status_t result = takeTurn(e, &turn, &apart);
+    thip_status_t result = takeTurn(e, &turn, false, &apart);
     for (const Step &s : e->steps) {
         // the array keeps what the last call left there, whoever made it; nothing in a K-split workspace has to start
         // at zero (every slot that is read has been written by the same dispatch)

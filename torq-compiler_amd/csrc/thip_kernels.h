@@ -65,7 +65,7 @@ struct Tuning {
     bool noFcWide = false;          // THIP_NO_FC_WIDE
     bool addGeneric = false;        // THIP_ADD_GENERIC: the quantised add always through the 64-bit ACT stage
     bool maxpoolGeneric = false;    // THIP_MAXPOOL_GENERIC: the any-window max pool kernel also for 2 x 2 stride 2
-    int decChain = -1;              // THIP_DEC_CHAIN=0 / 1: the records of a decoder's step as one launch never / wherever it takes them (-1: by cost)
+    int decChain = -1;              // THIP_DEC_CHAIN=0 / 1: the records of a decoder's step as one launch never / wherever it takes them, always (-1: by cost, and beside no other one)
     long long decChainWait = 20000000;  // THIP_DEC_CHAIN_WAIT: ticks of 10 ns that a workgroup of dec_chain waits for the others (0: gives up at once)
     int decSplit = 0;               // THIP_DEC_SPLIT: workgroups per 16-column tile of a dec_linear launch of at most four rows: 1 or 2 (0: by its size)
     int decAblate = 0;              // THIP_DEC_ABLATE: parts of dec_linear left out, for timing experiments (wrong results)
