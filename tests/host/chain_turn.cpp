@@ -2,6 +2,7 @@
 // the runtime when.
 #include <stdio.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <set>
@@ -130,6 +131,40 @@ static void beside() {
     turns.leave(&b);
 }
 
+// Behind a launch that gave up, records for a while, longer each time; then launches again.
+static void gaveUp() {
+    ChainTurns turns;
+    ChainMember a;
+    uint32_t word = 0;
+    a.stream = streamOf(1);
+    a.gaveUp = &word;
+    CHECK(turns.join(&a) == hipSuccess);
+    auto records = [&] {
+        uint32_t n = 0;
+        while (n < 1000000 && !dispatch(&turns, &a)) n++;
+        return n;
+    };
+    CHECK(records() == 0);
+    uint32_t wanted = ChainTurns::kGivenUpFirst;
+    for (int i = 0; i < 9; i++) {
+        word = 1;
+        CHECK(records() == wanted);
+        wanted = std::min(2 * wanted, ChainTurns::kGivenUpMost);
+    }
+    CHECK(wanted == ChainTurns::kGivenUpMost);
+    word = 1;
+    CHECK(records() == wanted);
+    for (uint32_t i = 0; i < wanted; i++) CHECK(dispatch(&turns, &a));
+    word = 1;
+    CHECK(records() == ChainTurns::kGivenUpFirst);
+    // who asked for the launch always has it
+    a.always = true;
+    word = 1;
+    CHECK(dispatch(&turns, &a) && dispatch(&turns, &a));
+    busy.clear();
+    turns.leave(&a);
+}
+
 // From several threads: nobody else's work is on its way when one launches.
 static void threads() {
     ChainTurns turns;
@@ -166,6 +201,7 @@ static void threads() {
 int main() {
     inTurn();
     beside();
+    gaveUp();
     threads();
     abandoned();
     if (failures == 0) puts("in order");

@@ -236,6 +236,76 @@ def test_gpu_new_inputs_and_executables_in_turn(device, monkeypatch):
 
 
 @pytest.mark.gpu
+def test_gpu_a_launch_that_gave_up_is_not_tried_again_at_once(device, monkeypatch):
+    """Workgroups that give up at their first wait: the step is still right, and the next ones run record by record."""
+    wl = w.decoder_step_workload(batch=1, layers=2, vocab=512, expose=True, seed=12)  # fewer k-blocks leave the sums of both ways in one order
+    print("[gpu-case]", wl.name, "gave up", flush=True)
+    ptrs, lens = _buffers(device, wl)
+
+    def dispatches(count, **env):
+        for name in ("THIP_DEC_CHAIN", "THIP_DEC_CHAIN_WAIT"):
+            monkeypatch.delenv(name, raising=False)
+        for name, value in env.items():
+            monkeypatch.setenv(name, value)
+        exe = thip.Executable(device, wl.program.serialize())
+        try:
+            assert (exe.launch_kernels()[0] == "dec_chain") == (env.get("THIP_DEC_CHAIN") != "0")
+            got = []
+            for _ in range(count):
+                exe.run_device(ptrs, lens)
+                got.append(_outputs(device, wl, ptrs))
+            return got
+        finally:
+            exe.close()
+
+    same = lambda x, y: all(np.array_equal(a, b) for a, b in zip(x, y))
+    try:
+        launch, records = dispatches(1, THIP_DEC_CHAIN="1")[0], dispatches(1, THIP_DEC_CHAIN="0")[0]
+        differ = not same(launch, records)  # (an assert would print them)
+        assert differ, "the two ways are told apart by the order of their sums"
+        got = dispatches(4, THIP_DEC_CHAIN_WAIT="0")
+        prog.check_decoder_step(wl, got[0], prog.assert_bf16_close, prog.assert_bit_exact)
+        assert [same(g, launch) for g in got] == [True, False, False, False] and all(same(g, records) for g in got[1:])
+        assert all(same(g, launch) for g in dispatches(4))
+    finally:
+        for q in ptrs:
+            device.free(q)
+
+
+@pytest.mark.gpu
+def test_gpu_beside_another_streams_kernels(device, monkeypatch):
+    """Steps as one launch while GEMMs that fill the chip come and go on another stream."""
+    monkeypatch.setenv("THIP_DEC_CHAIN", "1")
+    wl, busy = w.decoder_step_workload(batch=1, expose=True, seed=13, **STEP), w.fully_connected_workload(4096, 1024, 4096, realistic=True)
+    print("[gpu-case]", wl.name, busy.name, flush=True)
+    exe, gemm = _load(device, wl), thip.Executable(device, busy.program.serialize())
+    ptrs, lens = _buffers(device, wl)
+    gemm_ptrs, gemm_lens = _buffers(device, busy)
+    try:
+        exe.run_device(ptrs, lens)
+        want = _outputs(device, wl, ptrs)
+        prog.check_decoder_step(wl, want, prog.assert_bf16_close, prog.assert_bit_exact)
+        gemm.run_device(gemm_ptrs, gemm_lens)
+        product = _outputs(device, busy, gemm_ptrs)[0]
+        for k in range(30):
+            for _ in range(20):
+                gemm.enqueue_device(gemm_ptrs, gemm_lens)
+            for _ in range(1 + k % 3):
+                exe.enqueue_device(ptrs, lens)
+            exe.wait()
+            assert all(np.array_equal(a, b) for a, b in zip(_outputs(device, wl, ptrs), want)), k
+            if k % 4 == 3:
+                gemm.wait()
+        gemm.wait()
+        assert np.array_equal(_outputs(device, busy, gemm_ptrs)[0], product)
+    finally:
+        for e in (exe, gemm):
+            e.close()
+        for q in ptrs + gemm_ptrs:
+            device.free(q)
+
+
+@pytest.mark.gpu
 def test_gpu_threads(device, monkeypatch):
     """A thread for each of two decoders, as it comes: one launch or beside the other, every op is right, and each way leaves one result."""
     wls = [w.decoder_step_workload(batch=b, expose=True, seed=9 + b, **STEP) for b in (1, 2)]

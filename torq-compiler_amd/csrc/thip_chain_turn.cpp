@@ -29,6 +29,21 @@ void ChainTurns::leave(ChainMember *m) {
     members.erase(std::remove(members.begin(), members.end(), m), members.end());
 }
 
+// Whether this dispatch is one of those behind a launch that gave up.
+bool ChainMember::missesCus() {
+    if (gaveUp && __atomic_exchange_n(gaveUp, 0u, __ATOMIC_RELAXED) != 0) {
+        penalty = std::min(std::max(2 * penalty, ChainTurns::kGivenUpFirst), ChainTurns::kGivenUpMost);
+        apart = penalty;
+        since = 0;
+    }
+    if (apart == 0) {
+        if (penalty > 0 && ++since > penalty) penalty = 0;
+        return false;
+    }
+    apart--;
+    return true;
+}
+
 hipError_t ChainTurns::Turn::take(ChainTurns *turns, ChainMember *m, bool wanted, bool *chained) {
     *chained = false;
     lock = std::unique_lock<std::mutex>(turns->mutex);
@@ -44,6 +59,7 @@ hipError_t ChainTurns::Turn::take(ChainTurns *turns, ChainMember *m, bool wanted
             apart = true;
         }
     }
+    if (!apart && !m->always) apart = m->missesCus();
     if (apart) {  // others may enqueue at the same time
         lock.unlock();
         return hipSuccess;

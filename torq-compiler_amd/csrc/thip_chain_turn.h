@@ -14,9 +14,14 @@ struct ChainMember {
     hipStream_t stream = nullptr;
     bool always = false;                 // as one launch also beside others (THIP_DEC_CHAIN=1)
     std::atomic<bool> abandoned{false};  // a wait for its work timed out
+    uint32_t *gaveUp = nullptr;          // null, or in host memory: a launch whose workgroups gave up waiting for one another sets it
 
 private:
     friend class ChainTurns;
+    bool missesCus();
+    uint32_t apart = 0;                  // dispatches that still go record by record since one gave up
+    uint32_t penalty = 0;                // how many of them the last one cost
+    uint32_t since = 0;                  // launches since then
     bool enqueuing = false;              // a dispatch is
     bool busy = false;                   // there was one since the stream was last seen idle
 };
@@ -34,9 +39,15 @@ private:
 //
 // The workgroups of a launch wait for one another and need a CU each at the same time.  Two such launches at once could each hold
 // CUs that the other waits for, so where they are asked for beside others they take turns: a dispatch starts behind the last launch.
+// A launch that does not get all CUs (another process, a CU mask, somebody's long kernels) costs its patience of 200 ms and the whole step by one
+// workgroup (26 layers 51 ms; four 7).  What kept the CUs is likely to be there still, so the next kGivenUpFirst dispatches run record by record: at 26 layers
+// these lose the same 0.25 s by not being one launch.  Twice as many after each further launch that gives up, and as at first again when as many
+// launches went well.
 // Behind an abandoned executable's unfinished work (or what waits for that) nobody is put: record by record a dispatch waits for nothing.
 class ChainTurns {
 public:
+    static constexpr uint32_t kGivenUpFirst = 1024, kGivenUpMost = 65536;
+
     static ChainTurns &of(int ordinal);  // one per device and process
 
     // When an executable is made (its device is current): what turns need is there from then on.

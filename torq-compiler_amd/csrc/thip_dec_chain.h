@@ -48,13 +48,14 @@ static_assert(sizeof(ChainPhase) == 256, "a dword for each lane of a wave");
 
 struct DecChainArgs {
     const ChainPhase *phases;
-    uint32_t *sync;      // word 0 launches done, word 32 set by a workgroup that gave up, word 64 workgroups done, from word 96 on the exchange
+    uint32_t *sync;      // word 0 launches done, word 32 set by a workgroup that gave up, word 64 workgroups done, words kChainTell and the next one the
+                         // address of a word of host memory that is set where a workgroup gave up, from word kChainSyncHead on the exchange
     int32_t count, xRoom, redRoom;  // phases; bytes of LDS for input rows and for partial sums
     uint32_t byGridMul, byGridShift;  // division by the workgroups of the launch
     uint64_t waitTicks;  // of the 100 MHz clock: how long a workgroup waits for the others before it gives up
     uint8_t *bindings[64];
 };
-constexpr uint64_t kChainSyncHead = 96;  // words in front of the exchange
+constexpr uint64_t kChainSyncHead = 96, kChainTell = 66;
 
 // Index arithmetic of the weights, shared by the kernel and a check on the host.
 

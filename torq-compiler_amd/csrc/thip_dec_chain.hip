@@ -593,8 +593,8 @@ __device__ __forceinline__ void chainFinish(const DecChainArgs &p, const ChainGr
 // layer 6 x 1.0 are the exchange, 6 x 0.7 the adding up and storing, 4.0 the products and 6 waits of the gate / up and down phases for weights and their expansion.
 // Weights by LDS-DMA two blocks ahead, through LDS, were slower (512, 2048: 72 -> 77; 1152, 6912, 26 layers 616 -> 609): the vector pipes are busy as it is.
 //
-// Workgroups wait for one another, so all must get a CU.  The driver lets no two such launches run at once; where something else keeps a CU for longer than
-// waitTicks, whoever waits gives up, everyone returns, and the last workgroup makes the whole step by itself.
+// Workgroups wait for one another, so all must get a CU.  The driver lets no two such launches run at once (ChainTurns); where something else keeps a CU for
+// longer than waitTicks, whoever waits gives up, everyone returns, and the last workgroup makes the whole step by itself and tells the host.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kChainThreads) void dec_chain(DecChainArgs p) {
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
@@ -648,6 +648,8 @@ __global__ __launch_bounds__(kChainThreads) void dec_chain(DecChainArgs p) {
             sharedStore(p.sync, epoch + 1u);
             sharedStore(p.sync + 32, 0u);
             sharedStore(p.sync + 64, 0u);
+            // (an argument of the launch would be one more to keep all the way)
+            if (again) __hip_atomic_store((uint32_t *)(uintptr_t)globalLoad<uint64_t>(p.sync + kChainTell), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             q.say[0] = 0;
         }
         if (!again) return;

@@ -897,6 +897,7 @@ void thip_executable_destroy(thip_executable_t *e) {
         if (p) (void)hipFree(p);
     }
     dropPinned(e);
+    if (e->chain.gaveUp) (void)hipHostFree(e->chain.gaveUp);
     if (e->constData) (void)hipFree(e->constData);
     if (e->evStart) (void)hipEventDestroy(e->evStart);
     if (e->evStop) (void)hipEventDestroy(e->evStop);
@@ -935,6 +936,13 @@ static bool addStep(thip_executable_t *e, Step &&planned) {
         if (err == hipSuccess) err = hipMalloc((void **)&buffers[1], syncBytes);
         if (err == hipSuccess) err = hipMemcpy(buffers[0], chain.phases.data(), tableBytes, hipMemcpyHostToDevice);
         if (err == hipSuccess) err = hipMemset(buffers[1], 0, syncBytes);
+        if (err == hipSuccess && !e->chain.gaveUp) {
+            err = hipHostMalloc((void **)&e->chain.gaveUp, sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent);
+            if (err == hipSuccess) *e->chain.gaveUp = 0;
+        }
+        void *tell = nullptr;
+        if (err == hipSuccess) err = hipHostGetDevicePointer(&tell, e->chain.gaveUp, 0);
+        if (err == hipSuccess) err = hipMemcpy(buffers[1] + 4 * kChainTell, &tell, sizeof(tell), hipMemcpyHostToDevice);
         if (err == hipSuccess && !e->chained) {
             e->chain.stream = e->stream;
             e->chain.always = e->tuning.decChain == 1;
