@@ -2,7 +2,15 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <atomic>
+#include <condition_variable>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#define private public  // what a copy does between the steps of another one's end
 #include "thip_host_copy.h"
+#undef private
 
 using thip::CopyCrew;
 
@@ -22,7 +30,36 @@ static bool once(CopyCrew *crew, size_t bytes, unsigned seed, int steps) {
     return dst[bytes] == 0xa5;
 }
 
+// A copy ends while another one takes over the helpers: that one keeps them.
+static bool takenOver() {
+    CopyCrew crew;
+    char bytes[8] = {0};
+    CopyCrew::Copy next(nullptr, bytes, bytes + 4, 4);
+    std::thread other;
+    {
+        CopyCrew::Copy last(nullptr, bytes, bytes + 4, 4);
+        last.crew = &crew;
+        crew.copy = &last;
+        crew.inside = 1;  // a helper that is on its way out
+        other = std::thread([&] {
+            for (;; std::this_thread::yield()) {
+                std::lock_guard<std::mutex> lock(crew.mutex);
+                if (crew.copy) continue;  // `last` has not begun to end
+                crew.inside = 0;
+                crew.copy = &next;
+                return;
+            }
+        });
+    }
+    other.join();
+    std::lock_guard<std::mutex> lock(crew.mutex);
+    return crew.copy == &next;
+}
+
 int main() {
+    for (int i = 0; i < 20; i++) {
+        if (!takenOver()) return puts("the helpers were taken away"), 1;
+    }
     const size_t piece = CopyCrew::kPiece, most = piece * CopyCrew::kMaxPieces;
     const size_t sizes[] = {0, 1, piece - 1, piece, piece + 1, CopyCrew::kAlone, CopyCrew::kAlone + 1, 5 * piece + 77, most - 1, most};
     CopyCrew crew;

@@ -69,13 +69,16 @@ CopyCrew::Copy::Copy(CopyCrew *of, void *dst_, const void *src_, size_t bytes_)
 
 CopyCrew::Copy::~Copy() {
     if (!crew) return;
-    // no piece is left, so whoever is inside is on its way out
-    for (bool first = true;; first = false) {
+    {
+        std::lock_guard<std::mutex> lock(crew->mutex);
+        next.store(pieces, std::memory_order_relaxed);  // also if the dispatch failed half-way
+        crew->copy = nullptr;
+    }
+    // No piece is left, so whoever is inside is on its way out.  (Once the last one is, another copy may have the helpers.)
+    for (;;) {
         {
             std::lock_guard<std::mutex> lock(crew->mutex);
-            if (first) next.store(pieces, std::memory_order_relaxed);  // also if the dispatch failed half-way
-            crew->copy = nullptr;
-            if (crew->inside == 0) return;
+            if (crew->inside == 0 || crew->copy) return;
         }
         std::this_thread::yield();
     }
