@@ -591,7 +591,7 @@ __device__ __forceinline__ void chainFinish(const DecChainArgs &p, const ChainGr
 // Measured, us, one launch per record / this one: 26 layers of hidden 1152, feed-forward 6912, four heads of 256 on 1024 positions, one row,
 // with the 262144-column projection behind it 843 / 616 (its bytes at 5.05 TB/s: 207); 4 layers without that 117 / 88, two rows 117 / 99.  What bounds it: of 21 us a
 // layer 6 x 1.0 are the exchange, 6 x 0.7 the adding up and storing, 4.0 the products and 6 waits of the gate / up and down phases for weights and their expansion.
-// Weights by LDS-DMA two blocks ahead, through LDS, were slower (512, 2048: 72 -> 77; 1152, 6912, 26 layers 616 -> 609): the vector pipes are busy as it is.
+// Weights by LDS-DMA two blocks ahead, through LDS: 616 -> 609 there, 72 -> 77 at 512, 2048; the vector pipes are busy as it is.
 //
 // Workgroups wait for one another, so all must get a CU.  The driver lets no two such launches run at once (ChainTurns); where something else keeps a CU for
 // longer than waitTicks, whoever waits gives up, everyone returns, and the last workgroup makes the whole step by itself and tells the host.

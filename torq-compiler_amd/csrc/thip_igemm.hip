@@ -656,7 +656,10 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BLOCKS_PER_CU) void igemm_de
 #pragma unroll
     for (int x = 0; x < NF; x++) readFrag(smem, 0, x, af0, bf0);
 
-    int at = 0;  // tile kt's place in the ring
+    // Tile kt's place in the ring, carried along: kt % STAGES of an odd number of stages is several scalar instructions a step.  us, 64-byte k-tiles by
+    // division / carried: 256x768x3072 4.29 / 4.19, 512x1536x2048 5.98 / 5.77, 1024x512x1024 3.78 / 3.70; 640x4096x2048 16.7 / 16.8, 128 x 128 tiles 28.2 / 28.2,
+    // 3x3 14x14x512 -> 512, batch 8 17.7 / 17.9.
+    int at = 0;
     // One k-tile.  `steady` (a compile-time flag) is the branch-free body used while the tile it
     // refills the ring with exists and lies wholly below K; the rest go through the general body.
     auto step = [&](int kt, auto steady) {
@@ -1257,7 +1260,8 @@ static hipError_t launchIgemmDense(const IgemmArgs &a, const LaunchCtx &ctx) {
 }
 
 // Whether a tile's problem is ahead in k-tiles of 128 bytes: whole cache lines per tile row, half the barriers per byte, and fewer
-// stages for the same bytes in flight.  us, in 64-byte k-tiles / in these:
+// stages for the same bytes in flight.  Inputs that change from dispatch to dispatch, us, in 64-byte k-tiles / in these (whose ring place was already
+// carried along; before that, 512x4096x4096 14.7 / 13.9):
 //   64 x 64, three stages, three workgroups per CU   512x1536x2048 6.3 / 5.9, 512x4096x2048 11.9 / 10.9, 128x8192x2048 18.4 / 16.3, 640x4096x2048
 //     17.3 / 13.8; 3x3 28x28x256 -> 256, batch 4 11.1 / 9.2, 14x14x512 -> 512, batch 8 18.1 / 14.4; at K = 1280 5.75 / 5.69, at 768 4.5 / 4.6
 //   64 x 128, three stages   512x1024x4096 6.1 / 6.0, 512x2048x4096 9.6 / 8.6, 600x2048x4096 14.1 / 12.0, 1200x1024x2048 8.2 / 7.8
@@ -1270,6 +1274,8 @@ static hipError_t launchIgemmDense(const IgemmArgs &a, const LaunchCtx &ctx) {
 //   128 x 128    3000x1472x1024 9.1 / 10.0, 3000x2112x1024 13.8 / 12.7, 1400x2112x3072 20.0 / 17.3, 1400x5696x3072 48.3 / 38.6
 //   128 x 64     300x3136x4096 11.2 / 11.1, 300x5696x4096 20.2 / 19.5
 // (Four to six stages are 0 - 5 % behind three: the loads are bound by what they carry, not by their latency.)
+// Where everything a tile row reads stays in its XCD's L2, the same input again and again, 64-byte k-tiles are up to 6 % ahead on 128 x 64 tiles
+// (300x4096x4096 12.2 / 12.8; with other inputs each time 14.0 / 13.1, with weights out of the L2 as well 22.3 / 18.6): no program's use.
 bool igemmWideBetter(const IgemmArgs &a, uint32_t variant) {
     if ((a.loader != kLoaderDense && a.loader != kLoaderWindow) || a.skip != nullptr) return false;
     const bool half = a.Kp % 128 != 0, window = a.loader == kLoaderWindow;
@@ -1288,7 +1294,9 @@ static hipError_t launchIgemmWide(const IgemmArgs &a, uint32_t variant, const La
     case kIgemmDense64x64: return launchIgemmDense<64, 64, 2, 2, 3, 3, CONV, 128, HALF>(a, ctx);
     case kIgemmDense128x128: return tiles(128, 128) <= 256 ? launchIgemmDense<128, 128, 2, 2, 3, 1, CONV, 128, HALF>(a, ctx) : launchIgemmDense<128, 128, 2, 2, 2, 2, CONV, 128, HALF>(a, ctx);
     case kIgemmDense64x128:
-        // (one workgroup per CU has all registers: 512 x 4096 x 4096 13.7 us against 14.4)
+        // One workgroup per CU has all registers, two of them fill each other's gaps where there are tiles for it.  us, one / two: up to 256 tiles
+        // 448x4096x4096 13.0 / 13.2, 512x4096x4096 13.7 / 13.7 (the same input each time 12.7 / 12.9 - 13.2), 960x4096x2048 13.5 / 13.6, 512x1024x4096 5.7 / 5.65, weights
+        // out of the L2 8.6 / 8.7; beyond 576x1024x4096 7.9 / 7.8, 640x2048x4096 11.8 / 11.6, 1088x4096x2048 19.6 / 19.4, 1024x8192x4096 43.4 / 43.3.
         if constexpr (!CONV) return tiles(64, 128) <= 256 ? launchIgemmDense<64, 128, 2, 2, 3, 1, false, 128, HALF>(a, ctx) : launchIgemmDense<64, 128, 2, 2, 3, 2, false, 128, HALF>(a, ctx);
         return hipErrorInvalidValue;
     case kIgemmDense128x64:

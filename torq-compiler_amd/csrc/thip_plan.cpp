@@ -435,8 +435,8 @@ bool replayPays(size_t launches, uint64_t constantBytes) {
 
 // Intermediates between grouped linears (and the result of a small matmul that is one's input) are laid out in blocks of 32 columns, which the
 // reader's loads bring in whole lines, where every record that touches one knows how: one writes all of it, the others take it as rows or as the
-// residual sum.  Up to kDecLdsRows rows come through LDS, as they lie.  us, row by row / in blocks, 32 rows: 1152 -> 2 x 6912 10.9 / 9.9, 6912 -> 1152
-// 10.4 / 9.9, 1152 -> 1536 5.0 / 4.9.
+// residual sum.  Up to kDecLdsRows rows come through LDS, as they lie.  us, row by row / in blocks, 32 rows: 1152 -> 2 x 6912 11.0 / 9.9, 6912 -> 1152
+// 10.6 / 9.3, 1152 -> 1536 5.0 / 4.8, 1024 -> 1152 4.9 / 4.7.
 static void blockRows(const DescriptorView &v, std::vector<Step> &steps) {
     struct Use {
         size_t step;
