@@ -1,11 +1,11 @@
-// The turns of executables that have a dec_chain launch, on a HIP of this file's own: which dispatches wait for which, and what is asked of
-// the runtime when.
+// The turns of executables that have a dec_chain launch, on a HIP of this file's own: which dispatches are one launch, which of them wait for
+// which, and what is asked of the runtime when.
 #include <stdio.h>
 
 #include <algorithm>
+#include <chrono>
 #include <map>
 #include <mutex>
-#include <set>
 #include <thread>
 #include <vector>
 
@@ -13,34 +13,41 @@
 
 using namespace thip;
 
-// A stream is busy while it is in `busy`.  An event remembers the stream that it was recorded on last.
+// An event remembers the stream that it was recorded on last.
 static std::mutex held;
-static std::set<hipStream_t> busy;
 static std::map<hipEvent_t, hipStream_t> recorded;
-static std::vector<std::pair<hipStream_t, hipStream_t>> waits;  // who waits, for whose work
-static int created, failures;
+static thread_local std::vector<std::pair<hipStream_t, hipStream_t>> waits;  // who waits, for whose work
+static std::atomic<int> created{0}, failures{0};
+
+#define CHECK(what) do { if (!(what)) failures++, printf("line %d: %s\n", __LINE__, #what); } while (0)
 
 extern "C" hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
     *e = (hipEvent_t)(intptr_t)++created;
     return hipSuccess;
 }
 extern "C" hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+    std::lock_guard<std::mutex> lock(held);
     recorded[e] = s;
     return e ? hipSuccess : hipErrorInvalidHandle;
 }
 extern "C" hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+    std::lock_guard<std::mutex> lock(held);
     waits.push_back({s, recorded[e]});
     return hipSuccess;
 }
-extern "C" hipError_t hipStreamQuery(hipStream_t s) {
-    std::lock_guard<std::mutex> lock(held);
-    return busy.count(s) ? hipErrorNotReady : hipSuccess;
+// Neither is allowed while somebody captures a graph.
+extern "C" hipError_t hipStreamQuery(hipStream_t) {
+    CHECK(!"a query of a stream");
+    return hipSuccess;
 }
-extern "C" hipError_t hipGetLastError() { return hipSuccess; }
-
-#define CHECK(what) do { if (!(what)) failures++, printf("line %d: %s\n", __LINE__, #what); } while (0)
+extern "C" hipError_t hipEventQuery(hipEvent_t) {
+    CHECK(!"a query of an event");
+    return hipSuccess;
+}
 
 static hipStream_t streamOf(int n) { return (hipStream_t)(intptr_t)(100 * n); }
+static bool waited(const ChainMember &m, const ChainMember &behind) { return waits.size() == 1 && waits[0] == std::make_pair(m.stream, behind.stream); }
+static void later() { std::this_thread::sleep_for(std::chrono::nanoseconds(ChainTurns::kAtWork * 3 / 2)); }
 
 // One dispatch; whether it is one launch.
 static bool dispatch(ChainTurns *turns, ChainMember *m, bool wanted = true) {
@@ -48,87 +55,91 @@ static bool dispatch(ChainTurns *turns, ChainMember *m, bool wanted = true) {
     ChainTurns::Turn turn;
     bool chained = false;
     CHECK(turn.take(turns, m, wanted, &chained) == hipSuccess);
-    busy.insert(m->stream);
     return chained;
 }
 
-static void inTurn() {
+struct Three {
     ChainTurns turns;
-    ChainMember a, b;
-    a.stream = streamOf(1);
-    b.stream = streamOf(2);
-    a.always = b.always = true;
+    ChainMember a, b, c;
+    explicit Three(bool always) {
+        int n = 0;
+        for (ChainMember *m : {&a, &b, &c}) {
+            m->stream = streamOf(++n);
+            m->always = always;
+            CHECK(turns.join(m) == hipSuccess);
+        }
+    }
+};
+
+// Launches that are asked for beside others, one behind the other.
+static void inTurn() {
     const int before = created;
-    CHECK(turns.join(&a) == hipSuccess && turns.join(&b) == hipSuccess);
+    Three t(true);
     // a dispatch makes nothing (thip_executable_enqueue_noalloc)
     const int made = created;
     CHECK(made > before);
-    CHECK(dispatch(&turns, &a));
-    CHECK(waits.empty());
-    CHECK(dispatch(&turns, &a));
-    CHECK(waits.empty());
-    CHECK(dispatch(&turns, &b));
-    CHECK(waits.size() == 1 && waits[0] == std::make_pair(b.stream, a.stream));
-    CHECK(dispatch(&turns, &a));
-    CHECK(waits.size() == 1 && waits[0] == std::make_pair(a.stream, b.stream));
+    CHECK(dispatch(&t.turns, &t.a) && waits.empty());
+    CHECK(dispatch(&t.turns, &t.a) && waits.empty());
+    CHECK(dispatch(&t.turns, &t.b) && waited(t.b, t.a));
+    CHECK(dispatch(&t.turns, &t.a) && waited(t.a, t.b));
     CHECK(created == made);
-    busy.clear();
-    turns.leave(&a);
-    CHECK(dispatch(&turns, &b));
-    CHECK(waits.empty());
-    busy.clear();
-    turns.leave(&b);
+    later();  // not known to be done
+    CHECK(dispatch(&t.turns, &t.c) && waited(t.c, t.a));
+    t.c.finished();
+    CHECK(dispatch(&t.turns, &t.b) && waits.empty());
+    t.turns.leave(&t.b);
+    CHECK(dispatch(&t.turns, &t.a) && waits.empty());
 }
 
 // Nobody is put behind work that does not end: neither an abandoned executable's nor what waits for that.
-static void abandoned() {
-    ChainTurns turns;
-    ChainMember a, b, c;
-    a.stream = streamOf(1);
-    b.stream = streamOf(2);
-    c.stream = streamOf(3);
-    a.always = b.always = c.always = true;
-    for (ChainMember *m : {&a, &b, &c}) CHECK(turns.join(m) == hipSuccess);
-    CHECK(dispatch(&turns, &a));
-    CHECK(dispatch(&turns, &b));
-    a.abandoned = true;
-    CHECK(!dispatch(&turns, &c) && waits.empty());
-    CHECK(!dispatch(&turns, &b) && waits.empty());
-    busy.clear();  // its work has ended after all
-    CHECK(dispatch(&turns, &c));
-    CHECK(dispatch(&turns, &b));
-    CHECK(waits.size() == 1 && waits[0] == std::make_pair(b.stream, c.stream));
-    busy.clear();
-    for (ChainMember *m : {&a, &b, &c}) turns.leave(m);
+static void abandoned(bool always) {
+    Three t(always);
+    CHECK(dispatch(&t.turns, &t.a));
+    t.a.finished();
+    CHECK(dispatch(&t.turns, &t.b));
+    t.a.abandoned = true;
+    t.b.finished();
+    later();
+    CHECK(!dispatch(&t.turns, &t.c) && waits.empty());
+    t.c.finished();
+    CHECK(!dispatch(&t.turns, &t.b) && waits.empty());
+    t.b.finished();
+    t.turns.leave(&t.a);  // its work has ended after all
+    CHECK(dispatch(&t.turns, &t.c));
 }
 
-// One launch while nobody else is at work, records beside others; nobody waits.
+// One launch while nobody else is at work, records beside others.
 static void beside() {
-    ChainTurns turns;
-    ChainMember a, b;
-    a.stream = streamOf(1);
-    b.stream = streamOf(2);
-    CHECK(turns.join(&a) == hipSuccess && turns.join(&b) == hipSuccess);
-    CHECK(dispatch(&turns, &a) && dispatch(&turns, &a));
-    CHECK(!dispatch(&turns, &b) && !dispatch(&turns, &a) && !dispatch(&turns, &b));
-    busy.erase(b.stream);
-    CHECK(dispatch(&turns, &a) && !dispatch(&turns, &b));
-    busy.clear();
-    CHECK(dispatch(&turns, &b));
-    CHECK(!dispatch(&turns, &b, false));
+    Three t(false);
+    CHECK(dispatch(&t.turns, &t.a) && dispatch(&t.turns, &t.a));
+    CHECK(!dispatch(&t.turns, &t.b) && !dispatch(&t.turns, &t.a) && !dispatch(&t.turns, &t.b));
+    t.b.finished();
+    CHECK(dispatch(&t.turns, &t.a) && !dispatch(&t.turns, &t.b) && waits.empty());
+    t.a.finished();
+    CHECK(dispatch(&t.turns, &t.b) && waits.empty());
+    CHECK(!dispatch(&t.turns, &t.b, false));
+    // a caller that waits by other means is at work for a while; a launch of its is waited for all the same
+    CHECK(!dispatch(&t.turns, &t.c));
+    t.c.finished();
+    later();
+    CHECK(dispatch(&t.turns, &t.c) && waited(t.c, t.b));
+    // as long as it is being waited for
+    t.c.waiting();
+    later();
+    CHECK(!dispatch(&t.turns, &t.a));
+    t.a.finished();
+    t.c.finished();
+    CHECK(dispatch(&t.turns, &t.a) && waits.empty());
+    t.a.finished();
     {
-        // its launches are on their way, though its stream has none yet
+        // while its launches are enqueued, also if they are many
         ChainTurns::Turn turn;
-        bool chained = true;
-        CHECK(turn.take(&turns, &a, true, &chained) == hipSuccess && !chained);
-        busy.clear();
-        CHECK(!dispatch(&turns, &b));
-        busy.clear();
+        bool chained = false;
+        CHECK(turn.take(&t.turns, &t.a, false, &chained) == hipSuccess && !chained);
+        CHECK(!dispatch(&t.turns, &t.b));
+        t.b.finished();
     }
-    CHECK(dispatch(&turns, &b) && waits.empty());
-    busy.clear();
-    turns.leave(&a);
-    turns.leave(&b);
+    CHECK(!dispatch(&t.turns, &t.b));
 }
 
 // Behind a launch that gave up, records for a while, longer each time; then launches again.
@@ -161,49 +172,58 @@ static void gaveUp() {
     a.always = true;
     word = 1;
     CHECK(dispatch(&turns, &a) && dispatch(&turns, &a));
-    busy.clear();
-    turns.leave(&a);
 }
 
-// From several threads: nobody else's work is on its way when one launches.
-static void threads() {
+// From several threads: a launch waits for another one's, or that is done.
+static void threads(bool always) {
     ChainTurns turns;
     ChainMember members[4];
     std::atomic<int> bad{0}, launches{0};
+    hipStream_t launched = nullptr;  // whose launch is on its way
     std::vector<std::thread> all;
     for (int t = 0; t < 4; t++) {
         members[t].stream = streamOf(t + 1);
+        members[t].always = always;
         CHECK(turns.join(&members[t]) == hipSuccess);
     }
     for (int t = 0; t < 4; t++) {
         all.emplace_back([&, t] {
+            ChainMember &m = members[t];
             for (int i = 0; i < 2000; i++) {
                 {
                     ChainTurns::Turn turn;
                     bool chained = false;
-                    bad += turn.take(&turns, &members[t], i % 7 != 0, &chained) != hipSuccess;
+                    waits.clear();
+                    bad += turn.take(&turns, &m, i % 7 != 0, &chained) != hipSuccess;
                     std::lock_guard<std::mutex> lock(held);
-                    bad += chained && !busy.empty();
+                    bad += chained && launched && launched != m.stream && !(waits.size() == 1 && waits[0] == std::make_pair(m.stream, launched));
                     launches += chained;
-                    busy.insert(members[t].stream);
+                    if (chained) launched = m.stream;
                 }
-                if (i % 3 == 0) std::this_thread::yield();
-                std::lock_guard<std::mutex> lock(held);
-                busy.erase(members[t].stream);
+                if (i % 3 == 0) continue;  // the next one behind it
+                std::this_thread::yield();
+                m.waiting();
+                {
+                    std::lock_guard<std::mutex> lock(held);
+                    if (launched == m.stream) launched = nullptr;
+                }
+                m.finished();
             }
+            m.finished();
         });
     }
     for (std::thread &t : all) t.join();
     CHECK(bad == 0 && launches > 0);
-    for (ChainMember &m : members) turns.leave(&m);
 }
 
 int main() {
     inTurn();
+    abandoned(false);
+    abandoned(true);
     beside();
     gaveUp();
-    threads();
-    abandoned();
+    threads(false);
+    threads(true);
     if (failures == 0) puts("in order");
     return failures != 0;
 }

@@ -5,6 +5,7 @@ sums).  The no-allocation entry point takes that memory from the library's stati
 which every call on the GPU shares and which keeps the last call's contents: two calls in a row, the second on a
 smaller problem, must each give exactly what the ordinary entry point gives.
 """
+import ctypes
 import sys
 
 import numpy as np
@@ -103,7 +104,62 @@ def test_noalloc_refuses_what_does_not_fit_and_host_bindings(device):
     exe = Executable(device, wl.program.serialize())
     out = np.zeros((1, 256), dtype=np.uint16)
     st, keep = runtime.make_state([wl.inputs[0].ctypes.data, out.ctypes.data], [wl.inputs[0].nbytes, out.nbytes], [0, 0])
-    import ctypes
     code = runtime.lib().thip_executable_enqueue_noalloc(exe._h, ctypes.byref(st))
     exe.close()
     assert code == runtime.FAILED_PRECONDITION
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2], ids=["global", "thread_local", "relaxed"])
+def test_noalloc_while_a_graph_is_captured(device, monkeypatch, mode):
+    """Decoders dispatched while another stream of the process is under capture: the capture ends as it should, and so do the steps."""
+    hip = runtime.lib()  # the HIP runtime that the library runs on is one of its own
+    wls = [w.decoder_step_workload(batch=1, layers=2, hidden=256, heads=2, head_dim=64, ffn=512, vocab=512, cache_len=64, seed=s) for s in (3, 4)]
+    print("[gpu-case]", wls[0].name, "during a capture,", mode, flush=True)
+    monkeypatch.setenv("THIP_DEC_CHAIN", "0")
+    records = [Executable(device, x.program.serialize()) for x in wls]
+    monkeypatch.delenv("THIP_DEC_CHAIN")
+    exes = [Executable(device, x.program.serialize()) for x in wls]
+    assert all(e.launch_kernels()[0] == "dec_chain" for e in exes)
+    arrays = [list(x.inputs) + [np.zeros(s, d) for s, d in x.outputs] for x in wls]
+    sets = [([device.upload(a) for a in x], [a.nbytes for a in x]) for x in arrays]
+    out = [(s[0][3], x.outputs[0][0]) for s, x in zip(sets, wls)]
+    numbers = np.arange(1000, dtype=np.int32)
+    src, dst = device.upload(numbers), device.upload(np.zeros_like(numbers))
+    stream, graph, replay = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    try:
+        want = []  # each step as one launch, and record by record
+        for pair in (exes, records):
+            for e, s in zip(pair, sets):
+                e.run_device(*s)
+            want.append([device.download(p, shape, np.uint16) for p, shape in out])
+        assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
+        assert hip.hipStreamBeginCapture(stream, ctypes.c_int(mode)) == 0
+        copied = hip.hipMemcpyAsync(ctypes.c_void_p(dst), ctypes.c_void_p(src), ctypes.c_size_t(numbers.nbytes), ctypes.c_int(3), stream)
+        refused = []
+        for _ in range(3):
+            for e, s in zip(exes, sets):
+                try:
+                    e.enqueue_device_noalloc(*s)
+                except ThipError as err:
+                    refused.append(err)
+        ended = hip.hipStreamEndCapture(stream, ctypes.byref(graph))
+        assert (copied, ended, refused) == (0, 0, [])
+        for e in exes:
+            e.wait()
+        assert hip.hipGraphInstantiate(ctypes.byref(replay), graph, None, None, ctypes.c_size_t(0)) == 0
+        for _ in range(3):
+            assert hip.hipGraphLaunch(replay, stream) == 0 and hip.hipStreamSynchronize(stream) == 0
+        assert np.array_equal(device.download(dst, numbers.shape, numbers.dtype), numbers)
+        for i, (p, shape) in enumerate(out):
+            assert any(np.array_equal(device.download(p, shape, np.uint16), x[i]) for x in want), i
+    finally:
+        for handle, free in ((replay, hip.hipGraphExecDestroy), (graph, hip.hipGraphDestroy), (stream, hip.hipStreamDestroy)):
+            if handle:
+                free(handle)
+        for e in exes + records:
+            e.close()
+        for ptrs, _ in sets:
+            for p in ptrs:
+                device.free(p)
+        device.free(src)
+        device.free(dst)

@@ -1,9 +1,30 @@
 #include "thip_chain_turn.h"
 
 #include <algorithm>
+#include <chrono>
 #include <new>
 
 namespace thip {
+
+static int64_t nanoseconds() { return std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now().time_since_epoch()).count(); }
+
+void ChainMember::waiting() { busyUntil.store(INT64_MAX, std::memory_order_relaxed); }
+void ChainMember::finished() { busyUntil.store(0, std::memory_order_relaxed); }
+
+// Whether this dispatch is one of those behind a launch that gave up.
+bool ChainMember::missesCus() {
+    if (gaveUp && __atomic_exchange_n(gaveUp, 0u, __ATOMIC_RELAXED) != 0) {
+        penalty = std::min(std::max(2 * penalty, ChainTurns::kGivenUpFirst), ChainTurns::kGivenUpMost);
+        apart = penalty;
+        since = 0;
+    }
+    if (apart == 0) {
+        if (penalty > 0 && ++since > penalty) penalty = 0;
+        return false;
+    }
+    apart--;
+    return true;
+}
 
 ChainTurns &ChainTurns::of(int ordinal) {
     static ChainTurns turns[64];
@@ -29,42 +50,22 @@ void ChainTurns::leave(ChainMember *m) {
     members.erase(std::remove(members.begin(), members.end(), m), members.end());
 }
 
-// Whether this dispatch is one of those behind a launch that gave up.
-bool ChainMember::missesCus() {
-    if (gaveUp && __atomic_exchange_n(gaveUp, 0u, __ATOMIC_RELAXED) != 0) {
-        penalty = std::min(std::max(2 * penalty, ChainTurns::kGivenUpFirst), ChainTurns::kGivenUpMost);
-        apart = penalty;
-        since = 0;
-    }
-    if (apart == 0) {
-        if (penalty > 0 && ++since > penalty) penalty = 0;
-        return false;
-    }
-    apart--;
-    return true;
-}
-
 hipError_t ChainTurns::Turn::take(ChainTurns *turns, ChainMember *m, bool wanted, bool *chained) {
     *chained = false;
     lock = std::unique_lock<std::mutex>(turns->mutex);
     member = m;
-    m->enqueuing = m->busy = true;
+    const int64_t now = nanoseconds();
+    m->busyUntil.store(now + kAtWork, std::memory_order_relaxed);
     bool apart = !wanted;
-    for (ChainMember *x : turns->members) {
-        if (apart || x == m || !x->busy || (m->always && !x->abandoned)) continue;
-        if (!x->enqueuing && hipStreamQuery(x->stream) == hipSuccess) {
-            x->busy = false;
-        } else {
-            (void)hipGetLastError();  // not-ready is no error
-            apart = true;
-        }
+    for (const ChainMember *x : turns->members) {
+        apart = apart || (x != m && (x->abandoned || (!m->always && x->busyUntil.load(std::memory_order_relaxed) > now)));
     }
     if (!apart && !m->always) apart = m->missesCus();
     if (apart) {  // others may enqueue at the same time
         lock.unlock();
         return hipSuccess;
     }
-    if (m->always && turns->last && turns->last != m) {  // otherwise nobody else is at work
+    if (turns->last && turns->last != m && turns->last->busyUntil.load(std::memory_order_relaxed) != 0) {
         hipError_t err = hipEventRecord(turns->event, turns->last->stream);
         if (err == hipSuccess) err = hipStreamWaitEvent(m->stream, turns->event, 0);
         if (err != hipSuccess) return err;
@@ -75,9 +76,7 @@ hipError_t ChainTurns::Turn::take(ChainTurns *turns, ChainMember *m, bool wanted
 }
 
 ChainTurns::Turn::~Turn() {
-    if (!member) return;
-    if (!lock.owns_lock()) lock.lock();
-    member->enqueuing = false;
+    if (member) member->busyUntil.store(nanoseconds() + kAtWork, std::memory_order_relaxed);
 }
 
 }  // namespace thip

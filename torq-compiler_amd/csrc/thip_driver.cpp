@@ -406,12 +406,15 @@ static thip_status_t waitBounded(thip_executable_t *e, hipEvent_t event, const c
     }
 }
 static thip_status_t waitBounded(thip_executable_t *e, const char *what) {
+    e->chain.waiting();
     if (e->waitTimeoutMs <= 0) {
         THIP_HIP(hipStreamSynchronize(e->stream), what);
-        return THIP_OK;
+    } else {
+        THIP_HIP(hipEventRecord(e->evDone, e->stream), "hipEventRecord");
+        if (thip_status_t s = waitBounded(e, e->evDone, what)) return s;
     }
-    THIP_HIP(hipEventRecord(e->evDone, e->stream), "hipEventRecord");
-    return waitBounded(e, e->evDone, what);
+    e->chain.finished();
+    return THIP_OK;
 }
 
 static bool makeDirs(const std::string &path) {
@@ -567,7 +570,7 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
         break;
     }
     case kStepDecChain: {
-        if (!ctx.name && (apart || chainAliased(e, bp))) {
+        if (!ctx.name && apart) {
             for (uint32_t i = s.first; i < s.first + s.count; i++) {
                 if (thip_status_t st = launchOp(e, i, e->ops[i], bp, ctx, scratch)) return st;
             }
@@ -669,9 +672,12 @@ static bool retireReplay(thip_executable_t *e, thip_executable_t::Replay *r) {
 
 // Takes the turn of a dispatch, if its launches are such that executables take turns.  *apart: it runs record by record what otherwise is one launch;
 // `logged`: where a log or a dump is told of the records, in any case.
-static thip_status_t takeTurn(thip_executable_t *e, ChainTurns::Turn *turn, bool logged, bool *apart) {
+static thip_status_t takeTurn(thip_executable_t *e, uint8_t *const *bp, ChainTurns::Turn *turn, bool logged, bool *apart) {
     bool chained = true;
-    if (e->chained) THIP_HIP(turn->take(&ChainTurns::of(e->device->ordinal), &e->chain, !(logged && tellsRecords(e)), &chained), "waiting for another executable's launch");
+    if (e->chained) {
+        const bool wanted = !(logged && tellsRecords(e)) && !chainAliased(e, bp);
+        THIP_HIP(turn->take(&ChainTurns::of(e->device->ordinal), &e->chain, wanted, &chained), "waiting for another executable's launch");
+    }
     *apart = !chained;
     return THIP_OK;
 }
@@ -680,7 +686,7 @@ static thip_status_t takeTurn(thip_executable_t *e, ChainTurns::Turn *turn, bool
 static thip_status_t enqueueDevice(thip_executable_t *e, uint8_t *const *bp) {
     ChainTurns::Turn turn;
     bool apart;
-    if (thip_status_t s = takeTurn(e, &turn, true, &apart)) return s;
+    if (thip_status_t s = takeTurn(e, bp, &turn, true, &apart)) return s;
     if (apart) return enqueueOps(e, bp, true);
     const uint32_t nb = e->header.binding_count;
     const bool eligible = !e->graphsDisabled && replayPays(e->steps.size(), e->header.total_size - e->header.data_offset) && !tellsRecords(e);
@@ -1193,7 +1199,7 @@ static thip_status_t runLocked(thip_executable_t *e, const thip_dispatch_state_t
     auto enqueueStaged = [&] {
         ChainTurns::Turn turn;
         bool apart;
-        const thip_status_t s = takeTurn(e, &turn, true, &apart);
+        const thip_status_t s = takeTurn(e, bp, &turn, true, &apart);
         return s != THIP_OK ? s : enqueueOps(e, bp, apart);
     };
     if (thip_status_t s = allDevice ? enqueueDevice(e, bp) : enqueueStaged()) {
@@ -1273,7 +1279,7 @@ thip_status_t thip_executable_enqueue_noalloc(thip_executable_t *e, const thip_d
     const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0};
     ChainTurns::Turn turn;
     bool apart;
-    thip_status_t result = takeTurn(e, &turn, false, &apart);
+    thip_status_t result = takeTurn(e, bp, &turn, false, &apart);
     for (const Step &s : e->steps) {
         // the array keeps what the last call left there, whoever made it; nothing in a K-split workspace has to start
         // at zero (every slot that is read has been written by the same dispatch)
