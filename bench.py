@@ -197,21 +197,21 @@ class Loaded:
 TRAFFIC_SOURCES_SHA256 = {
     "thip_bandwidth.hip": "9f362b1c3295215d62fa4e31cb26409d5141f8a8775045b8e9241122a60a4c8f",
     "thip_conv_patch.hip": "d94cab362a7338f9f6d5bb67d3dd77222153b6a69f9850d0ab0fd328cac10d4e",
-    "thip_igemm.hip": "aa8ad5f15176fd44aa4c2f83db978f24aa78d03bad578edb76bc420e49ac2816",
+    "thip_igemm.hip": "8af44b0bac43ba07ac67de30f350a997f461de3dd2da725ee63a4fec357c9b61",
     "thip_igemm_direct.hip": "b6e3a10ba2c1865b144a6f8f770ee4f27d61829b54799ffb7286dd29adb85e6d",
     "thip_kernels_common.h": "b3c4244f20b719cf1485ae795905dff909881fc94ff47ec097c8d19ac569aa5e",
 }
 MEASURED_TRAFFIC = {
-    "fc_4096x4096x4096": (49381.0 * 1.9996 + 16584.1 * 1.0000) * 1024,
+    "fc_4096x4096x4096": (49381.0 * 1.9996 + 16588.8 * 1.0000) * 1024,
     "fc_512x4096x4096": (16453.5 * 1.9996 + 2048.0 * 1.0000) * 1024,
     "fc_16x2048x8192": (8408.0 * 1.9996 + 256.0 * 1.0000) * 1024,
     "conv_112x112x32_o64_3x3": (800.4 * 1.9996 + 784.0 * 1.0000) * 1024,
-    "conv3x3_56x56x256_o256_b32": (17257.0 * 1.9996 + 25301.2 * 1.0000) * 1024,
-    "conv3x3_56x56x96_o96_b32": (6340.0 * 1.9996 + 9524.9 * 1.0000) * 1024,
+    "conv3x3_56x56x256_o256_b32": (17251.1 * 1.9996 + 26002.0 * 1.0000) * 1024,
+    "conv3x3_56x56x96_o96_b32": (6340.0 * 1.9996 + 9591.4 * 1.0000) * 1024,
     "conv1x1_56x56x256_o1024_b32": (14417.5 * 1.9996 + 100352.0 * 1.0000) * 1024,
-    "depthwise_b64": (14209.0 * 1.9996 + 7774.4 * 1.0000) * 1024,
-    "depthwise_s1_b256": (63702.6 * 1.9996 + 113211.2 * 1.0000) * 1024,
-    "maxpool_b64": (25484.2 * 1.9996 + 12544.0 * 1.0000) * 1024,
+    "depthwise_b64": (14207.9 * 1.9996 + 7761.1 * 1.0000) * 1024,
+    "depthwise_s1_b256": (63708.8 * 1.9996 + 113200.1 * 1.0000) * 1024,
+    "maxpool_b64": (25464.6 * 1.9996 + 12544.0 * 1.0000) * 1024,
     "avgpool_b64": (2001.0 * 1.9996 + 80.0 * 1.0000) * 1024,
     "add_b64": (4723.0 * 1.9996 + 4704.0 * 1.0000) * 1024,
 }
