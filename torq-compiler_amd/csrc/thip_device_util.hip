@@ -275,6 +275,7 @@ Tuning tuningFromEnvironment() {
         t.plainRecords = t.plainRecords || flag(name);
     }
     t.padRows = digit("THIP_PAD_ROWS", -1);
+    t.irBlock = digit("THIP_IR_BLOCK", -1);
     if (const char *v = getenv("THIP_STEP_BYTES")) t.stepBytes = atoll(v);
     t.noFcDeep = flag("THIP_NO_FC_DEEP");
     t.noFcWide = flag("THIP_NO_FC_WIDE");

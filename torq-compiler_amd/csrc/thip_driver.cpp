@@ -524,6 +524,10 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
     hipError_t err = hipSuccess;
     switch (s.kind) {
     case kStepExpandDw: {
+        if (s.count == 3) {
+            err = launchIrBlock(irBlockArgs(viewOf(e), s, [&](const DescRef &r) { return r.space == kSpaceNone ? nullptr : (uint8_t *)resolve(e, r, bp); }), ctx);
+            break;
+        }
         const DescOp &x = e->ops[s.first], &d = e->ops[s.first + 1];
         IrExpandDwArgs a;
         memset(&a, 0, sizeof(a));

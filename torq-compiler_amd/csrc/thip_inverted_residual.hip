@@ -117,20 +117,7 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
         for (int s = 0; s < KS; s++) {
             const int kh = 2 * s + half < p.CKH ? 2 * s + half : 0;
             const int hi = (unsigned)(iy + kh) >= (unsigned)p.IH ? 0 : room;
-            int d = off[s] - clampRun(off[s]);
-            d = d < -15 ? -15 : d > 15 ? 15 : d;
-            unsigned __int128 v;
-            __builtin_memcpy(&v, &a[s], 16);
-            v = d >= 0 ? v >> (8 * d) : v << (-8 * d);
-            __builtin_memcpy(&a[s], &v, 16);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int l = lo - 4 * e, h = hi - 4 * e;
-                const uint32_t below = l <= 0 ? 0u : l >= 4 ? 0xffffffffu : (1u << (8 * l)) - 1u;
-                const uint32_t upto = h <= 0 ? 0u : h >= 4 ? 0xffffffffu : (1u << (8 * h)) - 1u;
-                const uint32_t in = upto & ~below;
-                a[s][e] = (int)(((uint32_t)a[s][e] & in) | (zp4 & ~in));
-            }
+            a[s] = fixRun16(a[s], off[s] - clampRun(off[s]), lo, hi, zp4);
         }
     };
     // the wave's first pixel, and its tiles' pixels behind it

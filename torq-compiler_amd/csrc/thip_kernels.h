@@ -65,6 +65,7 @@ struct Tuning {
     bool noFcWide = false;          // THIP_NO_FC_WIDE
     bool addGeneric = false;        // THIP_ADD_GENERIC: the quantised add always through the 64-bit ACT stage
     bool maxpoolGeneric = false;    // THIP_MAXPOOL_GENERIC: the any-window max pool kernel also for 2 x 2 stride 2
+    int irBlock = -1;               // THIP_IR_BLOCK=0 / 1: inverted-residual blocks as one launch never / wherever it takes them (-1: by cost)
     int decChain = -1;              // THIP_DEC_CHAIN=0 / 1: the records of a decoder's step as one launch never / wherever it takes them, always (-1: by cost, and beside no other one)
     long long decChainWait = 20000000;  // THIP_DEC_CHAIN_WAIT: ticks of 10 ns that a workgroup of dec_chain waits for the others (0: gives up at once)
     int decSplit = 0;               // THIP_DEC_SPLIT: workgroups per 16-column tile of a dec_linear launch of at most four rows: 1 or 2 (0: by its size)
@@ -177,6 +178,34 @@ bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL);
 // Checks the arguments and sets what is the launch's own to choose; false where the kernel does not take them.
 bool planIrExpandDw(IrExpandDwArgs *a);
 hipError_t launchIrExpandDw(const IrExpandDwArgs &a, const LaunchCtx &ctx);
+
+// The two convolutions of IrExpandDwArgs and, behind them, the pointwise one that alone reads their result (C -> O channels), and
+// the residual add behind that.
+struct IrBlockArgs {
+    const int8_t *x;        // [N][H][W][K]
+    const int8_t *wexp;     // [Np][Kp], zero padded
+    const int32_t *bias1, *scale1;  // [Np]
+    const int32_t *wdw;     // [3][C] dwords, byte kw of a dword = tap kw
+    const int32_t *bias2, *scale2;  // [C]
+    const int8_t *wproj;    // [at least O][Kp3], zero padded
+    const int32_t *bias3, *scale3;  // [O]
+    const int8_t *skip;     // [N][OH][OW][O], or null: no add
+    int8_t *out;            // [N][OH][OW][O]
+    int32_t N, H, W, K, Kp, Np, C, OH, OW, S, PT, PL, O, Kp3;
+    int32_t zp;             // of the depthwise op's input: what lies outside the image
+    Requant rq1, rq2, rq3, arq;  // all but the add's with a packed tail
+    int32_t addSkipFirst, addW0, addW1, addBias, addScale;
+    // CKH > 0: as in IrExpandDwArgs
+    int32_t CKH, CS, CPT, CPL, IH, IW, IC, runBytes, czp;
+    int64_t xBytes;
+    int32_t addFolded, columnBlocks, blockColumns, strips, stripRows, segments, segmentRows, cellRows, cellCols, regionColumns, blocks;  // planIrBlock sets these
+};
+// Checks the arguments and sets what is the launch's own to choose; false where the kernel does not take them.
+bool planIrBlock(IrBlockArgs *a);
+// Whether the kernel takes these operands, and whether it is ahead of the two launches that it replaces.
+bool irBlockFits(const IrBlockArgs &a);
+bool irBlockBetter(const IrBlockArgs &a);
+hipError_t launchIrBlock(const IrBlockArgs &a, const LaunchCtx &ctx);
 
 // The small records of the ring kernels (dense or window loader): whether the kernel without tiles in LDS takes these operands and is
 // ahead, and its launch.

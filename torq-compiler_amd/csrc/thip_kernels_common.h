@@ -82,6 +82,11 @@ struct WideRequant {
     int32_t t0lo, t0hi;  // clamp of acc + bias (the whole int32 range when rq.t0_clamp == 0)
     bool plain;          // on, pre == 0, no clamp of t0, zero point folded: requantWideT0<true> applies
     bool preOnly;        // on, pre > 0, no clamp of t0, zero point folded: requantPreShift applies
+    // plain, with int8's own maximum: requantPack4 makes four results from halves of registers
+    bool packed;
+    int packShift;       // shiftMinus32 - 8 (negative: to the left)
+    uint32_t packScale;  // 2^-packShift where that is to the left, in both halves
+    uint32_t packLo;     // out_min * 256, in both halves
     int alignShift;      // preOnly: rq.shift (3..31)
     long long rndAlign;  // preOnly: 2^(shift-1) + zp * 2^shift, added to the product before its bits [shift, shift+32) are taken
 };
@@ -113,6 +118,10 @@ __device__ __forceinline__ WideRequant wideRequant(const Requant &rq) {
     w.rnd64 = (long long)w.rnd * 4294967296LL + (whole ? 2147483648LL : 0LL);  // rnd may be negative (a folded negative zero point)
     w.plain = w.on && w.pre == 0 && !clampT0 && w.zp == 0;
     w.preOnly = w.on && w.pre > 0 && !clampT0 && w.zp == 0;
+    w.packed = w.plain && rq.out_max == 127 && rq.out_min >= -128 && rq.out_min <= 127;
+    w.packShift = w.shiftMinus32 - 8;
+    w.packScale = w.packShift < 0 ? 0x10001u << -w.packShift : 0x10001u;
+    w.packLo = ((uint32_t)rq.out_min & 0xffu) * 0x01000100u;
     w.alignShift = rq.shift & 31;
     w.rndAlign = (w.preOnly ? 1LL << (w.alignShift - 1) : 0LL) + (long long)rq.out_zp * (1LL << w.alignShift);
     return w;
@@ -173,11 +182,59 @@ __device__ __forceinline__ int32_t requantT0(int32_t t0, int32_t scale, long lon
     if (MODE == 3) return requantPreShift(t0, scale, w);
     return requantWideT0<MODE == 2>(t0, scale, w);
 }
+// 0 .. 3 as withRequantMode has them, and for requantPack4: 4 and 5, packed with packShift up to 0 or above it.
+template <typename F>
+__device__ __forceinline__ void withPackMode(const WideRequant &w, F &&f) {
+    if (w.packed && w.packShift <= 0) {
+        f(std::integral_constant<int, 4>{});
+    } else if (w.packed) {
+        f(std::integral_constant<int, 5>{});
+    } else {
+        withRequantMode(w, f);
+    }
+}
 // Four requantised values (each within int8 after the clamp) as the bytes of one dword.
 __device__ __forceinline__ uint32_t packBytes(int32_t a, int32_t b, int32_t c, int32_t d) {
     const uint32_t ab = __builtin_amdgcn_perm((uint32_t)b, (uint32_t)a, 0x0c0c0400u);  // [a.0, b.0, 0, 0]
     const uint32_t cd = __builtin_amdgcn_perm((uint32_t)d, (uint32_t)c, 0x04000c0cu);  // [0, 0, c.0, d.0]
     return ab | cd;
+}
+
+// Four results as the bytes of one dword; t0 and scale: anything with operator[].
+//
+// Modes 4 and 5 (WideRequant::packed): the product's high word is z = floor(y * 2^s), s = shiftMinus32, where y is the result before the
+// clamp and before its fraction is cut off.  Shifted to eight fraction bits and cut to 16 bits with saturation it is y * 256, and its
+// upper byte the result: a saturated half is 127 or -128, the result's own bounds.  The saturation to 16 bits comes for nothing
+// with the packing of two (v_cvt_pk_i16_i32); below eight fraction bits the missing factor is a v_pk_mad_i16 that saturates
+// (a half that the packing has saturated stays so), above them the excess is shifted out before it; out_min is a maximum on both halves.
+// 11 or 13 vector instructions for four results instead of 15: all of them issue at the same rate.
+typedef short v2s __attribute__((ext_vector_type(2)));
+template <int MODE, typename T, typename U>
+__device__ __forceinline__ uint32_t requantPack4(const T &t0, const U &scale, long long rnd, const Requant &rq, const WideRequant &w) {
+    if constexpr (MODE < 4) {
+        int32_t v[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = requantT0<MODE>(t0[e], scale[e], rnd, rq, w);
+        return packBytes(v[0], v[1], v[2], v[3]);
+    } else {
+        uint32_t half[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            int32_t a = mulhiPlusRnd(t0[2 * h], scale[2 * h], w), b = mulhiPlusRnd(t0[2 * h + 1], scale[2 * h + 1], w);
+            if (MODE == 5) {
+                a >>= w.packShift;
+                b >>= w.packShift;
+            }
+            uint32_t pair = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pk_i16(a, b));
+            if (MODE == 4) {
+                uint32_t scaled;
+                asm("v_pk_mad_i16 %0, %1, %2, 0 clamp" : "=v"(scaled) : "v"(pair), "s"(w.packScale));
+                pair = scaled;
+            }
+            half[h] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(v2s, pair), __builtin_bit_cast(v2s, w.packLo)));
+        }
+        return __builtin_amdgcn_perm(half[1], half[0], 0x07050301u);
+    }
 }
 
 // float -> bfloat16 bit pattern.
@@ -241,24 +298,27 @@ __device__ __forceinline__ void splitWork(long long t, const WorkSplit &w, int &
 // multiply-adds, a shift and a clamp (FAST; the launcher proves that nothing overflows).  Anything else takes the
 // generic 64-bit ACT stage.
 template <bool FAST>
+__device__ __forceinline__ uint32_t residualAdd4(uint32_t mine, uint32_t other, bool otherFirst, int32_t w0, int32_t w1, int32_t bias, int32_t scale,
+                                                 long long rnd, const Requant &rq, int32_t folded) {
+    const int32_t wm = otherFirst ? w1 : w0, wo = otherFirst ? w0 : w1;
+    int32_t v[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int32_t a = (int32_t)(int8_t)(mine >> (8 * e)), b = (int32_t)(int8_t)(other >> (8 * e));
+        if (FAST) {
+            v[e] = med3((a * wm + b * wo + folded) >> rq.shift, rq.out_min, rq.out_max);
+        } else {
+            v[e] = requant(a * wm + b * wo, bias, scale, rnd, rq);
+        }
+    }
+    return packBytes(v[0], v[1], v[2], v[3]);
+}
+template <bool FAST>
 __device__ __forceinline__ v4i residualAdd16(v4i mine, v4i other, bool otherFirst, int32_t w0, int32_t w1, int32_t bias, int32_t scale,
                                              long long rnd, const Requant &rq, int32_t folded) {
     v4i r;
-    const int32_t wm = otherFirst ? w1 : w0, wo = otherFirst ? w0 : w1;
 #pragma unroll
-    for (int g = 0; g < 4; g++) {
-        int32_t v[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int32_t a = (int32_t)(int8_t)((uint32_t)mine[g] >> (8 * e)), b = (int32_t)(int8_t)((uint32_t)other[g] >> (8 * e));
-            if (FAST) {
-                v[e] = med3((a * wm + b * wo + folded) >> rq.shift, rq.out_min, rq.out_max);
-            } else {
-                v[e] = requant(a * wm + b * wo, bias, scale, rnd, rq);
-            }
-        }
-        r[g] = (int)packBytes(v[0], v[1], v[2], v[3]);
-    }
+    for (int g = 0; g < 4; g++) r[g] = (int)residualAdd4<FAST>((uint32_t)mine[g], (uint32_t)other[g], otherFirst, w0, w1, bias, scale, rnd, rq, folded);
     return r;
 }
 // Whether the FAST form applies, and its constant: ((sum + bias) + 2^(shift-1)) >> shift, + zp, clamp equals
@@ -336,6 +396,25 @@ __device__ __forceinline__ void streamStore(void *p, T v) {
 struct __attribute__((packed)) UnalignedV4 {
     v4i v;
 };
+
+// 16 bytes that were read d bytes before (d < 0: behind) the place where they are wanted, put right; what lies outside [lo, hi) of them is padding.
+__device__ __forceinline__ v4i fixRun16(v4i bytes, int d, int lo, int hi, uint32_t zp4) {
+    d = d < -15 ? -15 : d > 15 ? 15 : d;
+    unsigned __int128 v;
+    __builtin_memcpy(&v, &bytes, 16);
+    v = d >= 0 ? v >> (8 * d) : v << (-8 * d);
+    v4i r;
+    __builtin_memcpy(&r, &v, 16);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int l = lo - 4 * e, h = hi - 4 * e;
+        const uint32_t below = l <= 0 ? 0u : l >= 4 ? 0xffffffffu : (1u << (8 * l)) - 1u;
+        const uint32_t upto = h <= 0 ? 0u : h >= 4 ? 0xffffffffu : (1u << (8 * h)) - 1u;
+        const uint32_t in = upto & ~below;
+        r[e] = (int)(((uint32_t)r[e] & in) | (zp4 & ~in));
+    }
+    return r;
+}
 
 // One window row of a few-channel convolution: 16 bytes starting at pixel (iy, ix0), channel 0.
 __device__ __forceinline__ v4i gatherRun(const int8_t *__restrict__ A, uint32_t entry, int iy0, int ix0, size_t base,

@@ -145,6 +145,24 @@ static bool matchExpandDw(const DescriptorView &v, const std::vector<uint32_t> &
     return true;
 }
 
+// Behind the two records that `s` stands for, the pointwise convolution that alone reads their result, its add folded into it or none.
+static void matchBlock(const DescriptorView &v, const Tuning &tuning, const std::vector<uint32_t> &uses, Step *s) {
+    const uint32_t last = s->first + 2;
+    if (last >= v.header.op_count) return;
+    const DescOp &e = v.ops[s->first], &d = v.ops[s->first + 1], &g = v.ops[last];
+    if (g.kind != kKindIgemm || g.loader != kLoaderDense || g.KH != 1 || g.KW != 1 || g.SH != 1 || g.SW != 1 || g.out_dtype != 1) return;
+    if (d.out.space != kSpaceTemp || !sameRef(d.out, g.in0) || uses[d.out.index] != 2 || g.K != d.C || g.M != (int64_t)d.N * d.OH * d.OW) return;
+    for (const DescRef *r : {&g.weights, &g.bias, &g.scale, &g.out}) {
+        if (r->offset % 16 != 0) return;
+    }
+    // workgroups read the rows around their own
+    if (sameBuffer(g.out, e.in0) || (g.in1.space != kSpaceNone && (sameBuffer(g.out, g.in1) || g.in1.offset % 16 != 0))) return;
+    const IrBlockArgs a = irBlockArgs(v, *s, [&](const DescRef &r) {
+        return r.space == kSpaceNone ? nullptr : (uint8_t *)(uintptr_t)(0x1000000 + (r.space == kSpaceConst ? v.consts[r.index].offset : 0) + r.offset);
+    });
+    if (tuning.irBlock >= 0 ? tuning.irBlock != 0 && irBlockFits(a) : irBlockBetter(a)) s->count = 3;
+}
+
 // Whether the copy of the rows and a kernel of aligned operands behind it are ahead of a record's own gather kernel, by the time that
 // either takes (us; storing the results costs both the same).  A k-tile of 64 costs the gather 0.55, 0.85, 1.5 or 2.5 in pieces of 8, 4, 2 or
 // 1 bytes and the aligned kernels 0.09, both more where the tiles outnumber the CUs; the copy is a launch (2.3) and its bytes at
@@ -510,6 +528,7 @@ std::vector<Step> planSteps(const DescriptorView &v, const Tuning &tuning) {
             s.first = i;
             s.count = 1;
         }
+        if (s.kind == kStepExpandDw) matchBlock(v, tuning, uses, &s);
         const DescOp *op = s.kind == kStepRecord ? &v.ops[i] : s.kind == kStepPadded ? &s.op : nullptr;
         s.route = !plain && op && op->kind == kKindIgemm ? igemmRoute(v, tuning, *op) : kIgemmOwnTile;
         i += s.count;

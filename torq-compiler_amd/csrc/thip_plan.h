@@ -15,7 +15,7 @@ namespace thip {
 
 enum StepKind {
     kStepRecord,    // one record, by its own launcher
-    kStepExpandDw,  // a pointwise convolution and the depthwise one behind it (ir_expand_dw_i8)
+    kStepExpandDw,  // a pointwise convolution and the depthwise one behind it (ir_expand_dw_i8); three records: and the pointwise one behind that (ir_block_i8)
     kStepPadded,    // a GEMM-shaped record whose channels fill no 16-byte chunks: its input padded, then a dense kernel
     kStepMatmulRt,  // a batch of int8 matmuls with a run-time input2: its transposes and its GEMMs (igemm_rt_i8)
     kStepDecChain,  // grouped linears and small matmuls of a decoder's step, each behind the one before it (dec_chain)
@@ -80,6 +80,41 @@ IgemmArgs igemmArgs(const DescriptorView &v, const DescOp &op, At &&at) {
         a.add_skip_first = ap.other_first;
         a.add_w0 = ap.w0; a.add_w1 = ap.w1; a.add_bias = ap.bias; a.add_scale = ap.scale;
         a.arq = Requant{ap.shift, ap.output_zp, ap.output_min, ap.output_max, 0, 0};
+    }
+    return a;
+}
+
+// The arguments of a step of three records that widen, convolve depthwise and narrow, its operands where `at` says.
+template <typename At>
+IrBlockArgs irBlockArgs(const DescriptorView &v, const Step &s, At &&at) {
+    const DescOp &e = v.ops[s.first], &d = v.ops[s.first + 1], &g = v.ops[s.first + 2];
+    const IgemmArgs last = igemmArgs(v, g, at);
+    IrBlockArgs a;
+    memset(&a, 0, sizeof(a));
+    a.x = (const int8_t *)at(e.in0);
+    a.wexp = (const int8_t *)at(e.weights);
+    a.bias1 = (const int32_t *)at(e.bias);
+    a.scale1 = (const int32_t *)at(e.scale);
+    a.wdw = (const int32_t *)at(d.weights);
+    a.bias2 = (const int32_t *)at(d.bias);
+    a.scale2 = (const int32_t *)at(d.scale);
+    a.wproj = last.Bp;
+    a.bias3 = last.bias;
+    a.scale3 = last.scale;
+    a.skip = last.skip;
+    a.out = (int8_t *)last.out;
+    a.N = d.N; a.H = d.H; a.W = d.W; a.K = e.K; a.Kp = e.Kp; a.Np = e.Np; a.C = d.C;
+    a.OH = d.OH; a.OW = d.OW; a.S = d.SW; a.PT = d.PT; a.PL = d.PL; a.O = g.Nn; a.Kp3 = g.Kp; a.zp = d.input_zp;
+    a.rq1 = Requant{e.shift, e.output_zp, e.output_min, e.output_max, e.pre_shift, e.t0_clamp};
+    a.rq2 = Requant{d.shift, d.output_zp, d.output_min, d.output_max, d.pre_shift, d.t0_clamp};
+    a.rq3 = last.rq;
+    a.arq = last.arq;
+    a.addSkipFirst = last.add_skip_first;
+    a.addW0 = last.add_w0; a.addW1 = last.add_w1; a.addBias = last.add_bias; a.addScale = last.add_scale;
+    if (e.loader == kLoaderRuns) {
+        a.CKH = e.KH; a.CS = e.SH; a.CPT = e.PT; a.CPL = e.PL; a.IH = e.H; a.IW = e.W; a.IC = e.C;
+        a.runBytes = e.KW * e.C; a.czp = e.input_zp;
+        a.xBytes = (int64_t)e.N * e.H * e.W * e.C;
     }
     return a;
 }
