@@ -25,3 +25,19 @@ def test_conv_patch(device, kw, monkeypatch):
     assert "conv_patch_i8" in families(launched), launched
     assert_bit_exact(got[0], want, wl.name)
     check_own_kernels(device, wl, [want], "device")
+
+
+@pytest.mark.parametrize("shift", [31, 32, 33, 40, 41, 45, 46])
+@pytest.mark.parametrize("bounds", [dict(output_min=-128), dict(output_min=17, output_zp=20), dict(output_min=-128, output_max=126)], ids=lambda b: "_".join(str(v) for v in b.values()))
+def test_packed_requant(device, shift, bounds, monkeypatch):
+    """Both packed tails at the ends of their shifts, and the ones beside them; bit for bit."""
+    top = min(shift - 11, 30)  # a multiplier's highest bit: results over all of int8 where the shift allows it
+    monkeypatch.setattr(w, "random_requant", lambda rng, n, realistic: (rng.integers(1 << top, (2 << top) - 1, size=n).astype("int32"), [shift] * n))
+    wl = w.conv2d_workload(N=17, H=56, W=54, C=16, O=48, realistic=True, **bounds)
+    print("[gpu-case]", wl.name, shift, bounds, flush=True)
+    launched = []
+    got, _ = run_on_gpu(device, wl, via="device", launched=launched)
+    assert "conv_patch_i8" in families(launched), launched
+    want = oracle_eval(wl)[0]
+    assert len(set(want.reshape(-1).tolist())) > 8, wl.name
+    assert_bit_exact(got[0], want, wl.name)

@@ -13,7 +13,9 @@ namespace thip {
 // column of 128 brings and multiplies 128 channels where there are 96 (56x56x96 -> 96, 32 images: 130 MB through LDS, 19.0 us; here 34
 // MB and 15.3).
 //
-// What is left is serial in a workgroup, mostly one to a CU: weights and patch into LDS, the MFMA steps, the epilogue.
+// What is left is serial in a workgroup, mostly one to a CU: weights and patch into LDS, the MFMA steps, the epilogue.  The sums start at
+// the bias and the results are packed as requantPack4 says, as each of the two waves of a SIMD issues a vector instruction in 8 cycles at most (56x56x96: 15.8
+// -> 15.4 us).  Weights in parts that are multiplied as they arrive (by LDS-DMA) are slower than all at once: 16.0 against 15.2.
 //
 // Pixels and weight rows are padded in LDS to pitches of 16-byte units that are no multiple of four, so that the eight
 // lanes that a ds_read_b128 serves at a time hit all banks once.
@@ -107,7 +109,11 @@ __global__ __launch_bounds__(512) void conv_patch_i8(IgemmArgs p, ConvPatchPlan 
 #pragma unroll
                 for (int j = 0; j < NB; j++) {
 #pragma unroll
-                    for (int r = 0; r < 16; r++) acc[i][j][r] = 0;
+                    for (int g = 0; g < 4; g++) {
+                        const v4i b4 = *(const v4i *)(ldsBias + 32 * j + 8 * g + 4 * half);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) acc[i][j][4 * g + e] = b4[e];
+                    }
                 }
             }
             struct Operands {
@@ -139,26 +145,21 @@ __global__ __launch_bounds__(512) void conv_patch_i8(IgemmArgs p, ConvPatchPlan 
                 load(s + 2, o0);
                 multiply(o1);
             }
-            withRequantMode(wrq, [&](auto tag) {
+            withPackMode(wrq, [&](auto tag) {
                 constexpr int kMode = decltype(tag)::value;
 #pragma unroll
                 for (int j = 0; j < NB; j++) {
-                    v4i b4[4], s4[4];
+                    v4i s4[4];
 #pragma unroll
-                    for (int g = 0; g < 4; g++) {
-                        b4[g] = *(const v4i *)(ldsBias + 32 * j + 8 * g + 4 * half);
-                        s4[g] = *(const v4i *)(ldsScale + 32 * j + 8 * g + 4 * half);
-                    }
+                    for (int g = 0; g < 4; g++) s4[g] = *(const v4i *)(ldsScale + 32 * j + 8 * g + 4 * half);
                     const int n = 32 * j + 16 * half;
 #pragma unroll
                     for (int i = 0; i < 2; i++) {
                         uint32_t d[4];
 #pragma unroll
                         for (int g = 0; g < 4; g++) {
-                            int32_t v[4];
-#pragma unroll
-                            for (int e = 0; e < 4; e++) v[e] = requantT0<kMode>((int32_t)((uint32_t)acc[i][j][4 * g + e] + (uint32_t)b4[g][e]), s4[g][e], rnd, p.rq, wrq);
-                            d[g] = packBytes(v[0], v[1], v[2], v[3]);
+                            const v4i t0 = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+                            d[g] = requantPack4<kMode>(t0, s4[g], rnd, p.rq, wrq);
                         }
                         const auto s02 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
                         const auto s13 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
