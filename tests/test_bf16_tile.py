@@ -25,6 +25,17 @@ def test_every_tile(device, tile, monkeypatch):
         assert kernels[-1].startswith("fc_bf16<%d," % {1: 64, 2: 64, 3: 128, 4: 128, 5: 256}[tile]) and len(kernels[-1].split(",")) == 8, kernels
 
 
+@pytest.mark.parametrize("tile", [0, 1, 2, 3, 4, 5])
+@pytest.mark.parametrize("columns", [57, 58, 59, 60, 61, 62, 63, 7, 1, 97, 258])
+def test_ragged_columns(device, tile, columns, monkeypatch):
+    """Every number of columns behind the last whole eight, rows that begin at any of their alignments; 0: the streaming form."""
+    monkeypatch.setenv("THIP_FC_TILE", str(tile))
+    wl = w.fully_connected_bf16_workload(70, 64, columns, clamp=(-0.5, 0.75) if columns % 2 else None)
+    print("[gpu-case]", tile, wl.name, flush=True)
+    got, _ = run_on_gpu(device, wl, via="device")
+    assert_bf16_close(got[0], oracle_eval(wl)[0], wl.name + " (gpu)", magnitude=_magnitude(wl))
+
+
 def test_nothing_beyond_k_reaches_a_result(device, monkeypatch):
     """K ends inside a k-tile: what follows a row in memory is the next row, infinite here, and must not be multiplied."""
     monkeypatch.setenv("THIP_FC_TILE", "1")

@@ -20,7 +20,8 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 // Bias, clamp, round to bf16 and store one 32 x 32 accumulator tile: register 4 q + e of lane (r, h) is
-// out[m0 + r][n0 + 8 q + 4 h + e].  fcBf16StoreQuad stores the four registers of one q.
+// out[m0 + r][n0 + 8 q + 4 h + e].  fcBf16StoreQuad stores the four registers of one q, at any alignment (14 x 1000 -> 521: 6.5 us in
+// single elements, 6.3).
 __device__ __forceinline__ void fcBf16StoreQuad(const FcBf16Args &p, const float (&a)[4], int m0, int n0, int r, int h, int q) {
     const int m = m0 + r;
     if (m >= p.M) return;
@@ -32,8 +33,8 @@ __device__ __forceinline__ void fcBf16StoreQuad(const FcBf16Args &p, const float
         const float t0 = a[e] + p.bias[ne];
         o[e] = bf16Bits(t0 < p.lo ? p.lo : (t0 > p.hi ? p.hi : t0));
     }
-    if ((p.N & 3) == 0 && n + 3 < p.N) {
-        *(v2i *)(p.out + (size_t)m * p.N + n) = v2i{(int)((uint32_t)o[0] | ((uint32_t)o[1] << 16)), (int)((uint32_t)o[2] | ((uint32_t)o[3] << 16))};
+    if (n + 3 < p.N) {
+        ((UnalignedV2 *)(p.out + (size_t)m * p.N + n))->v = v2i{(int)((uint32_t)o[0] | ((uint32_t)o[1] << 16)), (int)((uint32_t)o[2] | ((uint32_t)o[3] << 16))};
     } else {
 #pragma unroll
         for (int e = 0; e < 4; e++) {

@@ -30,14 +30,16 @@ __device__ __forceinline__ uint32_t packBf16(float lo, float hi) {
 // packed weights have in memory: FRAG weights go to LDS as they are, 4 KiB of 32 columns x 64 k at a time, and a
 // fragment read is 1 KiB in lane order.  Row-major weights (a run-time operand) are staged like the activations.
 //
-// The weights are the MFMA's row operand: register 4 q + e of lane (r, h) is out[m = r][n = 8 q + 4 h + e].  Two
-// v_permlane32_swap per pair of q give a lane 8 neighbouring columns of one row: one 16-byte store.
+// The weights are the MFMA's row operand: register 4 q + e of lane (r, h) is out[m = r][n = 8 q + 4 h + e].  The results go through LDS, each
+// wave's by itself, so that a store covers whole runs of a row: columns that are no whole eight, whose rows begin anywhere, cost
+// what others do (2048 x 1152 -> 6911 67.7 us in single elements, 43.3 in unaligned 16-byte pieces of a lane's own row, 35.0 in runs; 1649 x
+// 288 -> 4747 28.6, 13.5, 12.0; 2608 x 1024 -> 2530 33.7, 20.1, 19.9; 2048 x 1152 -> 6912 34.3 in aligned pieces, 34.0).
 //
 // KG groups of waves share a workgroup's outputs and take every KG-th k-tile each, with a ring of their own; their sums
 // meet in LDS (few tiles under a long K: more loads in flight per CU).
 //
 // Bound by the ring's data path (64 KiB per k-tile of a 256 x 256 tile in 1.1 us, 58 KB/us per CU where LDS-DMA loads alone, of lines in
-// the XCD's L2, reach 138; 0.86 us of MFMA work), with the launch, the ring fill and 28 MB of output at the end next to it: 2048 x 1152 -> 6912 takes 34.4 us (950 TFLOP/s).  Eight waves
+// the XCD's L2, reach 138; 0.86 us of MFMA work), with the launch, the ring fill and 28 MB of output at the end next to it: 2048 x 1152 -> 6912 takes 34.0 us (960 TFLOP/s).  Eight waves
 // on the 256 x 256 tile rather than four: 35.7 -> 34.4 us, and the epilogue of a short K 13.0 -> 9.1.
 // ---------------------------------------------------------------------------
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, int KG, bool FRAG>
@@ -255,51 +257,45 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *KG * 64, BLOCKS_PER_CU) void fc_b
     if (tid < BN) ldsBias[tid] = myBias;
     __syncthreads();
     if (KG > 1 && kg > 0) return;
-    const bool wide = (p.N & 7) == 0 && (((uintptr_t)p.out) & 15) == 0;
     // Bias, clamp, v_cvt_pk_bf16_f32 and the stores; a copy without the clamp's compares, which are half the instructions
-    // of an epilogue that every CU runs at the same time (a linear layer has none).
+    // of an epilogue that every CU runs at the same time (a linear layer has none).  32 rows of a wave's results pass through LDS, from where they are
+    // stored in runs of whole rows of the wave's columns, at any alignment.
+    constexpr int CHUNKS = WTN / 8;  // of eight results in a row of a wave
+    int8_t *mine = smem + BN * 4 + wave * (WTM * WTN * 2);
+    const int sc = lane % CHUNKS, sr = lane / CHUNKS, ns = n0 + wn * WTN + sc * 8;
     auto finish = [&](auto clampTag) {
         constexpr bool kClamp = decltype(clampTag)::value;
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int nl = wn * WTN + j * 32;
-            float b[16];
+        for (int i = 0; i < TM; i++) {
+            int8_t *rows = mine + i * (32 * WTN * 2);
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const float4 b4 = *(const float4 *)(ldsBias + nl + 8 * q + 4 * half);
-                b[4 * q] = b4.x; b[4 * q + 1] = b4.y; b[4 * q + 2] = b4.z; b[4 * q + 3] = b4.w;
-            }
+            for (int j = 0; j < TN; j++) {
 #pragma unroll
-            for (int i = 0; i < TM; i++) {
-                const int m = m0 + wm * WTM + i * 32 + fr;
-                uint32_t d[8];  // d[2 q + (e >> 1)]: columns 8 q + 4 half + e, + 1
+                for (int q = 0; q < 4; q++) {
+                    const float4 b4 = *(const float4 *)(ldsBias + wn * WTN + j * 32 + 8 * q + 4 * half);
+                    const float b[4] = {b4.x, b4.y, b4.z, b4.w};
+                    float v[4];
 #pragma unroll
-                for (int t = 0; t < 8; t++) {
-                    float v[2];
-#pragma unroll
-                    for (int e = 0; e < 2; e++) {
-                        v[e] = acc[j][i][2 * t + e] + b[2 * t + e];
+                    for (int e = 0; e < 4; e++) {
+                        v[e] = acc[j][i][4 * q + e] + b[e];
                         if (kClamp) v[e] = v[e] < p.lo ? p.lo : (v[e] > p.hi ? p.hi : v[e]);
                     }
-                    d[t] = packBf16(v[0], v[1]);
+                    *(v2i *)(rows + fr * (WTN * 2) + (((4 * j + q) ^ fr) % CHUNKS) * 16 + 8 * half) = v2i{(int)packBf16(v[0], v[1]), (int)packBf16(v[2], v[3])};
                 }
-                if (wide) {
-                    // columns 16 q2 .. of this 32: the lower half of the wave ends up with the first 8, the upper with the others
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
 #pragma unroll
-                    for (int q2 = 0; q2 < 2; q2++) {
-                        const auto s0 = __builtin_amdgcn_permlane32_swap(d[4 * q2], d[4 * q2 + 2], false, false);
-                        const auto s1 = __builtin_amdgcn_permlane32_swap(d[4 * q2 + 1], d[4 * q2 + 3], false, false);
-                        const int n = n0 + nl + 16 * q2 + 8 * half;
-                        if (m < p.M && n < p.N) *(v4i *)(p.out + (size_t)m * p.N + n) = v4i{(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
-                    }
-                } else if (m < p.M) {
+            for (int t = 0; t < CHUNKS / 2; t++) {
+                const int r = t * (64 / CHUNKS) + sr, m = m0 + wm * WTM + i * 32 + r;
+                const v4i v = *(const v4i *)(rows + r * (WTN * 2) + ((sc ^ r) % CHUNKS) * 16);
+                if (m >= p.M || ns >= p.N) continue;
+                uint16_t *out = p.out + (size_t)m * p.N + ns;
+                if (ns + 8 <= p.N) {
+                    ((UnalignedV4 *)out)->v = v;
+                } else {
 #pragma unroll
-                    for (int t = 0; t < 8; t++) {
-#pragma unroll
-                        for (int e = 0; e < 2; e++) {
-                            const int n = n0 + nl + 8 * (t >> 1) + 4 * half + 2 * (t & 1) + e;
-                            if (n < p.N) p.out[(size_t)m * p.N + n] = (uint16_t)(d[t] >> (16 * e));
-                        }
+                    for (int e = 0; e < 7; e++) {
+                        if (ns + e < p.N) out[e] = (uint16_t)((uint32_t)v[e >> 1] >> (16 * (e & 1)));
                     }
                 }
             }
@@ -312,7 +308,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *KG * 64, BLOCKS_PER_CU) void fc_b
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, int KG, bool FRAG>
 static hipError_t launchTile(const FcBf16Args &a, const LaunchCtx &ctx) {
     auto kernel = fc_bf16<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, KG, FRAG>;
-    constexpr size_t lds = (size_t)KG * STAGES * (BM + BN) * 128;
+    constexpr size_t ring = (size_t)KG * STAGES * (BM + BN) * 128, results = (size_t)BN * 4 + (size_t)BM * BN * 2, lds = ring > results ? ring : results;
     static std::once_flag once;
     static hipError_t configured = hipSuccess;
     std::call_once(once, [&] { configured = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });

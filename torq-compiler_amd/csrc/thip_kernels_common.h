@@ -396,6 +396,10 @@ __device__ __forceinline__ void streamStore(void *p, T v) {
 struct __attribute__((packed)) UnalignedV4 {
     v4i v;
 };
+// The same of 8 bytes.
+struct __attribute__((packed)) UnalignedV2 {
+    v2i v;
+};
 
 // 16 bytes that were read d bytes before (d < 0: behind) the place where they are wanted, put right; what lies outside [lo, hi) of them is padding.
 __device__ __forceinline__ v4i fixRun16(v4i bytes, int d, int lo, int hi, uint32_t zp4) {
