@@ -184,7 +184,9 @@ static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op
         break;
     }
     case kKindIgemm: {
-        const IgemmArgs a = igemmArgs(viewOf(e), op, [&](const DescRef &r) { return resolve(e, r, bp); });
+        auto at = [&](const DescRef &r) { return resolve(e, r, bp); };
+        const bool asIs = route == kIgemmDirect && e->ops[i].loader == kLoaderGather && op.in0.space != kSpacePlan;
+        const IgemmArgs a = asIs ? raggedArgs(viewOf(e), op, e->ops[i].C, at) : igemmArgs(viewOf(e), op, at);
         if (route == kIgemmDirect) err = launchIgemmDirect(a, ctx);
         else if (route == kIgemmPatch) err = launchConvPatch(a, ctx);
         else err = launchIgemm(a, op.variant, ctx, route == kIgemmWide);
@@ -569,7 +571,7 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
     }
     case kStepPadded: {
         uint8_t *const *buffers = &e->stepBuffers[2 * (size_t)(&s - e->steps.data())];
-        err = launchPadRows((const int8_t *)resolve(e, e->ops[s.first].in0, bp), (int8_t *)buffers[0], s.rows, s.from, s.to, ctx);
+        if (s.rows > 0) err = launchPadRows((const int8_t *)resolve(e, e->ops[s.first].in0, bp), (int8_t *)buffers[0], s.rows, s.from, s.to, ctx);
         if (err == hipSuccess) return launchOp(e, s.first, s.op, bp, ctx, scratch, buffers, s.route);
         break;
     }
@@ -927,7 +929,7 @@ static bool addStep(thip_executable_t *e, Step &&planned) {
         uint8_t **buffers = &e->stepBuffers[e->stepBuffers.size() - 2];
         const size_t rows = (size_t)step.rows * step.to, bytes = rows + step.constants.size();
         if (e->tuning.stepBytes >= 0 && (long long)bytes > e->tuning.stepBytes) err = hipErrorOutOfMemory;
-        if (err == hipSuccess) err = hipMalloc((void **)&buffers[0], rows);
+        if (err == hipSuccess && rows > 0) err = hipMalloc((void **)&buffers[0], rows);
         if (err == hipSuccess) err = hipMalloc((void **)&buffers[1], step.constants.size());
         if (err == hipSuccess) err = hipMemcpy(buffers[1], step.constants.data(), step.constants.size(), hipMemcpyHostToDevice);
         std::vector<uint8_t>().swap(step.constants);
@@ -965,7 +967,7 @@ static bool addStep(thip_executable_t *e, Step &&planned) {
         for (auto &ptr : placeholder) ptr = (uint8_t *)(uintptr_t)0x1000000;
         char name[96] = "";
         if (launchStep(e, step, placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name)}) == THIP_OK) {
-            if (step.kind == kStepPadded) e->launchNames.push_back("pad_rows_i8");
+            if (step.kind == kStepPadded && step.rows > 0) e->launchNames.push_back("pad_rows_i8");
             e->launchNames.push_back(name[0] ? name : opKernelName(e->ops[step.first]));
             return true;
         }

@@ -16,8 +16,13 @@ namespace thip {
 //
 // Bound by latency: one or two memory round trips, the LDS exchange and the launch.  A tile brings 64 bytes per k where a 64 x 64
 // tile brings 32 per output: taken up to two workgroups per CU only (igemmDirectBetter).
+//
+// RAGGED: rows (pixels) of no whole 16-byte chunks, as they are in memory.  A row's last chunk reaches into the next row, where the weights have zeros; the
+// last row's is read at the tensor's end and shifted.  1: rows of whole dwords, which a 16-byte load takes at no loss (1583 x 4184 -> 23 8.3 us;
+// rows copied to whole chunks first 15.7).  2: any other, whose chunks are put together from the dwords they lie in: a wave's 16-byte load at odd
+// addresses takes the CU 190 cycles in place of 30 (3 x 5637 -> 567 11.9 -> 9.0, 5x5 19x19x387 -> 134 31.7 -> 19.7).
 // ---------------------------------------------------------------------------
-template <bool WINDOW, int NW>
+template <bool WINDOW, int NW, int RAGGED>
 __global__ __launch_bounds__(NW * 64) void igemm_direct_i8(IgemmArgs p, FastDiv divC, FastDiv divKW, FastDiv divFrame, FastDiv divOW) {
     constexpr int U = 4;  // steps in flight
     __shared__ v4i partial[NW][4][64];
@@ -35,7 +40,9 @@ __global__ __launch_bounds__(NW * 64) void igemm_direct_i8(IgemmArgs p, FastDiv 
 
     int y0 = 0, x0 = 0;
     uint32_t imageRow = 0;
-    const int8_t *arow = p.A + (WINDOW ? 0 : (size_t)m * p.K);
+    const int pixel = RAGGED ? p.row_bytes : p.C;
+    const int8_t *arow = p.A + (WINDOW || RAGGED ? 0 : (size_t)m * p.K);
+    const uint32_t rowAt = RAGGED && !WINDOW ? (uint32_t)m * (uint32_t)pixel : 0u, last = RAGGED ? (uint32_t)p.a_bytes - 16u : 0u;
     if (WINDOW) {
         const int image = (int)fastDiv((uint32_t)m, divFrame), rem = m - image * (p.OH * p.OW);
         const int oy = (int)fastDiv((uint32_t)rem, divOW), ox = rem - oy * p.OW;
@@ -46,11 +53,45 @@ __global__ __launch_bounds__(NW * 64) void igemm_direct_i8(IgemmArgs p, FastDiv 
     const int8_t *wrow = p.Bp + (size_t)(n0 + fr) * p.Kp + 16 * half;
     const int zp4 = (int)((uint32_t)(p.input_zp & 0xff) * 0x01010101u);
     const int steps = (p.K + 31) / 32;
+    // A chunk of RAGGED rows is asked for with load and finished with finish.  One that would end behind A is read before its place, at A's end.  RAGGED 2,
+    // rows that are no whole dwords: read from the dword that it begins in, and the dword behind it (or A's last) too.
+    struct Chunk {
+        v4i v;
+        uint32_t off, behind;
+    };
+    auto load = [&](Chunk &c, uint32_t off) {
+        if (RAGGED) {
+            uint32_t at = off < last ? off : last;
+            if (RAGGED == 2) {
+                at &= ~3u;
+                c.behind = ((const UnalignedU32 *)(arow + (at < last - 4u ? at + 16u : last + 12u)))->v;
+            }
+            c.off = off;
+            c.v = ((const UnalignedV4 *)(arow + at))->v;
+        } else {
+            c.v = *(const v4i *)(arow + off);
+        }
+    };
+    auto finish = [&](const Chunk &c) {
+        if (!RAGGED) return c.v;
+        const uint32_t at = c.off < last ? c.off : last;
+        v4i x = c.v;
+        if (RAGGED == 2) {
+            // at A's end the dword was read up to four bytes early
+            const uint32_t base = at & ~3u, early = base + 4u > last ? base + 4u - last : 0u;
+            const uint32_t w[5] = {(uint32_t)x[0], (uint32_t)x[1], (uint32_t)x[2], (uint32_t)x[3], (uint32_t)((uint64_t)c.behind >> (8 * early))};
+#pragma unroll
+            for (int e = 0; e < 4; e++) x[e] = (int)__builtin_amdgcn_alignbyte(w[e + 1], w[e], at & 3u);
+        }
+        if (c.off != at) x = fixRun16(x, (int)(c.off - at), 0, 16, 0u);
+        return x;
+    };
     v16i acc;
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[r] = 0;
     for (int s0 = wave * U; s0 < steps; s0 += NW * U) {
-        v4i a[U], w[U];
+        Chunk a[U];
+        v4i w[U];
         bool inside[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
@@ -62,18 +103,18 @@ __global__ __launch_bounds__(NW * 64) void igemm_direct_i8(IgemmArgs p, FastDiv 
                 const int kh = (int)fastDiv((uint32_t)tap, divKW), kw = tap - kh * p.KW;
                 const int y = y0 + kh, x = x0 + kw;
                 inside[u] = (unsigned)y < (unsigned)p.H && (unsigned)x < (unsigned)p.W;
-                const uint32_t off = inside[u] ? ((imageRow + (uint32_t)y) * (uint32_t)p.W + (uint32_t)x) * (uint32_t)p.C + (uint32_t)c : 0u;
-                a[u] = *(const v4i *)(arow + off);
+                const uint32_t off = inside[u] ? ((imageRow + (uint32_t)y) * (uint32_t)p.W + (uint32_t)x) * (uint32_t)pixel + (uint32_t)c : 0u;
+                load(a[u], off);
             } else {
                 inside[u] = true;
-                a[u] = *(const v4i *)(arow + kk);
+                load(a[u], rowAt + (uint32_t)kk);
             }
             w[u] = *(const v4i *)(wrow + 32 * s);
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if (s0 + u >= steps) break;
-            v4i x = a[u];
+            v4i x = finish(a[u]);
             if (WINDOW) {
 #pragma unroll
                 for (int d = 0; d < 4; d++) x[d] = inside[u] ? x[d] : zp4;
@@ -106,8 +147,8 @@ __global__ __launch_bounds__(NW * 64) void igemm_direct_i8(IgemmArgs p, FastDiv 
         }
     }
     const size_t at = (size_t)m * p.N + n;
-    if (p.out_dtype == kDtypeI8 && whole && (p.N & 3) == 0) {
-        *(uint32_t *)((int8_t *)p.out + at) = packBytes(v[0], v[1], v[2], v[3]);
+    if (p.out_dtype == kDtypeI8 && whole) {
+        ((UnalignedU32 *)((int8_t *)p.out + at))->v = packBytes(v[0], v[1], v[2], v[3]);
     } else {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
@@ -123,12 +164,17 @@ static bool directTakes(const IgemmArgs &a) {
     const bool window = a.loader == kLoaderWindow;
     if (!a.A || !a.Bp || !a.bias || !a.scale || !a.out || a.M <= 0 || a.N <= 0 || a.K <= 0 || (!window && a.loader != kLoaderDense)) return false;
     if (a.K % 16 != 0 || a.Kp < (a.K + 31) / 32 * 32 || a.Np < (a.N + 31) / 32 * 32 || a.Kp % 16 != 0) return false;
-    if (((uintptr_t)a.A | (uintptr_t)a.Bp | (uintptr_t)a.bias | (uintptr_t)a.scale) & 15) return false;
+    if ((((uintptr_t)a.Bp | (uintptr_t)a.bias | (uintptr_t)a.scale) & 15) || (((uintptr_t)a.A & 15) && a.row_bytes == 0)) return false;
     if (a.out_dtype < kDtypeI8 || a.out_dtype > kDtypeI32 || ((uintptr_t)a.out & 3) || (a.skip && (((uintptr_t)a.skip & 3) || a.N % 4 != 0 || a.out_dtype != kDtypeI8))) return false;
     if (window) {
         if (a.C < 16 || a.C % 16 != 0 || a.KH <= 0 || a.KW <= 0 || a.H <= 0 || a.W <= 0 || a.OH <= 0 || a.OW <= 0 || a.SH <= 0 || a.SW <= 0 || a.PT < 0 || a.PL < 0) return false;
         if (a.M % (a.OH * a.OW) != 0 || (long long)a.K != (long long)a.KH * a.KW * a.C) return false;
-        if (a.a_bytes != (long long)(a.M / (a.OH * a.OW)) * a.H * a.W * a.C || a.a_bytes >= (1LL << 32)) return false;
+        if (a.a_bytes != (long long)(a.M / (a.OH * a.OW)) * a.H * a.W * (a.row_bytes ? a.row_bytes : a.C) || a.a_bytes >= (1LL << 32)) return false;
+    }
+    if (a.row_bytes != 0) {
+        // a row's last chunk reaches into the next one; behind the last row its load begins earlier
+        if (a.row_bytes < 0 || (a.row_bytes + 15) / 16 * 16 != a.C || a.a_bytes < 20 || a.a_bytes >= (1LL << 31)) return false;
+        if (!window && (a.K != a.C || a.a_bytes != (long long)a.M * a.row_bytes)) return false;
     }
     return true;
 }
@@ -145,10 +191,11 @@ bool igemmDirectBetter(const IgemmArgs &a) {
     return a.loader == kLoaderWindow ? tiles <= 1024 && bytes <= 50000000 : tiles <= 256 && bytes <= 25000000;
 }
 
-template <bool WINDOW, int NW>
+template <bool WINDOW, int NW, int RAGGED>
 static hipError_t launchDirect(const IgemmArgs &a, const LaunchCtx &ctx) {
     const long long tiles = directTiles(a);
-    THIP_ENQUEUE(ctx, kernelLabel("igemm_direct_i8", {(int)WINDOW, NW}), (igemm_direct_i8<WINDOW, NW>), dim3((unsigned)tiles), dim3(NW * 64), 0, a,
+    const std::string label = RAGGED ? kernelLabel("igemm_direct_i8", {(int)WINDOW, NW, RAGGED}) : kernelLabel("igemm_direct_i8", {(int)WINDOW, NW});
+    THIP_ENQUEUE(ctx, label, (igemm_direct_i8<WINDOW, NW, RAGGED>), dim3((unsigned)tiles), dim3(NW * 64), 0, a,
                  makeFastDiv((uint32_t)(WINDOW ? a.C : 1)), makeFastDiv((uint32_t)(WINDOW ? a.KW : 1)), makeFastDiv((uint32_t)(WINDOW ? a.OH * a.OW : 1)),
                  makeFastDiv((uint32_t)(WINDOW ? a.OW : 1)));
     return hipGetLastError();
@@ -160,8 +207,16 @@ hipError_t launchIgemmDirect(const IgemmArgs &a, const LaunchCtx &ctx) {
     // eight waves while that leaves a CU two workgroups (3x3 56x56x64 -> 64: 3.4 us against 3.8 with four), four beyond (142x142x144
     // -> 8, batch 3: 6.0 against 6.8)
     const bool few = directTiles(a) <= 400;
-    if (window) return few ? launchDirect<true, 8>(a, ctx) : launchDirect<true, 4>(a, ctx);
-    return few ? launchDirect<false, 8>(a, ctx) : launchDirect<false, 4>(a, ctx);
+    if (a.row_bytes % 4 != 0) {
+        if (window) return few ? launchDirect<true, 8, 2>(a, ctx) : launchDirect<true, 4, 2>(a, ctx);
+        return few ? launchDirect<false, 8, 2>(a, ctx) : launchDirect<false, 4, 2>(a, ctx);
+    }
+    if (a.row_bytes != 0) {
+        if (window) return few ? launchDirect<true, 8, 1>(a, ctx) : launchDirect<true, 4, 1>(a, ctx);
+        return few ? launchDirect<false, 8, 1>(a, ctx) : launchDirect<false, 4, 1>(a, ctx);
+    }
+    if (window) return few ? launchDirect<true, 8, 0>(a, ctx) : launchDirect<true, 4, 0>(a, ctx);
+    return few ? launchDirect<false, 8, 0>(a, ctx) : launchDirect<false, 4, 0>(a, ctx);
 }
 
 }  // namespace thip

@@ -60,7 +60,7 @@ struct Tuning {
     bool noK128 = false;            // THIP_NO_K128: no 128-byte k-tiles chosen at launch (the emitter reads the same switch for its own choice)
     bool noFcDeep = false;          // THIP_NO_FC_DEEP
     bool plainRecords = false;      // a switch asks for a tile or a loader by name: every record runs by its own launcher
-    int padRows = -1;               // THIP_PAD_ROWS=0 / 1: rows of ragged channels padded for the kernels of aligned operands never / wherever these take them (-1: by cost)
+    int padRows = -1;               // THIP_PAD_ROWS=0 / 1: rows of ragged channels padded for the kernels of aligned operands never / wherever these take them; 2: read as they are by igemm_direct_i8 wherever it takes them (-1: by cost)
     long long stepBytes = -1;       // THIP_STEP_BYTES: device memory that a launch may take for operands of its own (negative: what there is); records run where it is short
     bool noFcWide = false;          // THIP_NO_FC_WIDE
     bool addGeneric = false;        // THIP_ADD_GENERIC: the quantised add always through the 64-bit ACT stage
@@ -94,6 +94,7 @@ struct IgemmArgs {
     int32_t M, N, K, Kp, Np;
     int32_t H, W, C, OH, OW, SH, SW, PT, PL;
     int32_t KH, KW;         // window loader only
+    int32_t row_bytes;      // igemm_direct_i8 only: what a pixel of A takes where C is that rounded up to whole 16-byte chunks (0: C)
     int32_t input_zp;
     int32_t out_dtype;
     int64_t a_bytes;        // size of A in bytes (the run loader keeps its 16-byte loads inside it)

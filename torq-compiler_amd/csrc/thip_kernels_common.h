@@ -396,9 +396,12 @@ __device__ __forceinline__ void streamStore(void *p, T v) {
 struct __attribute__((packed)) UnalignedV4 {
     v4i v;
 };
-// The same of 8 bytes.
+// The same of 8 and 4 bytes.
 struct __attribute__((packed)) UnalignedV2 {
     v2i v;
+};
+struct __attribute__((packed)) UnalignedU32 {
+    uint32_t v;
 };
 
 // 16 bytes that were read d bytes before (d < 0: behind) the place where they are wanted, put right; what lies outside [lo, hi) of them is padding.

@@ -120,6 +120,11 @@ static bool matchMatmulRt(const DescriptorView &v, const std::vector<uint32_t> &
     return true;
 }
 
+// Where an operand lies, for the rules that ask for alignments only: aligned as a dispatch's are.
+static uint8_t *plannedAt(const DescriptorView &v, const DescRef &r) {
+    return r.space == kSpaceNone ? nullptr : (uint8_t *)(uintptr_t)(0x1000000 + (r.space == kSpaceConst ? v.consts[r.index].offset : 0) + r.offset);
+}
+
 // Whether the requant of a record has a tail of 32-bit arithmetic (see WideRequant).
 static bool narrowRequant(const DescOp &op) { return op.shift == 32 || (int64_t)op.shift + op.pre_shift >= 33; }
 
@@ -157,9 +162,7 @@ static void matchBlock(const DescriptorView &v, const Tuning &tuning, const std:
     }
     // workgroups read the rows around their own
     if (sameBuffer(g.out, e.in0) || (g.in1.space != kSpaceNone && (sameBuffer(g.out, g.in1) || g.in1.offset % 16 != 0))) return;
-    const IrBlockArgs a = irBlockArgs(v, *s, [&](const DescRef &r) {
-        return r.space == kSpaceNone ? nullptr : (uint8_t *)(uintptr_t)(0x1000000 + (r.space == kSpaceConst ? v.consts[r.index].offset : 0) + r.offset);
-    });
+    const IrBlockArgs a = irBlockArgs(v, *s, [&](const DescRef &r) { return plannedAt(v, r); });
     if (tuning.irBlock >= 0 ? tuning.irBlock != 0 && irBlockFits(a) : irBlockBetter(a)) s->count = 3;
 }
 
@@ -173,13 +176,42 @@ static void matchBlock(const DescriptorView &v, const Tuning &tuning, const std:
 //   left    60x24 -> 64 5.4 / 3.2, 30000x72 -> 40 9.7 / 5.3, 100000x776 -> 64 44.0 / 39.0, 3x3 112x112x8 -> 32 6.3 / 4.3,
 //           stride 2 112x112x40 -> 32, batch 32 22.3 / 15.6, 1x1 stride 2 56x56x264 -> 96, batch 4 7.3 / 5.9
 //   wrong   30000x130 -> 40 11.2 / 9.5 (taken), 100000x500 -> 64 29.7 / 37.9, pointwise 56x56x24 -> 96, batch 32 9.6 / 14.4 (left)
-static bool paddingPays(const DescOp &g, int64_t rows, int64_t Cp, int64_t K) {
+static double gatherTime(const DescOp &g) {
     auto tilesOf = [](int64_t n) { return (double)((n + 63) / 64); };
     const double tiles = tilesOf(g.M) * tilesOf(g.Nn), beyond = tiles > 256 ? tiles - 256 : 0;
     const double step = g.gran >= 8 ? 0.55 : g.gran >= 4 ? 0.85 : g.gran >= 2 ? 1.5 : 2.5;
-    const double own = 2.8 + step * tilesOf(g.K) * (1 + beyond / 600);
+    return 2.8 + step * tilesOf(g.K) * (1 + beyond / 600);
+}
+static bool paddingPays(const DescOp &g, int64_t rows, int64_t Cp, int64_t K) {
+    auto tilesOf = [](int64_t n) { return (double)((n + 63) / 64); };
+    const double tiles = tilesOf(g.M) * tilesOf(g.Nn), beyond = tiles > 256 ? tiles - 256 : 0;
     const double padded = 5.1 + 0.24e-6 * (double)rows * (double)(g.C + Cp) + 0.09 * tilesOf(K) * (1 + beyond / 170);
-    return padded + 0.8 < own;
+    return padded + 0.8 < gatherTime(g);
+}
+
+// Whether igemm_direct_i8 takes the rows of the gathered record `g` as they are, as `op` (with its weights spread, or itself), and is ahead of its own
+// kernel.  It is ahead of the copy and a kernel behind it as well, by that launch: over the 153 of 170 drawn linears and convolutions of 5 .. 7848
+// channels that it takes, own kernel / copied rows / rows as they are cost 2.78 / 1.55 / 1.00 times the best (us: linear 9x100 -> 2303 5.5 / 6.4 / 4.0,
+// 554x604 -> 117 13.4 / 6.6 / 4.0, 5x1379 -> 48 57.4 / 6.4 / 4.5; 3x3 30x30x98 -> 316 stride 2, batch 3 7.1 / 6.6 / 4.0, 56x56x40 -> 32, batch 2 6.5 / 6.5 / 4.0; stride 2
+// 1x1 56x56x264 -> 96, batch 4 6.1 / 7.8 / 4.2).  Left where the gather is short (60x24 -> 64 3.6 / 6.1 / 3.8, 3x3 112x112x8 -> 32 4.5 / 6.7 / 4.1) and
+// where K is long enough for the worse loads to cost that launch: 3x5637 -> 567 224 / 8.3 / 9.0 (few rows have a faster kernel behind the copy), 5x5
+// 19x19x387 -> 134 452 / 18.2 / 19.7.
+static bool asIsBetter(const DescriptorView &v, const Tuning &tuning, const DescOp &g, const DescOp &op) {
+    if (tuning.padRows == 0 || tuning.padRows == 1 || g.kind != kKindIgemm || g.loader != kLoaderGather) return false;
+    return igemmDirectBetter(raggedArgs(v, op, g.C, [&](const DescRef &r) { return plannedAt(v, r); })) && (tuning.padRows == 2 || (gatherTime(g) > 4.0 && g.K <= (g.M <= kFcSkinnyMaxRows ? 5000 : 9000)));
+}
+
+// Whether the weights of a window of one pixel are zeros from K to the end of the last chunk that igemm_direct_i8 reads, as they are packed.
+static bool zerosBehindRows(const DescriptorView &v, const DescOp &op) {
+    const int64_t end = roundUp(op.K, 32);
+    if (op.weights.space != kSpaceConst || op.K != op.C || op.Kp < end) return false;
+    const uint8_t *w = v.blob + v.header.data_offset + v.consts[op.weights.index].offset + op.weights.offset;
+    for (int64_t n = 0; n < op.Nn; n++) {
+        for (int64_t k = op.K; k < end; k++) {
+            if (w[n * op.Kp + k] != 0) return false;
+        }
+    }
+    return true;
 }
 
 // A convolution, fully_connected or matmul over a channel count that is no multiple of 16.  Its own kernel gathers the
@@ -191,44 +223,54 @@ static bool matchPadded(const DescriptorView &v, const Tuning &tuning, uint32_t 
     const bool pointwise = g.KH == 1 && g.KW == 1 && g.SH == 1 && g.SW == 1 && g.PT == 0 && g.PL == 0 && g.OH == g.H && g.OW == g.W;
     const int64_t C = g.C, Cp = roundUp(C, 16), taps = (int64_t)g.KH * g.KW, rows = (int64_t)g.N * g.H * g.W, K = taps * Cp, N = g.Nn;
     if (g.K != taps * C || g.Kp < g.K || g.PT < 0 || g.PL < 0 || rows * Cp >= (1LL << 31) || K >= (1LL << 31)) return false;
-    if (tuning.padRows >= 0 ? tuning.padRows == 0 : !paddingPays(g, rows, Cp, K)) return false;
+    if (tuning.padRows == 0) return false;
     DescOp op = g;
     op.C = (int32_t)Cp;
     op.K = (int32_t)K;
     op.gran = 16;
-    int64_t Kp = Cp, Np = N;
-    if (pointwise && g.M <= kFcSkinnyMaxRows) {
-        op.kind = kKindFcSkinny;
-    } else {
-        uint32_t variant;
-        op.loader = pointwise ? kLoaderDense : kLoaderWindow;
-        if (thip_gemm_tile_choice((int32_t)op.loader, g.M, N, K, Cp, g.out_dtype, 0, &variant, nullptr, 0) != THIP_OK) return false;
-        if (variant == kIgemmStream && g.out.offset % 16 != 0) return false;  // it stores whole 16-byte pieces; the record's kernel any
-        const IgemmTile &t = igemmTile(variant);
-        Kp = roundUp(K, t.bk);
-        Np = roundUp(N, t.bn);
-        op.variant = variant;
-    }
+    op.loader = pointwise ? kLoaderDense : kLoaderWindow;
     // the (bias, scale) arrays were padded for the record's own tile
-    for (const DescRef *r : {&g.bias, &g.scale}) {
-        if (r->space != kSpaceConst || v.consts[r->index].size - r->offset < (uint64_t)Np * 4) return false;
+    auto padded = [&](int64_t Kp, int64_t Np) {
+        op.Kp = (int32_t)Kp;
+        op.Np = (int32_t)Np;
+        for (const DescRef *r : {&g.bias, &g.scale}) {
+            if (r->space != kSpaceConst || v.consts[r->index].size - r->offset < (uint64_t)Np * 4) return false;
+        }
+        return true;
+    };
+    // rows as they are: the weights of a window of one pixel serve without being spread (igemmRoute)
+    const bool pays = paddingPays(g, rows, Cp, K), asIs = (pays || taps > 1) && padded(roundUp(K, 32), roundUp(N, 32)) && asIsBetter(v, tuning, g, op);
+    if (!asIs) {
+        if (tuning.padRows == 2 || (tuning.padRows < 0 && !pays)) return false;
+        int64_t Kp = Cp, Np = N;
+        if (pointwise && g.M <= kFcSkinnyMaxRows) {
+            op.kind = kKindFcSkinny;
+            op.loader = g.loader;
+        } else {
+            uint32_t variant;
+            if (thip_gemm_tile_choice((int32_t)op.loader, g.M, N, K, Cp, g.out_dtype, 0, &variant, nullptr, 0) != THIP_OK) return false;
+            if (variant == kIgemmStream && g.out.offset % 16 != 0) return false;  // it stores whole 16-byte pieces; the record's kernel any
+            const IgemmTile &t = igemmTile(variant);
+            Kp = roundUp(K, t.bk);
+            Np = roundUp(N, t.bn);
+            op.variant = variant;
+        }
+        if (!padded(Kp, Np)) return false;
+        op.in0 = DescRef{kSpacePlan, 0, 0};
     }
-    op.Kp = (int32_t)Kp;
-    op.Np = (int32_t)Np;
-    const uint64_t weightBytes = (uint64_t)roundUp(Np * Kp, 256);
+    const uint64_t weightBytes = (uint64_t)roundUp((int64_t)op.Np * op.Kp, 256);
     s->constants.assign(weightBytes + 128, 0);
     const uint8_t *w = v.blob + v.header.data_offset + v.consts[g.weights.index].offset + g.weights.offset;
     for (int64_t n = 0; n < N; n++) {
-        for (int64_t tap = 0; tap < taps; tap++) memcpy(&s->constants[(size_t)(n * Kp + tap * Cp)], w + n * g.Kp + tap * C, (size_t)C);
+        for (int64_t tap = 0; tap < taps; tap++) memcpy(&s->constants[(size_t)(n * op.Kp + tap * Cp)], w + n * g.Kp + tap * C, (size_t)C);
     }
     memset(&s->constants[weightBytes], g.input_zp, 128);  // what a tap outside the image reads
-    op.in0 = DescRef{kSpacePlan, 0, 0};
     op.weights = DescRef{kSpacePlan, 1, 0};
     op.table = op.kind == kKindIgemm && op.loader == kLoaderWindow ? DescRef{kSpacePlan, 1, weightBytes} : DescRef{kSpaceNone, 0, 0};
     s->kind = kStepPadded;
     s->first = first;
     s->count = 1;
-    s->rows = rows;
+    s->rows = asIs ? 0 : rows;
     s->from = (int32_t)C;
     s->to = (int32_t)Cp;
     s->op = op;
@@ -433,10 +475,8 @@ static bool matchDecChain(const DescriptorView &v, const Tuning &tuning, uint32_
 
 // The kernel that is ahead for a GEMM-shaped record.
 static IgemmRoute igemmRoute(const DescriptorView &v, const Tuning &tuning, const DescOp &op) {
-    // addresses that are aligned as a dispatch's are
-    const IgemmArgs a = igemmArgs(v, op, [&](const DescRef &r) {
-        return r.space == kSpaceNone ? nullptr : (uint8_t *)(uintptr_t)(0x1000000 + (r.space == kSpaceConst ? v.consts[r.index].offset : 0) + r.offset);
-    });
+    const IgemmArgs a = igemmArgs(v, op, [&](const DescRef &r) { return plannedAt(v, r); });
+    if (op.loader == kLoaderGather && op.KH == 1 && op.KW == 1 && zerosBehindRows(v, op) && asIsBetter(v, tuning, op, op)) return kIgemmDirect;
     return igemmDirectBetter(a) ? kIgemmDirect : convPatchBetter(a) ? kIgemmPatch : !tuning.noK128 && igemmWideBetter(a, op.variant) ? kIgemmWide : kIgemmOwnTile;
 }
 
@@ -530,7 +570,7 @@ std::vector<Step> planSteps(const DescriptorView &v, const Tuning &tuning) {
         }
         if (s.kind == kStepExpandDw) matchBlock(v, tuning, uses, &s);
         const DescOp *op = s.kind == kStepRecord ? &v.ops[i] : s.kind == kStepPadded ? &s.op : nullptr;
-        s.route = !plain && op && op->kind == kKindIgemm ? igemmRoute(v, tuning, *op) : kIgemmOwnTile;
+        s.route = plain || !op || op->kind != kKindIgemm ? kIgemmOwnTile : s.kind == kStepPadded && s.rows == 0 ? kIgemmDirect : igemmRoute(v, tuning, *op);
         i += s.count;
         steps.push_back(std::move(s));
     }

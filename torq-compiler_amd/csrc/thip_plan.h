@@ -16,7 +16,7 @@ namespace thip {
 enum StepKind {
     kStepRecord,    // one record, by its own launcher
     kStepExpandDw,  // a pointwise convolution and the depthwise one behind it (ir_expand_dw_i8); three records: and the pointwise one behind that (ir_block_i8)
-    kStepPadded,    // a GEMM-shaped record whose channels fill no 16-byte chunks: its input padded, then a dense kernel
+    kStepPadded,    // a GEMM-shaped record whose channels fill no 16-byte chunks: its input padded, then a dense kernel; or its weights padded only
     kStepMatmulRt,  // a batch of int8 matmuls with a run-time input2: its transposes and its GEMMs (igemm_rt_i8)
     kStepDecChain,  // grouped linears and small matmuls of a decoder's step, each behind the one before it (dec_chain)
 };
@@ -39,8 +39,9 @@ struct Step {
     int32_t batches;
     int64_t a_stride, b_stride, out_stride;
     int32_t bias, scale;
-    // kStepPadded: rows of `from` bytes padded to `to`, and the record that reads them.  Its operands of space kSpacePlan are the
-    // step's own: index 0 the padded rows, index 1 `constants` (on the device).
+    // kStepPadded: rows of `from` bytes padded to `to`, and the record that reads them; no rows: a record that reads them as they are, its
+    // weights alone padded (igemm_direct_i8).  Its operands of space kSpacePlan are the step's own: index 0 the padded rows, index 1
+    // `constants` (on the device).
     int64_t rows;
     int32_t from, to;
     DescOp op;
@@ -81,6 +82,20 @@ IgemmArgs igemmArgs(const DescriptorView &v, const DescOp &op, At &&at) {
         a.add_w0 = ap.w0; a.add_w1 = ap.w1; a.add_bias = ap.bias; a.add_scale = ap.scale;
         a.arq = Requant{ap.shift, ap.output_zp, ap.output_min, ap.output_max, 0, 0};
     }
+    return a;
+}
+
+// The same for igemm_direct_i8 on a record whose input's pixels are of `channels` bytes, no whole 16-byte chunks.  Its weights have zeros
+// from there to the next whole chunk: those that a step has spread, and any of a window of one pixel.
+template <typename At>
+IgemmArgs raggedArgs(const DescriptorView &v, const DescOp &op, int32_t channels, At &&at) {
+    IgemmArgs a = igemmArgs(v, op, at);
+    const bool pointwise = op.KH == 1 && op.KW == 1 && op.SH == 1 && op.SW == 1 && op.PT == 0 && op.PL == 0 && op.OH == op.H && op.OW == op.W;
+    a.loader = pointwise ? kLoaderDense : kLoaderWindow;
+    a.row_bytes = channels;
+    a.C = (channels + 15) / 16 * 16;
+    a.K = op.KH * op.KW * a.C;
+    a.a_bytes = (int64_t)op.N * op.H * op.W * channels;
     return a;
 }
 
