@@ -194,8 +194,7 @@ bool igemmDirectBetter(const IgemmArgs &a) {
 template <bool WINDOW, int NW, int RAGGED>
 static hipError_t launchDirect(const IgemmArgs &a, const LaunchCtx &ctx) {
     const long long tiles = directTiles(a);
-    const std::string label = RAGGED ? kernelLabel("igemm_direct_i8", {(int)WINDOW, NW, RAGGED}) : kernelLabel("igemm_direct_i8", {(int)WINDOW, NW});
-    THIP_ENQUEUE(ctx, label, (igemm_direct_i8<WINDOW, NW, RAGGED>), dim3((unsigned)tiles), dim3(NW * 64), 0, a,
+    THIP_ENQUEUE(ctx, (RAGGED ? kernelLabel("igemm_direct_i8", {(int)WINDOW, NW, RAGGED}) : kernelLabel("igemm_direct_i8", {(int)WINDOW, NW})), (igemm_direct_i8<WINDOW, NW, RAGGED>), dim3((unsigned)tiles), dim3(NW * 64), 0, a,
                  makeFastDiv((uint32_t)(WINDOW ? a.C : 1)), makeFastDiv((uint32_t)(WINDOW ? a.KW : 1)), makeFastDiv((uint32_t)(WINDOW ? a.OH * a.OW : 1)),
                  makeFastDiv((uint32_t)(WINDOW ? a.OW : 1)));
     return hipGetLastError();
