@@ -51,13 +51,13 @@ constexpr int kDecLdsSlot = 2048 + 128;  // a k-block's weights, scales and (roo
 
 // MR: groups of 16 input rows (1 or 2).  XLDS: the input rows come through LDS as well (at most four rows): then every
 // global load of a wave is an LDS-DMA load issued up front and each k-block is computed as soon as it has landed.
-// Otherwise the rows come through registers, CH k-blocks at a time, two such chunks in flight.  QB: the slots carry block biases.
+// Otherwise the rows come through registers, CH k-blocks at a time, two such chunks in flight, or (ONE) the one that a wave has at most.  QB: the slots carry block biases.
 // QC: the expansion clamps.
 // S (XLDS only): the 16-column tile is shared out over S workgroups of CW = 16 / S columns, each an MFMA's row operand made of S
 // k-blocks of its columns: operand row c holds column c % CW of k-block c / CW and input column c holds input row c % CW of k-block
 // c / CW, so of the 16 x 16 products the S blocks on the diagonal are wanted; their sum is the result.  The lanes, loads and expansions of
 // a workgroup are as full as with one k-block, of which it has S times fewer.
-template <int MR, int CH, bool XLDS, bool QB, bool QC, int S>
+template <int MR, int CH, bool XLDS, bool QB, bool QC, int S, bool ONE>
 __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p) {
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
     const int lane = threadIdx.x & 63;
@@ -87,8 +87,8 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
     const int nmat = p.pair ? 2 : 1;
     const int kblocks = p.K >> 7;  // K % 128 == 0
     const int units = (kblocks + S - 1) / S;  // S k-blocks each
-    const int nkb = wave < units ? (units - wave + NW - 1) / NW : 0;
-    const int maxkb = (units + NW - 1) / NW;
+    const int nkb = wave >= units ? 0 : ONE ? 1 : (units - wave + NW - 1) / NW;
+    const int maxkb = ONE ? 1 : (units + NW - 1) / NW;
     const int slotBytes = kDecSlotBytes + (QB ? 64 : 0);
     const int xRowBytes = XLDS ? M * S * 256 : 0;  // a unit of the input rows in LDS
     const unsigned regionBytes = (unsigned)maxkb * (unsigned)(xRowBytes + nmat * kDecLdsSlot);
@@ -188,8 +188,9 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
             if (nmat > 1) kblock(i, 1, xp);
         }
     } else {
+        constexpr int UN = ONE ? 1 : CH;
         struct XBuf {
-            v4i x[CH][4][MR];
+            v4i x[UN][4][MR];
         };
         // A load brings 64 bytes of each of 16 rows: half a line each where rows lie one behind the other, and a wave's second half only hits
         // while the first is in its CU's 32 KB cache, among the loads of 15 other waves.  Block by block it is 1 KB of whole lines.
@@ -202,8 +203,8 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
         // Loads only; a k-block the wave does not have and a row beyond M read nothing and feed zeros.
         auto loadChunk = [&](int ch, XBuf &b) {
 #pragma unroll
-            for (int u = 0; u < CH; u++) {
-                const int i = ch * CH + u;
+            for (int u = 0; u < UN; u++) {
+                const int i = ch * UN + u;
                 const int kb = wave + NW * i;
 #pragma unroll
                 for (int mr = 0; mr < MR; mr++) {
@@ -216,24 +217,30 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
         };
         auto computeChunk = [&](int ch, const XBuf &b) {
 #pragma unroll
-            for (int u = 0; u < CH; u++) {
-                const int i = ch * CH + u;
+            for (int u = 0; u < UN; u++) {
+                const int i = ch * UN + u;
                 if (i >= nkb) break;
                 kblock(i, 0, b.x[u]);
                 if (nmat > 1) kblock(i, 1, b.x[u]);
             }
         };
-        const int nchunks = (nkb + CH - 1) / CH;
-        XBuf b0, b1;
+        const int nchunks = (nkb + UN - 1) / UN;
+        XBuf b0;
         loadChunk(0, b0);
-        if (nchunks > 1) loadChunk(1, b1);
-        waitVmcnt<0>();  // the DMA burst (and the rows of two chunks) has landed; the compiler counts only its own loads
-        for (int ch = 0; ch < nchunks; ch += 2) {
-            computeChunk(ch, b0);
-            if (ch + 2 < nchunks) loadChunk(ch + 2, b0);
-            if (ch + 1 < nchunks) {
-                computeChunk(ch + 1, b1);
-                if (ch + 3 < nchunks) loadChunk(ch + 3, b1);
+        if constexpr (ONE) {
+            waitVmcnt<0>();
+            computeChunk(0, b0);
+        } else {
+            XBuf b1;
+            if (nchunks > 1) loadChunk(1, b1);
+            waitVmcnt<0>();  // the DMA burst (and the rows of two chunks) has landed; the compiler counts only its own loads
+            for (int ch = 0; ch < nchunks; ch += 2) {
+                computeChunk(ch, b0);
+                if (ch + 2 < nchunks) loadChunk(ch + 2, b0);
+                if (ch + 1 < nchunks) {
+                    computeChunk(ch + 1, b1);
+                    if (ch + 3 < nchunks) loadChunk(ch + 3, b1);
+                }
             }
         }
     }
@@ -310,15 +317,16 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
     *(v2i *)(p.add_out + decResultAt(p.blocked & kDecBlockedAdd, p.M, row, n, Nseg)) = v2i{(int)((uint32_t)z[0] | ((uint32_t)z[1] << 16)), (int)((uint32_t)z[2] | ((uint32_t)z[3] << 16))};
 }
 
-template <int MR, int CH, bool XLDS, bool QB, bool QC, int S = 1>
+template <int MR, int CH, bool XLDS, bool QB, bool QC, int S = 1, bool ONE = false>
 static hipError_t launchDecLinearT(const DecLinearArgs &a, int tiles, size_t lds, const LaunchCtx &ctx) {
-    auto kernel = dec_linear<MR, CH, XLDS, QB, QC, S>;
+    auto kernel = dec_linear<MR, CH, XLDS, QB, QC, S, ONE>;
     static std::once_flag once;
     static hipError_t configured = hipSuccess;
     std::call_once(once, [&] { configured = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); });
     if (configured != hipSuccess) return configured;
     const int groups = (a.M + a.rows_per_group - 1) / a.rows_per_group;
-    THIP_ENQUEUE(ctx, kernelLabel("dec_linear", {MR, CH, (int)XLDS, (int)QB, (int)QC, a.pair ? 2 : a.nseg, a.add_mode, S}), kernel, dim3((unsigned)tiles * S, (unsigned)groups),
+    THIP_ENQUEUE(ctx, (ONE ? kernelLabel("dec_linear", {MR, CH, (int)XLDS, (int)QB, (int)QC, a.pair ? 2 : a.nseg, a.add_mode, S, 1}) : kernelLabel("dec_linear", {MR, CH, (int)XLDS, (int)QB, (int)QC, a.pair ? 2 : a.nseg, a.add_mode, S})),
+                 kernel, dim3((unsigned)tiles * S, (unsigned)groups),
                  dim3((unsigned)a.nwaves * 64), lds, a);
     return hipGetLastError();
 }
@@ -381,11 +389,16 @@ static hipError_t launchDecLinearQ(const DecLinearArgs &in, int tiles, const Lau
     }
     const int groups = decLinearRowGroups(a.M, tiles, ctx.tuning);
     a.rows_per_group = (a.M + groups - 1) / groups;
-    // more workgroups than CUs: eight waves each, so that two of them (at four waves per SIMD) share a CU and the
-    // launch is one round of workgroups rather than two (decoder step at 32 tokens 1247 -> 1216 us, at 8 1028 -> 994)
-    if ((long long)tiles * groups > 256 && a.nwaves > kDecWaves) a.nwaves = kDecWaves;
+    // A wave of one k-block holds the rows of that one only (64 registers at most): two workgroups of 16 such waves share a CU.  Where K has more k-blocks
+    // than waves and the launch more workgroups than CUs, eight waves each, so that two of them (at four waves per SIMD) share one and the launch is
+    // one round of workgroups rather than two.  Steps of four layers, us, always eight / this: hidden 1152 at 32 rows 165.6 / 160.7, at 8 129.1 / 123.8;
+    // 1536 at 16 rows 134.1 / 130.0, at 32 155.4 / 148.7; 2048 at 20 rows 167.2 / 160.0 (with more than 12 such waves left at eight 164.7), at 12 157.2 / 147.5; 768 at 24 rows
+    // 107.6 / 103.8 (the registers alone).
+    const bool few = a.rows_per_group <= 16;
+    if ((long long)tiles * groups > 256 && a.nwaves < a.K / 128) a.nwaves = kDecWaves;
     const size_t lds = decLinearLds(a.K, nmat, 0, a.nwaves);
-    if (a.rows_per_group <= 16) return launchDecLinearT<1, 2, false, QB, QC>(a, tiles, lds, ctx);
+    if (a.nwaves >= a.K / 128) return few ? launchDecLinearT<1, 2, false, QB, QC, 1, true>(a, tiles, lds, ctx) : launchDecLinearT<2, 1, false, QB, QC, 1, true>(a, tiles, lds, ctx);
+    if (few) return launchDecLinearT<1, 2, false, QB, QC>(a, tiles, lds, ctx);
     return launchDecLinearT<2, 1, false, QB, QC>(a, tiles, lds, ctx);
 }
 
