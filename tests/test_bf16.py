@@ -289,6 +289,22 @@ def test_gpu_bf16_wide_n(device):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K,N,M", [(64, 32768 * 5 + 33, 1), (128, 32768 * 9 + 1, 3), (192, 32768 * 4 + 63, 33), (512, 32768 * 5, 40)])
+@pytest.mark.parametrize("scaled", [False, True])
+def test_gpu_bf16_wide_n_rounds(device, K, N, M, scaled):
+    """More columns than the chip's blocks make at a time: waves with one set of columns more than others, an odd and an even number of
+    loads per set, one of fewer steps than a load takes; rows of a last block that is not full."""
+    wl = w.expand_weights_workload(M=M, K=K, N=N, block=64) if scaled else w.fully_connected_bf16_workload(M, K, N, clamp=(-0.5, 0.75) if M == 3 else None)
+    print("[gpu-case]", wl.name, flush=True)
+    got, kernels = run_on_gpu(device, wl, via="device")
+    assert families(kernels) == ["fc_bf16_wide"], kernels
+    f = lambda bits: np.abs(orc.from_bf16(bits).astype(np.float64))
+    w16 = orc.expand_weights(wl.attrs["weights"], wl.attrs["scale"], wl.attrs["qbias"], block_size=64, output_min=wl.attrs["expand_min"], output_max=wl.attrs["expand_max"]) if scaled else wl.attrs["weights"]
+    magnitude = f(wl.inputs[0]) @ (f(w16) if f(w16).shape[0] == K else f(w16).T)
+    assert_bf16_close(got[0], oracle_eval(wl)[0].reshape(got[0].shape), wl.name + " (gpu)", magnitude=magnitude)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("waves", [4, 8, 16])
 def test_gpu_bf16_wide_n_waves_per_block(device, waves, monkeypatch):
     """The waves of a block share its input rows in LDS: four, eight or sixteen of them, every one with columns of its

@@ -22,15 +22,14 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 // Bias, clamp, round to bf16 and store one 32 x 32 accumulator tile: register 4 q + e of lane (r, h) is
 // out[m0 + r][n0 + 8 q + 4 h + e].  fcBf16StoreQuad stores the four registers of one q, at any alignment (14 x 1000 -> 521: 6.5 us in
 // single elements, 6.3).
-__device__ __forceinline__ void fcBf16StoreQuad(const FcBf16Args &p, const float (&a)[4], int m0, int n0, int r, int h, int q) {
+__device__ __forceinline__ void fcBf16StoreQuad(const FcBf16Args &p, const float (&a)[4], const float (&bias)[4], int m0, int n0, int r, int h, int q) {
     const int m = m0 + r;
     if (m >= p.M) return;
     const int n = n0 + 8 * q + 4 * h;
     uint16_t o[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-        const int ne = n + e < p.N ? n + e : p.N - 1;
-        const float t0 = a[e] + p.bias[ne];
+        const float t0 = a[e] + bias[e];
         o[e] = bf16Bits(t0 < p.lo ? p.lo : (t0 > p.hi ? p.hi : t0));
     }
     if (n + 3 < p.N) {
@@ -41,6 +40,13 @@ __device__ __forceinline__ void fcBf16StoreQuad(const FcBf16Args &p, const float
             if (n + e < p.N) p.out[(size_t)m * p.N + n + e] = o[e];
         }
     }
+}
+__device__ __forceinline__ void fcBf16StoreQuad(const FcBf16Args &p, const float (&a)[4], int m0, int n0, int r, int h, int q) {
+    const int n = n0 + 8 * q + 4 * h;
+    float bias[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) bias[e] = p.bias[n + e < p.N ? n + e : p.N - 1];
+    fcBf16StoreQuad(p, a, bias, m0, n0, r, h, q);
 }
 __device__ __forceinline__ void fcBf16Store(const FcBf16Args &p, const v16f &acc, int m0, int n0, int r, int h) {
 #pragma unroll
@@ -175,44 +181,44 @@ __global__ __launch_bounds__(256) void fc_bf16_reduce(FcBf16Args p) {
 // register buffers, the loads of one in flight while the other feeds the MFMAs.  The input rows of the block
 // (at most 32, and one slot of zeros for the lanes of rows it does not have) sit in LDS in fragment order, read
 // 16 bytes per lane right before each MFMA: with few rows that is a few KiB, and registers set the occupancy.
+// The blocks that the chip holds at once stay for all columns: the rows come to LDS once, under the first weights' loads, and the next column
+// block's first weights are under way while one is finished, its bias among its own weights (waited for by itself it waits behind the next ones').
+// K = 1152, us, a block per columns / this: 262144 columns of block-scaled int8 weights 66.0 / 59.4 for one row and 89.5 / 77 for 32, 65536 columns 20.6 / 18.5 and
+// 24.8 / 23.0, bf16 weights 26.7 / 22.9 and 29.5 / 26.0; 100000 columns of K = 512, 40 rows 39.2 / 23.1.
 // Weights in fragment order only (layouts 1 and 2).
 constexpr int kFcBf16WideMaxSteps = 24;  // 99 KiB of LDS for 32 input rows
 template <int Q8, int U, int W = 4>  // U: k-steps per register buffer; W: waves per block (they share the block's input rows in LDS)
-__global__ __launch_bounds__(64 * W) void fc_bf16_wide(FcBf16Args p, FastDiv qblk) {
+__global__ __launch_bounds__(64 * W) void fc_bf16_wide(FcBf16Args p, FastDiv qblk, FastDiv divSlots) {
     extern __shared__ __attribute__((aligned(16))) int8_t xs[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = lane & 31, h = lane >> 5;
     const int steps = (p.K + 63) / 64;
     const int m0 = blockIdx.y * 32;
-    // rows the block really has, plus one slot of zeros that the lanes of the missing rows all read
-    const int mt = p.M - m0 < 32 ? p.M - m0 : 32, slots = 2 * (mt + 1);
-    for (int i = threadIdx.x; i < steps * 4 * slots; i += 64 * W) {
-        const int slot = i % slots, sc = i / slots, c = sc & 3, s = sc >> 2;
-        const int hh = slot / (mt + 1), rr = slot - hh * (mt + 1);
-        const int k = s * 64 + 32 * hh + 8 * c;
-        v4i v = {0, 0, 0, 0};
-        if (rr < mt && k < p.K) v = *(const v4i *)(p.x + (size_t)(m0 + rr) * p.K + k);
-        *(v4i *)(xs + (size_t)i * 16) = v;
-    }
-    __syncthreads();
+    // as many rows as a block has (the last one's missing ones are zeros), plus one slot of zeros that the lanes of further rows all read
+    const int mt = p.M < 32 ? p.M : 32, slots = 2 * (mt + 1);
     const int xslot = (h * (mt + 1) + (r < mt ? r : mt)) * 16;
-    const int nb = blockIdx.x * W + wave;
-    if (nb >= (p.N + 31) / 32) return;
-    const int n0 = nb * 32;
+    const int blocks = (p.N + 31) / 32, stride = (int)gridDim.x * W;
     constexpr int PIECES = Q8 ? 2 : 4;  // 16-byte loads per lane per step
-    const int8_t *wbase = (const int8_t *)p.w + (size_t)nb * steps * (PIECES * 1024) + lane * 16;
     struct Buf {
         v4i w[U][PIECES];
         uint16_t qs[U];  // raw bf16 bits: converting here would wait for the load, and with it for every older one
         float qb[U];
+        float bias;  // of column r
     };
-    // Loads only, no use of a loaded value and no branch: the steps past the end re-read the last one (never used).
-    auto loadGroup = [&](int s0, Buf &b) {
+    struct Cursor {  // U steps of a column block
+        int nb, s0;
+    };
+    auto behind = [&](Cursor at) { return at.s0 + U < steps ? Cursor{at.nb, at.s0 + U} : Cursor{at.nb + stride, 0}; };
+    // Loads only, no use of a loaded value and no branch: steps past the end re-read the last one, blocks past it the last block (never used).
+    auto loadGroup = [&](Cursor at, Buf &b) {
+        const int nb = at.nb < blocks ? at.nb : blocks - 1, n0 = nb * 32;
+        const int8_t *wbase = (const int8_t *)p.w + (size_t)nb * steps * (PIECES * 1024);
+        b.bias = p.bias[n0 + r < p.N ? n0 + r : p.N - 1];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int s = s0 + u < steps ? s0 + u : steps - 1;
+            const int s = at.s0 + u < steps ? at.s0 + u : steps - 1;
 #pragma unroll
-            for (int c = 0; c < PIECES; c++) b.w[u][c] = *(const v4i *)(wbase + ((size_t)s * PIECES + c) * 1024);
+            for (int c = 0; c < PIECES; c++) b.w[u][c] = *(const v4i *)(wbase + ((size_t)s * PIECES + c) * 1024 + lane * 16);
             if (Q8) {
                 const int k = s * 64 + 32 * h;
                 const size_t g = fastDiv((uint32_t)(k < p.K ? k : 0), qblk);  // beyond K the input rows are zero
@@ -221,13 +227,26 @@ __global__ __launch_bounds__(64 * W) void fc_bf16_wide(FcBf16Args p, FastDiv qbl
             }
         }
     };
+    Cursor at{(int)blockIdx.x * W + __builtin_amdgcn_readfirstlane(wave), 0};
+    Buf b0, b1;
+    loadGroup(at, b0);
+    for (int i = threadIdx.x; i < steps * 4 * slots; i += 64 * W) {
+        const int sc = (int)fastDiv((uint32_t)i, divSlots), slot = i - sc * slots, c = sc & 3, s = sc >> 2;
+        const int hh = slot > mt, rr = slot - hh * (mt + 1);
+        const int k = s * 64 + 32 * hh + 8 * c;
+        v4i v = {0, 0, 0, 0};
+        if (rr < mt && m0 + rr < p.M && k < p.K) v = *(const v4i *)(p.x + (size_t)(m0 + rr) * p.K + k);
+        *(v4i *)(xs + (size_t)i * 16) = v;
+    }
+    __syncthreads();
+    if (at.nb >= blocks) return;
     v16f acc;
 #pragma unroll
     for (int e = 0; e < 16; e++) acc[e] = 0.0f;
-    auto compute = [&](int s0, const Buf &b) {
+    auto compute = [&](Cursor at, const Buf &b) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int s = s0 + u;
+            const int s = at.s0 + u;
             if (s >= steps) break;
 #pragma unroll
             for (int c = 0; c < 4; c++) {
@@ -246,15 +265,32 @@ __global__ __launch_bounds__(64 * W) void fc_bf16_wide(FcBf16Args p, FastDiv qbl
             }
         }
     };
-    Buf b0, b1;
-    loadGroup(0, b0);
-    for (int s0 = 0; s0 < steps; s0 += 2 * U) {
-        loadGroup(s0 + U, b1);
-        compute(s0, b0);
-        loadGroup(s0 + 2 * U, b0);
-        compute(s0 + U, b1);
+    // (the bias comes with the weights: a load of its own here would be waited for behind the next group's)
+    auto finish = [&](Cursor at, const Buf &b) {
+        if (at.s0 + U < steps) return;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            float bias[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) bias[e] = __shfl(b.bias, 8 * q + 4 * h + e);
+            const float a[4] = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+            fcBf16StoreQuad(p, a, bias, m0, at.nb * 32, r, h, q);
+        }
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[e] = 0.0f;
+    };
+    for (;;) {
+        const Cursor second = behind(at);
+        loadGroup(second, b1);
+        compute(at, b0);
+        finish(at, b0);
+        if (second.nb >= blocks) break;
+        at = behind(second);
+        loadGroup(at, b0);
+        compute(second, b1);
+        finish(second, b1);
+        if (at.nb >= blocks) break;
     }
-    fcBf16Store(p, acc, m0, n0, r, h);
 }
 
 template <int Q8, int U, int W>
@@ -265,19 +301,21 @@ static hipError_t launchFcBf16WideUW(const FcBf16Args &a, FastDiv blk, const Lau
     std::call_once(once, [&] { configured = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kFcBf16WideMaxSteps * 4 * 66 * 16); });
     if (configured != hipSuccess) return configured;
     const int steps = (a.K + 63) / 64, nblocks = (a.N + 31) / 32;
-    const dim3 grid((unsigned)((nblocks + W - 1) / W), (unsigned)((a.M + 31) / 32));
-    const int mt = a.M < 32 ? a.M : 32;
-    THIP_ENQUEUE(ctx, kernelLabel("fc_bf16_wide", {Q8, U, W}), kernel, grid, dim3(64 * W), (size_t)steps * 4 * 2 * (mt + 1) * 16, a, blk);
+    const int mt = a.M < 32 ? a.M : 32, slots = 2 * (mt + 1), rowBlocks = (a.M + 31) / 32;
+    const size_t lds = (size_t)steps * 4 * slots * 16;
+    // as many blocks as the chip holds (16 waves a CU)
+    const int perCu = std::max(1, std::min(16 / W, (int)(160 * 1024 / lds))), most = std::max(1, 256 * perCu / rowBlocks);
+    const dim3 grid((unsigned)std::min((nblocks + W - 1) / W, most), (unsigned)rowBlocks);
+    THIP_ENQUEUE(ctx, kernelLabel("fc_bf16_wide", {Q8, U, W}), kernel, grid, dim3(64 * W), lds, a, blk, makeFastDiv((uint32_t)slots));
     return hipGetLastError();
 }
 
 template <int Q8, int U>
 static hipError_t launchFcBf16WideU(const FcBf16Args &a, FastDiv blk, const LaunchCtx &ctx) {
     // Waves per block: they share one copy of the block's input rows in LDS (up to 99 KiB, read from L2 once per block),
-    // so more waves mean fewer copies and more waves per CU.  Measured at K = 1152, N = 65536, 1 / 32 / 64 rows, in us:
-    // bf16 weights 26.3 / 34.4 / 64.8 with four waves, 26.0 / 30.3 / 53.0 with eight, 26.6 / 29.3 / 30.2 with sixteen;
-    // block-scaled int8 weights 19.7 / 27.6 / 50.4, 19.4 / 23.5 / 34.3 and 23.9 / 26.2 / 28.6 (one block of sixteen
-    // waves per CU: its prologue overlaps with nothing).  THIP_FC_WIDE_WAVES forces a count.
+    // so more waves mean fewer copies and more waves per CU.  Measured at K = 1152, N = 65536, 1 / 32 / 64 rows, in us, blocks that made one set
+    // of columns each: bf16 weights 26.3 / 34.4 / 64.8 with four waves, 26.0 / 30.3 / 53.0 with eight, 26.6 / 29.3 / 30.2 with sixteen;
+    // block-scaled int8 weights 19.7 / 27.6 / 50.4, 19.4 / 23.5 / 34.3 and 23.9 / 26.2 / 28.6.  THIP_FC_WIDE_WAVES forces a count.
     constexpr bool fitsSixteen = U <= (Q8 ? 4 : 2);  // beyond that 128 registers per lane are not enough
     int waves = ctx.tuning->fcWideWaves;
     if (waves != 4 && waves != 8 && waves != 16) waves = (!Q8 || a.M > 32) ? 16 : 8;
