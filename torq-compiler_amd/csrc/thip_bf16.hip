@@ -41,18 +41,15 @@ __device__ __forceinline__ void fcBf16StoreQuad(const FcBf16Args &p, const float
         }
     }
 }
-__device__ __forceinline__ void fcBf16StoreQuad(const FcBf16Args &p, const float (&a)[4], int m0, int n0, int r, int h, int q) {
-    const int n = n0 + 8 * q + 4 * h;
-    float bias[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) bias[e] = p.bias[n + e < p.N ? n + e : p.N - 1];
-    fcBf16StoreQuad(p, a, bias, m0, n0, r, h, q);
-}
-__device__ __forceinline__ void fcBf16Store(const FcBf16Args &p, const v16f &acc, int m0, int n0, int r, int h) {
+// All of it; `bias`: column r's.
+__device__ __forceinline__ void fcBf16Store(const FcBf16Args &p, const v16f &acc, float bias, int m0, int n0, int r, int h) {
 #pragma unroll
     for (int q = 0; q < 4; q++) {
+        float b[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) b[e] = __shfl(bias, 8 * q + 4 * h + e);
         const float a[4] = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-        fcBf16StoreQuad(p, a, m0, n0, r, h, q);
+        fcBf16StoreQuad(p, a, b, m0, n0, r, h, q);
     }
 }
 
@@ -66,6 +63,7 @@ __global__ __launch_bounds__(NWAVES * 64) void fc_bf16(FcBf16Args p, FastDiv qbl
     const int n0 = blockIdx.x * 32, m0 = blockIdx.y * 32;
     const int nrow = n0 + r < p.N ? n0 + r : p.N - 1;  // clamped rows are never stored
     const int mrow = m0 + r < p.M ? m0 + r : p.M - 1;
+    const float bias = p.bias[nrow];  // asked for with the operands: when the sums are there, it is waited for (15 x 184 -> 1008 6.2 us, 5.5)
     const uint16_t *wrow = p.w + (size_t)nrow * p.K;
     const uint16_t *xrow = p.x + (size_t)mrow * p.K;
     // this block's slice of K (blockIdx.z of ksplit), then this wave's share of the slice
@@ -150,7 +148,7 @@ __global__ __launch_bounds__(NWAVES * 64) void fc_bf16(FcBf16Args p, FastDiv qbl
         for (int e = 0; e < 16; e++) mine[e * 64 + lane] = acc[e];
         return;
     }
-    fcBf16Store(p, acc, m0, n0, r, h);
+    fcBf16Store(p, acc, bias, m0, n0, r, h);
 }
 
 // Second kernel of a K split: a block per output tile adds the slices' partial tiles in slice order and finishes the
@@ -160,7 +158,10 @@ __global__ __launch_bounds__(256) void fc_bf16_reduce(FcBf16Args p) {
     const int lane = threadIdx.x & 63, q = threadIdx.x >> 6, r = lane & 31, h = lane >> 5;
     const int tile = blockIdx.y * gridDim.x + blockIdx.x;
     const float *parts = (const float *)p.workspace + (size_t)tile * p.ksplit * 1024 + (size_t)(4 * q) * 64 + lane;
-    float v[16][4];
+    const int n0 = blockIdx.x * 32;
+    float bias[4], v[16][4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) bias[e] = p.bias[n0 + 8 * q + 4 * h + e < p.N ? n0 + 8 * q + 4 * h + e : p.N - 1];
 #pragma unroll
     for (int z = 0; z < 16; z++) {
         const int zc = z < p.ksplit ? z : p.ksplit - 1;  // loads only, no branch: slices past the split re-read the last one
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(256) void fc_bf16_reduce(FcBf16Args p) {
 #pragma unroll
         for (int e = 0; e < 4; e++) a[e] += z < p.ksplit ? v[z][e] : 0.0f;
     }
-    fcBf16StoreQuad(p, a, blockIdx.y * 32, blockIdx.x * 32, r, h, q);
+    fcBf16StoreQuad(p, a, bias, blockIdx.y * 32, n0, r, h, q);
 }
 
 // fc_bf16_wide: the same product for a very wide N and a short K (a vocabulary projection): a wave owns a
@@ -268,14 +269,7 @@ __global__ __launch_bounds__(64 * W) void fc_bf16_wide(FcBf16Args p, FastDiv qbl
     // (the bias comes with the weights: a load of its own here would be waited for behind the next group's)
     auto finish = [&](Cursor at, const Buf &b) {
         if (at.s0 + U < steps) return;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            float bias[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) bias[e] = __shfl(b.bias, 8 * q + 4 * h + e);
-            const float a[4] = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-            fcBf16StoreQuad(p, a, bias, m0, at.nb * 32, r, h, q);
-        }
+        fcBf16Store(p, acc, b.bias, m0, at.nb * 32, r, h);
 #pragma unroll
         for (int e = 0; e < 16; e++) acc[e] = 0.0f;
     };

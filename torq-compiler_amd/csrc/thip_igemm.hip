@@ -1412,6 +1412,9 @@ __global__ __launch_bounds__(256) void fc_skinny(FcSkinnyArgs p) {
     const int wave = (int)((blockIdx.x * 256 + threadIdx.x) >> 6);
     const int n0 = wave * NW;
     if (n0 >= p.N) return;
+    // lane j finishes column j; what it needs for that comes with the operands (by one lane, asked for at the end: 1x2048 -> 2048 3.7 us, 3.0, by itself)
+    const int own = n0 + (lane < NW ? lane : 0), param = own < p.N ? own : p.N - 1;
+    const int32_t bias = p.bias[param], scale = p.scale[param];
     int32_t acc[MR][NW];
 #pragma unroll
     for (int m = 0; m < MR; m++) {
@@ -1450,22 +1453,15 @@ __global__ __launch_bounds__(256) void fc_skinny(FcSkinnyArgs p) {
             acc[m][j] = v;
         }
     }
-    if (lane == 0) {
-        const long long rnd = roundTerm(p.rq.shift);
+    if (own >= p.N || lane >= NW) return;
+    const long long rnd = roundTerm(p.rq.shift);
 #pragma unroll
-        for (int j = 0; j < NW; j++) {
-            const int n = n0 + j;
-            if (n < p.N) {
-                const int32_t bias = p.bias[n], scale = p.scale[n];
+    for (int m = 0; m < MR; m++) {
+        if (m >= p.M) break;
+        int32_t v = acc[m][0];
 #pragma unroll
-                for (int m = 0; m < MR; m++) {
-                    if (m < p.M) {
-                        storeElem(p.out, (size_t)m * p.N + n, requant(acc[m][j], bias, scale, rnd, p.rq),
-                                  p.out_dtype);
-                    }
-                }
-            }
-        }
+        for (int j = 1; j < NW; j++) v = lane == j ? acc[m][j] : v;
+        storeElem(p.out, (size_t)m * p.N + own, requant(v, bias, scale, rnd, p.rq), p.out_dtype);
     }
 }
 
