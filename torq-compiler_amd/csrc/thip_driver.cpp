@@ -607,7 +607,7 @@ static bool tellsRecords(const thip_executable_t *e) { return e->device->eventLo
 // Enqueues every kernel of the program.  `bp` holds one device pointer per binding.
 static thip_status_t enqueueOps(thip_executable_t *e, uint8_t *const *bp, bool apart = false) {
     if (!tellsRecords(e)) {
-        const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0};
+        const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0, e->device->ordinal};
         for (const Step &s : e->steps) {
             if (thip_status_t st = launchStep(e, s, bp, ctx, nullptr, apart)) return st;
         }
@@ -616,7 +616,7 @@ static thip_status_t enqueueOps(thip_executable_t *e, uint8_t *const *bp, bool a
     for (uint32_t i = 0; i < e->header.op_count; i++) {
         // a kernel launch is what starting an NSS task is on the reference's hardware
         logEvent(e, e->invocation, (int32_t)i, "NSS_START", "BEGIN", e->kernelNames[i].c_str());
-        if (thip_status_t s = launchOp(e, i, e->ops[i], bp, LaunchCtx{e->stream, &e->tuning, nullptr, 0})) return s;
+        if (thip_status_t s = launchOp(e, i, e->ops[i], bp, LaunchCtx{e->stream, &e->tuning, nullptr, 0, e->device->ordinal})) return s;
         logEvent(e, e->invocation, (int32_t)i, "NSS_START", "END", e->kernelNames[i].c_str());
         if (!e->device->dumpBuffersDir.empty()) {
             // buffer dumps: each record runs to its end and what it wrote is read back before the next one starts
@@ -966,7 +966,7 @@ static bool addStep(thip_executable_t *e, Step &&planned) {
         uint8_t *placeholder[64];
         for (auto &ptr : placeholder) ptr = (uint8_t *)(uintptr_t)0x1000000;
         char name[96] = "";
-        if (launchStep(e, step, placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name)}) == THIP_OK) {
+        if (launchStep(e, step, placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name), e->device->ordinal}) == THIP_OK) {
             if (step.kind == kStepPadded && step.rows > 0) e->launchNames.push_back("pad_rows_i8");
             e->launchNames.push_back(name[0] ? name : opKernelName(e->ops[step.first]));
             return true;
@@ -1050,7 +1050,7 @@ thip_status_t thip_executable_create(thip_device_t *device, const void *blob, si
         for (auto &ptr : placeholder) ptr = (uint8_t *)(uintptr_t)0x1000000;
         for (uint32_t i = 0; i < h.op_count; i++) {
             char name[96] = "";
-            if (thip_status_t st = launchOp(e, i, e->ops[i], placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name)})) return bail(st);
+            if (thip_status_t st = launchOp(e, i, e->ops[i], placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name), e->device->ordinal})) return bail(st);
             e->kernelNames[i] = name[0] ? name : opKernelName(e->ops[i]);
         }
     }
@@ -1282,7 +1282,7 @@ thip_status_t thip_executable_enqueue_noalloc(thip_executable_t *e, const thip_d
     if (!scratch) return fail(THIP_INTERNAL, "the static scratch array was not located");
     uint8_t *bp[64] = {nullptr};
     for (uint32_t i = 0; i < e->header.binding_count; i++) bp[i] = (uint8_t *)st->binding_ptrs[i];
-    const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0};
+    const LaunchCtx ctx{e->stream, &e->tuning, nullptr, 0, e->device->ordinal};
     ChainTurns::Turn turn;
     bool apart;
     thip_status_t result = takeTurn(e, bp, &turn, false, &apart);

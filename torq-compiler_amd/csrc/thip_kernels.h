@@ -82,6 +82,7 @@ struct LaunchCtx {
     const Tuning *tuning;
     char *name;
     size_t name_capacity;
+    int ordinal;  // the stream's device, which is the current one
 };
 
 struct IgemmArgs {

@@ -7,12 +7,15 @@
 #include "thip_kernels.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <initializer_list>
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "thip_descriptor.h"
@@ -36,6 +39,33 @@ static std::string kernelLabel(const char *name, std::initializer_list<int> para
     }
     return s + ">";
 }
+// A launch site's kernel on each device, as the runtime names it there.  A launch by that spares the search for the kernel that <<<>>> makes: 2.3 us of
+// the host's time in place of 2.5, where a call of one small kernel costs 3.4 in all and the kernel less.
+struct KernelHandles {
+    std::atomic<hipFunction_t> on[16];
+};
+template <typename... P, typename... A>
+static void launchKernel(KernelHandles &handles, void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, const LaunchCtx &ctx, A &&...args) {
+    std::tuple<P...> held(std::forward<A>(args)...);
+    std::apply([&](P &...p) {
+        void *at[] = {(void *)&p...};
+        hipFunction_t f = nullptr;
+        if (ctx.ordinal >= 0 && ctx.ordinal < 16) {
+            f = handles.on[ctx.ordinal].load(std::memory_order_acquire);
+            if (!f) {
+                if (hipGetFuncBySymbol(&f, (const void *)kernel) != hipSuccess) {
+                    (void)hipGetLastError();
+                    f = nullptr;
+                } else {
+                    handles.on[ctx.ordinal].store(f, std::memory_order_release);
+                }
+            }
+        }
+        if (f) (void)hipModuleLaunchKernel(f, grid.x, grid.y, grid.z, block.x, block.y, block.z, (unsigned)lds, ctx.stream, at, nullptr);
+        else (void)hipLaunchKernel((const void *)kernel, grid, block, at, lds, ctx.stream);
+    }, held);
+}
+
 static const char *labelText(const char *s) { return s; }
 static const char *labelText(const std::string &s) { return s.c_str(); }
 // A launch site.  With ctx.name set the launcher is only asked which kernel it would launch for these arguments (the
@@ -45,7 +75,8 @@ static const char *labelText(const std::string &s) { return s.c_str(); }
         if ((ctx).name) {                                                                 \
             snprintf((ctx).name, (ctx).name_capacity, "%s", labelText(label));            \
         } else {                                                                          \
-            hipLaunchKernelGGL(kernel, grid, block, lds, (ctx).stream, __VA_ARGS__);      \
+            static KernelHandles handles_;                                                \
+            launchKernel(handles_, kernel, grid, block, lds, ctx, __VA_ARGS__);           \
         }                                                                                 \
     } while (0)
 
