@@ -164,7 +164,7 @@ __global__ __launch_bounds__(512) void conv_patch_i8(IgemmArgs p, ConvPatchPlan 
                         const auto s02 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
                         const auto s13 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
                         const int m = t * 64 + 32 * i + fr;
-                        if (m < pixels && n < p.N) *(v4i *)(out + (size_t)m * p.N + n) = v4i{(int)s02[0], (int)s02[1], (int)s13[0], (int)s13[1]};
+                        if (m < pixels && n < p.N) storeRow16(out + (size_t)m * p.N + n, v4i{(int)s02[0], (int)s02[1], (int)s13[0], (int)s13[1]}, p.N - n);
                     }
                 }
             });
@@ -177,11 +177,11 @@ constexpr size_t kPatchMaxLds = 160 * 1024;
 // The pitch of rows of `bytes` (whole 16-byte units) in LDS.
 static int paddedPitch(int bytes) { return bytes / 16 % 4 == 0 ? bytes + 16 : bytes; }
 
-// Fills the plan; false where the kernel does not take the operands (whole 16-byte pieces of image, weights and results; the ring
-// kernel stores at any alignment).
+// Fills the plan; false where the kernel does not take the operands (whole 16-byte pieces of image and weights, results that begin at one, rows of
+// which may be of any length: 3x3 115x115x32 -> 40, batch 26, 20.5 us, the ring kernel 21 - 29).
 static bool planConvPatch(const IgemmArgs &a, ConvPatchPlan *q) {
     if (!a.A || !a.Bp || !a.bias || !a.scale || !a.out || (((uintptr_t)a.A | (uintptr_t)a.Bp | (uintptr_t)a.out) & 15)) return false;
-    if (a.loader != kLoaderWindow || a.out_dtype != kDtypeI8 || a.skip || a.M <= 0 || a.N <= 0 || a.N % 16 != 0 || a.N > 96 || a.C < 16 || a.C % 16 != 0) return false;
+    if (a.loader != kLoaderWindow || a.out_dtype != kDtypeI8 || a.skip || a.M <= 0 || a.N <= 0 || a.N > 96 || a.C < 16 || a.C % 16 != 0) return false;
     if (a.KH <= 0 || a.KW <= 0 || a.KH > 16 || a.KW > 16 || a.H <= 0 || a.W <= 0 || a.OH <= 0 || a.OW <= 0 || a.SH != 1 || a.SW != 1 || a.PT < 0 || a.PL < 0) return false;
     const long long frame = (long long)a.OH * a.OW, taps = (long long)a.KH * a.KW * a.C;
     if (a.M % frame != 0 || a.K != taps || taps > 8192 || (long long)a.H * a.W * a.C >= (1LL << 31)) return false;

@@ -169,9 +169,9 @@ static uint8_t *resolve(const thip_executable_t *e, const DescRef &r, uint8_t *c
 // Launches `op`, which is record i or stands in for it, or (ctx.name set) only asks its launcher which kernel it takes for these
 // operands.  `scratch` (or null): the static scratch array, which then stands in for the record's workspace intermediate.
 // `step` (or null): the buffers of space kSpacePlan.  `route`: the kernel of a GEMM-shaped record.
-// `blocked`: DecBlocked, the intermediates of a decoder's record that lie in blocks of columns.
+// `blocked`: DecBlocked, the intermediates of a decoder's record that lie in blocks of columns.  `planned`: a step's launch, not the record's own kernel.
 static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr,
-                              uint8_t *const *step = nullptr, IgemmRoute route = kIgemmOwnTile, int32_t blocked = 0) {
+                              uint8_t *const *step = nullptr, IgemmRoute route = kIgemmOwnTile, int32_t blocked = 0, bool planned = false) {
     auto resolve = [step](const thip_executable_t *exe, const DescRef &r, uint8_t *const *bindings) {
         return r.space == kSpacePlan ? step[r.index] + r.offset : ::resolve(exe, r, bindings);
     };
@@ -186,7 +186,8 @@ static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op
     case kKindIgemm: {
         auto at = [&](const DescRef &r) { return resolve(e, r, bp); };
         const bool asIs = route == kIgemmDirect && e->ops[i].loader == kLoaderGather && op.in0.space != kSpacePlan;
-        const IgemmArgs a = asIs ? raggedArgs(viewOf(e), op, e->ops[i].C, at) : igemmArgs(viewOf(e), op, at);
+        IgemmArgs a = asIs ? raggedArgs(viewOf(e), op, e->ops[i].C, at) : igemmArgs(viewOf(e), op, at);
+        a.any_rows = planned && !e->tuning.plainRecords;
         if (route == kIgemmDirect) err = launchIgemmDirect(a, ctx);
         else if (route == kIgemmPatch) err = launchConvPatch(a, ctx);
         else err = launchIgemm(a, op.variant, ctx, route == kIgemmWide);
@@ -572,7 +573,7 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
     case kStepPadded: {
         uint8_t *const *buffers = &e->stepBuffers[2 * (size_t)(&s - e->steps.data())];
         if (s.rows > 0) err = launchPadRows((const int8_t *)resolve(e, e->ops[s.first].in0, bp), (int8_t *)buffers[0], s.rows, s.from, s.to, ctx);
-        if (err == hipSuccess) return launchOp(e, s.first, s.op, bp, ctx, scratch, buffers, s.route);
+        if (err == hipSuccess) return launchOp(e, s.first, s.op, bp, ctx, scratch, buffers, s.route, 0, true);
         break;
     }
     case kStepDecChain: {
@@ -595,7 +596,7 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
         err = launchDecChain(a, e->device->computeUnits, ctx);
         break;
     }
-    default: return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch, nullptr, s.route, s.blocked);
+    default: return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch, nullptr, s.route, s.blocked, true);
     }
     if (err != hipSuccess) return fail(THIP_INTERNAL, "ops %u .. %u: launch failed: %s", s.first, s.first + s.count - 1, hipGetErrorString(err));
     return THIP_OK;

@@ -95,6 +95,7 @@ struct IgemmArgs {
     int32_t M, N, K, Kp, Np;
     int32_t H, W, C, OH, OW, SH, SW, PT, PL;
     int32_t KH, KW;         // window loader only
+    int32_t any_rows;       // the ring kernels: int8 results of rows of any length and alignment are requantised in registers too
     int32_t row_bytes;      // igemm_direct_i8 only: what a pixel of A takes where C is that rounded up to whole 16-byte chunks (0: C)
     int32_t input_zp;
     int32_t out_dtype;

@@ -434,6 +434,24 @@ struct __attribute__((packed)) UnalignedV2 {
 struct __attribute__((packed)) UnalignedU32 {
     uint32_t v;
 };
+// The first `count` of 16 result bytes, or all of them.
+__device__ __forceinline__ void storeRow16(int8_t *out, v4i v, int count) {
+    if (count >= 16) {
+        ((UnalignedV4 *)out)->v = v;
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        if (4 * q + 4 <= count) {
+            ((UnalignedU32 *)(out + 4 * q))->v = (uint32_t)v[q];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 3; e++) {
+                if (4 * q + e < count) out[4 * q + e] = (int8_t)((uint32_t)v[q] >> (8 * e));
+            }
+        }
+    }
+}
 
 // 16 bytes that were read d bytes before (d < 0: behind) the place where they are wanted, put right; what lies outside [lo, hi) of them is padding.
 __device__ __forceinline__ v4i fixRun16(v4i bytes, int d, int lo, int hi, uint32_t zp4) {
