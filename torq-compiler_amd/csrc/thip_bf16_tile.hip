@@ -257,12 +257,27 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *KG * 64, BLOCKS_PER_CU) void fc_b
     if (tid < BN) ldsBias[tid] = myBias;
     __syncthreads();
     if (KG > 1 && kg > 0) return;
+    // Eight results of row m from column n on, at any alignment.
+    auto store = [&](int m, int n, v4i v) {
+        if (m >= p.M || n >= p.N) return;
+        uint16_t *out = p.out + (size_t)m * p.N + n;
+        if (n + 8 <= p.N) {
+            ((UnalignedV4 *)out)->v = v;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 7; e++) {
+                if (n + e < p.N) out[e] = (uint16_t)((uint32_t)v[e >> 1] >> (16 * (e & 1)));
+            }
+        }
+    };
     // Bias, clamp, v_cvt_pk_bf16_f32 and the stores; a copy without the clamp's compares, which are half the instructions
     // of an epilogue that every CU runs at the same time (a linear layer has none).  32 rows of a wave's results pass through LDS, from where they are
-    // stored in runs of whole rows of the wave's columns, at any alignment.
+    // stored in runs of whole rows of the wave's columns.  Where those are 32, two v_permlane32_swap give a lane 8 neighbouring ones of a row, without that
+    // way round (654 x 1736 -> 208 9.0 us, through LDS 9.3).
+    constexpr bool kRuns = WTN > 32;
     constexpr int CHUNKS = WTN / 8;  // of eight results in a row of a wave
     int8_t *mine = smem + BN * 4 + wave * (WTM * WTN * 2);
-    const int sc = lane % CHUNKS, sr = lane / CHUNKS, ns = n0 + wn * WTN + sc * 8;
+    const int sc = lane % CHUNKS, sr = lane / CHUNKS;
     auto finish = [&](auto clampTag) {
         constexpr bool kClamp = decltype(clampTag)::value;
 #pragma unroll
@@ -270,6 +285,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *KG * 64, BLOCKS_PER_CU) void fc_b
             int8_t *rows = mine + i * (32 * WTN * 2);
 #pragma unroll
             for (int j = 0; j < TN; j++) {
+                uint32_t d[8];  // d[2 q + (e >> 1)]: columns 8 q + 4 half + e, + 1
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     const float4 b4 = *(const float4 *)(ldsBias + wn * WTN + j * 32 + 8 * q + 4 * half);
@@ -280,24 +296,24 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *KG * 64, BLOCKS_PER_CU) void fc_b
                         v[e] = acc[j][i][4 * q + e] + b[e];
                         if (kClamp) v[e] = v[e] < p.lo ? p.lo : (v[e] > p.hi ? p.hi : v[e]);
                     }
-                    *(v2i *)(rows + fr * (WTN * 2) + (((4 * j + q) ^ fr) % CHUNKS) * 16 + 8 * half) = v2i{(int)packBf16(v[0], v[1]), (int)packBf16(v[2], v[3])};
+                    d[2 * q] = packBf16(v[0], v[1]);
+                    d[2 * q + 1] = packBf16(v[2], v[3]);
+                    if (kRuns) *(v2i *)(rows + fr * (WTN * 2) + (((4 * j + q) ^ fr) % CHUNKS) * 16 + 8 * half) = v2i{(int)d[2 * q], (int)d[2 * q + 1]};
+                }
+                if (kRuns) continue;
+#pragma unroll
+                for (int q2 = 0; q2 < 2; q2++) {  // the lower half of the wave ends up with the first 8 of 16 columns, the upper with the others
+                    const auto s0 = __builtin_amdgcn_permlane32_swap(d[4 * q2], d[4 * q2 + 2], false, false);
+                    const auto s1 = __builtin_amdgcn_permlane32_swap(d[4 * q2 + 1], d[4 * q2 + 3], false, false);
+                    store(m0 + wm * WTM + i * 32 + fr, n0 + wn * WTN + j * 32 + 16 * q2 + 8 * half, v4i{(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]});
                 }
             }
+            if (!kRuns) continue;
             asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
 #pragma unroll
             for (int t = 0; t < CHUNKS / 2; t++) {
-                const int r = t * (64 / CHUNKS) + sr, m = m0 + wm * WTM + i * 32 + r;
-                const v4i v = *(const v4i *)(rows + r * (WTN * 2) + ((sc ^ r) % CHUNKS) * 16);
-                if (m >= p.M || ns >= p.N) continue;
-                uint16_t *out = p.out + (size_t)m * p.N + ns;
-                if (ns + 8 <= p.N) {
-                    ((UnalignedV4 *)out)->v = v;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 7; e++) {
-                        if (ns + e < p.N) out[e] = (uint16_t)((uint32_t)v[e >> 1] >> (16 * (e & 1)));
-                    }
-                }
+                const int r = t * (64 / CHUNKS) + sr;
+                store(m0 + wm * WTM + i * 32 + r, n0 + wn * WTN + sc * 8, *(const v4i *)(rows + r * (WTN * 2) + ((sc ^ r) % CHUNKS) * 16));
             }
         }
     };

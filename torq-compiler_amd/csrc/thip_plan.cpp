@@ -194,11 +194,11 @@ static bool paddingPays(const DescOp &g, int64_t rows, int64_t Cp, int64_t K) {
 // channels that it takes, own kernel / copied rows / rows as they are cost 2.78 / 1.55 / 1.00 times the best (us: linear 9x100 -> 2303 5.5 / 6.4 / 4.0,
 // 554x604 -> 117 13.4 / 6.6 / 4.0, 5x1379 -> 48 57.4 / 6.4 / 4.5; 3x3 30x30x98 -> 316 stride 2, batch 3 7.1 / 6.6 / 4.0, 56x56x40 -> 32, batch 2 6.5 / 6.5 / 4.0; stride 2
 // 1x1 56x56x264 -> 96, batch 4 6.1 / 7.8 / 4.2).  Left where the gather is short (60x24 -> 64 3.6 / 6.1 / 3.8, 3x3 112x112x8 -> 32 4.5 / 6.7 / 4.1) and
-// where K is long enough for the worse loads to cost that launch: 3x5637 -> 567 224 / 8.3 / 9.0 (few rows have a faster kernel behind the copy), 5x5
+// where K is long enough for the worse loads to cost that launch: 3x2801 -> 1608 - / 6.2 / 6.6 (few rows have a faster kernel behind the copy), 5x5
 // 19x19x387 -> 134 452 / 18.2 / 19.7.
 static bool asIsBetter(const DescriptorView &v, const Tuning &tuning, const DescOp &g, const DescOp &op) {
     if (tuning.padRows == 0 || tuning.padRows == 1 || g.kind != kKindIgemm || g.loader != kLoaderGather) return false;
-    return igemmDirectBetter(raggedArgs(v, op, g.C, [&](const DescRef &r) { return plannedAt(v, r); })) && (tuning.padRows == 2 || (gatherTime(g) > 4.0 && g.K <= (g.M <= kFcSkinnyMaxRows ? 5000 : 9000)));
+    return igemmDirectBetter(raggedArgs(v, op, g.C, [&](const DescRef &r) { return plannedAt(v, r); })) && (tuning.padRows == 2 || (gatherTime(g) > 4.0 && g.K <= (g.M <= kFcSkinnyMaxRows ? 2500 : 9000)));
 }
 
 // Whether the weights of a window of one pixel are zeros from K to the end of the last chunk that igemm_direct_i8 reads, as they are packed.
