@@ -142,7 +142,7 @@ __device__ __forceinline__ void igemmEpilogue(v16i (&acc)[WTN / 32][WTM / 32], i
 // (see igemm_stream_i8), and the lane stores them as one 128-bit word, at any alignment, those behind a row's end left out.  Only the (bias, scale)
 // vectors pass through LDS.  Rows of no whole 16 columns, through LDS / in registers, us: 2000x1024 -> 1000 6.9 / 5.9, 4096x2048 -> 4090 41.2 /
 // 38.2, 3x3 56x56x128 -> 136, batch 16 28.8 / 21.2, 1x1 56x56x64 -> 200, batch 16 12.4 / 7.5, 112x112x32 -> 24, batch 32 18.9 / 12.3.
-template <int WTM, int WTN, int NW, int BN, bool ADD, bool PLAIN>  // ADD: a residual add behind the requant (IgemmArgs::skip); PLAIN: see requantWideT0
+template <int WTM, int WTN, int NW, int BN, bool ADD, bool PLAIN, bool ANY>  // ADD: a residual add behind the requant (IgemmArgs::skip); PLAIN: see requantWideT0; ANY: rows of any length
 __device__ __forceinline__ void igemmEpilogueDirect(v16i (&acc)[WTN / 32][WTM / 32], int8_t *smem, const IgemmArgs &p, int m0,
                                                     int n0, int wm, int wn, int32_t myBias, int32_t myScale) {
     blockBarrier();
@@ -154,7 +154,7 @@ __device__ __forceinline__ void igemmEpilogueDirect(v16i (&acc)[WTN / 32][WTM / 
         ldsScale[tid] = myScale;
     }
     __syncthreads();
-    const bool wholeRows = p.N % 16 == 0 && ((uintptr_t)p.out & 15) == 0;
+    const bool wholeRows = !ANY || (p.N % 16 == 0 && ((uintptr_t)p.out & 15) == 0);
     const WideRequant wrq = wideRequant(p.rq);  // a 32-bit tail applies (the launcher checks); PLAIN: no pre-shift, no clamp of acc + bias, zero point folded
     const long long addRnd = roundTerm(p.arq.shift);
     int32_t addFolded = 0;
@@ -200,8 +200,10 @@ __device__ __forceinline__ void igemmEpilogueDirect(v16i (&acc)[WTN / 32][WTM / 
         }
     };
     if (wholeRows) finish(std::true_type{});
-    else finish(std::false_type{});
+    else if constexpr (ANY) finish(std::false_type{});
 }
+// Which kernels have the second copy of the epilogue: not those of four large tiles a CU, whose 128 registers it would spill (13.2 -> 21.2 us).
+constexpr bool igemmAnyRows(int BM, int BN, int blocksPerCu, bool add) { return !add && (BM * BN < 128 * 128 || blocksPerCu < 4); }
 
 // ---------------------------------------------------------------------------
 // igemm_i8
@@ -742,7 +744,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BLOCKS_PER_CU) void igemm_de
     for (; kt < KT; kt++) step(kt, std::false_type{});
 
     if (DIRECT) {
-        igemmEpilogueDirect<WTM, WTN, NW, BN, ADD, DIRECT == 1>(acc, smem, p, m0, n0, wm, wn, myBias, myScale);
+        igemmEpilogueDirect<WTM, WTN, NW, BN, ADD, DIRECT == 1, igemmAnyRows(BM, BN, BLOCKS_PER_CU, ADD)>(acc, smem, p, m0, n0, wm, wn, myBias, myScale);
     } else {
         igemmEpilogue<WTM, WTN, NW, BN>(acc, smem, p, m0, n0, wm, wn, myBias, myScale);
     }
@@ -1252,7 +1254,7 @@ static hipError_t launchIgemmDense(const IgemmArgs &a, const LaunchCtx &ctx) {
                        a.rq.out_zp >= -32768 && a.rq.out_zp <= 32767 && a.rq.out_min <= a.rq.out_max;
     const bool wide = (a.rq.shift >= 32 || (a.rq.pre_shift > 0 && a.rq.shift + a.rq.pre_shift == 33)) && a.rq.out_min <= a.rq.out_max;
     const bool wholeRows = a.N % 16 == 0 && ((uintptr_t)a.out & 15) == 0;
-    const bool inRegisters = a.out_dtype == kDtypeI8 && (wholeRows || (a.any_rows && !a.skip)) && !ctx.tuning->noDirectEpilogue;
+    const bool inRegisters = a.out_dtype == kDtypeI8 && (wholeRows || (a.any_rows && !a.skip && igemmAnyRows(BM, BN, BLOCKS_PER_CU, false))) && !ctx.tuning->noDirectEpilogue;
     const bool direct = inRegisters && plain;
     if (a.skip != nullptr) {
         // a residual add: the in-register epilogue of the small tile only (what a network's late, small layers take)
