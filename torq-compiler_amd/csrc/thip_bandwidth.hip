@@ -785,10 +785,13 @@ hipError_t launchMaxPool(const MaxPoolArgs &a, const LaunchCtx &ctx) {
 
 // Global average pool: one wave covers CC channel groups of VEC channels; the
 // 64 / CC lanes that share a channel group split the H*W pixels and are
-// combined with wave shuffles.
+// combined with wave shuffles.  With 16 lanes for 16 channels they are combined so that each ends with the sum of one channel, which it
+// finishes, and four pixels at a time are transposed for a dot product by channel (256 frames of
+// 7x7x1280 8.4 us, 6.0; one 4.4, 3.2).
 template <int VEC, int CC>
 __global__ __launch_bounds__(256) void avgpool_i8(AvgPoolArgs p) {
     constexpr int PG = 64 / CC;  // lanes per channel group
+    constexpr bool kByLane = VEC == 16 && PG == 16;
     const int lane = threadIdx.x & 63;
     const int wave = (int)((blockIdx.x * 256 + threadIdx.x) >> 6);
     const int cgroups = p.C / VEC;
@@ -813,13 +816,52 @@ __global__ __launch_bounds__(256) void avgpool_i8(AvgPoolArgs p) {
                 const int u = u0 + j * PG;
                 x[j].v = *(const typename ByteVec<VEC>::type *)(src + (size_t)(u < p.HW ? u : pg) * p.C);
             }
+            if constexpr (kByLane) {
+                // 1 for a pixel of the frame, 0 for one past it
+                uint32_t in = 0;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int32_t wj = u0 + j * PG < p.HW ? p.weight : 0;
+                for (int j = 0; j < 4; j++) in |= u0 + j * PG < p.HW ? 1u << (8 * j) : 0u;
 #pragma unroll
-                for (int v = 0; v < VEC; v++) acc[v] += (int32_t)x[j].b[v] * wj;
+                for (int d = 0; d < VEC / 4; d++) {
+                    uint32_t o[4];
+                    transpose4x4((uint32_t)x[0].v[d], (uint32_t)x[1].v[d], (uint32_t)x[2].v[d], (uint32_t)x[3].v[d], o);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[4 * d + e] = __builtin_amdgcn_sdot4((int)o[e], (int)in, acc[4 * d + e], false);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int32_t wj = u0 + j * PG < p.HW ? p.weight : 0;
+#pragma unroll
+                    for (int v = 0; v < VEC; v++) acc[v] += (int32_t)x[j].b[v] * wj;
+                }
             }
         }
+    }
+    const long long rnd = roundTerm(p.rq.shift);
+    if constexpr (kByLane) {
+        // half of the channels change places with each step: lane group pg is left with channel pg
+#pragma unroll
+        for (int v = 0; v < 8; v++) {
+            const auto x = __builtin_amdgcn_permlane32_swap((uint32_t)acc[v], (uint32_t)acc[v + 8], false, false);
+            acc[v] = (int32_t)(x[0] + x[1]);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const auto x = __builtin_amdgcn_permlane16_swap((uint32_t)acc[v], (uint32_t)acc[v + 4], false, false);
+            acc[v] = (int32_t)(x[0] + x[1]);
+        }
+#pragma unroll
+        for (int half = 2; half >= 1; half--) {
+            const bool upper = (pg & half) != 0;
+#pragma unroll
+            for (int v = 0; v < half; v++) {
+                const int32_t mine = upper ? acc[v + half] : acc[v], other = upper ? acc[v] : acc[v + half];
+                acc[v] = (int32_t)((uint32_t)mine + (uint32_t)__shfl_xor(other, half * CC, 64));
+            }
+        }
+        if (active) p.out[(size_t)n * p.C + c0 + pg] = (int8_t)requant((int32_t)((uint32_t)acc[0] * (uint32_t)p.weight), p.bias, p.scale, rnd, p.rq);
+        return;
     }
 #pragma unroll
     for (int v = 0; v < VEC; v++) {
@@ -829,7 +871,6 @@ __global__ __launch_bounds__(256) void avgpool_i8(AvgPoolArgs p) {
         acc[v] = s;
     }
     if (active && pg == 0) {
-        const long long rnd = roundTerm(p.rq.shift);
         Pack<VEC> o;
 #pragma unroll
         for (int v = 0; v < VEC; v++) o.b[v] = (int8_t)requant(acc[v], p.bias, p.scale, rnd, p.rq);

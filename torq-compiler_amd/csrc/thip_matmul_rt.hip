@@ -8,16 +8,6 @@ struct __attribute__((packed)) UnalignedWord {
     uint32_t v;
 };
 
-// Four rows of four bytes, transposed: word j of the result holds byte j of each row.
-__device__ __forceinline__ void transpose4x4(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3, uint32_t (&o)[4]) {
-    const uint32_t a = __builtin_amdgcn_perm(w1, w0, 0x05010400u), b = __builtin_amdgcn_perm(w1, w0, 0x07030602u);
-    const uint32_t c = __builtin_amdgcn_perm(w3, w2, 0x05010400u), d = __builtin_amdgcn_perm(w3, w2, 0x07030602u);
-    o[0] = __builtin_amdgcn_perm(c, a, 0x05040100u);
-    o[1] = __builtin_amdgcn_perm(c, a, 0x07060302u);
-    o[2] = __builtin_amdgcn_perm(d, b, 0x05040100u);
-    o[3] = __builtin_amdgcn_perm(d, b, 0x07060302u);
-}
-
 // ---------------------------------------------------------------------------
 // igemm_rt_i8: out[b][m][n] = R1(sum_k A[b][m][k] * B[b][k][n]) with ONE (bias, scale) pair, int8 / int16 / int32 results.
 //
