@@ -29,7 +29,7 @@ struct ConvPatchPlan {
     size_t lds;
 };
 
-template <int NB>
+template <int NB, bool ANY>  // ANY: rows of no whole 16 channels
 __global__ __launch_bounds__(512) void conv_patch_i8(IgemmArgs p, ConvPatchPlan q, FastDiv divPixel, FastDiv divCols, FastDiv divOW, FastDiv divRow) {
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -164,7 +164,10 @@ __global__ __launch_bounds__(512) void conv_patch_i8(IgemmArgs p, ConvPatchPlan 
                         const auto s02 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
                         const auto s13 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
                         const int m = t * 64 + 32 * i + fr;
-                        if (m < pixels && n < p.N) storeRow16(out + (size_t)m * p.N + n, v4i{(int)s02[0], (int)s02[1], (int)s13[0], (int)s13[1]}, p.N - n);
+                        const v4i v = {(int)s02[0], (int)s02[1], (int)s13[0], (int)s13[1]};
+                        if (m >= pixels || n >= p.N) continue;
+                        if (ANY) storeRow16(out + (size_t)m * p.N + n, v, p.N - n);
+                        else *(v4i *)(out + (size_t)m * p.N + n) = v;
                     }
                 }
             });
@@ -223,15 +226,15 @@ bool convPatchBetter(const IgemmArgs &a) {
     return a.C <= 112 && a.KH * a.KW >= 9 && a.M >= 49152 && planConvPatch(a, &q) && q.rows * a.KW >= 9;
 }
 
-template <int NB>
+template <int NB, bool ANY>
 static hipError_t launchPatch(const IgemmArgs &a, const ConvPatchPlan &q, const LaunchCtx &ctx) {
-    auto kernel = conv_patch_i8<NB>;
+    auto kernel = conv_patch_i8<NB, ANY>;
     static std::once_flag once;
     static hipError_t configured = hipSuccess;
     std::call_once(once, [&] { configured = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPatchMaxLds); });
     if (configured != hipSuccess) return configured;
     const int perCu = (int)(kPatchMaxLds / q.lds) < 2 ? 1 : 2, grid = q.strips < 256 * perCu ? q.strips : 256 * perCu;
-    THIP_ENQUEUE(ctx, kernelLabel("conv_patch_i8", {NB}), kernel, dim3((unsigned)grid), dim3(512), q.lds, a, q, makeFastDiv((uint32_t)(a.C / 16)), makeFastDiv((uint32_t)q.cols),
+    THIP_ENQUEUE(ctx, kernelLabel("conv_patch_i8", {NB, (int)ANY}), kernel, dim3((unsigned)grid), dim3(512), q.lds, a, q, makeFastDiv((uint32_t)(a.C / 16)), makeFastDiv((uint32_t)q.cols),
                  makeFastDiv((uint32_t)a.OW), makeFastDiv((uint32_t)(2 * q.steps)));
     return hipGetLastError();
 }
@@ -239,10 +242,11 @@ static hipError_t launchPatch(const IgemmArgs &a, const ConvPatchPlan &q, const 
 hipError_t launchConvPatch(const IgemmArgs &a, const LaunchCtx &ctx) {
     ConvPatchPlan q;
     if (!planConvPatch(a, &q)) return hipErrorInvalidValue;
+    const bool any = a.N % 16 != 0;
     switch ((a.N + 31) / 32) {
-    case 1: return launchPatch<1>(a, q, ctx);
-    case 2: return launchPatch<2>(a, q, ctx);
-    default: return launchPatch<3>(a, q, ctx);
+    case 1: return any ? launchPatch<1, true>(a, q, ctx) : launchPatch<1, false>(a, q, ctx);
+    case 2: return any ? launchPatch<2, true>(a, q, ctx) : launchPatch<2, false>(a, q, ctx);
+    default: return any ? launchPatch<3, true>(a, q, ctx) : launchPatch<3, false>(a, q, ctx);
     }
 }
 

@@ -140,7 +140,8 @@ __device__ __forceinline__ void igemmEpilogue(v16i (&acc)[WTN / 32][WTM / 32], i
 // 32-bit requant tail (no pre-shift, zero point folded into the rounding term): each accumulator tile is requantised in place, two v_permlane32_swap exchange
 // register groups between the wave halves so that a lane owns 16 consecutive channels of its row
 // (see igemm_stream_i8), and the lane stores them as one 128-bit word, at any alignment, those behind a row's end left out.  Only the (bias, scale)
-// vectors pass through LDS.  Rows of no whole 16 columns, through LDS / in registers, us: 2000x1024 -> 1000 6.9 / 5.9, 4096x2048 -> 4090 41.2 /
+// vectors pass through LDS.  Rows of no whole 16 columns (ANY, the plain tail, kernels of their own: in the same ones the second way of storing costs whole rows
+// up to 7 %), through LDS / in registers, us: 2000x1024 -> 1000 6.9 / 5.9, 4096x2048 -> 4090 41.2 /
 // 38.2, 3x3 56x56x128 -> 136, batch 16 28.8 / 21.2, 1x1 56x56x64 -> 200, batch 16 12.4 / 7.5, 112x112x32 -> 24, batch 32 18.9 / 12.3.
 template <int WTM, int WTN, int NW, int BN, bool ADD, bool PLAIN, bool ANY>  // ADD: a residual add behind the requant (IgemmArgs::skip); PLAIN: see requantWideT0; ANY: rows of any length
 __device__ __forceinline__ void igemmEpilogueDirect(v16i (&acc)[WTN / 32][WTM / 32], int8_t *smem, const IgemmArgs &p, int m0,
@@ -154,56 +155,49 @@ __device__ __forceinline__ void igemmEpilogueDirect(v16i (&acc)[WTN / 32][WTM / 
         ldsScale[tid] = myScale;
     }
     __syncthreads();
-    const bool wholeRows = !ANY || (p.N % 16 == 0 && ((uintptr_t)p.out & 15) == 0);
     const WideRequant wrq = wideRequant(p.rq);  // a 32-bit tail applies (the launcher checks); PLAIN: no pre-shift, no clamp of acc + bias, zero point folded
     const long long addRnd = roundTerm(p.arq.shift);
     int32_t addFolded = 0;
     const bool addFast = ADD && residualAddFolded(p.add_w0, p.add_w1, p.add_bias, p.add_scale, p.arq, &addFolded);
-    auto finish = [&](auto whole) {
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int nl = wn * WTN + j * 32;  // first channel of this tile column, relative to n0
-            v4i b4[4], s4[4];
+    for (int j = 0; j < TN; j++) {
+        const int nl = wn * WTN + j * 32;  // first channel of this tile column, relative to n0
+        v4i b4[4], s4[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            b4[q] = *(const v4i *)(ldsBias + nl + 8 * q + 4 * half);
+            s4[q] = *(const v4i *)(ldsScale + nl + 8 * q + 4 * half);
+        }
+        const int n = n0 + nl + 16 * half;
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            uint32_t d4[4];
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                b4[q] = *(const v4i *)(ldsBias + nl + 8 * q + 4 * half);
-                s4[q] = *(const v4i *)(ldsScale + nl + 8 * q + 4 * half);
+                int32_t v[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    v[e] = requantWideT0<PLAIN>((int32_t)((uint32_t)acc[j][i][4 * q + e] + (uint32_t)b4[q][e]), s4[q][e], wrq);
+                }
+                d4[q] = packBytes(v[0], v[1], v[2], v[3]);
             }
-            const int n = n0 + nl + 16 * half;
-#pragma unroll
-            for (int i = 0; i < TM; i++) {
-                uint32_t d4[4];
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    int32_t v[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        v[e] = requantWideT0<PLAIN>((int32_t)((uint32_t)acc[j][i][4 * q + e] + (uint32_t)b4[q][e]), s4[q][e], wrq);
-                    }
-                    d4[q] = packBytes(v[0], v[1], v[2], v[3]);
+            const auto s02 = __builtin_amdgcn_permlane32_swap(d4[0], d4[2], false, false);
+            const auto s13 = __builtin_amdgcn_permlane32_swap(d4[1], d4[3], false, false);
+            v4i outv = {(int)s02[0], (int)s02[1], (int)s13[0], (int)s13[1]};
+            const int m = m0 + wm * WTM + i * 32 + fr;
+            if (m < p.M && n < p.N) {
+                if (ADD) {
+                    const v4i other = *(const v4i *)(p.skip + (size_t)m * p.N + n);
+                    outv = addFast ? residualAdd16<true>(outv, other, p.add_skip_first != 0, p.add_w0, p.add_w1, p.add_bias, p.add_scale, addRnd, p.arq, addFolded)
+                                   : residualAdd16<false>(outv, other, p.add_skip_first != 0, p.add_w0, p.add_w1, p.add_bias, p.add_scale, addRnd, p.arq, 0);
                 }
-                const auto s02 = __builtin_amdgcn_permlane32_swap(d4[0], d4[2], false, false);
-                const auto s13 = __builtin_amdgcn_permlane32_swap(d4[1], d4[3], false, false);
-                v4i outv = {(int)s02[0], (int)s02[1], (int)s13[0], (int)s13[1]};
-                const int m = m0 + wm * WTM + i * 32 + fr;
-                if (m < p.M && n < p.N) {
-                    if (ADD) {
-                        const v4i other = *(const v4i *)(p.skip + (size_t)m * p.N + n);
-                        outv = addFast ? residualAdd16<true>(outv, other, p.add_skip_first != 0, p.add_w0, p.add_w1, p.add_bias, p.add_scale, addRnd, p.arq, addFolded)
-                                       : residualAdd16<false>(outv, other, p.add_skip_first != 0, p.add_w0, p.add_w1, p.add_bias, p.add_scale, addRnd, p.arq, 0);
-                    }
-                    int8_t *out = (int8_t *)p.out + (size_t)m * p.N + n;
-                    if (decltype(whole)::value) *(v4i *)out = outv;
-                    else storeRow16(out, outv, p.N - n);
-                }
+                int8_t *out = (int8_t *)p.out + (size_t)m * p.N + n;
+                if (!ANY) *(v4i *)out = outv;
+                else storeRow16(out, outv, p.N - n);
             }
         }
-    };
-    if (wholeRows) finish(std::true_type{});
-    else if constexpr (ANY) finish(std::false_type{});
+    }
 }
-// Which kernels have the second copy of the epilogue: not those of four large tiles a CU, whose 128 registers it would spill (13.2 -> 21.2 us).
-constexpr bool igemmAnyRows(int BM, int BN, int blocksPerCu, bool add) { return !add && (BM * BN < 128 * 128 || blocksPerCu < 4); }
 
 // ---------------------------------------------------------------------------
 // igemm_i8
@@ -744,7 +738,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BLOCKS_PER_CU) void igemm_de
     for (; kt < KT; kt++) step(kt, std::false_type{});
 
     if (DIRECT) {
-        igemmEpilogueDirect<WTM, WTN, NW, BN, ADD, DIRECT == 1, igemmAnyRows(BM, BN, BLOCKS_PER_CU, ADD)>(acc, smem, p, m0, n0, wm, wn, myBias, myScale);
+        igemmEpilogueDirect<WTM, WTN, NW, BN, ADD, DIRECT != 2, DIRECT == 3>(acc, smem, p, m0, n0, wm, wn, myBias, myScale);
     } else {
         igemmEpilogue<WTM, WTN, NW, BN>(acc, smem, p, m0, n0, wm, wn, myBias, myScale);
     }
@@ -1254,7 +1248,7 @@ static hipError_t launchIgemmDense(const IgemmArgs &a, const LaunchCtx &ctx) {
                        a.rq.out_zp >= -32768 && a.rq.out_zp <= 32767 && a.rq.out_min <= a.rq.out_max;
     const bool wide = (a.rq.shift >= 32 || (a.rq.pre_shift > 0 && a.rq.shift + a.rq.pre_shift == 33)) && a.rq.out_min <= a.rq.out_max;
     const bool wholeRows = a.N % 16 == 0 && ((uintptr_t)a.out & 15) == 0;
-    const bool inRegisters = a.out_dtype == kDtypeI8 && (wholeRows || (a.any_rows && !a.skip && igemmAnyRows(BM, BN, BLOCKS_PER_CU, false))) && !ctx.tuning->noDirectEpilogue;
+    const bool results8 = a.out_dtype == kDtypeI8 && !ctx.tuning->noDirectEpilogue, inRegisters = results8 && wholeRows;
     const bool direct = inRegisters && plain;
     if (a.skip != nullptr) {
         // a residual add: the in-register epilogue of the small tile only (what a network's late, small layers take)
@@ -1267,6 +1261,7 @@ static hipError_t launchIgemmDense(const IgemmArgs &a, const LaunchCtx &ctx) {
     }
     if (direct) return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 1, false, CONV, BK, HALF>(a, ctx);
     if (inRegisters && wide) return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 2, false, CONV, BK, HALF>(a, ctx);
+    if (results8 && !wholeRows && a.any_rows && plain) return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 3, false, CONV, BK, HALF>(a, ctx);
     return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 0, false, CONV, BK, HALF>(a, ctx);
 }
 
