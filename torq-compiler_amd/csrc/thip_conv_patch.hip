@@ -165,9 +165,13 @@ __global__ __launch_bounds__(512) void conv_patch_i8(IgemmArgs p, ConvPatchPlan 
                         const auto s13 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
                         const int m = t * 64 + 32 * i + fr;
                         const v4i v = {(int)s02[0], (int)s02[1], (int)s13[0], (int)s13[1]};
-                        if (m >= pixels || n >= p.N) continue;
-                        if (ANY) storeRow16(out + (size_t)m * p.N + n, v, p.N - n);
-                        else *(v4i *)(out + (size_t)m * p.N + n) = v;
+                        if (m < pixels && n < p.N) {
+                            if (ANY) storeRow16(out + (size_t)m * p.N + n, v, p.N - n);
+                            else *(v4i *)(out + (size_t)m * p.N + n) = v;
+                        }
+                        // Two tiles of channels: one after the other they need 123 registers in place of 171, and two workgroups share a CU where
+                        // LDS has room (115x115x32 -> 48, batch 26, 24.4 -> 19.3 us; one tile fits anyway, and loses 8 % by it).
+                        if (NB == 2) __builtin_amdgcn_sched_barrier(0);
                     }
                 }
             });
