@@ -195,24 +195,24 @@ class Loaded:
 # the kernel sources (under torq-compiler_amd/csrc) at that time, and a run whose kernel source -- the file the
 # workload's kernel lives in, or the helpers every kernel file includes -- has changed since reports traffic null.
 TRAFFIC_SOURCES_SHA256 = {
-    "thip_bandwidth.hip": "9f362b1c3295215d62fa4e31cb26409d5141f8a8775045b8e9241122a60a4c8f",
-    "thip_conv_patch.hip": "d94cab362a7338f9f6d5bb67d3dd77222153b6a69f9850d0ab0fd328cac10d4e",
-    "thip_igemm.hip": "8af44b0bac43ba07ac67de30f350a997f461de3dd2da725ee63a4fec357c9b61",
-    "thip_igemm_direct.hip": "b6e3a10ba2c1865b144a6f8f770ee4f27d61829b54799ffb7286dd29adb85e6d",
-    "thip_kernels_common.h": "b3c4244f20b719cf1485ae795905dff909881fc94ff47ec097c8d19ac569aa5e",
+    "thip_bandwidth.hip": "bf9ba4aac7ab8e50d318c3e4cdb8d14df9a6c2737c2a7778675ef1df6a1462a7",
+    "thip_conv_patch.hip": "a397507ec981f3e60ce17102fb215ad74c4c4b849f9cedc947b964899b1c1d78",
+    "thip_igemm.hip": "da7751fcfd3c41e522336a6c004db8aa490d4a0159bb4d464de957520e80b3a1",
+    "thip_igemm_direct.hip": "6f43ab6f2dcf92e68b7e778fff9cded80a6381b9f3a76965d24d2f7c323347bb",
+    "thip_kernels_common.h": "81d997303723a01ef0cb1b693d4d5f4b7f44e23beca9afd8b1b5a72c70aa67ca",
 }
 MEASURED_TRAFFIC = {
-    "fc_4096x4096x4096": (49381.0 * 1.9996 + 16588.8 * 1.0000) * 1024,
+    "fc_4096x4096x4096": (49385.5 * 1.9996 + 16584.0 * 1.0000) * 1024,
     "fc_512x4096x4096": (16453.5 * 1.9996 + 2048.0 * 1.0000) * 1024,
     "fc_16x2048x8192": (8408.0 * 1.9996 + 256.0 * 1.0000) * 1024,
     "conv_112x112x32_o64_3x3": (800.4 * 1.9996 + 784.0 * 1.0000) * 1024,
-    "conv3x3_56x56x256_o256_b32": (17251.1 * 1.9996 + 26002.0 * 1.0000) * 1024,
-    "conv3x3_56x56x96_o96_b32": (6340.0 * 1.9996 + 9591.4 * 1.0000) * 1024,
-    "conv1x1_56x56x256_o1024_b32": (14417.5 * 1.9996 + 100352.0 * 1.0000) * 1024,
-    "depthwise_b64": (14207.9 * 1.9996 + 7761.1 * 1.0000) * 1024,
-    "depthwise_s1_b256": (63708.8 * 1.9996 + 113200.1 * 1.0000) * 1024,
-    "maxpool_b64": (25464.6 * 1.9996 + 12544.0 * 1.0000) * 1024,
-    "avgpool_b64": (2001.0 * 1.9996 + 80.0 * 1.0000) * 1024,
+    "conv3x3_56x56x256_o256_b32": (17253.7 * 1.9996 + 26000.6 * 1.0000) * 1024,
+    "conv3x3_56x56x96_o96_b32": (6326.0 * 1.9996 + 9503.9 * 1.0000) * 1024,
+    "conv1x1_56x56x256_o1024_b32": (14410.0 * 1.9996 + 100352.0 * 1.0000) * 1024,
+    "depthwise_b64": (14208.7 * 1.9996 + 7771.2 * 1.0000) * 1024,
+    "depthwise_s1_b256": (63717.1 * 1.9996 + 113158.9 * 1.0000) * 1024,
+    "maxpool_b64": (25486.4 * 1.9996 + 12544.0 * 1.0000) * 1024,
+    "avgpool_b64": (1992.5 * 1.9996 + 80.0 * 1.0000) * 1024,
     "add_b64": (4723.0 * 1.9996 + 4704.0 * 1.0000) * 1024,
 }
 
