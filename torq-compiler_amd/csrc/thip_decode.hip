@@ -277,8 +277,12 @@ __global__ __launch_bounds__(kDecMaxWaves * 64) void dec_linear(DecLinearArgs p)
     for (int m = 0; m < 2; m++) {
         if (m >= nmat) break;
         v4f s = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        for (int w = 0; w < NW; w++) {
-            const v4f t = ((const v4f *)(smem + (size_t)w * regionBytes))[(m * MR + mr) * 64 + lane];
+        // ONE: a wave's sum and that of the eighth behind it first: 9 to 16 sums added in turn are further from the 64-bit sum than eight waves' of up to two
+        // k-blocks each (a model of both orders on the CPU, K = 2048: 4.01e-6 against 3.70e-6 rms; so paired 3.50e-6, and less than the eight's at every K from 1152 on).  The
+        // pairs cost a step of four layers at hidden 2048, 20 rows, 145.9 -> 148.5 us (eight waves 153.0), at 1152, 32 rows, 137.2 -> 137.9 (142.0).
+        for (int w = 0; w < (ONE ? kDecWaves : NW); w++) {
+            v4f t = ((const v4f *)(smem + (size_t)w * regionBytes))[(m * MR + mr) * 64 + lane];
+            if (ONE && w + kDecWaves < NW) t += ((const v4f *)(smem + (size_t)(w + kDecWaves) * regionBytes))[(m * MR + mr) * 64 + lane];
             s += t;
         }
         if constexpr (S > 1) {
@@ -391,7 +395,7 @@ static hipError_t launchDecLinearQ(const DecLinearArgs &in, int tiles, const Lau
     a.rows_per_group = (a.M + groups - 1) / groups;
     // A wave of one k-block holds the rows of that one only (64 registers at most): two workgroups of 16 such waves share a CU.  Where K has more k-blocks
     // than waves and the launch more workgroups than CUs, eight waves each, so that two of them (at four waves per SIMD) share one and the launch is
-    // one round of workgroups rather than two.  Steps of four layers, us, always eight / this: hidden 1152 at 32 rows 165.6 / 160.7, at 8 129.1 / 123.8;
+    // one round of workgroups rather than two.  Steps of four layers, us, always eight / this (sums added in turn; in pairs, as now, 0.4 to 1.8 % more): hidden 1152 at 32 rows 165.6 / 160.7, at 8 129.1 / 123.8;
     // 1536 at 16 rows 134.1 / 130.0, at 32 155.4 / 148.7; 2048 at 20 rows 167.2 / 160.0 (with more than 12 such waves left at eight 164.7), at 12 157.2 / 147.5; 768 at 24 rows
     // 107.6 / 103.8 (the registers alone).
     const bool few = a.rows_per_group <= 16;
