@@ -523,11 +523,20 @@ static bool chainAliased(const thip_executable_t *e, uint8_t *const *bp) {
 }
 
 // Launches one step: a record by its own launcher, a run of records by the kernel that does them as a whole.  `apart`: a chain record by record.
+// A run whose result lies where it still reads (a block in place) is launched in parts that read nothing that another workgroup of theirs writes.
 static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr, bool apart = false) {
     hipError_t err = hipSuccess;
+    auto recordByRecord = [&]() -> thip_status_t {
+        for (uint32_t i = s.first; i < s.first + s.count; i++) {
+            if (thip_status_t st = launchOp(e, i, e->ops[i], bp, ctx, scratch)) return st;
+        }
+        return THIP_OK;
+    };
     switch (s.kind) {
     case kStepExpandDw: {
-        if (s.count == 3) {
+        const bool shared = !ctx.name && writesWhatItReads(viewOf(e), s, bp);
+        if (s.count == 2 && shared) return recordByRecord();
+        if (s.count == 3 && !shared) {
             err = launchIrBlock(irBlockArgs(viewOf(e), s, [&](const DescRef &r) { return r.space == kSpaceNone ? nullptr : (uint8_t *)resolve(e, r, bp); }), ctx);
             break;
         }
@@ -552,9 +561,11 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
             a.xBytes = (int64_t)x.N * x.H * x.W * x.C;
         }
         err = launchIrExpandDw(a, ctx);
+        if (err == hipSuccess && s.count == 3) return launchOp(e, s.first + 2, e->ops[s.first + 2], bp, ctx, scratch, nullptr, s.route, 0, true);
         break;
     }
     case kStepMatmulRt: {
+        if (!ctx.name && writesWhatItReads(viewOf(e), s, bp)) return recordByRecord();
         const DescOp &g = e->ops[s.first + s.count - 1];
         MatmulRtArgs a;
         memset(&a, 0, sizeof(a));
@@ -577,12 +588,7 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
         break;
     }
     case kStepDecChain: {
-        if (!ctx.name && apart) {
-            for (uint32_t i = s.first; i < s.first + s.count; i++) {
-                if (thip_status_t st = launchOp(e, i, e->ops[i], bp, ctx, scratch)) return st;
-            }
-            return THIP_OK;
-        }
+        if (!ctx.name && apart) return recordByRecord();
         uint8_t *const *buffers = &e->stepBuffers[2 * (size_t)(&s - e->steps.data())];
         DecChainArgs a;
         memset(&a, 0, sizeof(a));

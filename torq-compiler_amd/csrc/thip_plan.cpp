@@ -160,8 +160,11 @@ static void matchBlock(const DescriptorView &v, const Tuning &tuning, const std:
     for (const DescRef *r : {&g.weights, &g.bias, &g.scale, &g.out}) {
         if (r->offset % 16 != 0) return;
     }
-    // workgroups read the rows around their own
-    if (sameBuffer(g.out, e.in0) || (g.in1.space != kSpaceNone && (sameBuffer(g.out, g.in1) || g.in1.offset % 16 != 0))) return;
+    if (g.in1.space != kSpaceNone && g.in1.offset % 16 != 0) return;
+    // workgroups read the rows around their own (what bindings share is only known with a dispatch: writesWhatItReads)
+    for (const DescRef *r : {&e.in0, &e.weights, &e.bias, &e.scale, &d.weights, &d.bias, &d.scale, &g.in1, &g.weights, &g.bias, &g.scale}) {
+        if (sameBuffer(g.out, *r)) return;
+    }
     const IrBlockArgs a = irBlockArgs(v, *s, [&](const DescRef &r) { return plannedAt(v, r); });
     if (tuning.irBlock >= 0 ? tuning.irBlock != 0 && irBlockFits(a) : irBlockBetter(a)) s->count = 3;
 }
@@ -557,6 +560,19 @@ static void blockRows(const DescriptorView &v, std::vector<Step> &steps) {
     }
 }
 
+bool writesWhatItReads(const DescriptorView &v, const Step &s, uint8_t *const *bp) {
+    const DescRef &out = v.ops[s.first + s.count - 1].out;
+    if (out.space != kSpaceBinding) return false;
+    const uint8_t *begin = bp[out.index], *end = begin + v.bindings[out.index].size;
+    for (uint32_t i = s.first; i < s.first + s.count; i++) {
+        const DescOp &op = v.ops[i];
+        for (const DescRef *r : {&op.in0, &op.in1, &op.weights, &op.bias, &op.scale, &op.table}) {
+            if (r->space == kSpaceBinding && r->index != out.index && bp[r->index] < end && begin < bp[r->index] + v.bindings[r->index].size) return true;
+        }
+    }
+    return false;
+}
+
 std::vector<Step> planSteps(const DescriptorView &v, const Tuning &tuning) {
     const bool plain = tuning.plainRecords;
     const std::vector<uint32_t> uses = tempUses(v, 0, v.header.op_count);
@@ -570,6 +586,7 @@ std::vector<Step> planSteps(const DescriptorView &v, const Tuning &tuning) {
         }
         if (s.kind == kStepExpandDw) matchBlock(v, tuning, uses, &s);
         const DescOp *op = s.kind == kStepRecord ? &v.ops[i] : s.kind == kStepPadded ? &s.op : nullptr;
+        if (s.kind == kStepExpandDw && s.count == 3) op = &v.ops[i + 2];
         s.route = plain || !op || op->kind != kKindIgemm ? kIgemmOwnTile : s.kind == kStepPadded && s.rows == 0 ? kIgemmDirect : igemmRoute(v, tuning, *op);
         i += s.count;
         steps.push_back(std::move(s));

@@ -32,7 +32,7 @@ enum IgemmRoute {
 struct Step {
     StepKind kind;
     uint32_t first, count;  // the records it stands for
-    IgemmRoute route;       // of the record, or of `op` (kStepPadded)
+    IgemmRoute route;       // of the record, of `op` (kStepPadded), or of the third record where it is launched by itself (kStepExpandDw)
     // kStepMatmulRt: the matrices of batch element 0, elements from one batch element to the next (0: shared), and the one
     // (bias, scale) pair
     DescRef a, b, out;
@@ -147,6 +147,10 @@ Chain layoutChain(const DescriptorView &v, uint32_t first, uint32_t most, int wo
 // tuning.plainRecords: one step per record, by the record's own kernel.  Routes are settled here, on all that their launchers ask: a dispatch's
 // buffers start at 16-byte boundaries, so the offsets say how its operands are aligned.
 std::vector<Step> planSteps(const DescriptorView &view, const Tuning &tuning);
+
+// Whether the step's last record writes a binding whose bytes, where the dispatch has them (`bp`: a pointer per binding), are another
+// binding's that the step reads.
+bool writesWhatItReads(const DescriptorView &v, const Step &s, uint8_t *const *bp);
 
 // Whether a dispatch of so many launches is worth a graph; `constantBytes`: what all of them read of weights.
 bool replayPays(size_t launches, uint64_t constantBytes);
