@@ -31,6 +31,7 @@ int main(int argc, char **argv) {
     const char *kinds[] = {"record", "ir_expand_dw_i8", "padded", "igemm_rt_i8", "dec_chain"}, *routes[] = {"", " igemm_direct_i8", " conv_patch_i8", " igemm_dense_k128_i8"};
     for (const Step &s : steps) {
         printf("%s %u %u%s", kinds[s.kind], s.first, s.count, routes[s.route]);
+        if (s.asIs) printf(" as it is");
         if (s.blocked) printf(" blocked %d", s.blocked);
         if (!bindings.empty() && writesWhatItReads(v, s, bindings.data())) printf(" shared");
         puts("");

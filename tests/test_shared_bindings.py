@@ -49,6 +49,36 @@ def test_other_runs_of_records_in_place(plan):
     assert plan(product, (A, B, A)) == plan(product, (A, B, B)) == [rt[0] + " shared"]
 
 
+# what a result in the place of its input runs by: a copy of the rows, or the op's own kernel, which takes 64 columns at a time
+PLACES = [
+    (lambda: w.fully_connected_workload(301, 301, 301, realistic=True), "padded 0 1 igemm_direct_i8 as it is"), (lambda: w.fully_connected_workload(77, 500, 500, realistic=True), "padded 0 1 igemm_direct_i8 as it is"),
+    (lambda: w.conv2d_workload(N=3, H=9, W=8, C=61, O=61, realistic=True), "padded 0 1 igemm_direct_i8 as it is"),
+    (lambda: w.fully_connected_workload(400, 63, 63, realistic=True), "record 0 1 igemm_direct_i8"), (lambda: w.fully_connected_workload(400, 64, 64, realistic=True), "record 0 1 igemm_direct_i8"),
+]
+PLACE_IDS = [c[0]().name for c in PLACES]
+
+
+def in_one_binding(wl):
+    """The same op from binding 0 to binding 0."""
+    p = Program()
+    x = p.binding(0, wl.inputs[0].shape)
+    attrs = dict(wl.attrs)
+    weights, scale_bias = attrs.pop("weights"), attrs.pop("scale_bias")
+    if len(wl.inputs[0].shape) == 2:
+        p.fully_connected(x, weights, scale_bias, init=x, **attrs)
+    else:
+        p.conv2d(x, weights, scale_bias, init=x, nhwc_input=attrs.pop("nhwc"), **attrs)
+    return w.Workload(wl.name, p, wl.inputs, [], wl.ops, wl.bytes, wl.attrs)
+
+
+@pytest.mark.parametrize("make,line", PLACES, ids=PLACE_IDS)
+def test_rows_that_are_written_over(plan, make, line):
+    wl = make()
+    assert plan(wl, (A, B)) == [line] and plan(wl, (A, A)) == [line + " shared"] and plan(wl, (A, A + wl.inputs[0].nbytes - 16)) == [line + " shared"]
+    (alone,) = plan(in_one_binding(wl), (A,))
+    assert alone in ((line[:-len(" as it is")], "padded 0 1") if line.startswith("padded") else ("record 0 1",)), alone
+
+
 def blocks(count, **kw):
     """`count` blocks beside one another in a program, block i from binding 2 i to binding 2 i + 1."""
     wls = [block(seed=1080 + i, **kw) for i in range(count)]
@@ -102,6 +132,33 @@ def test_gpu_blocks_in_place(device, add, how, monkeypatch):
         exe.close()
         for p in ptrs + other:
             device.free(p)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("make,line", PLACES, ids=PLACE_IDS)
+@pytest.mark.parametrize("bindings", [2, 1])
+def test_gpu_rows_that_are_written_over(device, make, line, bindings):
+    wl = make()
+    print("[gpu-case]", wl.name, "over its input", bindings, flush=True)
+    x, want = wl.inputs[0], oracle_eval(wl)[0]
+    exe = Executable(device, (wl if bindings == 2 else in_one_binding(wl)).program.serialize())
+    ptr, other = device.upload(x), device.upload(x)
+    try:
+        for how in (exe.run_device, exe.enqueue_device_noalloc):
+            runtime.check(runtime.lib().thip_device_h2d(device.handle, ptr, x.ctypes.data, x.nbytes))
+            device.synchronize()
+            how([ptr] * bindings, [x.nbytes] * bindings)
+            exe.wait()
+            assert_bit_exact(device.download(ptr, wl.outputs[0][0], np.int8), want.reshape(wl.outputs[0][0]), wl.name)
+        if bindings == 2:
+            runtime.check(runtime.lib().thip_device_h2d(device.handle, ptr, x.ctypes.data, x.nbytes))
+            device.synchronize()
+            exe.run_device([ptr, other], [x.nbytes] * 2)
+            assert_bit_exact(device.download(other, wl.outputs[0][0], np.int8), want.reshape(wl.outputs[0][0]), wl.name)
+    finally:
+        exe.close()
+        device.free(ptr)
+        device.free(other)
 
 
 @pytest.mark.gpu

@@ -583,9 +583,14 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
     }
     case kStepPadded: {
         uint8_t *const *buffers = &e->stepBuffers[2 * (size_t)(&s - e->steps.data())];
-        if (s.rows > 0) err = launchPadRows((const int8_t *)resolve(e, e->ops[s.first].in0, bp), (int8_t *)buffers[0], s.rows, s.from, s.to, ctx);
-        if (err == hipSuccess) return launchOp(e, s.first, s.op, bp, ctx, scratch, buffers, s.route, 0, true);
-        break;
+        const bool shared = s.asIs && !ctx.name && writesWhatItReads(viewOf(e), s, bp);
+        if (shared && !buffers[0]) return recordByRecord();  // no memory for the copy
+        if (s.asIs && !shared) return launchOp(e, s.first, s.op, bp, ctx, scratch, buffers, s.route, 0, true);
+        err = launchPadRows((const int8_t *)resolve(e, e->ops[s.first].in0, bp), (int8_t *)buffers[0], s.rows, s.from, s.to, ctx);
+        if (err != hipSuccess) break;
+        DescOp op = s.op;
+        op.in0 = DescRef{kSpacePlan, 0, 0};
+        return launchOp(e, s.first, op, bp, ctx, scratch, buffers, s.route, 0, true);
     }
     case kStepDecChain: {
         if (!ctx.name && apart) return recordByRecord();
@@ -602,7 +607,10 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
         err = launchDecChain(a, e->device->computeUnits, ctx);
         break;
     }
-    default: return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch, nullptr, s.route, s.blocked, true);
+    default: {
+        const bool shared = s.route == kIgemmDirect && !ctx.name && writesWhatItReads(viewOf(e), s, bp);
+        return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch, nullptr, shared ? kIgemmOwnTile : s.route, s.blocked, true);
+    }
     }
     if (err != hipSuccess) return fail(THIP_INTERNAL, "ops %u .. %u: launch failed: %s", s.first, s.first + s.count - 1, hipGetErrorString(err));
     return THIP_OK;
@@ -934,9 +942,15 @@ static bool addStep(thip_executable_t *e, Step &&planned) {
     hipError_t err = hipSuccess;
     if (step.kind == kStepPadded) {
         uint8_t **buffers = &e->stepBuffers[e->stepBuffers.size() - 2];
-        const size_t rows = (size_t)step.rows * step.to, bytes = rows + step.constants.size();
-        if (e->tuning.stepBytes >= 0 && (long long)bytes > e->tuning.stepBytes) err = hipErrorOutOfMemory;
-        if (err == hipSuccess && rows > 0) err = hipMalloc((void **)&buffers[0], rows);
+        const size_t rows = (size_t)step.rows * step.to, constants = step.constants.size();
+        auto room = [e](size_t bytes) { return e->tuning.stepBytes < 0 || (long long)bytes <= e->tuning.stepBytes; };
+        if (step.copies) err = room(rows + constants) ? hipMalloc((void **)&buffers[0], rows) : hipErrorOutOfMemory;
+        if (step.asIs && err != hipSuccess) {  // goes without
+            (void)hipGetLastError();
+            buffers[0] = nullptr;
+            err = hipSuccess;
+        }
+        if (err == hipSuccess && !room(constants)) err = hipErrorOutOfMemory;
         if (err == hipSuccess) err = hipMalloc((void **)&buffers[1], step.constants.size());
         if (err == hipSuccess) err = hipMemcpy(buffers[1], step.constants.data(), step.constants.size(), hipMemcpyHostToDevice);
         std::vector<uint8_t>().swap(step.constants);
@@ -974,7 +988,7 @@ static bool addStep(thip_executable_t *e, Step &&planned) {
         for (auto &ptr : placeholder) ptr = (uint8_t *)(uintptr_t)0x1000000;
         char name[96] = "";
         if (launchStep(e, step, placeholder, LaunchCtx{nullptr, &e->tuning, name, sizeof(name), e->device->ordinal}) == THIP_OK) {
-            if (step.kind == kStepPadded && step.rows > 0) e->launchNames.push_back("pad_rows_i8");
+            if (step.kind == kStepPadded && !step.asIs) e->launchNames.push_back("pad_rows_i8");
             e->launchNames.push_back(name[0] ? name : opKernelName(e->ops[step.first]));
             return true;
         }

@@ -37,6 +37,13 @@ static std::vector<uint32_t> tempUses(const DescriptorView &v, uint32_t first, u
     return uses;
 }
 
+// Whether a GEMM-shaped record stores into the bytes of the buffer that it reads.
+static bool inPlace(const DescOp &op) {
+    if (!sameBuffer(op.in0, op.out)) return false;
+    const uint64_t in = (uint64_t)op.N * op.H * op.W * op.C, out = (uint64_t)op.M * op.Nn * elemBytes(op.out_dtype);
+    return op.in0.offset < op.out.offset + out && op.out.offset < op.in0.offset + in;
+}
+
 // The value all `n` words of a constant have; false where they differ or are none.
 static bool uniformWords(const DescriptorView &v, const DescRef &r, int n, int32_t *out) {
     if (r.space != kSpaceConst) return false;
@@ -200,7 +207,7 @@ static bool paddingPays(const DescOp &g, int64_t rows, int64_t Cp, int64_t K) {
 // where K is long enough for the worse loads to cost that launch: 3x2801 -> 1608 - / 6.2 / 6.6 (few rows have a faster kernel behind the copy), 5x5
 // 19x19x387 -> 134 452 / 18.2 / 19.7.
 static bool asIsBetter(const DescriptorView &v, const Tuning &tuning, const DescOp &g, const DescOp &op) {
-    if (tuning.padRows == 0 || tuning.padRows == 1 || g.kind != kKindIgemm || g.loader != kLoaderGather) return false;
+    if (tuning.padRows == 0 || tuning.padRows == 1 || g.kind != kKindIgemm || g.loader != kLoaderGather || inPlace(g)) return false;
     return igemmDirectBetter(raggedArgs(v, op, g.C, [&](const DescRef &r) { return plannedAt(v, r); })) && (tuning.padRows == 2 || (gatherTime(g) > 4.0 && g.K <= (g.M <= kFcSkinnyMaxRows ? 2500 : 9000)));
 }
 
@@ -273,9 +280,11 @@ static bool matchPadded(const DescriptorView &v, const Tuning &tuning, uint32_t 
     s->kind = kStepPadded;
     s->first = first;
     s->count = 1;
-    s->rows = asIs ? 0 : rows;
+    s->rows = rows;
     s->from = (int32_t)C;
     s->to = (int32_t)Cp;
+    s->asIs = asIs;
+    s->copies = !asIs || (g.in0.space == kSpaceBinding && g.out.space == kSpaceBinding && g.in0.index != g.out.index);
     s->op = op;
     return true;
 }
@@ -476,11 +485,12 @@ static bool matchDecChain(const DescriptorView &v, const Tuning &tuning, uint32_
     return true;
 }
 
-// The kernel that is ahead for a GEMM-shaped record.
+// The kernel that is ahead for a GEMM-shaped record.  In place a record has its own, whose tiles take 64 columns or more: those of igemm_direct_i8 take 32,
+// and others of the same rows may still be reading where one stores.
 static IgemmRoute igemmRoute(const DescriptorView &v, const Tuning &tuning, const DescOp &op) {
     const IgemmArgs a = igemmArgs(v, op, [&](const DescRef &r) { return plannedAt(v, r); });
     if (op.loader == kLoaderGather && op.KH == 1 && op.KW == 1 && zerosBehindRows(v, op) && asIsBetter(v, tuning, op, op)) return kIgemmDirect;
-    return igemmDirectBetter(a) ? kIgemmDirect : convPatchBetter(a) ? kIgemmPatch : !tuning.noK128 && igemmWideBetter(a, op.variant) ? kIgemmWide : kIgemmOwnTile;
+    return !inPlace(op) && igemmDirectBetter(a) ? kIgemmDirect : convPatchBetter(a) ? kIgemmPatch : !tuning.noK128 && igemmWideBetter(a, op.variant) ? kIgemmWide : kIgemmOwnTile;
 }
 
 // A replay starts about 5 us later than a launch behind another, and costs the host 12 - 20 us in place of 3 per launch.  Launches that
@@ -587,7 +597,7 @@ std::vector<Step> planSteps(const DescriptorView &v, const Tuning &tuning) {
         if (s.kind == kStepExpandDw) matchBlock(v, tuning, uses, &s);
         const DescOp *op = s.kind == kStepRecord ? &v.ops[i] : s.kind == kStepPadded ? &s.op : nullptr;
         if (s.kind == kStepExpandDw && s.count == 3) op = &v.ops[i + 2];
-        s.route = plain || !op || op->kind != kKindIgemm ? kIgemmOwnTile : s.kind == kStepPadded && s.rows == 0 ? kIgemmDirect : igemmRoute(v, tuning, *op);
+        s.route = plain || !op || op->kind != kKindIgemm ? kIgemmOwnTile : s.kind == kStepPadded && s.asIs ? kIgemmDirect : igemmRoute(v, tuning, *op);
         i += s.count;
         steps.push_back(std::move(s));
     }

@@ -39,11 +39,12 @@ struct Step {
     int32_t batches;
     int64_t a_stride, b_stride, out_stride;
     int32_t bias, scale;
-    // kStepPadded: rows of `from` bytes padded to `to`, and the record that reads them; no rows: a record that reads them as they are, its
-    // weights alone padded (igemm_direct_i8).  Its operands of space kSpacePlan are the step's own: index 0 the padded rows, index 1
-    // `constants` (on the device).
+    // kStepPadded: rows of `from` bytes padded to `to`, and the record that reads them; or (asIs) a record that reads them as they are, its
+    // weights alone padded (igemm_direct_i8), and that reads them padded only where its result lies on them (copies).  Its operands of space
+    // kSpacePlan are the step's own: index 0 the padded rows, index 1 `constants` (on the device).
     int64_t rows;
     int32_t from, to;
+    bool asIs, copies;
     DescOp op;
     std::vector<uint8_t> constants;
     // kStepRecord, grouped linears and small matmuls: DecBlocked, the intermediates that lie in blocks of columns
