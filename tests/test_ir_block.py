@@ -8,9 +8,10 @@ from torq_compiler_amd import Program, workloads as w
 pytestmark = pytest.mark.gpu
 
 
-def block(N, H, W, C, E, O, stride, pad=(1, 1, 1, 1), add=None, first=None, zp=7, lowest=-128, seed=1070):
+def block(N, H, W, C, E, O, stride, pad=(1, 1, 1, 1), add=None, first=None, zp=7, lowest=-128, seed=1070, steep=None):
     """widen (pointwise, or `first` = (window, stride, pad) over few channels) -> depthwise 3x3 -> narrow, and with `add` (0 or 1: the place
-    of the block's input among the add's operands) the residual add; the intermediates leave no launch."""
+    of the block's input among the add's operands) the residual add; the intermediates leave no launch.  `steep`: the scale of a channel of the
+    depthwise op, at 1/2 and above a shift below 32 for all of them."""
     rng = np.random.default_rng(seed)
     x = rng.integers(-128, 128, size=(N, H, W, C)).astype(np.int8)
     layers = []
@@ -18,7 +19,10 @@ def block(N, H, W, C, E, O, stride, pad=(1, 1, 1, 1), add=None, first=None, zp=7
     for op, shape, fan, zin, zout, low in (("conv2d", (E, C, k, k), C * k * k, -3, -120, -120), ("depthwise_conv2d", (E, 1, 3, 3), 9, -120, -117, -117),
                                            ("conv2d", (O, E, 1, 1), E, -117, zp, lowest)):
         wt = rng.integers(-127, 128, size=shape).astype(np.int8)
-        mult, sh = w.quantize_multiplier(60 / (np.sqrt(fan) * 5400) * rng.uniform(0.8, 1.2, shape[0]))
+        scales = 60 / (np.sqrt(fan) * 5400) * rng.uniform(0.8, 1.2, shape[0])
+        if op == "depthwise_conv2d" and steep is not None:
+            scales[shape[0] // 2] = steep
+        mult, sh = w.quantize_multiplier(scales)
         sb, sf = w.derive_scale_bias(mult, sh, rng.integers(-4000, 4000, shape[0]), wt, zin)
         attrs = dict(input_zp=zin, output_zp=zout, output_min=low, output_max=127, shift_factor=sf)
         attrs.update(pad=(0, 0, 0, 0), stride=(1, 1))
@@ -69,6 +73,19 @@ def test_block(device, kw, monkeypatch):
     launched = []
     got, _ = run_on_gpu(device, wl, via="device", launched=launched)
     assert families(launched) == ["ir_block_i8"], launched
+    assert_bit_exact(got[0], oracle_network(wl), wl.name)
+
+
+@pytest.mark.parametrize("kw", CASES, ids=lambda kw: "x".join(str(v) for v in kw.values()))
+@pytest.mark.parametrize("steep", [0.6, 100.0])
+def test_block_with_a_steep_channel(device, kw, steep, monkeypatch):
+    """The kernel's other depthwise requant, of a shift below 32 for all channels."""
+    monkeypatch.setenv("THIP_IR_BLOCK", "1")
+    wl = block(steep=steep, **kw)
+    print("[gpu-case]", wl.name, steep, flush=True)
+    launched = []
+    got, _ = run_on_gpu(device, wl, via="device", launched=launched)
+    assert len(launched) == 1 and launched[0].startswith("ir_block_i8<") and launched[0].endswith(",3>"), launched
     assert_bit_exact(got[0], oracle_network(wl), wl.name)
 
 
