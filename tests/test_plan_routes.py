@@ -124,6 +124,30 @@ def test_ragged_channels_are_padded_where_that_is_measured_ahead(plan, make, pad
     assert [s.split()[0] for s in plan(make())] == ["padded" if padded else "record"]
 
 
+def with_output_zp(wl, record, zp):
+    """The serialised program, a record's zero point set by hand."""
+    class Changed:
+        @staticmethod
+        def serialize():
+            blob = bytearray(wl.program.serialize())
+            d = desc_interp.Descriptor(bytes(blob))
+            ops = np.frombuffer(blob, dtype=desc_interp.OP, count=len(d.ops), offset=int(d.header["ops_offset"]))
+            ops["output_zp"][record] = zp
+            return bytes(blob)
+
+    return w.Workload(wl.name, Changed, wl.inputs, wl.outputs, wl.ops, wl.bytes, wl.attrs)
+
+
+@pytest.mark.parametrize("steep", [None, 0.6])
+@pytest.mark.parametrize("zp,taken", [(-32768, True), (32767, True), (-32769, False), (32768, False), (1 << 30, False), (-(1 << 31), False)])
+def test_blocks_take_zero_points_that_fold_into_the_rounding(plan, steep, zp, taken, monkeypatch):
+    """The builder writes no others; a descriptor from elsewhere may."""
+    from test_ir_block import block
+    monkeypatch.setenv("THIP_IR_BLOCK", "1")
+    lines = plan(with_output_zp(block(N=1, H=12, W=12, C=16, E=48, O=32, stride=1, steep=steep), 1, zp))
+    assert (lines[0].split()[:3] == ["ir_expand_dw_i8", "0", "3"]) == taken, lines
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("make,offset,route", CASES, ids=IDS)
 def test_gpu_result_at_offset(device, make, offset, route):

@@ -355,7 +355,8 @@ static bool packedRequant(const Requant &rq, int mostShift) {
 
 // The depthwise op's 9 taps leave scales that start above 1/2 here and there, for all channels of an op a shift below 32 then: mode 3.
 static bool preShiftedRequant(const Requant &rq) {
-    return rq.shift >= 3 && rq.shift < 32 && rq.pre_shift == 33 - rq.shift && rq.t0_clamp == 0 && rq.out_min >= -128 && rq.out_max <= 127 && rq.out_min <= rq.out_max;
+    return rq.shift >= 3 && rq.shift < 32 && rq.pre_shift == 33 - rq.shift && rq.t0_clamp == 0 && rq.out_min >= -128 && rq.out_max <= 127 && rq.out_min <= rq.out_max && rq.out_zp >= -32768 &&
+           rq.out_zp <= 32767;
 }
 
 // The time of a launch, us: of a workgroup alone on its CU a start and its chunks, each of which costs something whatever its size, then a share a tile
