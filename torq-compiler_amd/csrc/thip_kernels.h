@@ -201,7 +201,7 @@ struct IrBlockArgs {
     // CKH > 0: as in IrExpandDwArgs
     int32_t CKH, CS, CPT, CPL, IH, IW, IC, runBytes, czp;
     int64_t xBytes;
-    int32_t addFolded, columnBlocks, blockColumns, strips, stripRows, segments, segmentRows, cellRows, cellCols, regionColumns, blocks;  // planIrBlock sets these
+    int32_t addFolded, columnBlocks, blockColumns, strips, stripRows, segments, segmentRows, cellRows, cellCols, regionColumns;  // planIrBlock sets these
 };
 // Checks the arguments and sets what is the launch's own to choose; false where the kernel does not take them.
 bool planIrBlock(IrBlockArgs *a);

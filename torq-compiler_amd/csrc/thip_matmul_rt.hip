@@ -4,10 +4,6 @@
 
 namespace thip {
 
-struct __attribute__((packed)) UnalignedWord {
-    uint32_t v;
-};
-
 // ---------------------------------------------------------------------------
 // igemm_rt_i8: out[b][m][n] = R1(sum_k A[b][m][k] * B[b][k][n]) with ONE (bias, scale) pair, int8 / int16 / int32 results.
 //
@@ -72,7 +68,7 @@ __global__ __launch_bounds__(256, 2) void igemm_rt_i8(MatmulRtArgs p) {
         int off = bBase + (k0 < p.K ? k0 : p.K) * p.N;
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            rb[r] = ((const UnalignedWord *)(p.B + (uint32_t)(off < bLast ? off : bLast)))->v;
+            rb[r] = ((const UnalignedU32 *)(p.B + (uint32_t)(off < bLast ? off : bLast)))->v;
             off = off < bLast ? off + p.N : off;
         }
     };
