@@ -30,8 +30,9 @@ int main(int argc, char **argv) {
     const std::vector<Step> steps = planSteps(v, tuningFromEnvironment());
     const char *kinds[] = {"record", "ir_expand_dw_i8", "padded", "igemm_rt_i8", "dec_chain"}, *routes[] = {"", " igemm_direct_i8", " conv_patch_i8", " igemm_dense_k128_i8"};
     for (const Step &s : steps) {
-        printf("%s %u %u%s", kinds[s.kind], s.first, s.count, routes[s.route]);
-        if (s.asIs) printf(" as it is");
+        printf("%s %u %u%s", s.kind == kStepExpandDw && s.count == 3 ? "ir_block_i8" : kinds[s.kind], s.first, s.count, routes[s.route]);
+        // the input's rows in no whole 16-byte chunks, read all the same
+        if (s.asIs || (s.kind == kStepRecord && s.route == kIgemmDirect && v.ops[s.first].loader == kLoaderGather)) printf(" as it is");
         if (s.blocked) printf(" blocked %d", s.blocked);
         if (!bindings.empty() && writesWhatItReads(v, s, bindings.data())) printf(" shared");
         puts("");

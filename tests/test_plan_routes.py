@@ -124,6 +124,35 @@ def test_ragged_channels_are_padded_where_that_is_measured_ahead(plan, make, pad
     assert [s.split()[0] for s in plan(make())] == ["padded" if padded else "record"]
 
 
+AS_IT_IS = " igemm_direct_i8 as it is"
+FC, CONV = w.fully_connected_workload, w.conv2d_workload
+LINES = list(zip([c[0] for c in RAGGED], [["padded 0 1" + AS_IT_IS]] * 2 + [["padded 0 1"], ["padded 0 1" + AS_IT_IS], ["padded 0 1 conv_patch_i8"]] + [["record 0 1"]] * 4 + [["record 0 1" + AS_IT_IS]])) + [
+    # few rows: to K = 2500; more: to 9000
+    (lambda: FC(9, 2500, 100), ["padded 0 1" + AS_IT_IS]), (lambda: FC(9, 2501, 100), ["padded 0 1"]), (lambda: FC(100, 8999, 32), ["padded 0 1" + AS_IT_IS]), (lambda: FC(100, 9001, 32), ["padded 0 1 igemm_direct_i8"]),
+    (lambda: CONV(N=1, H=19, W=19, C=387, O=134, KH=5, KW=5, pad=(2, 2, 2, 2)), ["padded 0 1 igemm_direct_i8"]), (lambda: CONV(N=1, H=19, W=19, C=359, O=134, KH=5, KW=5, pad=(2, 2, 2, 2)), ["padded 0 1" + AS_IT_IS]),
+    # 256 tiles of 32 x 32, and one row more
+    (lambda: FC(256, 77, 1024), ["padded 0 1" + AS_IT_IS]), (lambda: FC(257, 77, 1024), ["padded 0 1"]),
+    # a gather of one k-tile: in single bytes, in pieces of eight
+    (lambda: FC(40, 63, 63), ["record 0 1" + AS_IT_IS]), (lambda: FC(40, 56, 63), ["record 0 1"]), (lambda: FC(9, 100, 2303), ["record 0 1" + AS_IT_IS]),
+]
+
+
+@pytest.mark.parametrize("make,lines", LINES, ids=[c[0]().name for c in LINES])
+def test_ragged_rows_by_each_way(plan, make, lines):
+    assert plan(make()) == lines
+
+
+@pytest.mark.parametrize("kw,taken", [
+    (dict(N=1, H=224, W=224, C=3, E=32, O=16, stride=1, first=(3, 2, (0, 1, 0, 1))), True), (dict(N=1, H=112, W=112, C=16, E=96, O=32, stride=2, pad=(0, 1, 0, 1)), False),
+    (dict(N=4, H=112, W=112, C=16, E=96, O=32, stride=2, pad=(0, 1, 0, 1)), True), (dict(N=8, H=28, W=28, C=32, E=192, O=32, stride=1), False), (dict(N=64, H=28, W=28, C=32, E=192, O=32, stride=1), True),
+    (dict(N=200, H=14, W=14, C=64, E=384, O=64, stride=1), False),
+], ids=lambda v: "x".join(str(x) for x in v.values()) if isinstance(v, dict) else str(v))
+def test_blocks_are_one_launch_where_that_is_estimated_ahead(plan, kw, taken):
+    from test_ir_block import block
+    lines = plan(block(**kw))
+    assert (lines == ["ir_block_i8 0 3"]) if taken else [s.split()[:3] for s in lines] == [["ir_expand_dw_i8", "0", "2"], ["record", "2", "1"]], lines
+
+
 def with_output_zp(wl, record, zp):
     """The serialised program, a record's zero point set by hand."""
     class Changed:
@@ -145,7 +174,7 @@ def test_blocks_take_zero_points_that_fold_into_the_rounding(plan, steep, zp, ta
     from test_ir_block import block
     monkeypatch.setenv("THIP_IR_BLOCK", "1")
     lines = plan(with_output_zp(block(N=1, H=12, W=12, C=16, E=48, O=32, stride=1, steep=steep), 1, zp))
-    assert (lines[0].split()[:3] == ["ir_expand_dw_i8", "0", "3"]) == taken, lines
+    assert (lines[0].split()[:3] == ["ir_block_i8", "0", "3"]) == taken, lines
 
 
 @pytest.mark.gpu

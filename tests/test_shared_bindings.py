@@ -38,7 +38,7 @@ def test_a_block_in_place_is_told_from_one_that_is_not(plan, add, monkeypatch):
     wl = block(add=add, **WHOLE)
     size = wl.inputs[0].nbytes
     for out, shared in ((B, ""), (A, " shared"), (A + size - 16, " shared"), (A - size + 16, " shared"), (A + size, ""), (A - size, "")):
-        assert [s.replace(" igemm_direct_i8", "") for s in plan(wl, (A, out))] == ["ir_expand_dw_i8 0 3" + shared], hex(out)
+        assert [s.replace(" igemm_direct_i8", "") for s in plan(wl, (A, out))] == ["ir_block_i8 0 3" + shared], hex(out)
 
 
 def test_other_runs_of_records_in_place(plan):
@@ -53,7 +53,7 @@ def test_other_runs_of_records_in_place(plan):
 PLACES = [
     (lambda: w.fully_connected_workload(301, 301, 301, realistic=True), "padded 0 1 igemm_direct_i8 as it is"), (lambda: w.fully_connected_workload(77, 500, 500, realistic=True), "padded 0 1 igemm_direct_i8 as it is"),
     (lambda: w.conv2d_workload(N=3, H=9, W=8, C=61, O=61, realistic=True), "padded 0 1 igemm_direct_i8 as it is"),
-    (lambda: w.fully_connected_workload(400, 63, 63, realistic=True), "record 0 1 igemm_direct_i8"), (lambda: w.fully_connected_workload(400, 64, 64, realistic=True), "record 0 1 igemm_direct_i8"),
+    (lambda: w.fully_connected_workload(400, 63, 63, realistic=True), "record 0 1 igemm_direct_i8 as it is"), (lambda: w.fully_connected_workload(400, 64, 64, realistic=True), "record 0 1 igemm_direct_i8"),
 ]
 PLACE_IDS = [c[0]().name for c in PLACES]
 
