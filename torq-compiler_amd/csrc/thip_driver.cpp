@@ -186,11 +186,12 @@ static thip_status_t launchOp(thip_executable_t *e, uint32_t i, const DescOp &op
     case kKindIgemm: {
         auto at = [&](const DescRef &r) { return resolve(e, r, bp); };
         const bool asIs = route == kIgemmDirect && e->ops[i].loader == kLoaderGather && op.in0.space != kSpacePlan;
-        IgemmArgs a = asIs ? raggedArgs(viewOf(e), op, e->ops[i].C, at) : igemmArgs(viewOf(e), op, at);
-        a.any_rows = planned && !e->tuning.plainRecords;
+        const IgemmArgs a = asIs ? raggedArgs(viewOf(e), op, e->ops[i].C, at) : igemmArgs(viewOf(e), op, at);
+        LaunchCtx own = ctx;
+        own.any_rows = planned && !e->tuning.plainRecords;
         if (route == kIgemmDirect) err = launchIgemmDirect(a, ctx);
         else if (route == kIgemmPatch) err = launchConvPatch(a, ctx);
-        else err = launchIgemm(a, op.variant, ctx, route == kIgemmWide);
+        else err = launchIgemm(a, op.variant, own, route == kIgemmWide);
         break;
     }
     case kKindFcSkinny: {

@@ -1261,7 +1261,7 @@ static hipError_t launchIgemmDense(const IgemmArgs &a, const LaunchCtx &ctx) {
     }
     if (direct) return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 1, false, CONV, BK, HALF>(a, ctx);
     if (inRegisters && wide) return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 2, false, CONV, BK, HALF>(a, ctx);
-    if (results8 && !wholeRows && a.any_rows && plain) return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 3, false, CONV, BK, HALF>(a, ctx);
+    if (results8 && !wholeRows && ctx.any_rows && plain) return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 3, false, CONV, BK, HALF>(a, ctx);
     return launchIgemmDenseE<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, 0, false, CONV, BK, HALF>(a, ctx);
 }
 

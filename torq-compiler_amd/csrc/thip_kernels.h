@@ -83,6 +83,7 @@ struct LaunchCtx {
     char *name;
     size_t name_capacity;
     int ordinal;  // the stream's device, which is the current one
+    bool any_rows = false;  // the ring kernels: int8 results of rows of any length and alignment are requantised in registers too
 };
 
 struct IgemmArgs {
@@ -95,8 +96,6 @@ struct IgemmArgs {
     int32_t M, N, K, Kp, Np;
     int32_t H, W, C, OH, OW, SH, SW, PT, PL;
     int32_t KH, KW;         // window loader only
-    int32_t any_rows;       // the ring kernels: int8 results of rows of any length and alignment are requantised in registers too
-    int32_t row_bytes;      // igemm_direct_i8 only: what a pixel of A takes where C is that rounded up to whole 16-byte chunks (0: C)
     int32_t input_zp;
     int32_t out_dtype;
     int64_t a_bytes;        // size of A in bytes (the run loader keeps its 16-byte loads inside it)
@@ -110,7 +109,11 @@ struct IgemmArgs {
     Requant arq;
     int32_t stream_guarded;  // pixel-streaming kernel: keep every load and store under its bounds check (tests, tuning)
     int32_t stream_stage;    // pixel-streaming kernel: results leave through a per-wave LDS slice as whole rows (its launcher sets it)
+    int32_t row_bytes;       // igemm_direct_i8 only: what a pixel of A takes where C is that rounded up to whole 16-byte chunks (0: C)
 };
+// igemm_direct_i8 reads its divisors, which follow these, in two steps, the 64-byte line of the later ones with the first step's.  With eight
+// bytes more that line is a trip to memory of its own (3x3, one image, 112x112x32 -> 64 4.13 -> 4.31 us, 28x28x128 -> 128 4.85 -> 5.01).
+static_assert(sizeof(IgemmArgs) == 224, "where the kernels' further arguments lie");
 
 // Tile configurations of the igemm kernel.
 enum IgemmVariant : uint32_t {
