@@ -205,10 +205,11 @@ static bool planConvPatch(const IgemmArgs &a, ConvPatchPlan *q) {
     q->cols = (int)cols;
     long long most = room / rowBytes - a.KH + 1;
     if (most > a.OH) most = a.OH;
-    // a strip per CU where the images give as many
-    long long strips = (a.OH + most - 1) / most;
-    const long long wanted = (256 + images - 1) / images;
-    if (strips < wanted) strips = wanted < a.OH ? wanted : a.OH;
+    // As many strips as fill the CUs without beginning another round (a strip for each CU
+    // at least, rounded up, left a few CUs two: 605 drawn convolutions took 1.15 times as long, 53x53x64 -> 89, batch 19, 16.4 us in 266 strips, 11.7 in 209).
+    const long long rounds = (images * ((a.OH + most - 1) / most) + 255) / 256;
+    long long strips = 256 * rounds / images;
+    if (strips > a.OH) strips = a.OH;
     q->rows = (int)((a.OH + strips - 1) / strips);
     q->stripsPerImage = (a.OH + q->rows - 1) / q->rows;
     const long long all = images * q->stripsPerImage;
@@ -225,9 +226,15 @@ static bool planConvPatch(const IgemmArgs &a, ConvPatchPlan *q) {
 // and where the rule below says no:
 //   few pixels, whose strips are few or low   30x30x96 -> 96, 32 8.2 / 9.8; 160x160x64 -> 64, 2 (two rows each) 7.6 / 8.7
 //   many channels out, few taps, many in      56x56x48 -> 128, 20 9.8 / 12.0; 2x2 100x100x96 -> 64, 20 15.2 / 21.5; 64x64x128 -> 64, 32 19.2 / 22.6
+//   a second round of low strips              5x5 46x46x80 -> 33, 27 16.7 / 24.9; 7x7 40x40x80 -> 7, 40 26.0 / 42.4; 5x5 105x105x64 -> 53, 7 19.1 / 21.4
+//   rows that only rounding up makes three    104x104x16 -> 45, 5 6.2 / 7.5
+// Over 605 drawn ones (16 .. 112 channels in, 1 .. 96 out, windows of 3, 5 and 7) the choice costs 1.2 % of the better one's time, always the ring kernel 20 %, always this one 3 %.
 bool convPatchBetter(const IgemmArgs &a) {
     ConvPatchPlan q;
-    return a.C <= 112 && a.KH * a.KW >= 9 && a.M >= 49152 && planConvPatch(a, &q) && q.rows * a.KW >= 9;
+    if (a.C > 112 || a.KH * a.KW < 9 || a.M < 49152 || !planConvPatch(a, &q)) return false;
+    const int rounds = (q.strips + 255) / 256;
+    if (q.rows * a.KW < 9 || (long long)(a.M / a.OW) * a.KW < 1600LL * rounds) return false;
+    return rounds == 1 || ((q.rows >= a.KH || q.rows * a.OW > 160) && (a.N <= 32 || q.rows >= (a.KH < 4 ? a.KH : 4)));
 }
 
 template <int NB, bool ANY>
