@@ -50,3 +50,14 @@ def test_nothing_beyond_k_reaches_a_result(device, monkeypatch):
 def test_tile_by_shape(device, rows, k, columns, tile):
     _, kernels = run_on_gpu(device, w.fully_connected_bf16_workload(rows, k, columns), via="device")
     assert kernels[0].startswith("fc_bf16<%s," % (tile or 4)), kernels
+
+
+@pytest.mark.parametrize("tile,columns,runs", [(1, 264, 0), (1, 262, 0), (3, 264, 0), (3, 262, 1), (4, 264, 0), (4, 263, 1), (5, 264, 1), (5, 261, 1)])
+def test_how_results_are_stored(device, tile, columns, runs, monkeypatch):
+    """Runs of rows through LDS (2 in the label's last number) for ragged columns of the wider tiles and for the widest."""
+    monkeypatch.setenv("THIP_FC_TILE", str(tile))
+    wl = w.fully_connected_bf16_workload(300, 136, columns)
+    print("[gpu-case]", tile, wl.name, flush=True)
+    got, kernels = run_on_gpu(device, wl, via="device")
+    assert_bf16_close(got[0], oracle_eval(wl)[0], wl.name + " (gpu)", magnitude=_magnitude(wl))
+    assert kernels[-1].endswith(",%d>" % (1 + 2 * runs)), kernels

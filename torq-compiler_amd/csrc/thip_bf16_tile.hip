@@ -30,10 +30,13 @@ __device__ __forceinline__ uint32_t packBf16(float lo, float hi) {
 // packed weights have in memory: FRAG weights go to LDS as they are, 4 KiB of 32 columns x 64 k at a time, and a
 // fragment read is 1 KiB in lane order.  Row-major weights (a run-time operand) are staged like the activations.
 //
-// The weights are the MFMA's row operand: register 4 q + e of lane (r, h) is out[m = r][n = 8 q + 4 h + e].  The results go through LDS, each
+// The weights are the MFMA's row operand: register 4 q + e of lane (r, h) is out[m = r][n = 8 q + 4 h + e].  Two
+// v_permlane32_swap give a lane 8 neighbouring columns of a row: one 16-byte store, at any alignment.  RUNS: the results go through LDS instead, each
 // wave's by itself, so that a store covers whole runs of a row: columns that are no whole eight, whose rows begin anywhere, cost
 // what others do (2048 x 1152 -> 6911 67.7 us in single elements, 43.3 in unaligned 16-byte pieces of a lane's own row, 35.0 in runs; 1649 x
-// 288 -> 4747 28.6, 13.5, 12.0; 2608 x 1024 -> 2530 33.7, 20.1, 19.9; 2048 x 1152 -> 6912 34.3 in aligned pieces, 34.0).
+// 288 -> 4747 28.6, 13.5, 12.0; 2608 x 1024 -> 2530 33.7, 20.1, 19.9).  Where a wave's columns are 32 that way round costs more than it brings (654 x
+// 1736 -> 208 9.0, 9.3), and for aligned rows the 128 x 128 tiles lose by it (1267 x 384 -> 5584 10.6, 11.3; 2042 x 176 -> 5760 11.8, 12.9; 1993 x
+// 768 -> 5808 24.8, 26.1) while 256 x 256 ones do not (2048 x 1152 -> 6912 34.3, 34.0; 14 others alike): launchTile.
 //
 // KG groups of waves share a workgroup's outputs and take every KG-th k-tile each, with a ring of their own; their sums
 // meet in LDS (few tiles under a long K: more loads in flight per CU).
@@ -42,7 +45,7 @@ __device__ __forceinline__ uint32_t packBf16(float lo, float hi) {
 // the XCD's L2, reach 138; 0.86 us of MFMA work), with the launch, the ring fill and 28 MB of output at the end next to it: 2048 x 1152 -> 6912 takes 34.0 us (960 TFLOP/s).  Eight waves
 // on the 256 x 256 tile rather than four: 35.7 -> 34.4 us, and the epilogue of a short K 13.0 -> 9.1.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, int KG, bool FRAG>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, int KG, bool FRAG, bool RUNS>
 __global__ __launch_bounds__(WAVES_M *WAVES_N *KG * 64, BLOCKS_PER_CU) void fc_bf16(FcBf16Args p) {
     constexpr int NW = WAVES_M * WAVES_N;
     constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
@@ -271,10 +274,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *KG * 64, BLOCKS_PER_CU) void fc_b
         }
     };
     // Bias, clamp, v_cvt_pk_bf16_f32 and the stores; a copy without the clamp's compares, which are half the instructions
-    // of an epilogue that every CU runs at the same time (a linear layer has none).  32 rows of a wave's results pass through LDS, from where they are
-    // stored in runs of whole rows of the wave's columns.  Where those are 32, two v_permlane32_swap give a lane 8 neighbouring ones of a row, without that
-    // way round (654 x 1736 -> 208 9.0 us, through LDS 9.3).
-    constexpr bool kRuns = WTN > 32;
+    // of an epilogue that every CU runs at the same time (a linear layer has none).  RUNS: 32 rows of a wave's results pass through LDS.
     constexpr int CHUNKS = WTN / 8;  // of eight results in a row of a wave
     int8_t *mine = smem + BN * 4 + wave * (WTM * WTN * 2);
     const int sc = lane % CHUNKS, sr = lane / CHUNKS;
@@ -298,9 +298,9 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *KG * 64, BLOCKS_PER_CU) void fc_b
                     }
                     d[2 * q] = packBf16(v[0], v[1]);
                     d[2 * q + 1] = packBf16(v[2], v[3]);
-                    if (kRuns) *(v2i *)(rows + fr * (WTN * 2) + (((4 * j + q) ^ fr) % CHUNKS) * 16 + 8 * half) = v2i{(int)d[2 * q], (int)d[2 * q + 1]};
+                    if (RUNS) *(v2i *)(rows + fr * (WTN * 2) + (((4 * j + q) ^ fr) % CHUNKS) * 16 + 8 * half) = v2i{(int)d[2 * q], (int)d[2 * q + 1]};
                 }
-                if (kRuns) continue;
+                if (RUNS) continue;
 #pragma unroll
                 for (int q2 = 0; q2 < 2; q2++) {  // the lower half of the wave ends up with the first 8 of 16 columns, the upper with the others
                     const auto s0 = __builtin_amdgcn_permlane32_swap(d[4 * q2], d[4 * q2 + 2], false, false);
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *KG * 64, BLOCKS_PER_CU) void fc_b
                     store(m0 + wm * WTM + i * 32 + fr, n0 + wn * WTN + j * 32 + 16 * q2 + 8 * half, v4i{(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]});
                 }
             }
-            if (!kRuns) continue;
+            if (!RUNS) continue;
             asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
 #pragma unroll
             for (int t = 0; t < CHUNKS / 2; t++) {
@@ -321,18 +321,26 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N *KG * 64, BLOCKS_PER_CU) void fc_b
     else finish(std::true_type{});
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, int KG, bool FRAG>
-static hipError_t launchTile(const FcBf16Args &a, const LaunchCtx &ctx) {
-    auto kernel = fc_bf16<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, KG, FRAG>;
-    constexpr size_t ring = (size_t)KG * STAGES * (BM + BN) * 128, results = (size_t)BN * 4 + (size_t)BM * BN * 2, lds = ring > results ? ring : results;
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, int KG, bool FRAG, bool RUNS>
+static hipError_t launchTileRuns(const FcBf16Args &a, const LaunchCtx &ctx) {
+    auto kernel = fc_bf16<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, KG, FRAG, RUNS>;
+    constexpr size_t ring = (size_t)KG * STAGES * (BM + BN) * 128, results = (size_t)BN * 4 + (size_t)BM * BN * 2, lds = RUNS && results > ring ? results : ring;
     static std::once_flag once;
     static hipError_t configured = hipSuccess;
     std::call_once(once, [&] { configured = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
     if (configured != hipSuccess) return configured;
     const long long tiles = (long long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
     if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
-    THIP_ENQUEUE(ctx, kernelLabel("fc_bf16", {BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, KG, (int)FRAG}), kernel, dim3((unsigned)tiles), dim3(WAVES_M * WAVES_N * KG * 64), lds, a);
+    THIP_ENQUEUE(ctx, kernelLabel("fc_bf16", {BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, KG, (int)FRAG + 2 * (int)RUNS}), kernel, dim3((unsigned)tiles), dim3(WAVES_M * WAVES_N * KG * 64), lds, a);
     return hipGetLastError();
+}
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int BLOCKS_PER_CU, int KG, bool FRAG>
+static hipError_t launchTile(const FcBf16Args &a, const LaunchCtx &ctx) {
+    if constexpr (BN / WAVES_N > 32) {
+        if (BM == 256 || a.N % 8 != 0 || ((uintptr_t)a.out & 15)) return launchTileRuns<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, KG, FRAG, true>(a, ctx);
+    }
+    if constexpr (BM < 256) return launchTileRuns<BM, BN, WAVES_M, WAVES_N, STAGES, BLOCKS_PER_CU, KG, FRAG, false>(a, ctx);
+    return hipErrorInvalidValue;
 }
 
 // The tiles, by number (THIP_FC_TILE forces one).
