@@ -1,5 +1,6 @@
 """A caller may pass one piece of memory as an input and as an output: the results are those of every op as a launch of its own, whatever launches
 stand for several of them."""
+import ctypes
 import subprocess
 
 import numpy as np
@@ -178,3 +179,35 @@ def test_gpu_other_runs_of_records_in_place(device):
             exe.close()
             for p in ptrs:
                 device.free(p)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("make,kernels", [
+    (lambda: block(N=2, H=14, W=14, C=96, E=1152, O=96, stride=1), ["ir_block_i8"]), (lambda: w.fully_connected_workload(301, 301, 301, realistic=True), ["igemm_direct_i8"]),
+    (lambda: w.fully_connected_workload(400, 64, 64, realistic=True), ["igemm_direct_i8"]),
+], ids=["block", "ragged", "aligned"])
+def test_gpu_the_first_dispatch_in_place_while_a_graph_is_captured(device, make, kernels, monkeypatch):
+    """The kernels that only shared memory needs are known since creation: a capture of another stream, in the strictest mode, ends as it should."""
+    monkeypatch.setenv("THIP_IR_BLOCK", "1")
+    wl = make()
+    print("[gpu-case]", wl.name, "in place during a capture", flush=True)
+    hip, x = runtime.lib(), wl.inputs[0]
+    want = oracle_network(wl) if "layers" in wl.attrs else oracle_eval(wl)[0].reshape(wl.outputs[0][0])
+    exe = Executable(device, wl.program.serialize())
+    assert [k.split("<")[0] for k in exe.launch_kernels()] == kernels
+    ptr, other = device.upload(x), device.upload(x)
+    stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+    try:
+        assert hip.hipStreamCreate(ctypes.byref(stream)) == 0 and hip.hipStreamBeginCapture(stream, ctypes.c_int(0)) == 0
+        copied = hip.hipMemcpyAsync(ctypes.c_void_p(other), ctypes.c_void_p(other), ctypes.c_size_t(16), ctypes.c_int(3), stream)
+        exe.enqueue_device_noalloc([ptr, ptr], [x.nbytes] * 2)
+        assert (copied, hip.hipStreamEndCapture(stream, ctypes.byref(graph))) == (0, 0)
+        exe.wait()
+        assert_bit_exact(device.download(ptr, wl.outputs[0][0], np.int8), want, wl.name)
+    finally:
+        for handle, free in ((graph, hip.hipGraphDestroy), (stream, hip.hipStreamDestroy)):
+            if handle:
+                free(handle)
+        exe.close()
+        device.free(ptr)
+        device.free(other)

@@ -527,6 +527,11 @@ static bool chainAliased(const thip_executable_t *e, uint8_t *const *bp) {
 // A run whose result lies where it still reads (a block in place) is launched in parts that read nothing that another workgroup of theirs writes.
 static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *const *bp, const LaunchCtx &ctx, uint8_t *scratch = nullptr, bool apart = false) {
     hipError_t err = hipSuccess;
+    // asked for its kernel, a step asks for those that it launches on shared memory too
+    char others[96];
+    LaunchCtx behind = ctx;
+    behind.name = others;
+    behind.name_capacity = sizeof(others);
     auto recordByRecord = [&]() -> thip_status_t {
         for (uint32_t i = s.first; i < s.first + s.count; i++) {
             if (thip_status_t st = launchOp(e, i, e->ops[i], bp, ctx, scratch)) return st;
@@ -535,12 +540,11 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
     };
     switch (s.kind) {
     case kStepExpandDw: {
-        const bool shared = !ctx.name && writesWhatItReads(viewOf(e), s, bp);
+        const bool shared = !ctx.name && writesWhatItReads(viewOf(e), s, bp), block = s.count == 3 && !shared;
         if (s.count == 2 && shared) return recordByRecord();
-        if (s.count == 3 && !shared) {
-            err = launchIrBlock(irBlockArgs(viewOf(e), s, [&](const DescRef &r) { return r.space == kSpaceNone ? nullptr : (uint8_t *)resolve(e, r, bp); }), ctx);
-            break;
-        }
+        if (block) err = launchIrBlock(irBlockArgs(viewOf(e), s, [&](const DescRef &r) { return r.space == kSpaceNone ? nullptr : (uint8_t *)resolve(e, r, bp); }), ctx);
+        if (block && (err != hipSuccess || !ctx.name)) break;
+        const LaunchCtx &parts = block ? behind : ctx;
         const DescOp &x = e->ops[s.first], &d = e->ops[s.first + 1];
         IrExpandDwArgs a;
         memset(&a, 0, sizeof(a));
@@ -561,8 +565,8 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
             a.runBytes = x.KW * x.C; a.czp = x.input_zp;
             a.xBytes = (int64_t)x.N * x.H * x.W * x.C;
         }
-        err = launchIrExpandDw(a, ctx);
-        if (err == hipSuccess && s.count == 3) return launchOp(e, s.first + 2, e->ops[s.first + 2], bp, ctx, scratch, nullptr, s.route, 0, true);
+        err = launchIrExpandDw(a, parts);
+        if (err == hipSuccess && s.count == 3) return launchOp(e, s.first + 2, e->ops[s.first + 2], bp, parts, scratch, nullptr, s.route, 0, true);
         break;
     }
     case kStepMatmulRt: {
@@ -586,12 +590,16 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
         uint8_t *const *buffers = &e->stepBuffers[2 * (size_t)(&s - e->steps.data())];
         const bool shared = s.asIs && !ctx.name && writesWhatItReads(viewOf(e), s, bp);
         if (shared && !buffers[0]) return recordByRecord();  // no memory for the copy
-        if (s.asIs && !shared) return launchOp(e, s.first, s.op, bp, ctx, scratch, buffers, s.route, 0, true);
-        err = launchPadRows((const int8_t *)resolve(e, e->ops[s.first].in0, bp), (int8_t *)buffers[0], s.rows, s.from, s.to, ctx);
+        if (s.asIs && !shared) {
+            const thip_status_t st = launchOp(e, s.first, s.op, bp, ctx, scratch, buffers, s.route, 0, true);
+            if (st != THIP_OK || !ctx.name || !buffers[0]) return st;
+        }
+        const LaunchCtx &copied = s.asIs && ctx.name ? behind : ctx;
+        err = launchPadRows((const int8_t *)resolve(e, e->ops[s.first].in0, bp), (int8_t *)buffers[0], s.rows, s.from, s.to, copied);
         if (err != hipSuccess) break;
         DescOp op = s.op;
         op.in0 = DescRef{kSpacePlan, 0, 0};
-        return launchOp(e, s.first, op, bp, ctx, scratch, buffers, s.route, 0, true);
+        return launchOp(e, s.first, op, bp, copied, scratch, buffers, s.route, 0, true);
     }
     case kStepDecChain: {
         if (!ctx.name && apart) return recordByRecord();
@@ -610,7 +618,7 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
     }
     default: {
         const bool shared = s.route == kIgemmDirect && !ctx.name && writesWhatItReads(viewOf(e), s, bp);
-        return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch, nullptr, shared ? kIgemmOwnTile : s.route, s.blocked, true);
+        return launchOp(e, s.first, e->ops[s.first], bp, ctx, scratch, nullptr, shared ? kIgemmOwnTile : s.route, s.blocked, !shared);
     }
     }
     if (err != hipSuccess) return fail(THIP_INTERNAL, "ops %u .. %u: launch failed: %s", s.first, s.first + s.count - 1, hipGetErrorString(err));
