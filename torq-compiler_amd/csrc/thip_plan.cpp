@@ -200,8 +200,8 @@ static bool paddingPays(const DescOp &g, int64_t rows, int64_t Cp, int64_t K) {
 }
 
 // Whether igemm_direct_i8 takes the rows of the gathered record `g` as they are, as `op` (with its weights spread, or itself), and is ahead of its own
-// kernel.  It is ahead of the copy and a kernel behind it as well, by that launch: over the 153 of 170 drawn linears and convolutions of 5 .. 7848
-// channels that it takes, own kernel / copied rows / rows as they are cost 2.78 / 1.55 / 1.00 times the best (us: linear 9x100 -> 2303 5.5 / 6.4 / 4.0,
+// kernel.  It is ahead of the copy and a kernel behind it as well, by that launch: over the 256 of 330 drawn linears and convolutions of 5 .. 7972
+// channels that it takes, own kernel / copied rows / rows as they are cost 3.79 / 1.52 / 1.00 times the best, the choice over all 330 1.01 times (us: linear 9x100 -> 2303 5.5 / 6.4 / 4.0,
 // 554x604 -> 117 13.4 / 6.6 / 4.0, 5x1379 -> 48 57.4 / 6.4 / 4.5; 3x3 30x30x98 -> 316 stride 2, batch 3 7.1 / 6.6 / 4.0, 56x56x40 -> 32, batch 2 6.5 / 6.5 / 4.0; stride 2
 // 1x1 56x56x264 -> 96, batch 4 6.1 / 7.8 / 4.2).  Left where the gather is short (60x24 -> 64 3.6 / 6.1 / 3.8, 3x3 112x112x8 -> 32 4.5 / 6.7 / 4.1) and
 // where K is long enough for the worse loads to cost that launch: 3x2801 -> 1608 - / 6.2 / 6.6 (few rows have a faster kernel behind the copy), 5x5
