@@ -150,8 +150,9 @@ def test_ragged_rows_by_each_way(plan, make, lines):
     (dict(N=1, H=224, W=224, C=3, E=32, O=16, stride=1, first=(3, 2, (0, 1, 0, 1))), True), (dict(N=1, H=112, W=112, C=16, E=96, O=32, stride=2, pad=(0, 1, 0, 1)), False),
     (dict(N=4, H=112, W=112, C=16, E=96, O=32, stride=2, pad=(0, 1, 0, 1)), True), (dict(N=8, H=28, W=28, C=32, E=192, O=32, stride=1), False), (dict(N=64, H=28, W=28, C=32, E=192, O=32, stride=1), True),
     (dict(N=200, H=14, W=14, C=64, E=384, O=64, stride=1), False),
-    # more narrow channels than wide ones, or as many; and as many as two thirds
-    (dict(N=170, H=66, W=54, C=16, E=48, O=96, stride=1), False), (dict(N=101, H=64, W=55, C=16, E=96, O=96, stride=1), False), (dict(N=101, H=64, W=55, C=16, E=96, O=64, stride=1), True),
+    # many narrow channels, and few
+    (dict(N=170, H=66, W=54, C=16, E=48, O=96, stride=1), False), (dict(N=101, H=64, W=55, C=16, E=96, O=64, stride=1), False), (dict(N=192, H=51, W=56, C=64, E=128, O=64, stride=1), False),
+    (dict(N=101, H=64, W=55, C=16, E=96, O=16, stride=1), True),
 ], ids=lambda v: "x".join(str(x) for x in v.values()) if isinstance(v, dict) else str(v))
 def test_blocks_are_one_launch_where_that_is_estimated_ahead(plan, kw, taken):
     from test_ir_block import block

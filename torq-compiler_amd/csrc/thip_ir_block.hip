@@ -359,31 +359,30 @@ static bool preShiftedRequant(const Requant &rq) {
            rq.out_zp <= 32767;
 }
 
-// The time of a launch, us: of a workgroup alone on its CU a start and its chunks, each of which costs something whatever its size, then a share a tile
-// of a wave and a share an output row; of those that share a CU more.  Fitted to 897 launches (119 blocks of mobile networks of widths 0.5 .. 1 over
-// 96 .. 224 pixels, 1 .. 256 images, strips of every height), of which nine in ten lie within 10 %; of 891 others (irPairTime) seven in ten do, nine within 15 %.
+// The time of a launch, us: of a workgroup alone on its CU a start, its chunks, each of which costs something whatever its size, then a share a tile
+// of a wave and a share an output row, and at the end the add of its rows; of those that share a CU more.  Fitted (few channels: to first layers of mobile networks)
+// to 1850 blocks, half of them of mobile networks and the others of 16 .. 96 channels in and out, 1 .. 6 times as many wide ones, 7 .. 112 pixels, 1 .. 256 images:
+// nine in ten within 14 %.
 static double irBlockTime(const IrBlockArgs &a) {
     struct Cost {
-        double launch, start, chunk, tile, tileK, row, rowO, shared;
+        double launch, start, chunk, tile, tileK, row, rowO, add, shared;
         int perCu;
     };
-    constexpr Cost dense{4.0, 1.2, 0.43, 0.15, 0.105, 0.10, 0.034, 0.59, 2}, runs{2.9, 0.9, 0.36, 0.41, 0.0, 0.36, 0.074, 0.34, 4};
+    constexpr Cost dense{2.82, 2.23, 0.343, 0.184, 0.088, 0.046, 0.064, 0.065, 0.386, 2}, runs{2.9, 0.9, 0.36, 0.41, 0.0, 0.36, 0.074, 0.0, 0.34, 4};
     const Cost &c = a.CKH > 0 ? runs : dense;
     const int KS = (a.K + 31) / 32, OT = (a.O + 15) / 16, imageRows = a.cellRows < a.H ? a.cellRows : a.H;
     const long long blocks = (long long)a.N * a.strips * a.columnBlocks, room = 256LL * c.perCu, rest = blocks % room;
     const int tiles = (imageRows * a.regionColumns + 127) / 128, chunks = (a.C + 31) / 32;
-    const double alone = c.start + chunks * (c.chunk + tiles * (c.tile + c.tileK * (KS - 1)) + a.segmentRows * (c.row + c.rowO * OT));
+    const double alone = c.start + chunks * (c.chunk + tiles * (c.tile + c.tileK * (KS - 1)) + a.segmentRows * (c.row + c.rowO * OT)) + (a.skip ? a.segmentRows * OT * c.add : 0.0);
     auto together = [&](long long n) { return n > 0 ? alone * (1 + c.shared * (double)(n - 1)) : 0.0; };
     return c.launch + (double)(blocks / room) * together(c.perCu) + together((rest + 255) / 256);
 }
 
-// The time of ir_expand_dw_i8 and the pointwise convolution behind it, us, fitted to the same blocks: millions of widened, depthwise and narrow values, and
-// wide channels.  Narrow ones beyond two thirds of the wide, which those networks do not have, cost next to nothing more (66x54x16 -> 48 -> 96, 170 images, 48.6,
-// one launch 87.8).  Over 891 other blocks (16 .. 96 channels in and out, 1 .. 6 times as many wide ones, 7 .. 112 pixels, 1 .. 256 images) the choice costs 0.7 % of the
-// better one's time, always two launches 10 %, always one 28 %.
+// The time of ir_expand_dw_i8 and the pointwise convolution behind it, us, fitted to the same blocks (nine in ten within 15 %): millions of widened, depthwise
+// and narrow values, and wide channels.  The choice by the two costs 0.6 % of the better one's time over them, always two launches 5 %, always one 31 %.
 static double irPairTime(const IrBlockArgs &a) {
-    const double wide = 1e-6 * a.N * a.H * a.W * ((a.C + 31) / 32 * 32), out = 1e-6 * a.N * a.OH * a.OW, ch = 0.01 * a.C, narrow = std::min((double)a.O, a.C * 2 / 3.0);
-    return a.CKH > 0 ? 8.2 + 0.53 * wide + out * (0.73 * a.C + 0.44 * a.O) + 3.0 * ch : 6.8 + 0.183 * wide + out * (0.82 * a.C + 0.72 * narrow) + 0.32 * ch;
+    const double wide = 1e-6 * a.N * a.H * a.W * ((a.C + 31) / 32 * 32), out = 1e-6 * a.N * a.OH * a.OW, ch = 0.01 * a.C;
+    return a.CKH > 0 ? 8.2 + 0.53 * wide + out * (0.73 * a.C + 0.44 * a.O) + 3.0 * ch : 6.76 + 0.247 * wide + out * (0.75 * a.C + 0.357 * a.O) + 0.27 * ch;
 }
 
 bool planIrBlock(IrBlockArgs *args) {
