@@ -131,9 +131,10 @@ LINES = list(zip([c[0] for c in RAGGED], [["padded 0 1" + AS_IT_IS]] * 2 + [["pa
     (lambda: FC(9, 2500, 100), ["padded 0 1" + AS_IT_IS]), (lambda: FC(9, 2501, 100), ["padded 0 1"]), (lambda: FC(100, 8999, 32), ["padded 0 1" + AS_IT_IS]), (lambda: FC(100, 9001, 32), ["padded 0 1 igemm_direct_i8"]),
     (lambda: CONV(N=1, H=19, W=19, C=387, O=134, KH=5, KW=5, pad=(2, 2, 2, 2)), ["padded 0 1 igemm_direct_i8"]), (lambda: CONV(N=1, H=19, W=19, C=359, O=134, KH=5, KW=5, pad=(2, 2, 2, 2)), ["padded 0 1" + AS_IT_IS]),
     # a window over ragged results: strips in one round of the CUs, in two that are high, wide or narrow enough, and in two that are not
-    (lambda: CONV(N=19, H=53, W=53, C=64, O=89, pad=(1, 1, 1, 1)), [PATCH]), (lambda: CONV(N=20, H=64, W=64, C=112, O=8, KH=5, KW=5, pad=(2, 2, 2, 2)), [PATCH]),
-    (lambda: CONV(N=27, H=46, W=46, C=80, O=33, KH=5, KW=5, pad=(2, 2, 2, 2)), [OWN]), (lambda: CONV(N=40, H=40, W=40, C=80, O=7, KH=7, KW=7, pad=(3, 3, 3, 3)), [OWN]),
-    (lambda: CONV(N=7, H=105, W=105, C=64, O=53, KH=5, KW=5, pad=(2, 2, 2, 2)), [OWN]), (lambda: CONV(N=5, H=104, W=104, C=16, O=45, pad=(1, 1, 1, 1)), [OWN]),
+    (lambda: CONV(N=19, H=53, W=53, C=64, O=89, pad=(1, 1, 1, 1)), [PATCH]), (lambda: CONV(N=45, H=56, W=56, C=96, O=15, KH=5, KW=5, pad=(2, 2, 2, 2)), [PATCH]), (lambda: CONV(N=20, H=64, W=64, C=112, O=8, KH=5, KW=5, pad=(2, 2, 2, 2)), [OWN]),
+    (lambda: CONV(N=22, H=73, W=73, C=64, O=5, KH=7, KW=7, pad=(3, 3, 3, 3)), [OWN]), (lambda: CONV(N=27, H=46, W=46, C=80, O=33, KH=5, KW=5, pad=(2, 2, 2, 2)), [OWN]), (lambda: CONV(N=40, H=40, W=40, C=80, O=7, KH=7, KW=7, pad=(3, 3, 3, 3)), [OWN]),
+    (lambda: CONV(N=7, H=105, W=105, C=64, O=53, KH=5, KW=5, pad=(2, 2, 2, 2)), [OWN]), (lambda: CONV(N=6, H=122, W=122, C=96, O=28, KH=5, KW=5, pad=(2, 2, 2, 2)), [OWN]), (lambda: CONV(N=6, H=122, W=122, C=96, O=32, KH=5, KW=5, pad=(2, 2, 2, 2)), [PATCH]),
+    (lambda: CONV(N=5, H=104, W=104, C=16, O=45, pad=(1, 1, 1, 1)), [OWN]),
     # 256 tiles of 32 x 32, and one row more
     (lambda: FC(256, 77, 1024), ["padded 0 1" + AS_IT_IS]), (lambda: FC(257, 77, 1024), ["padded 0 1"]),
     # a gather of one k-tile: in single bytes, in pieces of eight

@@ -228,13 +228,16 @@ static bool planConvPatch(const IgemmArgs &a, ConvPatchPlan *q) {
 //   many channels out, few taps, many in      56x56x48 -> 128, 20 9.8 / 12.0; 2x2 100x100x96 -> 64, 20 15.2 / 21.5; 64x64x128 -> 64, 32 19.2 / 22.6
 //   a second round of low strips              5x5 46x46x80 -> 33, 27 16.7 / 24.9; 7x7 40x40x80 -> 7, 40 26.0 / 42.4; 5x5 105x105x64 -> 53, 7 19.1 / 21.4
 //   rows that only rounding up makes three    104x104x16 -> 45, 5 6.2 / 7.5
-// Over 605 drawn ones (16 .. 112 channels in, 1 .. 96 out, windows of 3, 5 and 7) the choice costs 1.2 % of the better one's time, always the ring kernel 20 %, always this one 3 %.
+//   ragged results in two rounds or more      5x5 122x122x96 -> 28, 6 21.3 / 25.0; 93x93x112 -> 18, 9 23.4 / 26.8; 7x7 73x73x64 -> 5, 22 26.4 / 38.8
+//   where the ring kernel's tiles are one     (43 drawn ones: up to 400 tiles 0.89 of its speed, to 512 1.00 in two rounds and 0.85 in three, beyond 1.21; whole results 1.06 and more)
+// Over 605 drawn ones (16 .. 112 channels in, 1 .. 96 out, windows of 3, 5 and 7) the choice costs 1.1 % of the better one's time, always the ring kernel 20 %, always this one 3 %.
 bool convPatchBetter(const IgemmArgs &a) {
     ConvPatchPlan q;
     if (a.C > 112 || a.KH * a.KW < 9 || a.M < 49152 || !planConvPatch(a, &q)) return false;
     const int rounds = (q.strips + 255) / 256;
     if (q.rows * a.KW < 9 || (long long)(a.M / a.OW) * a.KW < 1600LL * rounds) return false;
-    return rounds == 1 || ((q.rows >= a.KH || q.rows * a.OW > 160) && (a.N <= 32 || q.rows >= (a.KH < 4 ? a.KH : 4)));
+    if (rounds == 1) return true;
+    return (q.rows >= a.KH || q.rows * a.OW > 160) && (a.N <= 32 || q.rows >= (a.KH < 4 ? a.KH : 4)) && (a.N % 16 == 0 || a.M > (rounds == 2 ? 102400 : 131072));
 }
 
 template <int NB, bool ANY>
