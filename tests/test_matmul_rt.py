@@ -32,3 +32,14 @@ def test_runtime_input2(device, kw, tmp_path):
     finally:
         device.set_event_log(None)
     assert_bit_exact(got[0], want, wl.name + " record by record")
+
+
+@pytest.mark.parametrize("K", [1, 16, 127, 128, 129, 143, 144, 256, 257, 300, 400, 513])
+@pytest.mark.parametrize("B, M, N", [(2, 33, 17), (16, 1, 144), (9, 130, 250), (24, 400, 520)], ids=["32rows-ragged", "one-row", "64rows", "128rows"])
+def test_k_tiles(device, B, M, N, K):
+    """The ends of k-tiles: one, two and an odd number of them, rows of B that end a byte before, at and behind a chunk."""
+    wl = w.matmul_workload(B=B, M=M, K=K, N=N, out_dtype=np.int32, seed=K)
+    launched = []
+    got, _ = run_on_gpu(device, wl, via="device", launched=launched)
+    assert families(launched) == ["igemm_rt_i8"], launched
+    assert_bit_exact(got[0], oracle_eval(wl)[0], wl.name)

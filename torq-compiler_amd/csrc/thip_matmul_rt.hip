@@ -4,58 +4,66 @@
 
 namespace thip {
 
+constexpr int kRtRowB = 160;  // bytes of LDS from one row of B to the next: 8 rows of 32 columns lie in distinct banks
+
+// ds_read_b64_tr_b8: of 16 lanes' 8 bytes each, as 8 rows of 16, a lane gets a column.
+__device__ __forceinline__ v2i readTransposed(const int8_t *p) {
+    return __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i *)p);
+}
+
 // ---------------------------------------------------------------------------
 // igemm_rt_i8: out[b][m][n] = R1(sum_k A[b][m][k] * B[b][k][n]) with ONE (bias, scale) pair, int8 / int16 / int32 results.
 //
 // The MFMA wants 16 consecutive k of one column, and B has its columns side by side.  The records say so with a transpose
 // per batch into [N][Kp] and a GEMM per batch behind it: two launches per batch element, 5 us each whatever their size
-// (4 x 1024x128x1024 -> int16: eight launches, 47 us for 9.4 MB of operands).  Here a workgroup transposes the B tile on its
-// way into LDS: a thread loads the dwords of 16 rows of four columns (a wave: two runs of 128 bytes per row) and turns them with
-// 32 v_perm_b32 into the 16-byte chunks of four LDS rows, 1/BM of an instruction per product.  Batches are part of the grid.
+// (4 x 1024x128x1024 -> int16: eight launches, 47 us for 9.4 MB of operands).  Here a workgroup copies the B tile into LDS as it
+// lies, 16 bytes of a row at a time, and ds_read_b64_tr_b8 turns it on the way into the MFMA's registers.  Batches are part of the grid.
 //
-// LDS rows are 128 bytes of K; chunk c of row r sits at slot c ^ swizzle(r): (r >> 1) & 7 for A, whose rows are written 8
-// lanes at a time; for B, whose writes go to every fourth row, also bit 4 of the row, so that the eight lanes of a write phase
-// and the 16 rows of a read phase both fall into distinct banks.  Two buffers; the loads of a k-tile are in flight during the
-// MFMAs of the one before.  What lies beyond K is zero in B only; bytes beyond the tensors are never read.
+// LDS rows of A are 128 bytes of K, chunk c of row r at slot c ^ ((r >> 1) & 7); those of B are 128 columns and lie 160 bytes apart, so that
+// the 8 rows of 32 columns that 32 lanes read fall into distinct banks.  Two buffers, or two groups of waves (KG) with one each, which make
+// every other k-tile and add up at the end; the loads of a k-tile are in flight during the MFMAs of the one before.  What lies
+// beyond K is zero in B only; bytes beyond the tensors are never read.
 //
-// Bound by latency (one k-tile for K <= 128: load, MFMA, store, nothing to overlap but other workgroups) and then by
-// the stores: 4 x 1024x128x1024 -> int16 5.9 us.  MFMA operands, accumulator layout and requant tails are those of igemm_dense_i8.
+// Bound by a wave's issue (about one instruction in 5 cycles while it is alone on its SIMD: turning B with v_perm_b32 behind dword loads, 100 more
+// instructions a k-tile, took 0.8 us a k-tile where this takes 0.4; more k-tiles in flight change nothing) and then by the stores.  With v_perm_b32
+// and one group / now, us: 1 x 1024x1024x1024 10.0 / 5.7, 1 x 1x1024x1024 9.8 / 5.4, 16 x 32x512x64 6.4 / 4.2, 8 x 512x256x512 5.3 / 4.5,
+// 4 x 1024x128x1024 -> int16 5.77 / 5.40, 2 x 2048x1024x2048 -> int32 20.0 / 19.8.
+// MFMA operands, accumulator layout and requant tails are those of igemm_dense_i8.
 // ---------------------------------------------------------------------------
-template <int BM, int WAVES_M, int WAVES_N, int OUT>
-__global__ __launch_bounds__(256, 2) void igemm_rt_i8(MatmulRtArgs p) {
-    constexpr int BN = 128, LA = BM / 32;
+template <int BM, int WAVES_M, int WAVES_N, int OUT, int KG>
+__global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastDiv divTiles, FastDiv divTilesM) {
+    constexpr int BN = 128, LA = BM / 32, BUFS = KG == 1 ? 2 : 1;
     constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N, TM = WTM / 32, TN = WTN / 32;
-    constexpr int A_BYTES = BM * 128, BUF = (BM + BN) * 128;
+    constexpr int A_BYTES = BM * 128, BUF = A_BYTES + 128 * kRtRowB;
     static_assert(WAVES_M * WAVES_N == 4, "four waves");
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // in the group
+    const int group = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
     const int wm = wave / WAVES_N, wn = wave % WAVES_N;
     // each XCD gets a contiguous range of (batch, column tile, row tile)
-    const int tilesM = (p.M + BM - 1) / BM, tilesN = (p.N + BN - 1) / BN;
     int lin;
     {
         const int nb = (int)gridDim.x, pid = (int)blockIdx.x;
         const int per = nb / 8, rem = nb % 8, xcd = pid % 8, idx = pid / 8;
         lin = xcd * per + (xcd < rem ? xcd : rem) + idx;
     }
-    const int batch = lin / (tilesM * tilesN), tile = lin - batch * (tilesM * tilesN);
-    const int n0 = (tile / tilesM) * BN, m0 = (tile % tilesM) * BM;
-    // Offsets are from the start of the tensors, below 2^31 (matmulRtFits); the last ones at which a whole chunk / word still
-    // lies inside:
-    const int aLast = (int)p.a_bytes - 16, bLast = (int)p.b_bytes - 4;
-    const int KT = (p.K + 127) / 128;
+    const int batch = (int)fastDiv((uint32_t)lin, divTiles), tile = lin - batch * (int)divTiles.d;
+    const int tileN = (int)fastDiv((uint32_t)tile, divTilesM), n0 = tileN * BN, m0 = (tile - tileN * (int)divTilesM.d) * BM;
+    // Offsets are from the start of the tensors, below 2^31 (matmulRtFits); the last ones at which a whole chunk still lies
+    // inside:
+    const int aLast = (int)p.a_bytes - 16, bLast = (int)p.b_bytes - 16;
+    const int KT = (p.K + 128 * KG - 1) / (128 * KG);  // k-tiles of a group: group, group + KG, ...
 
-    const int bg = tid & 31, bc = tid >> 5;  // this thread's four columns and 16-row chunk of the B tile
-    const int bn = n0 + 4 * bg;
-    int aOff[LA];  // of this thread's chunks in k-tile 0
+    // chunk `chunk` of every 32nd row of both tiles is this thread's; offsets of those of k-tile 0
+    const int chunk = tid & 7, row0 = tid >> 3;
+    int aOff[LA];
 #pragma unroll
     for (int i = 0; i < LA; i++) {
-        const int id = tid + 256 * i, row = m0 + (id >> 3) < p.M ? m0 + (id >> 3) : p.M - 1;
-        aOff[i] = (int)(batch * p.a_stride) + row * p.K + (id & 7) * 16;
+        const int row = m0 + row0 + 32 * i;
+        aOff[i] = (int)(batch * p.a_stride) + (row < p.M ? row : p.M - 1) * p.K + chunk * 16;
     }
-    const int bBase = (int)(batch * p.b_stride) + bn;
-    v4i ra[LA];
-    uint32_t rb[16];
+    const int bOff = (int)(batch * p.b_stride) + n0 + row0 * p.N + chunk * 16;
+    v4i ra[LA], rb[4];
     // Loads only, no branch and no use of what is loaded: a load that would pass the end of its tensor starts as much
     // earlier, and store() moves its bytes to where they belong.
     auto load = [&](int kt) {
@@ -64,46 +72,37 @@ __global__ __launch_bounds__(256, 2) void igemm_rt_i8(MatmulRtArgs p) {
             const int off = aOff[i] + kt * 128;
             ra[i] = ((const UnalignedV4 *)(p.A + (uint32_t)(off < aLast ? off : aLast)))->v;
         }
-        const int k0 = kt * 128 + bc * 16;
-        int off = bBase + (k0 < p.K ? k0 : p.K) * p.N;
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            rb[r] = ((const UnalignedU32 *)(p.B + (uint32_t)(off < bLast ? off : bLast)))->v;
-            off = off < bLast ? off + p.N : off;
+        for (int i = 0; i < 4; i++) {
+            const int k = kt * 128 + 32 * i, off = bOff + (k < p.K ? k : p.K) * p.N;
+            rb[i] = ((const UnalignedV4 *)(p.B + (uint32_t)(off < bLast ? off : bLast)))->v;
         }
     };
     auto store = [&](int kt, int8_t *buf) {
+        if (kt * 128 + 144 > p.K) {  // K's end, and where N < 16 the rows whose chunk passes the end of the tensor, lie no further away
+            auto moved = [](v4i v, int past) {
+                if (past <= 0 || past >= 16) return v;
+                unsigned __int128 bytes;
+                __builtin_memcpy(&bytes, &v, 16);
+                bytes >>= 8 * past;
+                __builtin_memcpy(&v, &bytes, 16);
+                return v;
+            };
+#pragma unroll
+            for (int i = 0; i < LA; i++) ra[i] = moved(ra[i], aOff[i] + kt * 128 - aLast);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int k = kt * 128 + 32 * i;
+                rb[i] = k + row0 < p.K ? moved(rb[i], bOff + k * p.N - bLast) : v4i{0, 0, 0, 0};
+            }
+        }
 #pragma unroll
         for (int i = 0; i < LA; i++) {
-            const int id = tid + 256 * i, row = id >> 3, past = aOff[i] + kt * 128 - aLast;
-            if (past > 0 && past < 16) {  // the tensor's last bytes, and only where K is no multiple of 16
-                uint32_t w[8] = {(uint32_t)ra[i][0], (uint32_t)ra[i][1], (uint32_t)ra[i][2], (uint32_t)ra[i][3], 0, 0, 0, 0};
-                for (int e = 0; e < past; e++) {
-#pragma unroll
-                    for (int d = 0; d < 4; d++) w[d] = (w[d] >> 8) | (w[d + 1] << 24);
-                }
-                ra[i] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-            }
-            *(v4i *)(buf + row * 128 + (((id & 7) ^ ((row >> 1) & 7)) << 4)) = ra[i];
+            const int row = row0 + 32 * i;
+            *(v4i *)(buf + row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4)) = ra[i];
         }
-        // rows beyond K are zero, and among the last ones (several where N < 4) a word may have started early
-        const int k0 = kt * 128 + bc * 16;
-        if (kt * 128 + 132 > p.K) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int past = bBase + (k0 < p.K ? k0 + r : 0) * p.N - bLast;
-                if (past > 0) rb[r] >>= 8 * (past & 3);  // 1 .. 3 where the word holds a column at all
-                rb[r] = k0 + r < p.K ? rb[r] : 0;
-            }
-        }
-        uint32_t o[4][4];
-#pragma unroll
-        for (int a = 0; a < 4; a++) transpose4x4(rb[4 * a], rb[4 * a + 1], rb[4 * a + 2], rb[4 * a + 3], o[a]);
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int row = 4 * bg + j, swz = ((row >> 1) & 7) ^ ((row >> 4) & 1);
-            *(v4i *)(buf + A_BYTES + row * 128 + ((bc ^ swz) << 4)) = v4i{(int)o[0][j], (int)o[1][j], (int)o[2][j], (int)o[3][j]};
-        }
+        for (int i = 0; i < 4; i++) *(v4i *)(buf + A_BYTES + (row0 + 32 * i) * kRtRowB + chunk * 16) = rb[i];
     };
     v16i acc[TN][TM];
 #pragma unroll
@@ -115,16 +114,14 @@ __global__ __launch_bounds__(256, 2) void igemm_rt_i8(MatmulRtArgs p) {
         }
     }
     const int fr = lane & 31, half = lane >> 5;
-    load(0);
-    store(0, smem);
-    __syncthreads();
-    for (int kt = 0; kt < KT; kt++) {
-        if (kt + 1 < KT) load(kt + 1);
-        const int8_t *buf = smem + (kt & 1) * BUF;
-        const int steps = p.K - kt * 128 < 128 ? (p.K - kt * 128 + 31) / 32 : 4;
+    int8_t *const own = smem + group * (BUFS * BUF);
+    // of an operand's 16 columns and 8 rows a lane reads 8 bytes of row (lane & 15) / 2 and gets its column's
+    const int turned = A_BYTES + (16 * half + ((lane & 15) >> 1)) * kRtRowB + wn * WTN + (lane & 16) + 8 * (lane & 1);
+    auto multiply = [&](int kt, const int8_t *buf) {
+        const int steps = p.K - kt * 128 < 128 ? (p.K - kt * 128 + 31) / 32 : 4;  // none or fewer for a group whose k-tiles have ended
 #pragma unroll
         for (int s = 0; s < 4; s++) {
-            if (s >= steps) break;
+            if (s >= steps) continue;
             v4i af[TM], bf[TN];
 #pragma unroll
             for (int i = 0; i < TM; i++) {
@@ -133,8 +130,9 @@ __global__ __launch_bounds__(256, 2) void igemm_rt_i8(MatmulRtArgs p) {
             }
 #pragma unroll
             for (int j = 0; j < TN; j++) {
-                const int row = wn * WTN + j * 32 + fr, swz = ((row >> 1) & 7) ^ ((row >> 4) & 1);
-                bf[j] = *(const v4i *)(buf + A_BYTES + row * 128 + (((2 * s + half) ^ swz) << 4));
+                const int8_t *at = buf + turned + 32 * s * kRtRowB + 32 * j;
+                const v2i low = readTransposed(at), high = readTransposed(at + 8 * kRtRowB);
+                bf[j] = v4i{low[0], low[1], high[0], high[1]};
             }
 #pragma unroll
             for (int j = 0; j < TN; j++) {
@@ -142,8 +140,58 @@ __global__ __launch_bounds__(256, 2) void igemm_rt_i8(MatmulRtArgs p) {
                 for (int i = 0; i < TM; i++) acc[j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], af[i], acc[j][i], 0, 0, 0);
             }
         }
-        if (kt + 1 < KT) store(kt + 1, smem + ((kt + 1) & 1) * BUF);  // the other buffer: its readers met the barrier a k-tile ago
+    };
+    load(group);
+    store(group, own);
+    const int8_t *last = own;
+    if (KT > 1) {
+        load(KG + group);
         __syncthreads();
+        for (int it = 1; it < KT; it++) {
+            multiply((it - 1) * KG + group, last);
+            if (BUFS == 1) __syncthreads();
+            // two buffers: the readers of the other one met the barrier a k-tile ago
+            int8_t *next = own + (BUFS == 2 ? (it & 1) * BUF : 0);
+            store(it * KG + group, next);
+            load((it + 1) * KG + group);  // past the last one nobody uses it: behind a branch the compiler waits for it at once
+            last = next;
+            __syncthreads();
+        }
+    } else {
+        __syncthreads();
+    }
+    multiply((KT - 1) * KG + group, last);
+    if constexpr (KG > 1) {
+        // the second group's sums through LDS, 16 bytes a lane; the first one adds them to its own and goes on
+        static_assert(KG == 2, "one group besides the first");
+        v4i *const sums = (v4i *)smem;
+        __syncthreads();
+        if (group > 0) {
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+#pragma unroll
+                for (int i = 0; i < TM; i++) {
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        sums[(j * TM + i) * 1024 + q * 256 + tid] = v4i{acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]};
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        if (group > 0) return;
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+#pragma unroll
+            for (int i = 0; i < TM; i++) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const v4i v = sums[(j * TM + i) * 1024 + q * 256 + tid];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[j][i][4 * q + e] = (int)((uint32_t)acc[j][i][4 * q + e] + (uint32_t)v[e]);
+                }
+            }
+        }
     }
 
     // Register 4 q + e of lane (fr, half) is out[m = fr][n = 8 q + 4 half + e] of a 32 x 32 tile.  Results narrower than 32 bits
@@ -224,26 +272,27 @@ __global__ __launch_bounds__(256, 2) void igemm_rt_i8(MatmulRtArgs p) {
     }
 }
 
-template <int BM, int WAVES_M, int WAVES_N, int OUT>
+template <int BM, int WAVES_M, int WAVES_N, int OUT, int KG>
 static hipError_t launchRt(const MatmulRtArgs &a, const LaunchCtx &ctx) {
-    auto kernel = igemm_rt_i8<BM, WAVES_M, WAVES_N, OUT>;
-    constexpr size_t lds = 2 * (size_t)(BM + 128) * 128;
-    const long long tiles = (long long)a.batches * ((a.M + BM - 1) / BM) * ((a.N + 127) / 128);
-    if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
-    THIP_ENQUEUE(ctx, kernelLabel("igemm_rt_i8", {BM, WAVES_M, WAVES_N, OUT}), kernel, dim3((unsigned)tiles), dim3(256), lds, a);
+    auto kernel = igemm_rt_i8<BM, WAVES_M, WAVES_N, OUT, KG>;
+    const size_t lds = (size_t)(KG > 1 || a.K > 128 ? 2 : 1) * (BM * 128 + 128 * kRtRowB);
+    const long long tilesM = (a.M + BM - 1) / BM, tiles = tilesM * ((a.N + 127) / 128);
+    if (tiles * a.batches > 0x7fffffffLL) return hipErrorInvalidValue;
+    THIP_ENQUEUE(ctx, kernelLabel("igemm_rt_i8", {BM, WAVES_M, WAVES_N, OUT, KG}), kernel, dim3((unsigned)(tiles * a.batches)), dim3(256 * KG), lds, a,
+                 makeFastDiv((uint32_t)tiles), makeFastDiv((uint32_t)tilesM));
     return hipGetLastError();
 }
 
-// Rows of a tile.  A k-tile takes a workgroup about 1.3 us whatever its rows (the loads' latency), so up to one workgroup per
-// CU the smallest tile is ahead (1 x 1024x128x1024: 3.9 us on 32 rows, 4.5 on 64, 5.3 on 128); beyond that 64 rows (4 x
-// 1024x128x1024: 6.9, 5.9, 6.2), and from three workgroups of these per CU the operands' traffic counts (2 x 2000x1024x2000,
-// int32: 35.2, 27.9, 21.9).
+// Rows of a tile, us.  Up to one workgroup per CU the smallest tile is ahead (1 x 1024x1024x1024: 6.7 on 32 rows, 7.6 on 64, 9.6 on 128), and a second
+// group of waves where there is a second k-tile for it (5.7; four groups 5.7, and behind two on 2 x 300x700x300: 5.1, 5.6); beyond that 64 rows
+// (3 x 777x333x555 -> int16: 7.6, 6.6, 8.9; 8 x 512x256x512 4.7, 4.5, 5.5; 4 x 1024x128x1024 -> int16 5.6, 5.4, 6.1), and from three workgroups of these per
+// CU the operands' traffic counts (8 x 1024x256x1024 12.2, 9.9, 7.4; 2 x 2048x1024x2048 -> int32 26.8, 22.5, 19.8).
 template <int OUT>
 static hipError_t launchRtOut(const MatmulRtArgs &a, const LaunchCtx &ctx) {
     auto tiles = [&](int bm) { return (long long)a.batches * ((a.M + bm - 1) / bm) * ((a.N + 127) / 128); };
-    if (a.M <= 32 || tiles(32) <= 256) return launchRt<32, 1, 4, OUT>(a, ctx);
-    if (tiles(64) <= 768) return launchRt<64, 2, 2, OUT>(a, ctx);
-    return launchRt<128, 2, 2, OUT>(a, ctx);
+    if (a.M <= 32 || tiles(32) <= 256) return a.K <= 128 ? launchRt<32, 1, 4, OUT, 1>(a, ctx) : launchRt<32, 1, 4, OUT, 2>(a, ctx);
+    if (tiles(64) <= 768) return launchRt<64, 2, 2, OUT, 1>(a, ctx);
+    return launchRt<128, 2, 2, OUT, 1>(a, ctx);
 }
 
 hipError_t launchMatmulRt(const MatmulRtArgs &a, const LaunchCtx &ctx) {
