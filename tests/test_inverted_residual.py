@@ -8,7 +8,7 @@ from torq_compiler_amd import Program, workloads as w
 pytestmark = pytest.mark.gpu
 
 
-def block(N, H, W, C, E, stride, pad=(1, 1, 1, 1), shift=None, first=None, seed=1060):
+def block(N, H, W, C, E, stride, pad=(1, 1, 1, 1), shift=None, first=None, seed=1060, top=127):
     """widen (pointwise, or `first` = (window, stride, pad) over few channels) -> depthwise 3x3, the wide image an intermediate; `shift`: a literal requant range for both (results
     saturate, the general 32-bit tail) instead of one that spreads them."""
     rng = np.random.default_rng(seed)
@@ -21,7 +21,7 @@ def block(N, H, W, C, E, stride, pad=(1, 1, 1, 1), shift=None, first=None, seed=
         if shift is not None:
             sh = np.full(E, shift, dtype=np.int8)
         sb, sf = w.derive_scale_bias(mult, sh, rng.integers(-4000, 4000, E), wt, zp)
-        attrs = dict(input_zp=zp, output_zp=zout, output_min=-120 if op == "conv2d" else -128, output_max=127, shift_factor=sf)
+        attrs = dict(input_zp=zp, output_zp=zout, output_min=-120 if op == "conv2d" else -128, output_max=top, shift_factor=sf)
         attrs.update(pad=cpad, stride=(cs, cs)) if op == "conv2d" else attrs.update(pad=pad, stride=(stride, stride))
         layers.append(w.Layer(op, [len(layers)], attrs, wt, sb))
     H, W = (H + cpad[2] + cpad[3] - k) // cs + 1, (W + cpad[0] + cpad[1] - k) // cs + 1
@@ -93,6 +93,18 @@ def test_expand_depthwise_walk(device, kw):
 ], ids=lambda kw: "x".join(str(v) for v in kw.values()))
 def test_rows_no_window_reaches(device, kw):
     """Several images per workgroup whose last row lies below every window."""
+    wl = block(**kw)
+    print("[gpu-case]", wl.name, flush=True)
+    assert_bit_exact(fused(device, wl)[0], oracle_network(wl), wl.name)
+
+
+@pytest.mark.parametrize("kw", [
+    dict(N=1, H=9, W=10, C=32, E=48, stride=1), dict(N=1, H=11, W=3, C=16, E=32, stride=2), dict(N=1, H=5, W=65, C=16, E=32, stride=1),   # segments with fewer rows, or none
+    dict(N=257, H=7, W=7, C=160, E=960, stride=1), dict(N=259, H=13, W=14, C=96, E=592, stride=1), dict(N=66, H=2, W=1, C=64, E=1040, stride=1),  # a last workgroup of fewer images
+    dict(N=2, H=12, W=12, C=32, E=48, stride=1, top=100), dict(N=2, H=12, W=12, C=32, E=48, stride=2, shift=41), dict(N=2, H=9, W=9, C=3, E=48, stride=1, first=(3, 1, (1, 1, 1, 1)), top=90),
+], ids=lambda kw: "x".join(str(v) for v in kw.values()))
+def test_expand_depthwise_lanes(device, kw):
+    """Lanes that share a product but not its rows: short segments, workgroups with fewer images; results that are clamped below their type's maximum, and long shifts."""
     wl = block(**kw)
     print("[gpu-case]", wl.name, flush=True)
     assert_bit_exact(fused(device, wl)[0], oracle_network(wl), wl.name)

@@ -7,7 +7,7 @@
 namespace thip {
 
 constexpr int kIrChunk = 32;           // channels of a workgroup
-constexpr int kIrPitch = kIrChunk + 4;  // bytes of a cell in LDS: the padding spreads neighbouring cells over the banks
+constexpr int kIrPitch = kIrChunk / 2;  // bytes of a cell in LDS, in each of two planes
 
 struct IrStrip {
     int images;               // more than one only where a strip is a whole image

@@ -5,39 +5,40 @@
 
 namespace thip {
 
-// The requant tails that need 32-bit arithmetic only (withRequantMode without its 64-bit one; the planner keeps such records
+// The requant tails that need 32-bit arithmetic only (withPackMode without its 64-bit one; the planner keeps such records
 // apart).
 template <typename F>
-__device__ __forceinline__ void withNarrowRequantMode(const WideRequant &w, F &&f) {
-    if (w.plain) f(std::integral_constant<int, 2>{});
+__device__ __forceinline__ void withNarrowPackMode(const WideRequant &w, F &&f) {
+    if (w.packed && w.packShift <= 0) f(std::integral_constant<int, 4>{});
+    else if (w.packed) f(std::integral_constant<int, 5>{});
+    else if (w.plain) f(std::integral_constant<int, 2>{});
     else if (w.preOnly) f(std::integral_constant<int, 3>{});
     else f(std::integral_constant<int, 1>{});
 }
 
-// Columns of cells under the windows of one output row, in whole column groups of the threads.
-static inline int irCellColumns(int OW, int S) { return S == 1 ? 2 * ((OW + 1) / 2) + 2 : 2 * OW + 1; }
+// Columns of cells under the windows of one output row.
+static inline int irCellColumns(int OW, int S) { return (OW - 1) * S + 3; }
 
 // ---------------------------------------------------------------------------
 // ir_expand_dw_i8: a workgroup makes 32 channels of a strip of output rows of one image.
 //
 // Phase 1, the pointwise convolution: the strip's input pixels are rows of a dense [pixels][K] matrix; a wave takes 32 of
 // them at a time straight from memory in MFMA operand layout (K <= 192: at most six loads per lane, prefetched one tile ahead), the
-// 32 channels' weights stay in registers, and the requantised bytes go to LDS as cells [row][column][32 channels]. Cells outside the
-// image hold the depthwise op's zero point.
+// 32 channels' weights stay in registers, and the requantised bytes go to LDS as cells of 16 bytes [row][column] in each of two planes (channel
+// 8 a + 4 j + e is byte 4 a + e of plane j). Cells outside the image hold the depthwise op's zero point.
 // RUNS: a convolution over few channels instead (the first layer of an image network): K is one 16-byte run per window row, and the pixels are gathered from the image.
-// Phase 2, the depthwise convolution: a thread owns four channels of two output columns (one at stride 2) and walks down rows:
-// per input row three to four dwords from LDS, a byte transpose so that a dword holds one channel at neighbouring
-// columns, and one v_dot4_i32_i8 per window row, channel and output. No address clamping and no padding selects are left in the loop.
+// Phase 2, the depthwise convolution as a product, as in ir_block_i8: 16 channels x 16 pixels are one v_mfma_i32_16x16x64_i8 per window row with
+// the taps on the diagonals of 16 x 16 blocks. A lane owns a column of a segment of the strip's rows, of any image of the workgroup's, and walks down it: two 16-byte
+// loads from LDS a row, and its group's 8 neighbouring channels of a pixel are one 8-byte store.
 //
 // Why: apart, the two launches write the widened image and read it back (3.3 MB per image of a 224 x 224 mobile network, 6.7 MB of
-// its 11 MB of traffic), and at small batches each costs a dependent launch. Bound by the vector pipes: about 5 instructions
-// per widened byte and 9 per depthwise byte, most of them the requants.  Measured, us, the two launches / this one:
-//   batch 256  112x112x16 -> 96 stride 2 151 / 99, 56x56x32 -> 144 80 / 69, 28x28x32 -> 192 42 / 26, 14x14x96 -> 576 34 / 25
-//   batch 32   112x112x16 -> 96 stride 2 30.9 / 18.5, 56x56x32 -> 144 24.2 / 15.9, 14x14x96 -> 576 10.0 / 8.0
-//   batch 1    56x56x32 -> 144 6.8 / 4.8, 14x14x96 -> 576 6.7 / 3.8, 7x7x160 -> 960 6.8 / 4.1
-// and since, with pixels and cells reached by a walk instead of divisions and 32-bit offsets of the results (in a trace of the network,
-// batch 256): 224x224x3 -> 112x112x32 104.9 -> 94.9, 112x112x16 -> 96 stride 2 115.1 -> 108.6, 56x56x32 -> 144 80.0 -> 77.2. The busy
-// cycles are 90 % vector instructions there; more tiles prefetched, or strips of 26, 32 or 53 KB, change nothing.
+// its 11 MB of traffic), and at small batches each costs a dependent launch. About half of the cycles are vector instructions (5 per widened and 5 per depthwise
+// byte; with byte transposes and v_dot4_i32_i8 in phase 2 it was 9 per depthwise byte); the rest goes where a workgroup's phases and the launch's last round of workgroups wait.
+// us, in a trace of the network, with v_dot4_i32_i8 / now:
+//   batch 256  14x14x64 -> 384 17.4 / 15.1, 14x14x96 -> 576 24.6 / 23.8, its stride 2 17.3 / 16.2, 7x7x160 -> 960 17.0 / 15.0
+//   batch 32   7x7x160 -> 960 8.3 / 5.6, 14x14x96 -> 576 8.4 / 8.0, 14x14x64 -> 384 5.8 / 6.3
+// the whole network at 256 / 32 (host buffers) / 1 images 716 / 394 / 132.5 -> 695 / 386 / 131.1. Tried: phase 2's constants under way from the start on (registers spill from K = 96
+// on: 23.8 -> 25.5), the requants' constants from the host (no change, and spills), more tiles prefetched, or strips of 26, 32 or 53 KB (no change).
 // ---------------------------------------------------------------------------
 template <int KS, int S, bool RUNS>
 __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpandDwArgs p, FastDiv divW, FastDiv divH, FastDiv divCols, FastDiv divSegments) {
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
     const int fr = lane & 31, half = lane >> 5;
     v4i w[KS];
     v16i bias;
-    int scale[16];
+    v4i scale[4];
     {
         const int8_t *wrow = p.wexp + (size_t)(ch0 + fr) * p.Kp + 16 * half;
 #pragma unroll
@@ -76,8 +77,8 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 bias[4 * q + e] = b4[e];
-                scale[4 * q + e] = s4[e];
             }
+            scale[q] = s4;
         }
     }
     const int imageBytes = RUNS ? p.IH * p.IW * p.IC : 0;
@@ -127,7 +128,8 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
         return irWalkFrom(p, m, r, image, imageStep, rowStep, columnStep, first);
     };
     const int cellRowBytes = cellCols * kIrPitch, cellImageBytes = cellRows * cellRowBytes;
-    IrWalk cell = walkFrom(cellImageBytes, cellRowBytes, kIrPitch, (iyLo - iyFirst) * cellRowBytes + p.PL * kIrPitch + 4 * half);
+    const int planeBytes = images * cellImageBytes;
+    IrWalk cell = walkFrom(cellImageBytes, cellRowBytes, kIrPitch, (iyLo - iyFirst) * cellRowBytes + p.PL * kIrPitch + half * planeBytes);
     const int runRow = RUNS ? p.CS * p.IW * p.IC : 0, runColumn = RUNS ? p.CS * p.IC : 0;
     IrWalk run{};
     int khOff[KS];
@@ -157,12 +159,11 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
     loadTile(a0);
     {
         const int zp4 = (int)((uint32_t)(p.zp & 0xff) * 0x01010101u);
-        const int words = images * cellRows * cellCols * (kIrPitch / 4);
-        for (int i = tid * 4; i < words; i += 1024) *(v4i *)(cells + (size_t)i * 4) = v4i{zp4, zp4, zp4, zp4};  // LDS is rounded up to 16 bytes
+        for (int i = tid * 16; i < 2 * planeBytes; i += 4096) *(v4i *)(cells + i) = v4i{zp4, zp4, zp4, zp4};
     }
     __syncthreads();
     const WideRequant w1 = wideRequant(p.rq1);
-    withNarrowRequantMode(w1, [&](auto tag) {
+    withNarrowPackMode(w1, [&](auto tag) {
         constexpr int kMode = decltype(tag)::value;
         auto computeTile = [&](int t, v4i(&a)[KS]) {
             const int m = t * 32 + fr;
@@ -182,13 +183,13 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
             const bool inside = irHasCell(p, part, m, cell);
             irWalkOn(p, cell, cellImageBytes, cellRowBytes, kIrPitch);
             if (!inside) return;
+            v4i o;
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                int32_t v[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = requantT0<kMode>(acc[4 * q + e], scale[4 * q + e], 0, p.rq1, w1);
-                *(uint32_t *)(dst + 8 * q) = packBytes(v[0], v[1], v[2], v[3]);
+                const v4i t0 = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+                o[q] = (int)requantPack4<kMode>(t0, scale[q], 0, p.rq1, w1);
             }
+            *(v4i *)dst = o;
         };
         for (int t = wave; t < tiles; t += 8) {
             loadTile(a1);
@@ -198,110 +199,112 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
             computeTile(t + 4, a1);
         }
     });
+    // phase 2's weights and constants, under way while other waves widen: their registers are not free before
+    const int slot = lane & 15, group = lane >> 4;
+    // channels beyond C, half a chunk, are made of the chunk's first ones and stored nowhere
+    const bool whole = ch0 + 32 <= p.C, stored = whole || group < 2;
+    const uint32_t tapAt = whole || slot < 8 ? 8 * (slot >> 2) + (slot & 3) : 0, channelAt = stored ? 8 * group : 0;
+    uint32_t taps[2][3];
+    v4i bias2[2], scale2[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+#pragma unroll
+        for (int kh = 0; kh < 3; kh++) taps[j][kh] = (uint32_t)(p.wdw + (size_t)kh * p.C + ch0 + 4 * j)[tapAt];
+        bias2[j] = *(const v4i *)(p.bias2 + ch0 + 4 * j + channelAt);
+        scale2[j] = *(const v4i *)(p.scale2 + ch0 + 4 * j + channelAt);
+    }
     __syncthreads();
 
     // ---- phase 2 ----
-    constexpr int P = S == 1 ? 2 : 1;  // output columns of a thread
-    const int c4 = tid & 7, slot = tid >> 3;
-    if (ch0 + 4 * c4 >= p.C) return;
-    const int ch = ch0 + 4 * c4;
-    int wk[3][4], wks[3][4];
+    v4i wd[2][3];
 #pragma unroll
-    for (int kh = 0; kh < 3; kh++) {
-        const v4i w4 = *(const v4i *)(p.wdw + (size_t)kh * p.C + ch);
+    for (int j = 0; j < 2; j++) {
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            wk[kh][c] = w4[c];
-            wks[kh][c] = (int)((uint32_t)w4[c] << 8);
+        for (int kh = 0; kh < 3; kh++) {
+            const uint32_t tap = group < 3 ? (taps[j][kh] >> (8 * group) & 0xffu) << (8 * (slot & 3)) : 0u;
+#pragma unroll
+            for (int d = 0; d < 4; d++) wd[j][kh][d] = d == (slot >> 2) ? (int)tap : 0;
         }
     }
-    const v4i bias2 = *(const v4i *)(p.bias2 + ch), scale2 = *(const v4i *)(p.scale2 + ch);
     const WideRequant w2 = wideRequant(p.rq2);
-    const int colGroups = (p.OW + P - 1) / P, items = colGroups * p.segments * images;
-    const int rowBytes = cellCols * kIrPitch;
+    const int items = p.OW * p.segments * images, count = rows < p.segmentRows ? rows : p.segmentRows;
+    const uint32_t step = (uint32_t)(p.OW * p.C);
     int8_t *out = p.out + ((size_t)n * p.OH + oy0) * p.OW * p.C;
-    withNarrowRequantMode(w2, [&](auto tag) {
+    withNarrowPackMode(w2, [&](auto tag) {
         constexpr int kMode = decltype(tag)::value;
-        for (int item = slot; item < items; item += 32) {
-            int seg = 0, image = 0, j = item;
+        for (int first = wave * 16; first < items; first += 64) {
+            const int item = first + slot;
+            int seg = 0, image = 0, ox = item;
             if (p.segments * p.images > 1) {
                 seg = (int)fastDiv((uint32_t)item, divCols);
-                j -= seg * colGroups;
+                ox -= seg * p.OW;
             }
             if (p.images > 1) {
                 image = (int)fastDiv((uint32_t)seg, divSegments);
                 seg -= image * p.segments;
             }
-            const int oyA = seg * p.segmentRows, oyB = oyA + p.segmentRows < rows ? oyA + p.segmentRows : rows;
-            if (oyA >= oyB) continue;
-            const int ox = j * P;
-            const int8_t *src = cells + ((image * cellRows + oyA * S) * cellCols + ox * S) * kIrPitch + 4 * c4;
-            uint32_t dst = (uint32_t)(((image * p.OH + oyA) * p.OW + ox) * p.C + ch);
-            const bool second = P == 2 && ox + 1 < p.OW;
-            uint32_t ring[3][4];
-            auto row = [&](uint32_t(&o)[4]) {
-                const uint32_t x0 = *(const uint32_t *)src, x1 = *(const uint32_t *)(src + kIrPitch), x2 = *(const uint32_t *)(src + 2 * kIrPitch);
-                const uint32_t x3 = S == 1 ? *(const uint32_t *)(src + 3 * kIrPitch) : x2;  // stride 2: its weight is zero
-                const uint32_t lo01 = __builtin_amdgcn_perm(x1, x0, 0x05010400u), hi01 = __builtin_amdgcn_perm(x1, x0, 0x07030602u);
-                const uint32_t lo23 = S == 1 ? __builtin_amdgcn_perm(x3, x2, 0x05010400u) : x2, hi23 = S == 1 ? __builtin_amdgcn_perm(x3, x2, 0x07030602u) : x2;
-                o[0] = __builtin_amdgcn_perm(lo23, lo01, S == 1 ? 0x05040100u : 0x0c040100u);
-                o[1] = __builtin_amdgcn_perm(lo23, lo01, S == 1 ? 0x07060302u : 0x0c050302u);
-                o[2] = __builtin_amdgcn_perm(hi23, hi01, S == 1 ? 0x05040100u : 0x0c060100u);
-                o[3] = __builtin_amdgcn_perm(hi23, hi01, S == 1 ? 0x07060302u : 0x0c070302u);
-                src += rowBytes;
-            };
-            auto emit = [&](const uint32_t(&r0)[4], const uint32_t(&r1)[4], const uint32_t(&r2)[4]) {
-                int32_t v[P][4];
+            const int oyA = seg * p.segmentRows;
+            int left = rows - oyA < count ? rows - oyA : count;  // rows of its segment; a lane without any reads those of the first one
+            if (item >= items || left < 0) left = 0;
+            const int8_t *src = cells + (left > 0 ? image * cellImageBytes + oyA * S * cellRowBytes + ox * S * kIrPitch : 0) + (group < 3 ? group : 2) * kIrPitch;
+            if (!stored) left = 0;
+            uint32_t dst = (uint32_t)(((image * p.OH + oyA) * p.OW + ox) * p.C + ch0 + 8 * group);
+            v4i ring[3][2];
+            auto row = [&](v4i(&o)[2]) {
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    int32_t acc = __builtin_amdgcn_sdot4((int)r0[c], wk[0][c], bias2[c], false);
-                    acc = __builtin_amdgcn_sdot4((int)r1[c], wk[1][c], acc, false);
-                    acc = __builtin_amdgcn_sdot4((int)r2[c], wk[2][c], acc, false);
-                    v[0][c] = requantT0<kMode>(acc, scale2[c], 0, p.rq2, w2);
-                    if (P == 2) {
-                        acc = __builtin_amdgcn_sdot4((int)r0[c], wks[0][c], bias2[c], false);
-                        acc = __builtin_amdgcn_sdot4((int)r1[c], wks[1][c], acc, false);
-                        acc = __builtin_amdgcn_sdot4((int)r2[c], wks[2][c], acc, false);
-                        v[P - 1][c] = requantT0<kMode>(acc, scale2[c], 0, p.rq2, w2);
-                    }
-                }
-                *(uint32_t *)(out + dst) = packBytes(v[0][0], v[0][1], v[0][2], v[0][3]);
-                if (second) *(uint32_t *)(out + (dst + (uint32_t)p.C)) = packBytes(v[P - 1][0], v[P - 1][1], v[P - 1][2], v[P - 1][3]);
-                dst += (uint32_t)(p.OW * p.C);
+                for (int j = 0; j < 2; j++) o[j] = *(const v4i *)(src + j * planeBytes);
+                src += cellRowBytes;
             };
+            auto emit = [&](int r, const v4i(&r0)[2], const v4i(&r1)[2], const v4i(&r2)[2]) {
+                v2i o;
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    v4i acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wd[j][0], r0[j], bias2[j], 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wd[j][1], r1[j], acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wd[j][2], r2[j], acc, 0, 0, 0);
+                    o[j] = (int)requantPack4<kMode>(acc, scale2[j], 0, p.rq2, w2);
+                }
+                if (r < left) ((UnalignedV2 *)(out + dst))->v = o;
+                dst += step;
+            };
+            row(ring[0]);
             if (S == 1) {
-                row(ring[0]);
                 row(ring[1]);
-                for (int oy = oyA;;) {
+                for (int r = 0;;) {
                     row(ring[2]);
-                    emit(ring[0], ring[1], ring[2]);
-                    if (++oy >= oyB) break;
+                    emit(r, ring[0], ring[1], ring[2]);
+                    if (++r >= count) break;
                     row(ring[0]);
-                    emit(ring[1], ring[2], ring[0]);
-                    if (++oy >= oyB) break;
+                    emit(r, ring[1], ring[2], ring[0]);
+                    if (++r >= count) break;
                     row(ring[1]);
-                    emit(ring[2], ring[0], ring[1]);
-                    if (++oy >= oyB) break;
+                    emit(r, ring[2], ring[0], ring[1]);
+                    if (++r >= count) break;
                 }
             } else {
-                row(ring[0]);
-                for (int oy = oyA;;) {
+                for (int r = 0;;) {
                     row(ring[1]);
                     row(ring[2]);
-                    emit(ring[0], ring[1], ring[2]);
-                    if (++oy >= oyB) break;
+                    emit(r, ring[0], ring[1], ring[2]);
+                    if (++r >= count) break;
                     row(ring[1]);
                     row(ring[0]);
-                    emit(ring[2], ring[1], ring[0]);
-                    if (++oy >= oyB) break;
+                    emit(r, ring[2], ring[1], ring[0]);
+                    if (++r >= count) break;
                 }
             }
         }
     });
 }
 
-static size_t irLds(int images, int cellRows, int cellCols) { return ((size_t)images * cellRows * cellCols * kIrPitch + 15) / 16 * 16; }
+static size_t irLds(int images, int cellRows, int cellCols) { return (size_t)images * cellRows * cellCols * kIrPitch * 2; }
+// What a launch asks for: also the rows of cells below the strip that lanes of the last segment read where the segments make more rows than it has.
+static size_t irLaunchLds(const IrExpandDwArgs &a) {
+    const int rows = irCellRows(a, a.images, a.stripRows), read = (a.segments * a.segmentRows - 1) * a.S + 3;
+    return irLds(a.images, rows, a.cellCols) + (read > rows ? (size_t)(read - rows) * a.cellCols * kIrPitch : 0);
+}
 constexpr size_t kIrMaxLds = 64 * 1024;
+constexpr int kIrMaxImages = 12;  // of a workgroup
 
 bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL) {
     // a window of three rows with at most two above the image reaches into it
@@ -312,8 +315,8 @@ template <int KS, int S, bool RUNS = false>
 static hipError_t launchIr(const IrExpandDwArgs &a, const LaunchCtx &ctx) {
     const long long blocks = (long long)((a.N + a.images - 1) / a.images) * a.strips * ((a.C + kIrChunk - 1) / kIrChunk);
     if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    THIP_ENQUEUE(ctx, kernelLabel("ir_expand_dw_i8", {KS, S, (int)RUNS}), (ir_expand_dw_i8<KS, S, RUNS>), dim3((unsigned)blocks), dim3(256), irLds(a.images, irCellRows(a, a.images, a.stripRows), a.cellCols), a,
-                 makeFastDiv((uint32_t)a.W), makeFastDiv((uint32_t)a.H), makeFastDiv((uint32_t)(S == 1 ? (a.OW + 1) / 2 : a.OW)), makeFastDiv((uint32_t)a.segments));
+    THIP_ENQUEUE(ctx, kernelLabel("ir_expand_dw_i8", {KS, S, (int)RUNS}), (ir_expand_dw_i8<KS, S, RUNS>), dim3((unsigned)blocks), dim3(256), irLaunchLds(a), a,
+                 makeFastDiv((uint32_t)a.W), makeFastDiv((uint32_t)a.H), makeFastDiv((uint32_t)a.OW), makeFastDiv((uint32_t)a.segments));
     return hipGetLastError();
 }
 
@@ -331,6 +334,18 @@ static hipError_t launchIrS(const IrExpandDwArgs &a, const LaunchCtx &ctx) {
     }
 }
 
+// The time of a launch whose workgroups make `images` whole images each, us.  A CU runs as many workgroups at a time as its registers and LDS hold, and each such
+// round costs a start and what the tiles of pixels and the rows of 16 results of its workgroups take together.  Fitted to 256 images of 14x14x64 -> 384 by 1, 2, 4, 5, 6, 8, 9 and 11
+// (21.6, 17.0, 15.2, 19.1, 20.2, 18.0, 18.8, 21.8 us) and of 7x7x160 -> 960 (40.8, 26.4, 19.8, 19.3, 17.7, 15.5, 15.8, 15.1): a last round that is nearly empty costs
+// as much as what it saves.
+static double irTime(const IrExpandDwArgs &a, int images, size_t lds) {
+    const int KS = a.CKH > 0 ? (a.CKH + 1) / 2 : (a.K + 31) / 32, byLds = (int)(160 * 1024 / (lds + 1024)), perCu = byLds < (KS <= 3 ? 4 : 3) ? byLds : KS <= 3 ? 4 : 3;
+    const long long blocks = (long long)((a.N + images - 1) / images) * ((a.C + kIrChunk - 1) / kIrChunk), room = 256LL * perCu, rest = (blocks % room + 255) / 256;
+    const int tiles = (images * a.H * a.W + 31) / 32, columns = a.OW * images, segments = columns >= 64 ? 1 : 64 / columns, rows = (columns * segments + 15) / 16 * ((a.OH + segments - 1) / segments);
+    const double one = tiles * (0.05 + 0.006 * KS) + rows * 0.033, start = 2.5;
+    return (double)(blocks / room) * (start + perCu * one) + (rest > 0 ? start + (double)rest * one : 0.0);
+}
+
 bool planIrExpandDw(IrExpandDwArgs *args) {
     IrExpandDwArgs &a = *args;
     if (!a.x || !a.wexp || !a.bias1 || !a.scale1 || !a.wdw || !a.bias2 || !a.scale2 || !a.out) return false;
@@ -340,7 +355,7 @@ bool planIrExpandDw(IrExpandDwArgs *args) {
         // the runs of every output pixel start inside the image or its padding (the kernel checks every byte against the image)
         if (a.IH <= 0 || a.IW <= 0 || a.IC <= 0 || a.CS <= 0 || a.CPT < 0 || a.CPL < 0 || a.runBytes <= 0 || a.runBytes > 16 || a.runBytes % a.IC != 0) return false;
         if (a.xBytes != (int64_t)a.N * a.IH * a.IW * a.IC || a.xBytes < 16) return false;
-        // a workgroup's eight images and the padding around them, in 31 bits
+        // a workgroup's images and the padding around them, in 31 bits
         if ((long long)a.IH * a.IW * a.IC > (1LL << 27)) return false;
     } else if ((uintptr_t)a.x & 15) {
         return false;
@@ -353,32 +368,36 @@ bool planIrExpandDw(IrExpandDwArgs *args) {
     if ((long long)a.C > kIrMaxChannels) return false;
     // Four workgroups per CU (160 KB of LDS, 16 waves) overlap one another's phases: strips as high as 40 KB of cells hold
     // (56x56x32 -> 144, 256 images: 79 us at 20 KB, whose strips make more rows twice, 69 at 40, 76 at 64), lower where that
-    // leaves fewer than two workgroups per CU (14x14x96 -> 576, 32 images: 8.0 us with at least 512, 9.1 with 1024), and down
-    // to four rows; images that leave room share a workgroup (7x7x160 -> 960, 256 images: 37.3 us one by one, 17.3 by eight).
-    // Images that share cost no rows twice, so where the registers (K <= 64) let eight workgroups run on a CU they get 20 KB each
-    // (14x14x64 -> 384, 256 images: 23.4 -> 19.5 us; with K = 96 18.6 -> 21.0 at stride 2, with 160 18.7 -> 20.0, the other way).
+    // leaves fewer than two workgroups per CU (14x14x96 -> 576, 32 images: 8.0 us with at least 512, 9.1 with 1024), down
+    // to four rows, and to one where not every CU has a workgroup (a mobile network of one image: 133.4 us with four rows, 131.1 so).
+    // Images that leave room share a workgroup, as many as irTime says.
     constexpr size_t ldsAim = 40 * 1024;
     constexpr long long wgAim = 512;
     const long long perStrip = (long long)a.N * ((a.C + kIrChunk - 1) / kIrChunk);
     int strips = 1;
     auto rowsOf = [&](int s) { return (a.OH + s - 1) / s; };
     auto lds = [&](int images, int s) { return irLds(images, irCellRows(a, images, rowsOf(s)), a.cellCols); };
-    // phase 1's rounds of a workgroup's four waves: where not even every second CU has a workgroup they are the launch's time
-    auto rounds = [&](int s) { return (((rowsOf(s) - 1) * a.S + 3) * a.W + 127) / 128; };
-    while (rowsOf(strips) > 1 && (lds(1, strips) > ldsAim || (perStrip * strips < wgAim && rowsOf(strips) > 4) || (perStrip * strips < 128 && rounds(strips) > 2))) strips++;
+    while (rowsOf(strips) > 1 && (lds(1, strips) > ldsAim || (perStrip * strips < wgAim && rowsOf(strips) > 4) || perStrip * strips < 256)) strips++;
     a.stripRows = rowsOf(strips);
     a.strips = (a.OH + a.stripRows - 1) / a.stripRows;
+    // the launch's time by the rounds of workgroups that it takes: irTime
     a.images = 1;
     if (a.strips == 1) {
-        const size_t aim = a.CKH == 0 && a.K <= 64 ? ldsAim / 2 : ldsAim;
-        while (a.images < 8 && lds(a.images + 1, 1) <= aim && perStrip / (a.images + 1) >= 1024) a.images++;
+        double best = irTime(a, 1, lds(1, 1));
+        for (int images = 2; images <= kIrMaxImages && images <= a.N && lds(images, 1) <= kIrMaxLds; images++) {
+            const double time = irTime(a, images, lds(images, 1));
+            if (time < best) {
+                best = time;
+                a.images = images;
+            }
+        }
     }
     // 128 pixels on, in images, rows and columns
     a.stepImages = a.images > 1 ? 128 / (a.H * a.W) : 0;
     a.stepRows = (128 - a.stepImages * a.H * a.W) / a.W;
     a.stepColumns = (128 - a.stepImages * a.H * a.W) % a.W;
-    const int P = a.S == 1 ? 2 : 1, columns = (a.OW + P - 1) / P * a.images;
-    a.segments = columns >= 32 ? 1 : 32 / columns;
+    const int columns = a.OW * a.images;
+    a.segments = columns >= 64 ? 1 : 64 / columns;
     if (a.segments > a.stripRows) a.segments = a.stripRows;
     a.segmentRows = (a.stripRows + a.segments - 1) / a.segments;
     a.segments = (a.stripRows + a.segmentRows - 1) / a.segmentRows;
