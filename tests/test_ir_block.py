@@ -115,3 +115,17 @@ def test_other_requants_stay_apart(device, monkeypatch):
         got, _ = run_on_gpu(device, wl, via="device", launched=launched)
         assert "ir_block_i8" not in families(launched), launched
         assert_bit_exact(got[0], oracle_network(wl), wl.name)
+
+
+@pytest.mark.parametrize("N", [1, 3])
+@pytest.mark.parametrize("H,W,C,first", [(13, 71, 4, (4, 1, (3, 3, 3, 3))), (13, 70, 3, (4, 1, (0, 3, 3, 0))), (9, 40, 1, (3, 1, (2, 2, 2, 2))), (8, 35, 5, (3, 2, (2, 1, 0, 2))), (40, 150, 3, (3, 2, (1, 1, 1, 1))),
+                                         (5, 3, 4, (4, 1, (3, 3, 3, 3)))])
+def test_padding_of_a_first_layer(device, N, H, W, C, first, monkeypatch):
+    """Runs that begin or end in the padding at every byte of their dwords, in the first, the last and an inner image."""
+    monkeypatch.setenv("THIP_IR_BLOCK", "1")
+    wl = block(N, H, W, C, 32, 16, 1, first=first)
+    print("[gpu-case]", wl.name, flush=True)
+    launched = []
+    got, _ = run_on_gpu(device, wl, via="device", launched=launched)
+    assert families(launched) == ["ir_block_i8"], launched
+    assert_bit_exact(got[0], oracle_network(wl), wl.name)

@@ -44,7 +44,7 @@ constexpr int irBlockTiles(int S) { return S == 1 ? 6 : 10; }
 // Why: apart, the depthwise result (2.3 MB per image of a 224 x 224 mobile network) is written and read back by a launch of its own.  Bound by the
 // waves' issue: a wave issues one vector instruction in 8 cycles at most and most of these take the SIMD 4, so two waves a SIMD fill it only while neither
 // waits; about half of the cycles are vector instructions.  Measured, us, the two launches / this one:
-//   batch 256  224x224x3 -> 112x112x32 -> 16 115 / 93, 112x112x16 -> 96 stride 2 -> 32 123 / 94, 56x56x32 -> 144 -> 32 and the add 110 / 87,
+//   batch 256  224x224x3 -> 112x112x32 -> 16 115 / 90, 112x112x16 -> 96 stride 2 -> 32 123 / 94, 56x56x32 -> 144 -> 32 and the add 110 / 87,
 //              its stride 2 58 / 41, 28x28x32 -> 192 -> 32 41 / 27, stride 2 -> 64 22.4 / 20.3
 //   batch 32   28.0 / 17.2, 24.2 / 19.6, 24.1 / 19.1; 14.4 / 13.3, 12.2 / 13.4, 9.5 / 12.0 (the last two left to the two launches)
 //   batch 1    9.7 / 5.6, 8.4 / 8.1; 8.0 / 9.0 and 7.4 / 9.9 (left)
@@ -92,6 +92,9 @@ __global__ __launch_bounds__(256, RUNS ? 4 : 2) void ir_block_i8(IrBlockArgs p, 
     const int64_t before = (int64_t)n * imageBytes, behind = p.xBytes - before - 16;
     const int runLo = before < 1024 ? -(int)before : -1024, runHi = behind < 0x7fffffff ? (int)behind : 0x7fffffff;
     const int runRow = p.IW * p.IC;
+    int khOff[KS];  // from a window's first row to the lane's; beyond the window its first one again, against zero weights
+#pragma unroll
+    for (int s = 0; s < KS; s++) khOff[s] = (2 * s + half < p.CKH ? 2 * s + half : 0) * runRow;
     struct Tile {
         int cell, y, at;  // RUNS: its window's first row, and where in a row it starts
     };
@@ -110,10 +113,10 @@ __global__ __launch_bounds__(256, RUNS ? 4 : 2) void ir_block_i8(IrBlockArgs p, 
             e.cell = cellOf(m, iy, ix);
             e.y = iy * p.CS - p.CPT;
             e.at = (ix * p.CS - p.CPL) * p.IC;
+            const int first = e.y * runRow + e.at;
 #pragma unroll
             for (int s = 0; s < KS; s++) {
-                const int kh = 2 * s + half < p.CKH ? 2 * s + half : 0;
-                const int off = e.cell != half * planeBytes + trash ? (e.y + kh) * runRow + e.at : 0;
+                const int off = first + khOff[s];
                 a[s] = ((const UnalignedV4 *)(x + (off < runLo ? runLo : off > runHi ? runHi : off)))->v;
             }
         } else {
@@ -189,15 +192,45 @@ __global__ __launch_bounds__(256, RUNS ? 4 : 2) void ir_block_i8(IrBlockArgs p, 
     const WideRequant w1 = wideRequant(p.rq1), w2 = wideRequant(p.rq2), w3 = wideRequant(p.rq3);
     auto widenTile = [&](const Tile &e, v4i(&a)[KS], int8_t *buffer) {
         if constexpr (RUNS) {
-            // runs that were read elsewhere than they lie, or that reach into the padding, are put right
-            const bool bad = e.y < 0 || e.y + p.CKH > p.IH || e.at < 0 || e.at + p.runBytes > runRow || (e.y + p.CKH - 1) * runRow + e.at > runHi;
-            if (__ballot(bad && e.cell != half * planeBytes + trash) != 0) {
+            // runs that reach into the padding, or that were read elsewhere than they lie (at the tensor's two ends), are put right
+            const int first = e.y * runRow + e.at, last = first + (p.CKH - 1) * runRow;
+            const bool wanted = e.cell != half * planeBytes + trash;
+            const bool bad = e.y < 0 || e.y + p.CKH > p.IH || e.at < 0 || e.at + p.runBytes > runRow || last > runHi;
+            if (__ballot(bad && wanted) != 0) {
                 const uint32_t zp4 = (uint32_t)(p.czp & 0xff) * 0x01010101u;
+                if (__ballot((first < runLo || last > runHi) && wanted) != 0) {
 #pragma unroll
-                for (int s = 0; s < KS; s++) {
-                    const int kh = 2 * s + half < p.CKH ? 2 * s + half : 0, off = (e.y + kh) * runRow + e.at;
-                    // a row of the window outside the image is all padding
-                    a[s] = fixRun16(a[s], off - (off < runLo ? runLo : off > runHi ? runHi : off), -e.at, (unsigned)(e.y + kh) >= (unsigned)p.IH ? 0 : runRow - e.at, zp4);
+                    for (int s = 0; s < KS; s++) {
+                        const int kh = 2 * s + half < p.CKH ? 2 * s + half : 0, off = first + khOff[s];
+                        // a row of the window outside the image is all padding
+                        a[s] = fixRun16(a[s], off - (off < runLo ? runLo : off > runHi ? runHi : off), -e.at, (unsigned)(e.y + kh) >= (unsigned)p.IH ? 0 : runRow - e.at, zp4);
+                    }
+                } else {
+                    // masks of the bytes inside the row, the same for every row of the window: a quarter of fixRun16's instructions, in half of the tiles of a right-hand
+                    // block (224x224x3 -> 112x112x32 -> 16, 256 images: 97 us with fixRun16, 90 so)
+                    uint32_t in[4];
+#pragma unroll
+                    for (int d = 0; d < 4; d++) {
+                        const int past = 8 * (4 * d + 4 - (runRow - e.at));  // bits of the dword behind the row
+                        in[d] = (uint32_t)(0xffffffffull >> (past < 0 ? 0 : past > 32 ? 32 : past));
+                    }
+                    if (__ballot(e.at < 0) != 0) {
+#pragma unroll
+                        for (int d = 0; d < 4; d++) {
+                            const int before = 8 * (-e.at - 4 * d);
+                            in[d] &= (uint32_t)(0xffffffffull << (before < 0 ? 0 : before > 32 ? 32 : before));
+                        }
+                    }
+#pragma unroll
+                    for (int s = 0; s < KS; s++) {
+                        const int kh = 2 * s + half < p.CKH ? 2 * s + half : 0;
+                        const bool row = (unsigned)(e.y + kh) < (unsigned)p.IH;
+#pragma unroll
+                        for (int d = 0; d < 4; d++) {
+                            const uint32_t keep = row ? in[d] : 0u;
+                            a[s][d] = (int)(((uint32_t)a[s][d] & keep) | (zp4 & ~keep));
+                        }
+                    }
                 }
             }
         }
