@@ -44,13 +44,13 @@ constexpr int irBlockTiles(int S) { return S == 1 ? 6 : 10; }
 // Why: apart, the depthwise result (2.3 MB per image of a 224 x 224 mobile network) is written and read back by a launch of its own.  Bound by the
 // waves' issue: a wave issues one vector instruction in 8 cycles at most and most of these take the SIMD 4, so two waves a SIMD fill it only while neither
 // waits; about half of the cycles are vector instructions.  Measured, us, the two launches / this one:
-//   batch 256  224x224x3 -> 112x112x32 -> 16 115 / 90, 112x112x16 -> 96 stride 2 -> 32 123 / 94, 56x56x32 -> 144 -> 32 and the add 110 / 87,
-//              its stride 2 58 / 41, 28x28x32 -> 192 -> 32 41 / 27, stride 2 -> 64 22.4 / 20.3
-//   batch 32   28.0 / 17.2, 24.2 / 19.6, 24.1 / 19.1; 14.4 / 13.3, 12.2 / 13.4, 9.5 / 12.0 (the last two left to the two launches)
-//   batch 1    9.7 / 5.6, 8.4 / 8.1; 8.0 / 9.0 and 7.4 / 9.9 (left)
+//   batch 256  224x224x3 -> 112x112x32 -> 16 108 / 81, 112x112x16 -> 96 stride 2 -> 32 104 / 97, 56x56x32 -> 144 -> 32 and the add 98 / 86,
+//              its stride 2 48 / 42, 28x28x32 -> 192 -> 32 42 / 29, stride 2 -> 64 24 / 21
+//   batch 32   26.2 / 16.3, 22.1 / 17.6, 21.5 / 18.7, 13.2 / 12.3, 11.9 / 11.5; 9.9 / 13.3 (left to the two launches)
+//   batch 1    12.6 / 4.9; 7.7 / 7.8, 7.8 / 9.3, 7.2 / 10.1 (left)
 // and left at any batch: 14x14x64 -> 384 -> 64 24.9 / 33, 14x14x96 -> 576 -> 96 39.6 / 53, whose chunks are too small for what each costs.  Tried on it: four waves a SIMD
 // (their registers hold half the rows, the chunks' constants are fetched twice as often: 85 -> 103), waves that only widen beside waves that
-// only convolve (94), the next row's cells and products ahead of this one's requant (85).
+// only convolve (94), the next row's cells and products, or the next tile's, ahead of this one's requant (85; 56x56x32 -> 144 -> 32 89.7 -> 92.3).
 // ---------------------------------------------------------------------------
 template <int KS, int S, bool RUNS, int OT, int DW>
 __global__ __launch_bounds__(256, RUNS ? 4 : 2) void ir_block_i8(IrBlockArgs p, FastDiv divRegion, FastDiv divColumns) {
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(256, RUNS ? 4 : 2) void ir_block_i8(IrBlockArgs p, 
                     }
                 } else {
                     // masks of the bytes inside the row, the same for every row of the window: a quarter of fixRun16's instructions, in half of the tiles of a right-hand
-                    // block (224x224x3 -> 112x112x32 -> 16, 256 images: 97 us with fixRun16, 90 so)
+                    // block (224x224x3 -> 112x112x32 -> 16, 256 images: 97 us with fixRun16, 90 so, the narrow convolution as it was)
                     uint32_t in[4];
 #pragma unroll
                     for (int d = 0; d < 4; d++) {
@@ -273,21 +273,27 @@ __global__ __launch_bounds__(256, RUNS ? 4 : 2) void ir_block_i8(IrBlockArgs p, 
         }
     };
     // one output row of the lane's 4 OT channels, its requant, the add and the store
-    auto finishRow = [&](int r, const v4i(&sums)[OT], const v4i(&scale3)[OT], const uint32_t(&other)[OT]) {
-        withPackedRequant(w3, [&](auto tag) {
-            if (r < left) {
+    auto finishRow = [&](auto mode, auto adds, int r, const v4i(&sums)[OT], const v4i(&scale3)[OT], const uint32_t(&other)[OT]) {
+        if (r < left) {
 #pragma unroll
-                for (int t = 0; t < OT; t++) {
-                    uint32_t o = requantPack4<decltype(tag)::value>(sums[t], scale3[t], 0, p.rq3, w3);
-                    if (p.skip) o = residualAdd4<true>(o, other[t], p.addSkipFirst != 0, p.addW0, p.addW1, 0, 1, 0, p.arq, p.addFolded);
-                    *(uint32_t *)(p.out + firstOut + (laneOut + r * step + 4 * t)) = o;
-                }
+            for (int t = 0; t < OT; t++) {
+                uint32_t o = requantPack4<decltype(mode)::value>(sums[t], scale3[t], 0, p.rq3, w3);
+                if (decltype(adds)::value) o = residualAdd4<true>(o, other[t], p.addSkipFirst != 0, p.addW0, p.addW1, 0, 1, 0, p.arq, p.addFolded);
+                *(uint32_t *)(p.out + firstOut + (laneOut + r * step + 4 * t)) = o;
             }
+        }
+    };
+    // f(mode, adds): which requant the narrow convolution has and whether an add follows, asked once: branches in every row keep a wave from issuing (256 images,
+    // us, in every row / once: 224x224x3 -> 112x112x32 -> 16 90.4 / 80.8, 56x56x32 -> 144 -> 32 and the add 89.7 / 86.0, 28x28x32 -> 192 -> 32 30.0 / 28.9)
+    auto withFinish = [&](auto &&f) {
+        withPackedRequant(w3, [&](auto mode) {
+            if (p.skip) f(mode, std::true_type{});
+            else f(mode, std::false_type{});
         });
     };
-    auto loadSkip = [&](int r, uint32_t(&other)[OT]) {
+    auto loadSkip = [&](auto adds, int r, uint32_t(&other)[OT]) {
 #pragma unroll
-        for (int t = 0; t < OT; t++) other[t] = p.skip && r < left ? *(const uint32_t *)(p.skip + firstOut + (laneOut + r * step + 4 * t)) : 0u;
+        for (int t = 0; t < OT; t++) other[t] = decltype(adds)::value && r < left ? *(const uint32_t *)(p.skip + firstOut + (laneOut + r * step + 4 * t)) : 0u;
     };
     v4i bias3[OT], scale3[OT];
     auto loadNarrow = [&](const int32_t *from, v4i(&to)[OT]) {
@@ -337,14 +343,16 @@ __global__ __launch_bounds__(256, RUNS ? 4 : 2) void ir_block_i8(IrBlockArgs p, 
         loadNarrow(p.bias3, bias3);
         loadNarrow(p.scale3, scale3);
         __syncthreads();
-        depthwise(cells, [&](auto tag, long o) {
-            constexpr int r = decltype(tag)::value;
-            uint32_t other[OT];
-            loadSkip(r, other);
-            v4i sums[OT];
+        withFinish([&](auto mode, auto adds) {
+            depthwise(cells, [&](auto tag, long o) {
+                constexpr int r = decltype(tag)::value;
+                uint32_t other[OT];
+                loadSkip(adds, r, other);
+                v4i sums[OT];
 #pragma unroll
-            for (int t = 0; t < OT; t++) sums[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wproj[t], o, bias3[t], 0, 0, 0);
-            finishRow(r, sums, scale3, other);
+                for (int t = 0; t < OT; t++) sums[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wproj[t], o, bias3[t], 0, 0, 0);
+                finishRow(mode, adds, r, sums, scale3, other);
+            });
         });
     } else {
         v4i sum[RT][OT];
@@ -371,11 +379,13 @@ __global__ __launch_bounds__(256, RUNS ? 4 : 2) void ir_block_i8(IrBlockArgs p, 
             __syncthreads();
         }
         loadNarrow(p.scale3, scale3);
-        uint32_t other[RT][OT];
+        withFinish([&](auto mode, auto adds) {
+            uint32_t other[RT][OT];
 #pragma unroll
-        for (int r = 0; r < RT; r++) loadSkip(r, other[r]);
+            for (int r = 0; r < RT; r++) loadSkip(adds, r, other[r]);
 #pragma unroll
-        for (int r = 0; r < RT; r++) finishRow(r, sum[r], scale3, other[r]);
+            for (int r = 0; r < RT; r++) finishRow(mode, adds, r, sum[r], scale3, other[r]);
+        });
     }
 }
 
