@@ -41,7 +41,7 @@ __host__ __device__ inline IrStrip irStrip(const IrExpandDwArgs &p, int n, int s
 
 // A wave's next tile lies 128 pixels on.  Where its pixels are (the row and column of the cell, the cell, the first run) is
 // advanced by a constant and put right where a row or an image ends, without the divisions and products that say it for any pixel:
-// the launch is bound by the vector pipes (90 % of its busy cycles). Vector instructions of 256 images, millions of waves': the first
+// vector instructions are most of the launch. With dot products behind it, those of 256 images, millions of waves': the first
 // layer 47.4 -> 40.9, 112x112x16 -> 96 52.9 -> 49.5.
 struct IrWalk {
     int column, row, at;  // at: bytes, of the cell from `cells` or of the first run from x

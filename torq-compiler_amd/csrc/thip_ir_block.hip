@@ -41,14 +41,14 @@ constexpr int irBlockTiles(int S) { return S == 1 ? 6 : 10; }
 // RUNS: a convolution over few channels in the widening one's place (the first layer of an image network), as in ir_expand_dw_i8, to one chunk at most: there
 // are no sums to keep, so four waves a SIMD overlap one another's phases, and a strip may be a block of columns of its rows.
 //
-// Why: apart, the depthwise result (2.3 MB per image of a 224 x 224 mobile network) is written and read back by a launch of its own.  Bound by the
-// waves' issue: a wave issues one vector instruction in 8 cycles at most and most of these take the SIMD 4, so two waves a SIMD fill it only while neither
-// waits; about half of the cycles are vector instructions.  Measured, us, the two launches / this one:
+// Why: apart, the depthwise result (2.3 MB per image of a 224 x 224 mobile network) is written and read back by a launch of its own.  Bound by
+// vector instructions and MFMAs that two waves a SIMD overlap in part: an instruction takes the SIMD 4.3 to 4.6 cycles (a wave alone issues one in 5 to 5.7), which is 58 % of the cycles
+// (75 % of a first layer's, at four waves), and MFMAs 15 to 20 %.  Measured, us, the two launches / this one:
 //   batch 256  224x224x3 -> 112x112x32 -> 16 108 / 81, 112x112x16 -> 96 stride 2 -> 32 104 / 97, 56x56x32 -> 144 -> 32 and the add 98 / 86,
 //              its stride 2 48 / 42, 28x28x32 -> 192 -> 32 42 / 29, stride 2 -> 64 24 / 21
 //   batch 32   26.2 / 16.3, 22.1 / 17.6, 21.5 / 18.7, 13.2 / 12.3, 11.9 / 11.5; 9.9 / 13.3 (left to the two launches)
 //   batch 1    12.6 / 4.9; 7.7 / 7.8, 7.8 / 9.3, 7.2 / 10.1 (left)
-// and left at any batch: 14x14x64 -> 384 -> 64 24.9 / 33, 14x14x96 -> 576 -> 96 39.6 / 53, whose chunks are too small for what each costs.  Tried on it: four waves a SIMD
+// and left at any batch: 14x14x64 -> 384 -> 64 23.7 / 33, 14x14x96 -> 576 -> 96 38.5 / 53, whose chunks are too small for what each costs.  Tried on it: four waves a SIMD
 // (their registers hold half the rows, the chunks' constants are fetched twice as often: 85 -> 103), waves that only widen beside waves that
 // only convolve (94), the next row's cells and products, or the next tile's, ahead of this one's requant (85; 56x56x32 -> 144 -> 32 89.7 -> 92.3).
 // ---------------------------------------------------------------------------
