@@ -101,6 +101,7 @@ def test_rows_no_window_reaches(device, kw):
 @pytest.mark.parametrize("kw", [
     dict(N=1, H=9, W=10, C=32, E=48, stride=1), dict(N=1, H=11, W=3, C=16, E=32, stride=2), dict(N=1, H=5, W=65, C=16, E=32, stride=1),   # segments with fewer rows, or none
     dict(N=257, H=7, W=7, C=160, E=960, stride=1), dict(N=259, H=13, W=14, C=96, E=592, stride=1), dict(N=66, H=2, W=1, C=64, E=1040, stride=1),  # a last workgroup of fewer images
+    dict(N=1, H=5, W=640, C=16, E=32, stride=1), dict(N=1, H=5, W=640, C=16, E=32, stride=2), dict(N=600, H=34, W=5, C=16, E=272, stride=1), dict(N=300, H=66, W=3, C=32, E=272, stride=2),   # the widest rows, and the most LDS
     dict(N=2, H=12, W=12, C=32, E=48, stride=1, top=100), dict(N=2, H=12, W=12, C=32, E=48, stride=2, shift=41), dict(N=2, H=9, W=9, C=3, E=48, stride=1, first=(3, 1, (1, 1, 1, 1)), top=90),
 ], ids=lambda kw: "x".join(str(v) for v in kw.values()))
 def test_expand_depthwise_lanes(device, kw):

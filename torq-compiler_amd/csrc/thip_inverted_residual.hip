@@ -384,7 +384,8 @@ bool planIrExpandDw(IrExpandDwArgs *args) {
     a.images = 1;
     if (a.strips == 1) {
         double best = irTime(a, 1, lds(1, 1));
-        for (int images = 2; images <= kIrMaxImages && images <= a.N && lds(images, 1) <= kIrMaxLds; images++) {
+        // room for the rows below the last strip (irLaunchLds): at most 64 / columns of them a stride, 6 KB
+        for (int images = 2; images <= kIrMaxImages && images <= a.N && lds(images, 1) <= kIrMaxLds - 6 * 1024; images++) {
             const double time = irTime(a, images, lds(images, 1));
             if (time < best) {
                 best = time;
@@ -401,7 +402,7 @@ bool planIrExpandDw(IrExpandDwArgs *args) {
     if (a.segments > a.stripRows) a.segments = a.stripRows;
     a.segmentRows = (a.stripRows + a.segments - 1) / a.segments;
     a.segments = (a.stripRows + a.segmentRows - 1) / a.segmentRows;
-    return true;
+    return irLaunchLds(a) <= kIrMaxLds;
 }
 
 hipError_t launchIrExpandDw(const IrExpandDwArgs &in, const LaunchCtx &ctx) {
