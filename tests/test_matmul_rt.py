@@ -34,12 +34,33 @@ def test_runtime_input2(device, kw, tmp_path):
     assert_bit_exact(got[0], want, wl.name + " record by record")
 
 
-@pytest.mark.parametrize("K", [1, 16, 127, 128, 129, 143, 144, 256, 257, 300, 400, 513])
-@pytest.mark.parametrize("B, M, N", [(2, 33, 17), (16, 1, 144), (9, 130, 250), (24, 400, 520)], ids=["32rows-ragged", "one-row", "64rows", "128rows"])
-def test_k_tiles(device, B, M, N, K):
-    """The ends of k-tiles: one, two and an odd number of them, rows of B that end a byte before, at and behind a chunk."""
-    wl = w.matmul_workload(B=B, M=M, K=K, N=N, out_dtype=np.int32, seed=K)
+# the smallest tile with one group of waves and with two, 64 rows, 128 rows: (B, M, N), template arguments up to the k-tile groups
+TILES = [((2, 33, 17), (32, 1, 4)), ((16, 1, 144), (32, 1, 4)), ((16, 65, 1030), (64, 2, 2)), ((24, 400, 520), (128, 2, 2))]
+DTYPE_CODES = {np.int8: 1, np.int16: 2, np.int32: 3}
+
+
+def on_tile(device, wl, rows, K, out):
+    """Runs wl on the GPU, on tiles of `rows` and no others."""
+    print("[gpu-case]", wl.name, K, flush=True)
     launched = []
     got, _ = run_on_gpu(device, wl, via="device", launched=launched)
-    assert families(launched) == ["igemm_rt_i8"], launched
+    groups = 2 if rows[0] == 32 and K > 128 else 1
+    assert launched == ["igemm_rt_i8<%d,%d,%d,%d,%d>" % (rows + (DTYPE_CODES[out], groups))], launched
     assert_bit_exact(got[0], oracle_eval(wl)[0], wl.name)
+
+
+@pytest.mark.parametrize("K", [1, 16, 127, 128, 129, 143, 144, 256, 257, 300, 400, 513])
+@pytest.mark.parametrize("sizes, rows", TILES, ids=["32rows-ragged", "one-row", "64rows", "128rows"])
+def test_k_tiles(device, sizes, rows, K):
+    """The ends of k-tiles: one, two and an odd number of them, rows of B that end a byte before, at and behind a chunk."""
+    B, M, N = sizes
+    on_tile(device, w.matmul_workload(B=B, M=M, K=K, N=N, out_dtype=np.int32, seed=K), rows, K, np.int32)
+
+
+@pytest.mark.parametrize("K", [129, 400])
+@pytest.mark.parametrize("kw", [I8, dict(out_dtype=np.int16)], ids=["int8", "int16"])
+@pytest.mark.parametrize("sizes, rows", TILES, ids=["32rows-ragged", "one-row", "64rows", "128rows"])
+def test_k_tiles_of_narrow_results(device, sizes, rows, kw, K):
+    """Results narrower than the sums behind a loop of several k-tiles, with columns that fill no store."""
+    B, M, N = sizes
+    on_tile(device, w.matmul_workload(B=B, M=M, K=K, N=N - 1, seed=K, **kw), rows, K, kw["out_dtype"])

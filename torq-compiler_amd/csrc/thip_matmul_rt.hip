@@ -1,10 +1,13 @@
 // gfx950 kernel of torq_hl.matmul on int8 with a second operand that is produced at run time: igemm_rt_i8, a batch of
 // products in one launch, input2 read as it lies in memory.
+#include <mutex>
+
 #include "thip_kernels_common.h"
 
 namespace thip {
 
-constexpr int kRtRowB = 160;  // bytes of LDS from one row of B to the next: 8 rows of 32 columns lie in distinct banks
+// Bytes of LDS from one row of B to the next.
+constexpr int rtRowB(int BM) { return BM > 64 ? 160 : 128; }
 
 // ds_read_b64_tr_b8: of 16 lanes' 8 bytes each, as 8 rows of 16, a lane gets a column.
 __device__ __forceinline__ v2i readTransposed(const int8_t *p) {
@@ -19,22 +22,24 @@ __device__ __forceinline__ v2i readTransposed(const int8_t *p) {
 // (4 x 1024x128x1024 -> int16: eight launches, 47 us for 9.4 MB of operands).  Here a workgroup copies the B tile into LDS as it
 // lies, 16 bytes of a row at a time, and ds_read_b64_tr_b8 turns it on the way into the MFMA's registers.  Batches are part of the grid.
 //
-// LDS rows of A are 128 bytes of K, chunk c of row r at slot c ^ ((r >> 1) & 7); those of B are 128 columns and lie 160 bytes apart, so that
-// the 8 rows of 32 columns that 32 lanes read fall into distinct banks.  Two buffers, or two groups of waves (KG) with one each, which make
-// every other k-tile and add up at the end; the loads of a k-tile are in flight during the MFMAs of the one before.  What lies
-// beyond K is zero in B only; bytes beyond the tensors are never read.
+// LDS rows of A are 128 bytes of K, chunk c of row r at slot c ^ ((r >> 1) & 7); those of B are 128 columns, chunk c of row r at slot
+// c ^ (r & 7), or (tiles of 128 rows) at slot c of rows 160 bytes apart: the 8 rows of 32 columns that 32 lanes read fall into distinct
+// banks.  Two buffers, or two groups of waves (KG) with one each, which make every other k-tile and add up at the end; the loads of a
+// k-tile are in flight during the MFMAs of the one before.  What lies beyond K is zero in B only; bytes beyond the tensors are never read.
 //
 // Bound by a wave's issue (about one instruction in 5 cycles while it is alone on its SIMD: turning B with v_perm_b32 behind dword loads, 100 more
 // instructions a k-tile, took 0.8 us a k-tile where this takes 0.4; more k-tiles in flight change nothing) and then by the stores.  With v_perm_b32
 // and one group / now, us: 1 x 1024x1024x1024 10.0 / 5.7, 1 x 1x1024x1024 9.8 / 5.4, 16 x 32x512x64 6.4 / 4.2, 8 x 512x256x512 5.3 / 4.5,
-// 4 x 1024x128x1024 -> int16 5.77 / 5.40, 2 x 2048x1024x2048 -> int32 20.0 / 19.8.
+// 4 x 1024x128x1024 -> int16 5.77 / 5.40, 2 x 2048x1024x2048 -> int32 20.0 / 19.8.  Rows of B without a gap leave room for three workgroups of 64 rows
+// and two buffers a CU, 160 bytes apart for two: 8 x 1472x1024x512 (736 tiles of 64 rows) 16.3 / 13.2, 2 x 2304x256x1024 (576) 8.1 / 6.7.  Of 128 rows there
+// are two either way, and the slots' addresses cost 2 % (2 x 2048x1024x2048 -> int32 19.5 / 19.9).
 // MFMA operands, accumulator layout and requant tails are those of igemm_dense_i8.
 // ---------------------------------------------------------------------------
 template <int BM, int WAVES_M, int WAVES_N, int OUT, int KG>
 __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastDiv divTiles, FastDiv divTilesM) {
     constexpr int BN = 128, LA = BM / 32, BUFS = KG == 1 ? 2 : 1;
     constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N, TM = WTM / 32, TN = WTN / 32;
-    constexpr int A_BYTES = BM * 128, BUF = A_BYTES + 128 * kRtRowB;
+    constexpr int A_BYTES = BM * 128, ROWB = rtRowB(BM), TURN = ROWB == 128 ? 7 : 0, BUF = A_BYTES + 128 * ROWB;
     static_assert(WAVES_M * WAVES_N == 4, "four waves");
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
     const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // in the group
@@ -102,7 +107,7 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
             *(v4i *)(buf + row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4)) = ra[i];
         }
 #pragma unroll
-        for (int i = 0; i < 4; i++) *(v4i *)(buf + A_BYTES + (row0 + 32 * i) * kRtRowB + chunk * 16) = rb[i];
+        for (int i = 0; i < 4; i++) *(v4i *)(buf + A_BYTES + (row0 + 32 * i) * ROWB + ((chunk ^ (row0 & TURN)) << 4)) = rb[i];
     };
     v16i acc[TN][TM];
 #pragma unroll
@@ -116,9 +121,10 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
     const int fr = lane & 31, half = lane >> 5;
     int8_t *const own = smem + group * (BUFS * BUF);
     // of an operand's 16 columns and 8 rows a lane reads 8 bytes of row (lane & 15) / 2 and gets its column's
-    const int turned = A_BYTES + (16 * half + ((lane & 15) >> 1)) * kRtRowB + wn * WTN + (lane & 16) + 8 * (lane & 1);
-    auto multiply = [&](int kt, const int8_t *buf) {
-        const int steps = p.K - kt * 128 < 128 ? (p.K - kt * 128 + 31) / 32 : 4;  // none or fewer for a group whose k-tiles have ended
+    int turned[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++) turned[j] = A_BYTES + (16 * half + ((lane & 15) >> 1)) * ROWB + 8 * (lane & 1) + 16 * ((2 * (wn * TN + j) + (lane >> 4 & 1)) ^ (lane >> 1 & TURN));
+    auto multiply = [&](int steps, const int8_t *buf) {
 #pragma unroll
         for (int s = 0; s < 4; s++) {
             if (s >= steps) continue;
@@ -130,8 +136,8 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
             }
 #pragma unroll
             for (int j = 0; j < TN; j++) {
-                const int8_t *at = buf + turned + 32 * s * kRtRowB + 32 * j;
-                const v2i low = readTransposed(at), high = readTransposed(at + 8 * kRtRowB);
+                const int8_t *at = buf + turned[j] + 32 * s * ROWB;
+                const v2i low = readTransposed(at), high = readTransposed(at + 8 * ROWB);
                 bf[j] = v4i{low[0], low[1], high[0], high[1]};
             }
 #pragma unroll
@@ -148,7 +154,7 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
         load(KG + group);
         __syncthreads();
         for (int it = 1; it < KT; it++) {
-            multiply((it - 1) * KG + group, last);
+            multiply(4, last);  // whole k-tiles, all but a group's last one
             if (BUFS == 1) __syncthreads();
             // two buffers: the readers of the other one met the barrier a k-tile ago
             int8_t *next = own + (BUFS == 2 ? (it & 1) * BUF : 0);
@@ -160,7 +166,8 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
     } else {
         __syncthreads();
     }
-    multiply((KT - 1) * KG + group, last);
+    const int rest = p.K - ((KT - 1) * KG + group) * 128;
+    multiply(rest < 128 ? (rest + 31) / 32 : 4, last);  // none for a group whose k-tiles have ended
     if constexpr (KG > 1) {
         // the second group's sums through LDS, 16 bytes a lane; the first one adds them to its own and goes on
         static_assert(KG == 2, "one group besides the first");
@@ -275,7 +282,14 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
 template <int BM, int WAVES_M, int WAVES_N, int OUT, int KG>
 static hipError_t launchRt(const MatmulRtArgs &a, const LaunchCtx &ctx) {
     auto kernel = igemm_rt_i8<BM, WAVES_M, WAVES_N, OUT, KG>;
-    const size_t lds = (size_t)(KG > 1 || a.K > 128 ? 2 : 1) * (BM * 128 + 128 * kRtRowB);
+    constexpr size_t buffer = BM * 128 + 128 * rtRowB(BM);
+    if constexpr (2 * buffer > 64 * 1024) {
+        static std::once_flag once;
+        static hipError_t configured = hipSuccess;
+        std::call_once(once, [&] { configured = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(2 * buffer)); });
+        if (configured != hipSuccess) return configured;
+    }
+    const size_t lds = (KG > 1 || a.K > 128 ? 2 : 1) * buffer;
     const long long tilesM = (a.M + BM - 1) / BM, tiles = tilesM * ((a.N + 127) / 128);
     if (tiles * a.batches > 0x7fffffffLL) return hipErrorInvalidValue;
     THIP_ENQUEUE(ctx, kernelLabel("igemm_rt_i8", {BM, WAVES_M, WAVES_N, OUT, KG}), kernel, dim3((unsigned)(tiles * a.batches)), dim3(256 * KG), lds, a,
@@ -285,8 +299,9 @@ static hipError_t launchRt(const MatmulRtArgs &a, const LaunchCtx &ctx) {
 
 // Rows of a tile, us.  Up to one workgroup per CU the smallest tile is ahead (1 x 1024x1024x1024: 6.7 on 32 rows, 7.6 on 64, 9.6 on 128), and a second
 // group of waves where there is a second k-tile for it (5.7; four groups 5.7, and behind two on 2 x 300x700x300: 5.1, 5.6); beyond that 64 rows
-// (3 x 777x333x555 -> int16: 7.6, 6.6, 8.9; 8 x 512x256x512 4.7, 4.5, 5.5; 4 x 1024x128x1024 -> int16 5.6, 5.4, 6.1), and from three workgroups of these per
-// CU the operands' traffic counts (8 x 1024x256x1024 12.2, 9.9, 7.4; 2 x 2048x1024x2048 -> int32 26.8, 22.5, 19.8).
+// (3 x 777x333x555 -> int16: 7.6, 6.6, 8.9; 8 x 512x256x512 4.7, 4.5, 5.5; 4 x 1024x128x1024 -> int16 5.6, 5.4, 6.1) as long as all of them run at once: three a CU
+// hold two buffers of 24 KB each.  64 / 128 rows at 544 tiles of 64 rows 8 x 4352x256x128 6.8 / 7.0, at 664 2 x 10621x512x256 -> int32 11.6 / 13.9, at 736
+// 4 x 2941x1024x512 -> int32 15.5 / 16.8, at 816 4 x 3264x256x512 9.0 / 7.2, at 1024 8 x 1024x1024x1024 17.5 / 14.4 (of 84 drawn products of 257 .. 768 tiles one is faster on 128 rows by more than 1 %).
 template <int OUT>
 static hipError_t launchRtOut(const MatmulRtArgs &a, const LaunchCtx &ctx) {
     auto tiles = [&](int bm) { return (long long)a.batches * ((a.M + bm - 1) / bm) * ((a.N + 127) / 128); };
