@@ -12,6 +12,9 @@ I8 = dict(out_dtype=np.int8, scale=(1 << 30) + 12345, shift=41, output_zp=3)
 
 @pytest.mark.parametrize("kw", [
     dict(B=1, M=1, K=16, N=4), dict(B=3, M=5, K=7, N=3, **I8),            # fewer bytes per batch than one load
+    # fewer bytes of input2 than one load: four, fifteen as a column, as a row and of several columns, several batch elements
+    dict(B=1, M=16, K=4, N=1), dict(B=1, M=40, K=15, N=1, **I8), dict(B=1, M=16, K=1, N=15), dict(B=1, M=9, K=3, N=5, out_dtype=np.int32), dict(B=2, M=17, K=2, N=3), dict(B=5, M=6, K=3, N=1, batch1=False, **I8),
+    dict(B=7, M=5, K=7, N=2, batch2=False), dict(B=1, M=9000, K=5, N=2),
     dict(B=2, M=3, K=130, N=2, out_dtype=np.int32), dict(B=1, M=33, K=257, N=1), dict(B=2, M=40, K=129, N=3, **I8),
     dict(B=2, M=33, K=130, N=131, **I8), dict(B=2, M=31, K=100, N=129, bias=-77, out_dtype=np.int8, scale=3, shift=4, output_zp=-5, clamp=(-100, 90)),
     dict(B=3, M=70, K=200, N=90, batch1=False), dict(B=3, M=70, K=200, N=90, batch2=False, out_dtype=np.int32),

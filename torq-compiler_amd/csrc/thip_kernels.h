@@ -237,11 +237,11 @@ struct MatmulRtArgs {
     int32_t bias, scale, out_dtype;
     Requant rq;
 };
-// Whether the kernel's 32-bit offsets reach every byte of the tensors (and a row or a tile past them), and each holds one
-// load of it.
+// Whether the kernel's 32-bit offsets reach every byte of the tensors (and up to 33 rows past B, whose N is at most its bytes), and A holds
+// one load.
 inline bool matmulRtFits(int64_t aBytes, int64_t bBytes, int64_t M, int64_t N, int64_t K) {
     constexpr int64_t most = (1LL << 31) - 65536;
-    return aBytes >= 16 && bBytes >= 16 && aBytes + K + 256 <= most && bBytes + 33 * N + 256 <= most && M < most && N < most && K < most;
+    return aBytes >= 16 && bBytes >= 4 && aBytes + K + 256 <= most && bBytes + 17 * N + 256 <= most && M < most && N < most && K < most;
 }
 hipError_t launchMatmulRt(const MatmulRtArgs &a, const LaunchCtx &ctx);
 

@@ -54,9 +54,10 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
     }
     const int batch = (int)fastDiv((uint32_t)lin, divTiles), tile = lin - batch * (int)divTiles.d;
     const int tileN = (int)fastDiv((uint32_t)tile, divTilesM), n0 = tileN * BN, m0 = (tile - tileN * (int)divTilesM.d) * BM;
-    // Offsets are from the start of the tensors, below 2^31 (matmulRtFits); the last ones at which a whole chunk still lies
-    // inside:
-    const int aLast = (int)p.a_bytes - 16, bLast = (int)p.b_bytes - 16;
+    // Offsets are from the start of the tensors, which end below 2^31, and of 32 bits (matmulRtFits); the last ones at which a
+    // whole chunk still lies inside:
+    const int aLast = (int)p.a_bytes - 16;
+    const uint32_t bLast = p.b_bytes < 16 ? 0 : (uint32_t)p.b_bytes - 16;
     const int KT = (p.K + 128 * KG - 1) / (128 * KG);  // k-tiles of a group: group, group + KG, ...
 
     // chunk `chunk` of every 32nd row of both tiles is this thread's; offsets of those of k-tile 0
@@ -67,21 +68,28 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
         const int row = m0 + row0 + 32 * i;
         aOff[i] = (int)(batch * p.a_stride) + (row < p.M ? row : p.M - 1) * p.K + chunk * 16;
     }
-    const int bOff = (int)(batch * p.b_stride) + n0 + row0 * p.N + chunk * 16;
+    const uint32_t bOff = (uint32_t)(batch * p.b_stride) + (uint32_t)(n0 + chunk * 16) + (uint32_t)row0 * (uint32_t)p.N;
     v4i ra[LA], rb[4];
     // Loads only, no branch and no use of what is loaded: a load that would pass the end of its tensor starts as much
     // earlier, and store() moves its bytes to where they belong.
-    auto load = [&](int kt) {
+    auto loadA = [&](int kt) {
 #pragma unroll
         for (int i = 0; i < LA; i++) {
             const int off = aOff[i] + kt * 128;
             ra[i] = ((const UnalignedV4 *)(p.A + (uint32_t)(off < aLast ? off : aLast)))->v;
         }
+    };
+    auto loadB = [&](int kt) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int k = kt * 128 + 32 * i, off = bOff + (k < p.K ? k : p.K) * p.N;
-            rb[i] = ((const UnalignedV4 *)(p.B + (uint32_t)(off < bLast ? off : bLast)))->v;
+            const int k = kt * 128 + 32 * i;
+            const uint32_t off = bOff + (uint32_t)(k < p.K ? k : p.K) * (uint32_t)p.N;
+            rb[i] = ((const UnalignedV4 *)(p.B + (off < bLast ? off : bLast)))->v;
         }
+    };
+    auto load = [&](int kt) {
+        loadA(kt);
+        loadB(kt);
     };
     auto store = [&](int kt, int8_t *buf) {
         if (kt * 128 + 144 > p.K) {  // K's end, and where N < 16 the rows whose chunk passes the end of the tensor, lie no further away
@@ -98,7 +106,7 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int k = kt * 128 + 32 * i;
-                rb[i] = k + row0 < p.K ? moved(rb[i], bOff + k * p.N - bLast) : v4i{0, 0, 0, 0};
+                rb[i] = k + row0 < p.K ? moved(rb[i], (int)(bOff + (uint32_t)k * (uint32_t)p.N - bLast)) : v4i{0, 0, 0, 0};
             }
         }
 #pragma unroll
@@ -147,7 +155,16 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
             }
         }
     };
-    load(group);
+    loadA(group);
+    if (p.b_bytes < 16) {
+        // fewer bytes than a chunk, and so one k-tile: all of them, as a load from the tensor's start
+        uint32_t few[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int e = 0; e < 15; e++) few[e / 4] |= e < (int)p.b_bytes ? (uint32_t)(uint8_t)p.B[e] << (8 * (e % 4)) : 0u;
+        rb[0] = rb[1] = rb[2] = rb[3] = v4i{(int)few[0], (int)few[1], (int)few[2], (int)few[3]};
+    } else {
+        loadB(group);
+    }
     store(group, own);
     const int8_t *last = own;
     if (KT > 1) {
