@@ -1,5 +1,6 @@
 // The index arithmetic of ir_expand_dw_i8 on the host: every cell that a window reads is written once, by its own pixel, and nothing
-// else is written; the walk over the runs of a first layer names the runs of the same pixel.
+// else is written; the walk over the runs of a first layer names the runs of the same pixel; every result is made once, from its own window,
+// and no lane reads LDS that the launch does not ask for.
 // Arguments: N H W K C OH OW S PT PL, and for a first layer CKH CS CPT CPL IH IW IC KW behind them.  Prints the images per workgroup.
 #include <stdio.h>
 #include <stdlib.h>
@@ -68,6 +69,36 @@ int main(int argc, char **argv) {
                         if (writer[((size_t)im * s.cellRows + y) * p.cellCols + x] != (inside ? (im * p.H + iy) * p.W + ix : -1)) return fail("a cell of another pixel, or of none", n + im, iy, ix);
                     }
                 }
+            }
+        }
+    }
+    // the depthwise half: the loop of a wave over items of 16 columns
+    const size_t lds = irLaunchLds(p);
+    for (int n = 0; n < p.N; n += p.images) {
+        for (int strip = 0; strip < p.strips; strip++) {
+            const IrStrip s = irStrip(p, n, strip);
+            const int imageBytes = s.cellRows * rowBytes, items = p.OW * p.segments * s.images, walked = irWalkedRows(p, s);
+            const size_t planeBytes = (size_t)s.images * imageBytes;
+            std::vector<char> made((size_t)s.images * s.rows * p.OW, 0);
+            for (int first = 0; first < items; first += 16) {
+                for (int item = first; item < first + 16; item++) {
+                    const int ox = p.segments * p.images > 1 ? item % p.OW : item, seg = p.segments * p.images > 1 ? item / p.OW % p.segments : 0;
+                    const int image = p.images > 1 ? item / p.OW / p.segments : 0;
+                    const IrColumn c = irColumn(p, s, p.S, item < items, image, seg, ox);
+                    // rows (walked - 1) * S + 3 deep, three cells wide, in both planes
+                    const size_t end = (size_t)c.first + (size_t)((walked - 1) * p.S + 2) * rowBytes + 3 * kIrPitch + planeBytes;
+                    if (c.first < 0 || end > lds) return fail("a read behind the launch's LDS", n, strip, item);
+                    if (c.left < 0 || c.left > walked || (c.left > 0 && (image >= s.images || ox >= p.OW || c.oy + c.left > s.rows))) return fail("a result outside the strip", n, strip, item);
+                    for (int r = 0; r < c.left; r++) {
+                        if (c.first + r * p.S * rowBytes != image * imageBytes + (c.oy + r) * p.S * rowBytes + ox * p.S * kIrPitch) return fail("another window", n, strip, item);
+                        if ((c.oy + r) * p.S + 2 >= s.cellRows || ox * p.S + 2 >= p.cellCols) return fail("a window behind the cells", n, strip, item);
+                        char &m = made[((size_t)image * s.rows + c.oy + r) * p.OW + ox];
+                        if (m++) return fail("a result made twice", n, strip, item);
+                    }
+                }
+            }
+            for (size_t i = 0; i < made.size(); i++) {
+                if (!made[i]) return fail("a result that nobody makes", n, strip, (int)i);
             }
         }
     }

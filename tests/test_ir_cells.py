@@ -31,6 +31,16 @@ def check(tmp_path_factory):
 SHORT = [((300, 8, 8, 16, 256, 2, (0, 0, 0, 0)), 2), ((256, 14, 14, 96, 576, 2, (0, 0, 0, 0)), 4), ((300, 7, 7, 16, 256, 2, (1, 0, 1, 1)), 2)]
 
 
+# segments that make more rows than the last of them has, in strips that are shorter than the others, and where that took a launch past 64 KB of LDS
+DEEP = [(600, 34, 5, 16, 272, 1, (1, 1, 1, 1)), (300, 66, 3, 32, 272, 2, (1, 1, 1, 1)), (1, 64, 1, 16, 32, 1, (1, 1, 1, 1)), (1, 131, 1, 16, 32, 2, (1, 1, 1, 1)), (1, 11, 3, 16, 32, 2, (1, 1, 1, 1)),
+        (1, 5, 65, 16, 32, 1, (1, 1, 1, 1)), (1, 5, 640, 16, 32, 1, (1, 1, 1, 1)), (1, 300, 16, 16, 32, 1, (1, 1, 1, 1)), (259, 13, 14, 96, 592, 1, (1, 1, 1, 1)), (66, 2, 1, 64, 1040, 1, (1, 1, 1, 1))]
+
+
+@pytest.mark.parametrize("case", DEEP, ids=lambda c: "x".join(str(v) for v in c[:6]))
+def test_rows_below_the_strip(check, case):
+    check(*case)
+
+
 @pytest.mark.parametrize("runs", [False, True])
 @pytest.mark.parametrize("case,images", SHORT, ids=["8x8_s2", "14x14_s2", "7x7_s2_top"])
 def test_rows_no_window_reaches(check, case, images, runs):

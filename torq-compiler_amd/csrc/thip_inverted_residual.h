@@ -39,6 +39,36 @@ __host__ __device__ inline IrStrip irStrip(const IrExpandDwArgs &p, int n, int s
     return s;
 }
 
+inline size_t irLds(int images, int cellRows, int cellCols) { return (size_t)images * cellRows * cellCols * kIrPitch * 2; }
+
+// The bytes of LDS that a launch asks for: the cells, and the rows below the strip that lanes of the last segment read where the segments
+// make more rows than it has.
+inline size_t irLaunchLds(const IrExpandDwArgs &a) {
+    const int rows = irCellRows(a, a.images, a.stripRows), read = (a.segments * a.segmentRows - 1) * a.S + 3;
+    return irLds(a.images, rows, a.cellCols) + (read > rows ? (size_t)(read - rows) * a.cellCols * kIrPitch : 0);
+}
+
+// The rows of results that every lane walks down, those of the strip's highest segment.
+__host__ __device__ inline int irWalkedRows(const IrExpandDwArgs &p, const IrStrip &s) { return s.rows < p.segmentRows ? s.rows : p.segmentRows; }
+
+// A lane's column of results, of segment `seg` of image `image`.
+struct IrColumn {
+    int oy, left;  // its first row, and the rows that it stores
+    int first;     // where the first cell under its first window starts, bytes from the plane's start
+};
+
+// S: p.S, which the kernel knows when it is compiled.  Lanes without rows (an item that the strip does not have, a segment below its last
+// row) read those of the first column.
+__host__ __device__ inline IrColumn irColumn(const IrExpandDwArgs &p, const IrStrip &s, int S, bool item, int image, int seg, int ox) {
+    const int count = irWalkedRows(p, s), rowBytes = p.cellCols * kIrPitch;
+    IrColumn c;
+    c.oy = seg * p.segmentRows;
+    c.left = s.rows - c.oy < count ? s.rows - c.oy : count;
+    if (!item || c.left < 0) c.left = 0;
+    c.first = c.left > 0 ? image * s.cellRows * rowBytes + c.oy * S * rowBytes + ox * S * kIrPitch : 0;
+    return c;
+}
+
 // A wave's next tile lies 128 pixels on.  Where its pixels are (the row and column of the cell, the cell, the first run) is
 // advanced by a constant and put right where a row or an image ends, without the divisions and products that say it for any pixel:
 // vector instructions are most of the launch. With dot products behind it, those of 256 images, millions of waves': the first

@@ -59,7 +59,7 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
     n *= p.images;
     const int ch0 = chunk * kIrChunk;
     const IrStrip part = irStrip(p, n, strip);
-    const int images = part.images, oy0 = part.oy0, rows = part.rows, iyFirst = part.iyFirst, iyLo = part.iyLo, cellRows = part.cellRows, pixels = part.pixels;
+    const int images = part.images, oy0 = part.oy0, iyFirst = part.iyFirst, iyLo = part.iyLo, cellRows = part.cellRows, pixels = part.pixels;
     const int cellCols = p.cellCols;
 
     // ---- phase 1 ----
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
         }
     }
     const WideRequant w2 = wideRequant(p.rq2);
-    const int items = p.OW * p.segments * images, count = rows < p.segmentRows ? rows : p.segmentRows;
+    const int items = p.OW * p.segments * images, count = irWalkedRows(p, part);
     const uint32_t step = (uint32_t)(p.OW * p.C);
     int8_t *out = p.out + ((size_t)n * p.OH + oy0) * p.OW * p.C;
     withNarrowPackMode(w2, [&](auto tag) {
@@ -243,12 +243,10 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
                 image = (int)fastDiv((uint32_t)seg, divSegments);
                 seg -= image * p.segments;
             }
-            const int oyA = seg * p.segmentRows;
-            int left = rows - oyA < count ? rows - oyA : count;  // rows of its segment; a lane without any reads those of the first one
-            if (item >= items || left < 0) left = 0;
-            const int8_t *src = cells + (left > 0 ? image * cellImageBytes + oyA * S * cellRowBytes + ox * S * kIrPitch : 0) + (group < 3 ? group : 2) * kIrPitch;
-            if (!stored) left = 0;
-            uint32_t dst = (uint32_t)(((image * p.OH + oyA) * p.OW + ox) * p.C + ch0 + 8 * group);
+            const IrColumn column = irColumn(p, part, S, item < items, image, seg, ox);
+            const int left = stored ? column.left : 0;
+            const int8_t *src = cells + column.first + (group < 3 ? group : 2) * kIrPitch;
+            uint32_t dst = (uint32_t)(((image * p.OH + column.oy) * p.OW + ox) * p.C + ch0 + 8 * group);
             v4i ring[3][2];
             auto row = [&](v4i(&o)[2]) {
 #pragma unroll
@@ -297,12 +295,6 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
     });
 }
 
-static size_t irLds(int images, int cellRows, int cellCols) { return (size_t)images * cellRows * cellCols * kIrPitch * 2; }
-// What a launch asks for: also the rows of cells below the strip that lanes of the last segment read where the segments make more rows than it has.
-static size_t irLaunchLds(const IrExpandDwArgs &a) {
-    const int rows = irCellRows(a, a.images, a.stripRows), read = (a.segments * a.segmentRows - 1) * a.S + 3;
-    return irLds(a.images, rows, a.cellCols) + (read > rows ? (size_t)(read - rows) * a.cellCols * kIrPitch : 0);
-}
 constexpr size_t kIrMaxLds = 64 * 1024;
 constexpr int kIrMaxImages = 12;  // of a workgroup
 
