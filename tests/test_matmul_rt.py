@@ -48,7 +48,7 @@ def on_tile(device, wl, rows, K, out):
     launched = []
     got, _ = run_on_gpu(device, wl, via="device", launched=launched)
     groups = 2 if rows[0] == 32 and K > 128 else 1
-    assert launched == ["igemm_rt_i8<%d,%d,%d,%d,%d>" % (rows + (DTYPE_CODES[out], groups))], launched
+    assert launched == ["igemm_rt_i8<%d,%d,%d,%d,%d,0>" % (rows + (DTYPE_CODES[out], groups))], launched
     assert_bit_exact(got[0], oracle_eval(wl)[0], wl.name)
 
 

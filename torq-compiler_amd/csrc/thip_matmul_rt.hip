@@ -35,7 +35,9 @@ __device__ __forceinline__ v2i readTransposed(const int8_t *p) {
 // are two either way, and the slots' addresses cost 2 % (2 x 2048x1024x2048 -> int32 19.5 / 19.9).
 // MFMA operands, accumulator layout and requant tails are those of igemm_dense_i8.
 // ---------------------------------------------------------------------------
-template <int BM, int WAVES_M, int WAVES_N, int OUT, int KG>
+// FEW: B has fewer bytes than a chunk, and so one k-tile; all of them are read one by one, as a chunk from the tensor's start.  A test in the
+// other kernels cost 4 x 1024x128x1024 -> int16 0.8 %.
+template <int BM, int WAVES_M, int WAVES_N, int OUT, int KG, bool FEW>
 __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastDiv divTiles, FastDiv divTilesM) {
     constexpr int BN = 128, LA = BM / 32, BUFS = KG == 1 ? 2 : 1;
     constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N, TM = WTM / 32, TN = WTN / 32;
@@ -57,7 +59,7 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
     // Offsets are from the start of the tensors, which end below 2^31, and of 32 bits (matmulRtFits); the last ones at which a
     // whole chunk still lies inside:
     const int aLast = (int)p.a_bytes - 16;
-    const uint32_t bLast = p.b_bytes < 16 ? 0 : (uint32_t)p.b_bytes - 16;
+    const uint32_t bLast = FEW ? 0 : (uint32_t)p.b_bytes - 16;
     const int KT = (p.K + 128 * KG - 1) / (128 * KG);  // k-tiles of a group: group, group + KG, ...
 
     // chunk `chunk` of every 32nd row of both tiles is this thread's; offsets of those of k-tile 0
@@ -72,24 +74,26 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
     v4i ra[LA], rb[4];
     // Loads only, no branch and no use of what is loaded: a load that would pass the end of its tensor starts as much
     // earlier, and store() moves its bytes to where they belong.
-    auto loadA = [&](int kt) {
+    auto load = [&](int kt) {
 #pragma unroll
         for (int i = 0; i < LA; i++) {
             const int off = aOff[i] + kt * 128;
             ra[i] = ((const UnalignedV4 *)(p.A + (uint32_t)(off < aLast ? off : aLast)))->v;
         }
-    };
-    auto loadB = [&](int kt) {
+        if constexpr (FEW) {
+            uint32_t few[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 15; e++) few[e / 4] |= e < (int)p.b_bytes ? (uint32_t)(uint8_t)p.B[e] << (8 * (e % 4)) : 0u;
+            rb[0] = v4i{(int)few[0], (int)few[1], (int)few[2], (int)few[3]};
+            rb[1] = rb[2] = rb[3] = v4i{0, 0, 0, 0};  // K < 16
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int k = kt * 128 + 32 * i;
             const uint32_t off = bOff + (uint32_t)(k < p.K ? k : p.K) * (uint32_t)p.N;
             rb[i] = ((const UnalignedV4 *)(p.B + (off < bLast ? off : bLast)))->v;
         }
-    };
-    auto load = [&](int kt) {
-        loadA(kt);
-        loadB(kt);
     };
     auto store = [&](int kt, int8_t *buf) {
         if (kt * 128 + 144 > p.K) {  // K's end, and where N < 16 the rows whose chunk passes the end of the tensor, lie no further away
@@ -155,16 +159,7 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
             }
         }
     };
-    loadA(group);
-    if (p.b_bytes < 16) {
-        // fewer bytes than a chunk, and so one k-tile: all of them, as a load from the tensor's start
-        uint32_t few[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int e = 0; e < 15; e++) few[e / 4] |= e < (int)p.b_bytes ? (uint32_t)(uint8_t)p.B[e] << (8 * (e % 4)) : 0u;
-        rb[0] = rb[1] = rb[2] = rb[3] = v4i{(int)few[0], (int)few[1], (int)few[2], (int)few[3]};
-    } else {
-        loadB(group);
-    }
+    load(group);
     store(group, own);
     const int8_t *last = own;
     if (KT > 1) {
@@ -296,9 +291,9 @@ __global__ __launch_bounds__(256 * KG, 2) void igemm_rt_i8(MatmulRtArgs p, FastD
     }
 }
 
-template <int BM, int WAVES_M, int WAVES_N, int OUT, int KG>
+template <int BM, int WAVES_M, int WAVES_N, int OUT, int KG, bool FEW = false>
 static hipError_t launchRt(const MatmulRtArgs &a, const LaunchCtx &ctx) {
-    auto kernel = igemm_rt_i8<BM, WAVES_M, WAVES_N, OUT, KG>;
+    auto kernel = igemm_rt_i8<BM, WAVES_M, WAVES_N, OUT, KG, FEW>;
     constexpr size_t buffer = BM * 128 + 128 * rtRowB(BM);
     if constexpr (2 * buffer > 64 * 1024) {
         static std::once_flag once;
@@ -309,7 +304,7 @@ static hipError_t launchRt(const MatmulRtArgs &a, const LaunchCtx &ctx) {
     const size_t lds = (KG > 1 || a.K > 128 ? 2 : 1) * buffer;
     const long long tilesM = (a.M + BM - 1) / BM, tiles = tilesM * ((a.N + 127) / 128);
     if (tiles * a.batches > 0x7fffffffLL) return hipErrorInvalidValue;
-    THIP_ENQUEUE(ctx, kernelLabel("igemm_rt_i8", {BM, WAVES_M, WAVES_N, OUT, KG}), kernel, dim3((unsigned)(tiles * a.batches)), dim3(256 * KG), lds, a,
+    THIP_ENQUEUE(ctx, kernelLabel("igemm_rt_i8", {BM, WAVES_M, WAVES_N, OUT, KG, (int)FEW}), kernel, dim3((unsigned)(tiles * a.batches)), dim3(256 * KG), lds, a,
                  makeFastDiv((uint32_t)tiles), makeFastDiv((uint32_t)tilesM));
     return hipGetLastError();
 }
@@ -322,6 +317,7 @@ static hipError_t launchRt(const MatmulRtArgs &a, const LaunchCtx &ctx) {
 template <int OUT>
 static hipError_t launchRtOut(const MatmulRtArgs &a, const LaunchCtx &ctx) {
     auto tiles = [&](int bm) { return (long long)a.batches * ((a.M + bm - 1) / bm) * ((a.N + 127) / 128); };
+    if (a.b_bytes < 16) return launchRt<32, 1, 4, OUT, 1, true>(a, ctx);
     if (a.M <= 32 || tiles(32) <= 256) return a.K <= 128 ? launchRt<32, 1, 4, OUT, 1>(a, ctx) : launchRt<32, 1, 4, OUT, 2>(a, ctx);
     if (tiles(64) <= 768) return launchRt<64, 2, 2, OUT, 1>(a, ctx);
     return launchRt<128, 2, 2, OUT, 1>(a, ctx);
