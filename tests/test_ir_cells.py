@@ -48,6 +48,15 @@ def test_rows_no_window_reaches(check, case, images, runs):
     assert shared >= images, "the case is about images that share a workgroup"
 
 
+@pytest.mark.parametrize("case,images", [
+    ((32, 14, 14, 64, 384, 1, (1, 1, 1, 1)), 2), ((256, 14, 14, 64, 384, 1, (1, 1, 1, 1)), 4), ((256, 7, 7, 160, 960, 1, (1, 1, 1, 1)), 11), ((54, 16, 16, 32, 192, 2, (0, 1, 0, 1)), 2),
+    ((12, 10, 10, 96, 576, 1, (1, 1, 1, 1)), 1), ((1, 14, 14, 96, 576, 1, (1, 1, 1, 1)), 1),
+], ids=["14x14_b32", "14x14_b256", "7x7_b256", "16x16_b54", "10x10_b12", "14x14_b1"])
+def test_images_by_the_estimate(check, case, images):
+    """As many images a workgroup as are measured ahead: two where strips of one image had been cut in two."""
+    assert check(*case) == images
+
+
 def test_drawn_geometries(check):
     rng = np.random.default_rng(11)
     shared = 0

@@ -3,6 +3,8 @@
 #include "thip_inverted_residual.h"
 #include "thip_kernels_common.h"
 
+#include <math.h>
+
 namespace thip {
 
 // The requant tails that need 32-bit arithmetic only (withPackMode without its 64-bit one; the planner keeps such records
@@ -36,9 +38,11 @@ static inline int irCellColumns(int OW, int S) { return (OW - 1) * S + 3; }
 // byte; with byte transposes and v_dot4_i32_i8 in phase 2 it was 9 per depthwise byte); the rest goes where a workgroup's phases and the launch's last round of workgroups wait.
 // us, in a trace of the network, with v_dot4_i32_i8 / now:
 //   batch 256  14x14x64 -> 384 17.4 / 15.1, 14x14x96 -> 576 24.6 / 23.8, its stride 2 17.3 / 16.2, 7x7x160 -> 960 17.0 / 15.0
-//   batch 32   7x7x160 -> 960 8.3 / 5.6, 14x14x96 -> 576 8.4 / 8.0, 14x14x64 -> 384 5.8 / 6.3
-// the whole network at 256 / 32 (host buffers) / 1 images 716 / 394 / 132.5 -> 695 / 386 / 131.1. Tried: phase 2's constants under way from the start on (registers spill from K = 96
-// on: 23.8 -> 25.5), the requants' constants from the host (no change, and spills), more tiles prefetched, or strips of 26, 32 or 53 KB (no change).
+// and one behind another, in time from one to the next
+//   batch 32   7x7x160 -> 960 8.0 / 5.3, 14x14x96 -> 576 7.9 / 7.4, its stride 2 6.4 / 5.7, 14x14x64 -> 384 6.0 / 6.0, 28x28x32 -> 192 7.9 / 6.9
+//   batch 1    14x14x64 -> 384 3.9 / 4.0
+// the whole network at 256 images 716 -> 695 (at 32 in host memory and at one the runs of one build differ by as much as it gave). Tried: phase 2's constants under way from the start on (registers spill from K = 96
+// on: 23.8 -> 25.5), the requants' constants from the host (no change, and spills), more tiles prefetched (no change).
 // ---------------------------------------------------------------------------
 template <int KS, int S, bool RUNS>
 __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpandDwArgs p, FastDiv divW, FastDiv divH, FastDiv divCols, FastDiv divSegments) {
@@ -326,16 +330,42 @@ static hipError_t launchIrS(const IrExpandDwArgs &a, const LaunchCtx &ctx) {
     }
 }
 
-// The time of a launch whose workgroups make `images` whole images each, us.  A CU runs as many workgroups at a time as its registers and LDS hold, and each such
-// round costs a start and what the tiles of pixels and the rows of 16 results of its workgroups take together.  Fitted to 256 images of 14x14x64 -> 384 by 1, 2, 4, 5, 6, 8, 9 and 11
-// (21.6, 17.0, 15.2, 19.1, 20.2, 18.0, 18.8, 21.8 us) and of 7x7x160 -> 960 (40.8, 26.4, 19.8, 19.3, 17.7, 15.5, 15.8, 15.1): a last round that is nearly empty costs
-// as much as what it saves.
-static double irTime(const IrExpandDwArgs &a, int images, size_t lds) {
-    const int KS = a.CKH > 0 ? (a.CKH + 1) / 2 : (a.K + 31) / 32, byLds = (int)(160 * 1024 / (lds + 1024)), perCu = byLds < (KS <= 3 ? 4 : 3) ? byLds : KS <= 3 ? 4 : 3;
-    const long long blocks = (long long)((a.N + images - 1) / images) * ((a.C + kIrChunk - 1) / kIrChunk), room = 256LL * perCu, rest = (blocks % room + 255) / 256;
-    const int tiles = (images * a.H * a.W + 31) / 32, columns = a.OW * images, segments = columns >= 64 ? 1 : 64 / columns, rows = (columns * segments + 15) / 16 * ((a.OH + segments - 1) / segments);
-    const double one = tiles * (0.05 + 0.006 * KS) + rows * 0.033, start = 2.5;
-    return (double)(blocks / room) * (start + perCu * one) + (rest > 0 ? start + (double)rest * one : 0.0);
+// What follows from `images` and `stripRows`: strips, and segments of a strip's rows so that a wave's 16 columns and its rows fill four waves.
+static void irLayout(IrExpandDwArgs *args, int images, int stripRows) {
+    IrExpandDwArgs &a = *args;
+    a.images = images;
+    a.strips = (a.OH + stripRows - 1) / stripRows;
+    a.stripRows = stripRows;
+    const int columns = a.OW * images;
+    a.segments = columns >= 64 ? 1 : 64 / columns;
+    if (a.segments > stripRows) a.segments = stripRows;
+    a.segmentRows = (stripRows + a.segments - 1) / a.segments;
+    a.segments = (stripRows + a.segmentRows - 1) / a.segmentRows;
+}
+
+// The time of a launch, us: of a workgroup alone on its CU a start, the cells it clears, the tiles of pixels and the rows of 16 results of a wave; of
+// those that share a CU, as many as its registers and LDS hold, each one more; and the rounds of these.  Fitted to 9316 launches of 992 layers, by
+// every height of strips and up to 12 images a workgroup: 1 .. 256 images of 4 .. 112 pixels a side, 16 .. 192 channels in and 1 .. 6 times as many wide
+// ones, both strides, half of them of mobile networks; `runs` to 140 first layers.  Nine in ten of the launches near a layer's best are within 11 %.  The choice by it
+// takes 0.6 % longer than the best, strips of 40 KB in at least 512 workgroups (and images by their rounds) 6 %; in turn with that, 472 other layers took
+// 0.946 of the time, three of them more than 3 % longer, 7 % at most.  us, by that / now: 7x7x160 -> 960, 16 images 8.0 / 4.7,
+// 10x10x80 -> 480, 14 images 6.0 / 4.4, 14x14x64 -> 384, 126 images 12.0 / 9.3, 16 images 5.7 / 4.9, 32 images 6.04 / 6.02 (two strips of an image before, two images now).
+static double irTime(const IrExpandDwArgs &a) {
+    struct Cost {
+        double launch, start, fill, tile, tileK, row, more, moreFill, moreTile, moreTileK, moreRow;
+    };
+    constexpr Cost dense{2.72, 1.04, 0.126, 0.092, 0.039, 0.165, 0.59, 0.047, 0.0, 0.074, 0.075}, runs{3.03, 0.90, 0.221, 0.406, 0.241, 0.153, 0.75, 0.0, 0.0, 0.116, 0.073};
+    const Cost &c = a.CKH > 0 ? runs : dense;
+    const int KS = a.CKH > 0 ? (a.CKH + 1) / 2 : (a.K + 31) / 32, cellRows = irCellRows(a, a.images, a.stripRows);
+    int rows = a.strips == 1 ? cellRows - a.PT : cellRows;
+    if (rows > a.H) rows = a.H;
+    const size_t lds = irLaunchLds(a);
+    const int byLds = (int)(160 * 1024 / (lds + 1024)), perCu = byLds < (KS <= 3 ? 4 : 3) ? byLds : KS <= 3 ? 4 : 3;
+    const long long blocks = (long long)((a.N + a.images - 1) / a.images) * a.strips * ((a.C + kIrChunk - 1) / kIrChunk), room = 256LL * perCu, rest = (blocks % room + 255) / 256;
+    const double tiles = (double)(((long long)a.images * rows * a.W + 31) / 32), items = (a.OW * a.segments * a.images + 15) / 16, kb4 = (double)lds / 4096;
+    const double alone = c.start + kb4 * c.fill + ceil(tiles / 4) * (c.tile + c.tileK * (KS - 1)) + ceil(items / 4) * a.segmentRows * c.row;
+    const double more = c.more + kb4 * c.moreFill + tiles / 4 * (c.moreTile + c.moreTileK * (KS - 1)) + items / 4 * a.segmentRows * c.moreRow;
+    return c.launch + (double)(blocks / room) * (alone + (perCu - 1) * more) + (rest > 0 ? alone + (double)(rest - 1) * more : 0.0);
 }
 
 bool planIrExpandDw(IrExpandDwArgs *args) {
@@ -358,43 +388,37 @@ bool planIrExpandDw(IrExpandDwArgs *args) {
     if ((a.OH - 1) * a.S - a.PT >= a.H || (a.OW - 1) * a.S - a.PL >= a.W) return false;
     a.cellCols = irCellColumns(a.OW, a.S);
     if ((long long)a.C > kIrMaxChannels) return false;
-    // Four workgroups per CU (160 KB of LDS, 16 waves) overlap one another's phases: strips as high as 40 KB of cells hold
-    // (56x56x32 -> 144, 256 images: 79 us at 20 KB, whose strips make more rows twice, 69 at 40, 76 at 64), lower where that
-    // leaves fewer than two workgroups per CU (14x14x96 -> 576, 32 images: 8.0 us with at least 512, 9.1 with 1024), down
-    // to four rows, and to one where not every CU has a workgroup (a mobile network of one image: 133.4 us with four rows, 131.1 so).
-    // Images that leave room share a workgroup, as many as irTime says.
-    constexpr size_t ldsAim = 40 * 1024;
-    constexpr long long wgAim = 512;
+    // Strips of rows, or whole images, as the estimate has them, heights a fifth apart: neighbouring ones hardly differ.  Both ways end where a
+    // launch takes half as long again as the best one: it only gets longer behind that.
+    constexpr long long enough = 20000;  // workgroups: strips that make more of them gain nothing
     const long long perStrip = (long long)a.N * ((a.C + kIrChunk - 1) / kIrChunk);
-    int strips = 1;
-    auto rowsOf = [&](int s) { return (a.OH + s - 1) / s; };
-    auto lds = [&](int images, int s) { return irLds(images, irCellRows(a, images, rowsOf(s)), a.cellCols); };
-    while (rowsOf(strips) > 1 && (lds(1, strips) > ldsAim || (perStrip * strips < wgAim && rowsOf(strips) > 4) || perStrip * strips < 256)) strips++;
-    a.stripRows = rowsOf(strips);
-    a.strips = (a.OH + a.stripRows - 1) / a.stripRows;
-    // the launch's time by the rounds of workgroups that it takes: irTime
-    a.images = 1;
-    if (a.strips == 1) {
-        double best = irTime(a, 1, lds(1, 1));
-        // room for the rows below the last strip (irLaunchLds): at most 64 / columns of them a stride, 6 KB
-        for (int images = 2; images <= kIrMaxImages && images <= a.N && lds(images, 1) <= kIrMaxLds - 6 * 1024; images++) {
-            const double time = irTime(a, images, lds(images, 1));
-            if (time < best) {
-                best = time;
-                a.images = images;
-            }
+    double best = -1.0;
+    int images = 0, stripRows = 0;
+    auto consider = [&](int n, int rows) {
+        irLayout(&a, n, rows);
+        if (irLaunchLds(a) > kIrMaxLds) return true;
+        const double time = irTime(a);
+        if (best < 0.0 || time < best) {
+            best = time;
+            images = n;
+            stripRows = rows;
         }
+        return time < 1.5 * best;
+    };
+    const int fitting = ((int)(kIrMaxLds / irLds(1, 1, a.cellCols)) - 3) / a.S + 1;
+    for (int rows = a.OH < fitting ? a.OH : fitting; rows >= 1;) {
+        const int strips = (a.OH + rows - 1) / rows, even = (a.OH + strips - 1) / strips;
+        if (!consider(1, even) || (best >= 0.0 && perStrip * strips > enough)) break;
+        rows = even > 6 ? even * 4 / 5 : even - 1;
     }
+    for (int n = 2; n <= kIrMaxImages && n <= a.N && irLds(n, irCellRows(a, n, a.OH), a.cellCols) <= kIrMaxLds && consider(n, a.OH); n++) {}
+    if (best < 0.0) return false;
+    irLayout(&a, images, stripRows);
     // 128 pixels on, in images, rows and columns
     a.stepImages = a.images > 1 ? 128 / (a.H * a.W) : 0;
     a.stepRows = (128 - a.stepImages * a.H * a.W) / a.W;
     a.stepColumns = (128 - a.stepImages * a.H * a.W) % a.W;
-    const int columns = a.OW * a.images;
-    a.segments = columns >= 64 ? 1 : 64 / columns;
-    if (a.segments > a.stripRows) a.segments = a.stripRows;
-    a.segmentRows = (a.stripRows + a.segments - 1) / a.segments;
-    a.segments = (a.stripRows + a.segmentRows - 1) / a.segmentRows;
-    return irLaunchLds(a) <= kIrMaxLds;
+    return true;
 }
 
 hipError_t launchIrExpandDw(const IrExpandDwArgs &in, const LaunchCtx &ctx) {
