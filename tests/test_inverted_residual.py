@@ -101,7 +101,7 @@ def test_rows_no_window_reaches(device, kw):
 @pytest.mark.parametrize("kw", [
     dict(N=1, H=9, W=10, C=32, E=48, stride=1), dict(N=1, H=11, W=3, C=16, E=32, stride=2), dict(N=1, H=5, W=65, C=16, E=32, stride=1),   # segments with fewer rows, or none
     dict(N=257, H=7, W=7, C=160, E=960, stride=1), dict(N=259, H=13, W=14, C=96, E=592, stride=1), dict(N=66, H=2, W=1, C=64, E=1040, stride=1),  # a last workgroup of fewer images
-    dict(N=1, H=5, W=640, C=16, E=32, stride=1), dict(N=1, H=5, W=640, C=16, E=32, stride=2), dict(N=600, H=34, W=5, C=16, E=272, stride=1), dict(N=300, H=66, W=3, C=32, E=272, stride=2),   # the widest rows, and the most LDS
+    dict(N=1, H=5, W=510, C=16, E=32, stride=1), dict(N=1, H=5, W=407, C=16, E=32, stride=2), dict(N=2, H=100, W=640, C=16, E=32, stride=2), dict(N=600, H=34, W=5, C=16, E=272, stride=1), dict(N=300, H=66, W=3, C=32, E=272, stride=2),   # the widest rows of two windows and of one, and the most LDS
     dict(N=2, H=12, W=12, C=32, E=48, stride=1, top=100), dict(N=2, H=12, W=12, C=32, E=48, stride=2, shift=41), dict(N=2, H=9, W=9, C=3, E=48, stride=1, first=(3, 1, (1, 1, 1, 1)), top=90),
 ], ids=lambda kw: "x".join(str(v) for v in kw.values()))
 def test_expand_depthwise_lanes(device, kw):
@@ -109,3 +109,17 @@ def test_expand_depthwise_lanes(device, kw):
     wl = block(**kw)
     print("[gpu-case]", wl.name, flush=True)
     assert_bit_exact(fused(device, wl)[0], oracle_network(wl), wl.name)
+
+
+@pytest.mark.parametrize("kw", [
+    dict(N=1, H=5, W=511, C=16, E=32, stride=1), dict(N=1, H=5, W=640, C=16, E=32, stride=1), dict(N=2, H=40, W=600, C=16, E=48, stride=1), dict(N=1, H=5, W=640, C=16, E=32, stride=2),
+    dict(N=1, H=5, W=410, C=16, E=32, stride=2),
+], ids=lambda kw: "x".join(str(v) for v in kw.values()))
+def test_rows_too_wide_for_two_windows(device, kw):
+    """Strips of one row widen most pixels again: two launches where these are ahead."""
+    wl = block(**kw)
+    print("[gpu-case]", wl.name, flush=True)
+    launched = []
+    got, _ = run_on_gpu(device, wl, via="device", launched=launched)
+    assert "ir_expand_dw_i8" not in families(launched) and len(launched) == 2, launched
+    assert_bit_exact(got[0], oracle_network(wl), wl.name)

@@ -161,6 +161,23 @@ def test_blocks_are_one_launch_where_that_is_estimated_ahead(plan, kw, taken):
     assert (lines == ["ir_block_i8 0 3"]) if taken else [s.split()[:3] for s in lines] == [["ir_expand_dw_i8", "0", "2"], ["record", "2", "1"]], lines
 
 
+@pytest.mark.parametrize("kw,taken", [
+    (dict(N=1, H=5, W=510, C=16, E=32, stride=1), True), (dict(N=1, H=5, W=511, C=16, E=32, stride=1), False), (dict(N=16, H=100, W=640, C=16, E=96, stride=1), False),
+    (dict(N=1, H=5, W=407, C=16, E=32, stride=2), True), (dict(N=1, H=5, W=410, C=16, E=32, stride=2), False), (dict(N=1, H=98, W=640, C=16, E=32, stride=2), True),
+    (dict(N=1, H=97, W=640, C=16, E=32, stride=2), False),
+], ids=lambda v: "x".join(str(x) for x in v.values()) if isinstance(v, dict) else str(v))
+def test_pairs_with_rows_too_wide_for_two_windows(plan, kw, taken):
+    from test_inverted_residual import block
+    assert [s.split()[0] for s in plan(block(**kw))] == (["ir_expand_dw_i8"] if taken else ["record"] * 2)
+
+
+def test_wide_first_layers_are_one_launch_with_the_narrow_convolution(plan, monkeypatch):
+    """Blocks of columns: the pair's strips of one row are no measure for them."""
+    from test_ir_block import block
+    monkeypatch.setenv("THIP_IR_BLOCK", "1")
+    assert plan(block(N=1, H=30, W=640, C=3, E=32, O=16, stride=1, first=(3, 1, (1, 1, 1, 1)))) == ["ir_block_i8 0 3"]
+
+
 def with_output_zp(wl, record, zp):
     """The serialised program, a record's zero point set by hand."""
     class Changed:

@@ -307,6 +307,15 @@ bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL) {
     return PT >= 0 && PT <= 2 && PL >= 0 && PL <= 2 && (runRows > 0 ? runRows <= 4 : K > 0 && K % 16 == 0 && K <= 192) && (stride == 1 || stride == 2) && irLds(1, 3, irCellColumns(OW, stride)) <= kIrMaxLds;
 }
 
+bool irExpandDwBetter(int64_t wide, int OW, int stride) {
+    // Rows of which LDS holds no two windows leave strips of one row, whose pixels are widened three times (stride 2: half of them twice).  At
+    // stride 1 two launches are ahead of that: over 97 drawn layers of 511 .. 680 columns they cost 1.5 % of the better one's time, one launch
+    // 30 % (1x5x640x16 -> 32 10.7 / 7.1 us, 8x64x600x64 -> 128 46.1 / 38.0).  At stride 2 only where there is little work: over 124 layers of
+    // 205 .. 340 columns this line costs 2.8 %, always one launch 10 %, always two 16 % (1x16x320x16 -> 32 9.0 / 7.1, 8x64x340x64 -> 128 23.0 / 30.3).
+    if (irLds(1, 3 + stride, irCellColumns(OW, stride)) <= kIrMaxLds) return true;
+    return stride == 2 && wide >= 2000000;
+}
+
 template <int KS, int S, bool RUNS = false>
 static hipError_t launchIr(const IrExpandDwArgs &a, const LaunchCtx &ctx) {
     const long long blocks = (long long)((a.N + a.images - 1) / a.images) * a.strips * ((a.C + kIrChunk - 1) / kIrChunk);

@@ -181,6 +181,8 @@ struct IrExpandDwArgs {
 // A strip's results are addressed with 32 bits: its cells fit LDS, so they are fewer than 2^11 pixels.
 constexpr int kIrMaxChannels = 1 << 20;
 bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL);
+// Whether one launch is ahead of two, for a widened image of `wide` values.
+bool irExpandDwBetter(int64_t wide, int OW, int stride);
 // Checks the arguments and sets what is the launch's own to choose; false where the kernel does not take them.
 bool planIrExpandDw(IrExpandDwArgs *a);
 hipError_t launchIrExpandDw(const IrExpandDwArgs &a, const LaunchCtx &ctx);

@@ -135,28 +135,6 @@ static uint8_t *plannedAt(const DescriptorView &v, const DescRef &r) {
 // Whether the requant of a record has a tail of 32-bit arithmetic (see WideRequant).
 static bool narrowRequant(const DescOp &op) { return op.shift == 32 || (int64_t)op.shift + op.pre_shift >= 33; }
 
-// A pointwise convolution, or one over few channels, whose only reader is the 3 x 3 depthwise convolution right behind it.
-static bool matchExpandDw(const DescriptorView &v, const std::vector<uint32_t> &uses, uint32_t first, Step *s) {
-    if (first + 1 >= v.header.op_count) return false;
-    const DescOp &e = v.ops[first], &d = v.ops[first + 1];
-    const bool runs = e.loader == kLoaderRuns;
-    if (e.kind != kKindIgemm || (!runs && (e.loader != kLoaderDense || e.KH != 1 || e.KW != 1)) || e.in1.space != kSpaceNone || e.out_dtype != 1) return false;
-    if (runs && (e.SH != e.SW || e.OH != d.H || e.OW != d.W || e.N != d.N || (int64_t)e.N * e.H * e.W * e.C < 16 || (int64_t)e.H * e.W * e.C > (1LL << 27))) return false;
-    if (d.kind != kKindDepthwise || d.variant != kDepthwiseDot4Rows || d.KH != 3 || d.KW != 3 || d.SH != d.SW) return false;
-    if (e.out.space != kSpaceTemp || !sameRef(e.out, d.in0) || uses[e.out.index] != 2) return false;
-    if (d.C != e.Nn || d.C > kIrMaxChannels || (int64_t)d.N * d.H * d.W != e.M || !narrowRequant(e) || !narrowRequant(d)) return false;
-    if (!irExpandDwFits(e.K, runs ? e.KH : 0, d.OW, d.SW, d.PT, d.PL) || e.Kp < (runs ? (e.KH + 1) / 2 : (e.K + 31) / 32) * 32 || e.Np < (e.Nn + 31) / 32 * 32) return false;
-    if ((int64_t)d.H * d.W * e.K >= (1LL << 31) || (d.OH - 1) * d.SH - d.PT >= d.H || (d.OW - 1) * d.SW - d.PL >= d.W) return false;
-    for (const DescRef *r : {&e.in0, &e.weights, &e.bias, &e.scale, &d.weights, &d.bias, &d.scale, &d.out}) {
-        if (r->offset % 16 != 0 && !(runs && r == &e.in0)) return false;
-    }
-    if (sameBuffer(d.out, e.in0)) return false;
-    s->kind = kStepExpandDw;
-    s->first = first;
-    s->count = 2;
-    return true;
-}
-
 // Behind the two records that `s` stands for, the pointwise convolution that alone reads their result, its add folded into it or none.
 static void matchBlock(const DescriptorView &v, const Tuning &tuning, const std::vector<uint32_t> &uses, Step *s) {
     const uint32_t last = s->first + 2;
@@ -174,6 +152,32 @@ static void matchBlock(const DescriptorView &v, const Tuning &tuning, const std:
     }
     const IrBlockArgs a = irBlockArgs(v, *s, [&](const DescRef &r) { return plannedAt(v, r); });
     if (tuning.irBlock >= 0 ? tuning.irBlock != 0 && irBlockFits(a) : irBlockBetter(a)) s->count = 3;
+}
+
+// A pointwise convolution, or one over few channels, whose only reader is the 3 x 3 depthwise convolution right behind it, and with them the
+// pointwise convolution behind that where the three are ahead as one launch.
+static bool matchExpandDw(const DescriptorView &v, const Tuning &tuning, const std::vector<uint32_t> &uses, uint32_t first, Step *s) {
+    if (first + 1 >= v.header.op_count) return false;
+    const DescOp &e = v.ops[first], &d = v.ops[first + 1];
+    const bool runs = e.loader == kLoaderRuns;
+    if (e.kind != kKindIgemm || (!runs && (e.loader != kLoaderDense || e.KH != 1 || e.KW != 1)) || e.in1.space != kSpaceNone || e.out_dtype != 1) return false;
+    if (runs && (e.SH != e.SW || e.OH != d.H || e.OW != d.W || e.N != d.N || (int64_t)e.N * e.H * e.W * e.C < 16 || (int64_t)e.H * e.W * e.C > (1LL << 27))) return false;
+    if (d.kind != kKindDepthwise || d.variant != kDepthwiseDot4Rows || d.KH != 3 || d.KW != 3 || d.SH != d.SW) return false;
+    if (e.out.space != kSpaceTemp || !sameRef(e.out, d.in0) || uses[e.out.index] != 2) return false;
+    if (d.C != e.Nn || d.C > kIrMaxChannels || (int64_t)d.N * d.H * d.W != e.M || !narrowRequant(e) || !narrowRequant(d)) return false;
+    if (!irExpandDwFits(e.K, runs ? e.KH : 0, d.OW, d.SW, d.PT, d.PL) || e.Kp < (runs ? (e.KH + 1) / 2 : (e.K + 31) / 32) * 32 || e.Np < (e.Nn + 31) / 32 * 32) return false;
+    if ((int64_t)d.H * d.W * e.K >= (1LL << 31) || (d.OH - 1) * d.SH - d.PT >= d.H || (d.OW - 1) * d.SW - d.PL >= d.W) return false;
+    for (const DescRef *r : {&e.in0, &e.weights, &e.bias, &e.scale, &d.weights, &d.bias, &d.scale, &d.out}) {
+        if (r->offset % 16 != 0 && !(runs && r == &e.in0)) return false;
+    }
+    if (sameBuffer(d.out, e.in0)) return false;
+    s->kind = kStepExpandDw;
+    s->first = first;
+    s->count = 2;
+    matchBlock(v, tuning, uses, s);
+    if (s->count == 3 || irExpandDwBetter((int64_t)d.N * d.H * d.W * d.C, d.OW, d.SW)) return true;
+    *s = Step{};
+    return false;
 }
 
 // Whether the copy of the rows and a kernel of aligned operands behind it are ahead of a record's own gather kernel, by the time that
@@ -589,12 +593,11 @@ std::vector<Step> planSteps(const DescriptorView &v, const Tuning &tuning) {
     std::vector<Step> steps;
     for (uint32_t i = 0; i < v.header.op_count;) {
         Step s{};
-        if (plain || (!matchDecChain(v, tuning, i, &s) && !matchExpandDw(v, uses, i, &s) && !matchMatmulRt(v, uses, i, &s) && !matchPadded(v, tuning, i, &s))) {
+        if (plain || (!matchDecChain(v, tuning, i, &s) && !matchExpandDw(v, tuning, uses, i, &s) && !matchMatmulRt(v, uses, i, &s) && !matchPadded(v, tuning, i, &s))) {
             s.kind = kStepRecord;
             s.first = i;
             s.count = 1;
         }
-        if (s.kind == kStepExpandDw) matchBlock(v, tuning, uses, &s);
         const DescOp *op = s.kind == kStepRecord ? &v.ops[i] : s.kind == kStepPadded ? &s.op : nullptr;
         if (s.kind == kStepExpandDw && s.count == 3) op = &v.ops[i + 2];
         s.route = plain || !op || op->kind != kKindIgemm ? kIgemmOwnTile : s.kind == kStepPadded && s.asIs ? kIgemmDirect : igemmRoute(v, tuning, *op);
