@@ -154,6 +154,9 @@ def test_ragged_rows_by_each_way(plan, make, lines):
     # many narrow channels, and few
     (dict(N=170, H=66, W=54, C=16, E=48, O=96, stride=1), False), (dict(N=101, H=64, W=55, C=16, E=96, O=64, stride=1), False), (dict(N=192, H=51, W=56, C=64, E=128, O=64, stride=1), False),
     (dict(N=101, H=64, W=55, C=16, E=96, O=16, stride=1), True),
+    # two / one launch, us: 9.6 / 7.5, 8.0 / 6.4, 13.2 / 10.8; 33.7 / 37.7, 12.9 / 14.1
+    (dict(N=132, H=8, W=20, C=16, E=48, O=80, stride=1), True), (dict(N=7, H=74, W=34, C=48, E=48, O=32, stride=1), True), (dict(N=104, H=33, W=10, C=64, E=160, O=48, stride=1), True),
+    (dict(N=150, H=45, W=10, C=96, E=480, O=16, stride=1), False), (dict(N=33, H=49, W=49, C=32, E=192, O=32, stride=2), False),
 ], ids=lambda v: "x".join(str(x) for x in v.values()) if isinstance(v, dict) else str(v))
 def test_blocks_are_one_launch_where_that_is_estimated_ahead(plan, kw, taken):
     from test_ir_block import block

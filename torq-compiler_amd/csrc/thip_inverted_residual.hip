@@ -430,6 +430,11 @@ bool planIrExpandDw(IrExpandDwArgs *args) {
     return true;
 }
 
+double irExpandDwTime(const IrExpandDwArgs &in) {
+    IrExpandDwArgs a = in;
+    return planIrExpandDw(&a) ? irTime(a) : HUGE_VAL;
+}
+
 hipError_t launchIrExpandDw(const IrExpandDwArgs &in, const LaunchCtx &ctx) {
     IrExpandDwArgs a = in;
     if (!planIrExpandDw(&a)) return hipErrorInvalidValue;

@@ -43,12 +43,12 @@ constexpr int irBlockTiles(int S) { return S == 1 ? 6 : 10; }
 //
 // Why: apart, the depthwise result (2.3 MB per image of a 224 x 224 mobile network) is written and read back by a launch of its own.  Bound by
 // vector instructions and MFMAs that two waves a SIMD overlap in part: an instruction takes the SIMD 4.3 to 4.6 cycles (a wave alone issues one in 5 to 5.7), which is 58 % of the cycles
-// (75 % of a first layer's, at four waves), and MFMAs 15 to 20 %.  Measured, us, the two launches / this one:
-//   batch 256  224x224x3 -> 112x112x32 -> 16 108 / 81, 112x112x16 -> 96 stride 2 -> 32 104 / 97, 56x56x32 -> 144 -> 32 and the add 98 / 86,
-//              its stride 2 48 / 42, 28x28x32 -> 192 -> 32 42 / 29, stride 2 -> 64 24 / 21
-//   batch 32   26.2 / 16.3, 22.1 / 17.6, 21.5 / 18.7, 13.2 / 12.3, 11.9 / 11.5; 9.9 / 13.3 (left to the two launches)
-//   batch 1    12.6 / 4.9; 7.7 / 7.8, 7.8 / 9.3, 7.2 / 10.1 (left)
-// and left at any batch: 14x14x64 -> 384 -> 64 23.7 / 33, 14x14x96 -> 576 -> 96 38.5 / 53, whose chunks are too small for what each costs.  Tried on it: four waves a SIMD
+// (75 % of a first layer's, at four waves), and MFMAs 15 to 20 %.  Measured one behind another, us, the two launches / this one:
+//   batch 256  224x224x3 -> 112x112x32 -> 16 98 / 71, 112x112x16 -> 96 stride 2 -> 32 98 / 95, 56x56x32 -> 144 -> 32 and the add 88 / 83,
+//              its stride 2 45 / 39, 28x28x32 -> 192 -> 32 35 / 25
+//   batch 32   24.6 / 13.4, 21.5 / 17.5, 21.6 / 17.5, 12.8 / 12.5, 11.2 / 11.0
+//   batch 1    10.0 / 5.4; 8.1 / 8.1, 8.4 / 9.0, 7.8 / 9.9, 7.9 / 9.8 (left to the two launches)
+// and left at any batch: 14x14x64 -> 384 -> 64 21.1 / 33.3 (223 images), 14x14x96 -> 576 -> 96 38.5 / 53, whose chunks are too small for what each costs.  Tried on it: four waves a SIMD
 // (their registers hold half the rows, the chunks' constants are fetched twice as often: 85 -> 103), waves that only widen beside waves that
 // only convolve (94), the next row's cells and products, or the next tile's, ahead of this one's requant (85; 56x56x32 -> 144 -> 32 89.7 -> 92.3).
 // ---------------------------------------------------------------------------
@@ -403,17 +403,17 @@ static bool preShiftedRequant(const Requant &rq) {
 }
 
 // The time of a launch, us: of a workgroup alone on its CU a start, its chunks, each of which costs something whatever its size, then a share a tile
-// of a wave and a share an output row, and at the end the add of its rows; of those that share a CU more.  Fitted (few channels: to first layers of mobile networks)
-// to 1850 blocks, half of them of mobile networks and the others of 16 .. 96 channels in and out, 1 .. 6 times as many wide ones, 7 .. 112 pixels, 1 .. 256 images:
-// nine in ten within 14 %.
+// of a wave and a share an output row, and at the end the add of its rows; of those that share a CU more.  Fitted to 789 blocks by every height of strips (few
+// channels: 111 first layers), half of them of mobile networks and the others of 16 .. 96 channels in and out, 1 .. 6 times as many wide ones, 7 .. 112 pixels, 1 .. 256 images:
+// half of 1828 within 5 %, nine in ten within 18 %, those of 96 channels in up to 40 % low; strips by it take 0.3 % longer than the best.
 static double irBlockTime(const IrBlockArgs &a) {
     struct Cost {
         double launch, start, chunk, tile, tileK, row, rowO, add, shared;
         int perCu;
     };
-    constexpr Cost dense{2.82, 2.23, 0.343, 0.184, 0.088, 0.046, 0.064, 0.065, 0.386, 2}, runs{2.9, 0.9, 0.36, 0.41, 0.0, 0.36, 0.074, 0.0, 0.34, 4};
+    constexpr Cost dense{2.61, 1.41, 0.439, 0.174, 0.062, 0.051, 0.045, 0.086, 0.508, 2}, runs{2.62, 0.97, 0.01, 0.361, 0.067, 0.085, 0.067, 0.0, 0.434, 4};
     const Cost &c = a.CKH > 0 ? runs : dense;
-    const int KS = (a.K + 31) / 32, OT = (a.O + 15) / 16, imageRows = a.cellRows < a.H ? a.cellRows : a.H;
+    const int KS = a.CKH > 0 ? (a.CKH + 1) / 2 : (a.K + 31) / 32, OT = (a.O + 15) / 16, imageRows = a.cellRows < a.H ? a.cellRows : a.H;
     const long long blocks = (long long)a.N * a.strips * a.columnBlocks, room = 256LL * c.perCu, rest = blocks % room;
     const int tiles = (imageRows * a.regionColumns + 127) / 128, chunks = (a.C + 31) / 32;
     const double alone = c.start + chunks * (c.chunk + tiles * (c.tile + c.tileK * (KS - 1)) + a.segmentRows * (c.row + c.rowO * OT)) + (a.skip ? a.segmentRows * OT * c.add : 0.0);
@@ -421,11 +421,17 @@ static double irBlockTime(const IrBlockArgs &a) {
     return c.launch + (double)(blocks / room) * together(c.perCu) + together((rest + 255) / 256);
 }
 
-// The time of ir_expand_dw_i8 and the pointwise convolution behind it, us, fitted to the same blocks (nine in ten within 15 %): millions of widened, depthwise
-// and narrow values, and wide channels.  The choice by the two costs 0.6 % of the better one's time over them, always two launches 5 %, always one 31 %.
+// The time of ir_expand_dw_i8, by its own estimate, and the pointwise convolution behind it, us, by millions of depthwise and narrow values and wide channels: nine in
+// ten of the 1828 within 6 %.  The choice by the two costs 0.2 % of the better one's time over them and 1.3 at most, always two launches 6 %, always one 43 %; 45 of
+// them are more than 3 % behind the other way.  First layers are all one launch (two: 1.7 times the time).
 static double irPairTime(const IrBlockArgs &a) {
-    const double wide = 1e-6 * a.N * a.H * a.W * ((a.C + 31) / 32 * 32), out = 1e-6 * a.N * a.OH * a.OW, ch = 0.01 * a.C;
-    return a.CKH > 0 ? 8.2 + 0.53 * wide + out * (0.73 * a.C + 0.44 * a.O) + 3.0 * ch : 6.76 + 0.247 * wide + out * (0.75 * a.C + 0.357 * a.O) + 0.27 * ch;
+    IrExpandDwArgs f{};
+    f.x = a.x; f.wexp = a.wexp; f.bias1 = a.bias1; f.scale1 = a.scale1; f.wdw = a.wdw; f.bias2 = a.bias2; f.scale2 = a.scale2; f.out = a.out;
+    f.N = a.N; f.H = a.H; f.W = a.W; f.K = a.K; f.Kp = a.Kp; f.Np = a.Np; f.C = a.C; f.OH = a.OH; f.OW = a.OW; f.S = a.S; f.PT = a.PT; f.PL = a.PL;
+    f.CKH = a.CKH; f.CS = a.CS; f.CPT = a.CPT; f.CPL = a.CPL; f.IH = a.IH; f.IW = a.IW; f.IC = a.IC; f.runBytes = a.runBytes; f.xBytes = a.xBytes;
+    const double out = 1e-6 * a.N * a.OH * a.OW;
+    const double narrow = a.CKH > 0 ? 2.4 + out * (0.229 * a.C + 0.562 * a.O) : 2.42 + out * (0.234 * a.C + 0.409 * a.O) + 0.0018 * a.C + (a.skip ? 0.157 + 0.267 * out * a.O : 0.0);
+    return irExpandDwTime(f) + narrow;
 }
 
 bool planIrBlock(IrBlockArgs *args) {

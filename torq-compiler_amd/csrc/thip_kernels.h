@@ -185,6 +185,8 @@ bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL);
 bool irExpandDwBetter(int64_t wide, int OW, int stride);
 // Checks the arguments and sets what is the launch's own to choose; false where the kernel does not take them.
 bool planIrExpandDw(IrExpandDwArgs *a);
+// The launch's estimated time, us; infinite where the kernel does not take the arguments.
+double irExpandDwTime(const IrExpandDwArgs &a);
 hipError_t launchIrExpandDw(const IrExpandDwArgs &a, const LaunchCtx &ctx);
 
 // The two convolutions of IrExpandDwArgs and, behind them, the pointwise one that alone reads their result (C -> O channels), and
