@@ -26,7 +26,7 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
           "-Xclang", "-target-feature", "-Xclang", "-dot6-insts"]
 
 
-HEADERS = ["thip_kernels.h", "thip_kernels_common.h", "thip_descriptor.h", "thip_status.h", "thip_validate.h", "thip_plan.h", "thip_inverted_residual.h", "thip_dec_chain.h", "thip_host_copy.h", "thip_chain_turn.h"]
+HEADERS = ["thip_kernels.h", "thip_kernels_common.h", "thip_descriptor.h", "thip_status.h", "thip_validate.h", "thip_plan.h", "thip_inverted_residual.h", "thip_ir_depthwise.h", "thip_dec_chain.h", "thip_host_copy.h", "thip_chain_turn.h"]
 
 
 def _up_to_date(src, obj):

@@ -1,6 +1,7 @@
 // gfx950 kernel of the front half of an inverted-residual block: the pointwise convolution that widens the channels and the
 // 3 x 3 depthwise convolution behind it as one launch, the widened image never leaving LDS.
 #include "thip_inverted_residual.h"
+#include "thip_ir_depthwise.h"
 #include "thip_kernels_common.h"
 
 #include <math.h>
@@ -207,7 +208,7 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
     const int slot = lane & 15, group = lane >> 4;
     // channels beyond C, half a chunk, are made of the chunk's first ones and stored nowhere
     const bool whole = ch0 + 32 <= p.C, stored = whole || group < 2;
-    const uint32_t tapAt = whole || slot < 8 ? 8 * (slot >> 2) + (slot & 3) : 0, channelAt = stored ? 8 * group : 0;
+    const uint32_t tapAt = depthwiseTapAt(whole, slot), channelAt = stored ? 8 * group : 0;
     uint32_t taps[2][3];
     v4i bias2[2], scale2[2];
 #pragma unroll
@@ -221,15 +222,7 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
 
     // ---- phase 2 ----
     v4i wd[2][3];
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-#pragma unroll
-        for (int kh = 0; kh < 3; kh++) {
-            const uint32_t tap = group < 3 ? (taps[j][kh] >> (8 * group) & 0xffu) << (8 * (slot & 3)) : 0u;
-#pragma unroll
-            for (int d = 0; d < 4; d++) wd[j][kh][d] = d == (slot >> 2) ? (int)tap : 0;
-        }
-    }
+    depthwiseWeights(taps, slot, group, wd);
     const WideRequant w2 = wideRequant(p.rq2);
     const int items = p.OW * p.segments * images, count = irWalkedRows(p, part);
     const uint32_t step = (uint32_t)(p.OW * p.C);
@@ -252,20 +245,9 @@ __global__ __launch_bounds__(256, KS <= 3 ? 4 : 3) void ir_expand_dw_i8(IrExpand
             const int8_t *src = cells + column.first + (group < 3 ? group : 2) * kIrPitch;
             uint32_t dst = (uint32_t)(((image * p.OH + column.oy) * p.OW + ox) * p.C + ch0 + 8 * group);
             v4i ring[3][2];
-            auto row = [&](v4i(&o)[2]) {
-#pragma unroll
-                for (int j = 0; j < 2; j++) o[j] = *(const v4i *)(src + j * planeBytes);
-                src += cellRowBytes;
-            };
+            auto row = [&](v4i(&o)[2]) { depthwiseRow(src, planeBytes, cellRowBytes, o); };
             auto emit = [&](int r, const v4i(&r0)[2], const v4i(&r1)[2], const v4i(&r2)[2]) {
-                v2i o;
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    v4i acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wd[j][0], r0[j], bias2[j], 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wd[j][1], r1[j], acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wd[j][2], r2[j], acc, 0, 0, 0);
-                    o[j] = (int)requantPack4<kMode>(acc, scale2[j], 0, p.rq2, w2);
-                }
+                const v2i o = depthwiseResults<kMode>(wd, r0, r1, r2, bias2, scale2, p.rq2, w2);
                 if (r < left) ((UnalignedV2 *)(out + dst))->v = o;
                 dst += step;
             };

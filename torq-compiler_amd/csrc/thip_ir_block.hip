@@ -1,5 +1,6 @@
 // gfx950 kernel of a whole inverted-residual block: the pointwise convolution that widens the channels, the 3 x 3 depthwise
 // convolution, the pointwise one that narrows them again, and the residual add behind it, as one launch.
+#include "thip_ir_depthwise.h"
 #include "thip_kernels_common.h"
 
 #include <utility>
@@ -157,7 +158,7 @@ __global__ __launch_bounds__(256, RUNS ? 4 : 2) void ir_block_i8(IrBlockArgs p, 
     auto loadDepthwise = [&](int chunk) {
         const int ch0 = chunk * 32;
         const bool whole = ch0 + 32 <= p.C;
-        const uint32_t tapAt = whole || slot < 8 ? 4u * (8 * (slot >> 2) + (slot & 3)) : 0u, channelAt = whole || group < 2 ? 32u * group : 0u;
+        const uint32_t tapAt = 4 * depthwiseTapAt(whole, slot), channelAt = whole || group < 2 ? 32u * group : 0u;
 #pragma unroll
         for (int j = 0; j < 2; j++) {
 #pragma unroll
@@ -302,38 +303,17 @@ __global__ __launch_bounds__(256, RUNS ? 4 : 2) void ir_block_i8(IrBlockArgs p, 
     };
     // f(row, the narrowing convolution's operand): output rows of the strip one by one
     auto depthwise = [&](const int8_t *buffer, auto &&f) {
-        v4i wd[2][3];
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-#pragma unroll
-            for (int kh = 0; kh < 3; kh++) {
-                const uint32_t tap = group < 3 ? (taps[j][kh] >> (8 * group) & 0xffu) << (8 * (slot & 3)) : 0u;
-#pragma unroll
-                for (int d = 0; d < 4; d++) wd[j][kh][d] = d == (slot >> 2) ? (int)tap : 0;
-            }
-        }
-        v4i ring[3][2];
+        v4i wd[2][3], ring[3][2];
+        depthwiseWeights(taps, slot, group, wd);
         const int8_t *src = buffer + src0;
-        auto row = [&](v4i(&o)[2]) {
-#pragma unroll
-            for (int j = 0; j < 2; j++) o[j] = *(const v4i *)(src + j * planeBytes);
-            src += cellRowBytes;
-        };
+        auto row = [&](v4i(&o)[2]) { depthwiseRow(src, planeBytes, cellRowBytes, o); };
         row(ring[0]);
         if (S == 1) row(ring[1]);
         firstOf(std::make_integer_sequence<int, RT>{}, p.segmentRows, [&](auto tag) {
             constexpr int r = decltype(tag)::value, i0 = r * S % 3, i1 = (i0 + 1) % 3, i2 = (i0 + 2) % 3;
             if (S == 2) row(ring[i1]);
             row(ring[i2]);
-            v2i o;
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                v4i acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wd[j][0], ring[i0][j], bias2[j], 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wd[j][1], ring[i1][j], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wd[j][2], ring[i2][j], acc, 0, 0, 0);
-                o[j] = (int)requantPack4<DW>(acc, scale2[j], 0, p.rq2, w2);
-            }
-            f(tag, __builtin_bit_cast(long, o));
+            f(tag, __builtin_bit_cast(long, depthwiseResults<DW>(wd, ring[i0], ring[i1], ring[i2], bias2, scale2, p.rq2, w2)));
         });
     };
 
