@@ -33,7 +33,21 @@ int main(int argc, char **argv) {
     p.runBytes = v[17] * p.IC;
     p.xBytes = (int64_t)p.N * p.IH * p.IW * p.IC;
     if (p.CKH) p.Kp = 64;
+    const IrExpandDwArgs asked = p;
     if (!planIrExpandDw(&p)) return fail("refused", 0, 0, 0);
+    // what a program has chosen before its launches: the same layout, and none that does not fit
+    IrExpandDwArgs chosen = asked, again = asked;
+    if (!(irExpandDwTime(&chosen) < 1e9)) return fail("no time", 0, 0, 0);
+    again.images = chosen.images;
+    again.stripRows = chosen.stripRows;
+    if (!planIrExpandDw(&again) || memcmp(&again, &p, sizeof(p)) != 0) return fail("another layout", chosen.images, chosen.stripRows, 0);
+    const int wrong[][2] = {{13, p.OH}, {p.N + 1, p.OH}, {1, 0}, {0, 1}, {-1, 1}, {1, p.OH + 1}, {2, p.OH - 1}};
+    for (auto &w : wrong) {
+        again = asked;
+        again.images = w[0];
+        again.stripRows = w[1];
+        if (planIrExpandDw(&again)) return fail("taken", w[0], w[1], 0);
+    }
     const bool runs = p.CKH > 0;
     const int rowBytes = p.cellCols * kIrPitch;
     for (int n = 0; n < p.N; n += p.images) {

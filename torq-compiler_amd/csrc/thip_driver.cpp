@@ -565,6 +565,7 @@ static thip_status_t launchStep(thip_executable_t *e, const Step &s, uint8_t *co
             a.runBytes = x.KW * x.C; a.czp = x.input_zp;
             a.xBytes = (int64_t)x.N * x.H * x.W * x.C;
         }
+        a.images = s.images; a.stripRows = s.stripRows;
         err = launchIrExpandDw(a, parts);
         if (err == hipSuccess && s.count == 3) return launchOp(e, s.first + 2, e->ops[s.first + 2], bp, parts, scratch, nullptr, s.route, 0, true);
         break;

@@ -359,26 +359,9 @@ static double irTime(const IrExpandDwArgs &a) {
     return c.launch + (double)(blocks / room) * (alone + (perCu - 1) * more) + (rest > 0 ? alone + (double)(rest - 1) * more : 0.0);
 }
 
-bool planIrExpandDw(IrExpandDwArgs *args) {
+static bool chooseIrLayout(IrExpandDwArgs *args) {
     IrExpandDwArgs &a = *args;
-    if (!a.x || !a.wexp || !a.bias1 || !a.scale1 || !a.wdw || !a.bias2 || !a.scale2 || !a.out) return false;
-    if (a.N <= 0 || a.H <= 0 || a.W <= 0 || a.C <= 0 || a.C % 16 != 0 || a.OH <= 0 || a.OW <= 0) return false;
-    if (!irExpandDwFits(a.K, a.CKH, a.OW, a.S, a.PT, a.PL) || a.Kp < (a.CKH > 0 ? (a.CKH + 1) / 2 * 32 : (a.K + 31) / 32 * 32) || a.Np < (a.C + 31) / 32 * 32) return false;
-    if (a.CKH > 0) {
-        // the runs of every output pixel start inside the image or its padding (the kernel checks every byte against the image)
-        if (a.IH <= 0 || a.IW <= 0 || a.IC <= 0 || a.CS <= 0 || a.CPT < 0 || a.CPL < 0 || a.runBytes <= 0 || a.runBytes > 16 || a.runBytes % a.IC != 0) return false;
-        if (a.xBytes != (int64_t)a.N * a.IH * a.IW * a.IC || a.xBytes < 16) return false;
-        // a workgroup's images and the padding around them, in 31 bits
-        if ((long long)a.IH * a.IW * a.IC > (1LL << 27)) return false;
-    } else if ((uintptr_t)a.x & 15) {
-        return false;
-    }
-    if (((uintptr_t)a.wexp | (uintptr_t)a.bias1 | (uintptr_t)a.scale1 | (uintptr_t)a.wdw | (uintptr_t)a.bias2 | (uintptr_t)a.scale2) & 15) return false;
-    if (((uintptr_t)a.out) & 3 || (a.CKH == 0 && (long long)a.H * a.W * a.K >= (1LL << 31))) return false;
-    // every window starts inside the image or its padding and none needs a row the strip does not make
-    if ((a.OH - 1) * a.S - a.PT >= a.H || (a.OW - 1) * a.S - a.PL >= a.W) return false;
     a.cellCols = irCellColumns(a.OW, a.S);
-    if ((long long)a.C > kIrMaxChannels) return false;
     // Strips of rows, or whole images, as the estimate has them, heights a fifth apart: neighbouring ones hardly differ.  Both ways end where a
     // launch takes half as long again as the best one: it only gets longer behind that.
     constexpr long long enough = 20000;  // workgroups: strips that make more of them gain nothing
@@ -405,6 +388,36 @@ bool planIrExpandDw(IrExpandDwArgs *args) {
     for (int n = 2; n <= kIrMaxImages && n <= a.N && irLds(n, irCellRows(a, n, a.OH), a.cellCols) <= kIrMaxLds && consider(n, a.OH); n++) {}
     if (best < 0.0) return false;
     irLayout(&a, images, stripRows);
+    return true;
+}
+
+bool planIrExpandDw(IrExpandDwArgs *args) {
+    IrExpandDwArgs &a = *args;
+    if (!a.x || !a.wexp || !a.bias1 || !a.scale1 || !a.wdw || !a.bias2 || !a.scale2 || !a.out) return false;
+    if (a.N <= 0 || a.H <= 0 || a.W <= 0 || a.C <= 0 || a.C % 16 != 0 || a.OH <= 0 || a.OW <= 0) return false;
+    if (!irExpandDwFits(a.K, a.CKH, a.OW, a.S, a.PT, a.PL) || a.Kp < (a.CKH > 0 ? (a.CKH + 1) / 2 * 32 : (a.K + 31) / 32 * 32) || a.Np < (a.C + 31) / 32 * 32) return false;
+    if (a.CKH > 0) {
+        // the runs of every output pixel start inside the image or its padding (the kernel checks every byte against the image)
+        if (a.IH <= 0 || a.IW <= 0 || a.IC <= 0 || a.CS <= 0 || a.CPT < 0 || a.CPL < 0 || a.runBytes <= 0 || a.runBytes > 16 || a.runBytes % a.IC != 0) return false;
+        if (a.xBytes != (int64_t)a.N * a.IH * a.IW * a.IC || a.xBytes < 16) return false;
+        // a workgroup's images and the padding around them, in 31 bits
+        if ((long long)a.IH * a.IW * a.IC > (1LL << 27)) return false;
+    } else if ((uintptr_t)a.x & 15) {
+        return false;
+    }
+    if (((uintptr_t)a.wexp | (uintptr_t)a.bias1 | (uintptr_t)a.scale1 | (uintptr_t)a.wdw | (uintptr_t)a.bias2 | (uintptr_t)a.scale2) & 15) return false;
+    if (((uintptr_t)a.out) & 3 || (a.CKH == 0 && (long long)a.H * a.W * a.K >= (1LL << 31))) return false;
+    // every window starts inside the image or its padding and none needs a row the strip does not make
+    if ((a.OH - 1) * a.S - a.PT >= a.H || (a.OW - 1) * a.S - a.PL >= a.W) return false;
+    a.cellCols = irCellColumns(a.OW, a.S);
+    if ((long long)a.C > kIrMaxChannels) return false;
+    if (a.images == 0 && a.stripRows == 0) {
+        if (!chooseIrLayout(&a)) return false;
+    } else {
+        if (a.images < 1 || a.images > kIrMaxImages || a.images > a.N || a.stripRows < 1 || a.stripRows > a.OH || (a.images > 1 && a.stripRows != a.OH)) return false;
+        irLayout(&a, a.images, a.stripRows);
+        if (irLaunchLds(a) > kIrMaxLds) return false;
+    }
     // 128 pixels on, in images, rows and columns
     a.stepImages = a.images > 1 ? 128 / (a.H * a.W) : 0;
     a.stepRows = (128 - a.stepImages * a.H * a.W) / a.W;
@@ -412,9 +425,9 @@ bool planIrExpandDw(IrExpandDwArgs *args) {
     return true;
 }
 
-double irExpandDwTime(const IrExpandDwArgs &in) {
-    IrExpandDwArgs a = in;
-    return planIrExpandDw(&a) ? irTime(a) : HUGE_VAL;
+double irExpandDwTime(IrExpandDwArgs *args) {
+    IrExpandDwArgs &a = *args;
+    return a.N > 0 && a.H > 0 && a.W > 0 && a.C > 0 && a.OH > 0 && a.OW > 0 && irExpandDwFits(a.K, a.CKH, a.OW, a.S, a.PT, a.PL) && chooseIrLayout(&a) ? irTime(a) : HUGE_VAL;
 }
 
 hipError_t launchIrExpandDw(const IrExpandDwArgs &in, const LaunchCtx &ctx) {

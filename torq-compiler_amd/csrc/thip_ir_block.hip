@@ -406,12 +406,10 @@ static double irBlockTime(const IrBlockArgs &a) {
 // them are more than 3 % behind the other way.  First layers are all one launch (two: 1.7 times the time).
 static double irPairTime(const IrBlockArgs &a) {
     IrExpandDwArgs f{};
-    f.x = a.x; f.wexp = a.wexp; f.bias1 = a.bias1; f.scale1 = a.scale1; f.wdw = a.wdw; f.bias2 = a.bias2; f.scale2 = a.scale2; f.out = a.out;
-    f.N = a.N; f.H = a.H; f.W = a.W; f.K = a.K; f.Kp = a.Kp; f.Np = a.Np; f.C = a.C; f.OH = a.OH; f.OW = a.OW; f.S = a.S; f.PT = a.PT; f.PL = a.PL;
-    f.CKH = a.CKH; f.CS = a.CS; f.CPT = a.CPT; f.CPL = a.CPL; f.IH = a.IH; f.IW = a.IW; f.IC = a.IC; f.runBytes = a.runBytes; f.xBytes = a.xBytes;
+    f.N = a.N; f.H = a.H; f.W = a.W; f.K = a.K; f.C = a.C; f.OH = a.OH; f.OW = a.OW; f.S = a.S; f.PT = a.PT; f.PL = a.PL; f.CKH = a.CKH;
     const double out = 1e-6 * a.N * a.OH * a.OW;
     const double narrow = a.CKH > 0 ? 2.4 + out * (0.229 * a.C + 0.562 * a.O) : 2.42 + out * (0.234 * a.C + 0.409 * a.O) + 0.0018 * a.C + (a.skip ? 0.157 + 0.267 * out * a.O : 0.0);
-    return irExpandDwTime(f) + narrow;
+    return irExpandDwTime(&f) + narrow;
 }
 
 bool planIrBlock(IrBlockArgs *args) {

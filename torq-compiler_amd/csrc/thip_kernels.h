@@ -175,7 +175,8 @@ struct IrExpandDwArgs {
     // stride CS, whose H x W outputs take the pixels' place; K is unused
     int32_t CKH, CS, CPT, CPL, IH, IW, IC, runBytes, czp;
     int64_t xBytes;
-    int32_t images, stripRows, strips, segmentRows, segments, cellCols;  // planIrExpandDw sets these
+    int32_t images, stripRows;  // as irExpandDwTime has set them, or 0: planIrExpandDw chooses
+    int32_t strips, segmentRows, segments, cellCols;  // planIrExpandDw sets these
     int32_t stepImages, stepRows, stepColumns;  // and these: 128 pixels
 };
 // A strip's results are addressed with 32 bits: its cells fit LDS, so they are fewer than 2^11 pixels.
@@ -185,8 +186,9 @@ bool irExpandDwFits(int K, int runRows, int OW, int stride, int PT, int PL);
 bool irExpandDwBetter(int64_t wide, int OW, int stride);
 // Checks the arguments and sets what is the launch's own to choose; false where the kernel does not take them.
 bool planIrExpandDw(IrExpandDwArgs *a);
-// The launch's estimated time, us; infinite where the kernel does not take the arguments.
-double irExpandDwTime(const IrExpandDwArgs &a);
+// By the sizes alone: a launch's estimated time, us, infinite where the kernel does not take them, and in images and stripRows how it is made.  Choosing takes
+// the host 0.2 - 0.5 us, so a program chooses once (in every launch: three of 1x14x14x64 -> 384 10.8 / 12.1 us).
+double irExpandDwTime(IrExpandDwArgs *a);
 hipError_t launchIrExpandDw(const IrExpandDwArgs &a, const LaunchCtx &ctx);
 
 // The two convolutions of IrExpandDwArgs and, behind them, the pointwise one that alone reads their result (C -> O channels), and

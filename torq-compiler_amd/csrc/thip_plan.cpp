@@ -174,6 +174,12 @@ static bool matchExpandDw(const DescriptorView &v, const Tuning &tuning, const s
     s->kind = kStepExpandDw;
     s->first = first;
     s->count = 2;
+    IrExpandDwArgs a{};
+    a.N = d.N; a.H = d.H; a.W = d.W; a.K = e.K; a.C = d.C; a.OH = d.OH; a.OW = d.OW; a.S = d.SW; a.PT = d.PT; a.PL = d.PL; a.CKH = runs ? e.KH : 0;
+    if (irExpandDwTime(&a) < HUGE_VAL) {
+        s->images = a.images;
+        s->stripRows = a.stripRows;
+    }
     matchBlock(v, tuning, uses, s);
     if (s->count == 3 || irExpandDwBetter((int64_t)d.N * d.H * d.W * d.C, d.OW, d.SW)) return true;
     *s = Step{};

@@ -33,6 +33,7 @@ struct Step {
     StepKind kind;
     uint32_t first, count;  // the records it stands for
     IgemmRoute route;       // of the record, of `op` (kStepPadded), or of the third record where it is launched by itself (kStepExpandDw)
+    int32_t images, stripRows;  // kStepExpandDw: of a workgroup of ir_expand_dw_i8 (irExpandDwTime)
     // kStepMatmulRt: the matrices of batch element 0, elements from one batch element to the next (0: shared), and the one
     // (bias, scale) pair
     DescRef a, b, out;
