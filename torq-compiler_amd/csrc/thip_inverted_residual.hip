@@ -38,11 +38,11 @@ static inline int irCellColumns(int OW, int S) { return (OW - 1) * S + 3; }
 // its 11 MB of traffic), and at small batches each costs a dependent launch. About half of the cycles are vector instructions (5 per widened and 5 per depthwise
 // byte; with byte transposes and v_dot4_i32_i8 in phase 2 it was 9 per depthwise byte); the rest goes where a workgroup's phases and the launch's last round of workgroups wait.
 // us, in a trace of the network, with v_dot4_i32_i8 / now:
-//   batch 256  14x14x64 -> 384 17.4 / 15.1, 14x14x96 -> 576 24.6 / 23.8, its stride 2 17.3 / 16.2, 7x7x160 -> 960 17.0 / 15.0
+//   batch 256  14x14x64 -> 384 17.4 / 14.6, 14x14x96 -> 576 24.6 / 21.7, its stride 2 17.3 / 15.0, 7x7x160 -> 960 17.0 / 14.5
 // and one behind another, in time from one to the next
 //   batch 32   7x7x160 -> 960 8.0 / 5.3, 14x14x96 -> 576 7.9 / 7.4, its stride 2 6.4 / 5.7, 14x14x64 -> 384 6.0 / 6.0, 28x28x32 -> 192 7.9 / 6.9
 //   batch 1    14x14x64 -> 384 3.9 / 4.0
-// the whole network at 256 images 716 -> 695 (at 32 in host memory and at one the runs of one build differ by as much as it gave). Tried: phase 2's constants under way from the start on (registers spill from K = 96
+// the whole network at 256 images 716 -> 695, and 676 -> 672 with strips and images by irTime (at 32 in host memory and at one the runs of one build differ by as much as it gave). Tried: phase 2's constants under way from the start on (registers spill from K = 96
 // on: 23.8 -> 25.5), the requants' constants from the host (no change, and spills), more tiles prefetched (no change).
 // ---------------------------------------------------------------------------
 template <int KS, int S, bool RUNS>

@@ -312,8 +312,9 @@ static hipError_t launchRt(const MatmulRtArgs &a, const LaunchCtx &ctx) {
 // Rows of a tile, us.  Up to one workgroup per CU the smallest tile is ahead (1 x 1024x1024x1024: 6.7 on 32 rows, 7.6 on 64, 9.6 on 128), and a second
 // group of waves where there is a second k-tile for it (5.7; four groups 5.7, and behind two on 2 x 300x700x300: 5.1, 5.6); beyond that 64 rows
 // (3 x 777x333x555 -> int16: 7.6, 6.6, 8.9; 8 x 512x256x512 4.7, 4.5, 5.5; 4 x 1024x128x1024 -> int16 5.6, 5.4, 6.1) as long as all of them run at once: three a CU
-// hold two buffers of 24 KB each.  64 / 128 rows at 544 tiles of 64 rows 8 x 4352x256x128 6.8 / 7.0, at 664 2 x 10621x512x256 -> int32 11.6 / 13.9, at 736
-// 4 x 2941x1024x512 -> int32 15.5 / 16.8, at 816 4 x 3264x256x512 9.0 / 7.2, at 1024 8 x 1024x1024x1024 17.5 / 14.4 (of 84 drawn products of 257 .. 768 tiles one is faster on 128 rows by more than 1 %).
+// hold two buffers of 24 KB each.  64 / 128 rows at 544 tiles of 64 rows 8 x 4352x256x128 6.8 / 7.0, at 664 2 x 10621x512x256 -> int32 12.3 / 14.0, at 736
+// 4 x 2941x1024x512 -> int32 16.9 / 17.5, at 816 4 x 3264x256x512 8.8 / 7.0, at 1024 8 x 1024x1024x1024 17.7 / 15.0.  Of 84 drawn products of 257 .. 768 tiles two are
+// faster on 128 rows by more than 1 %, of 40 of more tiles eleven on 64 (short K, or 2 x 8512x512x512 -> int32, 1064 tiles, 18.1 / 20.8).
 template <int OUT>
 static hipError_t launchRtOut(const MatmulRtArgs &a, const LaunchCtx &ctx) {
     auto tiles = [&](int bm) { return (long long)a.batches * ((a.M + bm - 1) / bm) * ((a.N + 127) / 128); };
