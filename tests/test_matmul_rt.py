@@ -38,7 +38,8 @@ def test_runtime_input2(device, kw, tmp_path):
 
 
 # the smallest tile with one group of waves and with two, 64 rows, 128 rows: (B, M, N), template arguments up to the k-tile groups
-TILES = [((2, 33, 17), (32, 1, 4)), ((16, 1, 144), (32, 1, 4)), ((16, 65, 1030), (64, 2, 2)), ((24, 400, 520), (128, 2, 2))]
+TILES = [((2, 33, 17), (32, 1, 4)), ((16, 1, 144), (32, 1, 4)), ((9, 130, 250), (32, 1, 4)), ((16, 65, 1030), (64, 2, 2)), ((24, 400, 520), (128, 2, 2))]
+TILE_IDS = ["32rows-ragged", "one-row", "32rows-batches", "64rows", "128rows"]
 DTYPE_CODES = {np.int8: 1, np.int16: 2, np.int32: 3}
 
 
@@ -53,7 +54,7 @@ def on_tile(device, wl, rows, K, out):
 
 
 @pytest.mark.parametrize("K", [1, 16, 127, 128, 129, 143, 144, 256, 257, 300, 400, 513])
-@pytest.mark.parametrize("sizes, rows", TILES, ids=["32rows-ragged", "one-row", "64rows", "128rows"])
+@pytest.mark.parametrize("sizes, rows", TILES, ids=TILE_IDS)
 def test_k_tiles(device, sizes, rows, K):
     """The ends of k-tiles: one, two and an odd number of them, rows of B that end a byte before, at and behind a chunk."""
     B, M, N = sizes
@@ -62,7 +63,7 @@ def test_k_tiles(device, sizes, rows, K):
 
 @pytest.mark.parametrize("K", [129, 400])
 @pytest.mark.parametrize("kw", [I8, dict(out_dtype=np.int16)], ids=["int8", "int16"])
-@pytest.mark.parametrize("sizes, rows", TILES, ids=["32rows-ragged", "one-row", "64rows", "128rows"])
+@pytest.mark.parametrize("sizes, rows", TILES, ids=TILE_IDS)
 def test_k_tiles_of_narrow_results(device, sizes, rows, kw, K):
     """Results narrower than the sums behind a loop of several k-tiles, with columns that fill no store."""
     B, M, N = sizes
